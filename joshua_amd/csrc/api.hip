@@ -7,6 +7,7 @@
 #include "kernels_mfma_q4k.hpp"
 #include "kernels_graph.hpp"
 #include "kernels_mla.hpp"
+#include "split16.hpp"
 #include "kernels_mfma_q4k_gemm.hpp"
 #include "kernels_mfma_q4k_stream.hpp"
 #include "kernels_dot4_q4k.hpp"
@@ -2211,8 +2212,9 @@ struct jq_mla {
     float *lat = nullptr, *kpe = nullptr;  // the cache: [n_ctx][lkv] normed latents, [n_ctx][rope] rotated keys
     float scale = 0.0f;
     size_t n_past = 0;
-    // scratch, grown to the largest token count seen
-    size_t cap_tokens = 0;
+    Split16Latent *split16 = nullptr;  // keys and values per head for calls of many tokens (null: a geometry it does not take)
+    // scratch, grown to the largest token count seen; qabs and part to the largest of an absorbed call
+    size_t cap_tokens = 0, cap_absorbed = 0;
     float *t1 = nullptr, *t1n = nullptr, *qv = nullptr, *comp = nullptr, *qabs = nullptr, *part = nullptr, *ctx = nullptr;
     std::vector<void *> retired;  // outgrown scratch, kept until the object goes
     std::mutex mu;
@@ -2228,18 +2230,36 @@ void mla_free_scratch(jq_mla *m) {
     for (void *p : m->retired) (void)hipFree(p);
     m->retired.clear();
     m->t1 = m->t1n = m->qv = m->comp = m->qabs = m->part = m->ctx = nullptr;
-    m->cap_tokens = 0;
+    m->cap_tokens = m->cap_absorbed = 0;
 }
 
-// Scratch for calls of up to T tokens.  Buffers that are outgrown are retired, not freed: a HIP graph captured
-// over an earlier, smaller call still names them, and they go with the object (jq_mla_free).
-int mla_reserve(jq_mla *m, size_t T) {
-    if (T <= m->cap_tokens) return 0;
-    for (void *p : {(void *)m->t1, (void *)m->t1n, (void *)m->qv, (void *)m->comp, (void *)m->qabs, (void *)m->part, (void *)m->ctx})
-        if (p) m->retired.push_back(p);
-    m->t1 = m->t1n = m->qv = m->comp = m->qabs = m->part = m->ctx = nullptr;
-    m->cap_tokens = 0;
+// Tokens from which a call expands the cached latents to keys and values per head instead of absorbing the up-projection
+// into its queries.  Expanding costs 33.5 M multiply-adds a cached token and layer of DeepSeek-V3's size however many tokens
+// the call has, and saves 98 k a pair of tokens.  Whole calls, us, absorbed / expanded: 32 tokens behind 0, 1000, 4000: 307 / 308,
+// 399 / 511, 654 / 1063; 48 tokens 481 / 409, 652 / 613, 1171 / 1165; 96 tokens 975 / 544, 1326 / 732, 2358 / 1290; 192
+// tokens 2430 / 957, 2962 / 1130, 4518 / 1845.
+constexpr size_t MLA_EXPAND_TOKENS = 48;
+
+// Scratch for calls of up to T tokens, of which up to `absorbed` in absorbed form.  Buffers that are outgrown are retired,
+// not freed: a HIP graph captured over an earlier, smaller call still names them, and they go with the object (jq_mla_free).
+int mla_reserve(jq_mla *m, size_t T, size_t absorbed) {
     const jq_mla_config &c = m->cfg;
+    if (absorbed > m->cap_absorbed) {
+        for (float **p : {&m->qabs, &m->part}) {
+            if (*p) m->retired.push_back(*p);
+            *p = nullptr;
+        }
+        m->cap_absorbed = 0;
+        HIP_TRY(hipMalloc((void **)&m->qabs, absorbed * c.n_head * c.kv_lora_rank * sizeof(float)));
+        HIP_TRY(hipMalloc((void **)&m->part, std::max(absorbed, MLA_PART_SLOTS) * c.n_head * (c.kv_lora_rank + 2) * sizeof(float)));
+        m->cap_absorbed = absorbed;
+    }
+    if (T <= m->cap_tokens) return 0;
+    for (float **p : {&m->t1, &m->t1n, &m->qv, &m->comp, &m->ctx}) {
+        if (*p) m->retired.push_back(*p);
+        *p = nullptr;
+    }
+    m->cap_tokens = 0;
     const size_t qd = c.qk_nope_head_dim + c.qk_rope_head_dim;
     if (c.q_lora_rank) {
         HIP_TRY(hipMalloc((void **)&m->t1, T * c.q_lora_rank * sizeof(float)));
@@ -2247,8 +2267,6 @@ int mla_reserve(jq_mla *m, size_t T) {
     }
     HIP_TRY(hipMalloc((void **)&m->qv, T * c.n_head * qd * sizeof(float)));
     HIP_TRY(hipMalloc((void **)&m->comp, T * (c.kv_lora_rank + c.qk_rope_head_dim) * sizeof(float)));
-    HIP_TRY(hipMalloc((void **)&m->qabs, T * c.n_head * c.kv_lora_rank * sizeof(float)));
-    HIP_TRY(hipMalloc((void **)&m->part, std::max(T, MLA_PART_SLOTS) * c.n_head * (c.kv_lora_rank + 2) * sizeof(float)));
     HIP_TRY(hipMalloc((void **)&m->ctx, T * c.n_head * c.v_head_dim * sizeof(float)));
     m->cap_tokens = T;
     return 0;
@@ -2353,6 +2371,12 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
                            (const float *)m->kv_a_norm, (const float2 *)m->cs, m->lat, m->kpe, (int)nh, (int)nope, (int)rope,
                            (int)lkv, (int)pos, c.rms_eps);
         HIP_TRY(hipGetLastError());
+        if (m->split16 && S >= MLA_EXPAND_TOKENS) {
+            const int rc = split16_latent_attention(m->split16, m->qv, S, pos, m->lat, m->kpe, m->scale, m->ctx, s);
+            if (rc > 0) return 1;
+            if (rc == 0) return dispatch_matmul(m->o->type, m->o->dev, m->o->row_bytes, m->ctx, out, S, nh * vh, c.n_embd, s);
+            if (mla_reserve(m, S, S)) return 1;  // no memory for the expanded cache: the absorbed form
+        }
         // one token a workgroup in a decode step, four in a prefill; 16-byte loads when the latent width allows
         {
             const dim3 grid((unsigned)nh, (unsigned)((S + st - 1) / st));
@@ -2482,6 +2506,7 @@ int jq_mla_create(const jq_mla_config *cfg, const jq_weight *q_or_q_a, const flo
     HIP_TRY(hipMemcpy(m->cs, cs.data(), cs.size() * sizeof(float2), hipMemcpyHostToDevice));
     HIP_TRY(hipMalloc((void **)&m->lat, (size_t)c.n_ctx * lkv * sizeof(float)));
     HIP_TRY(hipMalloc((void **)&m->kpe, (size_t)c.n_ctx * rope * sizeof(float)));
+    if (split16_latent_fits(nope, rope, vh, lkv) && split16_latent_create(nh, c.n_ctx, m->wkv, kv_a_norm, &m->split16)) return 1;
     HIP_TRY(hipDeviceSynchronize());
     *out = m.release();
     return 0;
@@ -2490,6 +2515,7 @@ int jq_mla_create(const jq_mla_config *cfg, const jq_weight *q_or_q_a, const flo
 void jq_mla_free(jq_mla *m) {
     if (!m) return;
     mla_free_scratch(m);
+    split16_latent_free(m->split16);
     for (void *p : {(void *)m->q_a_norm, (void *)m->kv_a_norm, (void *)m->wkv, (void *)m->cs, (void *)m->lat, (void *)m->kpe,
                     (void *)m->qa_kva, (void *)m->qa_kva_out})
         if (p) (void)hipFree(p);
@@ -2505,7 +2531,8 @@ int jq_mla_forward(jq_mla *m, size_t n_tokens, size_t pos, const float *x, float
     if (pos + n_tokens > m->cfg.n_ctx) return fail("jq_mla_forward: %zu + %zu tokens exceed the context of %u", pos, n_tokens, m->cfg.n_ctx);
     if (n_tokens > 0x7FFF) return fail("jq_mla_forward: at most 32767 tokens a call");
     hipStream_t s = (hipStream_t)stream;
-    if (mla_reserve(m, n_tokens)) return 1;
+    // (a call that expands the cache leaves scratch for the absorbed ones below it too: they then allocate nothing)
+    if (mla_reserve(m, n_tokens, m->split16 ? std::min(n_tokens, MLA_EXPAND_TOKENS) : n_tokens)) return 1;
     const size_t bytes = n_tokens * m->cfg.n_embd * sizeof(float);
     if (ptrs_are_device) {
         if (mla_forward_dev(m, n_tokens, pos, x, out, s)) return 1;
@@ -2561,6 +2588,7 @@ struct Qwen3Model : jq_model {
     std::map<std::string, std::vector<float>> router_host;
     std::vector<jq_moe *> moe;
     int moe_scratch_at = -1;
+    Split16Cache split16;     // one layer's cache as operands of the many-token attention, made at its first use
 
     ~Qwen3Model() override;
     int step(const uint32_t *tokens, uint32_t n, const uint32_t *want, uint32_t n_want, hipStream_t s) override;
@@ -2763,6 +2791,12 @@ bool model_norm_mm(const jq_weight *w, const float *x, const float *res, const f
     return dispatch_q4k_dot4(w->dev, w->row_bytes, x, y, w->k, w->n, s, &nm, swiglu) == 0;
 }
 
+// Steps whose attention runs on split f16 operands (kernels_split16.hpp) instead of the f32 matrix cores.  Below, the copy of
+// the cache into operands, a launch more, eats what it gains.  Whole steps of four layers of Qwen3-8B's sizes, us, f32 / split:
+// 9 tokens 463 / 468, 16 tokens 501 / 504, 32 tokens 675 / 664, 256 tokens 1414 / 1318; behind 1000 tokens 9 tokens 840 / 678,
+// 256 tokens 1794 / 1517; behind 4000 tokens 9 tokens 1973 / 1237.
+bool split16_attention_pays(uint32_t T, uint32_t pos) { return T >= 32 || pos + T >= 128; }
+
 int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *want, uint32_t n_want, hipStream_t s) {
     const jq_qwen3_config &c = m->cfg;
     const int d = (int)c.head_dim, nh = (int)c.n_head, nkv = (int)c.n_kv_head, h = (int)c.hidden;
@@ -2848,24 +2882,22 @@ int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *w
             static const char *no_tiles = getenv("JQ_NO_ATTENTION_TILES");
             const int gq = nh / nkv;
             const dim3 tgrid((unsigned)((T + 15) / 16), (unsigned)nkv);
-#define JQ_ATT_TILES(GQ, KS)                                                                                        \
-    hipLaunchKernelGGL((jq::attention_tiles<128, GQ, KS>), tgrid, dim3(64 * GQ * KS), 0, s, qp, m->kc[l], m->vc[l],   \
-                       m->att, (int)T, nh, m->pos, (int)c.n_ctx, sqrt_d, q_stride)
-            // two key splits a workgroup once the last tokens walk 8 key tiles or more (up to 4 query heads a KV
-            // head: the merge of 8 would not fit the static LDS)
-            static const char *no_split_env = getenv("JQ_ATTENTION_TILES_NO_KEY_SPLIT");
-            const bool ksplit = !no_split_env && pos + T >= 128;
-            if (no_tiles || d != 128 || (gq != 1 && gq != 2 && gq != 4 && gq != 8)) {
+            int done = -1;
+            if (split16_attention_pays(T, pos) && !no_tiles && split16_attention_fits(d, nh, nkv))
+                done = split16_attention(&m->split16, qp, q_stride, (int)T, (int)pos, m->kc[l], m->vc[l], nh, nkv, (int)c.n_ctx, m->att, s);
+            if (done > 0) return 1;
+#define JQ_ATT_TILES(GQ)                                                                                          \
+    hipLaunchKernelGGL((jq::attention_tiles<128, GQ>), tgrid, dim3(64 * GQ), 0, s, qp, m->kc[l], m->vc[l], m->att,   \
+                       (int)T, nh, m->pos, (int)c.n_ctx, sqrt_d, q_stride)
+            if (done == 0) {
+            } else if (no_tiles || d != 128 || (gq != 1 && gq != 2 && gq != 4 && gq != 8)) {
                 size_t sm = ((size_t)d + jq::AR_CHUNK + 16) * sizeof(float);
                 hipLaunchKernelGGL(jq::attention_rows, dim3(T * nh), dim3(256), sm, s, qp, m->kc[l], m->vc[l], m->att, nh,
                                    nkv, d, m->pos, (int)c.n_ctx, sqrt_d, q_stride);
-            } else if (gq == 1 && ksplit) JQ_ATT_TILES(1, 2);
-            else if (gq == 1) JQ_ATT_TILES(1, 1);
-            else if (gq == 2 && ksplit) JQ_ATT_TILES(2, 2);
-            else if (gq == 2) JQ_ATT_TILES(2, 1);
-            else if (gq == 4 && ksplit) JQ_ATT_TILES(4, 2);
-            else if (gq == 4) JQ_ATT_TILES(4, 1);
-            else JQ_ATT_TILES(8, 1);
+            } else if (gq == 1) JQ_ATT_TILES(1);
+            else if (gq == 2) JQ_ATT_TILES(2);
+            else if (gq == 4) JQ_ATT_TILES(4);
+            else JQ_ATT_TILES(8);
 #undef JQ_ATT_TILES
         }
         if (model_mm(m, p + ".attn_output.weight", m->att, m->proj, T, s)) return 1;
@@ -2964,6 +2996,7 @@ int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *w
 Qwen3Model::~Qwen3Model() {
     Qwen3Model *m = this;
     model_free_scratch(m);
+    split16_cache_free(&m->split16);
     for (jq_moe *e : m->moe) jq_moe_free(e);
     for (auto &kv : m->q) jq_free(kv.second);
     for (auto &kv : m->fused) jq_free(kv.second);

@@ -1,0 +1,129 @@
+// Host side of the attention kernels on split f16 operands.
+#include "split16.hpp"
+
+#include "kernels_split16.hpp"
+
+namespace jqh {
+
+namespace {
+
+size_t tiles_of(size_t tokens) { return (tokens + jq::S16_TILE - 1) / jq::S16_TILE; }
+
+// hipMalloc that leaves no error behind where there is no memory.
+bool have(void **p, size_t bytes) {
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    *p = nullptr;
+    (void)hipGetLastError();
+    return false;
+}
+
+}  // namespace
+
+struct Split16Latent {
+    size_t n_head, n_ctx, ws_bytes = 0;
+    int ec;                              // exponent of the latents' scale
+    uint8_t *wfrags = nullptr;
+    float2 *fac = nullptr;
+    uint8_t *cf = nullptr, *rf = nullptr, *ws = nullptr;  // latents, rope keys, a group of heads' keys and values
+    float *ropeinv = nullptr;
+};
+
+bool split16_latent_fits(size_t nope, size_t rope, size_t vh, size_t lkv) {
+    return nope == jq::S16_HEAD && vh == jq::S16_HEAD && rope == jq::S16_ROPE && lkv == jq::S16_LKV;
+}
+
+int split16_latent_create(size_t n_head, size_t n_ctx, const float *wkv, const float *kv_norm, Split16Latent **out) {
+    std::unique_ptr<Split16Latent, void (*)(Split16Latent *)> s(new Split16Latent{n_head, n_ctx}, split16_latent_free);
+    float wmax = 0.0f;
+    for (int i = 0; i < jq::S16_LKV; i++) wmax = std::max(wmax, fabsf(kv_norm[i]));
+    // a normed latent's 2-norm is at most sqrt(512) times the largest norm weight
+    const float cmax = std::min(std::max(sqrtf((float)jq::S16_LKV) * wmax, 1e-20f), 1e20f);
+    int e;
+    (void)frexpf(cmax, &e);  // cmax < 2^e
+    s->ec = 14 - e;
+    HIP_TRY(hipMalloc((void **)&s->wfrags, n_head * 2 * (jq::S16_LKV / 16) * 8 * jq::S16_FRAG));
+    HIP_TRY(hipMalloc((void **)&s->fac, n_head * 2 * sizeof(float2)));
+    hipLaunchKernelGGL(jq::s16_up_projection, dim3(2, (unsigned)n_head), dim3(256), 0, nullptr, wkv, s->wfrags, s->fac, cmax, s->ec);
+    HIP_TRY(hipGetLastError());
+    *out = s.release();
+    return 0;
+}
+
+void split16_latent_free(Split16Latent *s) {
+    if (!s) return;
+    for (void *p : {(void *)s->wfrags, (void *)s->fac, (void *)s->cf, (void *)s->rf, (void *)s->ws, (void *)s->ropeinv})
+        if (p) (void)hipFree(p);
+    delete s;
+}
+
+int split16_latent_attention(Split16Latent *s, const float *q, size_t S, size_t pos, const float *lat, const float *kpe, float scale,
+                             float *out, hipStream_t stream) {
+    const size_t all = tiles_of(s->n_ctx), nt = tiles_of(pos + S), head_bytes = nt * jq::S16_KV_TILE;
+    if (!s->ws) {
+        // The whole context's keys and values of all heads up to 1 GiB, so that no later call allocates; longer contexts
+        // take the heads in groups.
+        const size_t most = (size_t)1 << 30, want = std::max(std::min(s->n_head * all * jq::S16_KV_TILE, most), all * jq::S16_KV_TILE);
+        if (!s->cf && !have((void **)&s->cf, all * (jq::S16_LKV / 16) * 2 * jq::S16_FRAG)) return -1;
+        if (!s->rf && !have((void **)&s->rf, all * jq::S16_ROPE_TILE)) return -1;
+        if (!s->ropeinv && !have((void **)&s->ropeinv, all * sizeof(float))) return -1;
+        if (!have((void **)&s->ws, want)) return -1;
+        s->ws_bytes = want;
+    }
+    hipLaunchKernelGGL(jq::s16_latent_tiles, dim3((unsigned)nt), dim3(256), 0, stream, lat, kpe, (int)(pos + S), ldexpf(1.0f, s->ec), s->cf,
+                       s->rf, s->ropeinv);
+    HIP_TRY(hipGetLastError());
+    size_t group = std::min(s->n_head, s->ws_bytes / head_bytes);
+    if (group >= 8 && group < s->n_head) group = group / 8 * 8;
+    for (size_t h0 = 0; h0 < s->n_head; h0 += group) {
+        const size_t hg = std::min(group, s->n_head - h0);
+        hipLaunchKernelGGL(jq::s16_expand, dim3((unsigned)(2 * hg * ((nt + 3) / 4))), dim3(256), 0, stream, (const uint8_t *)s->wfrags,
+                           (const float2 *)s->fac, (const uint8_t *)s->cf, (int)h0, (int)hg, (int)nt, s->ws);
+        HIP_TRY(hipGetLastError());
+        jq::S16Attention a{};
+        a.q = q + h0 * (jq::S16_HEAD + jq::S16_ROPE), a.q_stride = (int)(s->n_head * (jq::S16_HEAD + jq::S16_ROPE)), a.q_head = jq::S16_HEAD + jq::S16_ROPE;
+        a.kv = s->ws, a.inv = s->fac + 2 * h0, a.rope = s->rf, a.ropeinv = s->ropeinv;
+        a.out = out + h0 * jq::S16_HEAD, a.out_stride = (int)(s->n_head * jq::S16_HEAD);
+        a.T = (int)S, a.pos0 = (int)pos, a.n_tiles = (int)nt, a.heads = (int)hg, a.group = 1, a.blocks = (int)((S + 127) / 128);
+        a.scale_log2e = scale * 1.44269504088896340736f;
+        hipLaunchKernelGGL((jq::s16_attention<true, 1>), dim3((unsigned)(hg * a.blocks)), dim3(256), 0, stream, a);
+        HIP_TRY(hipGetLastError());
+    }
+    return 0;
+}
+
+void split16_cache_free(Split16Cache *c) {
+    if (c->ws) (void)hipFree(c->ws);
+    if (c->inv) (void)hipFree(c->inv);
+    *c = {};
+}
+
+bool split16_attention_fits(int d, int heads, int kv_heads) {
+    const int g = heads / kv_heads;
+    return d == 128 && heads % kv_heads == 0 && (g == 1 || g == 2 || g % 4 == 0);
+}
+
+int split16_attention(Split16Cache *c, const float *q, int q_stride, int T, int pos, const float *kc, const float *vc, int heads, int kv_heads,
+                      int n_ctx, float *out, hipStream_t stream) {
+    const size_t all = tiles_of((size_t)n_ctx);
+    if (!c->ws && !have((void **)&c->ws, (size_t)kv_heads * all * jq::S16_KV_TILE)) return -1;
+    if (!c->inv && !have((void **)&c->inv, (size_t)kv_heads * all * sizeof(float2))) return -1;
+    const int nt = (int)tiles_of((size_t)pos + T), g = heads / kv_heads, wh = std::min(g, 4);
+    hipLaunchKernelGGL(jq::s16_kv_tiles, dim3((unsigned)nt, (unsigned)kv_heads), dim3(256), 0, stream, kc, vc, n_ctx, pos + T, c->ws, c->inv);
+    HIP_TRY(hipGetLastError());
+    jq::S16Attention a{};
+    a.q = q, a.q_stride = q_stride, a.q_head = 128;
+    a.kv = c->ws, a.inv = c->inv;
+    a.out = out, a.out_stride = heads * 128;
+    a.T = T, a.pos0 = pos, a.n_tiles = nt, a.heads = heads, a.group = g;
+    const int tb = 32 * (4 / wh);
+    a.blocks = (T + tb - 1) / tb;
+    a.scale_log2e = (float)(1.4426950408889634 / sqrt(128.0));
+    const dim3 grid((unsigned)(heads / wh * a.blocks));
+    if (wh == 4) hipLaunchKernelGGL((jq::s16_attention<false, 4>), grid, dim3(256), 0, stream, a);
+    else if (wh == 2) hipLaunchKernelGGL((jq::s16_attention<false, 2>), grid, dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((jq::s16_attention<false, 1>), grid, dim3(256), 0, stream, a);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+}  // namespace jqh

@@ -120,6 +120,42 @@ def test_matrix_core_attention_for_the_deepseek_geometry():
     assert close(dev.forward(x[153:250], 153), ref.forward(x[153:250], 153))
 
 
+@pytest.mark.parametrize("n_head,steps", [(3, (47, 48, 129, 1)), (8, (160, 95, 48)), (16, (33, 127, 2))])
+def test_many_tokens_over_keys_and_values_per_head(n_head, steps):
+    """DeepSeek's head sizes from 48 tokens a call on: the cached latents expanded to keys and values, attention on split
+    f16 operands; calls below and above the line in turn, head counts that are no multiple of 8, part tiles of keys and
+    tokens, and inputs whose size (and with it the unnormed rope keys') differs a thousandfold between tokens."""
+    c = cfg(n_embd=256, n_head=n_head, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=128, context_length=320)
+    ref, dev = build(c, seed=800 + n_head)
+    total = sum(steps)
+    x = normal(15, (total, c["n_embd"])) * np.exp(np.linspace(-5.0, 2.0, total)[np.random.default_rng(3).permutation(total)])[:, None]
+    x, pos = x.astype(np.float32), 0
+    for n in steps:
+        assert close(dev.forward(x[pos:pos + n], pos), ref.forward(x[pos:pos + n], pos)), (pos, n)
+        pos += n
+
+
+def test_heads_in_groups_where_their_keys_and_values_exceed_the_buffer():
+    """256 heads of 4200 tokens are expanded in two groups (1 GiB of keys and values each at most).  The 256 are 32
+    copies of 8 and so are the output projection's columns: the sum is 32 times what the 8 alone give, up to the order of
+    the additions."""
+    c8 = cfg(n_embd=256, n_head=8, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=128, context_length=4224)
+    t8, few = build(c8, seed=900)
+    t8 = t8.t
+    raw = lambda name, rows: np.asarray(t8[name][1]).view(np.uint8).reshape(rows, -1)
+    q = np.tile(raw("q", 8 * 192), (32, 1))
+    kv_b = np.tile(raw("kv_b", 8 * 256), (32, 1))
+    o = np.tile(raw("o", 256), (1, 32))
+    w = {n: capi.Weight.upload(capi.Q8_0, np.ascontiguousarray(b), r, k)
+         for n, b, r, k in (("q", q, 256 * 192, 256), ("kv_a", raw("kv_a_mqa", 576), 576, 256), ("kv_b", kv_b, 65536, 512), ("o", o, 256, 32768))}
+    mc = capi.MlaConfig(n_embd=256, n_head=256, q_lora_rank=0, kv_lora_rank=512, qk_nope_head_dim=128, qk_rope_head_dim=64,
+                        v_head_dim=128, n_ctx=4224, rms_eps=1e-6, rope_theta=1e4)
+    many = capi.Mla(mc, w["q"], w["kv_a"], t8["kv_a_norm"], w["kv_b"], w["o"])
+    x = normal(16, (4200, 256))
+    a, b = few.forward(x, 0), many.forward(x, 0) / 32
+    assert np.abs(a - b).max() < 3e-4 * max(1.0, np.abs(a).max())
+
+
 def test_dense_kv_b_and_other_formats():
     c = cfg(kv_lora_rank=256, n_embd=256, v_head_dim=64)
     for qtype in (capi.Q4_K, capi.Q6_K):

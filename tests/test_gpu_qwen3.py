@@ -6,7 +6,7 @@ import pytest
 
 import oracle
 from oracle import qwen3 as oq
-from joshua_amd import capi
+from joshua_amd import capi, synth
 from joshua_amd.synth.model import qwen3_tensors
 
 pytestmark = pytest.mark.gpu
@@ -204,6 +204,29 @@ def test_long_prefill_chunks_split_their_keys_between_two_sets_of_waves(n_head, 
         ok, e = close(m.forward(chunk, pos), o.forward(chunk, pos))
         assert ok, f"pos {pos} +{step}: {e}"
         pos += step
+
+
+@pytest.mark.parametrize("n_head,n_kv,steps", [(8, 2, (32, 31, 64, 9, 8, 96)), (8, 8, (129, 33)), (16, 1, (160, 40)), (12, 6, (127, 128, 1)), (20, 4, (40, 60))])
+def test_attention_of_many_tokens_over_values_of_different_size(n_head, n_kv, steps):
+    """Steps on both sides of the line from which attention runs on split f16 operands (32 tokens, or 128 keys), with 4, 1,
+    16, 2 and 5 query heads a KV head (the last on the general kernel), part tiles of keys and tokens.  Every third token's
+    values are some 200 times the others', and the first 40 tokens hold none of those: the value tiles' scales differ."""
+    cfg = dict(CFG, n_ctx=256, n_layer=2, head_dim=128, n_head=n_head, n_kv_head=n_kv, hidden=256, vocab=600)
+    rng = np.random.default_rng(n_head)
+    wide = rng.normal(size=(600, 256)) * np.where(np.arange(256) < 32, 1e-3, 1.0)
+    wide[400:, :32] = rng.normal(size=(200, 32)) * 3.0                   # tokens 400 .. carry the first 32 columns
+    over = {"token_embd.weight": (capi.Q8_0, synth.quantize(capi.Q8_0, wide.astype(np.float32)))}
+    for i in range(2):
+        v = rng.normal(size=(n_kv * 128, 256)) / 16.0 * np.where(np.arange(256) < 32, 100.0, 0.5)
+        over[f"blk.{i}.attn_v.weight"] = (capi.Q8_0, synth.quantize(capi.Q8_0, v.astype(np.float32)))
+    m, o = make(cfg, 51, override=over)
+    pos = 0
+    for n in steps:
+        t = np.arange(pos, pos + n)
+        toks = np.where((t >= 40) & (t % 3 == 0), rng.integers(400, 600, size=n), rng.integers(0, 400, size=n))
+        ok, e = close(m.forward(toks, pos), o.forward([int(x) for x in toks], pos))
+        assert ok, f"pos {pos} +{n}: {e}"
+        pos += n
 
 
 @pytest.mark.parametrize("head_dim,n_head,n_kv", [(64, 4, 2), (128, 4, 1), (256, 2, 2), (192, 4, 2), (128, 8, 1),
