@@ -538,6 +538,7 @@ static __global__ __launch_bounds__(GROUP_PAIRS_THREADS) void moe_group_pairs_ra
     int *start = hist + chunks * E;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     constexpr int WAVES = GROUP_PAIRS_THREADS / 64;
+    const int bits = 32 - __builtin_clz((uint32_t)E);  // (the highest number, E - 1, is not all ones in them: 0xFFFFFFFF is)
     for (int i = threadIdx.x; i < chunks * E; i += GROUP_PAIRS_THREADS) hist[i] = 0;
     __syncthreads();
     uint32_t mine[GROUP_RANK_PER_WAVE];
@@ -548,22 +549,29 @@ static __global__ __launch_bounds__(GROUP_PAIRS_THREADS) void moe_group_pairs_ra
         mine[c] = 0xFFFFFFFFu, rank[c] = 0;
         if (chunk >= chunks) continue;  // the same for the whole wave
         const uint32_t e = pidx < P ? ids[pidx] : 0xFFFFFFFFu;
-        int before = 0, after = 0;
-        for (int j = 0; j < 64; j++) {
-            const bool same = (uint32_t)__shfl((int)e, j, 64) == e;
-            before += same && j < lane;
-            after += same && j > lane;
+        // the lanes that name this lane's expert: bit by bit, those that agree on it (a lane past the list agrees with its like only)
+        uint64_t same = ~0ull;
+        for (int b = 0; b < bits; b++) {
+            const uint64_t set = __ballot((e >> b) & 1u);
+            same &= (e >> b) & 1u ? set : ~set;
         }
+        const uint64_t lower = (1ull << lane) - 1;
+        const int before = __popcll(same & lower), after = __popcll(same & ~lower) - 1;
         mine[c] = e, rank[c] = before;
         if (e < (uint32_t)E && after == 0) hist[chunk * E + (int)e] = before + 1;
     }
     __syncthreads();
     for (int e = threadIdx.x; e < E; e += GROUP_PAIRS_THREADS) {  // counts -> counts in earlier chunks; the expert's total
         int run = 0;
-        for (int ch = 0; ch < chunks; ch++) {
-            const int c = hist[ch * E + e];
-            hist[ch * E + e] = run;
-            run += c;
+        for (int c0 = 0; c0 < chunks; c0 += 8) {  // (eight reads at a time: one by one each waits for the one before)
+            int c[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) c[i] = c0 + i < chunks ? hist[(c0 + i) * E + e] : 0;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                if (c0 + i < chunks) hist[(c0 + i) * E + e] = run;
+                run += c[i];
+            }
         }
         start[e] = run;
     }
