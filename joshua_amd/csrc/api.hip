@@ -7,6 +7,7 @@
 #include "kernels_mfma_q4k.hpp"
 #include "kernels_graph.hpp"
 #include "kernels_mla.hpp"
+#include "moe_split16.hpp"
 #include "split16.hpp"
 #include "kernels_mfma_q4k_gemm.hpp"
 #include "kernels_mfma_q4k_stream.hpp"
@@ -1272,6 +1273,17 @@ bool moe_has_gemm_i8(uint32_t type) {
            type == JQ_TYPE_Q5_1;
 }
 
+// Whether a call of T tokens through Q4_K experts runs on split f16 activations (moe_split16): from four pairs an expert on (below,
+// the kernels that keep a pair's activations in registers read less), and where its workgroups of 128 gate and up rows, or of
+// 256 down rows, fill the chip or half of it.  Layer calls, us, before / now: 2048 x 768, 128 experts (8 used), 64 tokens 157 /
+// 156, 100 tokens 199 / 161, 512 tokens 393 / 260, 4096 tokens 1325 / 1216; 4096 x 1536, 64 tokens 693 / 473; 7168 x 2048, 256
+// experts, 512 tokens 3110 / 2568; 1024 x 1024, 32 experts (4 used), 32 tokens 61 / 49.  A down projection of 64
+// workgroups (2048 rows of 8192, 8 experts) is the int8 GEMM's: the layer 205 against 233 at 64 tokens.
+bool moe_split16_pays(const jq_moe_config &c, size_t T) {
+    return T * c.n_expert_used >= 4 * (size_t)c.n_expert && (size_t)c.n_expert * ((c.inter + 127) / 128) >= 256;
+}
+bool moe_split16_down_pays(const jq_moe_config &c) { return (size_t)c.n_expert * ((c.hidden + 255) / 256) >= 128; }
+
 int moe_reserve_quantized(jq_moe *m, size_t T) {
     const jq_moe_config &c = m->cfg;
     const size_t P = T * c.n_expert_used, PR = P + T;
@@ -1284,6 +1296,8 @@ int moe_reserve_quantized(jq_moe *m, size_t T) {
     }
     if (m->gate->type == JQ_TYPE_Q4_K || m->down->type == JQ_TYPE_Q4_K)
         HIP_TRY(hipMalloc((void **)&m->qacts, std::max(T * (c.hidden / 256), PR * (c.inter / 256)) * jq::QS_REC + 16));
+    if (m->gate->type == JQ_TYPE_Q4_K && moe_split16_pays(c, T))
+        HIP_TRY(hipMalloc((void **)&m->split_acts, std::max(moe_split16_bytes(T, c.hidden), moe_split16_bytes(PR, c.inter))));
     if (P > c.n_expert && (moe_has_gemm_i8(m->gate->type) || moe_has_gemm_i8(m->down->type))) {
         // row groups of 16 pairs that never mix two experts: at most PR / 16 + one part-filled group an expert
         m->gtab_rows = PR / 16 + c.n_expert + 2;
@@ -2041,7 +2055,14 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
                              align_of({m->down, m->fold_shared ? m->sdown : nullptr}) >= 16;
     // few pairs an expert, by the cost estimate above: the expert's rows decoded once, its pairs streamed past
     const bool multi = max_group > 1 && expert_dot8;
-    if (same_gu && multi)
+    // Q4_K, four pairs an expert or more: exact products of split f16 activations
+    const bool split16 = max_group > 1 && m->split_acts && m->gate->type == JQ_TYPE_Q4_K && moe_split16_pays(c, T) && !expert_env;
+    if (same_gu && split16 && ((uintptr_t)x & 15) == 0 && moe_split16_takes(c.hidden, m->gate->row_bytes, a16, T))
+        rc = moe_split16({m->pgate, m->pup, m->gate->row_bytes, x, T, m->gexp, m->offsets, m->xrow, m->yrow, groups, (size_t)P + (size_t)extra * T,
+                          m->G, c.hidden, c.inter, clamp, m->split_acts}, s);
+    if (rc > 0) return 1;
+    const bool split_gu = rc == 0;
+    if (rc < 0 && same_gu && multi)
         rc = dispatch_moe_expert_dot8<true>(m->gate->type, m->pgate, m->pup, m->gate->row_bytes, a16, x, T, m->qi8, m->gexp,
                                             m->offsets, m->xrow, m->yrow, m->G, (int)c.hidden, (int)c.inter, groups, s, clamp);
     if (rc > 0) return 1;
@@ -2108,7 +2129,11 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
     }
     const int d16 = align_of({m->down, m->fold_shared ? m->sdown : nullptr});
     rc = -1;
-    if (fused_act && multi)
+    if (split_gu && m->down->type == JQ_TYPE_Q4_K && moe_split16_down_pays(c) && moe_split16_takes(c.inter, m->down->row_bytes, d16, (size_t)P + (size_t)extra * T))
+        rc = moe_split16({m->pdown, nullptr, m->down->row_bytes, m->G, (size_t)P + (size_t)extra * T, m->gexp, m->offsets, m->yrow, m->yrow, groups,
+                          (size_t)P + (size_t)extra * T, m->out, c.inter, c.hidden, clamp, m->split_acts}, s);
+    if (rc > 0) return 1;
+    if (rc < 0 && fused_act && multi)
         rc = dispatch_moe_expert_dot8<false>(m->down->type, m->pdown, nullptr, m->down->row_bytes, d16, m->G,
                                              (size_t)P + extra * T, m->qi8, m->gexp, m->offsets, m->yrow, m->yrow, m->out,
                                              (int)c.inter, (int)c.hidden, groups, s);

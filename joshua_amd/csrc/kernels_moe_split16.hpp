@@ -1,0 +1,316 @@
+// Grouped products of Q4_K experts with some tens of rows each, on the f16 matrix cores without loss of precision.
+//
+// A Q4_K weight is d p - dmin m with p = sc q an integer of at most 945: exact in f16.  An activation, scaled by a power of two
+// that puts its super-block's largest magnitude at 2^13 .. 2^14, is the sum of two f16 numbers hi + lo (22 bits).  So per
+// super-block and output
+//     I1 = sum p (hi + lo)     two v_mfma_f32_16x16x32_f16 a sub-block, products exact, f32 sums
+//     I2 = sum_j m_j XS_j      one more a super-block (XS_j: the sub-block's sum / 32, again hi + lo; the mins exact)
+//     y += s (d I1 - 32 dmin I2)
+// The packed nibbles go from memory to registers and become the second operand there: (w & 0xF) | 0x6400 is 1024 + q as f16, one
+// v_pk_fma_f16 with sc and -1024 sc makes two products (the high nibbles: 0x5400, 64 + q): 1.1 vector instructions a
+// weight, no LDS, and the unpacking of 64 rows serves every activation row of the tile.  (The int8 GEMM's two byte
+// planes of the same product cost four instructions a weight and pass through LDS, and its sums seven an output.)
+//
+// Element order.  Lane (n = lane % 16, g = lane / 16) holds weight row n and, of half a super-block (four sub-blocks, 64
+// bytes), bytes 16 g .. + 15: sub-blocks 2 (g / 2) and 2 (g / 2) + 1, elements 16 (g % 2) .. + 15 of each.  They make four
+// k-steps t = 2 (low / high nibble) + (first / second 8 bytes), in the order 0 2 1 3 4 6 5 7 of a step's eight.  The activation
+// planes are stored in that order, [row][super-block][half][t][plane][g] of 16 bytes, so a fragment is 16 rows' runs of
+// 64 bytes, gathered through the pair list by asynchronous loads into LDS.
+#pragma once
+#include "split16_parts.hpp"
+
+namespace jq {
+
+constexpr int MS16_PLANES = 1024, MS16_XS = 32;  // bytes a row and super-block: hi and lo of 256 elements; of 8 sums
+constexpr int MS16_RG = 3;                        // row groups of 16 a tile holds
+constexpr int MS16_ROWS = 16 * MS16_RG;
+constexpr int MS16_MAX_NB = 32;                   // super-blocks of a row (the scales of a tile wait in LDS)
+// weight rows of a workgroup whose waves take WT tiles of 16 each (DUAL: half of them gate rows, half up rows)
+constexpr int moe_split16_cols(int WT) { return 64 * WT; }
+
+struct MoeSplit16Acts {
+    uint8_t *planes, *xs;
+    float *s;
+};
+
+// grid (ceil(nb / 4), rows), four waves, a wave one (row, super-block).  Row r is X[sel ? sel[r] : r].  A super-block that
+// holds an inf or a NaN gets the scale NaN (and the row's result is NaN).
+static __global__ __launch_bounds__(256) void moe_split16_prep(const float *__restrict__ X, int k, MoeSplit16Acts a) {
+    const int lane = threadIdx.x & 63, nb = k / 256, sb = 4 * (int)blockIdx.x + (threadIdx.x >> 6), row = blockIdx.y;
+    if (sb >= nb) return;
+    const float4 v = *(const float4 *)(X + (size_t)row * k + 256 * sb + 4 * lane);
+    const uint32_t big = max(max(s16_abs(v.x), s16_abs(v.y)), max(s16_abs(v.z), s16_abs(v.w)));
+    uint32_t m = big;
+#pragma unroll
+    for (int off = 32; off; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
+    const bool finite = m < 0x7F800000u;
+    const int e = s16_exponent(m);
+    const float f = finite ? s16_pow2(e) : 0.0f;
+    // (order 0 2 1 3 of the lane's four)
+    const float x[4] = {finite ? v.x * f : 0.0f, finite ? v.z * f : 0.0f, finite ? v.y * f : 0.0f, finite ? v.w * f : 0.0f};
+    _Float16 hi[4], lo[4];
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        hi[i] = (_Float16)x[i];
+        lo[i] = (_Float16)(x[i] - (float)hi[i]);
+        sum += x[i];
+    }
+    const int j = lane >> 3, pos = 4 * (lane & 7);  // sub-block, element in it
+    const int hs = j >> 2, g = 2 * ((j >> 1) & 1) + (pos >> 4), t = 2 * (j & 1) + ((pos >> 3) & 1);
+    const size_t rec = (size_t)row * nb + sb;
+    uint8_t *d = a.planes + rec * MS16_PLANES + 512 * hs + 128 * t + 16 * g + 2 * (pos & 4);
+    __builtin_memcpy(__builtin_assume_aligned(d, 8), hi, 8);
+    __builtin_memcpy(__builtin_assume_aligned(d + 64, 8), lo, 8);
+#pragma unroll
+    for (int off = 4; off; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    if ((lane & 7) == 0) {
+        const float xs = sum * 0.03125f;
+        const _Float16 h = (_Float16)xs, l = (_Float16)(xs - (float)h);
+        ((_Float16 *)(a.xs + rec * MS16_XS))[j] = h;
+        ((_Float16 *)(a.xs + rec * MS16_XS))[8 + j] = l;
+    }
+    if (lane == 0) a.s[rec] = finite ? s16_pow2(-e) : __builtin_nanf("");
+}
+
+struct MoeSplit16 {
+    const uint8_t *const *wa, *const *wb;   // expert bases: gate and up, or down
+    size_t row_bytes;
+    MoeSplit16Acts acts;
+    const int *gexp, *offsets, *xsel, *yrow;  // groups' experts, first pairs; a pair's activation row and result row
+    float *Y;
+    int groups, n, nb, cols;                // cols: column blocks of the grid
+    MoeClamp clamp;
+};
+
+// A workgroup of four waves multiplies a tile of up to 48 pairs of one expert with 64 WT weight rows (DUAL: half gate rows, half
+// the up rows of the same columns, the gated unit in the epilogue); a wave owns WT tiles of 16 rows, RG row groups of 16 pairs.
+// Bound: the issue of matrix and vector instructions, which hardly overlap (a wave of WT = 4 and RG = 3 issues 204 MFMAs of 16 cycles
+// and ~560 vector instructions of 4 a super-block: that alone is 84 of gate and up's 141 us at 128 experts of 768 x 2048 and 512
+// tokens, the rest workgroups that do not divide evenly among the compute units, and their starts); the int8 GEMM took 3 x 102 us for
+// the three products where these take 141 + 68.
+template <bool DUAL, int RG, int WT>
+__device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert, int beg, int cnt, int cb, uint8_t *lds, float *s_lds,
+                                                 int *y_lds) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n16 = lane & 15, g = lane >> 4;
+    constexpr int BUF = RG * 8 * S16_FRAG;
+    constexpr int WD = DUAL ? WT / 2 : WT;  // tiles, and distinct columns' tiles
+    const int nb = a.nb, c0 = (4 * cb + wave) * 16 * WD;
+    if (tid < MS16_ROWS) y_lds[tid] = a.yrow[beg + min(tid, cnt - 1)];
+    // the scales of the tile's rows, [super-block][row]
+    for (int i = tid; i < 16 * RG * nb; i += 256) {
+        const int row = i % (16 * RG), sb = i / (16 * RG);
+        s_lds[i] = a.acts.s[(size_t)a.xsel[beg + min(row, cnt - 1)] * nb + sb];
+    }
+    uint32_t av[RG];          // this lane's share of a fragment: row n16 of each row group, 16-byte run g
+    const uint8_t *xsp[RG];   // and of the sums' operand (lane groups 2 and 3 meet zero mins)
+#pragma unroll
+    for (int r = 0; r < RG; r++) {
+        const uint32_t rec = (uint32_t)a.xsel[beg + min(16 * r + n16, cnt - 1)] * (uint32_t)nb;
+        av[r] = rec * MS16_PLANES + 16u * g;
+        xsp[r] = a.acts.xs + (size_t)rec * MS16_XS + 16 * (g & 1);
+    }
+    const uint8_t *wp[WT];
+#pragma unroll
+    for (int w = 0; w < WT; w++) {
+        const int row = c0 + 16 * (w % WD);
+        wp[w] = (w >= WD ? a.wb : a.wa)[expert] + (size_t)min(row + n16, a.n - 1) * a.row_bytes;
+    }
+    const uint32_t lds0 = s16_lds_offset(lds);
+    // wave w brings k-step w of a half: both planes of every row group
+    auto issue = [&](int sb, int hs) __attribute__((always_inline)) {
+        const uint8_t *base = a.acts.planes + (size_t)sb * MS16_PLANES + 512 * hs + 128 * wave;
+#pragma unroll
+        for (int r = 0; r < RG; r++)
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + hs * BUF + ((r * 4 + wave) * 2 + p) * S16_FRAG);
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(av[r]), "s"(base + 64 * p), "s"(dst) : "memory");
+            }
+    };
+    uint4 hdr[WT], hdrn[WT], q0[WT], q1[WT];
+    auto fetch = [&](int sb, int hs, uint4 (&q)[WT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int w = 0; w < WT; w++) q[w] = *(const uint4 *)(wp[w] + (size_t)sb * 144 + 16 + 64 * hs + 16 * g);
+    };
+    s16_f4 acc[WT][RG], i1[WT][RG];
+    const s16_f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < WT; w++)
+#pragma unroll
+        for (int r = 0; r < RG; r++) acc[w][r] = i1[w][r] = zero;
+    // (masks and magic numbers in registers: v_and_or_b32 takes one scalar operand and no two literals)
+    uint32_t m_lo = 0x000F000Fu, m_hi = 0x00F000F0u, o_lo = 0x64006400u, o_hi = 0x54005400u;
+    asm("" : "+s"(m_lo), "+s"(m_hi), "+v"(o_lo), "+v"(o_hi));
+    // byte selectors: scale 2 (g / 2) + nibble of the half's four into both f16 of a register, each under 0x64
+    const uint32_t sel0 = 0x04000400u + 0x00010001u * (uint32_t)(2 * (g >> 1)), sel1 = sel0 + 0x00010001u;
+    auto multiply = [&](const uint4 (&q)[WT], const uint32_t (&sc4)[WT], const uint8_t *l) __attribute__((always_inline)) {
+#pragma unroll
+        for (int nib = 0; nib < 2; nib++) {
+            s16_h8 b[2][WT];
+#pragma unroll
+            for (int w = 0; w < WT; w++) {
+                const s16_h2 k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
+                const s16_h2 sc = __builtin_bit_cast(s16_h2, __builtin_amdgcn_perm(0x64646464u, sc4[w], nib ? sel1 : sel0)) - k1024;
+                const s16_h2 off = sc * (nib ? (_Float16)-64.0f : (_Float16)-1024.0f);
+                const uint32_t words[4] = {q[w].x, q[w].y, q[w].z, q[w].w};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t even = words[i], odd = words[i] >> 8;
+                    const uint32_t e = nib ? (even & m_hi) | o_hi : (even & m_lo) | o_lo;
+                    const uint32_t o = nib ? (odd & m_hi) | o_hi : (odd & m_lo) | o_lo;
+                    const s16_h2 pe = __builtin_elementwise_fma(__builtin_bit_cast(s16_h2, e), sc, off);
+                    const s16_h2 po = __builtin_elementwise_fma(__builtin_bit_cast(s16_h2, o), sc, off);
+                    b[i >> 1][w][4 * (i & 1)] = pe[0], b[i >> 1][w][4 * (i & 1) + 1] = pe[1];
+                    b[i >> 1][w][4 * (i & 1) + 2] = po[0], b[i >> 1][w][4 * (i & 1) + 3] = po[1];
+                }
+            }
+#pragma unroll
+            for (int s8 = 0; s8 < 2; s8++)
+#pragma unroll
+                for (int p = 0; p < 2; p++)
+#pragma unroll
+                    for (int r = 0; r < RG; r++) {
+                        const s16_h8 x = *(const s16_h8 *)(l + ((r * 4 + 2 * nib + s8) * 2 + p) * S16_FRAG);
+#pragma unroll
+                        for (int w = 0; w < WT; w++) i1[w][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, b[s8][w], i1[w][r], 0, 0, 0);
+                    }
+        }
+    };
+    // the compiler waits for its own loads where their registers are first read: here, behind the wait for everything, and
+    // not behind the asynchronous loads issued next, which it would then wait for too
+    auto landed = [&](uint4 (&q)[WT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int w = 0; w < WT; w++) asm volatile("" : "+v"(q[w].x), "+v"(q[w].y), "+v"(q[w].z), "+v"(q[w].w));
+    };
+    issue(0, 0);
+#pragma unroll
+    for (int w = 0; w < WT; w++) hdr[w] = *(const uint4 *)wp[w];
+    fetch(0, 0, q0);
+    const uint32_t live = g < 2 ? 0xFFFFFFFFu : 0u;
+    for (int sb = 0; sb < nb; sb++) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        landed(q0), landed(hdr);
+        __syncthreads();  // the half has landed, and the other buffer's readers are done
+        issue(sb, 1);
+        fetch(sb, 1, q1);
+        s16_h8 xs[RG];
+#pragma unroll
+        for (int r = 0; r < RG; r++) xs[r] = *(const s16_h8 *)(xsp[r] + (size_t)sb * MS16_XS);
+        uint32_t sc4[WT];
+#pragma unroll
+        for (int w = 0; w < WT; w++) sc4[w] = hdr[w].y & 0x3F3F3F3Fu;
+        multiply(q0, sc4, lds + 16 * lane);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        landed(q1);
+#pragma unroll
+        for (int r = 0; r < RG; r++) asm volatile("" : "+v"(xs[r]));
+        __syncthreads();
+        const int next = min(sb + 1, nb - 1);
+        if (sb + 1 < nb) issue(sb + 1, 0);
+        fetch(next, 0, q0);
+#pragma unroll
+        for (int w = 0; w < WT; w++) {
+            hdrn[w] = *(const uint4 *)(wp[w] + (size_t)next * 144);
+            sc4[w] = (hdr[w].w & 0x0F0F0F0Fu) | ((hdr[w].y >> 2) & 0x30303030u);
+        }
+        multiply(q1, sc4, lds + BUF + 16 * lane);
+        // the min term, and the super-block's sums onto the results
+        s16_f4 s[RG];
+#pragma unroll
+        for (int r = 0; r < RG; r++) s[r] = *(const s16_f4 *)(s_lds + sb * 16 * RG + 16 * r + 4 * g);
+#pragma unroll
+        for (int w = 0; w < WT; w++) {
+            const uint32_t mn[2] = {hdr[w].z & 0x3F3F3F3Fu, ((hdr[w].w >> 4) & 0x0F0F0F0Fu) | ((hdr[w].z >> 2) & 0x30303030u)};
+            s16_h8 mins;
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                const s16_h2 k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
+                const uint32_t pair = __builtin_amdgcn_perm(0x64646464u, mn[j >> 2], j & 2 ? 0x04030402u : 0x04010400u);
+                const s16_h2 m = __builtin_bit_cast(s16_h2, __builtin_bit_cast(uint32_t, __builtin_bit_cast(s16_h2, pair) - k1024) & live);
+                mins[j] = m[0], mins[j + 1] = m[1];
+            }
+            const float d = f16_bits(hdr[w].x), dm = -32.0f * f16_bits(hdr[w].x >> 16);
+#pragma unroll
+            for (int r = 0; r < RG; r++) {
+                const s16_f4 i2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xs[r], mins, zero, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[w][r][i] = fmaf(s[r][i], fmaf(dm, i2[i], d * i1[w][r][i]), acc[w][r][i]);
+                i1[w][r] = zero;
+            }
+            hdr[w] = hdrn[w];
+        }
+    }
+    // every result first, then the stores one behind the other: a load or a branch between them would wait for each
+    const float limit = DUAL ? (expert >= a.clamp.n_routed ? a.clamp.shared : a.clamp.routed) : 0.0f;
+    const float top = limit > 0.0f ? limit : INFINITY;
+#pragma unroll
+    for (int r = 0; r < RG; r++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if constexpr (DUAL) {
+#pragma unroll
+                for (int w = 0; w < WD; w++) {
+                    float gt = acc[w][r][i], up = acc[(w + WD) % WT][r][i];
+                    gt = gt > top ? top : gt;
+                    up = up > top ? top : (up < -top ? -top : up);  // (comparisons: a NaN stays a NaN)
+                    acc[w][r][i] = silu(gt) * up;
+                }
+            }
+    int yr[RG][4];
+#pragma unroll
+    for (int r = 0; r < RG; r++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) yr[r][i] = y_lds[16 * r + 4 * g + i];
+#pragma unroll
+    for (int r = 0; r < RG; r++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float *y = a.Y + (size_t)yr[r][i] * a.n + c0 + n16;
+#pragma unroll
+            for (int w = 0; w < WD; w++)
+                if (16 * r + 4 * g + i < cnt && c0 + 16 * w + n16 < a.n) y[16 * w] = acc[w][r][i];
+        }
+}
+
+// grid: cols x tiles (a multiple of 8; an upper bound, the rest leaves at once), ids 8 apart (one XCD) holding the column
+// blocks of one tile, which read the same activation planes.
+inline int moe_split16_lds(int nb) { return 2 * MS16_RG * 8 * S16_FRAG + 4 * MS16_ROWS * (nb + 1); }
+
+template <bool DUAL, int WT>
+static __global__ __launch_bounds__(256, WT == 2 ? 3 : 2) void moe_split16(MoeSplit16 a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // two buffers of a half, the scales, the result rows
+    float *s_lds = (float *)(lds + 2 * MS16_RG * 8 * S16_FRAG);
+    int *y_lds = (int *)(s_lds + MS16_ROWS * a.nb);
+    const int id = blockIdx.x, lane = threadIdx.x & 63, mt = id / (8 * a.cols) * 8 + id % 8, cb = id / 8 % a.cols;
+    // which group tile mt belongs to: lane l counts the tiles of a run of groups
+    const int per = (a.groups + 63) / 64;
+    int local = 0;
+    for (int i = 0; i < per; i++) {
+        const int e = lane * per + i;
+        if (e < a.groups) local += (a.offsets[e + 1] - a.offsets[e] + MS16_ROWS - 1) / MS16_ROWS;
+    }
+    int incl = local;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += v;
+    }
+    if (mt >= __builtin_amdgcn_readlane(incl, 63)) return;  // past the last tile: the whole workgroup
+    int found = -1, first = incl - local;
+    if (mt >= first && mt < incl) {
+        for (int i = 0; i < per; i++) {
+            const int e = lane * per + i, t = e < a.groups ? (a.offsets[e + 1] - a.offsets[e] + MS16_ROWS - 1) / MS16_ROWS : 0;
+            if (found < 0 && mt < first + t) found = e;
+            else if (found < 0) first += t;
+        }
+    }
+    const int owner = __builtin_ctzll(__ballot(found >= 0));
+    const int grp = __builtin_amdgcn_readlane(found, owner), at = (mt - __builtin_amdgcn_readlane(first, owner)) * MS16_ROWS;
+    const int beg = a.offsets[grp] + at, cnt = min(a.offsets[grp + 1] - beg, MS16_ROWS), expert = a.gexp[grp];
+    if (cnt <= 16) moe_split16_tile<DUAL, 1, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds);
+    else if (cnt <= 32) moe_split16_tile<DUAL, 2, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds);
+    else moe_split16_tile<DUAL, 3, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds);
+}
+
+}  // namespace jq

@@ -17,46 +17,13 @@
 // and 9 of preparation.  Against 64-bit results the errors of both are the same (1.0e-4 and 1.5e-4 of the norm, the 16-bit
 // activations of the products around them).
 #pragma once
-#include "kernels_graph.hpp"
+#include "split16_parts.hpp"
 
 namespace jq {
 
-typedef _Float16 s16_h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 s16_h2 __attribute__((ext_vector_type(2)));
-typedef float s16_f2 __attribute__((ext_vector_type(2)));
-typedef float s16_f16 __attribute__((ext_vector_type(16)));
-
 constexpr int S16_TILE = 32;                         // keys (or tokens) of a tile
-constexpr int S16_FRAG = 1024;                       // bytes of a fragment
 constexpr int S16_KV_TILE = 2 * 8 * 2 * S16_FRAG;    // a head's K (128) and V (128) of a tile: 8 fragments each, two planes
 constexpr int S16_ROPE_TILE = 4 * 2 * S16_FRAG;      // the shared rope keys (64) of a tile
-
-// Asynchronous global -> LDS copy of 16 bytes a lane, the wave's landing one behind the other at lds_base (wave-uniform); awaited
-// by hand with s_waitcnt vmcnt.
-__device__ __forceinline__ uint32_t s16_lds_offset(const void *p) {
-    return (uint32_t)(uintptr_t)((__attribute__((address_space(3))) const void *)p);
-}
-__device__ __forceinline__ void s16_copy16(const void *gptr, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(__builtin_amdgcn_readfirstlane(lds_base)) : "memory");
-}
-
-__device__ __forceinline__ void s16_split(const float (&x)[8], s16_h8 &hi, s16_h8 &lo) {
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-        const s16_h2 h = __builtin_convertvector(s16_f2{x[i], x[i + 1]}, s16_h2);
-        const s16_h2 l = __builtin_convertvector(s16_f2{x[i] - (float)h[0], x[i + 1] - (float)h[1]}, s16_h2);
-        hi[i] = h[0], hi[i + 1] = h[1], lo[i] = l[0], lo[i + 1] = l[1];
-    }
-}
-
-// The exponent s that puts magnitudes up to `amax` (as float bits, sign cleared) below 2^14; zero, tiny, infinite and NaN
-// maxima are held within +-100, so that no power of two below over- or underflows.
-__device__ __forceinline__ int s16_exponent(uint32_t amax_bits) {
-    const int e = min(max((int)(amax_bits >> 23), 40), 240);
-    return 13 - (e - 127);
-}
-__device__ __forceinline__ float s16_pow2(int s) { return __builtin_bit_cast(float, (uint32_t)(127 + s) << 23); }
-__device__ __forceinline__ uint32_t s16_abs(float x) { return __builtin_bit_cast(uint32_t, x) & 0x7FFFFFFFu; }
 
 __device__ __forceinline__ uint32_t s16_block_max(uint32_t v, uint32_t *red) {  // 256 threads
 #pragma unroll
@@ -395,17 +362,24 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
     float vref = LATENT ? a.inv[2 * head + 1].y : s16_pow2(-113);  // the scale the outputs are held in: the largest inv.y so far
     const float khead = LATENT ? a.inv[2 * head].y : 1.0f;
 
-    issue(0, 0);
-    for (int tile = 0; tile < n_tiles; tile++) {
-        float kinv = khead, vinv = vref, tinv = 0.0f;
+    // the tile's scales, asked for with the tile
+    float kinv = khead, vinv = vref, tinv = 0.0f;
+    auto scales = [&](int tile) __attribute__((always_inline)) {
         if constexpr (LATENT) tinv = a.ropeinv[tile];
         else {
             const float2 v = a.inv[(size_t)kvh * a.n_tiles + tile];
             kinv = v.x, vinv = v.y;
         }
+    };
+    issue(0, 0);
+    scales(0);
+    for (int tile = 0; tile < n_tiles; tile++) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // (the compiler waits for the scales where they are first read: here, and not behind the loads issued next)
+        asm volatile("" : "+v"(kinv), "+v"(vinv), "+v"(tinv));
+        const float k_now = kinv, v_now = vinv, t_now = tinv;
         __syncthreads();  // the tile has landed, and the other buffer's readers are done
-        if (tile + 1 < n_tiles) issue(tile + 1, (tile + 1) & 1);
+        if (tile + 1 < n_tiles) issue(tile + 1, (tile + 1) & 1), scales(tile + 1);
         if (idle || tile * S16_TILE > mine) continue;  // (the whole wave; the barrier above is met all the same)
         const uint8_t *l = lds + (tile & 1) * STAGE + 16 * lane;
         s16_f16 sc;
@@ -419,7 +393,7 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
                 sc = s16_mma(kh, ql[s], sc);
                 sc = s16_mma(kl, qh[s], sc);
             }
-            const float to_head = (rinv * tinv) / (qinv * kinv);  // (powers of two)
+            const float to_head = (rinv * t_now) / (qinv * k_now);  // (powers of two)
 #pragma unroll
             for (int r = 0; r < 16; r++) sc[r] *= to_head;
         }
@@ -430,7 +404,7 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
             sc = s16_mma(kh, ql[KR + s], sc);
             sc = s16_mma(kl, qh[KR + s], sc);
         }
-        const float f = qinv * kinv * a.scale_log2e;
+        const float f = qinv * k_now * a.scale_log2e;
         const bool edge = tile * S16_TILE + 31 > a.pos0 + tw;  // some query of the wave does not see the whole tile
         float tmax = -INFINITY;
         if (edge) {
@@ -442,7 +416,7 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
         for (int r = 0; r < 16; r++) tmax = fmaxf(tmax, sc[r]);
         tmax = max_xor32(tmax) * f;
         const float mnew = fmaxf(m_run, tmax);  // finite from tile 0 on, whose first key every query sees
-        const float vnew = fmaxf(vref, vinv);
+        const float vnew = LATENT ? vref : fmaxf(vref, v_now);
         float keep = __builtin_amdgcn_exp2f(m_run - mnew);
         l_run *= keep;
         keep *= vref / vnew;
@@ -454,7 +428,7 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
         }
         m_run = mnew, vref = vnew;
         // weights times 2^10 (and the tile's share of vref, both powers of two): the small ones keep their bits in f16
-        const float up = LATENT ? 1.0f : vinv / vnew;
+        const float up = LATENT ? 1.0f : v_now / vnew;
         s16_h8 ph[2], pl[2];
         float psum = 0.0f;
 #pragma unroll

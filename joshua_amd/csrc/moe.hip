@@ -13,10 +13,10 @@ static void moe_free_scratch(jq_moe *m) {
     for (void *p : {(void *)m->logits, (void *)m->wts, (void *)m->G, (void *)m->U, (void *)m->out, (void *)m->sG,
                     (void *)m->sU, (void *)m->sH, (void *)m->sOut, (void *)m->ids, (void *)m->gexp,
                     (void *)m->offsets, (void *)m->xrow, (void *)m->yrow, (void *)m->qacts, (void *)m->qi8.xl,
-                    (void *)m->qi8.xh, (void *)m->qi8.sx, (void *)m->qi8.sxs, (void *)m->gacts, (void *)m->gtab, (void *)m->group_counts, (void *)m->sgate_logit})
+                    (void *)m->qi8.xh, (void *)m->qi8.sx, (void *)m->qi8.sxs, (void *)m->gacts, (void *)m->gtab, (void *)m->split_acts, (void *)m->group_counts, (void *)m->sgate_logit})
         if (p) (void)hipFree(p);
     if (m->backend && m->backend->release) m->backend->release(m);
-    m->qacts = nullptr;
+    m->qacts = m->split_acts = nullptr;
     m->group_counts = nullptr, m->sgate_logit = nullptr;
     m->gacts = nullptr, m->gtab = nullptr, m->gtab_rows = 0;
     m->qi8 = jq::ActsI8{nullptr, nullptr, nullptr, nullptr};
@@ -190,7 +190,7 @@ void moe_swap_scratch(jq_moe *a, jq_moe *b) {
     std::swap(a->out, b->out), std::swap(a->sG, b->sG), std::swap(a->sU, b->sU), std::swap(a->sH, b->sH);
     std::swap(a->sOut, b->sOut), std::swap(a->ids, b->ids), std::swap(a->gexp, b->gexp);
     std::swap(a->offsets, b->offsets), std::swap(a->xrow, b->xrow), std::swap(a->yrow, b->yrow);
-    std::swap(a->qacts, b->qacts), std::swap(a->gacts, b->gacts), std::swap(a->gtab, b->gtab);
+    std::swap(a->qacts, b->qacts), std::swap(a->gacts, b->gacts), std::swap(a->split_acts, b->split_acts), std::swap(a->gtab, b->gtab);
     std::swap(a->dense_x, b->dense_x), std::swap(a->dense_act, b->dense_act), std::swap(a->group_counts, b->group_counts);
     std::swap(a->dense_sact, b->dense_sact), std::swap(a->sgate_logit, b->sgate_logit);
     std::swap(a->gtab_rows, b->gtab_rows), std::swap(a->gtile_rgs, b->gtile_rgs), std::swap(a->qi8, b->qi8);

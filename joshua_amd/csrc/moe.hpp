@@ -43,6 +43,7 @@ struct jq_moe {
     uint32_t *ids = nullptr;
     int *gexp = nullptr, *offsets = nullptr, *xrow = nullptr, *yrow = nullptr;
     uint8_t *qacts = nullptr;  // activations as MFMA operand records (Q4_K experts, grouped path)
+    uint8_t *split_acts = nullptr;  // activations as f16 planes (Q4_K experts, moe_split16)
     uint8_t *gacts = nullptr;  // activations of the grouped int8 GEMM, and its tables
     int *gtab = nullptr;
     size_t gtab_rows = 0;      // row groups (and tiles) the tables hold

@@ -1,0 +1,25 @@
+// Grouped products of Q4_K experts on split f16 activations (kernels_moe_split16.hpp).
+#pragma once
+#include "core.hpp"
+#include "kernels_valu.hpp"
+
+namespace jqh {
+
+struct MoeSplit16Call {
+    const uint8_t *const *wa, *const *wb;   // device tables of expert bases: gate and up, or down and null
+    size_t row_bytes;
+    const float *X;                         // x_rows rows of k
+    size_t x_rows;
+    const int *gexp, *offsets, *xsel, *yrow;
+    int groups;
+    size_t pairs;
+    float *Y;                               // rows of n; with wb the gated unit's activations
+    size_t k, n;
+    jq::MoeClamp clamp;
+    uint8_t *acts;                          // moe_split16_bytes(x_rows, k)
+};
+size_t moe_split16_bytes(size_t rows, size_t k);
+bool moe_split16_takes(size_t k, size_t row_bytes, int base_align, size_t rows);
+int moe_split16(const MoeSplit16Call &c, hipStream_t s);
+
+}  // namespace jqh

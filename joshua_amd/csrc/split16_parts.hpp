@@ -1,0 +1,43 @@
+// f32 factors as two f16 numbers, hi = f16(x) and lo = f16(x - hi), behind a power of two that fits f16's range: what the
+// kernels on split f16 operands share.
+#pragma once
+#include "kernels_graph.hpp"
+
+namespace jq {
+
+typedef _Float16 s16_h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 s16_h2 __attribute__((ext_vector_type(2)));
+typedef float s16_f2 __attribute__((ext_vector_type(2)));
+typedef float s16_f4 __attribute__((ext_vector_type(4)));
+typedef float s16_f16 __attribute__((ext_vector_type(16)));
+
+constexpr int S16_FRAG = 1024;  // bytes of a fragment: 64 lanes x 8 elements
+
+// Asynchronous global -> LDS copy of 16 bytes a lane, the wave's landing one behind the other at lds_base (wave-uniform); awaited
+// by hand with s_waitcnt vmcnt.
+__device__ __forceinline__ uint32_t s16_lds_offset(const void *p) {
+    return (uint32_t)(uintptr_t)((__attribute__((address_space(3))) const void *)p);
+}
+__device__ __forceinline__ void s16_copy16(const void *gptr, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(__builtin_amdgcn_readfirstlane(lds_base)) : "memory");
+}
+
+__device__ __forceinline__ void s16_split(const float (&x)[8], s16_h8 &hi, s16_h8 &lo) {
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+        const s16_h2 h = __builtin_convertvector(s16_f2{x[i], x[i + 1]}, s16_h2);
+        const s16_h2 l = __builtin_convertvector(s16_f2{x[i] - (float)h[0], x[i + 1] - (float)h[1]}, s16_h2);
+        hi[i] = h[0], hi[i + 1] = h[1], lo[i] = l[0], lo[i + 1] = l[1];
+    }
+}
+
+// The exponent s that puts magnitudes up to `amax` (as float bits, sign cleared) below 2^14; zero, tiny, infinite and NaN
+// maxima are held within +-100, so that no power of two below over- or underflows.
+__device__ __forceinline__ int s16_exponent(uint32_t amax_bits) {
+    const int e = min(max((int)(amax_bits >> 23), 40), 240);
+    return 13 - (e - 127);
+}
+__device__ __forceinline__ float s16_pow2(int s) { return __builtin_bit_cast(float, (uint32_t)(127 + s) << 23); }
+__device__ __forceinline__ uint32_t s16_abs(float x) { return __builtin_bit_cast(uint32_t, x) & 0x7FFFFFFFu; }
+
+}  // namespace jq

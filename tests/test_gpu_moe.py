@@ -283,6 +283,50 @@ def test_many_tokens_take_the_grouped_int8_gemm(qtype, h, inter, E, k, tokens, s
     assert close(dev.forward(few), ora.forward(few))
 
 
+@pytest.mark.parametrize("h,inter,E,k,tokens,shared_inter,kw", [
+    (256, 256, 128, 4, 128, 0, {}),                                  # one super-block a row; 4 pairs an expert: tiles of one row group
+    (768, 256, 130, 5, 260, 256, dict(gating="sigmoid", swiglu_clamp=0.02, swiglu_clamp_shared=0.01)),  # a folded shared expert of 260 rows: six tiles
+    (512, 512, 64, 6, 400, 0, {}),                                   # 37 pairs an expert: two and three row groups
+    (1024, 1024, 32, 8, 330, 0, dict(weights_scale=2.5)),            # 82 pairs an expert: a whole tile and a part
+    (768, 768, 48, 4, 64, 768, {}),
+])
+def test_q4k_experts_on_split_f16_activations(h, inter, E, k, tokens, shared_inter, kw):
+    """Four pairs an expert and more where the workgroups fill the chip: the products of Q4_K weights are exact and the activations
+    held to 22 bits, so the layer lies within 1e-5 of the oracle's f32 (sums of 256 to 1024 f32 terms in another order)."""
+    ora, dev = build(capi.Q4_K, h, inter, E, k, 500 + h + E, shared_inter=shared_inter, **kw)
+    x = synth.normal(501 + tokens, (tokens, h)) * np.float32(4.0)
+    x[:, :32] *= np.float32(1e-5)                                     # a sub-block far below its super-block
+    got = dev.forward(x)
+    assert capi.last_kernel() == "moe_split16"
+    want = ora.forward(x)
+    assert np.array_equal(got, dev.forward(x))
+    assert np.abs(got - want).max() <= 1e-5 * max(1.0, np.abs(want).max())
+    few = synth.normal(502, (3, h))                                   # then a decode-sized call on the same layer
+    assert close(dev.forward(few), ora.forward(few))
+
+
+def test_q4k_experts_on_split_f16_activations_uneven_rows_and_non_finite_ones():
+    """300 of 400 tokens route alike (experts with seven tiles, with one, and with none), one token holds a NaN and one an
+    infinity: their rows come out NaN and nobody else's; the same layer with a down projection that the int8 GEMM runs."""
+    ora, dev = build(capi.Q4_K, 512, 256, 128, 4, 611)
+    x = synth.normal(612, (400, 512))
+    x[:300] = x[0] + 0.01 * x[:300]
+    x[7, 100], x[350, 300] = np.nan, np.inf
+    got = dev.forward(x)
+    assert capi.last_kernel() == "moe_split16"
+    bad = np.zeros(400, bool)
+    bad[[7, 350]] = True
+    assert np.all(np.isnan(got[bad])) and np.all(np.isfinite(got[~bad]))
+    want = ora.forward(x[~bad])
+    ids, ref = dev.route(x[~bad])[0], ora.route(x[~bad])[0]
+    same = np.array([set(a) == set(b) for a, b in zip(ids, ref)])     # (near-copies: a tie within rounding may fall otherwise)
+    assert same.mean() > 0.95
+    assert np.abs(got[~bad] - want)[same].max() <= 1e-5 * max(1.0, np.abs(want).max())
+    ora, dev = build(capi.Q4_K, 256, 4096, 8, 2, 613)                 # 8 workgroups of 256 down rows
+    x = synth.normal(614, (64, 256))
+    assert close(dev.forward(x), ora.forward(x)) and capi.last_kernel() != "moe_split16"
+
+
 @pytest.mark.parametrize("qtype", [capi.Q4_K, capi.MXFP4])
 def test_grouped_int8_gemm_with_pairs_that_fall_unevenly(qtype):
     """260 of 300 tokens route alike: two experts get 260 pairs and more (two tiles of 128 and a tail of tiles of 32),
