@@ -1284,6 +1284,22 @@ bool moe_split16_pays(const jq_moe_config &c, size_t T) {
 }
 bool moe_split16_down_pays(const jq_moe_config &c) { return (size_t)c.n_expert * ((c.hidden + 255) / 256) >= 128; }
 
+// Whether a call of T tokens through MXFP4 experts runs bucketed on the matrix cores' own FP4 (moe_mx).  Against one group a
+// pair: where its reading of the experts hit, 0.11 ps a weight, and its launches, 15 us more, are less than 0.16 ps a pair and
+// weight.  Against the other bucketed kernels: up to 96 pairs an expert, where the int8 GEMM's larger tiles draw level.
+// Layer calls, us, before / now: 7168 x 2048, 256 experts (8 used): 2 tokens 118 / 121 (hence three), 4 tokens
+// 218 / 198, 16 tokens 846 / 535, 64 tokens 1953 / 1070, 512 tokens 3911 / 1907; 2048 x 1024, 128 experts: 4 tokens 67 / 66, 8
+// tokens 118 / 62, 64 tokens 338 / 141, 512 tokens 524 / 318, 2048 tokens (128 an expert) 948 / 960; 4096 x 1536, 128 experts:
+// 512 tokens 1361 / 747, 2048 tokens 2306 / 2490 (4 used, 64 an expert: 1872 / 1415); 1024 x 1024, 32 experts (4 used): 8 tokens
+// 36 / 62, 16 tokens 91 / 35; 512 x 1024, 16 experts: 8 tokens 63 / 30.
+size_t moe_mx_upto(const jq_moe_config &c) { return 96 * (size_t)c.n_expert / c.n_expert_used; }
+bool moe_mx_pays(const jq_moe_config &c, size_t T, bool decode_sized) {
+    if (T < 3 || T > moe_mx_upto(c)) return false;
+    if (!decode_sized) return true;
+    const double E = c.n_expert, P = (double)T * c.n_expert_used, hit = E * (1.0 - std::pow(1.0 - 1.0 / E, P));
+    return 0.16 * P > 0.11 * hit + 15e6 / (3.0 * c.hidden * (double)c.inter);
+}
+
 int moe_reserve_quantized(jq_moe *m, size_t T) {
     const jq_moe_config &c = m->cfg;
     const size_t P = T * c.n_expert_used, PR = P + T;
@@ -1298,6 +1314,9 @@ int moe_reserve_quantized(jq_moe *m, size_t T) {
         HIP_TRY(hipMalloc((void **)&m->qacts, std::max(T * (c.hidden / 256), PR * (c.inter / 256)) * jq::QS_REC + 16));
     if (m->gate->type == JQ_TYPE_Q4_K && moe_split16_pays(c, T))
         HIP_TRY(hipMalloc((void **)&m->split_acts, std::max(moe_split16_bytes(T, c.hidden), moe_split16_bytes(PR, c.inter))));
+    const size_t mx_tokens = std::min(T, moe_mx_upto(c));
+    if (m->gate->type == JQ_TYPE_MXFP4 && m->down->type == JQ_TYPE_MXFP4 && mx_tokens >= 3 && c.hidden % 512 == 0 && c.inter % 512 == 0)
+        HIP_TRY(hipMalloc((void **)&m->split_acts, std::max(moe_mx_bytes(mx_tokens, c.hidden), moe_mx_bytes(mx_tokens * (c.n_expert_used + 1), c.inter))));
     if (P > c.n_expert && (moe_has_gemm_i8(m->gate->type) || moe_has_gemm_i8(m->down->type))) {
         // row groups of 16 pairs that never mix two experts: at most PR / 16 + one part-filled group an expert
         m->gtab_rows = PR / 16 + c.n_expert + 2;
@@ -1973,6 +1992,23 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
         decode_sized = by_pairs <= std::min(by_gemm, by_expert) && P <= 16384;
         if (!expert_env) expert_dot8 = by_expert < by_gemm;
     }
+    // What every expert's first byte is a multiple of (a view may start at any whole block, and blocks of 17,
+    // 34, 66, 210 bytes put that anywhere): 16-byte and 4-byte loads into LDS want it, the kernels that read
+    // through registers do not.
+    auto align_of = [](std::initializer_list<const jq_weight *> ws) {
+        uintptr_t bits = 0;
+        for (const jq_weight *w : ws)
+            if (w) bits |= (uintptr_t)w->dev;
+        return (bits & 15) == 0 ? 16 : (bits & 3) == 0 ? 4 : 1;
+    };
+    const int a16 = align_of({m->gate, m->up, m->fold_shared ? m->sgate : nullptr, m->fold_shared ? m->sup : nullptr});
+    const int d16 = align_of({m->down, m->fold_shared ? m->sdown : nullptr});
+    const bool same_gu = m->gate->type == m->up->type && m->gate->row_bytes == m->up->row_bytes;
+    // MXFP4 on the matrix cores' own FP4 (not where a way was asked for)
+    const bool mx = !pct_env && !expert_env && m->split_acts && m->gate->type == JQ_TYPE_MXFP4 && same_gu && moe_mx_pays(c, T, decode_sized) &&
+                    ((uintptr_t)x & 15) == 0 && moe_mx_takes(c.inter, c.hidden, m->gate->row_bytes, a16, T) &&
+                    m->down->type == JQ_TYPE_MXFP4 && moe_mx_takes(c.hidden, c.inter, m->down->row_bytes, d16, (size_t)P + (size_t)extra * T);
+    if (mx) decode_sized = expert_dot8 = false;
     bool planes_ready = false;
     jq::MoeGateIn gate_later{};
     if (decode_sized) {  // one group per pair, written by the gating kernel itself
@@ -2028,18 +2064,7 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
     }
     HIP_TRY(hipGetLastError());
     // silu(gate x) * (up x) of every pair into G, then down over it
-    // What every expert's first byte is a multiple of (a view may start at any whole block, and blocks of 17,
-    // 34, 66, 210 bytes put that anywhere): 16-byte and 4-byte loads into LDS want it, the kernels that read
-    // through registers do not.
-    auto align_of = [](std::initializer_list<const jq_weight *> ws) {
-        uintptr_t bits = 0;
-        for (const jq_weight *w : ws)
-            if (w) bits |= (uintptr_t)w->dev;
-        return (bits & 15) == 0 ? 16 : (bits & 3) == 0 ? 4 : 1;
-    };
-    const int a16 = align_of({m->gate, m->up, m->fold_shared ? m->sgate : nullptr, m->fold_shared ? m->sup : nullptr});
     int rc = -1;
-    const bool same_gu = m->gate->type == m->up->type && m->gate->row_bytes == m->up->row_bytes;
     // few tokens an expert (at most six on average): the int8 kernel that takes four rows an MFMA; more: the
     // f16 ring kernel, which reads a group's weights once for up to 16 rows
     const bool few = (size_t)P <= 6 * (size_t)c.n_expert;
@@ -2051,8 +2076,7 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
     static const char *gemm_from_env = getenv("JQ_MOE_GEMM_FROM_PAIRS_PER_EXPERT");
     const size_t gemm_from = gemm_from_env ? (size_t)atoll(gemm_from_env) : 16;
     const bool prefer_gemm = m->gacts && max_group > 1 && (size_t)P >= gemm_from * (size_t)c.n_expert &&
-                             c.hidden % 256 == 0 && c.inter % 256 == 0 && a16 >= 16 &&
-                             align_of({m->down, m->fold_shared ? m->sdown : nullptr}) >= 16;
+                             c.hidden % 256 == 0 && c.inter % 256 == 0 && a16 >= 16 && d16 >= 16;
     // few pairs an expert, by the cost estimate above: the expert's rows decoded once, its pairs streamed past
     const bool multi = max_group > 1 && expert_dot8;
     // Q4_K, four pairs an expert or more: exact products of split f16 activations
@@ -2060,6 +2084,9 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
     if (same_gu && split16 && ((uintptr_t)x & 15) == 0 && moe_split16_takes(c.hidden, m->gate->row_bytes, a16, T))
         rc = moe_split16({m->pgate, m->pup, m->gate->row_bytes, x, T, m->gexp, m->offsets, m->xrow, m->yrow, groups, (size_t)P + (size_t)extra * T,
                           m->G, c.hidden, c.inter, clamp, m->split_acts}, s);
+    if (mx)
+        rc = moe_mx({m->pgate, m->pup, m->gate->row_bytes, x, T, m->gexp, m->offsets, m->xrow, m->yrow, groups, (size_t)P + (size_t)extra * T,
+                     m->G, c.hidden, c.inter, clamp, m->split_acts}, s);
     if (rc > 0) return 1;
     const bool split_gu = rc == 0;
     if (rc < 0 && same_gu && multi)
@@ -2127,11 +2154,13 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
                                      m->yrow, m->U, (int)c.hidden, (int)c.inter, groups, max_group, s))
             return 1;
     }
-    const int d16 = align_of({m->down, m->fold_shared ? m->sdown : nullptr});
     rc = -1;
     if (split_gu && m->down->type == JQ_TYPE_Q4_K && moe_split16_down_pays(c) && moe_split16_takes(c.inter, m->down->row_bytes, d16, (size_t)P + (size_t)extra * T))
         rc = moe_split16({m->pdown, nullptr, m->down->row_bytes, m->G, (size_t)P + (size_t)extra * T, m->gexp, m->offsets, m->yrow, m->yrow, groups,
                           (size_t)P + (size_t)extra * T, m->out, c.inter, c.hidden, clamp, m->split_acts}, s);
+    if (split_gu && mx)
+        rc = moe_mx({m->pdown, nullptr, m->down->row_bytes, m->G, (size_t)P + (size_t)extra * T, m->gexp, m->offsets, m->yrow, m->yrow, groups,
+                     (size_t)P + (size_t)extra * T, m->out, c.inter, c.hidden, clamp, m->split_acts}, s);
     if (rc > 0) return 1;
     if (rc < 0 && fused_act && multi)
         rc = dispatch_moe_expert_dot8<false>(m->down->type, m->pdown, nullptr, m->down->row_bytes, d16, m->G,

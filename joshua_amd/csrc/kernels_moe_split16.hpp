@@ -33,10 +33,10 @@ struct MoeSplit16Acts {
     float *s;
 };
 
-// grid (ceil(nb / 4), rows), four waves, a wave one (row, super-block).  Row r is X[sel ? sel[r] : r].  A super-block that
+// grid (rows, ceil(nb / 4)), four waves, a wave one (row, super-block).  Row r is X[sel ? sel[r] : r].  A super-block that
 // holds an inf or a NaN gets the scale NaN (and the row's result is NaN).
 static __global__ __launch_bounds__(256) void moe_split16_prep(const float *__restrict__ X, int k, MoeSplit16Acts a) {
-    const int lane = threadIdx.x & 63, nb = k / 256, sb = 4 * (int)blockIdx.x + (threadIdx.x >> 6), row = blockIdx.y;
+    const int lane = threadIdx.x & 63, nb = k / 256, sb = 4 * (int)blockIdx.y + (threadIdx.x >> 6), row = blockIdx.x;
     if (sb >= nb) return;
     const float4 v = *(const float4 *)(X + (size_t)row * k + 256 * sb + 4 * lane);
     const uint32_t big = max(max(s16_abs(v.x), s16_abs(v.y)), max(s16_abs(v.z), s16_abs(v.w)));
@@ -282,31 +282,9 @@ static __global__ __launch_bounds__(256, WT == 2 ? 3 : 2) void moe_split16(MoeSp
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // two buffers of a half, the scales, the result rows
     float *s_lds = (float *)(lds + 2 * MS16_RG * 8 * S16_FRAG);
     int *y_lds = (int *)(s_lds + MS16_ROWS * a.nb);
-    const int id = blockIdx.x, lane = threadIdx.x & 63, mt = id / (8 * a.cols) * 8 + id % 8, cb = id / 8 % a.cols;
-    // which group tile mt belongs to: lane l counts the tiles of a run of groups
-    const int per = (a.groups + 63) / 64;
-    int local = 0;
-    for (int i = 0; i < per; i++) {
-        const int e = lane * per + i;
-        if (e < a.groups) local += (a.offsets[e + 1] - a.offsets[e] + MS16_ROWS - 1) / MS16_ROWS;
-    }
-    int incl = local;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int v = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += v;
-    }
-    if (mt >= __builtin_amdgcn_readlane(incl, 63)) return;  // past the last tile: the whole workgroup
-    int found = -1, first = incl - local;
-    if (mt >= first && mt < incl) {
-        for (int i = 0; i < per; i++) {
-            const int e = lane * per + i, t = e < a.groups ? (a.offsets[e + 1] - a.offsets[e] + MS16_ROWS - 1) / MS16_ROWS : 0;
-            if (found < 0 && mt < first + t) found = e;
-            else if (found < 0) first += t;
-        }
-    }
-    const int owner = __builtin_ctzll(__ballot(found >= 0));
-    const int grp = __builtin_amdgcn_readlane(found, owner), at = (mt - __builtin_amdgcn_readlane(first, owner)) * MS16_ROWS;
+    const int id = blockIdx.x, mt = id / (8 * a.cols) * 8 + id % 8, cb = id / 8 % a.cols;
+    int grp, at;
+    if (!s16_find_tile(a.offsets, a.groups, MS16_ROWS, mt, grp, at)) return;  // past the last tile: the whole workgroup
     const int beg = a.offsets[grp] + at, cnt = min(a.offsets[grp + 1] - beg, MS16_ROWS), expert = a.gexp[grp];
     if (cnt <= 16) moe_split16_tile<DUAL, 1, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds);
     else if (cnt <= 32) moe_split16_tile<DUAL, 2, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds);

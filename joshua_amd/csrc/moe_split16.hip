@@ -1,6 +1,7 @@
-// Host side of the grouped Q4_K products on split f16 activations.
+// Host side of the grouped expert products on exact operands: Q4_K on split f16 activations, MXFP4 on FP4 and FP8 digits.
 #include "moe_split16.hpp"
 
+#include "kernels_moe_mx.hpp"
 #include "kernels_moe_split16.hpp"
 
 namespace jqh {
@@ -30,12 +31,50 @@ int moe_split16(const MoeSplit16Call &c, hipStream_t s) {
     a.cols = (int)((c.n + per - 1) / per);
     const size_t tiles = (c.pairs / jq::MS16_ROWS + (size_t)c.groups + 7) / 8 * 8;
     if (tiles * a.cols > 0x7FFFFFFFull) return -1;
-    hipLaunchKernelGGL(jq::moe_split16_prep, dim3((unsigned)((nb + 3) / 4), (unsigned)c.x_rows), dim3(256), 0, s, c.X, (int)c.k, a.acts);
+    hipLaunchKernelGGL(jq::moe_split16_prep, dim3((unsigned)c.x_rows, (unsigned)((nb + 3) / 4)), dim3(256), 0, s, c.X, (int)c.k, a.acts);
     const int lds = jq::moe_split16_lds((int)nb);
     auto *kernel = c.wb ? (wt == 2 ? jq::moe_split16<true, 2> : jq::moe_split16<true, 4>) : (wt == 2 ? jq::moe_split16<false, 2> : jq::moe_split16<false, 4>);
     hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles * a.cols)), dim3(256), lds, s, a);
     HIP_TRY(hipGetLastError());
     note_kernel("moe_split16");
+    return 0;
+}
+
+size_t moe_mx_bytes(size_t rows, size_t k) { return rows * (k / jq::MX_CHUNK) * (jq::MX_CHUNK_ACTS + 64) + 256; }
+
+bool moe_mx_takes(size_t n, size_t k, size_t row_bytes, int base_align, size_t rows) {
+    return k % jq::MX_CHUNK == 0 && n % 16 == 0 && row_bytes % 16 == 0 && base_align >= 16 && 16 * row_bytes <= 0x7FFFFFFFull &&
+           rows * (k / jq::MX_CHUNK) * jq::MX_CHUNK_ACTS <= 0x7FFFFFFFull;
+}
+
+int moe_mx(const MoeSplit16Call &c, hipStream_t s) {
+    const size_t nc = c.k / jq::MX_CHUNK, recs = c.x_rows * nc;
+    jq::MoeMx a{};
+    a.acts.digits = c.acts;
+    a.acts.scales = (uint32_t *)(c.acts + recs * jq::MX_CHUNK_ACTS);
+    a.wa = c.wa, a.wb = c.wb, a.row_bytes = c.row_bytes;
+    a.gexp = c.gexp, a.offsets = c.offsets, a.xsel = c.xsel, a.yrow = c.yrow;
+    a.Y = c.Y, a.groups = c.groups, a.n = (int)c.n, a.nc = (int)nc, a.clamp = c.clamp;
+    // Tiles of 16 pairs on 8 waves from six pairs an expert on if those workgroups fill the chip twice, else of 8 pairs on 4 waves
+    // (7168 x 2048, 256 experts, the layer, us: 64 tokens 1129 / 1056, 512 tokens 1889 / 2384; 1024 x 1024, 32 experts, 16
+    // pairs each: 103 / 80).
+    const size_t wide = (c.wb ? 16 : 32) * 8;
+    const bool many = c.pairs >= 6 * (size_t)c.groups && (c.pairs / 16 + c.groups) * ((c.n + wide - 1) / wide) >= 512;
+    const int waves = many ? 8 : 4, rows = many ? 16 : 8;
+    const size_t per = (size_t)(c.wb ? 16 : 32) * waves, blocks = (c.n + per - 1) / per;
+    // A workgroup's start is some microseconds of dependent loads: about eight chunks each while two fill a compute unit (the
+    // layer of 256 experts, 64 tokens: 1068 with two blocks of the down projection, 1098 with one; 64 experts of 512, with
+    // eight of them and half a workgroup to a compute unit, 82 against 60 with one).
+    const size_t busy = std::min(c.pairs, c.pairs / rows + (size_t)c.groups) * blocks;
+    a.span = (int)std::max<size_t>(1, std::min({blocks, 8 / nc, busy / 512}));
+    a.cols = (int)((blocks + a.span - 1) / a.span);
+    const size_t tiles = (c.pairs / rows + (size_t)c.groups + 7) / 8 * 8;
+    if (tiles * a.cols > 0x7FFFFFFFull) return -1;
+    hipLaunchKernelGGL(jq::moe_mx_prep, dim3((unsigned)c.x_rows, (unsigned)((nc + 3) / 4)), dim3(256), 0, s, c.X, (int)c.k, a.acts);
+    auto *kernel = c.wb ? (many ? jq::moe_mx<true, 8, 4> : jq::moe_mx<true, 4, 2>) : (many ? jq::moe_mx<false, 8, 4> : jq::moe_mx<false, 4, 2>);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles * a.cols)), dim3(64 * waves), 0, s, a);
+    HIP_TRY(hipGetLastError());
+    note_kernel("moe_expert_dot8");  // (the route: bucketed, an expert's rows read once and its pairs taken past them)
     return 0;
 }
 

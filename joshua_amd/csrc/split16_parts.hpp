@@ -13,6 +13,10 @@ typedef float s16_f16 __attribute__((ext_vector_type(16)));
 
 constexpr int S16_FRAG = 1024;  // bytes of a fragment: 64 lanes x 8 elements
 
+// Weights behind a table of pointers: without the address space the compiler takes their loads for flat ones, which also
+// wait for (and are waited for as) LDS accesses.  (16 bytes, aligned to 4.)
+typedef uint32_t s16_u4 __attribute__((ext_vector_type(4), aligned(4)));
+
 // Asynchronous global -> LDS copy of 16 bytes a lane, the wave's landing one behind the other at lds_base (wave-uniform); awaited
 // by hand with s_waitcnt vmcnt.
 __device__ __forceinline__ uint32_t s16_lds_offset(const void *p) {
@@ -39,5 +43,43 @@ __device__ __forceinline__ int s16_exponent(uint32_t amax_bits) {
 }
 __device__ __forceinline__ float s16_pow2(int s) { return __builtin_bit_cast(float, (uint32_t)(127 + s) << 23); }
 __device__ __forceinline__ uint32_t s16_abs(float x) { return __builtin_bit_cast(uint32_t, x) & 0x7FFFFFFFu; }
+
+// An address that is the same in all lanes, where the compiler does not see that.
+__device__ __forceinline__ const uint8_t *s16_uniform(const uint8_t *p) {
+    const uint64_t v = (uint64_t)p;
+    return (const uint8_t *)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)v) |
+                             (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32);
+}
+
+// Of pairs sorted into groups (offsets [groups + 1]), cut into tiles of `rows` pairs that never mix two groups: which group
+// tile `mt` belongs to and its first pair there.  False past the last tile.  For whole waves; the results are uniform.
+__device__ __forceinline__ bool s16_find_tile(const int *__restrict__ offsets, int groups, int rows, int mt, int &grp, int &at) {
+    // lane l counts the tiles of a run of groups
+    const int lane = threadIdx.x & 63, per = (groups + 63) / 64;
+    int local = 0;
+    for (int i = 0; i < per; i++) {
+        const int e = lane * per + i;
+        if (e < groups) local += (offsets[e + 1] - offsets[e] + rows - 1) / rows;
+    }
+    int incl = local;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += v;
+    }
+    if (mt >= __builtin_amdgcn_readlane(incl, 63)) return false;
+    int found = -1, first = incl - local;
+    if (mt >= first && mt < incl) {
+        for (int i = 0; i < per; i++) {
+            const int e = lane * per + i, t = e < groups ? (offsets[e + 1] - offsets[e] + rows - 1) / rows : 0;
+            if (found < 0 && mt < first + t) found = e;
+            else if (found < 0) first += t;
+        }
+    }
+    const int owner = __builtin_ctzll(__ballot(found >= 0));
+    grp = __builtin_amdgcn_readlane(found, owner);
+    at = (mt - __builtin_amdgcn_readlane(first, owner)) * rows;
+    return true;
+}
 
 }  // namespace jq

@@ -327,6 +327,69 @@ def test_q4k_experts_on_split_f16_activations_uneven_rows_and_non_finite_ones():
     assert close(dev.forward(x), ora.forward(x)) and capi.last_kernel() != "moe_split16"
 
 
+@pytest.mark.parametrize("h,inter,E,k,tokens,shared_inter,kw", [
+    (512, 512, 16, 4, 9, 0, {}),                                                  # one chunk a row; tiles of 8 pairs, most part-filled
+    (1536, 512, 8, 2, 40, 512, dict(swiglu_clamp=0.02, swiglu_clamp_shared=0.01)),  # the shared expert's 40 pairs; limits that bite
+    (1024, 2048, 4, 2, 100, 0, {}),                                               # 50 pairs an expert: tiles of 16 on eight waves in gate and up
+    (4096, 1024, 32, 4, 130, 1024, dict(gating="sigmoid", weights_scale=2.5)),    # tiles of 16 in both, several column blocks a workgroup
+    (512, 1536, 64, 8, 12, 0, {}),                                                # one or two pairs an expert
+])
+def test_mxfp4_experts_on_the_matrix_cores_fp4(h, inter, E, k, tokens, shared_inter, kw):
+    """Bucketed MXFP4 calls on the FP4 matrix instructions: activations in 20 bits of their block's largest magnitude.
+    Against a float64 layer over the exact weights, routed as the device routes: an activation is off by at most 2^-19 of its
+    block's largest, in rms 2^-19 / sqrt 3 of it, and that largest is about 2.2 times the rms of a block of normal values, under
+    6 times that of a block of products: 2.5e-6 through gate and as much through up, 7e-6 through down.  A row within 2^-16 = 1.5e-5
+    of its norm (the 16-bit planes of the other kernels: 5e-5).  Gate values stay below about 0.1, twice the limits of the second
+    case: beyond them most of a clamped sum cancels (this rounding alone, in float64, gives 4.7e-6 there and 1.5e-5 at 0.74)."""
+    rw = synth.normal(900, (E, h), sigma=0.02)
+    parts = [synth.normal_quantized(capi.MXFP4, 901 + i, E * inter * h, 0.02).copy() for i in range(3)]
+    for p in parts:                       # the smallest scale, and blocks that stand for zeros (scale 0xFF)
+        p.reshape(-1, 17)[::37, 0] = 0
+        p.reshape(-1, 17)[5::41, 0] = 0xFF
+    shp = [synth.normal_quantized(capi.MXFP4, 905 + i, shared_inter * h, 0.02) for i in range(3)] if shared_inter else []
+
+    def up(b, n, kk):
+        return capi.Weight.upload(capi.MXFP4, b, n, kk)
+
+    shared = (up(shp[0], shared_inter, h), up(shp[1], shared_inter, h), up(shp[2], h, shared_inter)) if shp else None
+    cfg = capi.MoeConfig(E, k, h, inter, int(kw.get("gating") == "sigmoid"), 1, kw.get("weights_scale", 0.0), 1, 1,
+                         kw.get("swiglu_clamp", 0.0), kw.get("swiglu_clamp_shared", 0.0))
+    dev = capi.Moe(cfg, rw, up(parts[0], E * inter, h), up(parts[1], E * inter, h), up(parts[2], E * h, inter), shared=shared)
+    x = synth.normal(910 + tokens, (tokens, h)) * np.float32(2.0) ** (np.arange(tokens) % 9 - 12)[:, None].astype(np.float32)
+    ids, wts = dev.route(x)
+    got = dev.forward(x)
+    assert capi.last_kernel() == "moe_expert_dot8"
+
+    def deq(b, *shape):
+        return oracle.dequantize(capi.MXFP4, b).reshape(shape).astype(np.float64)
+
+    gw, uw, dw = deq(parts[0], E, inter, h), deq(parts[1], E, inter, h), deq(parts[2], E, h, inter)
+    sh = [deq(shp[0], shared_inter, h), deq(shp[1], shared_inter, h), deq(shp[2], h, shared_inter)] if shp else None
+
+    def ffn(v, a, b, c, limit):
+        gt, upv = a @ v, b @ v
+        if limit:
+            gt, upv = np.minimum(gt, limit), np.clip(upv, -limit, limit)
+        return c @ (gt / (1.0 + np.exp(-gt)) * upv)
+
+    want = np.zeros((tokens, h))
+    for t in range(tokens):
+        v = x[t].astype(np.float64)
+        for s in range(k):
+            e = ids[t, s]
+            want[t] += wts[t, s] * ffn(v, gw[e], uw[e], dw[e], kw.get("swiglu_clamp", 0.0))
+        if shp:
+            want[t] += ffn(v, *sh, kw.get("swiglu_clamp_shared", 0.0))
+    rows = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert rows.max() < 2.0 ** -16, rows.max()
+    # rows that hold an inf or a NaN stay their own
+    bad = x.copy()
+    bad[1, 3], bad[tokens - 1, h - 1] = np.inf, np.nan
+    again = dev.forward(bad)
+    assert np.all(np.isnan(again[tokens - 1])) and not np.any(np.isfinite(again[1]))
+    assert np.array_equal(again[[0] + list(range(2, tokens - 1))], got[[0] + list(range(2, tokens - 1))])
+
+
 @pytest.mark.parametrize("qtype", [capi.Q4_K, capi.MXFP4])
 def test_grouped_int8_gemm_with_pairs_that_fall_unevenly(qtype):
     """260 of 300 tokens route alike: two experts get 260 pairs and more (two tiles of 128 and a tail of tiles of 32),
