@@ -695,14 +695,20 @@ int dispatch_gemm_i8(const uint8_t *W, size_t row_bytes, const float *X, float *
     };
     if (tiles_of(shapes[2]) * std::max<size_t>(1, std::min<size_t>(nb / 4, 8)) < min_tiles) return -1;
     // Estimate per (shape, splits), in us, fitted to whole-call times of Q4_K products of 32 to 2048 rows
-    // against 1024 to 24576 weight rows of 4096 and 12288 columns (the picks are within 5 % of the best
-    // measured choice there; Q6_K runs ~10 % longer with the same ordering): the preparation, a fixed part,
+    // against 1024 to 24576 weight rows of 4096 and 12288 columns (over 180 shapes of Q4_K and Q6_K the picks
+    // are 0.8 % off the best measured choice on average, 16 % at worst; Q6_K runs ~10 % longer with the same ordering): the preparation, a fixed part,
     // the super-blocks a workgroup walks at a cost that grows with the workgroups at work (a large workgroup:
     // 5.0 us a super-block with 74 at work, 6.6 with 256; a small one: 2.5 with 64, 3.0 with 256, 4.7 when two
     // share every compute unit), and the sum's launch and its (splits + 1) m n floats, which the last-level
     // cache holds.
     const size_t acts_bytes = (groups * nb * (size_t)jq::QI_REC + 255) & ~(size_t)255;
     const size_t scratch_cap = tl_fixed_scratch ? tl_fixed_scratch->bytes : (size_t)1 << 40;
+    // whole rounds of workgroups, then what is left at its own cost (a last round of half the workgroups or fewer is short:
+    // 333 x 12288 x 4096 of Q6_K in four parts, 768 workgroups of 128 x 64, 111 us; in three, 576 of them, 137)
+    auto rounds = [](double wgs, double at_once, auto us) {
+        const double whole = std::floor(wgs / at_once), rest = wgs - whole * at_once;
+        return whole * us(at_once) + (rest > 0.0 ? us(rest) : 0.0);
+    };
     auto estimate = [&](const GemmI8Shape &sh, size_t sp) {
         const double wgs = (double)(tiles_of(sh) * sp), nbl = (double)(nb / sp);
         double us = 3.0 + 0.0035 * (double)(nb * groups);
@@ -710,9 +716,8 @@ int dispatch_gemm_i8(const uint8_t *W, size_t row_bytes, const float *X, float *
             us += 3.9 + nbl * (2.95 + 0.0029 * std::min(wgs, 512.0)) *
                             (wgs <= 512.0 ? 1.0 : wgs < 2048.0 ? std::ceil(wgs / 512.0) : wgs / 512.0);
         else if (sh.nw == 8)  // (six groups of weight rows instead of seven: six sevenths of the work a super-block)
-            us += 10.0 + nbl * (4.3 + 0.009 * std::min(wgs, 256.0)) * std::ceil(wgs / 256.0) * (sh.ng == 7 ? 1.0 : 0.88);
-        else if (wgs <= 256.0) us += 3.9 + nbl * (2.3 + 0.0027 * wgs);
-        else us += 3.9 + nbl * (3.1 + 0.0032 * std::min(wgs, 512.0)) * std::max(1.0, wgs / 512.0);
+            us += 10.0 + nbl * rounds(wgs, 256.0, [](double w) { return 4.3 + 0.009 * w; }) * (sh.ng == 7 ? 1.0 : 0.88);
+        else us += 3.9 + nbl * rounds(wgs, 512.0, [](double w) { return w <= 256.0 ? 2.3 + 0.0027 * w : 3.1 + 0.0032 * w; });
         if (sp > 1) us += 1.0 + 0.8 * (double)sp + (double)(sp + 1) * (double)(m * n) * 4.0 / 8.0e6;
         return us;
     };
