@@ -2394,6 +2394,11 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
     const size_t nh = c.n_head, nope = c.qk_nope_head_dim, rope = c.qk_rope_head_dim, vh = c.v_head_dim,
                  lkv = c.kv_lora_rank, qd = nope + rope;
     const float *comp = m->comp;
+    // one token over a Q4_K up-projection of DeepSeek's geometry: its blocks are read (9 MB at V3's size) instead of the
+    // 67 MB of their f32 copy.  128 heads behind 100 tokens, us: absorbing 7.1 / 5.4, merging the splits and multiplying with the value
+    // rows 4.8 + 8.0 / 6.1 in one launch.
+    const bool kv_q4k = S == 1 && m->kv_b && m->kv_b->type == JQ_TYPE_Q4_K && lkv == 512 && nope == 128 && vh % 64 == 0 &&
+                        m->kv_b->row_bytes == 288 && ((uintptr_t)m->kv_b->dev & 15) == 0;
     if (c.q_lora_rank) {
         float *t1 = m->t1;
         if (S == 1 && m->qa_kva) {  // one token: q_a and kv_a as one product over the rows laid end to end
@@ -2415,8 +2420,12 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
     const unsigned st = S == 1 ? 1 : 4;
     static const char *no_absorb_rope = getenv("JQ_MLA_NO_ABSORB_ROPE");
     if (S == 1 && !no_absorb_rope) {
-        // one token: the rotation / latent kernel's work rides in the first wave of the absorption's workgroups
-        if (vec4)
+        // one token: the rotation / latent kernel's work rides in a wave of the absorption's workgroups
+        if (kv_q4k)
+            hipLaunchKernelGGL(jq::mla_absorb_rope_q4k<8>, dim3((unsigned)nh + 1, 2), dim3(512), 0, s, m->qv, (const uint8_t *)m->kv_b->dev,
+                               m->qabs, (int)nh, (int)nope, (int)rope, (int)vh, (int)lkv, comp, (const float *)m->kv_a_norm,
+                               (const float2 *)m->cs, m->lat, m->kpe, (int)pos, c.rms_eps);
+        else if (vec4)
             hipLaunchKernelGGL(jq::mla_absorb_rope<4>, dim3((unsigned)nh + 1), dim3(512), 0, s, m->qv, (const float *)m->wkv, m->qabs,
                                (int)nh, (int)nope, (int)rope, (int)vh, (int)lkv, comp, (const float *)m->kv_a_norm,
                                (const float2 *)m->cs, m->lat, m->kpe, (int)pos, c.rms_eps);
@@ -2478,6 +2487,12 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
                  : G == 2 ? mla_launch_attention<2>(m, S, pos, (unsigned)n_split, s)
                           : mla_launch_attention<1>(m, S, pos, (unsigned)n_split, s);
         if (rc) return rc;
+    }
+    if (kv_q4k) {
+        hipLaunchKernelGGL(jq::mla_merge_vproj_q4k, dim3((unsigned)nh, (unsigned)(vh / 64)), dim3(512), 0, s, (const float *)m->part,
+                           (const uint8_t *)m->kv_b->dev, m->ctx, (int)nope, (int)vh, (int)n_split);
+        HIP_TRY(hipGetLastError());
+        return dispatch_matmul(m->o->type, m->o->dev, m->o->row_bytes, m->ctx, out, S, nh * vh, c.n_embd, s);
     }
     // the absorbed queries are spent: their buffer takes the merged latent sums
     hipLaunchKernelGGL(jq::mla_merge, dim3((unsigned)nh, (unsigned)S, (unsigned)((lkv + 127) / 128)), dim3(128), 0, s, (const float *)m->part, m->qabs, (int)nh,

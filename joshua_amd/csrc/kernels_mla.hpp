@@ -15,6 +15,7 @@
 //                     context split over workgroups (partial maximum, sum and vector per split)
 //   mla_merge         merge the splits into o_lat[h]
 //   mla_vproj         ctx[h] = W_v[h] o_lat[h]
+// (one token over a Q4_K up-projection: mla_absorb_rope_q4k, the attention, mla_merge_vproj_q4k)
 // around the quantized projections (q, kv_a, o), which run on the matmul kernels.
 #pragma once
 #include "kernels_graph.hpp"
@@ -421,6 +422,119 @@ __global__ __launch_bounds__(256) void mla_vproj(const float *__restrict__ olat,
             if (lane == 0 && s0 + t < S) ctx[((size_t)(s0 + t) * n_head + h) * vh + j] = v;
         }
     }
+}
+
+// ---- one token over a Q4_K up-projection: its blocks (288 bytes a row of 512) read instead of the 2 KB of f32 a row --------
+//
+// Lane l of a half-wave holds the same 8 columns of a super-block for every row: the nibbles of word l of its 32, columns
+// 64 c + 4 i .. + 3 (low) and 64 c + 32 + 4 i .. + 3 (high) with c = l / 8, i = l % 8; weights as decoded for the f32 copy,
+// w = d sc q - dmin m, with the offsets' products summed apart.
+struct MlaQ4kWord {
+    float lo[4], hi[4];      // q of the eight
+    float dl, dh, ml, mh;    // d sc and dmin m of the two sub-blocks
+};
+__device__ __forceinline__ MlaQ4kWord mla_q4k_word(const uint4 &hdr, uint32_t q, int c) {
+    MlaQ4kWord w;
+    uint32_t sc, mn;
+    q4k_scale_min_pair(hdr.y, hdr.z, hdr.w, c, sc, mn);
+    const float d = f16_bits(hdr.x), dmin = f16_bits(hdr.x >> 16);
+    w.dl = d * (float)(sc & 0xFFu), w.dh = d * (float)((sc >> 8) & 0xFFu);
+    w.ml = dmin * (float)(mn & 0xFFu), w.mh = dmin * (float)((mn >> 8) & 0xFFu);
+    const uint32_t lo = q & 0x0F0F0F0Fu, hi = (q >> 4) & 0x0F0F0F0Fu;
+#pragma unroll
+    for (int b = 0; b < 4; b++) w.lo[b] = (float)((lo >> (8 * b)) & 0xFFu), w.hi[b] = (float)((hi >> (8 * b)) & 0xFFu);
+    return w;
+}
+
+// mla_absorb_rope over Q4_K blocks: grid (n_head + 1, lkv / 256 super-blocks), 512 threads.  A half-wave takes every 16th of the
+// head's nope rows; their 16 sums meet in LDS.  Bound: latency of the rows' loads, all asked for ahead of the arithmetic.
+// 128 heads of 128 x 512: 5.4 us (the f32 rows, 33.5 MB: 7.1).
+template <int ROWS>  // rows a half-wave, nope / 16
+__global__ __launch_bounds__(512) void mla_absorb_rope_q4k(float *__restrict__ q, const uint8_t *__restrict__ Wkv,
+                                                            float *__restrict__ qabs, int n_head, int nope, int rope, int vh,
+                                                            int lkv, const float *__restrict__ comp, const float *__restrict__ w,
+                                                            const float2 *__restrict__ cs, float *__restrict__ lat,
+                                                            float *__restrict__ kpe, int pos0, float eps) {
+    __shared__ float red[16][256];
+    const int h = blockIdx.x, sb = blockIdx.y, tid = threadIdx.x, half = tid >> 5, l = tid & 31, c = l >> 3, nb = lkv / 256;
+    if (h == n_head) {
+        if (sb == 0 && tid < 64)
+            mla_rope_latent_wave(q, comp, w, cs, lat, kpe, n_head, nope, rope, lkv, pos0, eps, h, 0, tid);
+        return;
+    }
+    const uint8_t *src = Wkv + (((size_t)h * (nope + vh) + half) * nb + sb) * 144;
+    const size_t step = (size_t)16 * nb * 144;
+    uint4 hdr[ROWS];
+    uint32_t qs[ROWS];
+    float x[ROWS];
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) {
+        hdr[i] = *(const uint4 *)(src + i * step);
+        qs[i] = *(const uint32_t *)(src + i * step + 16 + 4 * l);
+        x[i] = q[(size_t)h * (nope + rope) + half + 16 * i];
+    }
+    float lo[4] = {0.0f, 0.0f, 0.0f, 0.0f}, hi[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ml = 0.0f, mh = 0.0f;
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) {
+        const MlaQ4kWord v = mla_q4k_word(hdr[i], qs[i], c);
+        const float a = x[i] * v.dl, b = x[i] * v.dh;
+#pragma unroll
+        for (int e = 0; e < 4; e++) lo[e] = fmaf(a, v.lo[e], lo[e]), hi[e] = fmaf(b, v.hi[e], hi[e]);
+        ml = fmaf(x[i], v.ml, ml), mh = fmaf(x[i], v.mh, mh);
+    }
+    const int at = 64 * c + 4 * (l & 7);
+    *(float4 *)&red[half][at] = float4{lo[0] - ml, lo[1] - ml, lo[2] - ml, lo[3] - ml};
+    *(float4 *)&red[half][at + 32] = float4{hi[0] - mh, hi[1] - mh, hi[2] - mh, hi[3] - mh};
+    __syncthreads();
+    if (tid < 256) {
+        float v = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) v += red[i][tid];
+        qabs[(size_t)h * lkv + 256 * sb + tid] = v;
+    } else if (sb == 0 && tid < 320) {  // (the rope slice of q[h]: nobody reads it here)
+        mla_rope_latent_wave(q, comp, w, cs, lat, kpe, n_head, nope, rope, lkv, pos0, eps, h, 0, tid - 256);
+    }
+}
+
+// mla_merge and mla_vproj of one token in one launch, over Q4_K blocks of 512 columns: grid (n_head, vh / 64), 512 threads.  A
+// workgroup merges the splits of its head (a thread a column), then wave w takes 8 value rows, a lane its 8 columns of either
+// super-block.  128 heads of 128 x 512 behind 100 tokens: 6.1 us (merging 4.8 and the f32 rows 8.0).
+__global__ __launch_bounds__(512) void mla_merge_vproj_q4k(const float *__restrict__ part, const uint8_t *__restrict__ Wkv,
+                                                            float *__restrict__ ctx, int nope, int vh, int n_split) {
+    constexpr int LKV = 512, NB = LKV / 256, ROWS = 8;
+    __shared__ __attribute__((aligned(16))) float ol[LKV];
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, sb = lane >> 5, l = lane & 31, c = l >> 3;
+    const int row0 = 64 * (int)blockIdx.y + ROWS * wave;
+    const uint8_t *src = Wkv + ((((size_t)h * (nope + vh)) + nope + row0) * NB + sb) * 144;
+    uint4 hdr[ROWS];
+    uint32_t qs[ROWS];
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) {
+        hdr[i] = *(const uint4 *)(src + (size_t)i * NB * 144);
+        qs[i] = *(const uint32_t *)(src + (size_t)i * NB * 144 + 16 + 4 * l);
+    }
+    const float *p = part + (size_t)h * n_split * (LKV + 2);
+    const float mi = lane < n_split ? p[(size_t)lane * (LKV + 2)] : -INFINITY;  // n_split <= 64
+    const float M = wave_max(mi);
+    const float fi = mi == -INFINITY ? 0.0f : __expf(mi - M);  // an empty split
+    const float L = wave_sum(lane < n_split ? p[(size_t)lane * (LKV + 2) + 1] * fi : 0.0f);
+    float v = 0.0f;
+#pragma unroll 8
+    for (int i = 0; i < n_split; i++) v = fmaf(p[(size_t)i * (LKV + 2) + 2 + tid], __shfl(fi, i, 64), v);
+    ol[tid] = v * (1.0f / L);
+    __syncthreads();
+    const float4 xl = *(const float4 *)&ol[256 * sb + 64 * c + 4 * (l & 7)], xh = *(const float4 *)&ol[256 * sb + 64 * c + 32 + 4 * (l & 7)];
+    const float sl = (xl.x + xl.y) + (xl.z + xl.w), sh = (xh.x + xh.y) + (xh.z + xh.w);
+    float mine = 0.0f;
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) {
+        const MlaQ4kWord w = mla_q4k_word(hdr[i], qs[i], c);
+        const float a = fmaf(w.lo[0], xl.x, fmaf(w.lo[1], xl.y, fmaf(w.lo[2], xl.z, w.lo[3] * xl.w)));
+        const float b = fmaf(w.hi[0], xh.x, fmaf(w.hi[1], xh.y, fmaf(w.hi[2], xh.z, w.hi[3] * xh.w)));
+        const float y = wave_sum(fmaf(w.dl, a, fmaf(w.dh, b, -fmaf(w.ml, sl, w.mh * sh))));
+        if (lane == i) mine = y;
+    }
+    if (lane < ROWS && row0 + lane < vh) ctx[(size_t)h * vh + row0 + lane] = mine;
 }
 
 }  // namespace jq
