@@ -354,6 +354,63 @@ __global__ __launch_bounds__(512) void mla_attention_mfma(const float *__restric
     }
 }
 
+// One token over a short context, 512 latent + 64 rope elements: a wave takes two heads and 16 cached tokens, whose rows it holds
+// in registers (a lane 8 latent elements and one rope element of each), so nothing waits for LDS or another wave; grid (n_head / 8,
+// n_split = ceil(context / 16)), four waves.  f32 throughout, output as mla_attention.  Bound: one trip to memory and the
+// launch: a layer's step of 128 heads behind 100 tokens 46.5 us where the matrix-core kernel, with its rows and sums going through
+// LDS between barriers on 16 compute units, makes it 52.3.
+constexpr int MLA_SHORT_TOKENS = 16;
+__global__ __launch_bounds__(256) void mla_attention_short(const float *__restrict__ qabs, const float *__restrict__ q,
+                                                            const float *__restrict__ lat, const float *__restrict__ kpe,
+                                                            float *__restrict__ part, int nope, int T, int n_split, float scale) {
+    constexpr int H = 2, N = MLA_SHORT_TOKENS;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h0 = ((int)blockIdx.x * 4 + wave) * H, split = blockIdx.y;
+    const int t0 = split * N, cnt = min(N, T - t0);
+    float4 qa[H][2], c[N][2];
+    float qp[H], kp[N];
+#pragma unroll
+    for (int h = 0; h < H; h++) {
+        const float4 *src = (const float4 *)(qabs + (size_t)(h0 + h) * MLA_M_LKV + 8 * lane);
+        qa[h][0] = src[0], qa[h][1] = src[1];
+        qp[h] = q[(size_t)(h0 + h) * (nope + MLA_M_ROPE) + nope + lane];
+    }
+#pragma unroll
+    for (int t = 0; t < N; t++) {
+        const size_t at = (size_t)min(t0 + t, T - 1);
+        const float4 *src = (const float4 *)(lat + at * MLA_M_LKV + 8 * lane);
+        c[t][0] = src[0], c[t][1] = src[1];
+        kp[t] = kpe[at * MLA_M_ROPE + lane];
+    }
+#pragma unroll
+    for (int h = 0; h < H; h++) {
+        float s[N], m = -INFINITY, l = 0.0f;
+#pragma unroll
+        for (int t = 0; t < N; t++) {
+            float v = qp[h] * kp[t];
+            v = fmaf(qa[h][0].x, c[t][0].x, fmaf(qa[h][0].y, c[t][0].y, fmaf(qa[h][0].z, c[t][0].z, fmaf(qa[h][0].w, c[t][0].w, v))));
+            v = fmaf(qa[h][1].x, c[t][1].x, fmaf(qa[h][1].y, c[t][1].y, fmaf(qa[h][1].z, c[t][1].z, fmaf(qa[h][1].w, c[t][1].w, v))));
+            s[t] = wave_sum(v) * scale;
+            if (t < cnt) m = fmaxf(m, s[t]);
+        }
+        float4 o[2] = {float4{0.0f, 0.0f, 0.0f, 0.0f}, float4{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+        for (int t = 0; t < N; t++) {
+            const float p = t < cnt ? __expf(s[t] - m) : 0.0f;
+            l += p;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                o[i].x = fmaf(p, c[t][i].x, o[i].x), o[i].y = fmaf(p, c[t][i].y, o[i].y);
+                o[i].z = fmaf(p, c[t][i].z, o[i].z), o[i].w = fmaf(p, c[t][i].w, o[i].w);
+            }
+        }
+        float *dst = part + ((size_t)(h0 + h) * n_split + split) * (MLA_M_LKV + 2);
+        if (lane == 0) dst[0] = m, dst[1] = l;
+        const float v[8] = {o[0].x, o[0].y, o[0].z, o[0].w, o[1].x, o[1].y, o[1].z, o[1].w};
+#pragma unroll
+        for (int i = 0; i < 8; i += 2) *(float2 *)(dst + 2 + 8 * lane + i) = float2{v[i], v[i + 1]};
+    }
+}
+
 // grid (n_head, S, ceil(lkv / 128)), 128 threads, one latent column each: merges the splits of (s, h)
 // into the normalised latent sum olat[s, h, :] = sum_i f_i o_i / sum_i f_i l_i, f_i = exp(m_i - max m).
 __global__ __launch_bounds__(128) void mla_merge(const float *__restrict__ part, float *__restrict__ olat, int n_head,

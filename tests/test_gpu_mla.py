@@ -120,6 +120,18 @@ def test_matrix_core_attention_for_the_deepseek_geometry():
     assert close(dev.forward(x[153:250], 153), ref.forward(x[153:250], 153))
 
 
+@pytest.mark.parametrize("n_head,prompt", [(8, 1), (8, 14), (24, 159), (32, 317)])
+def test_one_token_over_a_short_context(n_head, prompt):
+    """Steps in which a wave takes two heads and 16 cached tokens: contexts of one token, around whole runs of 16, and over the
+    line to the matrix-core kernel."""
+    c = cfg(n_embd=256, n_head=n_head, kv_lora_rank=512, qk_nope=64, qk_rope=64, v_head_dim=32, context_length=prompt + 8)
+    ref, dev = build(c, seed=750 + n_head)
+    x = normal(18, (prompt + 5, c["n_embd"])) * np.float32(2.0)
+    assert close(dev.forward(x[:prompt], 0), ref.forward(x[:prompt], 0))
+    for p in range(prompt, prompt + 5):
+        assert close(dev.forward(x[p:p + 1], p), ref.forward(x[p:p + 1], p), 1e-4), p
+
+
 @pytest.mark.parametrize("n_head,steps", [(3, (47, 48, 129, 1)), (8, (160, 95, 48)), (16, (33, 127, 2))])
 def test_many_tokens_over_keys_and_values_per_head(n_head, steps):
     """DeepSeek's head sizes from 48 tokens a call on: the cached latents expanded to keys and values, attention on split
