@@ -13,9 +13,7 @@ typedef float s16_f16 __attribute__((ext_vector_type(16)));
 
 constexpr int S16_FRAG = 1024;  // bytes of a fragment: 64 lanes x 8 elements
 
-// Weights behind a table of pointers: without the address space the compiler takes their loads for flat ones, which also
-// wait for (and are waited for as) LDS accesses.  (16 bytes, aligned to 4.)
-typedef uint32_t s16_u4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t s16_u4 __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes at any word
 
 // Asynchronous global -> LDS copy of 16 bytes a lane, the wave's landing one behind the other at lds_base (wave-uniform); awaited
 // by hand with s_waitcnt vmcnt.
