@@ -382,29 +382,37 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
         if (tile + 1 < n_tiles) issue(tile + 1, (tile + 1) & 1), scales(tile + 1);
         if (idle || tile * S16_TILE > mine) continue;  // (the whole wave; the barrier above is met all the same)
         const uint8_t *l = lds + (tile & 1) * STAGE + 16 * lane;
-        s16_f16 sc;
+        // scores in units of log2(e): the products of the rope part (latent) and of the head's 128 elements each behind a factor of
+        // their own, since that of one side has no bound in units of the other's (a head without keys, a query of zeros)
+        auto products = [&](const uint8_t *keys, int first, int steps, s16_f16 &sc) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) sc[r] = 0.0f;
-        if constexpr (LATENT) {
+            for (int r = 0; r < 16; r++) sc[r] = 0.0f;
 #pragma unroll
-            for (int s = 0; s < KR; s++) {
-                const s16_h8 kh = *(const s16_h8 *)(l + S16_KV_TILE + (2 * s) * S16_FRAG), kl = *(const s16_h8 *)(l + S16_KV_TILE + (2 * s + 1) * S16_FRAG);
-                sc = s16_mma(kh, qh[s], sc);
-                sc = s16_mma(kh, ql[s], sc);
-                sc = s16_mma(kl, qh[s], sc);
+            for (int s = 0; s < KN; s++) {
+                if (s >= steps) break;
+                const s16_h8 kh = *(const s16_h8 *)(keys + (2 * s) * S16_FRAG), kl = *(const s16_h8 *)(keys + (2 * s + 1) * S16_FRAG);
+                sc = s16_mma(kh, qh[first + s], sc);
+                sc = s16_mma(kh, ql[first + s], sc);
+                sc = s16_mma(kl, qh[first + s], sc);
             }
-            const float to_head = (rinv * t_now) / (qinv * k_now);  // (powers of two)
+        };
+        s16_f16 sc;
+        if constexpr (LATENT) {
+            s16_f16 sr;
+            products(l + S16_KV_TILE, 0, KR, sr);
+            const float fr = rinv * t_now * a.scale_log2e;
 #pragma unroll
-            for (int r = 0; r < 16; r++) sc[r] *= to_head;
-        }
+            for (int r = 0; r < 16; r++) sr[r] *= fr;
+            products(l, KR, KN, sc);
+            const float f = qinv * k_now * a.scale_log2e;
 #pragma unroll
-        for (int s = 0; s < KN; s++) {
-            const s16_h8 kh = *(const s16_h8 *)(l + (2 * s) * S16_FRAG), kl = *(const s16_h8 *)(l + (2 * s + 1) * S16_FRAG);
-            sc = s16_mma(kh, qh[KR + s], sc);
-            sc = s16_mma(kh, ql[KR + s], sc);
-            sc = s16_mma(kl, qh[KR + s], sc);
+            for (int r = 0; r < 16; r++) sc[r] = fmaf(sc[r], f, sr[r]);
+        } else {
+            products(l, 0, KN, sc);
+            const float f = qinv * k_now * a.scale_log2e;
+#pragma unroll
+            for (int r = 0; r < 16; r++) sc[r] *= f;
         }
-        const float f = qinv * k_now * a.scale_log2e;
         const bool edge = tile * S16_TILE + 31 > a.pos0 + tw;  // some query of the wave does not see the whole tile
         float tmax = -INFINITY;
         if (edge) {
@@ -414,7 +422,7 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
         }
 #pragma unroll
         for (int r = 0; r < 16; r++) tmax = fmaxf(tmax, sc[r]);
-        tmax = max_xor32(tmax) * f;
+        tmax = max_xor32(tmax);
         const float mnew = fmaxf(m_run, tmax);  // finite from tile 0 on, whose first key every query sees
         const float vnew = LATENT ? vref : fmaxf(vref, v_now);
         float keep = __builtin_amdgcn_exp2f(m_run - mnew);
@@ -436,8 +444,7 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
             float p[8];
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                p[i] = __builtin_amdgcn_exp2f(fmaf(sc[8 * ks + i], f, 10.0f - mnew));
-                if (edge && tile * S16_TILE + 16 * ks + 8 * (i >> 2) + 4 * hf + (i & 3) > my_key) p[i] = 0.0f;
+                p[i] = __builtin_amdgcn_exp2f(sc[8 * ks + i] + (10.0f - mnew));  // (a masked key: 0)
                 psum += p[i];
                 if constexpr (!LATENT) p[i] *= up;
             }

@@ -34,7 +34,7 @@ __device__ __forceinline__ void s16_split(const float (&x)[8], s16_h8 &hi, s16_h
 }
 
 // The exponent s that puts magnitudes up to `amax` (as float bits, sign cleared) below 2^14; zero, tiny, infinite and NaN
-// maxima are held within +-100, so that no power of two below over- or underflows.
+// maxima are held within +-100, so that no power of two below over- or underflows (a product or quotient of two of them may).
 __device__ __forceinline__ int s16_exponent(uint32_t amax_bits) {
     const int e = min(max((int)(amax_bits >> 23), 40), 240);
     return 13 - (e - 127);

@@ -147,6 +147,31 @@ def test_many_tokens_over_keys_and_values_per_head(n_head, steps):
         pos += n
 
 
+@pytest.mark.parametrize("zero", ["queries and up-projection", "queries", "keys of the up-projection", "rope keys and queries"])
+def test_heads_whose_queries_or_keys_are_zero(zero):
+    """48 tokens a call and more, where a score is the sum of two products that each have scales of their own: heads of zeros
+    (pruned or padded ones) in every place, beside heads with values.  Head 1 has the zeros, head 2 keeps all."""
+    c = cfg(n_embd=256, n_head=3, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=128, context_length=160)
+    ref, _ = build(c, seed=860)
+    rows = {n: (256 if n != "kv_b" else 512, np.asarray(ref.t[n][1]).view(np.uint8)) for n in ("q", "kv_a_mqa", "kv_b", "o")}
+    shape = {"q": (576, 256), "kv_a_mqa": (576, 256), "kv_b": (768, 512), "o": (256, 384)}
+    raw = {n: rows[n][1].reshape(shape[n][0], -1).copy() for n in rows}
+    if "queries" in zero:
+        raw["q"][192 + (128 if "rope" in zero else 0):192 + (192 if "rope" in zero or "up" in zero else 128)] = 0
+    if "up-projection" in zero:
+        raw["kv_b"][256:256 + (256 if "queries" in zero else 128)] = 0
+    if "rope keys" in zero:
+        raw["kv_a_mqa"][512:] = 0
+    t = dict(ref.t, **{n: (capi.Q8_0, b.reshape(-1)) for n, b in raw.items()})
+    w = {n: capi.Weight.upload(capi.Q8_0, raw[n].reshape(-1), *shape[n]) for n in raw}
+    mc = capi.MlaConfig(n_embd=256, n_head=3, q_lora_rank=0, kv_lora_rank=512, qk_nope_head_dim=128, qk_rope_head_dim=64,
+                        v_head_dim=128, n_ctx=160, rms_eps=1e-6, rope_theta=1e4)
+    dev, want = capi.Mla(mc, w["q"], w["kv_a_mqa"], t["kv_a_norm"], w["kv_b"], w["o"]), om.MlaOracle(c, t)
+    x = normal(19, (130, 256))
+    assert close(dev.forward(x[:64], 0), want.forward(x[:64], 0))
+    assert close(dev.forward(x[64:], 64), want.forward(x[64:], 64))
+
+
 def test_heads_in_groups_where_their_keys_and_values_exceed_the_buffer():
     """256 heads of 4200 tokens are expanded in two groups (1 GiB of keys and values each at most).  The 256 are 32
     copies of 8 and so are the output projection's columns: the sum is 32 times what the 8 alone give, up to the order of
