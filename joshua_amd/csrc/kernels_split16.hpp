@@ -25,6 +25,15 @@ constexpr int S16_TILE = 32;                         // keys (or tokens) of a ti
 constexpr int S16_KV_TILE = 2 * 8 * 2 * S16_FRAG;    // a head's K (128) and V (128) of a tile: 8 fragments each, two planes
 constexpr int S16_ROPE_TILE = 4 * 2 * S16_FRAG;      // the shared rope keys (64) of a tile
 
+// What the attention knows of a tile: the powers of two that undo its scales (k: of the keys, or of the rope keys; v: of the
+// values), and a bit per key that holds an infinity or a NaN.  Such an element counts as zero in the tile: 0, the weight of a
+// key that a query does not see, times it would reach that query's sums, and a scale that follows it would take the other
+// keys' bits.  The queries that see the key are NaN.
+struct __attribute__((aligned(16))) S16Tile {
+    float k, v;
+    uint32_t bad, unused;
+};
+
 __device__ __forceinline__ uint32_t s16_block_max(uint32_t v, uint32_t *red) {  // 256 threads
 #pragma unroll
     for (int off = 32; off; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off, 64));
@@ -39,14 +48,15 @@ __device__ __forceinline__ s16_f16 s16_mma(const s16_h8 &a, const s16_h8 &b, con
 }
 
 // ---- keys and values of a cache [kv_head][n_ctx][128] f32 as fragments -----------------------------------------------------
-// grid (tiles, kv heads), 256 threads.  Rows at and past n_keys are zero.  inv[kv head][tile] = the powers of two that
-// undo the tile's scales of K and V.  Bound: memory (twice the cache's bytes).
+// grid (tiles, kv heads), 256 threads.  Rows at and past n_keys are zero.  Bound: memory (twice the cache's bytes).
 __global__ __launch_bounds__(256) void s16_kv_tiles(const float *__restrict__ kc, const float *__restrict__ vc, int n_ctx, int n_keys,
-                                                    uint8_t *__restrict__ ws, float2 *__restrict__ inv) {
+                                                    uint8_t *__restrict__ ws, S16Tile *__restrict__ info) {
     constexpr int D = 128, PAD = 4;
     __shared__ __attribute__((aligned(16))) float vt[S16_TILE][D + PAD];
-    __shared__ uint32_t red[4];
+    __shared__ uint32_t red[4], bad;
     const int tile = blockIdx.x, kvh = blockIdx.y, tid = threadIdx.x;
+    if (tid == 0) bad = 0;
+    __syncthreads();
     const float *kb = kc + ((size_t)kvh * n_ctx + (size_t)tile * S16_TILE) * D, *vb = vc + ((size_t)kvh * n_ctx + (size_t)tile * S16_TILE) * D;
     uint8_t *out = ws + ((size_t)kvh * gridDim.x + tile) * S16_KV_TILE;
     // K: chunk (k-step s, lane) = row lane % 32, columns 16 s + 8 (lane / 32) ..; two chunks a thread
@@ -61,6 +71,7 @@ __global__ __launch_bounds__(256) void s16_kv_tiles(const float *__restrict__ kc
             const float4 v = live ? *(const float4 *)(kb + (size_t)row * D + col + i) : float4{0.f, 0.f, 0.f, 0.f};
             kx[u][i] = v.x, kx[u][i + 1] = v.y, kx[u][i + 2] = v.z, kx[u][i + 3] = v.w;
         }
+        if (!s16_make_finite(kx[u])) atomicOr(&bad, 1u << row);
 #pragma unroll
         for (int i = 0; i < 8; i++) km = max(km, s16_abs(kx[u][i]));
     }
@@ -68,12 +79,15 @@ __global__ __launch_bounds__(256) void s16_kv_tiles(const float *__restrict__ kc
     for (int u = 0; u < 4; u++) {
         const int c = tid + 256 * u, row = c >> 5, col = 4 * (c & 31);
         const float4 v = tile * S16_TILE + row < n_keys ? *(const float4 *)(vb + (size_t)row * D + col) : float4{0.f, 0.f, 0.f, 0.f};
-        *(float4 *)&vt[row][col] = v;
-        vm = max(max(vm, max(s16_abs(v.x), s16_abs(v.y))), max(s16_abs(v.z), s16_abs(v.w)));
+        float x[4] = {v.x, v.y, v.z, v.w};
+        if (!s16_make_finite(x)) atomicOr(&bad, 1u << row);
+        *(float4 *)&vt[row][col] = float4{x[0], x[1], x[2], x[3]};
+#pragma unroll
+        for (int i = 0; i < 4; i++) vm = max(vm, s16_abs(x[i]));
     }
     const int ke = s16_exponent(s16_block_max(km, red)), ve = s16_exponent(s16_block_max(vm, red));  // (their barriers publish vt)
     const float kf = s16_pow2(ke), vf = s16_pow2(ve);
-    if (tid == 0) inv[(size_t)kvh * gridDim.x + tile] = float2{s16_pow2(-ke), s16_pow2(-ve)};
+    if (tid == 0) info[(size_t)kvh * gridDim.x + tile] = S16Tile{s16_pow2(-ke), s16_pow2(-ve), bad, 0u};
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         const int c = tid + 256 * u, s = c >> 6, lane = c & 63;
@@ -138,21 +152,25 @@ __global__ __launch_bounds__(256) void s16_up_projection(const float *__restrict
 }
 
 // grid tiles, 256 threads: the normed latents of 32 tokens as fragments [tile][k-step 32][plane] (times 2^ec), their rope keys
-// as [tile][k-step 4][plane] with a scale a tile, ropeinv[tile] the power of two that undoes it.
+// as [tile][k-step 4][plane] with a scale a tile, info[tile].k the power of two that undoes it.
 __global__ __launch_bounds__(256) void s16_latent_tiles(const float *__restrict__ lat, const float *__restrict__ kpe, int n_keys, float cscale,
-                                                        uint8_t *__restrict__ cf, uint8_t *__restrict__ rf, float *__restrict__ ropeinv) {
-    __shared__ uint32_t red[4];
+                                                        uint8_t *__restrict__ cf, uint8_t *__restrict__ rf, S16Tile *__restrict__ info) {
+    __shared__ uint32_t red[4], bad;
     const int tile = blockIdx.x, tid = threadIdx.x, lane = tid & 63, row = lane & 31, key = tile * S16_TILE + row;
     const bool live = key < n_keys;
     float x[8];
+    bool whole = true;
     auto fetch = [&](const float *src) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 8; i += 4) {
             const float4 v = live ? *(const float4 *)(src + i) : float4{0.f, 0.f, 0.f, 0.f};
             x[i] = v.x, x[i + 1] = v.y, x[i + 2] = v.z, x[i + 3] = v.w;
         }
+        whole &= s16_make_finite(x);
     };
     s16_h8 hi, lo;
+    if (tid == 0) bad = 0;
+    __syncthreads();
     uint8_t *out = cf + (size_t)tile * (S16_LKV / 16) * 2 * S16_FRAG + 16 * lane;
 #pragma unroll 4
     for (int s = tid >> 6; s < S16_LKV / 16; s += 4) {
@@ -165,12 +183,13 @@ __global__ __launch_bounds__(256) void s16_latent_tiles(const float *__restrict_
     }
     const int s = tid >> 6;
     fetch(kpe + (size_t)key * S16_ROPE + 16 * s + 8 * (lane >> 5));
+    if (!whole) atomicOr(&bad, 1u << row);
     uint32_t m = 0;
 #pragma unroll
     for (int i = 0; i < 8; i++) m = max(m, s16_abs(x[i]));
     const int e = s16_exponent(s16_block_max(m, red));
     const float f = s16_pow2(e);
-    if (tid == 0) ropeinv[tile] = s16_pow2(-e);
+    if (tid == 0) info[tile] = S16Tile{s16_pow2(-e), 1.0f, bad, 0u};
 #pragma unroll
     for (int i = 0; i < 8; i++) x[i] *= f;
     s16_split(x, hi, lo);
@@ -272,9 +291,9 @@ struct S16Attention {
     const float *q;            // token t's head h at q + t * q_stride + h * q_head: 128 elements (latent: and 64 rotated ones)
     int q_stride, q_head;
     const uint8_t *kv;         // [kv head][tile]{K, V}
-    const float2 *inv;         // latent: fac of this call's first head, [head][2]; else [kv head][tile]
+    const S16Tile *info;       // latent: [tile], of the rope keys; else [kv head][tile]
+    const float2 *fac;         // latent: of this call's first head, [head][2]
     const uint8_t *rope;       // latent: [tile]
-    const float *ropeinv;      // latent: [tile]
     float *out;                // [t][out_stride], head h at h * 128
     int out_stride;
     int T, pos0, n_tiles;      // tokens of the step at positions pos0 .., tiles of the cache
@@ -358,26 +377,26 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int r = 0; r < 16; r++) o[t][r] = 0.0f;
+    bool spoilt = false;                    // the query sees a key that is not finite
     float m_run = -INFINITY, l_run = 0.0f;  // of the lane's query; the sum over this lane's keys only
-    float vref = LATENT ? a.inv[2 * head + 1].y : s16_pow2(-113);  // the scale the outputs are held in: the largest inv.y so far
-    const float khead = LATENT ? a.inv[2 * head].y : 1.0f;
+    float vref = LATENT ? a.fac[2 * head + 1].y : s16_pow2(-113);  // the scale the outputs are held in: the largest inv.y so far
+    const float khead = LATENT ? a.fac[2 * head].y : 1.0f;
 
-    // the tile's scales, asked for with the tile
-    float kinv = khead, vinv = vref, tinv = 0.0f;
+    // what is known of the tile, asked for with the tile
+    float kinv = 0.0f, vinv = vref;
+    uint32_t bad = 0;
     auto scales = [&](int tile) __attribute__((always_inline)) {
-        if constexpr (LATENT) tinv = a.ropeinv[tile];
-        else {
-            const float2 v = a.inv[(size_t)kvh * a.n_tiles + tile];
-            kinv = v.x, vinv = v.y;
-        }
+        const S16Tile v = a.info[(LATENT ? 0 : (size_t)kvh * a.n_tiles) + tile];
+        kinv = v.k, vinv = v.v, bad = v.bad;
     };
     issue(0, 0);
     scales(0);
     for (int tile = 0; tile < n_tiles; tile++) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         // (the compiler waits for the scales where they are first read: here, and not behind the loads issued next)
-        asm volatile("" : "+v"(kinv), "+v"(vinv), "+v"(tinv));
-        const float k_now = kinv, v_now = vinv, t_now = tinv;
+        asm volatile("" : "+v"(kinv), "+v"(vinv), "+v"(bad));
+        const float k_now = kinv, v_now = vinv;
+        const uint32_t bad_now = (uint32_t)__builtin_amdgcn_readfirstlane((int)bad);
         __syncthreads();  // the tile has landed, and the other buffer's readers are done
         if (tile + 1 < n_tiles) issue(tile + 1, (tile + 1) & 1), scales(tile + 1);
         if (idle || tile * S16_TILE > mine) continue;  // (the whole wave; the barrier above is met all the same)
@@ -400,11 +419,11 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
         if constexpr (LATENT) {
             s16_f16 sr;
             products(l + S16_KV_TILE, 0, KR, sr);
-            const float fr = rinv * t_now * a.scale_log2e;
+            const float fr = rinv * k_now * a.scale_log2e;
 #pragma unroll
             for (int r = 0; r < 16; r++) sr[r] *= fr;
             products(l, KR, KN, sc);
-            const float f = qinv * k_now * a.scale_log2e;
+            const float f = qinv * khead * a.scale_log2e;
 #pragma unroll
             for (int r = 0; r < 16; r++) sc[r] = fmaf(sc[r], f, sr[r]);
         } else {
@@ -412,6 +431,10 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
             const float f = qinv * k_now * a.scale_log2e;
 #pragma unroll
             for (int r = 0; r < 16; r++) sc[r] *= f;
+        }
+        if (bad_now) {
+            const int seen = my_key - tile * S16_TILE;  // the tile's last key that the lane's query sees
+            spoilt |= (bad_now & (seen < 0 ? 0u : 0xFFFFFFFFu >> (31 - min(seen, 31)))) != 0;
         }
         const bool edge = tile * S16_TILE + 31 > a.pos0 + tw;  // some query of the wave does not see the whole tile
         float tmax = -INFINITY;
@@ -451,19 +474,19 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
             s16_split(p, ph[ks], pl[ks]);
         }
         l_run += psum;
+        const uint8_t *lv = l + S16_KV_TILE / 2;
 #pragma unroll
         for (int ks = 0; ks < 2; ks++)
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                const uint8_t *lv = l + S16_KV_TILE / 2 + (2 * t + ks) * 2 * S16_FRAG;
-                const s16_h8 vh = *(const s16_h8 *)lv, vl = *(const s16_h8 *)(lv + S16_FRAG);
+                const s16_h8 vh = *(const s16_h8 *)(lv + (4 * t + 2 * ks) * S16_FRAG), vl = *(const s16_h8 *)(lv + (4 * t + 2 * ks + 1) * S16_FRAG);
                 o[t] = s16_mma(vh, ph[ks], o[t]);
                 o[t] = s16_mma(vh, pl[ks], o[t]);
                 o[t] = s16_mma(vl, ph[ks], o[t]);
             }
     }
     if (tw + n >= a.T) return;
-    const float inv = vref / sum_xor32(l_run);
+    const float inv = spoilt ? __builtin_nanf("") : vref / sum_xor32(l_run);
     float *op = a.out + (size_t)(tw + n) * a.out_stride + (size_t)head * 128;
 #pragma unroll
     for (int t = 0; t < 4; t++)

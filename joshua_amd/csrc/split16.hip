@@ -25,7 +25,7 @@ struct Split16Latent {
     uint8_t *wfrags = nullptr;
     float2 *fac = nullptr;
     uint8_t *cf = nullptr, *rf = nullptr, *ws = nullptr;  // latents, rope keys, a group of heads' keys and values
-    float *ropeinv = nullptr;
+    jq::S16Tile *info = nullptr;
 };
 
 bool split16_latent_fits(size_t nope, size_t rope, size_t vh, size_t lkv) {
@@ -51,7 +51,7 @@ int split16_latent_create(size_t n_head, size_t n_ctx, const float *wkv, const f
 
 void split16_latent_free(Split16Latent *s) {
     if (!s) return;
-    for (void *p : {(void *)s->wfrags, (void *)s->fac, (void *)s->cf, (void *)s->rf, (void *)s->ws, (void *)s->ropeinv})
+    for (void *p : {(void *)s->wfrags, (void *)s->fac, (void *)s->cf, (void *)s->rf, (void *)s->ws, (void *)s->info})
         if (p) (void)hipFree(p);
     delete s;
 }
@@ -65,12 +65,12 @@ int split16_latent_attention(Split16Latent *s, const float *q, size_t S, size_t 
         const size_t most = (size_t)1 << 30, want = std::max(std::min(s->n_head * all * jq::S16_KV_TILE, most), all * jq::S16_KV_TILE);
         if (!s->cf && !have((void **)&s->cf, all * (jq::S16_LKV / 16) * 2 * jq::S16_FRAG)) return -1;
         if (!s->rf && !have((void **)&s->rf, all * jq::S16_ROPE_TILE)) return -1;
-        if (!s->ropeinv && !have((void **)&s->ropeinv, all * sizeof(float))) return -1;
+        if (!s->info && !have((void **)&s->info, all * sizeof(jq::S16Tile))) return -1;
         if (!have((void **)&s->ws, want)) return -1;
         s->ws_bytes = want;
     }
     hipLaunchKernelGGL(jq::s16_latent_tiles, dim3((unsigned)nt), dim3(256), 0, stream, lat, kpe, (int)(pos + S), ldexpf(1.0f, s->ec), s->cf,
-                       s->rf, s->ropeinv);
+                       s->rf, s->info);
     HIP_TRY(hipGetLastError());
     size_t group = std::min(s->n_head, s->ws_bytes / head_bytes);
     if (group >= 8 && group < s->n_head) group = group / 8 * 8;
@@ -81,7 +81,7 @@ int split16_latent_attention(Split16Latent *s, const float *q, size_t S, size_t 
         HIP_TRY(hipGetLastError());
         jq::S16Attention a{};
         a.q = q + h0 * (jq::S16_HEAD + jq::S16_ROPE), a.q_stride = (int)(s->n_head * (jq::S16_HEAD + jq::S16_ROPE)), a.q_head = jq::S16_HEAD + jq::S16_ROPE;
-        a.kv = s->ws, a.inv = s->fac + 2 * h0, a.rope = s->rf, a.ropeinv = s->ropeinv;
+        a.kv = s->ws, a.info = s->info, a.fac = s->fac + 2 * h0, a.rope = s->rf;
         a.out = out + h0 * jq::S16_HEAD, a.out_stride = (int)(s->n_head * jq::S16_HEAD);
         a.T = (int)S, a.pos0 = (int)pos, a.n_tiles = (int)nt, a.heads = (int)hg, a.group = 1, a.blocks = (int)((S + 127) / 128);
         a.scale_log2e = scale * 1.44269504088896340736f;
@@ -93,7 +93,7 @@ int split16_latent_attention(Split16Latent *s, const float *q, size_t S, size_t 
 
 void split16_cache_free(Split16Cache *c) {
     if (c->ws) (void)hipFree(c->ws);
-    if (c->inv) (void)hipFree(c->inv);
+    if (c->info) (void)hipFree(c->info);
     *c = {};
 }
 
@@ -106,13 +106,13 @@ int split16_attention(Split16Cache *c, const float *q, int q_stride, int T, int 
                       int n_ctx, float *out, hipStream_t stream) {
     const size_t all = tiles_of((size_t)n_ctx);
     if (!c->ws && !have((void **)&c->ws, (size_t)kv_heads * all * jq::S16_KV_TILE)) return -1;
-    if (!c->inv && !have((void **)&c->inv, (size_t)kv_heads * all * sizeof(float2))) return -1;
+    if (!c->info && !have((void **)&c->info, (size_t)kv_heads * all * sizeof(jq::S16Tile))) return -1;
     const int nt = (int)tiles_of((size_t)pos + T), g = heads / kv_heads, wh = std::min(g, 4);
-    hipLaunchKernelGGL(jq::s16_kv_tiles, dim3((unsigned)nt, (unsigned)kv_heads), dim3(256), 0, stream, kc, vc, n_ctx, pos + T, c->ws, c->inv);
+    hipLaunchKernelGGL(jq::s16_kv_tiles, dim3((unsigned)nt, (unsigned)kv_heads), dim3(256), 0, stream, kc, vc, n_ctx, pos + T, c->ws, (jq::S16Tile *)c->info);
     HIP_TRY(hipGetLastError());
     jq::S16Attention a{};
     a.q = q, a.q_stride = q_stride, a.q_head = 128;
-    a.kv = c->ws, a.inv = c->inv;
+    a.kv = c->ws, a.info = (const jq::S16Tile *)c->info;
     a.out = out, a.out_stride = heads * 128;
     a.T = T, a.pos0 = pos, a.n_tiles = nt, a.heads = heads, a.group = g;
     const int tb = 32 * (4 / wh);

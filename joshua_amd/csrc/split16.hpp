@@ -19,7 +19,7 @@ int split16_latent_attention(Split16Latent *s, const float *q, size_t S, size_t 
 // The decoder's: a copy of one layer's cache as operands, made anew by each call.
 struct Split16Cache {
     uint8_t *ws = nullptr;
-    float2 *inv = nullptr;
+    void *info = nullptr;  // [kv head][tile]: scales
 };
 void split16_cache_free(Split16Cache *c);
 bool split16_attention_fits(int d, int heads, int kv_heads);

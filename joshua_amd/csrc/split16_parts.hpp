@@ -42,6 +42,18 @@ __device__ __forceinline__ int s16_exponent(uint32_t amax_bits) {
 __device__ __forceinline__ float s16_pow2(int s) { return __builtin_bit_cast(float, (uint32_t)(127 + s) << 23); }
 __device__ __forceinline__ uint32_t s16_abs(float x) { return __builtin_bit_cast(uint32_t, x) & 0x7FFFFFFFu; }
 
+// Zeros in place of infinities and NaNs; whether there were none.
+template <int N>
+__device__ __forceinline__ bool s16_make_finite(float (&x)[N]) {
+    bool all = true;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const bool is = s16_abs(x[i]) < 0x7F800000u;
+        all &= is, x[i] = is ? x[i] : 0.0f;
+    }
+    return all;
+}
+
 // An address that is the same in all lanes, where the compiler does not see that.
 __device__ __forceinline__ const uint8_t *s16_uniform(const uint8_t *p) {
     const uint64_t v = (uint64_t)p;

@@ -172,6 +172,22 @@ def test_heads_whose_queries_or_keys_are_zero(zero):
     assert close(dev.forward(x[64:], 64), want.forward(x[64:], 64))
 
 
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("at", [0, 40, 63])
+def test_a_token_that_is_not_finite_stays_out_of_those_in_front(at, value):
+    """64 tokens a call, whose tiles of 32 keys hold tokens of which some queries see only a part: a token of NaNs is in the
+    results of those behind it, in this call and the next, and in none in front."""
+    c = cfg(n_embd=256, n_head=3, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=128, context_length=160)
+    ref, dev = build(c, seed=870)
+    x = normal(20, (128, 256))
+    want = ref.forward(x[:64], 0)
+    x[at, 7] = value
+    got = dev.forward(x[:64], 0)
+    assert close(got[:at], want[:at])
+    assert not np.isfinite(got[at:]).any(axis=1).any()
+    assert not np.isfinite(dev.forward(x[64:], 64)).any()
+
+
 def test_heads_in_groups_where_their_keys_and_values_exceed_the_buffer():
     """256 heads of 4200 tokens are expanded in two groups (1 GiB of keys and values each at most).  The 256 are 32
     copies of 8 and so are the output projection's columns: the sum is 32 times what the 8 alone give, up to the order of

@@ -229,6 +229,29 @@ def test_attention_of_many_tokens_over_values_of_different_size(n_head, n_kv, st
         pos += n
 
 
+@pytest.mark.parametrize("at", [0, 45, 79])
+def test_a_token_that_is_not_finite_stays_out_of_those_in_front(at):
+    """Steps of 80 and 48 tokens, whose attention takes keys in tiles of 32: a token whose embedding is NaN is in the logits of
+    those behind it and in none in front."""
+    cfg = dict(CFG, n_ctx=160, n_layer=2, head_dim=128, n_head=8, n_kv_head=2)
+    emb = np.random.default_rng(4).normal(size=(768, 512)).astype(np.float32)
+    blocks = synth.quantize(capi.Q8_0, emb).copy()
+    np.asarray(blocks).view(np.uint8).reshape(768, -1)[700, :2] = (0x00, 0x7E)   # the scale of its first block: NaN
+    m, o = make(cfg, 53, override={"token_embd.weight": (capi.Q8_0, blocks)})
+    toks = [int(t) for t in np.random.default_rng(5).integers(0, 700, size=128)]
+    front = [p for p in range(0, 80, 3) if p < at] + ([at - 1] if at else [])
+    behind = [p for p in (at, 46, 64, 79) if p >= at]
+    ref = [o.forward(toks[:p + 1], 0) for p in front[-1:]]
+    toks[at] = 700
+    m.reset()
+    got = m.logits_at(toks[:80], 0, front + behind)
+    assert np.isfinite(got[:len(front)]).all() and not np.isfinite(got[len(front):]).any()
+    if front:
+        ok, e = close(got[len(front) - 1], ref[0])
+        assert ok, e
+    assert not np.isfinite(m.logits_at(toks[80:], 80, [0, 47])).any()
+
+
 @pytest.mark.parametrize("head_dim,n_head,n_kv", [(64, 4, 2), (128, 4, 1), (256, 2, 2), (192, 4, 2), (128, 8, 1),
                                                   (128, 2, 2), (128, 4, 2)])
 def test_decode_over_several_key_chunks(head_dim, n_head, n_kv):
