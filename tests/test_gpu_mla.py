@@ -172,6 +172,53 @@ def test_heads_whose_queries_or_keys_are_zero(zero):
     assert close(dev.forward(x[64:], 64), want.forward(x[64:], 64))
 
 
+def f16(x):
+    return x.astype(np.float16).astype(np.float64)
+
+
+def test_many_tokens_hold_every_operand_to_more_than_f16():
+    """Latent attention of 200 tokens against 64 bits.  The inputs are unit vectors, so that the products in front of the attention
+    are columns of their weights, and the error is the attention's and that of the 16-bit activations of the product behind it:
+    half a step of 2^-15 of the largest of 256, 0.9e-5 of the norm for values of which that is 3 times the rest.  An operand
+    that was held to f16 alone would show: each is rounded in turn here, on the CPU, and is twice over the bound or more."""
+    nh, S, rng = 2, 200, np.random.default_rng(6)
+    shape = {"q": (nh * 192, 256), "kv_a": (576, 256), "kv_b": (nh * 256, 512), "o": (256, nh * 128)}
+    sigma = {"q": 2.0, "kv_a": 1.0, "kv_b": 0.05, "o": 0.1}
+    blocks = {n: quantized(capi.Q8_0, 880 + i, *shape[n], sigma[n]) for i, n in enumerate(sorted(shape))}
+    W = {n: oracle.dequantize(capi.Q8_0, b).reshape(shape[n]).astype(np.float64) for n, b in blocks.items()}
+    w = {n: capi.Weight.upload(capi.Q8_0, b, *shape[n]) for n, b in blocks.items()}
+    norm = (1.0 + 0.1 * normal(890, (512,))).astype(np.float32)
+    mc = capi.MlaConfig(n_embd=256, n_head=nh, q_lora_rank=0, kv_lora_rank=512, qk_nope_head_dim=128, qk_rope_head_dim=64,
+                        v_head_dim=128, n_ctx=256, rms_eps=1e-6, rope_theta=1e4)
+    idx = rng.permutation(256)[:S]
+    got = capi.Mla(mc, w["q"], w["kv_a"], norm, w["kv_b"], w["o"]).forward(np.eye(256, dtype=np.float32)[idx], 0)
+
+    angle = np.arange(S)[:, None] * 1e4 ** (-np.arange(0, 64, 2) / 64.0)
+    turn = lambda v: np.stack([v[..., 0::2] * np.cos(angle) - v[..., 1::2] * np.sin(angle),
+                               v[..., 1::2] * np.cos(angle) + v[..., 0::2] * np.sin(angle)], -1).reshape(v.shape)
+    q, comp = W["q"][:, idx].T.reshape(S, nh, 192), W["kv_a"][:, idx].T
+    lat = comp[:, :512] / np.sqrt((comp[:, :512] ** 2).mean(1, keepdims=True) + 1e-6) * norm
+    kpe, up = turn(comp[:, 512:]), W["kv_b"].reshape(nh, 2, 128, 512)
+
+    def block(**rounded):
+        as_is = lambda v: v
+        r = {n: rounded.get(n, as_is) for n in ("latents", "up", "queries", "rope", "keys", "values", "weights")}
+        ctx = []
+        for h in range(nh):
+            k, v = (r["latents"](lat) @ r["up"](u).T for u in up[h])
+            s = r["queries"](q[:, h, :128]) @ r["keys"](k).T + r["queries"](turn(q[:, h, 128:])) @ r["rope"](kpe).T
+            s = np.where(np.tri(S, dtype=bool), s / np.sqrt(192.0), -np.inf)
+            e = np.exp(s - s.max(1, keepdims=True))
+            ctx.append(r["weights"](e) @ r["values"](v) / e.sum(1, keepdims=True))
+        return np.concatenate(ctx, 1) @ W["o"].T
+
+    want = block()
+    err = lambda y: np.linalg.norm(y - want) / np.linalg.norm(want)
+    assert err(got) < 3e-5, err(got)
+    for n in ("latents", "up", "queries", "rope", "keys", "values", "weights"):
+        assert err(block(**{n: f16})) > 8e-5, (n, err(block(**{n: f16})))
+
+
 @pytest.mark.parametrize("value", [np.nan, np.inf])
 @pytest.mark.parametrize("at", [0, 40, 63])
 def test_a_token_that_is_not_finite_stays_out_of_those_in_front(at, value):

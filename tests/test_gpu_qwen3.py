@@ -229,6 +229,52 @@ def test_attention_of_many_tokens_over_values_of_different_size(n_head, n_kv, st
         pos += n
 
 
+def test_attention_of_many_tokens_holds_every_operand_to_more_than_f16():
+    """One layer over 200 tokens against 64 bits.  The embeddings are unit vectors, so that queries, keys and values are columns
+    of their weights, and the down projection is zero: the error is the attention's and that of the 16-bit activations of the
+    two products behind it (half a step of 2^-15 of the largest of 256 each).  An operand that was held to f16 alone would
+    show: each is rounded in turn here, on the CPU, and is twice over the bound or more."""
+    nh, nkv, h, S, rng = 8, 2, 256, 200, np.random.default_rng(8)
+    cfg = dict(CFG, n_ctx=256, n_layer=1, hidden=h, head_dim=128, n_head=nh, n_kv_head=nkv, ffn=256, vocab=256)
+    q8 = lambda v: (capi.Q8_0, synth.quantize(capi.Q8_0, np.ascontiguousarray(v, dtype=np.float32)))
+    over = {"token_embd.weight": q8(np.eye(256)), "output.weight": q8(rng.normal(size=(256, h))),
+            "blk.0.ffn_down.weight": q8(np.zeros((h, 256))), "blk.0.attn_output.weight": q8(rng.normal(size=(h, nh * 128)) * 0.2),
+            "blk.0.attn_q_norm.weight": (0, (3.0 + rng.normal(size=128)).astype(np.float32))}
+    over.update({f"blk.0.attn_{n}.weight": q8(rng.normal(size=(r * 128, h))) for n, r in (("q", nh), ("k", nkv), ("v", nkv))})
+    m, o = make(cfg, 55, override=over)
+    W = {n: oracle.dequantize(t, d).reshape(-1, nh * 128 if n == "blk.0.attn_output.weight" else 256).astype(np.float64)
+         for n, (t, d) in o.t.items() if t != 0}
+    F = {n: np.asarray(d).astype(np.float64) for n, (t, d) in o.t.items() if t == 0}
+    toks = rng.permutation(256)[:S]
+    got = m.logits_at(toks, 0, list(range(S)))
+
+    rms = lambda v, w: v / np.sqrt((v * v).mean(-1, keepdims=True) + cfg["rms_eps"]) * w
+    angle = np.arange(S)[:, None, None] * cfg["rope_theta"] ** (-np.arange(64) / 64.0)
+    turn = lambda v: np.concatenate([v[..., :64] * np.cos(angle) - v[..., 64:] * np.sin(angle),
+                                     v[..., 64:] * np.cos(angle) + v[..., :64] * np.sin(angle)], -1)
+    x = W["token_embd.weight"][toks]
+    n1 = rms(x, F["blk.0.attn_norm.weight"])
+    q, k, v = ((n1 @ W[f"blk.0.attn_{n}.weight"].T).reshape(S, -1, 128) for n in "qkv")
+    q, k = turn(rms(q, F["blk.0.attn_q_norm.weight"])), turn(rms(k, F["blk.0.attn_k_norm.weight"]))
+
+    def logits(**rounded):
+        r = {n: rounded.get(n, lambda v: v) for n in ("queries", "keys", "values", "weights")}
+        ctx = []
+        for i in range(nh):
+            s = r["queries"](q[:, i]) @ r["keys"](k[:, i // 4]).T
+            s = np.where(np.tri(S, dtype=bool), s / np.sqrt(128.0), -np.inf)
+            e = np.exp(s - s.max(1, keepdims=True))
+            ctx.append(r["weights"](e) @ r["values"](v[:, i // 4]) / e.sum(1, keepdims=True))
+        return rms(x + np.concatenate(ctx, 1) @ W["blk.0.attn_output.weight"].T, F["output_norm.weight"]) @ W["output.weight"].T
+
+    want = logits()
+    err = lambda y: np.linalg.norm(y - want) / np.linalg.norm(want)
+    f16 = lambda v: v.astype(np.float16).astype(np.float64)
+    assert err(got) < 3e-5, err(got)
+    for n in ("queries", "keys", "values", "weights"):
+        assert err(logits(**{n: f16})) > 8e-5, (n, err(logits(**{n: f16})))
+
+
 @pytest.mark.parametrize("at", [0, 45, 79])
 def test_a_token_that_is_not_finite_stays_out_of_those_in_front(at):
     """Steps of 80 and 48 tokens, whose attention takes keys in tiles of 32: a token whose embedding is NaN is in the logits of
