@@ -1305,6 +1305,31 @@ bool moe_mx_pays(const jq_moe_config &c, size_t T, bool decode_sized) {
     return 0.16 * P > 0.11 * hit + 15e6 / (3.0 * c.hidden * (double)c.inter);
 }
 
+// Bytes of the activations of moe_split16 or moe_mx in calls of up to T tokens of this layer, 0 where it runs neither.
+size_t moe_split_need(const jq_moe *m, size_t T) {
+    const jq_moe_config &c = m->cfg;
+    const size_t rows = c.n_expert_used + 1;  // of the pair buffers, a token
+    if (m->gate->type == JQ_TYPE_Q4_K)
+        return moe_split16_pays(c, T) ? std::max(moe_split16_bytes(T, c.hidden), moe_split16_bytes(T * rows, c.inter)) : 0;
+    const size_t t = std::min(T, moe_mx_upto(c));
+    if (m->gate->type == JQ_TYPE_MXFP4 && m->down->type == JQ_TYPE_MXFP4 && t >= 3 && c.hidden % 512 == 0 && c.inter % 512 == 0)
+        return std::max(moe_mx_bytes(t, c.hidden), moe_mx_bytes(t * rows, c.inter));
+    return 0;
+}
+
+// (without the buffer the older kernels run)
+int moe_grow_quantized(jq_moe *m) {
+    const size_t need = moe_split_need(m, m->cap_tokens);
+    if (need <= m->split_bytes) return 0;
+    if (m->split_acts) HIP_TRY(hipFree(m->split_acts));
+    m->split_bytes = need;
+    if (hipMalloc((void **)&m->split_acts, need) != hipSuccess) {
+        m->split_acts = nullptr;
+        (void)hipGetLastError();
+    }
+    return 0;
+}
+
 int moe_reserve_quantized(jq_moe *m, size_t T) {
     const jq_moe_config &c = m->cfg;
     const size_t P = T * c.n_expert_used, PR = P + T;
@@ -1317,11 +1342,6 @@ int moe_reserve_quantized(jq_moe *m, size_t T) {
     }
     if (m->gate->type == JQ_TYPE_Q4_K || m->down->type == JQ_TYPE_Q4_K)
         HIP_TRY(hipMalloc((void **)&m->qacts, std::max(T * (c.hidden / 256), PR * (c.inter / 256)) * jq::QS_REC + 16));
-    if (m->gate->type == JQ_TYPE_Q4_K && moe_split16_pays(c, T))
-        HIP_TRY(hipMalloc((void **)&m->split_acts, std::max(moe_split16_bytes(T, c.hidden), moe_split16_bytes(PR, c.inter))));
-    const size_t mx_tokens = std::min(T, moe_mx_upto(c));
-    if (m->gate->type == JQ_TYPE_MXFP4 && m->down->type == JQ_TYPE_MXFP4 && mx_tokens >= 3 && c.hidden % 512 == 0 && c.inter % 512 == 0)
-        HIP_TRY(hipMalloc((void **)&m->split_acts, std::max(moe_mx_bytes(mx_tokens, c.hidden), moe_mx_bytes(mx_tokens * (c.n_expert_used + 1), c.inter))));
     if (P > c.n_expert && (moe_has_gemm_i8(m->gate->type) || moe_has_gemm_i8(m->down->type))) {
         // row groups of 16 pairs that never mix two experts: at most PR / 16 + one part-filled group an expert
         m->gtab_rows = PR / 16 + c.n_expert + 2;
@@ -2010,7 +2030,8 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
     const int d16 = align_of({m->down, m->fold_shared ? m->sdown : nullptr});
     const bool same_gu = m->gate->type == m->up->type && m->gate->row_bytes == m->up->row_bytes;
     // MXFP4 on the matrix cores' own FP4 (not where a way was asked for)
-    const bool mx = !pct_env && !expert_env && m->split_acts && m->gate->type == JQ_TYPE_MXFP4 && same_gu && moe_mx_pays(c, T, decode_sized) &&
+    const bool split_room = m->split_acts && moe_split_need(m, T) <= m->split_bytes;
+    const bool mx = !pct_env && !expert_env && split_room && m->gate->type == JQ_TYPE_MXFP4 && same_gu && moe_mx_pays(c, T, decode_sized) &&
                     ((uintptr_t)x & 15) == 0 && moe_mx_takes(c.inter, c.hidden, m->gate->row_bytes, a16, T) &&
                     m->down->type == JQ_TYPE_MXFP4 && moe_mx_takes(c.hidden, c.inter, m->down->row_bytes, d16, (size_t)P + (size_t)extra * T);
     if (mx) decode_sized = expert_dot8 = false;
@@ -2085,7 +2106,7 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
     // few pairs an expert, by the cost estimate above: the expert's rows decoded once, its pairs streamed past
     const bool multi = max_group > 1 && expert_dot8;
     // Q4_K, four pairs an expert or more: exact products of split f16 activations
-    const bool split16 = max_group > 1 && m->split_acts && m->gate->type == JQ_TYPE_Q4_K && moe_split16_pays(c, T) && !expert_env;
+    const bool split16 = max_group > 1 && split_room && m->gate->type == JQ_TYPE_Q4_K && moe_split16_pays(c, T) && !expert_env;
     if (same_gu && split16 && ((uintptr_t)x & 15) == 0 && moe_split16_takes(c.hidden, m->gate->row_bytes, a16, T))
         rc = moe_split16({m->pgate, m->pup, m->gate->row_bytes, x, T, m->gexp, m->offsets, m->xrow, m->yrow, groups, (size_t)P + (size_t)extra * T,
                           m->G, c.hidden, c.inter, clamp, m->split_acts}, s);
@@ -2246,7 +2267,7 @@ bool moe_takes_quantized(const jq_weight *gate, const jq_weight *up, const jq_we
     return !dense_elem_bytes(gate->type) && !dense_elem_bytes(up->type) && !dense_elem_bytes(down->type);
 }
 
-const MoeBackend g_quantized_moe{moe_takes_quantized, moe_reserve_quantized, nullptr,
+const MoeBackend g_quantized_moe{moe_takes_quantized, moe_reserve_quantized, moe_grow_quantized, nullptr,
                                  [](jq_moe *m, size_t T, const float *x, float *y, hipStream_t s, MoePreNorm *pre) {
                                      return moe_forward_dev(m, T, x, y, s, pre);
                                  }};

@@ -376,7 +376,7 @@ int forward_dense(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s, 
     return moe_forward_dense(m, T, x, nullptr, y, s);
 }
 
-const MoeBackend g_dense_moe{takes_dense, reserve_dense, release_dense, forward_dense};
+const MoeBackend g_dense_moe{takes_dense, reserve_dense, nullptr, release_dense, forward_dense};
 const RegisterMoeBackend g_register_dense_moe(&g_dense_moe);
 
 }  // namespace

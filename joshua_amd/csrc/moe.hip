@@ -16,7 +16,7 @@ static void moe_free_scratch(jq_moe *m) {
                     (void *)m->qi8.xh, (void *)m->qi8.sx, (void *)m->qi8.sxs, (void *)m->gacts, (void *)m->gtab, (void *)m->split_acts, (void *)m->group_counts, (void *)m->sgate_logit})
         if (p) (void)hipFree(p);
     if (m->backend && m->backend->release) m->backend->release(m);
-    m->qacts = m->split_acts = nullptr;
+    m->qacts = m->split_acts = nullptr, m->split_bytes = 0;
     m->group_counts = nullptr, m->sgate_logit = nullptr;
     m->gacts = nullptr, m->gtab = nullptr, m->gtab_rows = 0;
     m->qi8 = jq::ActsI8{nullptr, nullptr, nullptr, nullptr};
@@ -26,8 +26,7 @@ static void moe_free_scratch(jq_moe *m) {
     m->cap_tokens = 0;
 }
 
-int moe_reserve(jq_moe *m, size_t T) {
-    if (T <= m->cap_tokens) return 0;
+static int moe_reserve_tokens(jq_moe *m, size_t T) {
     moe_free_scratch(m);
     const jq_moe_config &c = m->cfg;
     // rows of the pair buffers: the routed pairs, then one per token for a folded shared expert
@@ -54,6 +53,11 @@ int moe_reserve(jq_moe *m, size_t T) {
     }
     m->cap_tokens = T;
     return 0;
+}
+
+int moe_reserve(jq_moe *m, size_t T) {
+    if (T > m->cap_tokens && moe_reserve_tokens(m, T)) return 1;
+    return m->backend->grow ? m->backend->grow(m) : 0;
 }
 
 jq::MoeGateParams moe_gate_params(const jq_moe_config &c) {
@@ -190,7 +194,8 @@ void moe_swap_scratch(jq_moe *a, jq_moe *b) {
     std::swap(a->out, b->out), std::swap(a->sG, b->sG), std::swap(a->sU, b->sU), std::swap(a->sH, b->sH);
     std::swap(a->sOut, b->sOut), std::swap(a->ids, b->ids), std::swap(a->gexp, b->gexp);
     std::swap(a->offsets, b->offsets), std::swap(a->xrow, b->xrow), std::swap(a->yrow, b->yrow);
-    std::swap(a->qacts, b->qacts), std::swap(a->gacts, b->gacts), std::swap(a->split_acts, b->split_acts), std::swap(a->gtab, b->gtab);
+    std::swap(a->qacts, b->qacts), std::swap(a->gacts, b->gacts), std::swap(a->gtab, b->gtab);
+    std::swap(a->split_acts, b->split_acts), std::swap(a->split_bytes, b->split_bytes);
     std::swap(a->dense_x, b->dense_x), std::swap(a->dense_act, b->dense_act), std::swap(a->group_counts, b->group_counts);
     std::swap(a->dense_sact, b->dense_sact), std::swap(a->sgate_logit, b->sgate_logit);
     std::swap(a->gtab_rows, b->gtab_rows), std::swap(a->gtile_rgs, b->gtile_rgs), std::swap(a->qi8, b->qi8);

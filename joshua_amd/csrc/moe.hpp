@@ -19,6 +19,7 @@ struct MoePreNorm {
 struct MoeBackend {
     bool (*takes)(const jq_weight *gate, const jq_weight *up, const jq_weight *down);
     int (*reserve)(jq_moe *m, size_t T);   // scratch beside moe_reserve's
+    int (*grow)(jq_moe *m);                // (or null) what a layer asks for by its own weights, see moe_reserve
     void (*release)(jq_moe *m);            // and its end
     int (*forward)(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s, MoePreNorm *pre);
 };
@@ -43,7 +44,10 @@ struct jq_moe {
     uint32_t *ids = nullptr;
     int *gexp = nullptr, *offsets = nullptr, *xrow = nullptr, *yrow = nullptr;
     uint8_t *qacts = nullptr;  // activations as MFMA operand records (Q4_K experts, grouped path)
-    uint8_t *split_acts = nullptr;  // activations as f16 planes (Q4_K experts, moe_split16)
+    // activations as f16 planes (Q4_K experts, moe_split16) or FP8 digits (MXFP4, moe_mx), and the bytes that there are for them, or
+    // that could not be had (then the buffer is null)
+    uint8_t *split_acts = nullptr;
+    size_t split_bytes = 0;
     uint8_t *gacts = nullptr;  // activations of the grouped int8 GEMM, and its tables
     int *gtab = nullptr;
     size_t gtab_rows = 0;      // row groups (and tiles) the tables hold
@@ -60,6 +64,8 @@ struct jq_moe {
 
 namespace jqh {
 
+// Scratch for calls of up to T tokens.  That of another layer of the model may have come with it (moe_swap_scratch), whose weights
+// have other types: what depends on those is looked at in every call.
 int moe_reserve(jq_moe *m, size_t T);
 int moe_route_dev(jq_moe *m, size_t T, const float *x, hipStream_t s, jq::MoePairGroups pg,
                   jq::ActsI8 planes = jq::ActsI8{nullptr, nullptr, nullptr, nullptr}, bool *planes_made = nullptr,

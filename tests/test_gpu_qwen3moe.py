@@ -156,3 +156,27 @@ def test_load_failures_of_a_qwen3moe_file(tmp_path):
     attempt("nokey.gguf", full, md=md, expect="missing GGUF metadata key `qwen3moe.expert_used_count`")
     attempt("toomany.gguf", full, md=gw.qwen3_metadata(dict(cfg, n_expert_used=9)),
             expect="expert_used_count 9 must be in 1..=expert_count 8")
+
+
+@pytest.mark.parametrize("first", [capi.MXFP4, capi.Q6_K])
+def test_layers_whose_experts_are_of_different_types_share_scratch(first):
+    """The layers of a model take turns with one set of buffers, made by the first.  900 tokens over 64 experts: the activations
+    of a Q4_K layer take 17 MB, those of MXFP4 at most 15 (up to 96 pairs an expert) and a Q6_K layer has none, so the Q4_K
+    layers behind them have to ask for their own."""
+    cfg = dict(CFG, n_layer=3, hidden=512, n_ctx=912, vocab=512, n_expert=64, n_expert_used=8, expert_ffn=512)
+    E, h, eff, T = 64, 512, 512, 900
+    tensors = {n: (qt, d) for n, qt, d in qwen3_tensors(cfg, 71, "q4_k", share_layers=True)}
+    for i, n in enumerate(("gate", "up", "down")):
+        tensors[f"blk.0.ffn_{n}_exps.weight"] = (first, synth.normal_quantized(first, 72 + i, E * eff * h, h ** -0.5))
+    m = capi.Qwen3(capi.Qwen3Config(3, h, cfg["n_head"], cfg["n_kv_head"], cfg["head_dim"], 0, 512, 912, cfg["rms_eps"],
+                                    cfg["rope_theta"], E, 8, eff, 1))
+    for name, (qt, data) in tensors.items():
+        m.set_tensor(name, qt, data)
+    toks = np.random.default_rng(73).integers(0, 512, size=T + 6)
+    m.logits_at(toks[:T], 0, [])
+    assert capi.last_kernel() == "moe_split16"
+    m.reset()
+    o = oq.Qwen3Oracle(cfg, tensors, avx2=oracle.have_avx2())
+    assert close(m.forward(toks[:T], 0), o.forward([int(t) for t in toks[:T]], 0))
+    assert close(m.forward(toks[T:], T), o.forward([int(t) for t in toks[T:]], T))
+    m.close()
