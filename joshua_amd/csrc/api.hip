@@ -2017,6 +2017,9 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
         decode_sized = by_pairs <= std::min(by_gemm, by_expert) && P <= 16384;
         if (!expert_env) expert_dot8 = by_expert < by_gemm;
     }
+    // One token is never bucketed: the kernels behind take a call whose groups hold one pair each (max_group 1) to have
+    // a group a pair, where a bucketed one has a group an expert.
+    decode_sized |= T == 1;
     // What every expert's first byte is a multiple of (a view may start at any whole block, and blocks of 17,
     // 34, 66, 210 bytes put that anywhere): 16-byte and 4-byte loads into LDS want it, the kernels that read
     // through registers do not.

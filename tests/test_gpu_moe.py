@@ -237,6 +237,16 @@ def test_experts_that_are_views_at_odd_block_offsets(qtype, lead_blocks):
     dev.close()
 
 
+@pytest.mark.parametrize("E,k,shared_inter", [(8, 7, 0), (8, 8, 256), (16, 14, 0)])
+def test_one_token_that_takes_nearly_every_expert(E, k, shared_inter):
+    """One token of Q4_K experts with short rows whose pairs hit most experts: by the estimate of costs it would be bucketed, but
+    the kernels for one row a group take such a call to have a group a pair."""
+    ora, dev = build(capi.Q4_K, 512, 256, E, k, 95 + E, shared_inter=shared_inter)
+    for seed in range(3):
+        x = synth.normal(96 + seed, (1, 512))
+        assert close(dev.forward(x), ora.forward(x))
+
+
 @pytest.mark.parametrize("tokens", [9, 20, 40])
 def test_few_tokens_an_expert_take_the_int8_quads_kernel(tokens):
     """16 experts, top-2: 18 to 80 pairs over 16 experts is at most five a group on average, the range of the
