@@ -9,10 +9,12 @@ namespace {
 
 size_t tiles_of(size_t tokens) { return (tokens + jq::S16_TILE - 1) / jq::S16_TILE; }
 
-// hipMalloc that leaves no error behind where there is no memory.
-bool have(void **p, size_t bytes) {
-    if (hipMalloc(p, bytes) == hipSuccess) return true;
+// hipMalloc that leaves no error behind; `refused` is set where there is no memory (and not under a stream's capture, say).
+bool have(void **p, size_t bytes, bool *refused) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return true;
     *p = nullptr;
+    *refused |= e == hipErrorOutOfMemory;
     (void)hipGetLastError();
     return false;
 }
@@ -20,7 +22,8 @@ bool have(void **p, size_t bytes) {
 }  // namespace
 
 struct Split16Latent {
-    size_t n_head, n_ctx, ws_bytes = 0;
+    size_t n_head, n_ctx, ws_bytes = 0;  // (0: not asked for yet)
+    bool refused = false;                // there was no memory for the buffers below
     int ec;                              // exponent of the latents' scale
     uint8_t *wfrags = nullptr;
     float2 *fac = nullptr;
@@ -32,6 +35,22 @@ bool split16_latent_fits(size_t nope, size_t rope, size_t vh, size_t lkv) {
     return nope == jq::S16_HEAD && vh == jq::S16_HEAD && rope == jq::S16_ROPE && lkv == jq::S16_LKV;
 }
 
+// Bytes of an object's keys and values: those of all heads over the whole context, so that no later call allocates, up to
+// 512 MiB (what the absorbed form's scratch takes for 1000 tokens of 128 heads); longer contexts take the heads in groups.
+// 4096 tokens of DeepSeek-V3's size in chunks of 512: 7.5 ms, with 256 MiB 7.8; 512 tokens behind 8000: 2.5 and 3.9.
+static size_t latent_ws_bytes(const Split16Latent *s) {
+    return s->ws_bytes ? s->ws_bytes : std::min(s->n_head * tiles_of(s->n_ctx) * jq::S16_KV_TILE, (size_t)512 << 20);
+}
+
+// Heads of a group of a call over nt tiles: as even as fits, by eights where they fit (a head then keeps to one XCD); 0 where
+// not one fits.
+static size_t latent_group(const Split16Latent *s, size_t nt) {
+    const size_t fit = std::min(s->n_head, latent_ws_bytes(s) / (nt * jq::S16_KV_TILE));
+    if (fit == 0) return 0;
+    const size_t groups = (s->n_head + fit - 1) / fit, even = (s->n_head + groups - 1) / groups, eights = (even + 7) / 8 * 8;
+    return eights <= fit ? eights : even;
+}
+
 int split16_latent_create(size_t n_head, size_t n_ctx, const float *wkv, const float *kv_norm, Split16Latent **out) {
     std::unique_ptr<Split16Latent, void (*)(Split16Latent *)> s(new Split16Latent{n_head, n_ctx}, split16_latent_free);
     float wmax = 0.0f;
@@ -41,8 +60,10 @@ int split16_latent_create(size_t n_head, size_t n_ctx, const float *wkv, const f
     int e;
     (void)frexpf(cmax, &e);  // cmax < 2^e
     s->ec = 14 - e;
-    HIP_TRY(hipMalloc((void **)&s->wfrags, n_head * 2 * (jq::S16_LKV / 16) * 8 * jq::S16_FRAG));
-    HIP_TRY(hipMalloc((void **)&s->fac, n_head * 2 * sizeof(float2)));
+    *out = nullptr;
+    if (!have((void **)&s->wfrags, n_head * 2 * (jq::S16_LKV / 16) * 8 * jq::S16_FRAG, &s->refused) ||
+        !have((void **)&s->fac, n_head * 2 * sizeof(float2), &s->refused))
+        return 0;
     hipLaunchKernelGGL(jq::s16_up_projection, dim3(2, (unsigned)n_head), dim3(256), 0, nullptr, wkv, s->wfrags, s->fac, cmax, s->ec);
     HIP_TRY(hipGetLastError());
     *out = s.release();
@@ -58,22 +79,27 @@ void split16_latent_free(Split16Latent *s) {
 
 int split16_latent_attention(Split16Latent *s, const float *q, size_t S, size_t pos, const float *lat, const float *kpe, float scale,
                              float *out, hipStream_t stream) {
-    const size_t all = tiles_of(s->n_ctx), nt = tiles_of(pos + S), head_bytes = nt * jq::S16_KV_TILE;
+    const size_t all = tiles_of(s->n_ctx), nt = tiles_of(pos + S);
+    if (s->refused) return -1;
     if (!s->ws) {
-        // The whole context's keys and values of all heads up to 1 GiB, so that no later call allocates; longer contexts
-        // take the heads in groups.
-        const size_t most = (size_t)1 << 30, want = std::max(std::min(s->n_head * all * jq::S16_KV_TILE, most), all * jq::S16_KV_TILE);
-        if (!s->cf && !have((void **)&s->cf, all * (jq::S16_LKV / 16) * 2 * jq::S16_FRAG)) return -1;
-        if (!s->rf && !have((void **)&s->rf, all * jq::S16_ROPE_TILE)) return -1;
-        if (!s->info && !have((void **)&s->info, all * sizeof(jq::S16Tile))) return -1;
-        if (!have((void **)&s->ws, want)) return -1;
+        size_t want = latent_ws_bytes(s);
+        bool none = false;
+        const bool rest = (s->cf || have((void **)&s->cf, all * (jq::S16_LKV / 16) * 2 * jq::S16_FRAG, &s->refused)) &&
+                          (s->rf || have((void **)&s->rf, all * jq::S16_ROPE_TILE, &s->refused)) &&
+                          (s->info || have((void **)&s->info, all * sizeof(jq::S16Tile), &s->refused));
+        while (rest && !have((void **)&s->ws, want, &none)) {  // half as much, down to one head
+            if (!none || want / 2 < all * jq::S16_KV_TILE) break;
+            want /= 2;
+        }
+        s->refused |= none && !s->ws;
+        if (!s->ws) return -1;
         s->ws_bytes = want;
     }
+    const size_t group = latent_group(s, nt);
+    if (group == 0) return -1;
     hipLaunchKernelGGL(jq::s16_latent_tiles, dim3((unsigned)nt), dim3(256), 0, stream, lat, kpe, (int)(pos + S), ldexpf(1.0f, s->ec), s->cf,
                        s->rf, s->info);
     HIP_TRY(hipGetLastError());
-    size_t group = std::min(s->n_head, s->ws_bytes / head_bytes);
-    if (group >= 8 && group < s->n_head) group = group / 8 * 8;
     for (size_t h0 = 0; h0 < s->n_head; h0 += group) {
         const size_t hg = std::min(group, s->n_head - h0);
         hipLaunchKernelGGL(jq::s16_expand, dim3((unsigned)(2 * hg * ((nt + 3) / 4))), dim3(256), 0, stream, (const uint8_t *)s->wfrags,
@@ -105,8 +131,9 @@ bool split16_attention_fits(int d, int heads, int kv_heads) {
 int split16_attention(Split16Cache *c, const float *q, int q_stride, int T, int pos, const float *kc, const float *vc, int heads, int kv_heads,
                       int n_ctx, float *out, hipStream_t stream) {
     const size_t all = tiles_of((size_t)n_ctx);
-    if (!c->ws && !have((void **)&c->ws, (size_t)kv_heads * all * jq::S16_KV_TILE)) return -1;
-    if (!c->info && !have((void **)&c->info, (size_t)kv_heads * all * sizeof(jq::S16Tile))) return -1;
+    if (c->refused) return -1;
+    if (!c->ws && !have((void **)&c->ws, (size_t)kv_heads * all * jq::S16_KV_TILE, &c->refused)) return -1;
+    if (!c->info && !have((void **)&c->info, (size_t)kv_heads * all * sizeof(jq::S16Tile), &c->refused)) return -1;
     const int nt = (int)tiles_of((size_t)pos + T), g = heads / kv_heads, wh = std::min(g, 4);
     hipLaunchKernelGGL(jq::s16_kv_tiles, dim3((unsigned)nt, (unsigned)kv_heads), dim3(256), 0, stream, kc, vc, n_ctx, pos + T, c->ws, (jq::S16Tile *)c->info);
     HIP_TRY(hipGetLastError());

@@ -236,7 +236,7 @@ def test_a_token_that_is_not_finite_stays_out_of_those_in_front(at, value):
 
 
 def test_heads_in_groups_where_their_keys_and_values_exceed_the_buffer():
-    """256 heads of 4200 tokens are expanded in two groups (1 GiB of keys and values each at most).  The 256 are 32
+    """256 heads of 4200 tokens are expanded in three groups (512 MiB of keys and values each at most).  The 256 are 32
     copies of 8 and so are the output projection's columns: the sum is 32 times what the 8 alone give, up to the order of
     the additions."""
     c8 = cfg(n_embd=256, n_head=8, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=128, context_length=4224)
@@ -254,6 +254,20 @@ def test_heads_in_groups_where_their_keys_and_values_exceed_the_buffer():
     x = normal(16, (4200, 256))
     a, b = few.forward(x, 0), many.forward(x, 0) / 32
     assert np.abs(a - b).max() < 3e-4 * max(1.0, np.abs(a).max())
+
+
+def test_memory_of_an_object_over_a_long_context():
+    """Keys and values of 128 heads over 16384 positions would be 2 GiB, and 512 MiB are taken; beside them 130 MB of the
+    up-projection as f32 and as operands, 75 of the cache and its copy as operands, and 60 of scratch."""
+    import torch
+    w = {n: capi.Weight.upload(capi.Q8_0, quantized(capi.Q8_0, 910 + i, r, k), r, k)
+         for i, (n, r, k) in enumerate((("q", 128 * 192, 256), ("kv_a", 576, 256), ("kv_b", 32768, 512), ("o", 256, 16384)))}
+    mc = capi.MlaConfig(n_embd=256, n_head=128, q_lora_rank=0, kv_lora_rank=512, qk_nope_head_dim=128, qk_rope_head_dim=64,
+                        v_head_dim=128, n_ctx=16384, rms_eps=1e-6, rope_theta=1e4)
+    before = torch.cuda.mem_get_info()[0]
+    dev = capi.Mla(mc, w["q"], w["kv_a"], np.ones(512, np.float32), w["kv_b"], w["o"])
+    dev.forward(normal(21, (64, 256)), 0)
+    assert before - torch.cuda.mem_get_info()[0] < 900 << 20
 
 
 @pytest.mark.parametrize("n_head,vh,prompt", [(4, 64, 1), (4, 128, 300), (32, 128, 40), (32, 64, 700)])
