@@ -282,7 +282,7 @@ typedef struct {
  * of the two.  o_proj [n_embd, n_head*v].  The weights must outlive the object.
  * Device memory beside them: the cache, the up-projection in f32, and scratch that grows to the largest call (about
  * 4 KB a token, head and 512 of kv_lora_rank).  With DeepSeek's head sizes (128 + 64 queries, 128 values, 512 latents) also half a
- * megabyte a head, and from the first call of 48 tokens on 1 KB a position and head of
+ * megabyte a head, and from the first call of 48 tokens that is cheaper over expanded keys and values 1 KB a position and head of
  * the context, 512 MiB at most, and 2.3 KB a position; where there is none to be had, such calls run as the shorter ones do. */
 int jq_mla_create(const jq_mla_config *cfg, const jq_weight *q_or_q_a, const float *q_a_norm,
                   const jq_weight *q_b, const jq_weight *kv_a_mqa, const float *kv_a_norm,

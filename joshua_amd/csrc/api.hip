@@ -2316,12 +2316,23 @@ void mla_free_scratch(jq_mla *m) {
     m->cap_tokens = m->cap_absorbed = 0;
 }
 
-// Tokens from which a call expands the cached latents to keys and values per head instead of absorbing the up-projection
-// into its queries.  Expanding costs 33.5 M multiply-adds a cached token and layer of DeepSeek-V3's size however many tokens
-// the call has, and saves 98 k a pair of tokens.  Whole calls, us, absorbed / expanded: 32 tokens behind 0, 1000, 4000: 307 / 308,
-// 399 / 511, 654 / 1063; 48 tokens 481 / 409, 652 / 613, 1171 / 1165; 96 tokens 975 / 544, 1326 / 732, 2358 / 1290; 192
-// tokens 2430 / 957, 2962 / 1130, 4518 / 1845.
+// Whether a call expands the cached latents to keys and values per head instead of absorbing the up-projection into its queries:
+// from 48 tokens on (whole calls of DeepSeek-V3's size, us, absorbed / expanded: 32 tokens behind 0, 1000, 4000: 307 / 308,
+// 399 / 511, 654 / 1063; 48 tokens 481 / 409, 652 / 613), and there by the estimate of both.
 constexpr size_t MLA_EXPAND_TOKENS = 48;
+bool mla_expands(const jq_mla *m, size_t S, size_t pos) {
+    static const bool asked = getenv("JQ_MLA_ATTENTION") || getenv("JQ_MLA_SPLIT");  // for the absorbed form's kernels
+    return m->split16 && !asked && S >= MLA_EXPAND_TOKENS && split16_latent_pays(m->split16, S, pos);
+}
+
+// The largest call of up to S tokens that may be absorbed somewhere in the context: after a call of S, smaller ones find their
+// scratch there wherever they stand.  (Tried at some sizes and places; what falls between them is reserved when it comes.)
+size_t mla_absorbed_tokens(const jq_mla *m, size_t S) {
+    for (size_t t = S; t >= MLA_EXPAND_TOKENS; t -= std::max<size_t>(t / 16, 1))
+        for (size_t i = 0; i <= 16; i++)
+            if (!mla_expands(m, t, (m->cfg.n_ctx - t) * i / 16)) return std::min(S, t + t / 16);
+    return std::min(S, MLA_EXPAND_TOKENS);
+}
 
 // Scratch for calls of up to T tokens, of which up to `absorbed` in absorbed form.  Buffers that are outgrown are retired,
 // not freed: a HIP graph captured over an earlier, smaller call still names them, and they go with the object (jq_mla_free).
@@ -2463,12 +2474,12 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
                            (const float *)m->kv_a_norm, (const float2 *)m->cs, m->lat, m->kpe, (int)nh, (int)nope, (int)rope,
                            (int)lkv, (int)pos, c.rms_eps);
         HIP_TRY(hipGetLastError());
-        if (m->split16 && S >= MLA_EXPAND_TOKENS) {
+        if (mla_expands(m, S, pos)) {
             const int rc = split16_latent_attention(m->split16, m->qv, S, pos, m->lat, m->kpe, m->scale, m->ctx, s);
             if (rc > 0) return 1;
             if (rc == 0) return dispatch_matmul(m->o->type, m->o->dev, m->o->row_bytes, m->ctx, out, S, nh * vh, c.n_embd, s);
-            if (mla_reserve(m, S, S)) return 1;  // no memory for the expanded cache: the absorbed form
         }
+        if (S > m->cap_absorbed && mla_reserve(m, S, S)) return 1;
         // one token a workgroup in a decode step, four in a prefill; 16-byte loads when the latent width allows
         {
             const dim3 grid((unsigned)nh, (unsigned)((S + st - 1) / st));
@@ -2490,7 +2501,8 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
     // One token over a short context: waves of two heads and 16 tokens (a layer's step of 128 heads, us, matrix cores / this: behind
     // 4 tokens 51.3 / 44.6, 100 tokens 52.3 / 46.5, 230 tokens 53.4 / 49.9, 460 tokens 54.7 / 55.0, 950 tokens 59.5 / 68.1).
     constexpr size_t MLA_SHORT_CONTEXT = 320;
-    if (S == 1 && total <= MLA_SHORT_CONTEXT && !mla_env && lkv == jq::MLA_M_LKV && rope == jq::MLA_M_ROPE && nh % 8 == 0 && nope % 4 == 0) {
+    static const char *split_env = getenv("JQ_MLA_SPLIT");
+    if (S == 1 && total <= MLA_SHORT_CONTEXT && !mla_env && !split_env && lkv == jq::MLA_M_LKV && rope == jq::MLA_M_ROPE && nh % 8 == 0 && nope % 4 == 0) {
         n_split = (total + jq::MLA_SHORT_TOKENS - 1) / jq::MLA_SHORT_TOKENS;
         hipLaunchKernelGGL(jq::mla_attention_short, dim3((unsigned)(nh / 8), (unsigned)n_split), dim3(256), 0, s, (const float *)m->qabs,
                            (const float *)m->qv, (const float *)m->lat, (const float *)m->kpe, m->part, (int)nope, (int)total,
@@ -2501,7 +2513,6 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
         const size_t wgs = S * (nh / 32);
         n_split = std::min<size_t>({(256 + wgs - 1) / wgs, (total + 31) / 32, (size_t)jq::MLA_SPLIT_MAX,
                                     std::max<size_t>(MLA_PART_SLOTS / S, 1)});
-        static const char *split_env = getenv("JQ_MLA_SPLIT");
         if (split_env) n_split = std::min<size_t>(n_split, (size_t)atoi(split_env));
         n_split = std::max<size_t>(n_split, 1);
         hipLaunchKernelGGL(jq::mla_attention_mfma, dim3((unsigned)(nh / 32), (unsigned)n_split, (unsigned)S), dim3(512), 0, s,
@@ -2638,8 +2649,7 @@ int jq_mla_forward(jq_mla *m, size_t n_tokens, size_t pos, const float *x, float
     if (pos + n_tokens > m->cfg.n_ctx) return fail("jq_mla_forward: %zu + %zu tokens exceed the context of %u", pos, n_tokens, m->cfg.n_ctx);
     if (n_tokens > 0x7FFF) return fail("jq_mla_forward: at most 32767 tokens a call");
     hipStream_t s = (hipStream_t)stream;
-    // (a call that expands the cache leaves scratch for the absorbed ones below it too: they then allocate nothing)
-    if (mla_reserve(m, n_tokens, m->split16 ? std::min(n_tokens, MLA_EXPAND_TOKENS) : n_tokens)) return 1;
+    if (n_tokens > m->cap_tokens && mla_reserve(m, n_tokens, mla_absorbed_tokens(m, n_tokens))) return 1;
     const size_t bytes = n_tokens * m->cfg.n_embd * sizeof(float);
     if (ptrs_are_device) {
         if (mla_forward_dev(m, n_tokens, pos, x, out, s)) return 1;

@@ -51,6 +51,20 @@ static size_t latent_group(const Split16Latent *s, size_t nt) {
     return eights <= fit ? eights : even;
 }
 
+// Both sides in us, fitted to calls of 48 to 1024 tokens behind 0 to 32000 with 128 and 32 heads (within 10 %, the absorbed
+// form's vector kernel, for head counts that are no multiple of 32, within 25 %).  Expanded, a group of g heads: 0.0266 a tile and
+// head to expand and, a workgroup walking all tiles, 1.76 a tile while there is one to a compute unit.  128 heads, absorbed /
+// expanded in groups as here: 48 tokens behind 0, 4000, 8000, 16000: 139 / 32, 829 / 671, 1527 / 1690, 2924 / 5045; 128 tokens behind
+// 4000, 8000, 16000: 1707 / 718, 3105 / 1735, 5881 / 5112; 512 tokens behind 4000, 16000: 7016 / 1037, 23784 / 5423.
+bool split16_latent_pays(const Split16Latent *s, size_t S, size_t pos) {
+    const size_t nt = tiles_of(pos + S), g = latent_group(s, nt), nh = s->n_head;
+    if (g == 0 || s->refused) return false;
+    const double wgs = (double)(g * ((S + 127) / 128)), keys = (double)pos + (double)S / 2;
+    const double expanded = (double)((nh + g - 1) / g) * (20.0 + (double)nt * (1.76 * std::max(1.0, wgs / 233.0) + 0.0266 * (double)g));
+    const double walk = nh % 32 == 0 ? 0.174 * std::ceil((double)(S * nh) / (32 * 256)) : 0.27 * std::max(1.0, 0.75 * (double)(S * ((nh + 7) / 8)) / 256);
+    return expanded < 0.92 * (35.0 + 0.017 * (double)(S * nh) + walk * keys);  // (level with it: the form that needs no buffer)
+}
+
 int split16_latent_create(size_t n_head, size_t n_ctx, const float *wkv, const float *kv_norm, Split16Latent **out) {
     std::unique_ptr<Split16Latent, void (*)(Split16Latent *)> s(new Split16Latent{n_head, n_ctx}, split16_latent_free);
     float wmax = 0.0f;

@@ -256,6 +256,26 @@ def test_heads_in_groups_where_their_keys_and_values_exceed_the_buffer():
     assert np.abs(a - b).max() < 3e-4 * max(1.0, np.abs(a).max())
 
 
+def test_many_tokens_where_expanding_stops_paying():
+    """64 tokens of 128 heads behind 10000 others are absorbed again (keys and values of two groups of heads would be expanded,
+    each walked by half as many workgroups as there are compute units), and 64 behind 600 are not.  Columns of 32 copies of 4
+    heads, as above: against an object of those 4, which expands in both places."""
+    c4 = cfg(n_embd=256, n_head=4, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=128, context_length=10112)
+    t4, few = build(c4, seed=920)
+    raw = lambda name, rows: np.asarray(t4.t[name][1]).view(np.uint8).reshape(rows, -1)
+    w = {n: capi.Weight.upload(capi.Q8_0, np.ascontiguousarray(b), r, k)
+         for n, b, r, k in (("q", np.tile(raw("q", 768), (32, 1)), 128 * 192, 256), ("kv_a", raw("kv_a_mqa", 576), 576, 256),
+                            ("kv_b", np.tile(raw("kv_b", 1024), (32, 1)), 32768, 512), ("o", np.tile(raw("o", 256), (1, 32)), 256, 16384))}
+    mc = capi.MlaConfig(n_embd=256, n_head=128, q_lora_rank=0, kv_lora_rank=512, qk_nope_head_dim=128, qk_rope_head_dim=64,
+                        v_head_dim=128, n_ctx=10112, rms_eps=1e-6, rope_theta=1e4)
+    many = capi.Mla(mc, w["q"], w["kv_a"], t4.t["kv_a_norm"], w["kv_b"], w["o"])
+    x, pos = normal(22, (10112, 256)), 0
+    for n in (600, 64, 9384, 64):
+        a, b = few.forward(x[pos:pos + n], pos), many.forward(x[pos:pos + n], pos) / 32
+        assert np.abs(a - b).max() < 3e-4 * max(1.0, np.abs(a).max()), pos
+        pos += n
+
+
 def test_memory_of_an_object_over_a_long_context():
     """Keys and values of 128 heads over 16384 positions would be 2 GiB, and 512 MiB are taken; beside them 130 MB of the
     up-projection as f32 and as operands, 75 of the cache and its copy as operands, and 60 of scratch."""
