@@ -74,7 +74,7 @@ int moe_mx(const MoeSplit16Call &c, hipStream_t s) {
     auto *kernel = c.wb ? (many ? jq::moe_mx<true, 8, 4> : jq::moe_mx<true, 4, 2>) : (many ? jq::moe_mx<false, 8, 4> : jq::moe_mx<false, 4, 2>);
     hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles * a.cols)), dim3(64 * waves), 0, s, a);
     HIP_TRY(hipGetLastError());
-    note_kernel("moe_expert_dot8");  // (the route: bucketed, an expert's rows read once and its pairs taken past them)
+    note_kernel("moe_mx");
     return 0;
 }
 

@@ -368,7 +368,7 @@ def test_mxfp4_experts_on_the_matrix_cores_fp4(h, inter, E, k, tokens, shared_in
     x = synth.normal(910 + tokens, (tokens, h)) * np.float32(2.0) ** (np.arange(tokens) % 9 - 12)[:, None].astype(np.float32)
     ids, wts = dev.route(x)
     got = dev.forward(x)
-    assert capi.last_kernel() == "moe_expert_dot8"
+    assert capi.last_kernel() == "moe_mx"
 
     def deq(b, *shape):
         return oracle.dequantize(capi.MXFP4, b).reshape(shape).astype(np.float64)
