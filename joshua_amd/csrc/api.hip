@@ -693,31 +693,42 @@ int dispatch_gemm_i8(const uint8_t *W, size_t row_bytes, const float *X, float *
         const size_t mt = sh.nsplit ? 32 : 32 * (size_t)sh.nw, nt = 16 * (size_t)sh.ng;
         return ((m + mt - 1) / mt) * ((n + nt - 1) / nt);
     };
+    // Workgroups of a launch of that many tiles: rounded up to eights (the rest empty) where the row tiles divide 8, so that
+    // an XCD keeps to its column tiles.
+    auto grid_of = [&](const GemmI8Shape &sh) {
+        const size_t mt = sh.nsplit ? 32 : 32 * (size_t)sh.nw, ty = (m + mt - 1) / mt, t = tiles_of(sh);
+        return 8 % ty == 0 ? (t + 7) / 8 * 8 : t;
+    };
     if (tiles_of(shapes[2]) * std::max<size_t>(1, std::min<size_t>(nb / 4, 8)) < min_tiles) return -1;
     // Estimate per (shape, splits), in us, fitted to whole-call times of Q4_K products of 32 to 2048 rows
-    // against 1024 to 24576 weight rows of 4096 and 12288 columns (over 180 shapes of Q4_K and Q6_K the picks
-    // are 0.8 % off the best measured choice on average, 16 % at worst; Q6_K runs ~10 % longer with the same ordering): the preparation, a fixed part,
+    // against 1024 to 24576 weight rows of 4096 and 12288 columns (Q6_K runs ~10 % longer with the same ordering): the preparation, a fixed part,
     // the super-blocks a workgroup walks at a cost that grows with the workgroups at work (a large workgroup:
     // 5.0 us a super-block with 74 at work, 6.6 with 256; a small one: 2.5 with 64, 3.0 with 256, 4.7 when two
-    // share every compute unit), and the sum's launch and its (splits + 1) m n floats, which the last-level
-    // cache holds.
+    // share every compute unit), the starts of further rounds, and the sum's launch and its (splits + 1) m n floats, which the
+    // last-level cache holds.  Over 1321 shapes of Q4_K, Q6_K, Q8_0 and MXFP4 (9 to 2048 rows, 512 to 32000 x 1024 to 16384) the
+    // picks are 0.6 % off the best measured choice on average, 4 % at the 95th percentile, 19 % at worst.
     const size_t acts_bytes = (groups * nb * (size_t)jq::QI_REC + 255) & ~(size_t)255;
     const size_t scratch_cap = tl_fixed_scratch ? tl_fixed_scratch->bytes : (size_t)1 << 40;
-    // whole rounds of workgroups, then what is left at its own cost (a last round of half the workgroups or fewer is short:
-    // 333 x 12288 x 4096 of Q6_K in four parts, 768 workgroups of 128 x 64, 111 us; in three, 576 of them, 137)
+    // Whole rounds of workgroups, then what is left at its own cost (a last round of half the workgroups or fewer is short:
+    // 333 x 12288 x 4096 of Q6_K in four parts, 768 workgroups of 128 x 64, 111 us; in three, 576 of them, 137).  The empty
+    // workgroups count: they go to the last XCDs, and the first ones hold as many more (215 x 3910 x 8960 of Q8_0 as seven parts of 35
+    // tiles, 245 large workgroups in a grid of 280, 35 of them on an XCD's 32 compute units: 88 us; five parts of 41, 59).
     auto rounds = [](double wgs, double at_once, auto us) {
         const double whole = std::floor(wgs / at_once), rest = wgs - whole * at_once;
         return whole * us(at_once) + (rest > 0.0 ? us(rest) : 0.0);
     };
     auto estimate = [&](const GemmI8Shape &sh, size_t sp) {
-        const double wgs = (double)(tiles_of(sh) * sp), nbl = (double)(nb / sp);
+        const double wgs = (double)(grid_of(sh) * sp), nbl = (double)(nb / sp);
         double us = 3.0 + 0.0035 * (double)(nb * groups);
         if (sh.nsplit)  // 3.1 us a super-block with 64 at work, 3.4 with 256, 4.4 with 512 (two a compute unit), in whole rounds
             us += 3.9 + nbl * (2.95 + 0.0029 * std::min(wgs, 512.0)) *
                             (wgs <= 512.0 ? 1.0 : wgs < 2048.0 ? std::ceil(wgs / 512.0) : wgs / 512.0);
         else if (sh.nw == 8)  // (six groups of weight rows instead of seven: six sevenths of the work a super-block)
-            us += 10.0 + nbl * rounds(wgs, 256.0, [](double w) { return 4.3 + 0.009 * w; }) * (sh.ng == 7 ? 1.0 : 0.88);
-        else us += 3.9 + nbl * rounds(wgs, 512.0, [](double w) { return w <= 256.0 ? 2.3 + 0.0027 * w : 3.1 + 0.0032 * w; });
+            us += 10.0 + nbl * rounds(wgs, 256.0, [](double w) { return 4.3 + 0.009 * w; }) * (sh.ng == 7 ? 1.0 : 0.88) +
+                  6.0 * (std::ceil(wgs / 256.0) - 1.0);
+        else
+            us += 3.9 + nbl * rounds(wgs, 512.0, [](double w) { return w <= 256.0 ? 2.3 + 0.0027 * w : 3.1 + 0.0032 * w; }) +
+                  3.0 * std::max(0.0, wgs / 512.0 - 1.5);
         if (sp > 1) us += 1.0 + 0.8 * (double)sp + (double)(sp + 1) * (double)(m * n) * 4.0 / 8.0e6;
         return us;
     };
@@ -744,8 +755,7 @@ int dispatch_gemm_i8(const uint8_t *W, size_t row_bytes, const float *X, float *
     if (scratch.get(acts_bytes + (splits > 1 ? splits * m * n * sizeof(float) : 0), s, &acts)) return 1;
     float *parts = (float *)(acts + acts_bytes);
     const size_t mt = best->nsplit ? 32 : 32 * (size_t)best->nw, nt = 16 * (size_t)best->ng;
-    const size_t tx = (n + nt - 1) / nt, ty = (m + mt - 1) / mt;
-    const size_t grid = 8 % ty == 0 ? (tx * ty + 7) / 8 * 8 : tx * ty;
+    const size_t tx = (n + nt - 1) / nt, ty = (m + mt - 1) / mt, grid = grid_of(*best);
     if (grid > 0x7FFFFFFFull) return -1;
     hipError_t attr_rc = hipSuccess;
 #define JQ_GEMM_I8(NW_, NG_, NSPLIT_)                                                                                 \

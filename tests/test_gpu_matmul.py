@@ -1097,6 +1097,7 @@ KERNEL_OF_SHAPE = [  # which kernel serves the shapes the benchmarks quote: (for
     (capi.Q4_K, 16, 2048, 768, "q4k_stream_mfma"),
     (capi.Q4_K, 512, 4096, 14336, "q4k_gemm_i8"),           # 256 tiles of 256 x 112
     (capi.Q4_K, 128, 4096, 14336, "q4k_gemm_i8+splitk"),    # 224 tiles of 128 x 64, two splits
+    (capi.Q4_K, 333, 4096, 24576, "q4k_gemm_i8"),           # 1152 tiles of 128 x 64: no second part, whose sum costs more than it saves
     (capi.Q4_K, 128, 4096, 4096, "q4k_gemm_i8+splitk"),     # 64 tiles of 128 x 64: split over k
     (capi.Q4_K, 512, 4096, 1024, "q4k_gemm_i8+splitk"),
     (capi.Q4_K, 128, 4096, 256, "q4k_gemm_mfma+splitk"),    # a small product: the f16 kernel
