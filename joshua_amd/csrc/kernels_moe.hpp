@@ -548,8 +548,8 @@ static __global__ __launch_bounds__(GROUP_PAIRS_THREADS) void moe_group_pairs_ra
         const int chunk = wave + WAVES * c, pidx = 64 * chunk + lane;
         mine[c] = 0xFFFFFFFFu, rank[c] = 0;
         if (chunk >= chunks) continue;  // the same for the whole wave
-        const uint32_t e = pidx < P ? ids[pidx] : 0xFFFFFFFFu;
-        // the lanes that name this lane's expert: bit by bit, those that agree on it (a lane past the list agrees with its like only)
+        const uint32_t named = pidx < P ? ids[pidx] : 0xFFFFFFFFu, e = named < (uint32_t)E ? named : 0xFFFFFFFFu;
+        // the lanes that name this lane's expert: bit by bit, those that agree on it (a lane that names none agrees with its like only)
         uint64_t same = ~0ull;
         for (int b = 0; b < bits; b++) {
             const uint64_t set = __ballot((e >> b) & 1u);
