@@ -260,7 +260,11 @@ static __global__ __launch_bounds__(256) void moe_gate_topk(const float *__restr
         sum = (red[0] + red[1]) + (red[2] + red[3]);
         for (int e = lane; e < p.E; e += NT) probs[e] = probs[e] / sum;
     }
-    for (int e = lane; e < p.E; e += NT) sel[e] = probs[e] + (bias && !p.logit_bias() ? bias[e] : 0.0f);
+    // (a score that is not a number comes last: every slot below gets an expert, whatever the activations were)
+    for (int e = lane; e < p.E; e += NT) {
+        const float v = probs[e] + (bias && !p.logit_bias() ? bias[e] : 0.0f);
+        sel[e] = v == v ? v : -INFINITY;
+    }
     __syncthreads();
     if (p.n_group > 1) {
         const int per = p.E / p.n_group;

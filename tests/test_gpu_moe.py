@@ -400,6 +400,24 @@ def test_mxfp4_experts_on_the_matrix_cores_fp4(h, inter, E, k, tokens, shared_in
     assert np.array_equal(again[[0] + list(range(2, tokens - 1))], got[[0] + list(range(2, tokens - 1))])
 
 
+@pytest.mark.parametrize("tokens", [1, 3, 40, 200])
+def test_tokens_that_are_not_finite_under_expert_groups(tokens):
+    """Routing over groups of experts, on a layer that was never called: a token whose scores compare with nothing still gets
+    experts (scratch holds none from before), its own row alone is NaN, and the others are what they are without it."""
+    for seed in range(2):
+        ora, dev = build(capi.Q4_K, 512, 256, 32, 6, 710 + seed, gating="sigmoid", n_group=4, topk_group=2, weights_scale=2.5,
+                         router_bias=np.linspace(-0.05, 0.05, 32).astype(np.float32))
+        x = synth.normal(711 + seed, (tokens, 512))
+        bad = np.zeros(tokens, bool)
+        bad[[0, tokens // 2, tokens - 1][:max(1, tokens // 3)]] = True
+        x[bad, 17] = np.nan
+        got = dev.forward(x)
+        assert np.all(np.isnan(got[bad]))
+        assert bad.all() or close(got[~bad], ora.forward(x[~bad]))
+        ids, _ = dev.route(x)
+        assert ids.max() < 32
+
+
 @pytest.mark.parametrize("qtype", [capi.Q4_K, capi.MXFP4])
 def test_grouped_int8_gemm_with_pairs_that_fall_unevenly(qtype):
     """260 of 300 tokens route alike: two experts get 260 pairs and more (two tiles of 128 and a tail of tiles of 32),
