@@ -2048,6 +2048,9 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
                     ((uintptr_t)x & 15) == 0 && moe_mx_takes(c.inter, c.hidden, m->gate->row_bytes, a16, T) &&
                     m->down->type == JQ_TYPE_MXFP4 && moe_mx_takes(c.hidden, c.inter, m->down->row_bytes, d16, (size_t)P + (size_t)extra * T);
     if (mx) decode_sized = expert_dot8 = false;
+    // Q4_K, four pairs an expert or more: exact products of split f16 activations
+    const bool split16 = !decode_sized && split_room && m->gate->type == JQ_TYPE_Q4_K && same_gu && moe_split16_pays(c, T) && !expert_env &&
+                         ((uintptr_t)x & 15) == 0 && moe_split16_takes(c.hidden, m->gate->row_bytes, a16, T);
     bool planes_ready = false;
     jq::MoeGateIn gate_later{};
     if (decode_sized) {  // one group per pair, written by the gating kernel itself
@@ -2091,7 +2094,7 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
             uintptr_t bits = 0;
             for (const jq_weight *w : ws) bits |= w ? ((uintptr_t)w->dev | (uintptr_t)w->row_bytes) : 0;
             static const char *no_router_planes = getenv("JQ_MOE_NO_ROUTER_PLANES");
-            if (!no_router_planes && !expert_dot8 && m->gate->type == JQ_TYPE_Q4_K && m->up->type == JQ_TYPE_Q4_K &&
+            if (!no_router_planes && !expert_dot8 && !split16 && m->gate->type == JQ_TYPE_Q4_K && m->up->type == JQ_TYPE_Q4_K &&
                 m->gate->row_bytes == m->up->row_bytes && (size_t)P <= 6 * (size_t)c.n_expert &&
                 moe_q4k_quads_takes(m->qi8, m->gate->row_bytes, (bits & 15) ? 4 : 16, x, (int)c.hidden))
                 planes = m->qi8;
@@ -2118,9 +2121,7 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
                              c.hidden % 256 == 0 && c.inter % 256 == 0 && a16 >= 16 && d16 >= 16;
     // few pairs an expert, by the cost estimate above: the expert's rows decoded once, its pairs streamed past
     const bool multi = max_group > 1 && expert_dot8;
-    // Q4_K, four pairs an expert or more: exact products of split f16 activations
-    const bool split16 = max_group > 1 && split_room && m->gate->type == JQ_TYPE_Q4_K && moe_split16_pays(c, T) && !expert_env;
-    if (same_gu && split16 && ((uintptr_t)x & 15) == 0 && moe_split16_takes(c.hidden, m->gate->row_bytes, a16, T))
+    if (split16)
         rc = moe_split16({m->pgate, m->pup, m->gate->row_bytes, x, T, m->gexp, m->offsets, m->xrow, m->yrow, groups, (size_t)P + (size_t)extra * T,
                           m->G, c.hidden, c.inter, clamp, m->split_acts}, s);
     if (mx)
