@@ -190,16 +190,30 @@ def test_prefill_of_many_tokens_with_4096_wide_rows(mix):
 
 
 @pytest.mark.parametrize("n_head,n_kv", [(4, 1), (4, 2), (2, 2), (8, 1)])
-def test_long_prefill_chunks_split_their_keys_between_two_sets_of_waves(n_head, n_kv):
-    """From 128 keys on the tiled attention gives the key tiles of even and odd number to two sets of waves
-    and merges their running softmax states (up to four query heads a KV head; eight keep one set): a chunk
-    from position 0, chunks that start inside a key tile, an odd number of key tiles, a last tile part empty."""
+def test_long_prefill_chunks(n_head, n_kv):
+    """Attention on split f16 operands with four, two, one and eight query heads a KV head: a chunk from position 0, chunks
+    that start inside a key tile, an odd number of key tiles, a last tile part empty."""
     cfg = dict(CFG, n_ctx=400, n_layer=2, head_dim=128, n_head=n_head, n_kv_head=n_kv)
     m, o = make(cfg, 33)
     rng = np.random.default_rng(14)
     toks = [int(t) for t in rng.integers(0, cfg["vocab"], size=390)]
     pos = 0
     for step in (137, 150, 9, 94):
+        chunk = toks[pos:pos + step]
+        ok, e = close(m.forward(chunk, pos), o.forward(chunk, pos))
+        assert ok, f"pos {pos} +{step}: {e}"
+        pos += step
+
+
+@pytest.mark.parametrize("n_head,n_kv", [(4, 1), (4, 2), (2, 2), (8, 1)])
+def test_short_prefill_chunks(n_head, n_kv):
+    """Steps of 9 to 31 tokens below 128 keys, on the f32 matrix cores with the same head counts: whole and part tiles of 16
+    tokens and keys, up to the line from which the split operands take over and one step past it."""
+    cfg = dict(CFG, n_ctx=160, n_layer=2, head_dim=128, n_head=n_head, n_kv_head=n_kv)
+    m, o = make(cfg, 34)
+    toks = [int(t) for t in np.random.default_rng(16).integers(0, cfg["vocab"], size=160)]
+    pos = 0
+    for step in (9, 16, 31, 17, 24, 30, 20):
         chunk = toks[pos:pos + step]
         ok, e = close(m.forward(chunk, pos), o.forward(chunk, pos))
         assert ok, f"pos {pos} +{step}: {e}"
