@@ -9,7 +9,7 @@ namespace {
 
 size_t tiles_of(size_t tokens) { return (tokens + jq::S16_TILE - 1) / jq::S16_TILE; }
 
-// hipMalloc that leaves no error behind; `refused` is set where there is no memory (and not under a stream's capture, say).
+// hipMalloc that leaves no error behind; `refused` is set where there is no memory.
 bool have(void **p, size_t bytes, bool *refused) {
     const hipError_t e = hipMalloc(p, bytes);
     if (e == hipSuccess) return true;
@@ -96,6 +96,12 @@ int split16_latent_attention(Split16Latent *s, const float *q, size_t S, size_t 
     const size_t all = tiles_of(s->n_ctx), nt = tiles_of(pos + S);
     if (s->refused) return -1;
     if (!s->ws) {
+        // nothing can be allocated while the stream is captured: this call is absorbed, and a later one asks
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            return -1;
+        }
         size_t want = latent_ws_bytes(s);
         bool none = false;
         const bool rest = (s->cf || have((void **)&s->cf, all * (jq::S16_LKV / 16) * 2 * jq::S16_FRAG, &s->refused)) &&

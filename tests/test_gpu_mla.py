@@ -276,6 +276,44 @@ def test_many_tokens_where_expanding_stops_paying():
         pos += n
 
 
+def test_a_capture_of_the_first_call_that_would_expand():
+    """64 tokens of 128 heads behind 10000 others are absorbed, so an object that has seen only such calls and shorter ones holds no
+    buffer for expanded keys and values, and none can be had while a graph is captured: 64 tokens at the front are then absorbed
+    too.  The graph replays to what an object of 4 of the heads gives (columns of 32 copies, as above), with eager work between."""
+    import torch
+    c4 = cfg(n_embd=256, n_head=4, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=128, context_length=10112)
+    t4, few = build(c4, seed=930)
+    raw = lambda name, rows: np.asarray(t4.t[name][1]).view(np.uint8).reshape(rows, -1)
+    w = {n: capi.Weight.upload(capi.Q8_0, np.ascontiguousarray(b), r, k)
+         for n, b, r, k in (("q", np.tile(raw("q", 768), (32, 1)), 128 * 192, 256), ("kv_a", raw("kv_a_mqa", 576), 576, 256),
+                            ("kv_b", np.tile(raw("kv_b", 1024), (32, 1)), 32768, 512), ("o", np.tile(raw("o", 256), (1, 32)), 256, 16384))}
+    mc = capi.MlaConfig(n_embd=256, n_head=128, q_lora_rank=0, kv_lora_rank=512, qk_nope_head_dim=128, qk_rope_head_dim=64,
+                        v_head_dim=128, n_ctx=10112, rms_eps=1e-6, rope_theta=1e4)
+    many = capi.Mla(mc, w["q"], w["kv_a"], t4.t["kv_a_norm"], w["kv_b"], w["o"])
+    x = torch.from_numpy(normal(23, (64, 256))).cuda()
+    y = torch.zeros(64, 256, device="cuda")
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        for n in [40] * 250 + [64]:
+            many.forward_dev(n, many.cached_tokens, x.data_ptr(), y.data_ptr(), stream.cuda_stream)
+        stream.synchronize()
+        many.reset()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            many.forward_dev(64, 0, x.data_ptr(), y.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        want = few.forward(x.cpu().numpy(), 0)
+        for rep in range(3):
+            y.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            got = y.cpu().numpy() / 32
+            assert np.abs(got - want).max() < 3e-4 * max(1.0, np.abs(want).max()), rep
+    del graph
+    torch.cuda.synchronize()
+    capi.stream_release(stream.cuda_stream)
+
+
 def test_memory_of_an_object_over_a_long_context():
     """Keys and values of 128 heads over 16384 positions would be 2 GiB, and 512 MiB are taken; beside them 130 MB of the
     up-projection as f32 and as operands, 75 of the cache and its copy as operands, and 60 of scratch."""
