@@ -2920,10 +2920,11 @@ bool model_norm_mm(const jq_weight *w, const float *x, const float *res, const f
 }
 
 // Steps whose attention runs on split f16 operands (kernels_split16.hpp) instead of the f32 matrix cores.  Below, the copy of
-// the cache into operands, a launch more, eats what it gains.  Whole steps of four layers of Qwen3-8B's sizes, us, f32 / split:
-// 9 tokens 463 / 468, 16 tokens 501 / 504, 32 tokens 675 / 664, 256 tokens 1414 / 1318; behind 1000 tokens 9 tokens 840 / 678,
-// 256 tokens 1794 / 1517; behind 4000 tokens 9 tokens 1973 / 1237.
-bool split16_attention_pays(uint32_t T, uint32_t pos) { return T >= 32 || pos + T >= 128; }
+// the cache into operands, a launch more, eats what it gains (33 tokens, us a layer: 10.6 / 5.4 + 8.3; 64: 14.8 / 5.0 + 9.8).  Whole
+// steps of four layers of Qwen3-8B's sizes, us, f32 / split: 32 tokens 686 / 704, 48 tokens 844 / 851, 64 tokens 898 / 900, 80 tokens
+// 964 / 954, 112 tokens 946 / 920, 256 tokens 1414 / 1318; behind 1000 tokens 9 tokens 840 / 678, 256 tokens 1794 / 1517; behind
+// 4000 tokens 9 tokens 1973 / 1237.  Where heads are grouped as no f32 kernel takes them (`tiled` false) the line is 32 tokens.
+bool split16_attention_pays(uint32_t T, uint32_t pos, bool tiled) { return T >= (tiled ? 64u : 32u) || pos + T >= 128; }
 
 int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *want, uint32_t n_want, hipStream_t s) {
     const jq_qwen3_config &c = m->cfg;
@@ -3010,15 +3011,16 @@ int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *w
             static const char *no_tiles = getenv("JQ_NO_ATTENTION_TILES");
             const int gq = nh / nkv;
             const dim3 tgrid((unsigned)((T + 15) / 16), (unsigned)nkv);
+            const bool tiled = d == 128 && (gq == 1 || gq == 2 || gq == 4 || gq == 8);
             int done = -1;
-            if (split16_attention_pays(T, pos) && !no_tiles && split16_attention_fits(d, nh, nkv))
+            if (split16_attention_pays(T, pos, tiled) && !no_tiles && split16_attention_fits(d, nh, nkv))
                 done = split16_attention(&m->split16, qp, q_stride, (int)T, (int)pos, m->kc[l], m->vc[l], nh, nkv, (int)c.n_ctx, m->att, s);
             if (done > 0) return 1;
 #define JQ_ATT_TILES(GQ)                                                                                          \
     hipLaunchKernelGGL((jq::attention_tiles<128, GQ>), tgrid, dim3(64 * GQ), 0, s, qp, m->kc[l], m->vc[l], m->att,   \
                        (int)T, nh, m->pos, (int)c.n_ctx, sqrt_d, q_stride)
             if (done == 0) {
-            } else if (no_tiles || d != 128 || (gq != 1 && gq != 2 && gq != 4 && gq != 8)) {
+            } else if (no_tiles || !tiled) {
                 size_t sm = ((size_t)d + jq::AR_CHUNK + 16) * sizeof(float);
                 hipLaunchKernelGGL(jq::attention_rows, dim3(T * nh), dim3(256), sm, s, qp, m->kc[l], m->vc[l], m->att, nh,
                                    nkv, d, m->pos, (int)c.n_ctx, sqrt_d, q_stride);

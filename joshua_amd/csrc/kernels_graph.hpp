@@ -175,7 +175,7 @@ static __global__ __launch_bounds__(256) void attention_rows(const float *__rest
 // P V as it stands when the product's inner index g stands for key 4 g + j in step j on both sides; the
 // outputs come out as O[token 4 g + j][dimension], so a token's rescaling factor is fetched from the lane
 // that holds its statistics.  Scores are divided by sqrt(d) as the reference does (src/embedding.rs:386).
-// Steps of 32 tokens or 128 keys and more run on split f16 operands instead (kernels_split16.hpp).
+// Steps of 64 tokens or 128 keys and more run on split f16 operands instead (kernels_split16.hpp).
 constexpr int AT_PAD = 4;  // floats a staged row is longer than D: 16 rows then fall into different banks
 
 template <int D, int G>

@@ -220,10 +220,11 @@ def test_short_prefill_chunks(n_head, n_kv):
         pos += step
 
 
-@pytest.mark.parametrize("n_head,n_kv,steps", [(8, 2, (32, 31, 64, 9, 8, 96)), (8, 8, (129, 33)), (16, 1, (160, 40)), (12, 6, (127, 128, 1)), (20, 4, (40, 60))])
+@pytest.mark.parametrize("n_head,n_kv,steps", [(8, 2, (32, 31, 64, 9, 8, 96)), (8, 2, (63, 64, 9)), (8, 2, (64, 63, 9)),
+                                                (8, 8, (129, 33)), (16, 1, (160, 40)), (24, 2, (32, 31, 40)), (12, 6, (127, 128, 1)), (20, 4, (40, 60))])
 def test_attention_of_many_tokens_over_values_of_different_size(n_head, n_kv, steps):
-    """Steps on both sides of the line from which attention runs on split f16 operands (32 tokens, or 128 keys), with 4, 1,
-    16, 2 and 5 query heads a KV head (the last on the general kernel), part tiles of keys and tokens.  Every third token's
+    """Steps on both sides of the line from which attention runs on split f16 operands (64 tokens, or 128 keys; with 12 and 16
+    heads a KV head 32 tokens), with 4, 1, 16, 12, 2 and 5 query heads a KV head (the last on the general kernel), part tiles of keys and tokens.  Every third token's
     values are some 200 times the others', and the first 40 tokens hold none of those: the value tiles' scales differ."""
     cfg = dict(CFG, n_ctx=256, n_layer=2, head_dim=128, n_head=n_head, n_kv_head=n_kv, hidden=256, vocab=600)
     rng = np.random.default_rng(n_head)
