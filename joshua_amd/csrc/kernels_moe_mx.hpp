@@ -107,8 +107,8 @@ struct MoeMx {
 // The chunks of all blocks are one stream: asynchronous loads bring a chunk of the wave's rows (contiguous 16-byte pieces; read
 // straight into operands, each lane touches a cache line of its own, five lookups for its 68 bytes: 1330 us the layer below)
 // into a slot in LDS that is free again as soon as its words are in registers, and the digits of the pairs, gathered, into two buffers.
-// Bound: memory.  DeepSeek-V3's size, 64 tokens (222 of 256 experts and the shared one, 5.24 GB): the layer 1061 us, 4.9 TB/s of
-// weights over the whole call where a large copy moves 5.1 (on the int8 kernels 2004).  At 512 tokens 1.9 ms (3.9): the digits
+// Bound: memory.  DeepSeek-V3's size, 64 tokens (222 of 256 experts and the shared one, 5.24 GB): the layer 1058 us, 4.9 TB/s of
+// weights over the whole call where a large copy moves 5.1 (on the int8 kernels 2016).  At 512 tokens 1.9 ms (3.9): the digits
 // cost four columns a pair, and tiles of 16 pairs are read again from the second level cache.
 template <bool DUAL, int WAVES, int NG, int MAXNG>
 __device__ __forceinline__ void moe_mx_tile(const MoeMx &a, int expert, int beg, int cnt, int cb0, uint8_t *lds, int *y_lds) {

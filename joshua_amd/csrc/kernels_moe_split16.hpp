@@ -85,10 +85,10 @@ struct MoeSplit16 {
 
 // A workgroup of four waves multiplies a tile of up to 48 pairs of one expert with 64 WT weight rows (DUAL: half gate rows, half
 // the up rows of the same columns, the gated unit in the epilogue); a wave owns WT tiles of 16 rows, RG row groups of 16 pairs.
-// Bound: the issue of matrix and vector instructions, which hardly overlap (a wave of WT = 4 and RG = 3 issues 204 MFMAs of 16 cycles
-// and ~560 vector instructions of 4 a super-block: that alone is 84 of gate and up's 141 us at 128 experts of 768 x 2048 and 512
-// tokens, the rest workgroups that do not divide evenly among the compute units, and their starts); the int8 GEMM took 3 x 102 us for
-// the three products where these take 141 + 68.
+// Bound: the issue of matrix and vector instructions, which hardly overlap, then what the workgroups wait for at their starts and
+// between halves: at 128 experts of 768 x 2048 and 512 tokens (32 pairs an expert) the counters show 25 % of the compute units' busy
+// cycles in matrix instructions (16 cycles each) and 28 % in vector instructions (4 cycles each), in gate and up as in down.  The
+// int8 GEMM took 3 x 102 us for the three products where these take 138 + 68.
 template <bool DUAL, int RG, int WT>
 __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert, int beg, int cnt, int cb, uint8_t *lds, float *s_lds,
                                                  int *y_lds) {

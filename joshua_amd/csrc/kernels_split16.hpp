@@ -17,11 +17,12 @@
 // 4 (l / 32) + r % 4 of register r): running maximum, sum and the output's rescaling stay in the lane, and the
 // weights are the second operand of O^T += V^T P^T as they stand, the keys of V's fragments in that same order.
 //
-// Bound: the matrix cores (40 % busy), then the LDS reads of a tile by each of the four waves.  Measured against the f32 matrix
-// cores' kernels: the decoder's attention of 2048 tokens, 32 / 8 heads of 128, 606 -> 137 us a layer (751 TFLOP/s of f16
-// products); latent attention of DeepSeek-V3's size, 512 tokens behind 0 .. 3584 (on average): 3060 us of attention on the
-// absorbed queries, 645 of value projection, 208 of absorption, 122 of merging -> 247 us of expanding, 287 of attention
-// and 9 of preparation.  Against 64-bit results the errors of both are the same (1.0e-4 and 1.5e-4 of the norm, the 16-bit
+// Bound: the matrix cores (by counters 50 % of the compute units' busy cycles in the decoder's attention and in the expansion, 54 in
+// latent attention; no bank conflicts), then the LDS reads of a tile by each of the four waves.  Measured against the f32 matrix
+// cores' kernels: the decoder's attention of 2048 tokens, 32 / 8 heads of 128, 606 -> 129 us a layer (796 TFLOP/s of f16
+// products) and 10 of preparation; latent attention of DeepSeek-V3's size, 512 tokens behind 0 .. 3584 (on average): 3060 us of
+// attention on the absorbed queries, 645 of value projection, 208 of absorption, 122 of merging -> 249 us of expanding, 273 of
+// attention and 10 of preparation.  Against 64-bit results the errors of both are the same (1.0e-4 and 1.5e-4 of the norm, the 16-bit
 // activations of the products around them).
 #pragma once
 #include "split16_parts.hpp"
