@@ -2121,9 +2121,10 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
                              c.hidden % 256 == 0 && c.inter % 256 == 0 && a16 >= 16 && d16 >= 16;
     // few pairs an expert, by the cost estimate above: the expert's rows decoded once, its pairs streamed past
     const bool multi = max_group > 1 && expert_dot8;
+    const bool few_pairs = (size_t)P < 16 * (size_t)c.n_expert;
     if (split16)
         rc = moe_split16({m->pgate, m->pup, m->gate->row_bytes, x, T, m->gexp, m->offsets, m->xrow, m->yrow, groups, (size_t)P + (size_t)extra * T,
-                          m->G, c.hidden, c.inter, clamp, m->split_acts}, s);
+                          m->G, c.hidden, c.inter, clamp, m->split_acts, few_pairs}, s);
     if (mx)
         rc = moe_mx({m->pgate, m->pup, m->gate->row_bytes, x, T, m->gexp, m->offsets, m->xrow, m->yrow, groups, (size_t)P + (size_t)extra * T,
                      m->G, c.hidden, c.inter, clamp, m->split_acts}, s);
@@ -2197,7 +2198,7 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
     rc = -1;
     if (split_gu && m->down->type == JQ_TYPE_Q4_K && moe_split16_down_pays(c) && moe_split16_takes(c.inter, m->down->row_bytes, d16, (size_t)P + (size_t)extra * T))
         rc = moe_split16({m->pdown, nullptr, m->down->row_bytes, m->G, (size_t)P + (size_t)extra * T, m->gexp, m->offsets, m->yrow, m->yrow, groups,
-                          (size_t)P + (size_t)extra * T, m->out, c.inter, c.hidden, clamp, m->split_acts}, s);
+                          (size_t)P + (size_t)extra * T, m->out, c.inter, c.hidden, clamp, m->split_acts, few_pairs}, s);
     if (split_gu && mx)
         rc = moe_mx({m->pdown, nullptr, m->down->row_bytes, m->G, (size_t)P + (size_t)extra * T, m->gexp, m->offsets, m->yrow, m->yrow, groups,
                      (size_t)P + (size_t)extra * T, m->out, c.inter, c.hidden, clamp, m->split_acts}, s);

@@ -22,7 +22,7 @@
 namespace jq {
 
 constexpr int MS16_PLANES = 1024, MS16_XS = 32;  // bytes a row and super-block: hi and lo of 256 elements; of 8 sums
-constexpr int MS16_RG = 3;                        // row groups of 16 a tile holds
+constexpr int MS16_RG = 3;                        // row groups of 16 a tile holds at most
 constexpr int MS16_ROWS = 16 * MS16_RG;
 constexpr int MS16_MAX_NB = 32;                   // super-blocks of a row (the scales of a tile wait in LDS)
 // weight rows of a workgroup whose waves take WT tiles of 16 each (DUAL: half of them gate rows, half up rows)
@@ -80,6 +80,7 @@ struct MoeSplit16 {
     const int *gexp, *offsets, *xsel, *yrow;  // groups' experts, first pairs; a pair's activation row and result row
     float *Y;
     int groups, n, nb, cols;                // cols: column blocks of the grid
+    int rows;                               // pairs of a tile, 32 or 48
     MoeClamp clamp;
 };
 
@@ -133,12 +134,20 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
 #pragma unroll
         for (int w = 0; w < WT; w++) q[w] = *(const uint4 *)(wp[w] + (size_t)sb * 144 + 16 + 64 * hs + 16 * g);
     };
-    s16_f4 acc[WT][RG], i1[WT][RG];
+    // The products with the low plane in sums of their own, where registers are left: eight matrix instructions instead of 16 then
+    // round a sum of the super-block's size.  128 experts of 2048 x 768, 6 to 16 pairs each: the layer's error against 64 bits
+    // 7.3e-7 -> 5.9e-7 (the f32 products of the ring kernel 6.3e-7), its time, with tiles of 32 pairs there, 150 tokens 160.7 -> 162.5 us,
+    // 250 tokens 183.8 -> 187.1.  Three row groups keep one chain.
+    constexpr bool APART = RG <= 2;
+    s16_f4 acc[WT][RG], i1[WT][RG], low[APART ? WT : 1][APART ? RG : 1];
     const s16_f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < WT; w++)
 #pragma unroll
-        for (int r = 0; r < RG; r++) acc[w][r] = i1[w][r] = zero;
+        for (int r = 0; r < RG; r++) {
+            acc[w][r] = i1[w][r] = zero;
+            if constexpr (APART) low[w][r] = zero;
+        }
     // (masks and magic numbers in registers: v_and_or_b32 takes one scalar operand and no two literals)
     uint32_t m_lo = 0x000F000Fu, m_hi = 0x00F000F0u, o_lo = 0x64006400u, o_hi = 0x54005400u;
     asm("" : "+s"(m_lo), "+s"(m_hi), "+v"(o_lo), "+v"(o_hi));
@@ -173,7 +182,10 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
                     for (int r = 0; r < RG; r++) {
                         const s16_h8 x = *(const s16_h8 *)(l + ((r * 4 + 2 * nib + s8) * 2 + p) * S16_FRAG);
 #pragma unroll
-                        for (int w = 0; w < WT; w++) i1[w][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, b[s8][w], i1[w][r], 0, 0, 0);
+                        for (int w = 0; w < WT; w++) {
+                            s16_f4 &to = APART && p ? low[APART ? w : 0][APART ? r : 0] : i1[w][r];
+                            to = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, b[s8][w], to, 0, 0, 0);
+                        }
                     }
         }
     };
@@ -234,6 +246,7 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
 #pragma unroll
             for (int r = 0; r < RG; r++) {
                 const s16_f4 i2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xs[r], mins, zero, 0, 0, 0);
+                if constexpr (APART) i1[w][r] += low[w][r], low[w][r] = zero;
 #pragma unroll
                 for (int i = 0; i < 4; i++) acc[w][r][i] = fmaf(s[r][i], fmaf(dm, i2[i], d * i1[w][r][i]), acc[w][r][i]);
                 i1[w][r] = zero;
@@ -284,8 +297,8 @@ static __global__ __launch_bounds__(256, WT == 2 ? 3 : 2) void moe_split16(MoeSp
     int *y_lds = (int *)(s_lds + MS16_ROWS * a.nb);
     const int id = blockIdx.x, mt = id / (8 * a.cols) * 8 + id % 8, cb = id / 8 % a.cols;
     int grp, at;
-    if (!s16_find_tile(a.offsets, a.groups, MS16_ROWS, mt, grp, at)) return;  // past the last tile: the whole workgroup
-    const int beg = a.offsets[grp] + at, cnt = min(a.offsets[grp + 1] - beg, MS16_ROWS), expert = a.gexp[grp];
+    if (!s16_find_tile(a.offsets, a.groups, a.rows, mt, grp, at)) return;  // past the last tile: the whole workgroup
+    const int beg = a.offsets[grp] + at, cnt = min(a.offsets[grp + 1] - beg, a.rows), expert = a.gexp[grp];
     if (cnt <= 16) moe_split16_tile<DUAL, 1, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds);
     else if (cnt <= 32) moe_split16_tile<DUAL, 2, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds);
     else moe_split16_tile<DUAL, 3, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds);

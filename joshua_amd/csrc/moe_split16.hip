@@ -29,7 +29,10 @@ int moe_split16(const MoeSplit16Call &c, hipStream_t s) {
     const int wt = c.pairs < (c.wb ? 48 : 16) * (size_t)c.groups ? 2 : 4;
     const size_t per = jq::moe_split16_cols(wt) / (c.wb ? 2 : 1);
     a.cols = (int)((c.n + per - 1) / per);
-    const size_t tiles = (c.pairs / jq::MS16_ROWS + (size_t)c.groups + 7) / 8 * 8;
+    // Calls of fewer than 16 pairs an expert, which the ring kernel's f32 products would run, take two row groups a tile at most,
+    // also of an expert with more pairs: those keep the products with the low plane apart (see moe_split16_tile).
+    a.rows = c.few ? 32 : jq::MS16_ROWS;
+    const size_t tiles = (c.pairs / (size_t)a.rows + (size_t)c.groups + 7) / 8 * 8;
     if (tiles * a.cols > 0x7FFFFFFFull) return -1;
     hipLaunchKernelGGL(jq::moe_split16_prep, dim3((unsigned)c.x_rows, (unsigned)((nb + 3) / 4)), dim3(256), 0, s, c.X, (int)c.k, a.acts);
     const int lds = jq::moe_split16_lds((int)nb);

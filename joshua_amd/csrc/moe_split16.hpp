@@ -18,6 +18,7 @@ struct MoeSplit16Call {
     size_t k, n;
     jq::MoeClamp clamp;
     uint8_t *acts;                          // moe_split16_bytes(x_rows, k), or moe_mx_bytes
+    bool few = false;                       // (moe_split16) fewer than 16 routed pairs an expert
 };
 size_t moe_split16_bytes(size_t rows, size_t k);
 bool moe_split16_takes(size_t k, size_t row_bytes, int base_align, size_t rows);

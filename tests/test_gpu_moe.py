@@ -315,6 +315,36 @@ def test_q4k_experts_on_split_f16_activations(h, inter, E, k, tokens, shared_int
     assert close(dev.forward(few), ora.forward(few))
 
 
+@pytest.mark.parametrize("alike", [0, 40])
+def test_q4k_experts_on_split_f16_activations_against_64_bits(alike):
+    """Ten pairs an expert, the calls that the ring kernel's f32 products ran before: no further from 64 bits than those.  The
+    activations' 22 to 23 bits are 4e-8 of a product; the rest are the roundings of the f32 sums, fewer where the products with the
+    low plane have sums of their own.  Norm of the error here: 5.9e-7, in one chain 7.3e-7; the ring kernel's, at 128
+    experts of 2048 x 768, 6.3e-7."""
+    h, inter, E, k, T = 2048, 512, 64, 8, 80
+    ora, dev = build(capi.Q4_K, h, inter, E, k, 640)
+    x = synth.normal(641, (T, h))
+    x[:alike] = x[0] + np.float32(0.05) * x[:alike]                    # experts of 40 pairs and more beside others of a few
+    got = dev.forward(x)
+    assert capi.last_kernel() == "moe_split16"
+    ids = np.asarray(dev.route(x)[0]).reshape(T, k)
+    rows = [oracle.dequantize(capi.Q4_K, synth.normal_quantized(capi.Q4_K, 641 + i, E * inter * h, 0.02)).reshape(E, n, kk)
+            for i, (n, kk) in enumerate(((inter, h), (inter, h), (h, inter)))]
+    x = x.astype(np.float64)
+    z = x @ synth.normal(640, (E, h), sigma=0.02).astype(np.float64).T
+    want = np.zeros((T, h))
+    top = np.take_along_axis(z, ids.astype(np.int64), 1)
+    wts = np.exp(top - top.max(1, keepdims=True))
+    wts /= wts.sum(1, keepdims=True)
+    for e in range(E):
+        t, slot = np.nonzero(ids == e)
+        g, u, d = (r[e].astype(np.float64) for r in rows)
+        a = x[t] @ g.T
+        want[t] += wts[t, slot, None] * ((a / (1.0 + np.exp(-a)) * (x[t] @ u.T)) @ d.T)
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert err < 6.4e-7, err
+
+
 def test_q4k_experts_on_split_f16_activations_uneven_rows_and_non_finite_ones():
     """300 of 400 tokens route alike (experts with seven tiles, with one, and with none), one token holds a NaN and one an
     infinity: their rows come out NaN and nobody else's; the same layer with a down projection that the int8 GEMM runs."""
