@@ -22,6 +22,7 @@
 #include "kernels_moe_q4k_quads.hpp"
 #include "kernels_mfma_q4k_rows16.hpp"
 #include "kernels_mfma_q4k_gemm_i8.hpp"
+#include "kernels_mfma_gemm_h6.hpp"
 #include "kernels_valu.hpp"
 #include "kernels_mfma_decoded.hpp"
 
@@ -794,6 +795,106 @@ int dispatch_gemm_i8(const uint8_t *W, size_t row_bytes, const float *X, float *
     return 0;
 }
 
+// Leave to use that much LDS, asked for once a kernel.
+template <auto KERN>
+hipError_t big_lds_once(int lds) {
+    static const hipError_t rc = hipFuncSetAttribute((const void *)KERN, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    return rc;
+}
+
+// Q4_K with 128 activation rows or more on f16 and FP6 operands (kq_gemm_h6): 512 x 14336 x 4096 99 us against the int8 GEMM's
+// 127, 2048 x 24576 x 4096 577 against 732, 512 x 4096 x 4096 50 against 52 (whole calls; 50
+// shapes of 128 to 2048 rows, 0.77 to 1.01 of the int8 GEMM's time).  Below 128 rows the int8 GEMM is as fast (64 to 127 rows:
+// 0.90 to 1.07) and keeps them: there unpacking the weights is most of the work in both.  `name` is the route's, the one that
+// callers of jq_last_kernel know the many-row product by, whichever arithmetic it runs on.
+// Returns -1 when the shape is outside its reach, where a fixed scratch holds the int8 GEMM's records but not these (12352 bytes
+// for 16 rows of 256 against 9280), and where the environment names a shape or a switch of that GEMM.  JQ_GEMM_H6 = 0
+// switches this one off, JQ_GEMM_H6_SHAPE and _SPLITS force the choice, _MIN_M moves the fewest rows.
+template <class F>
+int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n,
+                     hipStream_t s, const char *name, const char *name_split, bool swiglu_pairs = false) {
+    static const char *mode = getenv("JQ_GEMM_H6"), *i8_mode = getenv("JQ_Q4K_GEMM_I8"), *i8_shape = getenv("JQ_Q4K_GEMM_I8_SHAPE");
+    static const char *shape_env = getenv("JQ_GEMM_H6_SHAPE"), *splits_env = getenv("JQ_GEMM_H6_SPLITS");
+    static const char *min_m_env = getenv("JQ_GEMM_H6_MIN_M");
+    static const size_t min_m = min_m_env ? std::max<size_t>((size_t)atoll(min_m_env), 2) : 128;
+    if ((mode && mode[0] == '0') || i8_mode || i8_shape || m < min_m || k % 256 != 0 || k == 0 || row_bytes % 16 != 0 ||
+        row_bytes > ((size_t)1 << 27) || ((uintptr_t)W & 15) != 0 || ((uintptr_t)X & 15) != 0 || m > 0x7FFFFFF0ull || n > 0x7FFFFFF0ull)
+        return -1;
+    struct Shape {
+        int nw, ng;
+    };
+    static const Shape shapes[] = {{8, 7}, {8, 6}, {4, 4}};
+    const size_t nb = k / 256, groups = (m + 15) / 16;
+    const size_t acts_bytes = (groups * nb * (size_t)jq::H6_REC + 255) & ~(size_t)255;
+    const size_t scratch_cap = tl_fixed_scratch ? tl_fixed_scratch->bytes : (size_t)1 << 40;
+    if (acts_bytes > scratch_cap) return -1;
+    auto rows_of = [&](const Shape &sh) { return (m + 32 * (size_t)sh.nw - 1) / (32 * (size_t)sh.nw); };
+    auto tiles_of = [&](const Shape &sh) { return rows_of(sh) * ((n + 16 * (size_t)sh.ng - 1) / (16 * (size_t)sh.ng)); };
+    auto grid_of = [&](const Shape &sh) { return 8 % rows_of(sh) == 0 ? (tiles_of(sh) + 7) / 8 * 8 : tiles_of(sh); };
+    if (!min_m_env && tiles_of(shapes[2]) * std::max<size_t>(1, std::min<size_t>(nb / 4, 8)) < 64) return -1;
+    auto rounds = [](double wgs, double at_once, auto us) {
+        const double whole = std::floor(wgs / at_once), rest = wgs - whole * at_once;
+        return whole * us(at_once) + (rest > 0.0 ? us(rest) : 0.0);
+    };
+    // In us, the int8 GEMM's form of estimate (dispatch_gemm_i8) fitted to 714 times of this one's three shapes in 1 to 8 parts: the
+    // preparation, a fixed start, the super-blocks a workgroup walks at a cost that grows with the workgroups at work, the
+    // starts of further rounds, the sum of the parts.  Over 70 shapes the picks are 0.6 % off the best measured choice on
+    // average, 4 % at the 95th percentile, 10 % at worst.
+    auto estimate = [&](const Shape &sh, size_t sp) {
+        const double wgs = (double)(grid_of(sh) * sp), nbl = (double)(nb / sp);
+        double us = 3.2 + 0.0048 * (double)(nb * groups);
+        if (sh.nw == 8)
+            us += 6.4 + nbl * rounds(wgs, 256.0, [](double w) { return 3.4 + 0.0035 * w; }) * (sh.ng == 7 ? 1.0 : 0.92) +
+                  4.2 * (std::ceil(wgs / 256.0) - 1.0);
+        else
+            us += 6.6 + nbl * rounds(wgs, 512.0, [](double w) { return w <= 256.0 ? 2.24 + 0.0011 * w : 3.06 + 0.0011 * w; }) +
+                  2.5 * std::max(0.0, wgs / 512.0 - 1.5);
+        if (sp > 1) us += 0.09 * (double)sp + (double)(sp + 1) * (double)(m * n) * 4.0 / 3.4e6;
+        return us;
+    };
+    const Shape *best = nullptr;
+    size_t splits = 1;
+    double best_us = 0.0;
+    int want_nw = 0, want_ng = 0;
+    const bool forced = shape_env && sscanf(shape_env, "%d,%d", &want_nw, &want_ng) == 2;
+    for (const Shape &sh : shapes) {
+        if (forced && (sh.nw != want_nw || sh.ng != want_ng)) continue;
+        for (size_t sp = 1; sp <= 8; sp++) {
+            if (nb % sp != 0 || (sp > 1 && nb / sp < 4)) continue;
+            if (splits_env && sp != (size_t)atoi(splits_env)) continue;
+            if (sp > 1 && (m * n > 0x3FFFFFFFull || acts_bytes + sp * m * n * sizeof(float) > scratch_cap)) continue;
+            const double us = estimate(sh, sp);
+            if (!best || us < best_us) best = &sh, splits = sp, best_us = us;
+        }
+    }
+    if (!best) return -1;
+    const size_t tx = (n + 16 * (size_t)best->ng - 1) / (16 * (size_t)best->ng), ty = rows_of(*best), grid = grid_of(*best);
+    if (grid > 0x7FFFFFFFull) return -1;
+    CallScratch scratch;
+    uint8_t *acts = nullptr;
+    if (scratch.get(acts_bytes + (splits > 1 ? splits * m * n * sizeof(float) : 0), s, &acts)) return 1;
+    float *parts = (float *)(acts + acts_bytes);
+    auto launch = [&](auto kern, int lds, int nw, hipError_t rc) {
+        if (rc != hipSuccess) return fail("hipFuncSetAttribute: %s", hipGetErrorString(rc));
+        const dim3 prep((unsigned)nb, (unsigned)groups);
+        if (swiglu_pairs) hipLaunchKernelGGL(jq::kq_gemm_h6_prep<true>, prep, dim3(128), 0, s, X, (int)m, (int)k, acts);
+        else hipLaunchKernelGGL(jq::kq_gemm_h6_prep<false>, prep, dim3(128), 0, s, X, (int)m, (int)k, acts);
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid, (unsigned)splits), dim3(64 * nw), lds, s, W, row_bytes, (const uint8_t *)acts,
+                           splits > 1 ? parts : Y, (int)m, (int)n, (int)(nb / splits), (int)groups, (int)tx, (int)ty, (int)nb,
+                           splits > 1 ? m * n : (size_t)0);
+        if (splits > 1)
+            hipLaunchKernelGGL(jq::splitk_sum, dim3((unsigned)((m * n + 1023) / 1024)), dim3(256), 0, s, parts, Y, m * n, (int)splits);
+        return 0;
+    };
+#define JQ_GEMM_H6(NW_, NG_) launch(jq::kq_gemm_h6<F, NW_, NG_>, jq::h6_lds_bytes<NG_>(), NW_, big_lds_once<&jq::kq_gemm_h6<F, NW_, NG_>>(jq::h6_lds_bytes<NG_>()))
+    const int rc = best->nw == 4 ? JQ_GEMM_H6(4, 4) : best->ng == 7 ? JQ_GEMM_H6(8, 7) : JQ_GEMM_H6(8, 6);
+#undef JQ_GEMM_H6
+    if (rc) return rc;
+    note_kernel(splits > 1 ? name_split : name);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
 // Q4_K with more than 16 activation rows: prepare the fixed-point activation planes in the
 // call scratch of the stream, then the MFMA GEMM, split over k when its tiles alone would leave
 // compute units idle.
@@ -957,7 +1058,8 @@ int dispatch_matmul(uint32_t type, const uint8_t *W, size_t row_bytes, const flo
         return dispatch_q4k_gemm(W, row_bytes, X, Y, m, k, n, s);
     if (type == JQ_TYPE_Q4_K && q4k_mfma_applies(m, k, n)) return dispatch_q4k_mfma(W, row_bytes, X, Y, m, k, n, s);
     if (type == JQ_TYPE_Q4_K && m > Q4K_MFMA_MAX_M) {
-        const int rc = dispatch_gemm_i8<jq::QiQ4K>(W, row_bytes, X, Y, m, k, n, s, "q4k_gemm_i8", "q4k_gemm_i8+splitk");
+        int rc = dispatch_gemm_h6<jq::H6Q4K>(W, row_bytes, X, Y, m, k, n, s, "q4k_gemm_i8", "q4k_gemm_i8+splitk");
+        if (rc < 0) rc = dispatch_gemm_i8<jq::QiQ4K>(W, row_bytes, X, Y, m, k, n, s, "q4k_gemm_i8", "q4k_gemm_i8+splitk");
         if (rc >= 0) return rc;
     }
     // every other format (Q6_K, Q2_K, Q8_0, IQ2_XXS, MXFP4, Q5_K, Q4_0, Q3_K, Q5_0, Q4_1, Q5_1): the same GEMM wherever the MFMA GEMM over decoded weights would run otherwise (from 17
@@ -3078,6 +3180,9 @@ int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *w
                 const jq_weight *wd = dn->second;
                 int rc = -1;
                 if (wd->type == JQ_TYPE_Q4_K)
+                    rc = dispatch_gemm_h6<jq::H6Q4K>(wd->dev, wd->row_bytes, m->g, m->proj, T, wd->k, wd->n, s, "q4k_gemm_i8",
+                                                     "q4k_gemm_i8+splitk", true);
+                if (rc < 0 && wd->type == JQ_TYPE_Q4_K)
                     rc = dispatch_gemm_i8<jq::QiQ4K>(wd->dev, wd->row_bytes, m->g, m->proj, T, wd->k, wd->n, s, "q4k_gemm_i8",
                                                      "q4k_gemm_i8+splitk", true);
                 else if (wd->type == JQ_TYPE_Q6_K)

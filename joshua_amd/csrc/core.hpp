@@ -83,7 +83,8 @@ struct FixedScratchScope {
 // jq_matmul_t_noalloc serves the same requests from a fixed array in device memory instead (below): it
 // installs the array for the calling thread with FixedScratchScope, and get() then hands out that
 // array, or fails when the request exceeds it, and never reaches an allocator.
-constexpr size_t SCRATCH_KEEP = 64u << 20;
+// (2048 activation rows of 12288 are 76 MB of prepared records, kq_gemm_h6)
+constexpr size_t SCRATCH_KEEP = 128u << 20;
 class CallScratch {
     std::unique_lock<std::mutex> lock_;
     hipStream_t stream_ = nullptr;

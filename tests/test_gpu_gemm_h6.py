@@ -1,0 +1,97 @@
+"""Q4_K products of many activation rows on f16 and FP6 operands (kq_gemm_h6) against 64-bit products of the decoded weights.
+
+The library takes the kernel from 128 activation rows on and picks the workgroup shape and the split over k by an estimate; with
+both forced through the environment (read at the first dispatch, hence the child process) every shape runs at the edges of its
+tiles."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CHILD = r"""
+import os, sys
+import numpy as np
+sys.path.insert(0, %r)
+import oracle
+from joshua_amd import capi, synth
+splits = int(os.environ["JQ_GEMM_H6_SPLITS"])
+name = "q4k_gemm_i8" + ("+splitk" if splits > 1 else "")
+
+
+def parts(blocks, n, k):
+    # d sc (q - 8), and the factor d of it, of every element
+    b = blocks.reshape(n, k // 256, 144)
+    d = b[:, :, 0:2].copy().view(np.float16).astype(np.float64)[:, :, 0]
+    s = b[:, :, 4:16].astype(np.int64)
+    sc = np.concatenate([s[:, :, :4] & 63, (s[:, :, 8:] & 15) | s[:, :, :4] >> 6 << 4], 2)
+    q = b[:, :, 16:].reshape(n, k // 256, 4, 1, 32)
+    q = np.concatenate([q & 15, q >> 4], 3).reshape(n, k // 256, 8, 32).astype(np.int64)
+    return (sc[..., None] * (q - 8)).astype(np.float64).reshape(n, -1, 256), d
+
+
+def check(blocks, lhs, what, rms=None):
+    m, k = lhs.shape
+    n = blocks.size // (k // 256 * 144)
+    got = capi.Weight.upload(capi.Q4_K, blocks, n, k).matmul_t(m, lhs)
+    assert capi.last_kernel() == name, capi.last_kernel()
+    w = oracle.dequantize(capi.Q4_K, blocks).reshape(n, k).astype(np.float64)
+    x = lhs.astype(np.float64)
+    want = x @ w.T
+    # With s <= 2^-14 of a super-block's largest magnitude: the remainder l <= 8 s of an activation as E2M3 is at most s / 2 off,
+    # p as E2M3 codes of 2^-7 p at most max(|p| / 16, 8): an element adds at most d s (|p| / 2 + 8 max(|p| / 16, 8)).  The mean of a
+    # sub-block and its weight in two bf16 parts each: 2^-16 of the terms.  f32 sums: 2^-20 of them.
+    p, d = parts(blocks, n, k)
+    s = np.abs(x.reshape(m, -1, 256)).max(2) * 2.0 ** -14
+    off = np.abs(d) * (np.abs(p) / 2 + 8 * np.maximum(np.abs(p) / 16, 8)).sum(2)
+    bound = s @ off.T + (2.0 ** -16 + 2.0 ** -20) * (np.abs(x) @ np.abs(w).T + np.abs(x) @ (np.abs(p) * np.abs(d)[..., None]).reshape(n, k).T)
+    err = np.abs(got - want)
+    assert np.all(err <= bound), (what, float((err / np.maximum(bound, 1e-300)).max()))
+    if rms is not None:  # the remainders left out would show as 1e-4
+        rel = np.sqrt((err ** 2).mean() / (want ** 2).mean())
+        assert rel <= rms, (what, float(rel))
+    return got
+
+
+rng = np.random.default_rng(4)
+sizes = [(17, 256, 64), (33, 512, 113), (64, 1024, 97), (129, 768, 112), (257, 512, 300), (256, 1024, 96)] if splits == 1 else [(40, 4096, 100), (300, 4096, 130)]
+for m, k, n in sizes:
+    check(synth.normal_quantized(capi.Q4_K, 5 + n, n * k, 0.02), synth.normal(6 + k, (m, k)), (m, k, n), 2e-5)
+n, k = 80, 2048 if splits == 1 else 4096
+raw = rng.integers(0, 256, (n * k // 256, 144), dtype=np.uint8)   # every scale, min and code
+raw[:, 0:2] = (rng.uniform(-1e-3, 1e-3, n * k // 256)).astype(np.float16).view(np.uint8).reshape(-1, 2)
+raw[:, 2:4] = (rng.uniform(-1e-3, 1e-3, n * k // 256)).astype(np.float16).view(np.uint8).reshape(-1, 2)
+raw[::7, 0:2] = 0
+lhs = synth.normal(9, (50, k))
+check(raw.reshape(-1), lhs, "random blocks", 2e-5)
+# rows whose groups of 16 span twelve orders of magnitude, of one non-zero element, with an empty stretch, at f32's ends
+lhs[0] *= (10.0 ** rng.integers(-6, 7, size=k // 16)).repeat(16).astype(np.float32)
+lhs[1] = 0
+lhs[1, 1234] = 3.5
+lhs[2, 512:1024] = 0
+lhs[3] *= np.float32(1e30)
+lhs[4] *= np.float32(1e-30)
+lhs[5] = np.float32(65519.0)     # just below the next power of two's f16
+got = check(raw.reshape(-1), lhs, "rows of every range")
+lhs[7, 100], lhs[8, 2000], lhs[9, 5] = np.inf, np.nan, -np.inf
+other = capi.Weight.upload(capi.Q4_K, raw.reshape(-1), n, k).matmul_t(50, lhs)
+assert np.all(np.isnan(other[7:10])), "a row that is not finite"
+assert np.array_equal(np.delete(other, [7, 8, 9], 0), np.delete(got, [7, 8, 9], 0)), "its neighbours"
+if splits == 1:  # SwiGLU in the preparation: the down projection of a decoder's prompt
+    from tests.test_gpu_qwen3 import CFG, make, close
+    m, o = make(dict(CFG, n_ctx=64), 77, "q4_k")
+    tokens = rng.integers(0, 768, 45).tolist()
+    ok, e = close(m.forward(tokens, 0), o.forward(tokens, 0))
+    assert ok, e
+print("h6 ok")
+"""
+
+
+@pytest.mark.parametrize("shape,splits", [("8,7", 1), ("8,6", 1), ("4,4", 1), ("8,7", 2), ("4,4", 4)])
+def test_gemm_on_f16_and_fp6_operands(shape, splits):
+    env = dict(os.environ, JQ_GEMM_H6_SHAPE=shape, JQ_GEMM_H6_SPLITS=str(splits), JQ_GEMM_H6_MIN_M="17", JQ_Q4K_NO_ROWS16="1")
+    res = subprocess.run([sys.executable, "-c", CHILD.replace("%r", repr(ROOT), 1)], env=env, capture_output=True, text=True, timeout=110)
+    assert res.returncode == 0 and "h6 ok" in res.stdout, res.stdout + res.stderr
