@@ -2434,9 +2434,9 @@ void mla_free_scratch(jq_mla *m) {
 // from 48 tokens on (whole calls of DeepSeek-V3's size, us, absorbed / expanded: 32 tokens behind 0, 1000, 4000: 307 / 308,
 // 399 / 511, 654 / 1063; 48 tokens 481 / 409, 652 / 613), and there by the estimate of both.
 constexpr size_t MLA_EXPAND_TOKENS = 48;
-bool mla_expands(const jq_mla *m, size_t S, size_t pos) {
+bool mla_expands(const jq_mla *m, size_t S, size_t pos, bool fresh = false) {
     static const bool asked = getenv("JQ_MLA_ATTENTION") || getenv("JQ_MLA_SPLIT");  // for the absorbed form's kernels
-    return m->split16 && !asked && S >= MLA_EXPAND_TOKENS && split16_latent_pays(m->split16, S, pos);
+    return m->split16 && !asked && S >= MLA_EXPAND_TOKENS && split16_latent_pays(m->split16, S, pos, fresh);
 }
 
 // The largest call of up to S tokens that may be absorbed somewhere in the context: after a call of S, smaller ones find their
@@ -2444,7 +2444,7 @@ bool mla_expands(const jq_mla *m, size_t S, size_t pos) {
 size_t mla_absorbed_tokens(const jq_mla *m, size_t S) {
     for (size_t t = S; t >= MLA_EXPAND_TOKENS; t -= std::max<size_t>(t / 16, 1))
         for (size_t i = 0; i <= 16; i++)
-            if (!mla_expands(m, t, (m->cfg.n_ctx - t) * i / 16)) return std::min(S, t + t / 16);
+            if (!mla_expands(m, t, (m->cfg.n_ctx - t) * i / 16, true)) return std::min(S, t + t / 16);
     return std::min(S, MLA_EXPAND_TOKENS);
 }
 
@@ -2543,6 +2543,7 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
     const size_t nh = c.n_head, nope = c.qk_nope_head_dim, rope = c.qk_rope_head_dim, vh = c.v_head_dim,
                  lkv = c.kv_lora_rank, qd = nope + rope;
     const float *comp = m->comp;
+    if (m->split16 && split16_latent_overwrites(m->split16, pos, s)) return 1;
     // one token over a Q4_K up-projection of DeepSeek's geometry: its blocks are read (9 MB at V3's size) instead of the
     // 67 MB of their f32 copy.  128 heads behind 100 tokens, us: absorbing 7.1 / 5.4, merging the splits and multiplying with the value
     // rows 4.8 + 8.0 / 6.1 in one launch.

@@ -159,12 +159,12 @@ __global__ __launch_bounds__(256) void s16_up_projection(const float *__restrict
     }
 }
 
-// grid tiles, 256 threads: the normed latents of 32 tokens as fragments [tile][k-step 32][plane] (times 2^ec), their rope keys
+// grid tiles (from tile0 on), 256 threads: the normed latents of 32 tokens as fragments [tile][k-step 32][plane] (times 2^ec), their rope keys
 // as [tile][k-step 4][plane] with a scale a tile, info[tile].k the power of two that undoes it.
-__global__ __launch_bounds__(256) void s16_latent_tiles(const float *__restrict__ lat, const float *__restrict__ kpe, int n_keys, float cscale,
+__global__ __launch_bounds__(256) void s16_latent_tiles(const float *__restrict__ lat, const float *__restrict__ kpe, int tile0, int n_keys, float cscale,
                                                         uint8_t *__restrict__ cf, uint8_t *__restrict__ rf, S16Tile *__restrict__ info) {
     __shared__ uint32_t red[4], bad;
-    const int tile = blockIdx.x, tid = threadIdx.x, lane = tid & 63, row = lane & 31, key = tile * S16_TILE + row;
+    const int tile = tile0 + (int)blockIdx.x, tid = threadIdx.x, lane = tid & 63, row = lane & 31, key = tile * S16_TILE + row;
     const bool live = key < n_keys;
     float x[8];
     bool whole = true;
@@ -206,8 +206,8 @@ __global__ __launch_bounds__(256) void s16_latent_tiles(const float *__restrict_
     *(s16_h8 *)(out + (2 * s + 1) * S16_FRAG) = lo;
 }
 
-// Keys (part 0) and values (part 1) of `heads` heads from head h0 on, for every cached token, written as the fragments the
-// attention below reads: [head - h0][tile]{K, V}.  grid (token blocks x 2 heads) of four waves; a workgroup multiplies 128
+// Keys (part 0) and values (part 1) of `heads` heads from head h0 on, for the n_tiles tiles of cached tokens from tile0 on, written
+// as the fragments the attention below reads: [head - h0][tile of `stride`]{K, V}.  grid (token blocks x 2 heads) of four waves; a workgroup multiplies 128
 // rows of the up-projection with 128 latents, k in stages of 32 through two LDS buffers.  The accumulators leave as whole
 // fragments: of K the product is made with the projection's rows first (a lane holds eight columns of one key), of V with the
 // latents first (eight keys of one column).
@@ -300,12 +300,13 @@ __device__ __forceinline__ void s16_expand_workgroup(const uint8_t *__restrict__
 }
 
 __global__ __launch_bounds__(256, 2) void s16_expand(const uint8_t *__restrict__ wfrags, const float2 *__restrict__ fac, const uint8_t *__restrict__ cf,
-                                                     int h0, int heads, int n_tiles, uint8_t *__restrict__ ws) {
+                                                     int h0, int heads, int tile0, int n_tiles, int stride, uint8_t *__restrict__ ws) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[2 * 2 * 8 * 2 * S16_FRAG];
     // a head stays on one XCD (ids 8 apart), whose L2 then holds its rows while the token blocks go by
     const int hp = (int)blockIdx.x % (2 * heads), tb = (int)blockIdx.x / (2 * heads), h = hp % heads, part = hp / heads;
     const uint8_t *wf = wfrags + ((size_t)(h0 + h) * 2 + part) * (S16_LKV / 16) * 8 * S16_FRAG;
-    uint8_t *out = ws + (size_t)h * n_tiles * S16_KV_TILE;
+    uint8_t *out = ws + ((size_t)h * stride + tile0) * S16_KV_TILE;
+    cf += (size_t)tile0 * (S16_LKV / 16) * 2 * S16_FRAG;
     const float f = fac[2 * (h0 + h) + part].x;
     if (part) s16_expand_workgroup<true>(wf, cf, f, n_tiles, tb, out, lds);
     else s16_expand_workgroup<false>(wf, cf, f, n_tiles, tb, out, lds);
@@ -321,7 +322,7 @@ struct S16Attention {
     const uint8_t *rope;       // latent: [tile]
     float *out;                // [t][out_stride], head h at h * 128
     int out_stride;
-    int T, pos0, n_tiles;      // tokens of the step at positions pos0 .., tiles of the cache
+    int T, pos0, n_tiles;      // tokens of the step at positions pos0 .., tiles that a head's lie apart
     int heads, group;          // query heads of this call; how many of them share a KV head (latent: 1)
     int blocks;                // token blocks
     float scale_log2e;         // the softmax scale times log2(e)

@@ -29,6 +29,13 @@ struct Split16Latent {
     float2 *fac = nullptr;
     uint8_t *cf = nullptr, *rf = nullptr, *ws = nullptr;  // latents, rope keys, a group of heads' keys and values
     jq::S16Tile *info = nullptr;
+    // Tokens whose keys and values lie in ws, where it holds all heads over the whole context: a part of the cache like the latents
+    // they are made of, which a call adds its own tokens to.  4096 tokens in chunks of 512: 7.0 ms with every chunk expanding all in
+    // front of it again, 5.3 without.
+    size_t ready = 0;
+    // A call of this object was captured: its replays write tokens without this knowing, and each has to leave the keys and values
+    // of all tokens in front of it, so that from then on every call expands them all.
+    bool captured = false;
 };
 
 bool split16_latent_fits(size_t nope, size_t rope, size_t vh, size_t lkv) {
@@ -37,7 +44,7 @@ bool split16_latent_fits(size_t nope, size_t rope, size_t vh, size_t lkv) {
 
 // Bytes of an object's keys and values: those of all heads over the whole context, so that no later call allocates, up to
 // 512 MiB (what the absorbed form's scratch takes for 1000 tokens of 128 heads); longer contexts take the heads in groups.
-// 4096 tokens of DeepSeek-V3's size in chunks of 512: 7.5 ms, with 256 MiB 7.8; 512 tokens behind 8000: 2.5 and 3.9.
+// 512 tokens of DeepSeek-V3's size behind 8000, 512 MiB against 256: 2.5 and 3.9 ms.
 static size_t latent_ws_bytes(const Split16Latent *s) {
     return s->ws_bytes ? s->ws_bytes : std::min(s->n_head * tiles_of(s->n_ctx) * jq::S16_KV_TILE, (size_t)512 << 20);
 }
@@ -51,16 +58,29 @@ static size_t latent_group(const Split16Latent *s, size_t nt) {
     return eights <= fit ? eights : even;
 }
 
+static bool latent_keeps(const Split16Latent *s) { return !s->captured && latent_ws_bytes(s) >= s->n_head * tiles_of(s->n_ctx) * jq::S16_KV_TILE; }
+// The first tile that a call has to expand.
+static size_t latent_first_tile(const Split16Latent *s) { return latent_keeps(s) ? s->ready / jq::S16_TILE : 0; }
+
+int split16_latent_overwrites(Split16Latent *s, size_t pos, hipStream_t stream) {
+    s->ready = std::min(s->ready, pos);
+    if (s->captured) return 0;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(stream, &capture));
+    s->captured = capture != hipStreamCaptureStatusNone;
+    return 0;
+}
+
 // Both sides in us, fitted to calls of 48 to 1024 tokens behind 0 to 32000 with 128 and 32 heads (within 10 %, the absorbed
 // form's vector kernel, for head counts that are no multiple of 32, within 25 %).  Expanded, a group of g heads: 0.0266 a tile and
 // head to expand and, a workgroup walking all tiles, 1.76 a tile while there is one to a compute unit.  128 heads, absorbed /
 // expanded in groups as here: 48 tokens behind 0, 4000, 8000, 16000: 139 / 32, 829 / 671, 1527 / 1690, 2924 / 5045; 128 tokens behind
 // 4000, 8000, 16000: 1707 / 718, 3105 / 1735, 5881 / 5112; 512 tokens behind 4000, 16000: 7016 / 1037, 23784 / 5423.
-bool split16_latent_pays(const Split16Latent *s, size_t S, size_t pos) {
-    const size_t nt = tiles_of(pos + S), g = latent_group(s, nt), nh = s->n_head;
+bool split16_latent_pays(const Split16Latent *s, size_t S, size_t pos, bool fresh) {
+    const size_t nt = tiles_of(pos + S), made = fresh ? 0 : latent_first_tile(s), g = latent_group(s, nt), nh = s->n_head;
     if (g == 0 || s->refused) return false;
     const double wgs = (double)(g * ((S + 127) / 128)), keys = (double)pos + (double)S / 2;
-    const double expanded = (double)((nh + g - 1) / g) * (20.0 + (double)nt * (1.76 * std::max(1.0, wgs / 233.0) + 0.0266 * (double)g));
+    const double expanded = (double)((nh + g - 1) / g) * (20.0 + (double)nt * 1.76 * std::max(1.0, wgs / 233.0) + (double)(nt - made) * 0.0266 * (double)g);
     const double walk = nh % 32 == 0 ? 0.174 * std::ceil((double)(S * nh) / (32 * 256)) : 0.27 * std::max(1.0, 0.75 * (double)(S * ((nh + 7) / 8)) / 256);
     return expanded < 0.92 * (35.0 + 0.017 * (double)(S * nh) + walk * keys);  // (level with it: the form that needs no buffer)
 }
@@ -117,23 +137,27 @@ int split16_latent_attention(Split16Latent *s, const float *q, size_t S, size_t 
     }
     const size_t group = latent_group(s, nt);
     if (group == 0) return -1;
-    hipLaunchKernelGGL(jq::s16_latent_tiles, dim3((unsigned)nt), dim3(256), 0, stream, lat, kpe, (int)(pos + S), ldexpf(1.0f, s->ec), s->cf,
-                       s->rf, s->info);
+    // tiles from t0 on are to be made, the heads' tiles lie `stride` apart
+    const bool keeps = latent_keeps(s);
+    const size_t t0 = latent_first_tile(s), stride = keeps ? all : nt, made = nt - t0;
+    hipLaunchKernelGGL(jq::s16_latent_tiles, dim3((unsigned)made), dim3(256), 0, stream, lat, kpe, (int)t0, (int)(pos + S), ldexpf(1.0f, s->ec),
+                       s->cf, s->rf, s->info);
     HIP_TRY(hipGetLastError());
     for (size_t h0 = 0; h0 < s->n_head; h0 += group) {
         const size_t hg = std::min(group, s->n_head - h0);
-        hipLaunchKernelGGL(jq::s16_expand, dim3((unsigned)(2 * hg * ((nt + 3) / 4))), dim3(256), 0, stream, (const uint8_t *)s->wfrags,
-                           (const float2 *)s->fac, (const uint8_t *)s->cf, (int)h0, (int)hg, (int)nt, s->ws);
+        hipLaunchKernelGGL(jq::s16_expand, dim3((unsigned)(2 * hg * ((made + 3) / 4))), dim3(256), 0, stream, (const uint8_t *)s->wfrags,
+                           (const float2 *)s->fac, (const uint8_t *)s->cf, (int)h0, (int)hg, (int)t0, (int)made, (int)stride, s->ws);
         HIP_TRY(hipGetLastError());
         jq::S16Attention a{};
         a.q = q + h0 * (jq::S16_HEAD + jq::S16_ROPE), a.q_stride = (int)(s->n_head * (jq::S16_HEAD + jq::S16_ROPE)), a.q_head = jq::S16_HEAD + jq::S16_ROPE;
         a.kv = s->ws, a.info = s->info, a.fac = s->fac + 2 * h0, a.rope = s->rf;
         a.out = out + h0 * jq::S16_HEAD, a.out_stride = (int)(s->n_head * jq::S16_HEAD);
-        a.T = (int)S, a.pos0 = (int)pos, a.n_tiles = (int)nt, a.heads = (int)hg, a.group = 1, a.blocks = (int)((S + 127) / 128);
+        a.T = (int)S, a.pos0 = (int)pos, a.n_tiles = (int)stride, a.heads = (int)hg, a.group = 1, a.blocks = (int)((S + 127) / 128);
         a.scale_log2e = scale * 1.44269504088896340736f;
         hipLaunchKernelGGL((jq::s16_attention<true, 1>), dim3((unsigned)(hg * a.blocks)), dim3(256), 0, stream, a);
         HIP_TRY(hipGetLastError());
     }
+    if (keeps) s->ready = pos + S;
     return 0;
 }
 

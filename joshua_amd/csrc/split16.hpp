@@ -12,8 +12,12 @@ bool split16_latent_fits(size_t nope, size_t rope, size_t vh, size_t lkv);
 // the operands (half a megabyte a head) *out is null, and the object's calls are absorbed ones.
 int split16_latent_create(size_t n_head, size_t n_ctx, const float *wkv, const float *kv_norm, Split16Latent **out);
 void split16_latent_free(Split16Latent *s);
-// Whether a call of S tokens behind `pos` is cheaper with expanded keys and values than absorbed.
-bool split16_latent_pays(const Split16Latent *s, size_t S, size_t pos);
+// The cached tokens from `pos` on are about to be written by work on that stream: their keys and values, if they were
+// expanded, are not those of the cache any more.
+int split16_latent_overwrites(Split16Latent *s, size_t pos, hipStream_t stream);
+// Whether a call of S tokens behind `pos` is cheaper with expanded keys and values than absorbed; `fresh`: where none of those
+// in front are expanded already.
+bool split16_latent_pays(const Split16Latent *s, size_t S, size_t pos, bool fresh);
 // out[t][n_head * 128] for S tokens at positions pos .. over the cached latents and rotated rope keys of pos + S tokens;
 // q [t][n_head * 192] rotated.  0: done, 1: failed, -1: no memory for the expanded keys and values (then not asked for again).
 int split16_latent_attention(Split16Latent *s, const float *q, size_t S, size_t pos, const float *lat, const float *kpe, float scale,

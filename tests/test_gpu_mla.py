@@ -387,3 +387,58 @@ def test_create_rejects_wrong_shapes():
                         v_head_dim=32, n_ctx=16, rms_eps=1e-6, rope_theta=1e4)
     with pytest.raises(capi.JoshuaHipError, match="attn_q is"):
         capi.Mla(mc, w, w, np.ones(64, np.float32), w, w)
+
+
+@pytest.mark.parametrize("n_head", [3, 32])
+def test_calls_add_to_the_keys_and_values_of_earlier_ones(n_head):
+    """Calls of many tokens expand those since the last such call only, short ones in between (absorbed) and part-filled tiles of
+    32 tokens among them; after a reset other tokens take all places."""
+    c = cfg(n_embd=256, n_head=n_head, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=128, context_length=640)
+    ref, dev = build(c, seed=940)
+    for seed, steps in ((24, (50, 1, 1, 64, 100, 3, 49, 200)), (25, (48, 47, 96, 160)), (26, (40, 33, 130))):
+        x, pos = normal(seed, (sum(steps), 256)), 0
+        for n in steps:
+            assert close(dev.forward(x[pos:pos + n], pos), ref.forward(x[pos:pos + n], pos)), (steps, pos)
+            pos += n
+        dev.reset()
+        ref, _ = build(c, seed=940)
+
+
+def test_a_captured_call_behind_tokens_that_were_not_expanded():
+    """64 tokens behind 100 that the call before expanded are captured; the graph is replayed behind 100 others that short, absorbed
+    calls wrote, and so were never expanded."""
+    import torch
+    c = cfg(n_embd=256, n_head=4, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=128, context_length=192)
+    _, dev = build(c, seed=950)
+    _, fresh = build(c, seed=950)
+    a, b = (torch.from_numpy(normal(seed, (100, 256))).cuda() for seed in (27, 28))
+    x = torch.from_numpy(normal(29, (64, 256))).cuda()
+    y, rest = torch.zeros(64, 256, device="cuda"), torch.zeros(100, 256, device="cuda")
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+
+    def run(m, t, steps):
+        m.reset()
+        for n in steps:
+            p = m.cached_tokens
+            m.forward_dev(n, p, t.data_ptr() + 1024 * p, rest.data_ptr(), stream.cuda_stream)
+
+    with torch.cuda.stream(stream):
+        run(dev, a, (100,))
+        dev.forward_dev(64, 100, x.data_ptr(), y.data_ptr(), stream.cuda_stream)
+        stream.synchronize()
+        run(dev, a, (100,))
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            dev.forward_dev(64, 100, x.data_ptr(), y.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        for t, steps in ((a, (100,)), (b, (40, 40, 20)), (b, (100,)), (a, (30, 30, 40))):
+            run(fresh, t, steps)
+            want = fresh.forward(x.cpu().numpy(), 100)
+            run(dev, t, steps)
+            y.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.abs(y.cpu().numpy() - want).max() < 3e-4 * max(1.0, np.abs(want).max()), steps
+    del graph
+    torch.cuda.synchronize()
+    capi.stream_release(stream.cuda_stream)
