@@ -2175,7 +2175,7 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
                            (uintptr_t)pre->a.hn_out | (uintptr_t)m->router_w) & 15) == 0;
             if (!pre->fused)
                 hipLaunchKernelGGL(jq::rmsnorm_rows, dim3((unsigned)T), dim3(1024), 0, s, (float *)pre->a.x, pre->a.res, pre->a.w,
-                                   pre->a.eps, pre->a.hn_out, (int)c.hidden);
+                                   pre->a.eps, pre->a.hn_out, (int)c.hidden, (int)c.hidden);
         }
         if (moe_route_dev(m, T, x, s, jq::MoePairGroups{m->gexp, m->offsets, m->xrow, m->yrow, extra}, planes, &planes_ready,
                           late ? &gate_later : nullptr, pre && pre->fused ? &pre->a : nullptr))
@@ -2186,7 +2186,7 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
         if (pre) {
             pre->fused = false;
             hipLaunchKernelGGL(jq::rmsnorm_rows, dim3((unsigned)T), dim3(1024), 0, s, (float *)pre->a.x, pre->a.res, pre->a.w,
-                               pre->a.eps, pre->a.hn_out, (int)c.hidden);
+                               pre->a.eps, pre->a.hn_out, (int)c.hidden, (int)c.hidden);
         }
         // few pairs an expert of Q4_K with short rows: gate and up will run on the kernel that takes four rows an MFMA,
         // which reads x as fixed-point planes; the router launch leaves them behind
@@ -2403,8 +2403,7 @@ struct jq_mla {
     const jq_weight *q, *q_b, *kv_a, *kv_b, *o;
     float *q_a_norm = nullptr, *kv_a_norm = nullptr;
     float *wkv = nullptr;   // the KV up-projection as dense f32 [n_head * (nope + vh), lkv]
-    uint8_t *qa_kva = nullptr;  // q_a's rows followed by kv_a's in one allocation (same format and width): one product a single-token step
-    float *qa_kva_out = nullptr;  // its result, q_lora_rank + lkv + rope floats
+    uint8_t *qa_kva = nullptr;  // q_a's rows followed by kv_a's in one allocation (same format and width): one product
     float2 *cs = nullptr;   // [n_ctx][rope / 2] (cos, sin), scaled by the YaRN mscale
     float *lat = nullptr, *kpe = nullptr;  // the cache: [n_ctx][lkv] normed latents, [n_ctx][rope] rotated keys
     float scale = 0.0f;
@@ -2448,6 +2447,13 @@ size_t mla_absorbed_tokens(const jq_mla *m, size_t S) {
     return std::min(S, MLA_EXPAND_TOKENS);
 }
 
+// Floats of a result row of q_a and kv_a as one product, where a call of S tokens takes them so: always for one token, for more
+// where the rows keep to 16 bytes (rmsnorm_rows).  0: two products.  512 tokens of DeepSeek-V3's size: 35 + 30 us, as one 44.
+size_t mla_qa_kva(const jq_mla *m, size_t S) {
+    const size_t n = m->qa_kva ? m->q->n + m->kv_a->n : 0;
+    return S == 1 || n % 4 == 0 ? n : 0;
+}
+
 // Scratch for calls of up to T tokens, of which up to `absorbed` in absorbed form.  Buffers that are outgrown are retired,
 // not freed: a HIP graph captured over an earlier, smaller call still names them, and they go with the object (jq_mla_free).
 int mla_reserve(jq_mla *m, size_t T, size_t absorbed) {
@@ -2470,11 +2476,12 @@ int mla_reserve(jq_mla *m, size_t T, size_t absorbed) {
     m->cap_tokens = 0;
     const size_t qd = c.qk_nope_head_dim + c.qk_rope_head_dim;
     if (c.q_lora_rank) {
-        HIP_TRY(hipMalloc((void **)&m->t1, T * c.q_lora_rank * sizeof(float)));
+        // (with q_a and kv_a as one product, a row holds both results)
+        HIP_TRY(hipMalloc((void **)&m->t1, std::max<size_t>({mla_qa_kva(m, 1), mla_qa_kva(m, T) * T, T * (size_t)c.q_lora_rank}) * sizeof(float)));
         HIP_TRY(hipMalloc((void **)&m->t1n, T * c.q_lora_rank * sizeof(float)));
     }
     HIP_TRY(hipMalloc((void **)&m->qv, T * c.n_head * qd * sizeof(float)));
-    HIP_TRY(hipMalloc((void **)&m->comp, T * (c.kv_lora_rank + c.qk_rope_head_dim) * sizeof(float)));
+    if (!mla_qa_kva(m, 2)) HIP_TRY(hipMalloc((void **)&m->comp, T * (c.kv_lora_rank + c.qk_rope_head_dim) * sizeof(float)));
     HIP_TRY(hipMalloc((void **)&m->ctx, T * c.n_head * c.v_head_dim * sizeof(float)));
     m->cap_tokens = T;
     return 0;
@@ -2543,6 +2550,7 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
     const size_t nh = c.n_head, nope = c.qk_nope_head_dim, rope = c.qk_rope_head_dim, vh = c.v_head_dim,
                  lkv = c.kv_lora_rank, qd = nope + rope;
     const float *comp = m->comp;
+    int comp_stride = (int)(lkv + rope);
     if (m->split16 && split16_latent_overwrites(m->split16, pos, s)) return 1;
     // one token over a Q4_K up-projection of DeepSeek's geometry: its blocks are read (9 MB at V3's size) instead of the
     // 67 MB of their f32 copy.  128 heads behind 100 tokens, us: absorbing 7.1 / 5.4, merging the splits and multiplying with the value
@@ -2550,15 +2558,15 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
     const bool kv_q4k = S == 1 && m->kv_b && m->kv_b->type == JQ_TYPE_Q4_K && lkv == 512 && nope == 128 && vh % 64 == 0 &&
                         m->kv_b->row_bytes == 288 && ((uintptr_t)m->kv_b->dev & 15) == 0;
     if (c.q_lora_rank) {
-        float *t1 = m->t1;
-        if (S == 1 && m->qa_kva) {  // one token: q_a and kv_a as one product over the rows laid end to end
-            if (dispatch_matmul(m->q->type, m->qa_kva, m->q->row_bytes, x, m->qa_kva_out, 1, c.n_embd, m->q->n + m->kv_a->n, s)) return 1;
-            t1 = m->qa_kva_out, comp = m->qa_kva_out + m->q->n;
+        const size_t both = mla_qa_kva(m, S), t1_stride = both ? both : c.q_lora_rank;
+        if (both) {  // q_a and kv_a as one product over the rows laid end to end
+            if (dispatch_matmul(m->q->type, m->qa_kva, m->q->row_bytes, x, m->t1, S, c.n_embd, t1_stride, s)) return 1;
+            comp = m->t1 + m->q->n, comp_stride = (int)t1_stride;
         } else if (dispatch_matmul(m->q->type, m->q->dev, m->q->row_bytes, x, m->t1, S, c.n_embd, c.q_lora_rank, s)) {
             return 1;
         }
-        hipLaunchKernelGGL(jq::rmsnorm_rows, dim3((unsigned)S), dim3(1024), 0, s, t1, (const float *)nullptr,
-                           (const float *)m->q_a_norm, c.rms_eps, m->t1n, (int)c.q_lora_rank);
+        hipLaunchKernelGGL(jq::rmsnorm_rows, dim3((unsigned)S), dim3(1024), 0, s, m->t1, (const float *)nullptr,
+                           (const float *)m->q_a_norm, c.rms_eps, m->t1n, (int)c.q_lora_rank, (int)t1_stride);
         HIP_TRY(hipGetLastError());
         if (dispatch_matmul(m->q_b->type, m->q_b->dev, m->q_b->row_bytes, m->t1n, m->qv, S, c.q_lora_rank, nh * qd, s)) return 1;
     } else if (dispatch_matmul(m->q->type, m->q->dev, m->q->row_bytes, x, m->qv, S, c.n_embd, nh * qd, s)) {
@@ -2585,9 +2593,9 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
                                (const float2 *)m->cs, m->lat, m->kpe, (int)pos, c.rms_eps);
         HIP_TRY(hipGetLastError());
     } else {
-        hipLaunchKernelGGL(jq::mla_rope_latent, dim3((unsigned)nh + 1, (unsigned)S), dim3(64), 0, s, m->qv, comp,
-                           (const float *)m->kv_a_norm, (const float2 *)m->cs, m->lat, m->kpe, (int)nh, (int)nope, (int)rope,
-                           (int)lkv, (int)pos, c.rms_eps);
+        hipLaunchKernelGGL(jq::mla_rope_latent, dim3((unsigned)S, (unsigned)((nh + jq::MLA_ROPE_HEADS - 1) / jq::MLA_ROPE_HEADS) + 1), dim3(256), 0, s,
+                           m->qv, comp, (const float *)m->kv_a_norm, (const float2 *)m->cs, m->lat, m->kpe, (int)nh, (int)nope,
+                           (int)rope, (int)lkv, (int)pos, c.rms_eps, (int)S, comp_stride);
         HIP_TRY(hipGetLastError());
         if (mla_expands(m, S, pos)) {
             const int rc = split16_latent_attention(m->split16, m->qv, S, pos, m->lat, m->kpe, m->scale, m->ctx, s);
@@ -2729,10 +2737,10 @@ int jq_mla_create(const jq_mla_config *cfg, const jq_weight *q_or_q_a, const flo
     HIP_TRY(hipMemcpy(m->kv_a_norm, kv_a_norm, lkv * sizeof(float), hipMemcpyHostToDevice));
     if (c.q_lora_rank && m->q->type == m->kv_a->type && m->q->row_bytes == m->kv_a->row_bytes && !getenv("JQ_MLA_NO_FUSED_QA_KVA")) {
         const size_t qa_bytes = m->q->n * m->q->row_bytes, kva_bytes = m->kv_a->n * m->kv_a->row_bytes;
-        HIP_TRY(hipMalloc((void **)&m->qa_kva, qa_bytes + kva_bytes));
+        HIP_TRY(hipMalloc((void **)&m->qa_kva, qa_bytes + kva_bytes + 64));  // (the spare bytes of jq_upload)
+        HIP_TRY(hipMemset(m->qa_kva + qa_bytes + kva_bytes, 0, 64));
         HIP_TRY(hipMemcpy(m->qa_kva, m->q->dev, qa_bytes, hipMemcpyDeviceToDevice));
         HIP_TRY(hipMemcpy(m->qa_kva + qa_bytes, m->kv_a->dev, kva_bytes, hipMemcpyDeviceToDevice));
-        HIP_TRY(hipMalloc((void **)&m->qa_kva_out, (m->q->n + m->kv_a->n) * sizeof(float)));
     }
     const std::vector<float2> cs = mla_rope_table(c);
     HIP_TRY(hipMalloc((void **)&m->cs, cs.size() * sizeof(float2)));
@@ -2750,7 +2758,7 @@ void jq_mla_free(jq_mla *m) {
     mla_free_scratch(m);
     split16_latent_free(m->split16);
     for (void *p : {(void *)m->q_a_norm, (void *)m->kv_a_norm, (void *)m->wkv, (void *)m->cs, (void *)m->lat, (void *)m->kpe,
-                    (void *)m->qa_kva, (void *)m->qa_kva_out})
+                    (void *)m->qa_kva})
         if (p) (void)hipFree(p);
     delete m;
 }
@@ -3075,7 +3083,7 @@ int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *w
             normed = fq != m->fused.end() &&
                      model_norm_mm(fq->second, xc, pending, w_an, c.rms_eps, xo, v_fused ? nullptr : m->hn, m->cat, false, s);
         if (normed) std::swap(xc, xo);
-        else hipLaunchKernelGGL(jq::rmsnorm_rows, dim3(T), dim3(1024), 0, s, xc, pending, w_an, c.rms_eps, m->hn, h);
+        else hipLaunchKernelGGL(jq::rmsnorm_rows, dim3(T), dim3(1024), 0, s, xc, pending, w_an, c.rms_eps, m->hn, h, h);
         if (fq != m->fused.end()) {  // one launch for q|k(|v) of a single token
             const jq_weight *w = fq->second;
             if (!normed && dispatch_matmul(w->type, w->dev, w->row_bytes, m->hn, m->cat, 1, w->k, w->n, s)) return 1;
@@ -3108,7 +3116,9 @@ int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *w
             hipLaunchKernelGGL(jq::attention_merge, dim3(T * nh), dim3(128), 2 * n_chunks * sizeof(float), s, m->part, m->att, d,
                                n_chunks);
         } else {
-            hipLaunchKernelGGL(jq::qkv_norm_rope_cache, dim3(T * (nh + 2 * nkv)), dim3(64), 0, s, qp, kp, vp, w_qn, w_kn,
+            // (four workgroups or more to a compute unit, no more parts than waves have heads)
+            const unsigned parts = std::min((unsigned)(nh + 2 * nkv + 3) / 4, std::max(1u, 1024 / (unsigned)T));
+            hipLaunchKernelGGL(jq::qkv_norm_rope_cache, dim3((unsigned)T, parts), dim3(256), 0, s, qp, kp, vp, w_qn, w_kn,
                                c.rms_eps, nh, nkv, d, m->pos, c.rope_theta, m->kc[l], m->vc[l], (int)c.n_ctx, q_stride,
                                k_stride, v_stride);
             // head dimension 128 and 1, 2, 4 or 8 query heads a KV head: tiles of 16 tokens on the f32 matrix cores
@@ -3159,7 +3169,7 @@ int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *w
         const bool normed2 = fg != m->fused.end() && model_norm_mm(fg->second, xc, m->proj, w_fn, c.rms_eps, xo, nullptr,
                                                                    paired ? m->mid : m->cat, paired, s);
         if (normed2) std::swap(xc, xo), activated = paired;
-        else hipLaunchKernelGGL(jq::rmsnorm_rows, dim3(T), dim3(1024), 0, s, xc, m->proj, w_fn, c.rms_eps, m->hn, h);
+        else hipLaunchKernelGGL(jq::rmsnorm_rows, dim3(T), dim3(1024), 0, s, xc, m->proj, w_fn, c.rms_eps, m->hn, h, h);
         // many tokens over a paired gate|up matrix: one product with twice the rows (768 GEMM tiles at Qwen3-8B's
         // sizes fill the 256 compute units three times over; two products of 384 tiles leave half of them idle
         // in their second rounds), then SwiGLU over the alternating results
@@ -3219,7 +3229,7 @@ int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *w
         bool again = false;
         for (uint32_t j = 0; j < i; j++) again |= want[j] == want[i];
         hipLaunchKernelGGL(jq::rmsnorm_rows, dim3(1), dim3(1024), 0, s, xc + at, pending && !again ? pending + at : nullptr, w_on,
-                           c.rms_eps, m->hn + (size_t)i * h, h);
+                           c.rms_eps, m->hn + (size_t)i * h, h, h);
     }
     // tie_word_embeddings conversions ship no output head (src/quantized_qwen3_moe.rs:739-743)
     const char *head = m->q.count("output.weight") ? "output.weight" : "token_embd.weight";
