@@ -4,6 +4,8 @@
 
 #include <sys/stat.h>
 
+#include <cstring>
+
 #include "gguf.hpp"
 #include "json.hpp"
 #include "kernels_graph.hpp"
@@ -11,6 +13,7 @@
 jq_model::~jq_model() {
     for (void *p : {(void *)logits, (void *)pick, (void *)pick_v, (void *)pick_i})
         if (p) (void)hipFree(p);
+    if (staged) (void)hipHostFree(staged);
 }
 
 int jq_model::init_outputs() {
@@ -18,8 +21,37 @@ int jq_model::init_outputs() {
         hipMalloc((void **)&pick_v, jq::ARGMAX_PARTS * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&pick_i, jq::ARGMAX_PARTS * sizeof(int)) != hipSuccess || reserve_logits(1))
         return fail("%s: logits allocation failed", arch);
+    (void)reserve_staged(vocab * sizeof(float));
     return 0;
 }
+
+// Logits for host memory leave by a kernel's stores to pinned memory and one copy there: the runtime's copy to pageable memory is
+// 25 us behind the step's last kernel, a launch, a wait and a copy of its own, where this is 7 (32000 floats; 151936: 44 and 21,
+// 1048576: 256 and 197).  Up to 4 MiB are kept; what is larger is bound by the copying either way.
+bool jq_model::reserve_staged(size_t bytes) {
+    constexpr size_t KEEP = (size_t)4 << 20;
+    if (bytes <= staged_bytes) return true;
+    if (bytes > KEEP) return false;
+    void *fresh = nullptr;
+    if (hipHostMalloc(&fresh, bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (staged) (void)hipHostFree(staged);  // (no step uses it: each waits for its own copy)
+    staged = (float *)fresh, staged_bytes = bytes;
+    return true;
+}
+
+namespace {
+
+__global__ __launch_bounds__(256) void copy_floats(const float *__restrict__ src, float *__restrict__ dst, size_t n) {
+    const size_t i = 4 * ((size_t)blockIdx.x * 256 + threadIdx.x);
+    if (i + 4 <= n) *(float4 *)(dst + i) = *(const float4 *)(src + i);
+    else
+        for (size_t j = i; j < n; j++) dst[j] = src[j];
+}
+
+}  // namespace
 
 int jq_model::reserve_logits(size_t rows) {
     if (rows <= logit_cap) return 0;
@@ -96,8 +128,14 @@ int jq_model_forward(jq_model *m, const uint32_t *tokens, uint32_t n_tokens, uin
     if (m->step(tokens, n_tokens, want, n_want, s)) return 1;
     m->n_past = pos + n_tokens;
     m->logit_rows = n_want;
-    if (logits && n_want) {
-        HIP_TRY(hipMemcpyAsync(logits, m->logits, (size_t)n_want * m->vocab * sizeof(float),
+    const size_t floats = (size_t)n_want * m->vocab;
+    if (logits && n_want && !logits_on_device && m->reserve_staged(floats * sizeof(float))) {
+        hipLaunchKernelGGL(copy_floats, dim3((unsigned)((floats + 1023) / 1024)), dim3(256), 0, s, m->logits, m->staged, floats);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(s));
+        memcpy(logits, m->staged, floats * sizeof(float));
+    } else if (logits && n_want) {
+        HIP_TRY(hipMemcpyAsync(logits, m->logits, floats * sizeof(float),
                                logits_on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
         if (!logits_on_device) HIP_TRY(hipStreamSynchronize(s));
     }

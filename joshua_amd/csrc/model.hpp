@@ -8,6 +8,8 @@ struct jq_model {
     uint32_t vocab = 0, n_ctx = 0;
     uint32_t n_past = 0;          // tokens fed so far
     float *logits = nullptr;      // [logit_rows][vocab]: the wanted positions of the last step
+    float *staged = nullptr;      // pinned host memory that a kernel writes logits to on their way to the caller's
+    size_t staged_bytes = 0;
     size_t logit_cap = 0, logit_rows = 0;
     uint32_t *pick = nullptr;
     float *pick_v = nullptr;      // the greedy pick's candidates, one per slice of the logits
@@ -25,6 +27,7 @@ struct jq_model {
     virtual void forget() {}
     int init_outputs();           // the pick's buffers and one row of logits
     int reserve_logits(size_t rows);
+    bool reserve_staged(size_t bytes);  // false: more than is kept for it, or no memory
 };
 
 namespace jqh {

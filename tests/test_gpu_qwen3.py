@@ -476,3 +476,19 @@ def test_long_context_with_five_query_heads_a_kv_head():
     got, ref = m.forward(toks[pos:pos + 16], pos), o.forward(toks[pos:pos + 16], pos)
     ok, e = close(got, ref)
     assert ok, e
+
+
+def test_logits_in_host_memory_are_those_on_the_device():
+    """One row, three rows (odd counts of floats) and 40, which are more than what leaves through pinned memory at once."""
+    import torch
+    from joshua_amd.capi import lib
+    m, _ = make(dict(CFG, n_layer=1, vocab=30001, n_ctx=64), 91, "q4_k")
+    t = np.random.default_rng(3).integers(0, 30001, 40).astype(np.uint32)
+    for want in ([39], [0, 17, 39], list(range(40)), [39]):
+        w = np.array(want, np.uint32)
+        host, dev = np.full((w.size, 30001), np.nan, np.float32), torch.full((w.size, 30001), float("nan"), device="cuda")
+        for ptr, on_device in ((host.ctypes.data, 0), (dev.data_ptr(), 1)):
+            m.reset()
+            assert lib().jq_model_forward(m._h, t.ctypes.data, t.size, 0, w.ctypes.data, w.size, ptr, on_device, None) == 0
+        torch.cuda.synchronize()
+        assert np.isfinite(host).all() and np.array_equal(host, dev.cpu().numpy()), want
