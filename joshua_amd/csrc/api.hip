@@ -233,7 +233,7 @@ int dispatch_q4k_dot4(const uint8_t *W, size_t row_bytes, const float *X, float 
             note_kernel("q4k_gemv_mfma_lds");
 #define JQ_MFMA_LDS(NORM, SWIGLU) \
     hipLaunchKernelGGL((jq::gemv_mfma_lds<jq::QvQ4K, NORM, SWIGLU>), dim3((unsigned)G), dim3(1024), 0, s, W, X, Y, wk.n, wk.G, \
-                       wk.rounds, wk.extra, nm.res, nm.w, nm.eps, nm.x_out, nm.hn_out)
+                       wk.rounds, wk.extra, nm.res, nm.w, nm.eps, nm.x_out, nm.hn_out, 0, 0)
             if (norm && swiglu) JQ_MFMA_LDS(true, true);
             else if (norm) JQ_MFMA_LDS(true, false);
             else if (swiglu) JQ_MFMA_LDS(false, true);
@@ -265,6 +265,26 @@ int dispatch_q4k_dot4(const uint8_t *W, size_t row_bytes, const float *X, float 
     const unsigned grid = (unsigned)std::min<size_t>(tiles, std::max<size_t>(cap, 1));
     note_kernel("q4k_gemv_dot4");
     hipLaunchKernelGGL(jq::q4k_gemv_dot4, dim3(grid), dim3((unsigned)(64 * nb)), 0, s, W, row_bytes, X, Y, (int)k, (int)n);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+// The product of a Q4_K matrix with one row of attention results that still lie as the parts of up to eight chunks of keys (as
+// attention_split leaves them): the merge happens in the product's start.  Rows of 4096 columns, heads of d, where
+// dispatch_q4k_dot4 takes the same kernel; -1 elsewhere, and where the environment asks for another one.  Behind more chunks each
+// workgroup's merge (of 16 KB a chunk) costs more than the launch it saves.
+int dispatch_q4k_merged(const jq_weight *w, const float *part, int n_chunks, int d, float *Y, hipStream_t s) {
+    static const bool asked = getenv("JQ_Q4K_DOT4") || getenv("JQ_Q4K_GEMV_MFMA") || getenv("JQ_Q4K_DOT4_GRID") || getenv("JQ_NO_MERGE_IN_GEMV");
+    const size_t n = w->n;
+    if (asked || w->type != JQ_TYPE_Q4_K || w->k != 4096 || w->row_bytes != (size_t)jq::QD_ROW || ((uintptr_t)w->dev & 15) != 0 || n < 2048 ||
+        n > 0x7FFFFFF0ull || n_chunks > 8 || d % 4 != 0)
+        return -1;
+    const size_t tiles = (n + 15) / 16, rounds_up = (tiles + 255) / 256, G = (tiles + rounds_up - 1) / rounds_up;
+    const jq::QvWork wk{(int)n, (int)G, (int)(tiles / G), (int)(tiles % G)};
+    note_kernel("q4k_gemv_mfma_lds");
+    auto *kern = n_chunks <= 4 ? jq::gemv_mfma_lds<jq::QvQ4K, false, false, 4> : jq::gemv_mfma_lds<jq::QvQ4K, false, false, 8>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)G), dim3(1024), 0, s, w->dev, part, Y, wk.n, wk.G, wk.rounds, wk.extra, nullptr, nullptr, 0.0f, nullptr,
+                       nullptr, n_chunks, d);
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -332,7 +352,7 @@ int dispatch_q2k_mfma(const uint8_t *W, size_t row_bytes, const float *X, float 
     const size_t tiles = (n + 15) / 16, rounds_up = (tiles + 255) / 256, G = (tiles + rounds_up - 1) / rounds_up;
     const jq::QvWork wk{(int)n, (int)G, (int)(tiles / G), (int)(tiles % G)};
     note_kernel("q2k_gemv_mfma_lds");
-    hipLaunchKernelGGL(jq::gemv_mfma_lds<jq::QvQ2K>, dim3((unsigned)G), dim3(1024), 0, s, W, X, Y, wk.n, wk.G, wk.rounds, wk.extra, nullptr, nullptr, 0.0f, nullptr, nullptr);
+    hipLaunchKernelGGL(jq::gemv_mfma_lds<jq::QvQ2K>, dim3((unsigned)G), dim3(1024), 0, s, W, X, Y, wk.n, wk.G, wk.rounds, wk.extra, nullptr, nullptr, 0.0f, nullptr, nullptr, 0, 0);
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -351,7 +371,7 @@ int launch_i8_gemv(const char *name, const uint8_t *W, size_t row_bytes, const f
     const jq::QvWork wk{(int)n, (int)G, (int)(tiles / G), (int)(tiles % G)};
     note_kernel(name);
     hipLaunchKernelGGL(jq::gemv_mfma_lds<F>, dim3((unsigned)G), dim3(1024), 0, s, W, X, Y, wk.n, wk.G, wk.rounds, wk.extra, nullptr,
-                       nullptr, 0.0f, nullptr, nullptr);
+                       nullptr, 0.0f, nullptr, nullptr, 0, 0);
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -455,7 +475,7 @@ int dispatch_q6k_dot4(const uint8_t *W, size_t row_bytes, const float *X, float 
         note_kernel(ng == 1 ? "q6k_gemv_mfma_lds" : "q6k_gemv_mfma_cols");
         if (ng == 1)
             hipLaunchKernelGGL(jq::gemv_mfma_lds<jq::QvQ6K>, dim3((unsigned)G), dim3(1024), 0, s, W, X, Y, wk.n, wk.G, wk.rounds, wk.extra,
-                               nullptr, nullptr, 0.0f, nullptr, nullptr);
+                               nullptr, nullptr, 0.0f, nullptr, nullptr, 0, 0);
         else if (ng == 2)
             hipLaunchKernelGGL((jq::gemv_mfma_cols<jq::QvQ6K, 2>), dim3((unsigned)G), dim3(1024), 0, s, W, X, Y, wk.n, wk.G, wk.rounds, wk.extra, wk.nb);
         else
@@ -3103,6 +3123,7 @@ int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *w
                    model_mm(m, p + ".attn_v.weight", m->hn, m->vb, T, s)) {
             return 1;
         }
+        bool o_done = false;
         if (split) {  // head norm, rotation and cache writes happen inside the attention kernel
             const int n_tri = (int)(T * nkv * n_chunks);
 #define JQ_ATT_SPLIT(D)                                                                                          \
@@ -3113,8 +3134,15 @@ int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *w
             else if (d == 128) JQ_ATT_SPLIT(128);
             else JQ_ATT_SPLIT(256);
 #undef JQ_ATT_SPLIT
-            hipLaunchKernelGGL(jq::attention_merge, dim3(T * nh), dim3(128), 2 * n_chunks * sizeof(float), s, m->part, m->att, d,
-                               n_chunks);
+            auto wo = m->q.find(p + ".attn_output.weight");
+            if (T == 1 && wo != m->q.end()) {
+                const int rc = dispatch_q4k_merged(wo->second, m->part, n_chunks, d, m->proj, s);
+                if (rc > 0) return 1;
+                o_done = rc == 0;
+            }
+            if (!o_done)
+                hipLaunchKernelGGL(jq::attention_merge, dim3(T * nh), dim3(128), 2 * n_chunks * sizeof(float), s, m->part, m->att, d,
+                                   n_chunks);
         } else {
             // (four workgroups or more to a compute unit, no more parts than waves have heads)
             const unsigned parts = std::min((unsigned)(nh + 2 * nkv + 3) / 4, std::max(1u, 1024 / (unsigned)T));
@@ -3144,7 +3172,7 @@ int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *w
             else JQ_ATT_TILES(8);
 #undef JQ_ATT_TILES
         }
-        if (model_mm(m, p + ".attn_output.weight", m->att, m->proj, T, s)) return 1;
+        if (!o_done && model_mm(m, p + ".attn_output.weight", m->att, m->proj, T, s)) return 1;
         if (c.n_expert) {
             // x + moe(norm(x)) (reference: src/quantized_qwen3_moe.rs:806-812)
             jq_moe *moe = m->moe[l];

@@ -369,6 +369,10 @@ __device__ __forceinline__ void async_load16_s(const uint8_t *sbase, uint32_t vo
 //     arguments of their own so that the leading ones arrive preloaded.
 //   * SWIGLU: the matrix holds gate and up rows alternately (row 2j gate_j, row 2j + 1 up_j) and
 //     Y[j] = silu(gate_j . x) * (up_j . x), n / 2 values (reference: src/quantized_qwen3_moe.rs:397-401).
+//   * MERGE: the activations are the parts that attention_split left of a head's chunks of keys (up to MERGE of them), and
+//     every wave merges the four values a lane it prepares, by attention_merge's arithmetic.  The reads are ordinary ones in front
+//     of the first tile, which starts that much later: 4096 x 4096 behind 4 chunks of 32 heads 6.5 us where the merging
+//     launch took 3.3, the product 4.7, and there was the gap between them.
 // The kernel's LDS, one block of bytes so that a launch which runs two kernels' bodies side by side can give both the
 // same block: the ring, the partial sums [FL][16][68], the waves' staging areas where the ring has no room for
 // them, the waves' sums of squares.
@@ -382,12 +386,39 @@ struct GemvMfmaLds {
     static constexpr int BYTES = SS_AT + 64;
 };
 
+// Elements col .. col + 3 of sum_ch exp(m_ch - m) acc_ch / sum_ch exp(m_ch - m) l_ch, the parts (m, l, acc[d]) of head col / d's
+// chunks lying one behind the other (attention_merge).
+template <int CHUNKS>
+__device__ __forceinline__ float4 merged_parts(const float *__restrict__ part, int n_chunks, int d, int col) {
+    const int h = col / d;
+    const float *pp = part + (size_t)h * n_chunks * (d + 2);
+    float2 ml[CHUNKS], lo[CHUNKS], hi[CHUNKS];
+#pragma unroll
+    for (int j = 0; j < CHUNKS; j++) {
+        const float *p = pp + (size_t)min(j, n_chunks - 1) * (d + 2);
+        ml[j] = *(const float2 *)p;
+        lo[j] = *(const float2 *)(p + 2 + (col - h * d)), hi[j] = *(const float2 *)(p + 4 + (col - h * d));
+    }
+    float top = -INFINITY, tot = 0.0f;
+    float4 a = float4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < CHUNKS; j++) top = fmaxf(top, ml[j].x);  // (past the last chunk: that one again)
+#pragma unroll
+    for (int j = 0; j < CHUNKS; j++) {
+        const float w = j < n_chunks && ml[j].y > 0.0f ? expf(ml[j].x - top) : 0.0f;
+        if (j < n_chunks) tot = fmaf(ml[j].y, w, tot);
+        if (w > 0.0f) a.x = fmaf(w, lo[j].x, a.x), a.y = fmaf(w, lo[j].y, a.y), a.z = fmaf(w, hi[j].x, a.z), a.w = fmaf(w, hi[j].y, a.w);
+    }
+    return float4{a.x / tot, a.y / tot, a.z / tot, a.w / tot};
+}
+
 // `b`: the workgroup's number among the G of this product.
-template <class F, bool NORM, bool SWIGLU>
+template <class F, bool NORM, bool SWIGLU, int MERGE = 0>
 __device__ __forceinline__ void gemv_mfma_lds_body(uint8_t *lds, int b, const uint8_t *__restrict__ W,
                                                    const float *__restrict__ X, float *__restrict__ Y, int n, int G,
                                                    int rounds, int extra, const float *nm_res, const float *nm_w,
-                                                   float nm_eps, float *nm_x_out, float *nm_hn_out) {
+                                                   float nm_eps, float *nm_x_out, float *nm_hn_out, int mg_chunks = 0, int mg_d = 0) {
+    static_assert(MERGE == 0 || !NORM, "parts or a residual row");
     typedef GemvMfmaLds<F> L;
     constexpr int SLOTS = F::SLOTS, FL = L::FL;      // ring slots (three: two tiles in flight); tiles a flush
     static_assert(!NORM || (2048 <= F::ROW_LDS && F::SLOTS == 3), "the norm's operands wait in a wave's row of ring slot 1");
@@ -423,7 +454,13 @@ __device__ __forceinline__ void gemv_mfma_lds_body(uint8_t *lds, int b, const ui
     // counted by hand)
     uint32_t *stage = (uint32_t *)(STAGE_IN_RING ? ring + (SLOTS - 1) * SLOT_BYTES + wave * F::ROW_LDS : stage_mem + wave * STAGE);
     float *x_raw = (float *)((uint8_t *)stage + F::STAGE_BYTES);
-    async_load16(X + 256 * wave + 4 * lane, lds_offset_of(x_raw));
+    float4 v;
+    if constexpr (MERGE > 0) {
+        v = merged_parts<MERGE>(X, mg_chunks, mg_d, 256 * wave + 4 * lane);
+        asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w));  // here, and not behind the tiles' loads
+    } else {
+        async_load16(X + 256 * wave + 4 * lane, lds_offset_of(x_raw));
+    }
     // norm weight and residual columns wait in the wave's row of ring slot 1, which no tile enters before the
     // activations are prepared
     float *w_raw = (float *)(ring + SLOT_BYTES + wave * F::ROW_LDS), *r_raw = w_raw + 256;
@@ -439,8 +476,10 @@ __device__ __forceinline__ void gemv_mfma_lds_body(uint8_t *lds, int b, const ui
     // (asked for in front of it, tile 1 delays the preparation: a wave stands at a load until the memory
     // pipeline accepts it; measured slower both on a resident activation row and behind another kernel)
     fetch(0);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
-    float4 v = *(const float4 *)&x_raw[4 * lane];
+    if constexpr (MERGE == 0) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+        v = *(const float4 *)&x_raw[4 * lane];
+    }
     if (NORM) {
         if (nm_res) {
             const float4 rr = *(const float4 *)&r_raw[4 * lane];
@@ -509,14 +548,14 @@ __device__ __forceinline__ void gemv_mfma_lds_body(uint8_t *lds, int b, const ui
     }
 }
 
-template <class F, bool NORM = false, bool SWIGLU = false>
+template <class F, bool NORM = false, bool SWIGLU = false, int MERGE = 0>
 __global__ __launch_bounds__(1024) void gemv_mfma_lds(const uint8_t *__restrict__ W, const float *__restrict__ X,
                                                       float *__restrict__ Y, int n, int G, int rounds, int extra,
                                                       const float *nm_res, const float *nm_w, float nm_eps,
-                                                      float *nm_x_out, float *nm_hn_out) {
+                                                      float *nm_x_out, float *nm_hn_out, int mg_chunks, int mg_d) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[GemvMfmaLds<F>::BYTES];
-    gemv_mfma_lds_body<F, NORM, SWIGLU>(lds, (int)blockIdx.x, W, X, Y, n, G, rounds, extra, nm_res, nm_w, nm_eps, nm_x_out,
-                                        nm_hn_out);
+    gemv_mfma_lds_body<F, NORM, SWIGLU, MERGE>(lds, (int)blockIdx.x, W, X, Y, n, G, rounds, extra, nm_res, nm_w, nm_eps, nm_x_out,
+                                               nm_hn_out, mg_chunks, mg_d);
 }
 
 // The same kernel for rows of more than 16 super-blocks (up to 16 NG): a tile is 16 rows x one pass of 16

@@ -492,3 +492,19 @@ def test_logits_in_host_memory_are_those_on_the_device():
             assert lib().jq_model_forward(m._h, t.ctypes.data, t.size, 0, w.ctypes.data, w.size, ptr, on_device, None) == 0
         torch.cuda.synchronize()
         assert np.isfinite(host).all() and np.array_equal(host, dev.cpu().numpy()), want
+
+
+@pytest.mark.parametrize("n_head,n_kv,d", [(64, 8, 64), (32, 4, 128), (16, 16, 256)])
+def test_output_projection_that_merges_the_attention_of_a_step(n_head, n_kv, d):
+    """Attention results of 4096 values into a Q4_K output projection: one to eight chunks of 64 keys are merged in the product's
+    start (up to four, and up to eight), nine by a launch of their own."""
+    cfg = dict(CFG, n_layer=1, hidden=2048, n_head=n_head, n_kv_head=n_kv, head_dim=d, ffn=256, vocab=512, n_ctx=520)
+    m, o = make(cfg, 95, "q4_k")
+    toks = np.random.default_rng(16).integers(0, 512, 520).tolist()
+    pos = 0
+    for prompt, steps in ((3, 2), (57, 4), (120, 6), (65, 3), (190, 4), (55, 6)):
+        for n in [prompt] + [1] * steps:
+            ok, e = close(m.forward(toks[pos:pos + n], pos), o.forward(toks[pos:pos + n], pos))
+            assert ok, f"pos {pos}: {e}"
+            pos += n
+    assert pos > 512
