@@ -184,18 +184,22 @@ int dispatch_q4k_dot4(const uint8_t *W, size_t row_bytes, const float *X, float 
     // rows, with the decoder's norm form (4608 x 2048, q|k of a Qwen3-30B-A3B-shaped layer with residual add and RMSNorm:
     // one launch where there were rmsnorm_rows and the one-shot matrix-core GEMV).  JQ_Q4K_GEMV_TILE = 0 switches it off.
     static const char *tile_env = getenv("JQ_Q4K_GEMV_TILE");
-    if (mode == "auto" && !swiglu && !(tile_env && tile_env[0] == '0') && nb == 8 && k == 2048 && row_bytes == nb * 144 &&
+    // Six super-blocks (DeepSeek-V3's queries behind their down-projection) the same way: 24576 x 1536 6.0 us against 7.8 for the one-shot
+    // kernel, 4096 x 1536 4.0 against 5.4, and the norm rides along.
+    if (mode == "auto" && !swiglu && !(tile_env && tile_env[0] == '0') && (nb == 8 || nb == 6) && k == 256 * nb && row_bytes == nb * 144 &&
         n >= 64 && n <= 0x7FFFFFF0ull) {
         const jq::QdNorm nm = norm ? *norm : jq::QdNorm{};
-        constexpr int lds = jq::gemv_mfma_tile_lds<jq::QvQ4K, 8>();
-        static_assert(lds <= 64 * 1024, "within the default dynamic LDS limit");
+        static_assert(jq::gemv_mfma_tile_lds<jq::QvQ4K, 8>() <= 64 * 1024, "within the default dynamic LDS limit");
         note_kernel("q4k_gemv_mfma_tile");
-        if (norm)
-            hipLaunchKernelGGL((jq::gemv_mfma_tile<jq::QvQ4K, 8, true>), dim3((unsigned)((n + 15) / 16)), dim3(512), lds, s, W, X, Y,
-                               (int)n, nm.res, nm.w, nm.eps, nm.x_out, nm.hn_out);
-        else
-            hipLaunchKernelGGL((jq::gemv_mfma_tile<jq::QvQ4K, 8, false>), dim3((unsigned)((n + 15) / 16)), dim3(512), lds, s, W, X, Y,
-                               (int)n, nullptr, nullptr, 0.0f, nullptr, nullptr);
+        auto launch = [&](auto kern, int waves, int lds) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)((n + 15) / 16)), dim3(64 * waves), lds, s, W, X, Y, (int)n, nm.res, nm.w, nm.eps, nm.x_out,
+                               nm.hn_out);
+        };
+        constexpr int lds8 = jq::gemv_mfma_tile_lds<jq::QvQ4K, 8>(), lds6 = jq::gemv_mfma_tile_lds<jq::QvQ4K, 6>();
+        if (nb == 8 && norm) launch(jq::gemv_mfma_tile<jq::QvQ4K, 8, true>, 8, lds8);
+        else if (nb == 8) launch(jq::gemv_mfma_tile<jq::QvQ4K, 8, false>, 8, lds8);
+        else if (norm) launch(jq::gemv_mfma_tile<jq::QvQ4K, 6, true>, 6, lds6);
+        else launch(jq::gemv_mfma_tile<jq::QvQ4K, 6, false>, 6, lds6);
         HIP_TRY(hipGetLastError());
         return 0;
     }
@@ -2585,10 +2589,19 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
         } else if (dispatch_matmul(m->q->type, m->q->dev, m->q->row_bytes, x, m->t1, S, c.n_embd, c.q_lora_rank, s)) {
             return 1;
         }
-        hipLaunchKernelGGL(jq::rmsnorm_rows, dim3((unsigned)S), dim3(1024), 0, s, m->t1, (const float *)nullptr,
-                           (const float *)m->q_a_norm, c.rms_eps, m->t1n, (int)c.q_lora_rank, (int)t1_stride);
-        HIP_TRY(hipGetLastError());
-        if (dispatch_matmul(m->q_b->type, m->q_b->dev, m->q_b->row_bytes, m->t1n, m->qv, S, c.q_lora_rank, nh * qd, s)) return 1;
+        // one token over Q4_K: the norm in the product's launch, where a kernel has both
+        int both_rc = -1;
+        if (S == 1 && m->q_b->type == JQ_TYPE_Q4_K) {
+            const jq::QdNorm norm{nullptr, m->q_a_norm, c.rms_eps, m->t1n, nullptr};
+            both_rc = dispatch_q4k_dot4(m->q_b->dev, m->q_b->row_bytes, m->t1, m->qv, c.q_lora_rank, nh * qd, s, &norm);
+            if (both_rc > 0) return 1;
+        }
+        if (both_rc < 0) {
+            hipLaunchKernelGGL(jq::rmsnorm_rows, dim3((unsigned)S), dim3(1024), 0, s, m->t1, (const float *)nullptr,
+                               (const float *)m->q_a_norm, c.rms_eps, m->t1n, (int)c.q_lora_rank, (int)t1_stride);
+            HIP_TRY(hipGetLastError());
+        }
+        if (both_rc < 0 && dispatch_matmul(m->q_b->type, m->q_b->dev, m->q_b->row_bytes, m->t1n, m->qv, S, c.q_lora_rank, nh * qd, s)) return 1;
     } else if (dispatch_matmul(m->q->type, m->q->dev, m->q->row_bytes, x, m->qv, S, c.n_embd, nh * qd, s)) {
         return 1;
     }

@@ -30,9 +30,9 @@ __device__ __forceinline__ void gemv_mfma_tile_body(uint8_t *gemv_tile_lds, int 
                                                     const float *__restrict__ X, float *__restrict__ Y, int n,
                                                     const float *nm_res, const float *nm_w, float nm_eps, float *nm_x_out,
                                                     float *nm_hn_out) {
-    static_assert(NB == 2 || NB == 4 || NB == 8 || NB == 16, "a row of 2, 4, 8 or 16 super-blocks");
+    static_assert(NB >= 2 && NB <= 16, "a row of 2 to 16 super-blocks");
     constexpr int RB = NB * F::BLOCK, ROW_LDS = moe_mfma_row_lds(RB), LOADS = (RB + 1023) / 1024;
-    constexpr int STG = gemv_mfma_tile_stage<F, NB>(), RPW = 16 / NB;  // tile rows a wave copies
+    constexpr int STG = gemv_mfma_tile_stage<F, NB>(), RPW = (16 + NB - 1) / NB;  // tile rows a wave copies (past the last: that one again)
     static_assert(RB % 16 == 0, "rows are copied 16 bytes a lane");
     const uint64_t *table = qv_stage_table<F>(gemv_tile_lds);
     uint8_t *tile = gemv_tile_lds + qv_table_bytes<F>();  // [16][ROW_LDS]
@@ -51,7 +51,7 @@ __device__ __forceinline__ void gemv_mfma_tile_body(uint8_t *gemv_tile_lds, int 
     const uint32_t tile0 = lds_offset_of(tile);
 #pragma unroll
     for (int i = 0; i < RPW; i++) {
-        const int rr = wave + NB * i;
+        const int rr = min(wave + NB * i, 15);
         const uint8_t *src = W + (size_t)min(row0 + rr, n - 1) * RB;
         const uint32_t dst = tile0 + (uint32_t)rr * ROW_LDS;
 #pragma unroll
@@ -71,7 +71,7 @@ __device__ __forceinline__ void gemv_mfma_tile_body(uint8_t *gemv_tile_lds, int 
         ss = wave_sum(ss);
         if (lane == 0) ss_lds[wave] = ss;
         const float4 g = *(const float4 *)&w_raw[4 * lane];
-        if (first) *(float4 *)(nm_x_out + 256 * wave + 4 * lane) = v;
+        if (first && nm_x_out) *(float4 *)(nm_x_out + 256 * wave + 4 * lane) = v;
         v = float4{v.x * g.x, v.y * g.y, v.z * g.z, v.w * g.w};
     }
     typename F::Acts acts = F::prepare(v, stage, lane);
@@ -95,6 +95,7 @@ __device__ __forceinline__ void gemv_mfma_tile_body(uint8_t *gemv_tile_lds, int 
 #pragma unroll
     for (int q = 0; q < RPW; q++) {
         const int rr = wave + NB * q;
+        if (16 % NB != 0 && rr >= 16) break;  // (the same for the whole wave)
         float sum = lane < 4 * NB ? part[rr * 68 + lane] : 0.0f;
         sum = wave_sum(sum);
         if (lane == 0 && row0 + rr < n) Y[row0 + rr] = sum;

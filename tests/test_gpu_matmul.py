@@ -1150,6 +1150,20 @@ def test_q4k_mfma_gemv_over_rows_of_2048(n):
     assert close(got, oracle.matmul_t(capi.Q4_K, (1, k, n), lhs, blocks, avx2=oracle.have_avx2()))
 
 
+@pytest.mark.parametrize("n", [64, 100, 2048 + 9, 24576 - 7])
+def test_q4k_mfma_gemv_over_rows_of_1536(n):
+    """Six waves a tile, which copy its 16 rows in three turns, the last of them part-filled."""
+    k = 1536
+    blocks = make_blocks(capi.Q4_K, n, k, 530 + n % 89)
+    lhs = synth.normal(531, (1, k))
+    w = capi.Weight.upload(capi.Q4_K, blocks, n, k)
+    got = w.matmul_t(1, lhs)
+    assert capi.last_kernel() == "q4k_gemv_mfma_tile"
+    assert close(got, oracle.matmul_t(capi.Q4_K, (1, k, n), lhs, blocks, avx2=oracle.have_avx2()))
+    lhs[0, 1500] = np.nan
+    assert np.all(np.isnan(w.matmul_t(1, lhs)))
+
+
 @pytest.mark.parametrize("qtype,kernel", [(capi.Q6_K, "q6k_gemv_mfma_tile"), (capi.Q8_0, "q8_0_gemv_mfma_tile"),
                                           (capi.Q5_K, "q5k_gemv_mfma_tile")])
 @pytest.mark.parametrize("n", [64, 512 + 7, 16 * 700 + 3])

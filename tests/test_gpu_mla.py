@@ -442,3 +442,15 @@ def test_a_captured_call_behind_tokens_that_were_not_expanded():
     del graph
     torch.cuda.synchronize()
     capi.stream_release(stream.cuda_stream)
+
+
+def test_one_token_whose_query_norm_rides_in_the_product():
+    """A Q4_K query up-projection of 1536 columns: RMSNorm and product of a single token are one launch; several tokens, and other
+    formats, take two."""
+    c = cfg(n_embd=256, n_head=4, q_lora_rank=1536, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=128)
+    for qtype in (capi.Q4_K, capi.Q8_0):
+        ref, dev = build(c, qtype=qtype, seed=960)
+        x, pos = normal(30, (12, 256)), 0
+        for n in (3, 1, 1, 6, 1):
+            assert close(dev.forward(x[pos:pos + n], pos), ref.forward(x[pos:pos + n], pos)), (qtype, pos)
+            pos += n
