@@ -67,6 +67,11 @@ __device__ __forceinline__ float h6_bf16_value(uint32_t b) { return __builtin_bi
 
 // grid (k / 256 super-blocks, groups of 16 activation rows), 128 threads, one sub-block each.  Rows from m_rows on are
 // zero operands.  With PAIRS the activations are silu(gate) * up over rows of 2 k floats in which gate_j and up_j alternate.
+//
+// Memory bounds it.  A lane's own sub-block is 128 bytes, so its loads touch a line a lane.  That costs nothing while the
+// caches hold the rest of the line (8.0 us at 512 x 14336, either way), but the pairs' 256 bytes a lane do not survive there: 2048 x
+// 12288 pairs took 86 us so and take 50 with whole rows of memory turned by the LDS, of 54 that 276 MB take in a large copy.  For
+// plain rows the detour costs 1 us.  rows_sh's padding: 16 lanes that read 16 rows at one column take 16 different groups of banks.
 template <bool PAIRS>
 __global__ __launch_bounds__(128) void kq_gemm_h6_prep(const float *__restrict__ X, int m_rows, int k, uint8_t *__restrict__ out) {
     __shared__ float amax_sh[2][16], xs_sh[16][8];
@@ -74,12 +79,24 @@ __global__ __launch_bounds__(128) void kq_gemm_h6_prep(const float *__restrict__
     const int b = blockIdx.x, row = 16 * (int)blockIdx.y + i;
     uint8_t *rec = out + ((size_t)blockIdx.y * gridDim.x + b) * H6_REC;
     float v[32];
-    if (row < m_rows && PAIRS) {
-        const float4 *src = (const float4 *)(X + 2 * ((size_t)row * k + 256 * b + 32 * (4 * h + g)));
+    if constexpr (PAIRS) {
+        __shared__ __align__(16) float rows_sh[16][260];
 #pragma unroll
-        for (int q = 0; q < 16; q++) {
-            const float4 a = src[q];
-            v[2 * q] = silu(a.x) * a.y, v[2 * q + 1] = silu(a.z) * a.w;
+        for (int q = 0; q < 8; q++) {
+            const int r = 8 * h + q, at = 16 * (int)blockIdx.y + r;
+            float4 a = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (at < m_rows) {
+                const float4 *src = (const float4 *)(X + 2 * ((size_t)at * k + 256 * b + 4 * lane));
+                const float4 u = src[0], w = src[1];
+                a = {silu(u.x) * u.y, silu(u.z) * u.w, silu(w.x) * w.y, silu(w.z) * w.w};
+            }
+            *(float4 *)&rows_sh[r][4 * lane] = a;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const float4 a = *(const float4 *)&rows_sh[i][32 * (4 * h + g) + 4 * q];
+            v[4 * q] = a.x, v[4 * q + 1] = a.y, v[4 * q + 2] = a.z, v[4 * q + 3] = a.w;
         }
     } else if (row < m_rows) {
         const float4 *src = (const float4 *)(X + (size_t)row * k + 256 * b + 32 * (4 * h + g));
