@@ -195,11 +195,11 @@ int dispatch_q4k_dot4(const uint8_t *W, size_t row_bytes, const float *X, float 
             hipLaunchKernelGGL(kern, dim3((unsigned)((n + 15) / 16)), dim3(64 * waves), lds, s, W, X, Y, (int)n, nm.res, nm.w, nm.eps, nm.x_out,
                                nm.hn_out);
         };
-        constexpr int lds8 = jq::gemv_mfma_tile_lds<jq::QvQ4K, 8>(), lds6 = jq::gemv_mfma_tile_lds<jq::QvQ4K, 6>();
+        constexpr int lds8 = jq::gemv_mfma_tile_lds<jq::QvQ4K, 8>(), lds6 = jq::gemv_mfma_tile_lds<jq::QvQ4KFine, 6>();
         if (nb == 8 && norm) launch(jq::gemv_mfma_tile<jq::QvQ4K, 8, true>, 8, lds8);
         else if (nb == 8) launch(jq::gemv_mfma_tile<jq::QvQ4K, 8, false>, 8, lds8);
-        else if (norm) launch(jq::gemv_mfma_tile<jq::QvQ4K, 6, true>, 6, lds6);
-        else launch(jq::gemv_mfma_tile<jq::QvQ4K, 6, false>, 6, lds6);
+        else if (norm) launch(jq::gemv_mfma_tile<jq::QvQ4KFine, 6, true>, 6, lds6);
+        else launch(jq::gemv_mfma_tile<jq::QvQ4KFine, 6, false>, 6, lds6);
         HIP_TRY(hipGetLastError());
         return 0;
     }
@@ -678,7 +678,7 @@ int dispatch_q4k_rows16(const uint8_t *W, size_t row_bytes, const float *X, floa
     return 0;
 }
 
-// Q4_K, Q6_K, Q2_K and Q8_0 with many activation rows on the int8 matrix cores: the activations as two int8 planes per
+// Many activation rows on the int8 matrix cores (Q4_K up to 127 of them, dispatch_gemm_h6's products from there on): the activations as two int8 planes per
 // 256-element super-block in the call scratch of the stream, then kq_gemm_i8 with the workgroup shape and the
 // split over k that an estimate fitted to measurements prefers.  Returns -1 when the shape is outside its
 // reach or the product is tiny.  JQ_Q4K_GEMM_I8 = 0 switches it off; JQ_Q4K_GEMM_I8_SHAPE and _SPLITS force the
@@ -1213,7 +1213,7 @@ int jq_matmul_t_f16(const jq_weight *w, size_t m, const uint16_t *lhs, size_t lh
     if (!lhs || !dst) return fail("jq_matmul_t_f16: lhs/dst is null");
     hipStream_t s = (hipStream_t)stream;
     // f16 -> f32, the f32 product, f32 -> f16 (reference: src/mxfp4.rs:242-258, src/iq2xxs.rs:396-412): the f32
-    // operands live in the stream's second kept buffer (up to 64 MB; a stream-ordered allocation beyond), so
+    // operands live in the stream's second kept buffer (up to 128 MB; a stream-ordered allocation beyond), so
     // device callers are not synchronised and a call on a warmed-up stream allocates nothing
     const size_t h16_bytes = ptrs_are_device ? 0 : std::max(lhs_len, dst_len) * sizeof(uint16_t);
     const size_t x_bytes = (lhs_len * sizeof(float) + 255) & ~(size_t)255, y_bytes = (dst_len * sizeof(float) + 255) & ~(size_t)255;
@@ -2472,10 +2472,15 @@ size_t mla_absorbed_tokens(const jq_mla *m, size_t S) {
 }
 
 // Floats of a result row of q_a and kv_a as one product, where a call of S tokens takes them so: always for one token, for more
-// where the rows keep to 16 bytes (rmsnorm_rows).  0: two products.  512 tokens of DeepSeek-V3's size: 35 + 30 us, as one 44.
+// where the rows keep to 16 bytes (rmsnorm_rows) and kv_a by itself has the 64 tiles times splits from which on the GEMMs take it
+// (dispatch_gemm_i8): products with fewer keep more digits of the activations (3e-7 of the result against 2.7e-5), which the
+// latents would lose.  0: two products.  512 tokens of DeepSeek-V3's size: 35 + 30 us, as one 44.
 size_t mla_qa_kva(const jq_mla *m, size_t S) {
-    const size_t n = m->qa_kva ? m->q->n + m->kv_a->n : 0;
-    return S == 1 || n % 4 == 0 ? n : 0;
+    if (!m->qa_kva) return 0;
+    const size_t n = m->q->n + m->kv_a->n, k = m->cfg.n_embd;
+    if (S == 1) return n;
+    const size_t tiles = (S + 127) / 128 * ((m->kv_a->n + 63) / 64) * std::max<size_t>(1, std::min<size_t>(k / 1024, 8));
+    return n % 4 == 0 && k % 256 == 0 && S >= 128 && tiles >= 64 ? n : 0;
 }
 
 // Scratch for calls of up to T tokens, of which up to `absorbed` in absorbed form.  Buffers that are outgrown are retired,
@@ -2505,7 +2510,7 @@ int mla_reserve(jq_mla *m, size_t T, size_t absorbed) {
         HIP_TRY(hipMalloc((void **)&m->t1n, T * c.q_lora_rank * sizeof(float)));
     }
     HIP_TRY(hipMalloc((void **)&m->qv, T * c.n_head * qd * sizeof(float)));
-    if (!mla_qa_kva(m, 2)) HIP_TRY(hipMalloc((void **)&m->comp, T * (c.kv_lora_rank + c.qk_rope_head_dim) * sizeof(float)));
+    HIP_TRY(hipMalloc((void **)&m->comp, T * (c.kv_lora_rank + c.qk_rope_head_dim) * sizeof(float)));
     HIP_TRY(hipMalloc((void **)&m->ctx, T * c.n_head * c.v_head_dim * sizeof(float)));
     m->cap_tokens = T;
     return 0;

@@ -116,6 +116,74 @@ struct QvQ4K {
     __device__ static __forceinline__ float block_dot_lane(const uint8_t *blk, const Acts &a, int c) { return qv_block_dot_lane(blk, a, c); }
 };
 
+// Q4_K with the activations in 23-bit fixed point per sub-block, X = 65536 X2 + 256 X1 + X0 in three signed byte planes (the
+// bytes of the f32 word x / s + 2^23 + 2^22 + 0x8080 about 128, 128 and 64): for the rows whose other kernel, q4k_gemv_mfma
+// (kernels_mfma_q4k.hpp), holds its activations so.  Rows 4c + p of the A operand are plane p of sub-block 2c, in a second product of
+// 2c + 1, so that the even and the odd sub-block take two MFMAs each; |sum q X| <= 32 x 15 x 4161407 < 2^31.  Products and sums
+// against 64 bits: 3e-7 (1536 columns, as q4k_gemv_mfma), with the two planes above 2.1e-5.
+struct QvQ4KFine {
+    static constexpr int BLOCK = QvQ4K::BLOCK, STAGE_BYTES = (3 * 64 + 8) * 4 + 8 * 8;  // planes, zeros, {s, sum of X} a sub-block
+    static constexpr float RANGE = 4161407.0f, MAGIC = 12615808.0f;                   // 2^22 - 1 - 0x8080; 2^23 + 2^22 + 0x8080
+    struct Acts {
+        qv_i4 a_even[2], a_odd[2];
+        float s_e, s_o, xs_e, xs_o;
+    };
+    __device__ static __forceinline__ void scale(Acts &a, float f) { a.s_e *= f, a.s_o *= f; }
+    __device__ static __forceinline__ Acts prepare(const float4 v, uint32_t *stage, int lane) {
+        const int r = lane & 15, c = lane >> 4;
+        float2 *side = (float2 *)(stage + 200);
+        const float amax = max_row8(fmaxf(fmaxf(mag_or_inf(v.x), mag_or_inf(v.y)), fmaxf(mag_or_inf(v.z), mag_or_inf(v.w))));
+        const float top = fmaxf(amax, 1e-30f), inv = RANGE / top;  // (finite: a smaller amax is 2^-23 x 1e-30 off at most)
+        const uint32_t t0 = __builtin_bit_cast(uint32_t, fmaf(v.x, inv, MAGIC)), t1 = __builtin_bit_cast(uint32_t, fmaf(v.y, inv, MAGIC));
+        const uint32_t t2 = __builtin_bit_cast(uint32_t, fmaf(v.z, inv, MAGIC)), t3 = __builtin_bit_cast(uint32_t, fmaf(v.w, inv, MAGIC));
+        const int sum = isum_row8((int)(t0 + t1 + t2 + t3 - 4 * __builtin_bit_cast(uint32_t, MAGIC)));
+        const uint32_t lo01 = __builtin_amdgcn_perm(t1, t0, 0x05010400u), lo23 = __builtin_amdgcn_perm(t3, t2, 0x05010400u);
+        const uint32_t hi01 = __builtin_amdgcn_perm(t1, t0, 0x0c0c0602u), hi23 = __builtin_amdgcn_perm(t3, t2, 0x0c0c0602u);
+        stage[lane] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u) ^ 0x80808080u;
+        stage[64 + lane] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u) ^ 0x80808080u;
+        stage[128 + lane] = (__builtin_amdgcn_perm(hi23, hi01, 0x05040100u) + 0x40404040u) ^ 0x80808080u;
+        if (lane < 8) stage[192 + lane] = 0;
+        if ((lane & 7) == 0) side[lane >> 3] = float2{amax < INFINITY ? top / RANGE : NAN, (float)sum};
+        asm volatile("" ::: "memory");  // (written as scalars, read back as vectors)
+        const bool mine = (r >> 2) == c && (r & 3) < 3;
+        const uint32_t *ev = mine ? stage + 64 * (r & 3) + 16 * c : stage + 192, *od = mine ? ev + 8 : ev;
+        Acts a;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint4 x = *(const uint4 *)(ev + 4 * h), y = *(const uint4 *)(od + 4 * h);
+            a.a_even[h] = qv_i4{(int)x.x, (int)x.y, (int)x.z, (int)x.w};
+            a.a_odd[h] = qv_i4{(int)y.x, (int)y.y, (int)y.z, (int)y.w};
+        }
+        const float2 fe = side[2 * c], fo = side[2 * c + 1];
+        a.s_e = fe.x, a.xs_e = fe.y, a.s_o = fo.x, a.xs_o = fo.y;
+        asm volatile("" ::: "memory");
+        return a;
+    }
+    __device__ static __forceinline__ float joined(qv_i4 C) {
+        return (float)(int)(((uint32_t)C[2] << 16) + ((uint32_t)C[1] << 8) + (uint32_t)C[0]);
+    }
+    __device__ static __forceinline__ float block_dot_lane(const uint8_t *blk, const Acts &a, int c) {
+        const uint4 hdr = *(const uint4 *)blk;
+        qv_i4 E = {0, 0, 0, 0}, O = {0, 0, 0, 0};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint4 q = *(const uint4 *)(blk + 16 + 32 * c + 16 * h);
+            constexpr uint32_t LOW = 0x0F0F0F0Fu;
+            E = __builtin_amdgcn_mfma_i32_16x16x64_i8(a.a_even[h], qv_i4{(int)(q.x & LOW), (int)(q.y & LOW), (int)(q.z & LOW), (int)(q.w & LOW)}, E, 0, 0, 0);
+            O = __builtin_amdgcn_mfma_i32_16x16x64_i8(a.a_odd[h], qv_i4{(int)(q.x >> 4 & LOW), (int)(q.y >> 4 & LOW), (int)(q.z >> 4 & LOW), (int)(q.w >> 4 & LOW)},
+                                                      O, 0, 0, 0);
+        }
+        uint32_t scp, mnp;
+        q4k_scale_min_pair(hdr.y, hdr.z, hdr.w, c, scp, mnp);
+        const float d = f16_bits(hdr.x), dmin = f16_bits(hdr.x >> 16);
+        const float d_e = d * (float)(scp & 0xFFu), d_o = d * (float)((scp >> 8) & 0xFFu);
+        const float m_e = dmin * (float)(mnp & 0xFFu), m_o = dmin * (float)((mnp >> 8) & 0xFFu);
+        // (the scale last: its rounding is then one of the difference, not of the two terms that nearly cancel)
+        const float even = fmaf(d_e, joined(E), -m_e * a.xs_e), odd = fmaf(d_o, joined(O), -m_o * a.xs_o);
+        return fmaf(even, a.s_e, odd * a.s_o);
+    }
+};
+
 // The same for the kernel that keeps the operands of four columns: the accumulator start as the one word
 // that is not zero, and the four scale factors of a lane group in LDS (16 bytes a wave, column and lane group,
 // read back once a tile), 18 registers a column instead of 24.

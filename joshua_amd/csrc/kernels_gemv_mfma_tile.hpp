@@ -3,7 +3,8 @@
 // tile and streams tiles through a ring; here a tile of 16 rows is a few KB, so a workgroup of NB waves takes ONE
 // tile, wave w its column w, and every byte of the launch is asked for in its first microsecond (the shape of the
 // expert kernel moe_gate_up_mfma, kernels_moe_mfma.hpp).  The arithmetic is the policies' of the one-row kernel:
-// activations as 15-bit fixed point a 32-element sub-block in a block-diagonal A operand, exact integer sums
+// activations as 15-bit fixed point a 32-element sub-block in a block-diagonal A operand (rows of six
+// super-blocks: 23-bit, QvQ4KFine), exact integer sums
 // (reference arithmetic: src/kquant_dot.rs:407-483 for Q4_K; the row-by-row schedule it replaces:
 // src/quant_matmul.rs:110-249).
 //

@@ -454,3 +454,13 @@ def test_one_token_whose_query_norm_rides_in_the_product():
         for n in (3, 1, 1, 6, 1):
             assert close(dev.forward(x[pos:pos + n], pos), ref.forward(x[pos:pos + n], pos)), (qtype, pos)
             pos += n
+
+
+def test_query_and_latent_down_projections_as_one_product():
+    """256 tokens over 4096 columns take q_a and kv_a as one product, 96 take two: both between single tokens, which take one."""
+    c = cfg(n_embd=4096, n_head=2, q_lora_rank=256, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=128, context_length=640)
+    ref, dev = build(c, seed=970)
+    x, pos = normal(31, (620, 4096)), 0
+    for n in (256, 1, 96, 1, 257, 9):
+        assert close(dev.forward(x[pos:pos + n], pos), ref.forward(x[pos:pos + n], pos)), pos
+        pos += n
