@@ -184,8 +184,9 @@ int dispatch_q4k_dot4(const uint8_t *W, size_t row_bytes, const float *X, float 
     // rows, with the decoder's norm form (4608 x 2048, q|k of a Qwen3-30B-A3B-shaped layer with residual add and RMSNorm:
     // one launch where there were rmsnorm_rows and the one-shot matrix-core GEMV).  JQ_Q4K_GEMV_TILE = 0 switches it off.
     static const char *tile_env = getenv("JQ_Q4K_GEMV_TILE");
-    // Six super-blocks (DeepSeek-V3's queries behind their down-projection) the same way: 24576 x 1536 6.0 us against 7.8 for the one-shot
-    // kernel, 4096 x 1536 4.0 against 5.4, and the norm rides along.
+    // Six super-blocks (DeepSeek-V3's queries behind their down-projection) the same way: 24576 x 1536 6.4 us against 7.8 for the one-shot
+    // kernel, 4096 x 1536 4.0 against 5.4, 64 x 1536 3.6 against 5.1, and the norm rides along (9.4 us cold for 2.4, a boundary and 9.5).
+    // Their activations keep the 23 bits of that kernel (QvQ4KFine).
     if (mode == "auto" && !swiglu && !(tile_env && tile_env[0] == '0') && (nb == 8 || nb == 6) && k == 256 * nb && row_bytes == nb * 144 &&
         n >= 64 && n <= 0x7FFFFFF0ull) {
         const jq::QdNorm nm = norm ? *norm : jq::QdNorm{};
