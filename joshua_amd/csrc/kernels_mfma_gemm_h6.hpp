@@ -8,13 +8,18 @@
 // where x' = x / s, s the power of two that takes the super-block's largest magnitude to 2^14 .. 2^15.  p is an integer of magnitude up
 // to 504, so exact in f16.  x' = h + l, h = f16(x'), and
 //
-//   x' p = h p + l p:   h p on v_mfma_f32_16x16x32_f16, exact products;   l p, 2^-12 of it, on v_mfma_f32_16x16x128_f8f6f4 with
-//                       both factors rounded to E2M3 (four significant bits), 1/4 of the cycles
+//   x' p = h p + l p:   h p on v_mfma_f32_16x16x32_f16, exact products;   l p, 2^-12 of it, on v_mfma_scale_f32_16x16x128_f8f6f4 with
+//                       both factors rounded to E2M3, 1/4 of the cycles.  p's codes stand on a scale of their own sub-block, the power of
+//                       two in sc / 32, so that they use E2M3's range whatever sc is (one scale for all, that of sc = 32..63, left
+//                       nothing of l p where sc is 1: 2.0e-4 off).  l's stand on the super-block's: at most 8, clamped at 7.5.
 //
 // into one f32 sum; the second term is one v_mfma_f32_16x16x32_bf16 a super-block with X and W in two bf16 parts each, added to
-// the result unscaled.  Against 64 bits the result is 0.9e-5 off (relative, normal activations against quantized normal
-// weights; 0.6e-5 against random blocks), the int8 GEMM's 16-bit fixed point (kernels_mfma_q4k_gemm_i8.hpp) 2.7e-5.  Taking q
-// about 8 is worth a factor of 2.5 of that: the codes' common part, which the min term would take away again, stays out of l p.
+// the result unscaled.  Off 64 bits (relative 2-norm, 160 x 1024 x 2048; in front of each the int8 GEMM's 16-bit fixed point,
+// kernels_mfma_q4k_gemm_i8.hpp): normal activations 2.7e-5 / 0.9e-5 against quantized normal weights, 2.7e-5 / 0.5e-5 against random
+// blocks, 2.7e-5 / 0.8e-5 .. 0.6e-5 against blocks with scales up to 63 .. 1 whose weights lie about zero; cubes of normal numbers
+// 7.1e-5 / 1.3e-5; one activation in 256 a hundred times the others 1.4e-4 / 2.0e-5.  Only rows that fixed point happens to hold
+// exactly, one non-zero activation a super-block (1e-7 / 0.8e-5) or all of them equal (1e-6 / 3.9e-5), are further off here.
+// Taking q about 8 is worth a factor of 2.5: the codes' common part, which the min term would take away again, stays out of l p.
 //
 // Why: the int8 GEMM needs 16 instructions of 16 cycles for 16 x 16 x 256 of the product and seven vector instructions for every
 // output and super-block to join its three integer sums; here it is 11 and two (the factor d s, the addition).
@@ -30,7 +35,7 @@
 // 4900 and the LDS moves operands for some 6500 (128 bytes a clock); the clock itself falls with the density of the work (2.1 GHz
 // at 10300 clocks a super-block, 1.8 at 8400), so power is the next bound.  Waves of 64 activation rows (four a workgroup, half
 // the LDS reads) take 131 us: one wave a SIMD has nothing to hide its vector instructions behind.
-// E2M1 codes of p, a third less to read, would be 2.6e-5 off 64 bits.
+// E2M1 codes of p, a third less to read, would be 2.6e-5 off 64 bits.  The codes' scales cost 1.3 us of a call (88.7 us, 89.9).
 #pragma once
 #include "kernels_dot4_q4k.hpp"
 
@@ -170,10 +175,11 @@ __global__ __launch_bounds__(128) void kq_gemm_h6_prep(const float *__restrict__
 
 // LDS: for either half of a super-block and every 16 weight rows 4 steps x 64 lanes x 16 bytes of f16 operands, then
 // their E2M3 codes (64 lanes x 16 bytes and x 8); behind the halves, twice (by the super-block's parity), for every 16 rows
-// the min operand's two parts (16 rows x 16 bytes each) and the 16 factors d.
-constexpr int H6_T_LO = 4096, H6_HALF = H6_T_LO + 1536, H6_META = 512 + 64;
+// the min operand's two parts (16 rows x 16 bytes each) and the 16 factors d; behind those, for either half, the exponents of
+// the codes' scales, 64 lanes x 8 groups of 16 rows: one read gives a lane those of all groups.
+constexpr int H6_T_LO = 4096, H6_HALF = H6_T_LO + 1536, H6_META = 512 + 64, H6_EXPS = 512;
 template <int NG>
-constexpr int h6_lds_bytes() { return 2 * NG * (H6_HALF + H6_META); }
+constexpr int h6_lds_bytes() { return 2 * NG * (H6_HALF + H6_META) + 2 * H6_EXPS; }
 
 // Memory behind an address that is the same in all lanes of a wave, read at a scalar and a lane's own offset: neither costs a
 // vector instruction or a register pair, as the lanes' 64-bit addresses would.
@@ -197,6 +203,7 @@ struct H6Q4K {  // w = d sc (q - 8) + (8 d sc - dmin m), 6-bit sc and m, q in 0.
     struct Raw {
         h6_u4 hdr, q0, q1;
         h6_h2 sc, off;  // 2^10 sc and -sc / 16
+        float unit;     // the codes' scale, a power of two: sc / 32 with its mantissa cleared
         h6_h32 p;
     };
     __device__ __forceinline__ static void fetch_header(const H6Memory &mem, uint32_t blk, uint32_t row_at, Raw &raw) {
@@ -206,14 +213,16 @@ struct H6Q4K {  // w = d sc (q - 8) + (8 d sc - dmin m), 6-bit sc and m, q in 0.
         raw.q0 = mem.load16(blk + 16 + 64 * h, row_at + 32 * (uint32_t)(g >> 1));
         raw.q1 = mem.load16(blk + 32 + 64 * h, row_at + 32 * (uint32_t)(g >> 1));
     }
-    // The sub-block's scale; its part of the row's min operand, and d.
-    __device__ __forceinline__ static void header(Raw &raw, int g, int i, int h, uint8_t *meta) {
+    // The sub-block's scale and its codes'; its part of the row's min operand, and d.
+    __device__ __forceinline__ static void header(Raw &raw, int g, int i, int h, uint8_t *meta, uint8_t *exponent) {
         const h6_u4 hdr = raw.hdr;
         const uint32_t s4 = h == 0 ? hdr.y & 0x3F3F3F3Fu : (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
         const uint32_t m4 = h == 0 ? hdr.z & 0x3F3F3F3Fu : ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
         const float sc = (float)((s4 >> (8 * g)) & 0xFFu), mn = (float)((m4 >> (8 * g)) & 0xFFu);
         const _Float16 sc16 = (_Float16)(1024.0f * sc), off16 = (_Float16)(-0.0625f * sc);
         raw.sc = h6_h2{sc16, sc16}, raw.off = h6_h2{off16, off16};
+        const uint32_t unit = __builtin_bit_cast(uint32_t, 0.03125f * fmaxf(sc, 1.0f)) & 0x7F800000u;
+        raw.unit = __builtin_bit_cast(float, unit), *exponent = (uint8_t)(unit >> 23);
         const float d = f16_bits(hdr.x), dmin = f16_bits(hdr.x >> 16);
         const float w = fmaf(256.0f * d, sc, -(32.0f * dmin) * mn);
         const uint32_t first = h6_bf16_bits(w);
@@ -237,7 +246,7 @@ struct H6Q4K {  // w = d sc (q - 8) + (8 d sc - dmin m), 6-bit sc and m, q in 0.
                                                              raw.p[8 * st + 4], raw.p[8 * st + 5], raw.p[8 * st + 6], raw.p[8 * st + 7]};
     }
     __device__ __forceinline__ static void codes(Raw &raw, int lane, uint8_t *tile) {
-        const h6_u6 six = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(raw.p, 1.0f);
+        const h6_u6 six = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(raw.p, raw.unit);
         *(h6_u4 *)(tile + H6_T_LO + lane * 16) = h6_u4{six[0], six[1], six[2], six[3]};
         *(h6_u2 *)(tile + H6_T_LO + 1024 + lane * 8) = h6_u2{six[4], six[5]};
     }
@@ -251,7 +260,7 @@ template <class F, int NW, int NG>
 __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict__ W, size_t row_bytes,
                                                       const uint8_t *__restrict__ acts, float *__restrict__ Y, int m_rows, int n,
                                                       int nb, int groups, int tx, int ty, int nb_total, size_t split_stride) {
-    static_assert(NG <= NW, "one group of 16 weight rows a wave unpacks");
+    static_assert(NG <= NW && NG <= 8, "one group of 16 weight rows a wave unpacks, a byte each of a lane's eight exponents");
     constexpr int NT = 16 * NG, MT = 32 * NW;
     extern __shared__ __attribute__((aligned(16))) uint8_t h6_lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
@@ -276,6 +285,7 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
     const H6Memory wsrc(W + (size_t)first_row * row_bytes + (size_t)b_first * F::BLOCK);
     const uint32_t wlane = (uint32_t)min(r, n - 1 - first_row) * (uint32_t)row_bytes;
     uint8_t *const own = h6_lds + wu * H6_HALF, *const meta_lds = h6_lds + 2 * NG * H6_HALF;
+    uint8_t *const exps = meta_lds + 2 * NG * H6_META + lane * 8;
     const uint32_t l16 = lane * 16;
 
     h6_h8 A[2][4];    // f16 operands of four steps, the fifth's in place of the first's
@@ -306,7 +316,7 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
         for (int st = 0; st < 4; st++) load_hi(mg, 0, st);
         load_lo(mg, 0, 0);
     }
-    F::header(raw, g, r, 0, meta_lds + wu * H6_META);
+    F::header(raw, g, r, 0, meta_lds + wu * H6_META, exps + wu);
     h6_each(std::make_integer_sequence<int, 16>{}, [&](auto uc) __attribute__((always_inline)) { F::template pair<decltype(uc)::value>(raw, g, lane, own); });
     F::codes(raw, lane, own);
     F::fetch(wsrc, 0, wlane, g, 1, raw);
@@ -340,6 +350,7 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
             // the half that is unpacked meanwhile: the second of this super-block, then the first of the next
             uint8_t *const next = own + (h ^ 1) * (NG * H6_HALF);
             uint8_t *const next_meta = meta_lds + ((b + h) & 1) * (NG * H6_META) + wu * H6_META;
+            const h6_u2 units = *(const h6_u2 *)(exps + h * H6_EXPS);
             const uint32_t src_next = (uint32_t)b1 * F::BLOCK;
             auto operand = [&](auto tc) __attribute__((always_inline)) {
                 constexpr Step st = step_of(h, decltype(tc)::value);
@@ -372,7 +383,7 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
                 }
                 if constexpr (h == 1 && st.kind == 2) d[st.cg & 1] = *(const float *)(meta + st.cg * H6_META + 512 + 4 * r);
                 // the next half's weights become operands among the matrix instructions; then the half after that is asked for
-                if constexpr (t == 1) F::header(raw, g, r, h ^ 1, next_meta);
+                if constexpr (t == 1) F::header(raw, g, r, h ^ 1, next_meta, exps + (h ^ 1) * H6_EXPS + wu);
                 if constexpr (t >= 2 && t < 18) F::template pair<t - 2>(raw, g, lane, next);
                 if constexpr (t == 18) F::codes(raw, lane, next);
                 if constexpr (t == 19) F::fetch(wsrc, src_next, wlane, g, h, raw), F::fetch_header(wsrc, src_next, wlane, raw);
@@ -383,7 +394,7 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
                         acc[mg][st.cg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(minA[mg], __builtin_bit_cast(h6_b8, w), acc[mg][st.cg], 0, 0, 0);
                     else if constexpr (st.kind == 4)
                         sb[mg][st.cg] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                            h6_operand6(L[mg]), h6_operand6(h6_u6{w[0], w[1], w[2], w[3], w2[0], w2[1]}), sb[mg][st.cg], 2, 2, 0, 0, 0, 0);
+                            h6_operand6(L[mg]), h6_operand6(h6_u6{w[0], w[1], w[2], w[3], w2[0], w2[1]}), sb[mg][st.cg], 2, 2, 0, 0x7F7F7F7F, st.cg & 3, (int)units[st.cg >> 2]);
                     else
                         sb[mg][st.cg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[mg][st.kind], __builtin_bit_cast(h6_h8, w),
                                                                                h == 0 && st.kind == 0 ? zero : sb[mg][st.cg], 0, 0, 0);

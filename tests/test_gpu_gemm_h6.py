@@ -7,7 +7,11 @@ import os
 import subprocess
 import sys
 
+import numpy as np
 import pytest
+
+import oracle
+from joshua_amd import capi
 
 pytestmark = pytest.mark.gpu
 
@@ -95,3 +99,41 @@ def test_gemm_on_f16_and_fp6_operands(shape, splits):
     env = dict(os.environ, JQ_GEMM_H6_SHAPE=shape, JQ_GEMM_H6_SPLITS=str(splits), JQ_GEMM_H6_MIN_M="17", JQ_Q4K_NO_ROWS16="1")
     res = subprocess.run([sys.executable, "-c", CHILD.replace("%r", repr(ROOT), 1)], env=env, capture_output=True, text=True, timeout=110)
     assert res.returncode == 0 and "h6 ok" in res.stdout, res.stdout + res.stderr
+
+
+def q4k_blocks(d, dmin, sc, mn, q):
+    """Blocks of [n][super-blocks]: d, dmin, sc and mn [..., 8] of six bits, q [..., 8, 32] of four."""
+    b = np.zeros(d.shape + (144,), np.uint8)
+    b[..., 0:2] = d.astype(np.float16)[..., None].view(np.uint8)
+    b[..., 2:4] = dmin.astype(np.float16)[..., None].view(np.uint8)
+    b[..., 4:8] = sc[..., :4] | sc[..., 4:] >> 4 << 6
+    b[..., 8:12] = mn[..., :4] | mn[..., 4:] >> 4 << 6
+    b[..., 12:16] = (sc[..., 4:] & 15) | (mn[..., 4:] & 15) << 4
+    b[..., 16:] = (q[..., 0::2, :] | q[..., 1::2, :] << 4).reshape(d.shape + (128,))
+    return b.reshape(-1)
+
+
+@pytest.mark.parametrize("scales", ["at most 1", "at most 2", "at most 4", "at most 8", "at most 63", "all 1", "all 31", "all 63", "one of 1"])
+def test_error_whatever_the_weights_scales(scales):
+    """Super-blocks whose six-bit scales are small, and activations that meet a small scale among large ones: the error against 64
+    bits does not depend on them.  The weights lie about zero (dmin m = 8 d sc), so that the codes' product is all of the result.
+
+    In root mean square the remainder l is at most 2^-10 / sqrt(12) of its activation (f16), and E2M3 takes at most 2^-3 / sqrt(12) of
+    each of its product's two factors: sqrt(2) / 12 2^-13 = 1.44e-5 of the result.  (Factors below E2M3's normal numbers lose
+    more of themselves, and are that much less of the sum.)"""
+    rng = np.random.default_rng(17)
+    m, k, n = 160, 2048, 1024
+    t = 63 if scales == "one of 1" else int(scales.split()[-1])
+    sc = np.full((n, k // 256, 8), t, np.uint8) if scales.startswith("all") else rng.integers(1, t + 1, (n, k // 256, 8), dtype=np.uint8)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    if scales == "one of 1":
+        sc[:, :, 3] = 1
+        x.reshape(m, -1, 8, 32)[:, :, [0, 1, 2, 4, 5, 6, 7]] *= np.float32(2e-5)
+    d = rng.uniform(1e-4, 1e-3, (n, k // 256)).astype(np.float16)
+    mn = np.round(sc * (63.0 / t)).astype(np.uint8)
+    q = rng.integers(0, 16, (n, k // 256, 8, 32), dtype=np.uint8)
+    blocks = q4k_blocks(d, d.astype(np.float64) * 8 * t / 63, sc, mn, q)
+    got = capi.Weight.upload(capi.Q4_K, blocks, n, k).matmul_t(m, x)
+    want = x.astype(np.float64) @ oracle.dequantize(capi.Q4_K, blocks).reshape(n, k).astype(np.float64).T
+    rel = np.sqrt(((got - want) ** 2).mean() / (want ** 2).mean())
+    assert rel <= 1.45e-5, float(rel)
