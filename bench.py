@@ -145,7 +145,7 @@ def matmul_workload(torch, capi, synth, qtype: int, n: int, k: int, m: int, seed
         tflops = 2.0 * m * n * k / ms / 1e9
         res["useful_tflops"] = round(tflops, 1)
         res["mfma_frac_of_f16_peak"] = round(tflops / F16_MFMA_PEAK_TFLOPS, 4)
-        if "gemm_i8" in kernel:
+        if capi.last_arithmetic() == "int8":
             # the many-row GEMM multiplies on the int8 matrix cores (two int8 planes of activations: two integer MACs a
             # useful one); against that unit's dense peak, counting useful operations only
             res["mfma_frac_of_int8_peak"] = round(tflops / INT8_MFMA_PEAK_TOPS, 4)

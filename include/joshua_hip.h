@@ -68,8 +68,14 @@ const char *jq_last_error(void);
 /* Name of the kernel that the calling thread's last jq_matmul_t / jq_matmul_t_noalloc /
  * jq_try_matmul_fused call chose ("" before the first one): which kernel serves a shape
  * depends on measured crossover points, and tests pin the choice with this
- * (no counterpart in the reference, which has one kernel per format). */
+ * (no counterpart in the reference, which has one kernel per format).  The matrix-core GEMM
+ * over many activation rows has one name a format, "q4k_gemm_i8" and its like with "+splitk"
+ * where k is split; jq_last_arithmetic tells its forms apart. */
 const char *jq_last_kernel(void);
+
+/* What that GEMM multiplied: "int8" (two 8-bit planes a factor), or "f16+fp6" (Q4_K from 128
+ * activation rows on: f16 products, their remainders in FP6); "" after any other kernel. */
+const char *jq_last_arithmetic(void);
 
 /* Elements and bytes per block of a type id; nonzero for an unknown id
  * (reference: src/gguf_ext.rs:483-512 type_size_bytes). */

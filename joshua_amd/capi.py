@@ -28,7 +28,7 @@ TYPE_NAMES = {Q8_0: "Q8_0", Q2_K: "Q2_K", Q4_K: "Q4_K", Q6_K: "Q6_K", IQ2_XXS: "
 
 # Every symbol include/joshua_hip.h declares.
 EXPORTS = (
-    "jq_last_error", "jq_last_kernel", "jq_block_geometry", "jq_init", "jq_upload", "jq_view", "jq_free", "jq_dtype", "jq_rows",
+    "jq_last_error", "jq_last_kernel", "jq_last_arithmetic", "jq_block_geometry", "jq_init", "jq_upload", "jq_view", "jq_free", "jq_dtype", "jq_rows",
     "jq_cols", "jq_storage_size_in_bytes", "jq_device_ptr", "jq_matmul_t", "jq_matmul_t_f16", "jq_matmul_t_noalloc", "jq_try_matmul_fused", "jq_dequantize", "jq_decode_raw_to_f32", "jq_stream_release",
     "jq_embedding", "jq_stream_synchronize", "jq_moe_create", "jq_moe_set_shared_gate", "jq_moe_free", "jq_moe_route", "jq_moe_forward",
     "jq_mla_create", "jq_mla_free", "jq_mla_forward", "jq_mla_reset", "jq_mla_cached_tokens",
@@ -113,6 +113,7 @@ def lib(path: str = LIB_PATH, beside_torch: bool = True) -> ctypes.CDLL:
         sz, u32, vp, i32 = ctypes.c_size_t, ctypes.c_uint32, ctypes.c_void_p, ctypes.c_int
         L.jq_last_error.restype = ctypes.c_char_p
         L.jq_last_kernel.restype = ctypes.c_char_p
+        L.jq_last_arithmetic.restype = ctypes.c_char_p
         L.jq_block_geometry.argtypes = [u32, ctypes.POINTER(sz), ctypes.POINTER(sz)]
         L.jq_init.argtypes = [i32]
         L.jq_upload.argtypes = [u32, vp, sz, sz, sz, i32, ctypes.POINTER(vp)]
@@ -208,6 +209,11 @@ def last_error() -> str:
 def last_kernel() -> str:
     """The kernel the calling thread's last matmul call chose."""
     return lib().jq_last_kernel().decode()
+
+
+def last_arithmetic() -> str:
+    """What the matrix-core GEMM over many rows multiplied, "int8" or "f16+fp6"; "" after any other kernel."""
+    return lib().jq_last_arithmetic().decode()
 
 
 def stream_release(stream: int = 0) -> None:

@@ -815,7 +815,7 @@ int dispatch_gemm_i8(const uint8_t *W, size_t row_bytes, const float *X, float *
     JQ_GEMM_I8(2, 4, true)
 #undef JQ_GEMM_I8
     if (attr_rc != hipSuccess) return fail("hipFuncSetAttribute: %s", hipGetErrorString(attr_rc));
-    note_kernel(splits > 1 ? name_split : name);
+    note_kernel(splits > 1 ? name_split : name, "int8");
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -830,8 +830,8 @@ hipError_t big_lds_once(int lds) {
 // Q4_K with 128 activation rows or more on f16 and FP6 operands (kq_gemm_h6): 512 x 14336 x 4096 99 us against the int8 GEMM's
 // 127, 2048 x 24576 x 4096 577 against 732, 512 x 4096 x 4096 50 against 52 (whole calls; 50
 // shapes of 128 to 2048 rows, 0.77 to 1.01 of the int8 GEMM's time).  Below 128 rows the int8 GEMM is as fast (64 to 127 rows:
-// 0.90 to 1.07) and keeps them: there unpacking the weights is most of the work in both.  `name` is the route's, the one that
-// callers of jq_last_kernel know the many-row product by, whichever arithmetic it runs on.
+// 0.90 to 1.07) and keeps them: there unpacking the weights is most of the work in both.  `name` is the one that
+// callers of jq_last_kernel know the many-row product by; jq_last_arithmetic says which of the two ran.
 // Returns -1 when the shape is outside its reach, where a fixed scratch holds the int8 GEMM's records but not these (12352 bytes
 // for 16 rows of 256 against 9280), and where the environment names a shape or a switch of that GEMM.  JQ_GEMM_H6 = 0
 // switches this one off, JQ_GEMM_H6_SHAPE and _SPLITS force the choice, _MIN_M moves the fewest rows.
@@ -915,7 +915,7 @@ int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *
     const int rc = best->nw == 4 ? JQ_GEMM_H6(4, 4) : best->ng == 7 ? JQ_GEMM_H6(8, 7) : JQ_GEMM_H6(8, 6);
 #undef JQ_GEMM_H6
     if (rc) return rc;
-    note_kernel(splits > 1 ? name_split : name);
+    note_kernel(splits > 1 ? name_split : name, "f16+fp6");
     HIP_TRY(hipGetLastError());
     return 0;
 }

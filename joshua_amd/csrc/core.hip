@@ -8,8 +8,8 @@ namespace jqh {
 
 thread_local char g_err[512] = "";
 // Name of the kernel the calling thread's last matmul dispatch chose (jq_last_kernel).
-thread_local const char *g_last_kernel = "";
-void note_kernel(const char *name) { g_last_kernel = name; }
+thread_local const char *g_last_kernel = "", *g_last_arithmetic = "";
+void note_kernel(const char *name, const char *arithmetic) { g_last_kernel = name, g_last_arithmetic = arithmetic; }
 
 int fail(const char *fmt, ...) {
     va_list ap;
@@ -190,6 +190,7 @@ extern "C" {
 
 const char *jq_last_error(void) { return g_err; }
 const char *jq_last_kernel(void) { return g_last_kernel; }
+const char *jq_last_arithmetic(void) { return g_last_arithmetic; }
 
 int jq_block_geometry(uint32_t ggml_type, size_t *elems, size_t *bytes) {
     Geometry g;

@@ -30,7 +30,7 @@ struct jq_weight {
 namespace jqh {
 
 int fail(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
-void note_kernel(const char *name);  // what jq_last_kernel reports
+void note_kernel(const char *name, const char *arithmetic = "");  // what jq_last_kernel and jq_last_arithmetic report
 
 #define HIP_TRY(expr)                                                                      \
     do {                                                                                   \

@@ -41,7 +41,7 @@ def check(blocks, lhs, what, rms=None):
     m, k = lhs.shape
     n = blocks.size // (k // 256 * 144)
     got = capi.Weight.upload(capi.Q4_K, blocks, n, k).matmul_t(m, lhs)
-    assert capi.last_kernel() == name, capi.last_kernel()
+    assert (capi.last_kernel(), capi.last_arithmetic()) == (name, "f16+fp6"), (capi.last_kernel(), capi.last_arithmetic())
     w = oracle.dequantize(capi.Q4_K, blocks).reshape(n, k).astype(np.float64)
     x = lhs.astype(np.float64)
     want = x @ w.T
@@ -137,3 +137,16 @@ def test_error_whatever_the_weights_scales(scales):
     want = x.astype(np.float64) @ oracle.dequantize(capi.Q4_K, blocks).reshape(n, k).astype(np.float64).T
     rel = np.sqrt(((got - want) ** 2).mean() / (want ** 2).mean())
     assert rel <= 1.45e-5, float(rel)
+
+
+@pytest.mark.parametrize("qtype,m,k,n,kernel,arithmetic", [
+    (capi.Q4_K, 127, 4096, 14336, "q4k_gemm_i8", "int8"), (capi.Q4_K, 128, 4096, 14336, "q4k_gemm_i8", "f16+fp6"),
+    (capi.Q4_K, 512, 4096, 14336, "q4k_gemm_i8", "f16+fp6"), (capi.Q4_K, 128, 4096, 256, "q4k_gemm_mfma", ""),
+    (capi.Q6_K, 512, 4096, 1024, "q6k_gemm_i8", "int8"), (capi.Q4_K, 1, 4096, 4096, "q4k_gemv_mfma_lds", "")])
+def test_arithmetic_chosen_for_a_shape(qtype, m, k, n, kernel, arithmetic):
+    import torch
+    w = capi.Weight.upload(qtype, np.zeros(n * k // 256 * (144 if qtype == capi.Q4_K else 210), np.uint8), n, k)
+    x, y = torch.zeros(m * k, device="cuda"), torch.empty(m * n, device="cuda")
+    w.matmul_t_dev(m, x.data_ptr(), m * k, y.data_ptr(), m * n, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert (capi.last_kernel().split("+")[0], capi.last_arithmetic()) == (kernel, arithmetic)
