@@ -150,9 +150,9 @@ int jq_matmul_t_f16(const jq_weight *w, size_t m, const uint16_t *lhs, size_t lh
  * product split over k) lives in one fixed array of JQ_NOALLOC_SCRATCH_BYTES in each
  * device's memory, held from library load until the process ends.  The call makes no
  * hipMalloc / hipFree and fails, dst untouched, when the product needs more scratch than
- * the array holds (one activation row never needs any; Q4_K needs about 9 KB per 16
- * activation rows and 256 columns up to 256 rows and 4 m k bytes beyond; the other
- * formats 4 m k bytes from 8 rows on; a product split over k adds 4 m n bytes a split).
+ * the array holds (one activation row never needs any; the matrix-core GEMM needs 9280 bytes
+ * per 16 activation rows and 256 columns, whichever arithmetic it runs on, other kernels up to
+ * 4 m k bytes; a product split over k adds 4 m n bytes a split).
  * Every call on a device shares that device's array: calls whose kernels overlap on
  * one device (two streams, two threads) race; calls on one stream are safe.
  * Where jq_matmul_t would split a product over k into more partial results than the

@@ -832,8 +832,7 @@ hipError_t big_lds_once(int lds) {
 // shapes of 128 to 2048 rows, 0.77 to 1.01 of the int8 GEMM's time).  Below 128 rows the int8 GEMM is as fast (64 to 127 rows:
 // 0.90 to 1.07) and keeps them: there unpacking the weights is most of the work in both.  `name` is the one that
 // callers of jq_last_kernel know the many-row product by; jq_last_arithmetic says which of the two ran.
-// Returns -1 when the shape is outside its reach, where a fixed scratch holds the int8 GEMM's records but not these (12352 bytes
-// for 16 rows of 256 against 9280), and where the environment names a shape or a switch of that GEMM.  JQ_GEMM_H6 = 0
+// Returns -1 when the shape is outside its reach and where the environment names a shape or a switch of that GEMM.  JQ_GEMM_H6 = 0
 // switches this one off, JQ_GEMM_H6_SHAPE and _SPLITS force the choice, _MIN_M moves the fewest rows.
 template <class F>
 int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n,
@@ -850,13 +849,25 @@ int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *
     };
     static const Shape shapes[] = {{8, 7}, {8, 6}, {4, 4}};
     const size_t nb = k / 256, groups = (m + 15) / 16;
-    const size_t acts_bytes = (groups * nb * (size_t)jq::H6_REC + 255) & ~(size_t)255;
     const size_t scratch_cap = tl_fixed_scratch ? tl_fixed_scratch->bytes : (size_t)1 << 40;
-    if (acts_bytes > scratch_cap) return -1;
-    auto rows_of = [&](const Shape &sh) { return (m + 32 * (size_t)sh.nw - 1) / (32 * (size_t)sh.nw); };
-    auto tiles_of = [&](const Shape &sh) { return rows_of(sh) * ((n + 16 * (size_t)sh.ng - 1) / (16 * (size_t)sh.ng)); };
-    auto grid_of = [&](const Shape &sh) { return 8 % rows_of(sh) == 0 ? (tiles_of(sh) + 7) / 8 * 8 : tiles_of(sh); };
-    if (!min_m_env && tiles_of(shapes[2]) * std::max<size_t>(1, std::min<size_t>(nb / 4, 8)) < 64) return -1;
+    // A fixed scratch that holds the int8 GEMM's records of all rows, three quarters of these in size, takes the rows in two turns;
+    // what neither GEMM's records fit fails there as it did.  (1024 x 12288: 36 MB in 32.)
+    size_t turn = m;
+    auto acts_of = [&](size_t rows) { return ((rows + 15) / 16 * nb * (size_t)jq::H6_REC + 255) & ~(size_t)255; };
+    if (acts_of(m) > scratch_cap) {
+        if (groups * nb * (size_t)jq::QI_REC > scratch_cap) return -1;
+        turn = (groups + 1) / 2 * 16;
+        if (acts_of(turn) > scratch_cap) return -1;
+    }
+    const size_t acts_bytes = acts_of(turn);
+    // tiles of a turn's rows, of the weight rows, workgroups of its launch
+    auto rows_of = [&](const Shape &sh, size_t rows) { return (rows + 32 * (size_t)sh.nw - 1) / (32 * (size_t)sh.nw); };
+    auto cols_of = [&](const Shape &sh) { return (n + 16 * (size_t)sh.ng - 1) / (16 * (size_t)sh.ng); };
+    auto grid_of = [&](const Shape &sh, size_t rows) {
+        const size_t ty = rows_of(sh, rows), tiles = ty * cols_of(sh);
+        return 8 % ty == 0 ? (tiles + 7) / 8 * 8 : tiles;
+    };
+    if (!min_m_env && rows_of(shapes[2], m) * cols_of(shapes[2]) * std::max<size_t>(1, std::min<size_t>(nb / 4, 8)) < 64) return -1;
     auto rounds = [](double wgs, double at_once, auto us) {
         const double whole = std::floor(wgs / at_once), rest = wgs - whole * at_once;
         return whole * us(at_once) + (rest > 0.0 ? us(rest) : 0.0);
@@ -866,7 +877,7 @@ int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *
     // starts of further rounds, the sum of the parts.  Over 70 shapes the picks are 0.6 % off the best measured choice on
     // average, 4 % at the 95th percentile, 10 % at worst.
     auto estimate = [&](const Shape &sh, size_t sp) {
-        const double wgs = (double)(grid_of(sh) * sp), nbl = (double)(nb / sp);
+        const double wgs = (double)(grid_of(sh, m) * sp), nbl = (double)(nb / sp);
         double us = 3.2 + 0.0048 * (double)(nb * groups);
         if (sh.nw == 8)
             us += 6.4 + nbl * rounds(wgs, 256.0, [](double w) { return 3.4 + 0.0035 * w; }) * (sh.ng == 7 ? 1.0 : 0.92) +
@@ -887,28 +898,32 @@ int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *
         for (size_t sp = 1; sp <= 8; sp++) {
             if (nb % sp != 0 || (sp > 1 && nb / sp < 4)) continue;
             if (splits_env && sp != (size_t)atoi(splits_env)) continue;
-            if (sp > 1 && (m * n > 0x3FFFFFFFull || acts_bytes + sp * m * n * sizeof(float) > scratch_cap)) continue;
+            if (sp > 1 && (m * n > 0x3FFFFFFFull || acts_bytes + sp * turn * n * sizeof(float) > scratch_cap)) continue;
             const double us = estimate(sh, sp);
             if (!best || us < best_us) best = &sh, splits = sp, best_us = us;
         }
     }
     if (!best) return -1;
-    const size_t tx = (n + 16 * (size_t)best->ng - 1) / (16 * (size_t)best->ng), ty = rows_of(*best), grid = grid_of(*best);
-    if (grid > 0x7FFFFFFFull) return -1;
+    if (grid_of(*best, m) > 0x7FFFFFFFull) return -1;
     CallScratch scratch;
     uint8_t *acts = nullptr;
-    if (scratch.get(acts_bytes + (splits > 1 ? splits * m * n * sizeof(float) : 0), s, &acts)) return 1;
+    if (scratch.get(acts_bytes + (splits > 1 ? splits * turn * n * sizeof(float) : 0), s, &acts)) return 1;
     float *parts = (float *)(acts + acts_bytes);
     auto launch = [&](auto kern, int lds, int nw, hipError_t rc) {
         if (rc != hipSuccess) return fail("hipFuncSetAttribute: %s", hipGetErrorString(rc));
-        const dim3 prep((unsigned)nb, (unsigned)groups);
-        if (swiglu_pairs) hipLaunchKernelGGL(jq::kq_gemm_h6_prep<true>, prep, dim3(128), 0, s, X, (int)m, (int)k, acts);
-        else hipLaunchKernelGGL(jq::kq_gemm_h6_prep<false>, prep, dim3(128), 0, s, X, (int)m, (int)k, acts);
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid, (unsigned)splits), dim3(64 * nw), lds, s, W, row_bytes, (const uint8_t *)acts,
-                           splits > 1 ? parts : Y, (int)m, (int)n, (int)(nb / splits), (int)groups, (int)tx, (int)ty, (int)nb,
-                           splits > 1 ? m * n : (size_t)0);
-        if (splits > 1)
-            hipLaunchKernelGGL(jq::splitk_sum, dim3((unsigned)((m * n + 1023) / 1024)), dim3(256), 0, s, parts, Y, m * n, (int)splits);
+        for (size_t m0 = 0; m0 < m; m0 += turn) {
+            const size_t rows = std::min(turn, m - m0), row_groups = (rows + 15) / 16, outs = rows * n;
+            const float *x = X + m0 * k * (swiglu_pairs ? 2 : 1);
+            float *y = Y + m0 * n;
+            const dim3 prep((unsigned)nb, (unsigned)row_groups);
+            if (swiglu_pairs) hipLaunchKernelGGL(jq::kq_gemm_h6_prep<true>, prep, dim3(128), 0, s, x, (int)rows, (int)k, acts);
+            else hipLaunchKernelGGL(jq::kq_gemm_h6_prep<false>, prep, dim3(128), 0, s, x, (int)rows, (int)k, acts);
+            hipLaunchKernelGGL(kern, dim3((unsigned)grid_of(*best, rows), (unsigned)splits), dim3(64 * nw), lds, s, W, row_bytes,
+                               (const uint8_t *)acts, splits > 1 ? parts : y, (int)rows, (int)n, (int)(nb / splits), (int)row_groups,
+                               (int)cols_of(*best), (int)rows_of(*best, rows), (int)nb, splits > 1 ? outs : (size_t)0);
+            if (splits > 1)
+                hipLaunchKernelGGL(jq::splitk_sum, dim3((unsigned)((outs + 1023) / 1024)), dim3(256), 0, s, parts, y, outs, (int)splits);
+        }
         return 0;
     };
 #define JQ_GEMM_H6(NW_, NG_) launch(jq::kq_gemm_h6<F, NW_, NG_>, jq::h6_lds_bytes<NG_>(), NW_, big_lds_once<&jq::kq_gemm_h6<F, NW_, NG_>>(jq::h6_lds_bytes<NG_>()))

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 import oracle
-from joshua_amd import capi
+from joshua_amd import capi, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -150,3 +150,34 @@ def test_arithmetic_chosen_for_a_shape(qtype, m, k, n, kernel, arithmetic):
     w.matmul_t_dev(m, x.data_ptr(), m * k, y.data_ptr(), m * n, torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     assert (capi.last_kernel().split("+")[0], capi.last_arithmetic()) == (kernel, arithmetic)
+
+
+def device_product(call, m, k, n, x, stream):
+    import torch
+    y = torch.full((m, n), float("nan"), device="cuda")
+    call(m, x.data_ptr(), m * k, y.data_ptr(), m * n, stream)
+    return y
+
+
+@pytest.mark.parametrize("m,k,n,whole", [(128, 4096, 1024, True), (300, 2048, 2000, True), (900, 4096, 4096, True), (3072, 4096, 4096, True),
+                                         (1024, 12288, 4096, False), (1077, 12288, 640, False), (130, 98304, 256, False)])
+def test_the_call_that_allocates_nothing_takes_the_same_arithmetic(m, k, n, whole):
+    """Also where the prepared activations of all rows do not fit its scratch (from m k = 11.1M elements on; above 14.8M it fails).
+    `whole`: both calls split k alike, so that not even the order of a sum differs."""
+    import torch
+    blocks = synth.normal_quantized(capi.Q4_K, 61, n * k, 0.02)
+    w = capi.Weight.upload(capi.Q4_K, blocks, n, k)
+    x = torch.from_numpy(synth.normal(62, (m, k))).cuda()
+    s = torch.cuda.current_stream().cuda_stream
+    ref = device_product(w.matmul_t_dev, m, k, n, x, s)
+    names = [(capi.last_kernel(), capi.last_arithmetic())]
+    new = device_product(w.matmul_t_noalloc, m, k, n, x, s)
+    names.append((capi.last_kernel(), capi.last_arithmetic()))
+    torch.cuda.synchronize()
+    assert [a for _, a in names] == ["f16+fp6"] * 2, names
+    if whole:
+        assert torch.equal(ref, new), names
+    wd = torch.from_numpy(oracle.dequantize(capi.Q4_K, blocks).reshape(n, k)).cuda().double()
+    want = x.double() @ wd.T
+    for got in (ref, new):
+        assert ((got - want).square().mean() / want.square().mean()).sqrt().item() <= 1.45e-5
