@@ -157,11 +157,12 @@ int CallScratch::get(size_t bytes, hipStream_t s, uint8_t **out) {
         *out = f->ptr;
         return 0;
     }
-    if (bytes > SCRATCH_KEEP) {
+    auto stream_ordered = [&]() -> int {
         HIP_TRY(hipMallocAsync((void **)&transient_, bytes, s));
         *out = transient_;
         return 0;
-    }
+    };
+    if (bytes > SCRATCH_KEEP) return stream_ordered();
     int dev = 0;
     HIP_TRY(hipGetDevice(&dev));
     StreamBuffer *b;
@@ -173,6 +174,14 @@ int CallScratch::get(size_t bytes, hipStream_t s, uint8_t **out) {
     }
     lock_ = std::unique_lock<std::mutex>(b->mu);
     if (b->bytes < bytes) {
+        if (bytes > SCRATCH_CAPTURABLE) {
+            hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
+            if (capture != hipStreamCaptureStatusNone) {
+                lock_.unlock();
+                return stream_ordered();
+            }
+        }
         const size_t want = std::min(SCRATCH_KEEP, std::max<size_t>({(bytes + 0xFFFFF) & ~(size_t)0xFFFFF, 2 * b->bytes,
                                                                       (size_t)1 << 20}));
         uint8_t *fresh = nullptr;

@@ -78,13 +78,14 @@ struct FixedScratchScope {
 // host threads that share a stream enqueue their calls one after the other.  Larger requests are
 // stream-ordered allocations, freed behind the call's launches.  First use and growth allocate: neither
 // is possible while the stream is being captured, so a caller warms a stream up with its largest call
-// before capturing it.
+// before capturing it.  Requests above SCRATCH_CAPTURABLE need no such call: where the buffer does not hold one yet
+// and the stream is being captured, it is a stream-ordered allocation of the graph, like those above SCRATCH_KEEP.
 //
 // jq_matmul_t_noalloc serves the same requests from a fixed array in device memory instead (below): it
 // installs the array for the calling thread with FixedScratchScope, and get() then hands out that
 // array, or fails when the request exceeds it, and never reaches an allocator.
 // (2048 activation rows of 12288 are 76 MB of prepared records, kq_gemm_h6)
-constexpr size_t SCRATCH_KEEP = 128u << 20;
+constexpr size_t SCRATCH_KEEP = 128u << 20, SCRATCH_CAPTURABLE = 64u << 20;
 class CallScratch {
     std::unique_lock<std::mutex> lock_;
     hipStream_t stream_ = nullptr;

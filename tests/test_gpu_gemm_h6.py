@@ -181,3 +181,28 @@ def test_the_call_that_allocates_nothing_takes_the_same_arithmetic(m, k, n, whol
     want = x.double() @ wd.T
     for got in (ref, new):
         assert ((got - want).square().mean() / want.square().mean()).sqrt().item() <= 1.45e-5
+
+
+def test_capture_on_a_stream_that_never_ran_a_product_of_that_size():
+    """Scratch between 64 and 128 MB (114 here): a cold stream can be captured, as it can above."""
+    import torch
+    m, k, n = 3072, 12288, 256
+    w = capi.Weight.upload(capi.Q4_K, synth.normal_quantized(capi.Q4_K, 63, n * k, 0.02), n, k)
+    x = torch.from_numpy(synth.normal(64, (m, k))).cuda()
+    want = device_product(w.matmul_t_dev, m, k, n, x, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    stream, y = torch.cuda.Stream(), torch.full((m, n), float("nan"), device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        w.matmul_t_dev(m, x.data_ptr(), m * k, y.data_ptr(), m * n, stream.cuda_stream)
+    for _ in range(3):
+        y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+        device_product(w.matmul_t_dev, m, k, n, x, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+    del graph
+    torch.cuda.synchronize()
+    capi.stream_release(stream.cuda_stream)
