@@ -2596,7 +2596,7 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
                  lkv = c.kv_lora_rank, qd = nope + rope;
     const float *comp = m->comp;
     int comp_stride = (int)(lkv + rope);
-    if (m->split16 && split16_latent_overwrites(m->split16, pos, s)) return 1;
+    if (m->split16) split16_latent_overwrites(m->split16, pos, s);
     // one token over a Q4_K up-projection of DeepSeek's geometry: its blocks are read (9 MB at V3's size) instead of the
     // 67 MB of their f32 copy.  128 heads behind 100 tokens, us: absorbing 7.1 / 5.4, merging the splits and multiplying with the value
     // rows 4.8 + 8.0 / 6.1 in one launch.

@@ -19,6 +19,14 @@ bool have(void **p, size_t bytes, bool *refused) {
     return false;
 }
 
+// Whether the stream is being captured; also where it does not say (the null stream beside another's capture).
+bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) == hipSuccess) return capture != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 }  // namespace
 
 struct Split16Latent {
@@ -62,13 +70,10 @@ static bool latent_keeps(const Split16Latent *s) { return !s->captured && latent
 // The first tile that a call has to expand.
 static size_t latent_first_tile(const Split16Latent *s) { return latent_keeps(s) ? s->ready / jq::S16_TILE : 0; }
 
-int split16_latent_overwrites(Split16Latent *s, size_t pos, hipStream_t stream) {
+void split16_latent_overwrites(Split16Latent *s, size_t pos, hipStream_t stream) {
     s->ready = std::min(s->ready, pos);
-    if (s->captured) return 0;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    HIP_TRY(hipStreamIsCapturing(stream, &capture));
-    s->captured = capture != hipStreamCaptureStatusNone;
-    return 0;
+    if (s->captured) return;
+    s->captured = capturing(stream);
 }
 
 // Both sides in us, fitted to calls of 48 to 1024 tokens behind 0 to 32000 with 128 and 32 heads (within 10 %, the absorbed
@@ -117,11 +122,7 @@ int split16_latent_attention(Split16Latent *s, const float *q, size_t S, size_t 
     if (s->refused) return -1;
     if (!s->ws) {
         // nothing can be allocated while the stream is captured: this call is absorbed, and a later one asks
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
-            (void)hipGetLastError();
-            return -1;
-        }
+        if (capturing(stream)) return -1;
         size_t want = latent_ws_bytes(s);
         bool none = false;
         const bool rest = (s->cf || have((void **)&s->cf, all * (jq::S16_LKV / 16) * 2 * jq::S16_FRAG, &s->refused)) &&

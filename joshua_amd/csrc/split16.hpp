@@ -14,7 +14,7 @@ int split16_latent_create(size_t n_head, size_t n_ctx, const float *wkv, const f
 void split16_latent_free(Split16Latent *s);
 // The cached tokens from `pos` on are about to be written by work on that stream: their keys and values, if they were
 // expanded, are not those of the cache any more.
-int split16_latent_overwrites(Split16Latent *s, size_t pos, hipStream_t stream);
+void split16_latent_overwrites(Split16Latent *s, size_t pos, hipStream_t stream);
 // Whether a call of S tokens behind `pos` is cheaper with expanded keys and values than absorbed; `fresh`: where none of those
 // in front are expanded already.
 bool split16_latent_pays(const Split16Latent *s, size_t S, size_t pos, bool fresh);
