@@ -842,7 +842,7 @@ int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *
     static const char *min_m_env = getenv("JQ_GEMM_H6_MIN_M");
     static const size_t min_m = min_m_env ? std::max<size_t>((size_t)atoll(min_m_env), 2) : 128;
     if ((mode && mode[0] == '0') || i8_mode || i8_shape || m < min_m || k % 256 != 0 || k == 0 || row_bytes % 16 != 0 ||
-        row_bytes > ((size_t)1 << 27) || ((uintptr_t)W & 15) != 0 || ((uintptr_t)X & 15) != 0 || m > 0x7FFFFFF0ull || n > 0x7FFFFFF0ull)
+        !jq::h6_offsets_hold(k / 256, row_bytes) || ((uintptr_t)W & 15) != 0 || ((uintptr_t)X & 15) != 0 || m > 0x7FFFFFF0ull || n > 0x7FFFFFF0ull)
         return -1;
     struct Shape {
         int nw, ng;

@@ -65,6 +65,10 @@ typedef float h6_f4 __attribute__((ext_vector_type(4)));
 //   the 16 scales
 constexpr int H6_HI = 8192, H6_LO_HALF = 1536, H6_MIN = H6_HI + 2 * H6_LO_HALF, H6_SCALE = H6_MIN + 1024, H6_REC = H6_SCALE + 64;
 
+// Whether the kernel's offsets hold rows of that many super-blocks: a record's from the start of its row group in 31 bits, a weight
+// block's from the first of 16 rows in 32.
+constexpr bool h6_offsets_hold(size_t nb, size_t row_bytes) { return nb <= 0x7FFFFFFFu / H6_REC && row_bytes <= (size_t)1 << 27; }
+
 __device__ __forceinline__ uint32_t h6_bf16_bits(float x) {
     return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)x);
 }

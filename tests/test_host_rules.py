@@ -53,3 +53,24 @@ int main() {
     puts("ok");
 }
 """)
+
+
+def test_offsets_of_the_f16_fp6_gemm_stay_in_their_registers(tmp_path):
+    """Every byte that the kernel reads of a record's row group lies below 2^31 from its start, of 16 weight rows below 2^32, for the
+    longest rows that the rule lets through, also where a paired matrix's rows lie two rows apart."""
+    assert "ok" in run(tmp_path, r"""
+#include <hip/hip_runtime.h>
+#include "core.hpp"
+#include "kernels_mfma_gemm_h6.hpp"
+int main() {
+    size_t longest = 0;
+    for (size_t nb = 1; nb < (size_t)1 << 21; nb++)
+        for (size_t apart : {144 * nb, 288 * nb})
+            if (jq::h6_offsets_hold(nb, apart)) {
+                longest = nb > longest ? nb : longest;
+                if (nb * jq::H6_REC > 0x7FFFFFFFull || 15 * apart + 144 * nb > 0xFFFFFFFFull) return 1;
+            }
+    if (longest < 100000) return 2;
+    puts("ok");
+}
+""")
