@@ -508,3 +508,51 @@ def test_output_projection_that_merges_the_attention_of_a_step(n_head, n_kv, d):
             assert ok, f"pos {pos}: {e}"
             pos += n
     assert pos > 512
+
+
+MERGE_CHILD = r"""
+import sys, numpy as np
+sys.path.insert(0, sys.argv[1])
+from tests.test_gpu_qwen3 import CFG, make
+out = []
+for n_head, n_kv, d in ((64, 8, 64), (32, 4, 128)):
+    m, _ = make(dict(CFG, n_layer=1, hidden=2048, n_head=n_head, n_kv_head=n_kv, head_dim=d, ffn=256, vocab=512, n_ctx=520), 96, "q4_k")
+    toks, pos = np.random.default_rng(18).integers(0, 512, 520).tolist(), 0
+    for prompt in (3, 60, 70, 130, 200):
+        m.forward(toks[pos:pos + prompt], pos)
+        pos += prompt
+        for _ in range(3):
+            out.append(m.forward(toks[pos:pos + 1], pos))
+            pos += 1
+np.save(sys.argv[2], np.stack(out))
+"""
+
+
+def test_merging_in_the_output_projection_leaves_the_bits_of_the_merging_launch(tmp_path):
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    got = []
+    for name, env in (("merged", {}), ("apart", {"JQ_NO_MERGE_IN_GEMV": "1"})):
+        path = str(tmp_path / (name + ".npy"))
+        res = subprocess.run([sys.executable, "-c", MERGE_CHILD, root, path], env=dict(os.environ, **env), capture_output=True, text=True,
+                             timeout=110)
+        assert res.returncode == 0, res.stdout + res.stderr
+        got.append(np.load(path))
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("mix", ["q4_k_m", "q4_k"])
+def test_single_token_steps_with_1536_wide_rows(mix):
+    """hidden = 1536: residual add, RMSNorm and product of a single token as one launch of six waves a tile, the stored residual row and
+    (q4_k_m: an attn_v of another format) the stored normalised row among its results."""
+    cfg = dict(CFG, n_layer=4, hidden=1536, n_head=4, n_kv_head=2, head_dim=128, ffn=768, vocab=512, n_ctx=40)
+    m, o = make(cfg, 37, mix)
+    if mix == "q4_k_m":
+        assert any(qt != capi.Q4_K for n, qt, _ in qwen3_tensors(cfg, 37, mix) if n.endswith("attn_v.weight"))
+    toks, pos = np.random.default_rng(19).integers(0, 512, 24).tolist(), 0
+    for n in (5, 1, 1, 1, 9, 1, 1):
+        ok, e = close(m.forward(toks[pos:pos + n], pos), o.forward(toks[pos:pos + n], pos))
+        assert ok, f"pos {pos}: {e}"
+        pos += n
