@@ -123,7 +123,9 @@ const void *jq_device_ptr(const jq_weight *w);
  * on, and from 8 against 8M weights or more) uses one scale per 256 elements, which
  * resolves each super-block to 2^-16 of its largest magnitude (2^-12 of the sum of the
  * terms' magnitudes on such rows; the reference's integer path quantises activations to 8
- * bits per 256, src/quant_matmul.rs:184).  In that GEMM the formats with a scale per 32
+ * bits per 256, src/quant_matmul.rs:184), and from 128 rows on Q4_K's holds them as f16 with a
+ * remainder of four significant bits, relative to each element down to 2^-19 of the
+ * super-block's largest.  In that GEMM the formats with a scale per 32
  * elements (Q8_0, MXFP4, Q4_0, Q4_1, Q5_0, Q5_1) have the eight blocks of a 256-run put on
  * the run's largest scale at 15 or 16 bits: exact where the scales are equal or a few powers
  * of two apart, else each weight to 2^-15 of the run's largest magnitude or better.  A row

@@ -827,10 +827,11 @@ hipError_t big_lds_once(int lds) {
     return rc;
 }
 
-// Q4_K with 128 activation rows or more on f16 and FP6 operands (kq_gemm_h6): 512 x 14336 x 4096 99 us against the int8 GEMM's
-// 127, 2048 x 24576 x 4096 577 against 732, 512 x 4096 x 4096 50 against 52 (whole calls; 50
-// shapes of 128 to 2048 rows, 0.77 to 1.01 of the int8 GEMM's time).  Below 128 rows the int8 GEMM is as fast (64 to 127 rows:
-// 0.90 to 1.07) and keeps them: there unpacking the weights is most of the work in both.  `name` is the one that
+// Q4_K with 128 activation rows or more on f16 and FP6 operands (kq_gemm_h6), us against the int8 GEMM's, whole calls back to back:
+// 512 x 14336 x 4096 95 / 116, 2048 x 24576 x 4096 604 / 738, 512 x 4096 x 4096 48 / 50.  166 shapes of 128 to 2048 rows against
+// 1000 to 24576 weight rows of 1024 to 16384: 0.77 to 1.08 of its time, 0.91 on average; the 18 that are more than 2 % slower, by
+// 0.5 to 2 us, are those against some 1000 weight rows and 333 to 512 rows against 4096.  Below 128 rows the int8 GEMM is as fast
+// (64 to 127 rows: 0.90 to 1.07) and keeps them: there unpacking the weights is most of the work in both.  `name` is the one that
 // callers of jq_last_kernel know the many-row product by; jq_last_arithmetic says which of the two ran.
 // Returns -1 when the shape is outside its reach and where the environment names a shape or a switch of that GEMM.  JQ_GEMM_H6 = 0
 // switches this one off, JQ_GEMM_H6_SHAPE and _SPLITS force the choice, _MIN_M moves the fewest rows.
@@ -874,8 +875,8 @@ int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *
     };
     // In us, the int8 GEMM's form of estimate (dispatch_gemm_i8) fitted to 714 times of this one's three shapes in 1 to 8 parts: the
     // preparation, a fixed start, the super-blocks a workgroup walks at a cost that grows with the workgroups at work, the
-    // starts of further rounds, the sum of the parts.  Over 70 shapes the picks are 0.6 % off the best measured choice on
-    // average, 4 % at the 95th percentile, 10 % at worst.
+    // starts of further rounds, the sum of the parts.  Over 166 shapes the picks are 0.7 % off the best measured choice on
+    // average, 5 % at the 95th percentile, 12 % at worst.
     auto estimate = [&](const Shape &sh, size_t sp) {
         const double wgs = (double)(grid_of(sh, m) * sp), nbl = (double)(nb / sp);
         double us = 3.2 + 0.0048 * (double)(nb * groups);

@@ -31,7 +31,7 @@ __device__ __forceinline__ void gemv_mfma_tile_body(uint8_t *gemv_tile_lds, int 
                                                     const float *__restrict__ X, float *__restrict__ Y, int n,
                                                     const float *nm_res, const float *nm_w, float nm_eps, float *nm_x_out,
                                                     float *nm_hn_out) {
-    static_assert(NB >= 2 && NB <= 16, "a row of 2 to 16 super-blocks");
+    static_assert(NB >= 2 && NB <= 16, "a row of 2 to 16 super-blocks");  // (6, 8 and 16 are dispatched; the others are not measured)
     constexpr int RB = NB * F::BLOCK, ROW_LDS = moe_mfma_row_lds(RB), LOADS = (RB + 1023) / 1024;
     constexpr int STG = gemv_mfma_tile_stage<F, NB>(), RPW = (16 + NB - 1) / NB;  // tile rows a wave copies (past the last: that one again)
     static_assert(RB % 16 == 0, "rows are copied 16 bytes a lane");

@@ -29,13 +29,13 @@
 // multiplication, into one of two LDS buffers of operand-ordered halves (one barrier a half); the activations come prepared in
 // operand order (kq_gemm_h6_prep) straight from global memory, four f16 steps ahead.  k runs outside the groups of weight rows,
 // so that these loads spread over the whole iteration: with the groups outside and a super-block's operands kept in registers
-// all 200 KB were asked for in the last seventh of an iteration (91 us at 512 x 14336 x 4096 against 85).
+// all 200 KB were asked for in the last seventh of an iteration, 7 % slower at 512 x 14336 x 4096.
 //
-// What bounds it (512 x 4096 x 14336, 85 us of kernel, the int8 GEMM 99): 8400 clocks a super-block, of which the matrix cores work
-// 4900 and the LDS moves operands for some 6500 (128 bytes a clock); the clock itself falls with the density of the work (2.1 GHz
-// at 10300 clocks a super-block, 1.8 at 8400), so power is the next bound.  Waves of 64 activation rows (four a workgroup, half
-// the LDS reads) take 131 us: one wave a SIMD has nothing to hide its vector instructions behind.
-// E2M1 codes of p, a third less to read, would be 2.6e-5 off 64 bits.  The codes' scales cost 1.3 us of a call (88.7 us, 89.9).
+// 512 x 14336 x 4096: 90 us of kernel where the int8 GEMM takes 112 (kernel trace, calls back to back), of the calls' 91 and 112
+// among others, 95 and 116 back to back.  Of 151 500 clocks that the chip is busy the matrix cores work 78 800 and the LDS moves
+// operands for 60 400 (counters): neither is full, and two waves a SIMD have a barrier every half super-block.  Waves of 64
+// activation rows (four a workgroup, half the LDS reads) take 131 us: one wave a SIMD has nothing to hide its vector instructions
+// behind.  E2M1 codes of p, a third less to read, would be 2.6e-5 off 64 bits.  The codes' scales cost 1.3 us of a call.
 #pragma once
 #include "kernels_dot4_q4k.hpp"
 

@@ -1,5 +1,5 @@
 // Matmul for many activation rows on the int8 matrix cores: every format but Q4_K, whose products take it from 64 to 127 rows and
-// kq_gemm_h6 (kernels_mfma_gemm_h6.hpp) from there on, 89 us for the 109 of this one.  The arithmetic is written out for Q4_K; Q6_K (w = d sc (q - 32), signed 8-bit sc, no min term) takes the same path with
+// kq_gemm_h6 (kernels_mfma_gemm_h6.hpp) from there on, 91 us for the 112 of this one at 512 x 14336 x 4096.  The arithmetic is written out for Q4_K; Q6_K (w = d sc (q - 32), signed 8-bit sc, no min term) takes the same path with
 // p = sc (q - 32), Q2_K with a one-byte p = sc q and sixteen sub-blocks in I2, Q8_0 with eight blocks put on
 // a common scale (QiQ2K, QiQ8_0 below).
 //
