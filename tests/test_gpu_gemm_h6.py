@@ -27,14 +27,15 @@ name = "q4k_gemm_i8" + ("+splitk" if splits > 1 else "")
 
 
 def parts(blocks, n, k):
-    # d sc (q - 8), and the factor d of it, of every element
+    # p = sc (q - 8) of every element, its factor d, and the power of two in sc / 32 that its code stands on
     b = blocks.reshape(n, k // 256, 144)
     d = b[:, :, 0:2].copy().view(np.float16).astype(np.float64)[:, :, 0]
     s = b[:, :, 4:16].astype(np.int64)
     sc = np.concatenate([s[:, :, :4] & 63, (s[:, :, 8:] & 15) | s[:, :, :4] >> 6 << 4], 2)
     q = b[:, :, 16:].reshape(n, k // 256, 4, 1, 32)
     q = np.concatenate([q & 15, q >> 4], 3).reshape(n, k // 256, 8, 32).astype(np.int64)
-    return (sc[..., None] * (q - 8)).astype(np.float64).reshape(n, -1, 256), d
+    unit = 2.0 ** (np.floor(np.log2(np.maximum(sc, 1))) - 5)
+    return (sc[..., None] * (q - 8)).astype(np.float64).reshape(n, -1, 256), d, unit.repeat(32, 2)
 
 
 def check(blocks, lhs, what, rms=None):
@@ -46,11 +47,11 @@ def check(blocks, lhs, what, rms=None):
     x = lhs.astype(np.float64)
     want = x @ w.T
     # With s <= 2^-14 of a super-block's largest magnitude: the remainder l <= 8 s of an activation as E2M3 is at most s / 2 off,
-    # p as E2M3 codes of 2^-7 p at most max(|p| / 16, 8): an element adds at most d s (|p| / 2 + 8 max(|p| / 16, 8)).  The mean of a
+    # p as E2M3 codes of 2^-7 p / unit at most max(|p| / 16, 8 unit): an element adds at most d s (|p| / 2 + 8 of that).  The mean of a
     # sub-block and its weight in two bf16 parts each: 2^-16 of the terms.  f32 sums: 2^-20 of them.
-    p, d = parts(blocks, n, k)
+    p, d, unit = parts(blocks, n, k)
     s = np.abs(x.reshape(m, -1, 256)).max(2) * 2.0 ** -14
-    off = np.abs(d) * (np.abs(p) / 2 + 8 * np.maximum(np.abs(p) / 16, 8)).sum(2)
+    off = np.abs(d) * (np.abs(p) / 2 + 8 * np.maximum(np.abs(p) / 16, 8 * unit)).sum(2)
     bound = s @ off.T + (2.0 ** -16 + 2.0 ** -20) * (np.abs(x) @ np.abs(w).T + np.abs(x) @ (np.abs(p) * np.abs(d)[..., None]).reshape(n, k).T)
     err = np.abs(got - want)
     assert np.all(err <= bound), (what, float((err / np.maximum(bound, 1e-300)).max()))
