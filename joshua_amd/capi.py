@@ -212,7 +212,7 @@ def last_kernel() -> str:
 
 
 def last_arithmetic() -> str:
-    """What the matrix-core GEMM over many rows multiplied, "int8" or "f16+fp6"; "" after any other kernel."""
+    """What the matrix-core GEMM multiplied: "int8", "f16+fp6", or "f16 pairs" (up to 16 rows); "" after any other kernel."""
     return lib().jq_last_arithmetic().decode()
 
 

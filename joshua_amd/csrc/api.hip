@@ -7,6 +7,7 @@
 #include "kernels_mfma_q4k.hpp"
 #include "kernels_graph.hpp"
 #include "kernels_mla.hpp"
+#include "few_rows.hpp"
 #include "moe_split16.hpp"
 #include "split16.hpp"
 #include "kernels_mfma_q4k_gemm.hpp"
@@ -1019,11 +1020,49 @@ int dispatch_gemm_decoded(uint32_t type, const uint8_t *W, size_t row_bytes, con
     }
 }
 
+// Which products of up to 16 rows the kernel of kernels_few_rows.hpp takes: where it is the fastest (us, then the kernels before it).
+// One row, where no one-row kernel takes the row length: against the f32 row kernels (Q8_0 6000 x 5120 13.9 / 19.1, 4096 x 2560 6.6 / 7.6;
+// MXFP4 6000 x 5120 10.2 / 18.9; Q6_K 14336 x 11264 43 / 58, but 11008 x 3840 18.6 / 18.0).
+// More rows, Q6_K, Q8_0, MXFP4: against the f32 row kernel, the one-row kernel once a row, the int8 GEMM (14336 x 4096: Q6_K 2 rows
+// 18.9 / 21.6, 16 rows 22 / 42; Q8_0 4 rows 18 / 43; MXFP4 8 rows 12 / 41; 1500 x 2304: 6.3 to 6.8 / 6.2 to 45).
+// Q4_K: two rows are faster on the one-row kernels' up to 64M weights (11008 x 3840 13.4 / 12.2, 14336 x 11264 28 / 47).  More:
+// rows that are no multiple of 4096 long 10 to 40 / 11 to 134; the others have dispatch_q4k_rows16, whose time does not grow with the
+// rows (4096 x 4096: 7.4 to 8.8 / 9.3; 14336 x 4096: 12.7 to 17 / 14.6; 4096 x 12288: 16 to 20 / 23; 12000 x 8192: 21 to 29 / 24).
+bool few_rows_better(uint32_t type, size_t m, size_t k, size_t n) {
+    static const char *off = getenv("JQ_FEW_ROWS");
+    if ((off && off[0] == '0') || m > 16) return false;
+    const size_t weights = n * k;
+    switch (type) {
+    case JQ_TYPE_Q4_K:
+        if (m == 1 || n < 1024 || k < 1024) return false;
+        if (m == 2) return weights >= ((size_t)64 << 20) && k != 4096;
+        return k % 4096 != 0 || k > 4 * 4096 || (m <= 8 ? k > 4096 || n <= 8192 : n <= 4096);
+    case JQ_TYPE_Q6_K: return weights >= (m == 1 ? (size_t)64 << 20 : (size_t)2 << 20);
+    case JQ_TYPE_Q8_0: return weights >= (m == 1 ? (size_t)8 << 20 : (size_t)2 << 20);
+    case JQ_TYPE_MXFP4: return weights >= (m == 1 ? (size_t)16 << 20 : (size_t)2 << 20);
+    default: return false;
+    }
+}
+
+// From 8 rows against 8M weights on (a format other than Q4_K) the name that callers know the many-row product by.
+const char *few_rows_name(uint32_t type, size_t m, size_t k, size_t n) {
+    if (m >= 8 && n * k >= ((size_t)8 << 20)) {
+        if (type == JQ_TYPE_Q6_K) return "q6k_gemm_i8+splitk";
+        if (type == JQ_TYPE_Q8_0) return "q8_0_gemm_i8+splitk";
+        if (type == JQ_TYPE_MXFP4) return "mxfp4_gemm_i8+splitk";
+    }
+    return "few_rows";
+}
+
 // All pointers are device pointers; shapes already validated; m, n > 0.
 int dispatch_matmul(uint32_t type, const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m,
                     size_t k, size_t n, hipStream_t s) {
     if (m > 0x7FFFFFFF || k > 0x7FFFFFFF || n > 0x7FFFFFFF) return fail("matmul: dimension exceeds 2^31-1");
     if (dense_elem_bytes(type)) return dense_matmul(type, W, row_bytes, X, Y, m, k, n, s);
+    if (m >= 2 && few_rows_better(type, m, k, n)) {
+        const int rc = few_rows_matmul(type, W, row_bytes, X, Y, m, k, n, few_rows_name(type, m, k, n), s);
+        if (rc >= 0) return rc;
+    }
     if (type == JQ_TYPE_Q4_K && m == 1) {
         const int rc = dispatch_q4k_dot4(W, row_bytes, X, Y, k, n, s);
         if (rc >= 0) return rc;
@@ -1049,18 +1088,8 @@ int dispatch_matmul(uint32_t type, const uint8_t *W, size_t row_bytes, const flo
         if (rc >= 0) return rc;
         rc = dispatch_i8_gemv(type, W, row_bytes, X, Y, k, n, s);
         if (rc >= 0) return rc;
-    }
-    // Q6_K and Q8_0 with two or three activation rows against a matrix of 16M weights or more: the one-row kernel
-    // once a row (4096 x 12288 of Q6_K, two rows: 23 us against 28 for the f32 row kernel; the int8 GEMM's 38 us
-    // are the same for 2 to 16 rows)
-    if ((type == JQ_TYPE_Q6_K || type == JQ_TYPE_Q8_0) && (m == 2 || m == 3) && n * k >= ((size_t)16 << 20)) {
-        static const char *no_loop = getenv("JQ_NO_ONE_ROW_LOOP");
-        int rc = no_loop ? -1 : 0;
-        for (size_t r = 0; r < m && rc == 0; r++)
-            rc = type == JQ_TYPE_Q6_K ? dispatch_q6k_dot4(W, row_bytes, X + r * k, Y + r * n, k, n, s)
-                                      : dispatch_q8_0_dot4(W, row_bytes, X + r * k, Y + r * n, k, n, s);
-        if (rc == 0) return 0;
-        if (rc > 0) return rc;  // (a kernel that declines does so at the first row, before anything is launched)
+        if (few_rows_better(type, 1, k, n)) rc = few_rows_matmul(type, W, row_bytes, X, Y, 1, k, n, few_rows_name(type, 1, k, n), s);
+        if (rc >= 0) return rc;
     }
     // Q4_K with a few activation rows.  Rows of 4096, 1024 weight rows or more: the int8 matrix-core kernel
     // on the one-row kernel's weight stream, in passes of 16 activation rows.  Other row lengths: one or two

@@ -1,0 +1,11 @@
+// Products of a few activation rows with packed weights (kernels_few_rows.hpp).
+#pragma once
+#include "core.hpp"
+
+namespace jqh {
+
+// Device pointers, shapes validated, k and n > 0.  -1: the call is outside its reach.
+int few_rows_matmul(uint32_t type, const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n,
+                    const char *name, hipStream_t s);
+
+}  // namespace jqh

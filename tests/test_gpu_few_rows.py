@@ -1,0 +1,102 @@
+"""Products of up to 16 activation rows on pairs of f16 numbers (few_rows) against 64-bit products of the decoded weights."""
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+import oracle
+from joshua_amd import capi, synth
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+TYPES = [capi.Q4_K, capi.Q6_K, capi.Q8_0, capi.MXFP4]
+
+
+def check(qtype, blocks, n, k, lhs, rms=3e-7, w=None):
+    """An activation s (hi + lo) is at most 2^-22 of itself off (2^-38 of its super-block's largest), the product of the two remainders,
+    left out, 2^-22 of the whole; f32 sums: some 8 roundings a super-block, a dozen of those, 8 waves, within a matrix instruction up to
+    four a result: 2^-18 of the terms' magnitudes in all.  Q4_K's terms are those of sc (q - 8) and of what it leaves."""
+    m = len(lhs)
+    got = (w or capi.Weight.upload(qtype, blocks, n, k)).matmul_t(m, lhs)
+    assert capi.last_arithmetic() == "f16 pairs", (capi.last_kernel(), capi.last_arithmetic())
+    d, x = oracle.dequantize(qtype, blocks).reshape(n, k).astype(np.float64), lhs.astype(np.float64)
+    mag = np.abs(d)
+    if qtype == capi.Q4_K:
+        b = blocks.reshape(n, k // 256, 144)
+        s = b[:, :, 4:16].astype(np.int64)
+        sc = np.concatenate([s[:, :, :4] & 63, (s[:, :, 8:] & 15) | s[:, :, :4] >> 6 << 4], 2)
+        mn = np.concatenate([s[:, :, 4:8] & 63, s[:, :, 8:] >> 4 | s[:, :, 4:8] >> 6 << 4], 2)
+        f = np.abs(b[:, :, 0:4].copy().view(np.float16).astype(np.float64))
+        mag = mag + 2 * (8 * f[:, :, :1] * sc + f[:, :, 1:] * mn).repeat(32, 2).reshape(n, k)
+    top = np.abs(x.reshape(m, -1, 256)).max(2).repeat(256, 1)
+    want, err = x @ d.T, None
+    err = np.abs(got - want)
+    bound = 2.0 ** -18 * (np.abs(x) @ mag.T) + 2.0 ** -36 * (top @ mag.T)
+    assert np.all(err <= bound), (m, k, n, float((err / np.maximum(bound, 1e-300)).max()))
+    if rms:
+        assert np.sqrt((err ** 2).mean() / (want ** 2).mean()) <= rms
+    return got
+
+
+# a tile of 16 weight rows a workgroup, two, four; their ragged ends; rows of 8 to 17 super-blocks over up to 8 waves
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("m,k,n", [(3, 2304, 1025), (4, 2048, 1039), (5, 4352, 1024), (8, 2560, 4097), (9, 2048, 5001), (16, 2304, 8223),
+                                   (16, 2048, 12289), (7, 1280, 12337), (13, 1280, 16399)])
+def test_edges_of_tiles(qtype, m, k, n):
+    blocks = synth.normal_quantized(qtype, 5 + n, n * k, 0.02)
+    check(qtype, blocks, n, k, synth.normal(6 + k, (m, k)))
+
+
+@pytest.mark.parametrize("qtype,k,n", [(capi.Q8_0, 5120, 1700), (capi.MXFP4, 4096, 4096), (capi.Q6_K, 7936, 8460)])
+def test_one_row_that_no_other_kernel_takes(qtype, k, n):
+    check(qtype, synth.normal_quantized(qtype, 7, n * k, 0.02), n, k, synth.normal(8, (1, k)))
+
+
+@pytest.mark.parametrize("qtype,step", [(capi.Q6_K, 210), (capi.MXFP4, 136)])
+def test_blocks_at_every_offset_to_16_bytes(qtype, step):
+    """Rows of an odd number of super-blocks from an offset into the allocation, up to its last byte."""
+    k, n = 9 * 256, 1100
+    raw = synth.normal_quantized(qtype, 9, (n * 9 + 3) * 256, 0.02)
+    parent = capi.Weight.upload(qtype, raw, n * 9 + 3, 256)
+    lhs = synth.normal(10, (6, k))
+    for first in (1, 2, 3):
+        check(qtype, raw[first * step:first * step + n * 9 * step], n, k, lhs, w=parent.view(first * step, n, k))
+
+
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("m", [5, 12])
+def test_every_scale_and_rows_of_every_range(qtype, m):
+    n, k = 1040, 2304
+    rng = np.random.default_rng(3)
+    if qtype == capi.Q8_0:
+        raw = rng.integers(0, 256, (n * k // 32, 34), dtype=np.uint8)
+        raw[:, :2] = (rng.uniform(-1, 1, len(raw)) * 2.0 ** rng.integers(-12, 1, len(raw))).astype(np.float16)[:, None].view(np.uint8)
+        raw[::11, :2] = 0
+        raw[:8, :2] = 0
+    elif qtype == capi.MXFP4:
+        raw = rng.integers(0, 256, (n * k // 32, 17), dtype=np.uint8)
+        raw[:, 0] = rng.integers(110, 140, len(raw))
+        raw[::13, 0] = 0xFF   # stands for zeros
+        raw[::17, 0] = 0
+        raw[:8, 0] = 0xFF
+    else:
+        size, at = (144, [0, 2]) if qtype == capi.Q4_K else (210, [208])
+        raw = rng.integers(0, 256, (n * k // 256, size), dtype=np.uint8)
+        for i in at:
+            raw[:, i:i + 2] = (rng.uniform(-1, 1, len(raw)) * 1e-3).astype(np.float16)[:, None].view(np.uint8)
+        raw[::7, at[0]:at[0] + 2] = 0
+    lhs = synth.normal(9, (m, k))
+    lhs[0] *= (10.0 ** rng.integers(-6, 7, size=k // 16)).repeat(16).astype(np.float32)
+    lhs[1] = 0
+    lhs[1, 1234] = 3.5
+    lhs[2, 512:1024] = 0
+    lhs[3] *= np.float32(1e30)
+    lhs[4] *= np.float32(1e-30)
+    got = check(qtype, raw.reshape(-1), n, k, lhs, rms=None)
+    lhs[0, 100], lhs[2, 2000] = np.inf, np.nan
+    other = capi.Weight.upload(qtype, raw.reshape(-1), n, k).matmul_t(m, lhs)
+    assert not np.isfinite(other[[0, 2]]).any()
+    assert np.array_equal(np.delete(other, [0, 2], 0), np.delete(got, [0, 2], 0))
