@@ -1028,9 +1028,25 @@ int dispatch_gemm_decoded(uint32_t type, const uint8_t *W, size_t row_bytes, con
 // Q4_K: two rows are faster on the one-row kernels' up to 64M weights (11008 x 3840 13.4 / 12.2, 14336 x 11264 28 / 47).  More:
 // rows that are no multiple of 4096 long 10 to 40 / 11 to 134; the others have dispatch_q4k_rows16, whose time does not grow with the
 // rows (4096 x 4096: 7.4 to 8.8 / 9.3; 14336 x 4096: 12.7 to 17 / 14.6; 4096 x 12288: 16 to 20 / 23; 12000 x 8192: 21 to 29 / 24).
+//
+// 17 rows and more: where its estimate is below that of what would run else, fitted to 24 shapes of 17 to 256 rows: the int8 GEMM, with at
+// most 127 rows 14.6 us and 0.62 a million weights (23 to 52 us at 4096 x 4096 to 14336 x 4096) or 0.5 a super-block of k, a third
+// more beyond; Q4_K a tenth less; rows of 4096 also dispatch_q4k_rows16's passes.  us, before / now: 32 rows x 14336 x 4096 Q4_K 27 / 19,
+// Q6_K 43 / 26, MXFP4 42 / 17; 64 rows x 3000 x 2560 22 to 25 / 11 to 12; 96 rows x 4096 x 4096 24 to 26 / 17 to 19;
+// 64 rows x 9000 x 9984 Q6_K 71 / 71, 127 rows 79 / 109 (hence the margin).  From 128 rows Q4_K is dispatch_gemm_h6's, and prepared
+// activations that the second level cache of an XCD does not hold are slow (200 rows x 1100 x 12288 41 / 55).
 bool few_rows_better(uint32_t type, size_t m, size_t k, size_t n) {
-    static const char *off = getenv("JQ_FEW_ROWS");
-    if ((off && off[0] == '0') || m > 16) return false;
+    static const char *off = getenv("JQ_FEW_ROWS"), *i8_shape = getenv("JQ_Q4K_GEMM_I8_SHAPE"), *i8_min_m = getenv("JQ_Q4K_GEMM_I8_MIN_M");
+    if (off && off[0] == '0') return false;
+    if (m > 16) {
+        const bool q4 = type == JQ_TYPE_Q4_K;
+        if ((!q4 && type != JQ_TYPE_Q6_K && type != JQ_TYPE_Q8_0 && type != JQ_TYPE_MXFP4) || i8_shape || i8_min_m || n < 512 || k < 1024 ||
+            n * k < ((size_t)2 << 20) || m > (q4 ? 127 : 255) || (m > 127 && m * k > 1500000))
+            return false;
+        double us = std::max(14.6 + 0.62e-6 * (double)(n * k), 9.0 + 0.5 * (double)(k / 256)) * (m > 127 ? 1.3 : 1.0) * (q4 ? 0.9 : 1.0);
+        if (q4 && k == 4096) us = std::min(us, 3.0 + (double)((m + 15) / 16) * (4.3 + 0.527 * (double)n / 1024.0));
+        return few_rows_many_us(type, m, k, n) < 0.92 * us;
+    }
     const size_t weights = n * k;
     switch (type) {
     case JQ_TYPE_Q4_K:
@@ -1044,13 +1060,13 @@ bool few_rows_better(uint32_t type, size_t m, size_t k, size_t n) {
     }
 }
 
-// From 8 rows against 8M weights on (a format other than Q4_K) the name that callers know the many-row product by.
+// The name that callers know the product by: from 8 rows against 8M weights on (a format other than Q4_K) the many-row GEMM's, from 17
+// rows on that of the GEMM that took it else.
 const char *few_rows_name(uint32_t type, size_t m, size_t k, size_t n) {
-    if (m >= 8 && n * k >= ((size_t)8 << 20)) {
-        if (type == JQ_TYPE_Q6_K) return "q6k_gemm_i8+splitk";
-        if (type == JQ_TYPE_Q8_0) return "q8_0_gemm_i8+splitk";
-        if (type == JQ_TYPE_MXFP4) return "mxfp4_gemm_i8+splitk";
-    }
+    if (type == JQ_TYPE_Q4_K) return m <= 16 ? "few_rows" : m < 64 ? "q4k_gemm_mfma+splitk" : "q4k_gemm_i8+splitk";
+    if ((m >= 8 && n * k >= ((size_t)8 << 20)) || m >= 64)
+        return type == JQ_TYPE_Q6_K ? "q6k_gemm_i8+splitk" : type == JQ_TYPE_Q8_0 ? "q8_0_gemm_i8+splitk" : "mxfp4_gemm_i8+splitk";
+    if (m > 16) return "gemm_decoded_mfma+splitk";
     return "few_rows";
 }
 
@@ -1060,7 +1076,7 @@ int dispatch_matmul(uint32_t type, const uint8_t *W, size_t row_bytes, const flo
     if (m > 0x7FFFFFFF || k > 0x7FFFFFFF || n > 0x7FFFFFFF) return fail("matmul: dimension exceeds 2^31-1");
     if (dense_elem_bytes(type)) return dense_matmul(type, W, row_bytes, X, Y, m, k, n, s);
     if (m >= 2 && few_rows_better(type, m, k, n)) {
-        const int rc = few_rows_matmul(type, W, row_bytes, X, Y, m, k, n, few_rows_name(type, m, k, n), s);
+        const int rc = (m <= 16 ? few_rows_matmul : few_rows_many_matmul)(type, W, row_bytes, X, Y, m, k, n, few_rows_name(type, m, k, n), s);
         if (rc >= 0) return rc;
     }
     if (type == JQ_TYPE_Q4_K && m == 1) {

@@ -419,4 +419,224 @@ static __global__ __launch_bounds__(512, 2) void few_rows(const uint8_t *__restr
     }
 }
 
+// ---- more than 16 rows -------------------------------------------------------------------------------------------------------
+
+// Prepared activations, for every 16 rows and super-block: 8 k-steps of two fragments (first numbers, second numbers), the operand
+// of the mins, the 16 rows' units.
+constexpr int FR_MIN = 16 * S16_FRAG, FR_UNIT = FR_MIN + S16_FRAG, FR_REC = FR_UNIT + 64;
+
+// A lane's 64 elements of a row -> its share of the fragments, and the row's unit.
+template <class F>
+__device__ __forceinline__ void fr_operands(const float (&x)[64], s16_h8 (&hi)[8], s16_h8 (&lo)[8], s16_h8 &xs, float &unit) {
+    float amax = 0.0f;  // (a NaN is passed over here and stays one below)
+#pragma unroll
+    for (int i = 0; i < 64; i += 2) asm volatile("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(amax) : "v"(x[i]), "v"(x[i + 1]));
+    amax = max_xor32(max_xor16(amax));
+    const bool finite = amax < INFINITY;
+    const int e = s16_exponent(__builtin_bit_cast(uint32_t, amax));
+    const float f = finite ? s16_pow2(e) : 0.0f;
+    unit = finite ? s16_pow2(-e) : __builtin_nanf("");
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+        const float v[8] = {x[F::at(s, 0)], x[F::at(s, 1)], x[F::at(s, 2)], x[F::at(s, 3)], x[F::at(s, 4)], x[F::at(s, 5)], x[F::at(s, 6)], x[F::at(s, 7)]};
+        fr_split(v, f, f, hi[s], lo[s]);
+    }
+    if constexpr (F::MINS) {
+        float sum[2] = {0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 64; i++) sum[i >> 5] += x[i];
+        const s16_f2 v = {sum[0] * (0.03125f * f), sum[1] * (0.03125f * f)};
+        const s16_h2 h = __builtin_convertvector(v, s16_h2);
+        const s16_f2 left = {v[0] - (float)h[0], v[1] - (float)h[1]};
+        const s16_h2 l = __builtin_convertvector(left, s16_h2);
+        const s16_h2 j = __builtin_convertvector(s16_f2{left[0] - (float)l[0], left[1] - (float)l[1]}, s16_h2);
+        xs = s16_h8{h[0], h[1], l[0], l[1], h[0], h[1], j[0], j[1]};
+    }
+}
+
+// grid (super-blocks, groups of 16 rows), a wave each
+template <class F>
+static __global__ __launch_bounds__(64) void few_rows_prep(const float *__restrict__ X, int m, int nb, uint8_t *__restrict__ out) {
+    const int lane = threadIdx.x, r = lane & 15, g = lane >> 4, row = 16 * (int)blockIdx.y + r;
+    uint8_t *rec = out + ((size_t)blockIdx.y * nb + blockIdx.x) * FR_REC;
+    const float *src = X + (size_t)min(row, m - 1) * nb * 256 + 256 * blockIdx.x;
+    float x[64], unit;
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const float4 v = *(const float4 *)(src + F::quad(g, q));
+        x[4 * q] = v.x, x[4 * q + 1] = v.y, x[4 * q + 2] = v.z, x[4 * q + 3] = v.w;
+    }
+    s16_h8 hi[8], lo[8], xs;
+    fr_operands<F>(x, hi, lo, xs, unit);
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+        *(s16_h8 *)(rec + (2 * s * 64 + lane) * 16) = hi[s];
+        *(s16_h8 *)(rec + ((2 * s + 1) * 64 + lane) * 16) = lo[s];
+    }
+    if constexpr (F::MINS) *(s16_h8 *)(rec + FR_MIN + 16 * lane) = xs;
+    if (g == 0) *(float *)(rec + FR_UNIT + 4 * r) = unit;
+}
+
+template <class F>
+constexpr int few_rows_many_lds(int waves, int nt, int mt) {
+    const int stage = waves * 256 * nt * F::PIECES, sums = waves * nt * mt * 1024;
+    return stage > sums ? stage : sums;
+}
+
+// few_rows for 16 MT activation rows a workgroup.  Bound: the prepared activations on their way from the second level cache, some 35 bytes a
+// clock and compute unit (32 rows x 12288 x 4096: 25 us, of them 19 for the 1.5 MB that each compute unit reads), with more tiles a
+// workgroup the issue of instructions.  32 rows x 14336 x 4096: Q4_K 27 -> 19 us, Q6_K 43 -> 26, MXFP4 42 -> 17.
+// The activations' operands come prepared, straight into registers, AHEAD k-steps before they are multiplied; the weights of NT tiles as
+// in few_rows.  Workgroups 8 apart (one XCD) hold the row blocks of one column block.
+template <class F, int NT, int MT, int AHEAD>
+static __global__ __launch_bounds__(512, 2) void few_rows_many(const uint8_t *__restrict__ W, uint32_t row_bytes, const uint8_t *__restrict__ acts,
+                                                               float *__restrict__ Y, int m, int n, int nb, int groups, int blocks) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t fr_lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+    const int waves = blockDim.x >> 6, id = blockIdx.x, n0 = (id / 8 / blocks * 8 + id % 8) * 16 * NT, g0 = id / 8 % blocks * MT;
+    if (n0 >= n) return;
+    constexpr bool EVEN = F::ALIGN == 16;
+    constexpr int TILE = 256 * F::PIECES, COPIES = (F::PIECES + 3) / 4;
+    const uint8_t *const first = W + (size_t)n0 * row_bytes;
+    const uint32_t mis = EVEN ? 0u : (uint32_t)(uintptr_t)first & 15u;
+    const uint8_t *const base = s16_uniform(first - mis);
+    uint32_t at[NT][COPIES];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int j = 0; j < COPIES; j++) {
+            const int piece_id = min(64 * j + lane, 16 * F::PIECES - 1), row = 16 * t + piece_id / F::PIECES, piece = min(piece_id % F::PIECES, F::REAL - 1);
+            const uint32_t off = (uint32_t)min(row, n - 1 - n0) * row_bytes;
+            at[t][j] = EVEN ? off + 16u * piece : (off + mis) << 4 | (uint32_t)piece;
+        }
+    uint8_t *const own = fr_lds + wave * NT * TILE;
+    const uint32_t own_at = s16_lds_offset(own);
+    const uint8_t *const my_w = own + 16 * F::PIECES * r;
+    auto fetch_w = [&](int sb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int j = 0; j < COPIES; j++) {
+                const uint32_t dst = __builtin_amdgcn_readfirstlane(own_at + t * TILE + 1024 * j), shift = (uint32_t)sb * F::BLOCK;
+                const uint32_t off = EVEN ? at[t][j] + shift : (((at[t][j] >> 4) + shift) & ~15u) + ((at[t][j] & 15u) << 4);
+                if (F::PIECES % 4 == 0 || j + 1 < COPIES || lane < 16 * (F::PIECES % 4))
+                    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst) : "memory");
+            }
+    };
+    uint32_t rec[MT];  // the groups' records; past the last group: the last one again, not stored
+#pragma unroll
+    for (int j = 0; j < MT; j++) rec[j] = (uint32_t)(min(g0 + j, groups - 1) - g0) * (uint32_t)nb * FR_REC;
+    const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc((void *)s16_uniform(acts + (size_t)g0 * nb * FR_REC), 0, 0xFFFFFFFFu, 0x00027000);
+    const int l16 = 16 * lane;
+    s16_h8 A[AHEAD][MT][2];
+    auto load = [&](int sb, int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < MT; j++)
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+                A[s % AHEAD][j][p] = __builtin_bit_cast(s16_h8, __builtin_amdgcn_raw_buffer_load_b128(src, l16, (int)(rec[j] + (uint32_t)sb * FR_REC + (2 * s + p) * S16_FRAG), 0));
+    };
+    const s16_f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    s16_f4 acc[NT][MT];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int j = 0; j < MT; j++) acc[t][j] = zero;
+    if (wave < nb) {
+        fetch_w(wave);
+#pragma unroll
+        for (int s = 0; s < AHEAD; s++) load(wave, s);
+    }
+    for (int sb = wave; sb < nb; sb += waves) {
+        const int next = sb + waves < nb ? sb + waves : sb;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        typename F::Raw raw[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            uint32_t skip = 0;
+            if constexpr (!EVEN) skip = (mis + (uint32_t)min(16 * t + r, n - 1 - n0) * row_bytes + (uint32_t)sb * F::BLOCK) & 15u;
+            raw[t].load(my_w + t * TILE + skip, g);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (next != sb) fetch_w(next);
+        __builtin_amdgcn_sched_barrier(0);
+        F w[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) w[t].begin(raw[t], g);
+        constexpr bool APART = NT * MT <= 4;  // the products with the remainders in sums of their own, where registers are left
+        s16_f4 sums[NT][MT], low[APART ? NT : 1][APART ? MT : 1];
+        s16_h8 xs[MT];
+        s16_f4 unit[MT];
+        auto step = [&](auto sc) __attribute__((always_inline)) {
+            constexpr int S = decltype(sc)::value;
+            s16_h8 a[MT][2];
+#pragma unroll
+            for (int j = 0; j < MT; j++) a[j][0] = A[S % AHEAD][j][0], a[j][1] = A[S % AHEAD][j][1];
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                s16_h8 p[F::PLANES];
+                w[t].template step<S>(raw[t], p);
+#pragma unroll
+                for (int j = 0; j < MT; j++) sums[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j][0], p[0], S == 0 ? zero : sums[t][j], 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < MT; j++) {
+                    s16_f4 &to = APART ? low[APART ? t : 0][APART ? j : 0] : sums[t][j];
+                    to = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j][1], p[0], APART && S == 0 ? zero : to, 0, 0, 0);
+                }
+                if constexpr (F::PLANES == 2) {
+#pragma unroll
+                    for (int j = 0; j < MT; j++) {
+                        s16_f4 &to = APART ? low[APART ? t : 0][APART ? j : 0] : sums[t][j];
+                        to = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j][0], p[1], to, 0, 0, 0);
+                    }
+                }
+            }
+            if constexpr (S + AHEAD < 8) load(sb, S + AHEAD);
+            else load(next, S + AHEAD - 8);
+            if constexpr (S == 7 - AHEAD) {
+#pragma unroll
+                for (int j = 0; j < MT; j++) {
+                    const int at_sb = (int)(rec[j] + (uint32_t)sb * FR_REC);
+                    if constexpr (F::MINS) xs[j] = __builtin_bit_cast(s16_h8, __builtin_amdgcn_raw_buffer_load_b128(src, l16, at_sb + FR_MIN, 0));
+                    unit[j] = __builtin_bit_cast(s16_f4, __builtin_amdgcn_raw_buffer_load_b128(src, 16 * g, at_sb + FR_UNIT, 0));
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        step(std::integral_constant<int, 0>{}), step(std::integral_constant<int, 1>{}), step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{}), step(std::integral_constant<int, 4>{}), step(std::integral_constant<int, 5>{});
+        step(std::integral_constant<int, 6>{}), step(std::integral_constant<int, 7>{});
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int j = 0; j < MT; j++) {
+                s16_f4 i2 = zero;
+                if constexpr (APART) sums[t][j] += low[t][j];
+                if constexpr (F::MINS) i2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xs[j], w[t].mins, zero, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float sum = w[t].d * sums[t][j][i];
+                    acc[t][j][i] = fmaf(unit[j][i], F::MINS ? fmaf(w[t].dm, i2[i], sum) : sum, acc[t][j][i]);
+                }
+            }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int j = 0; j < MT; j++) *(s16_f4 *)(fr_lds + ((wave * NT * MT + t * MT + j) * 64 + lane) * 16) = acc[t][j];
+    __syncthreads();
+    for (int i = tid; i < NT * MT * 64; i += 64 * waves) {
+        s16_f4 v = zero;
+        for (int w = 0; w < waves; w++) v += *(const s16_f4 *)(fr_lds + (w * NT * MT * 64 + i) * 16);
+        const int t = (i >> 6) / MT, j = (i >> 6) % MT, col = n0 + 16 * t + (i & 15), row = 16 * (g0 + j) + 4 * ((i >> 4) & 3);
+        if (col < n) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (row + q < m) Y[(size_t)(row + q) * n + col] = v[q];
+        }
+    }
+}
+
 }  // namespace jq

@@ -1,4 +1,4 @@
-"""Products of up to 16 activation rows on pairs of f16 numbers (few_rows) against 64-bit products of the decoded weights."""
+"""Products of up to some 100 activation rows on pairs of f16 numbers (few_rows, few_rows_many) against 64-bit products of the decoded weights."""
 import os
 import subprocess
 import sys
@@ -50,6 +50,39 @@ def test_edges_of_tiles(qtype, m, k, n):
     check(qtype, blocks, n, k, synth.normal(6 + k, (m, k)))
 
 
+MANY = r"""
+import sys
+sys.path.insert(0, %r)
+from joshua_amd import capi, synth
+from tests.test_gpu_few_rows import TYPES, check
+for m, k, n in [(17, 2304, 1025), (33, 2048, 1039), (48, 4352, 1024), (64, 1280, 2111), (65, 2048, 1100), (127, 2304, 1055)]:
+    for qtype in TYPES:
+        check(qtype, synth.normal_quantized(qtype, 5 + n, n * k, 0.02), n, k, synth.normal(6 + k, (m, k)))
+print("many ok")
+"""
+
+
+@pytest.mark.parametrize("shape", ["1,2", "2,2", "4,2", "2,3", "2,4"])
+def test_more_than_16_rows_in_every_workgroup_shape(shape):
+    """The shape is read at the first product, hence the child process."""
+    res = subprocess.run([sys.executable, "-c", MANY % ROOT], env=dict(os.environ, JQ_FEW_ROWS_SHAPE=shape), capture_output=True, text=True, timeout=110)
+    assert res.returncode == 0 and "many ok" in res.stdout, res.stdout + res.stderr
+
+
+@pytest.mark.parametrize("qtype,m,k,n,name", [(capi.Q4_K, 61, 7168, 2112, "q4k_gemm_mfma+splitk"), (capi.Q6_K, 100, 4096, 4096, "q6k_gemm_i8+splitk"),
+                                              (capi.Q8_0, 40, 2304, 1500, "gemm_decoded_mfma+splitk"), (capi.MXFP4, 160, 2048, 1024, "mxfp4_gemm_i8+splitk")])
+def test_the_call_that_allocates_nothing(qtype, m, k, n, name):
+    import torch
+    w = capi.Weight.upload(qtype, synth.normal_quantized(qtype, 61, n * k, 0.02), n, k)
+    x, y = torch.from_numpy(synth.normal(62, (m, k))).cuda(), torch.full((2, m, n), float("nan"), device="cuda")
+    s = torch.cuda.current_stream().cuda_stream
+    for i, call in enumerate((w.matmul_t_dev, w.matmul_t_noalloc)):
+        call(m, x.data_ptr(), m * k, y[i].data_ptr(), m * n, s)
+        assert (capi.last_kernel(), capi.last_arithmetic()) == (name, "f16 pairs")
+    torch.cuda.synchronize()
+    assert torch.equal(y[0], y[1])
+
+
 @pytest.mark.parametrize("qtype,k,n", [(capi.Q8_0, 5120, 1700), (capi.MXFP4, 4096, 4096), (capi.Q6_K, 7936, 8460)])
 def test_one_row_that_no_other_kernel_takes(qtype, k, n):
     check(qtype, synth.normal_quantized(qtype, 7, n * k, 0.02), n, k, synth.normal(8, (1, k)))
@@ -63,11 +96,12 @@ def test_blocks_at_every_offset_to_16_bytes(qtype, step):
     parent = capi.Weight.upload(qtype, raw, n * 9 + 3, 256)
     lhs = synth.normal(10, (6, k))
     for first in (1, 2, 3):
-        check(qtype, raw[first * step:first * step + n * 9 * step], n, k, lhs, w=parent.view(first * step, n, k))
+        for rows in (lhs, np.concatenate([lhs] * 4)):
+            check(qtype, raw[first * step:first * step + n * 9 * step], n, k, rows, w=parent.view(first * step, n, k))
 
 
 @pytest.mark.parametrize("qtype", TYPES)
-@pytest.mark.parametrize("m", [5, 12])
+@pytest.mark.parametrize("m", [5, 12, 40])
 def test_every_scale_and_rows_of_every_range(qtype, m):
     n, k = 1040, 2304
     rng = np.random.default_rng(3)
