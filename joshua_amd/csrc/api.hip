@@ -849,7 +849,7 @@ int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *
     struct Shape {
         int nw, ng;
     };
-    static const Shape shapes[] = {{8, 7}, {8, 6}, {4, 4}};
+    static const Shape shapes[] = {{8, 8}, {8, 7}, {8, 6}, {4, 4}};
     const size_t nb = k / 256, groups = (m + 15) / 16;
     const size_t scratch_cap = tl_fixed_scratch ? tl_fixed_scratch->bytes : (size_t)1 << 40;
     // A fixed scratch that holds the int8 GEMM's records of all rows, three quarters of these in size, takes the rows in two turns;
@@ -869,12 +869,13 @@ int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *
         const size_t ty = rows_of(sh, rows), tiles = ty * cols_of(sh);
         return 8 % ty == 0 ? (tiles + 7) / 8 * 8 : tiles;
     };
-    if (!min_m_env && rows_of(shapes[2], m) * cols_of(shapes[2]) * std::max<size_t>(1, std::min<size_t>(nb / 4, 8)) < 64) return -1;
+    if (!min_m_env && rows_of(shapes[3], m) * cols_of(shapes[3]) * std::max<size_t>(1, std::min<size_t>(nb / 4, 8)) < 64) return -1;
     auto rounds = [](double wgs, double at_once, auto us) {
         const double whole = std::floor(wgs / at_once), rest = wgs - whole * at_once;
         return whole * us(at_once) + (rest > 0.0 ? us(rest) : 0.0);
     };
-    // In us, the int8 GEMM's form of estimate (dispatch_gemm_i8) fitted to 714 times of this one's three shapes in 1 to 8 parts: the
+    // In us, the int8 GEMM's form of estimate (dispatch_gemm_i8) fitted to 714 times of this one's shapes of seven, six and four groups in 1 to 8 parts (eight groups: 1.09 of
+    // seven's super-block, 512 to 2048 rows x 4096 to 24576): the
     // preparation, a fixed start, the super-blocks a workgroup walks at a cost that grows with the workgroups at work, the
     // starts of further rounds, the sum of the parts.  Over 166 shapes the picks are 0.7 % off the best measured choice on
     // average, 5 % at the 95th percentile, 12 % at worst.
@@ -882,7 +883,7 @@ int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *
         const double wgs = (double)(grid_of(sh, m) * sp), nbl = (double)(nb / sp);
         double us = 3.2 + 0.0048 * (double)(nb * groups);
         if (sh.nw == 8)
-            us += 6.4 + nbl * rounds(wgs, 256.0, [](double w) { return 3.4 + 0.0035 * w; }) * (sh.ng == 7 ? 1.0 : 0.92) +
+            us += 6.4 + nbl * rounds(wgs, 256.0, [](double w) { return 3.4 + 0.0035 * w; }) * (sh.ng == 8 ? 1.09 : sh.ng == 7 ? 1.0 : 0.92) +
                   4.2 * (std::ceil(wgs / 256.0) - 1.0);
         else
             us += 6.6 + nbl * rounds(wgs, 512.0, [](double w) { return w <= 256.0 ? 2.24 + 0.0011 * w : 3.06 + 0.0011 * w; }) +
@@ -900,7 +901,7 @@ int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *
         for (size_t sp = 1; sp <= 8; sp++) {
             if (nb % sp != 0 || (sp > 1 && nb / sp < 4)) continue;
             if (splits_env && sp != (size_t)atoi(splits_env)) continue;
-            if (sp > 1 && (m * n > 0x3FFFFFFFull || acts_bytes + sp * turn * n * sizeof(float) > scratch_cap)) continue;
+            if (sp > 1 && (m * n > 0x3FFFFFFFull || acts_bytes + (sp - 1) * turn * n * sizeof(float) > scratch_cap)) continue;
             const double us = estimate(sh, sp);
             if (!best || us < best_us) best = &sh, splits = sp, best_us = us;
         }
@@ -909,8 +910,8 @@ int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *
     if (grid_of(*best, m) > 0x7FFFFFFFull) return -1;
     CallScratch scratch;
     uint8_t *acts = nullptr;
-    if (scratch.get(acts_bytes + (splits > 1 ? splits * turn * n * sizeof(float) : 0), s, &acts)) return 1;
-    float *parts = (float *)(acts + acts_bytes);
+    if (scratch.get(acts_bytes + (splits - 1) * turn * n * sizeof(float), s, &acts)) return 1;
+    float *parts = (float *)(acts + acts_bytes);  // of all parts of k but the first, which is summed in place
     auto launch = [&](auto kern, int lds, int nw, hipError_t rc) {
         if (rc != hipSuccess) return fail("hipFuncSetAttribute: %s", hipGetErrorString(rc));
         for (size_t m0 = 0; m0 < m; m0 += turn) {
@@ -921,15 +922,15 @@ int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *
             if (swiglu_pairs) hipLaunchKernelGGL(jq::kq_gemm_h6_prep<true>, prep, dim3(128), 0, s, x, (int)rows, (int)k, acts);
             else hipLaunchKernelGGL(jq::kq_gemm_h6_prep<false>, prep, dim3(128), 0, s, x, (int)rows, (int)k, acts);
             hipLaunchKernelGGL(kern, dim3((unsigned)grid_of(*best, rows), (unsigned)splits), dim3(64 * nw), lds, s, W, row_bytes,
-                               (const uint8_t *)acts, splits > 1 ? parts : y, (int)rows, (int)n, (int)(nb / splits), (int)row_groups,
-                               (int)cols_of(*best), (int)rows_of(*best, rows), (int)nb, splits > 1 ? outs : (size_t)0);
+                               (const uint8_t *)acts, y, (int)rows, (int)n, (int)(nb / splits), (int)row_groups,
+                               (int)cols_of(*best), (int)rows_of(*best, rows), (int)nb, parts);
             if (splits > 1)
-                hipLaunchKernelGGL(jq::splitk_sum, dim3((unsigned)((outs + 1023) / 1024)), dim3(256), 0, s, parts, y, outs, (int)splits);
+                hipLaunchKernelGGL(jq::splitk_add, dim3((unsigned)((outs + 1023) / 1024)), dim3(256), 0, s, parts, y, outs, (int)splits - 1);
         }
         return 0;
     };
 #define JQ_GEMM_H6(NW_, NG_) launch(jq::kq_gemm_h6<F, NW_, NG_>, jq::h6_lds_bytes<NG_>(), NW_, big_lds_once<&jq::kq_gemm_h6<F, NW_, NG_>>(jq::h6_lds_bytes<NG_>()))
-    const int rc = best->nw == 4 ? JQ_GEMM_H6(4, 4) : best->ng == 7 ? JQ_GEMM_H6(8, 7) : JQ_GEMM_H6(8, 6);
+    const int rc = best->nw == 4 ? JQ_GEMM_H6(4, 4) : best->ng == 8 ? JQ_GEMM_H6(8, 8) : best->ng == 7 ? JQ_GEMM_H6(8, 7) : JQ_GEMM_H6(8, 6);
 #undef JQ_GEMM_H6
     if (rc) return rc;
     note_kernel(splits > 1 ? name_split : name, "f16+fp6");

@@ -31,6 +31,9 @@
 // so that these loads spread over the whole iteration: with the groups outside and a super-block's operands kept in registers
 // all 200 KB were asked for in the last seventh of an iteration, 7 % slower at 512 x 14336 x 4096.
 //
+// Groups: seven make 256 workgroups of 512 x 14336, eight of 2048 x 4096 (calls: 156 -> 110 us, with rows of 12288 400 -> 317, against
+// the better of six groups' 344 workgroups and small tiles) and, with k in four parts, of 512 x 4096 (51 -> 44); nothing fits more.
+//
 // 512 x 14336 x 4096: 90 us of kernel where the int8 GEMM takes 112 (kernel trace, calls back to back), of the calls' 91 and 112
 // among others, 95 and 116 back to back.  Of 151 500 clocks that the chip is busy the matrix cores work 78 800 and the LDS moves
 // operands for 60 400 (counters): neither is full, and two waves a SIMD have a barrier every half super-block.  Waves of 64
@@ -263,7 +266,7 @@ __device__ __forceinline__ h6_i8 h6_operand6(h6_u6 v) {
 template <class F, int NW, int NG>
 __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict__ W, size_t row_bytes,
                                                       const uint8_t *__restrict__ acts, float *__restrict__ Y, int m_rows, int n,
-                                                      int nb, int groups, int tx, int ty, int nb_total, size_t split_stride) {
+                                                      int nb, int groups, int tx, int ty, int nb_total, float *__restrict__ parts) {
     static_assert(NG <= NW && NG <= 8, "one group of 16 weight rows a wave unpacks, a byte each of a lane's eight exponents");
     constexpr int NT = 16 * NG, MT = 32 * NW;
     extern __shared__ __attribute__((aligned(16))) uint8_t h6_lds[];
@@ -277,7 +280,7 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
     }
     if (bx >= tx || by >= ty) return;
     const int n0 = bx * NT, m0 = by * MT, b_first = (int)blockIdx.y * nb;
-    Y += (size_t)blockIdx.y * split_stride;
+    if (blockIdx.y > 0) Y = parts + (size_t)(blockIdx.y - 1) * m_rows * n;  // k in parts: the first one's sums in place, splitk_add
 
     // everything is read behind an address that is the same in all lanes of a wave
     const int wv = __builtin_amdgcn_readfirstlane(wave), wu = min(wv, NG - 1);  // (waves past the last group unpack it too)
@@ -343,7 +346,7 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
         if (t < 3 * NG) return Step{t % NG, t < NG ? 5 : t / NG - 1};
         return Step{(t - 3 * NG) / 3, 2 + (t - 3 * NG) % 3};
     };
-    constexpr int AHEAD = 4;
+    constexpr int AHEAD = NG == 8 ? 2 : 4;  // operand reads; with eight groups the registers are just enough for two (no difference in time)
     for (int b = 0; b < nb; b++) {
         const int b1 = min(b + 1, nb - 1);
         const uint8_t *meta = meta_lds + (b & 1) * (NG * H6_META);
@@ -438,6 +441,26 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
                 if (col < n) Y[(size_t)row * n + col] = acc[mg][cg][i];
             }
         }
+}
+
+// Y[i] += P[0][i], then P[1][i], .. P[parts - 1][i], four elements a thread.
+__global__ __launch_bounds__(256) void splitk_add(const float *__restrict__ P, float *__restrict__ Y, size_t count, int parts) {
+    const size_t i = 4 * ((size_t)blockIdx.x * 256 + threadIdx.x);
+    if (i >= count) return;
+    if ((count & 3) == 0) {
+        float4 a = *(const float4 *)(Y + i);
+        for (int p = 0; p < parts; p++) {
+            const float4 b = *(const float4 *)(P + (size_t)p * count + i);
+            a.x += b.x, a.y += b.y, a.z += b.z, a.w += b.w;
+        }
+        *(float4 *)(Y + i) = a;
+    } else {
+        for (size_t j = i; j < count && j < i + 4; j++) {
+            float a = Y[j];
+            for (int p = 0; p < parts; p++) a += P[(size_t)p * count + j];
+            Y[j] = a;
+        }
+    }
 }
 
 }  // namespace jq

@@ -102,6 +102,11 @@ def test_gemm_on_f16_and_fp6_operands(shape, splits):
     assert res.returncode == 0 and "h6 ok" in res.stdout, res.stdout + res.stderr
 
 
+@pytest.mark.parametrize("splits", [1, 4])
+def test_workgroups_of_eight_groups_of_weight_rows(splits):
+    test_gemm_on_f16_and_fp6_operands("8,8", splits)
+
+
 def q4k_blocks(d, dmin, sc, mn, q):
     """Blocks of [n][super-blocks]: d, dmin, sc and mn [..., 8] of six bits, q [..., 8, 32] of four."""
     b = np.zeros(d.shape + (144,), np.uint8)
