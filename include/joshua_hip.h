@@ -73,8 +73,8 @@ const char *jq_last_error(void);
  * where k is split; jq_last_arithmetic tells its forms apart. */
 const char *jq_last_kernel(void);
 
-/* What that GEMM multiplied: "int8" (two 8-bit planes a factor), "f16+fp6" (Q4_K from 128
- * activation rows on: f16 products, their remainders in FP6) or "f16 pairs" (two f16 numbers a
+/* What that GEMM multiplied: "int8" (two 8-bit planes a factor), "f16+fp6" (Q4_K and MXFP4 from
+ * 128 activation rows on: f16 products, their remainders in FP6) or "f16 pairs" (two f16 numbers a
  * factor, 22 bits: up to some 100 activation rows, also after the kernel "few_rows" and under the
  * names "q4k_gemm_mfma" and "gemm_decoded_mfma" that fewer than 64 rows go by); "" after any other. */
 const char *jq_last_arithmetic(void);

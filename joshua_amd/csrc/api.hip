@@ -8,6 +8,7 @@
 #include "kernels_graph.hpp"
 #include "kernels_mla.hpp"
 #include "few_rows.hpp"
+#include "gemm_h6.hpp"
 #include "moe_split16.hpp"
 #include "split16.hpp"
 #include "kernels_mfma_q4k_gemm.hpp"
@@ -23,7 +24,6 @@
 #include "kernels_moe_q4k_quads.hpp"
 #include "kernels_mfma_q4k_rows16.hpp"
 #include "kernels_mfma_q4k_gemm_i8.hpp"
-#include "kernels_mfma_gemm_h6.hpp"
 #include "kernels_valu.hpp"
 #include "kernels_mfma_decoded.hpp"
 
@@ -680,7 +680,7 @@ int dispatch_q4k_rows16(const uint8_t *W, size_t row_bytes, const float *X, floa
     return 0;
 }
 
-// Many activation rows on the int8 matrix cores (Q4_K up to 127 of them, dispatch_gemm_h6's products from there on): the activations as two int8 planes per
+// Many activation rows on the int8 matrix cores (Q4_K up to 127 of them, gemm_h6's products from there on): the activations as two int8 planes per
 // 256-element super-block in the call scratch of the stream, then kq_gemm_i8 with the workgroup shape and the
 // split over k that an estimate fitted to measurements prefers.  Returns -1 when the shape is outside its
 // reach or the product is tiny.  JQ_Q4K_GEMM_I8 = 0 switches it off; JQ_Q4K_GEMM_I8_SHAPE and _SPLITS force the
@@ -821,123 +821,6 @@ int dispatch_gemm_i8(const uint8_t *W, size_t row_bytes, const float *X, float *
     return 0;
 }
 
-// Leave to use that much LDS, asked for once a kernel.
-template <auto KERN>
-hipError_t big_lds_once(int lds) {
-    static const hipError_t rc = hipFuncSetAttribute((const void *)KERN, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    return rc;
-}
-
-// Q4_K with 128 activation rows or more on f16 and FP6 operands (kq_gemm_h6), us against the int8 GEMM's, whole calls back to back:
-// 512 x 14336 x 4096 95 / 116, 2048 x 24576 x 4096 604 / 738, 512 x 4096 x 4096 48 / 50.  166 shapes of 128 to 2048 rows against
-// 1000 to 24576 weight rows of 1024 to 16384: 0.77 to 1.08 of its time, 0.91 on average; the 18 that are more than 2 % slower, by
-// 0.5 to 2 us, are those against some 1000 weight rows and 333 to 512 rows against 4096.  Below 128 rows the int8 GEMM is as fast
-// (64 to 127 rows: 0.90 to 1.07) and keeps them: there unpacking the weights is most of the work in both.  `name` is the one that
-// callers of jq_last_kernel know the many-row product by; jq_last_arithmetic says which of the two ran.
-// Returns -1 when the shape is outside its reach and where the environment names a shape or a switch of that GEMM.  JQ_GEMM_H6 = 0
-// switches this one off, JQ_GEMM_H6_SHAPE and _SPLITS force the choice, _MIN_M moves the fewest rows.
-template <class F>
-int dispatch_gemm_h6(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n,
-                     hipStream_t s, const char *name, const char *name_split, bool swiglu_pairs = false) {
-    static const char *mode = getenv("JQ_GEMM_H6"), *i8_mode = getenv("JQ_Q4K_GEMM_I8"), *i8_shape = getenv("JQ_Q4K_GEMM_I8_SHAPE");
-    static const char *shape_env = getenv("JQ_GEMM_H6_SHAPE"), *splits_env = getenv("JQ_GEMM_H6_SPLITS");
-    static const char *min_m_env = getenv("JQ_GEMM_H6_MIN_M");
-    static const size_t min_m = min_m_env ? std::max<size_t>((size_t)atoll(min_m_env), 2) : 128;
-    if ((mode && mode[0] == '0') || i8_mode || i8_shape || m < min_m || k % 256 != 0 || k == 0 || row_bytes % 16 != 0 ||
-        !jq::h6_offsets_hold(k / 256, row_bytes) || ((uintptr_t)W & 15) != 0 || ((uintptr_t)X & 15) != 0 || m > 0x7FFFFFF0ull || n > 0x7FFFFFF0ull)
-        return -1;
-    struct Shape {
-        int nw, ng;
-    };
-    static const Shape shapes[] = {{8, 8}, {8, 7}, {8, 6}, {4, 4}};
-    const size_t nb = k / 256, groups = (m + 15) / 16;
-    const size_t scratch_cap = tl_fixed_scratch ? tl_fixed_scratch->bytes : (size_t)1 << 40;
-    // A fixed scratch that holds the int8 GEMM's records of all rows, three quarters of these in size, takes the rows in two turns;
-    // what neither GEMM's records fit fails there as it did.  (1024 x 12288: 36 MB in 32.)
-    size_t turn = m;
-    auto acts_of = [&](size_t rows) { return ((rows + 15) / 16 * nb * (size_t)jq::H6_REC + 255) & ~(size_t)255; };
-    if (acts_of(m) > scratch_cap) {
-        if (groups * nb * (size_t)jq::QI_REC > scratch_cap) return -1;
-        turn = (groups + 1) / 2 * 16;
-        if (acts_of(turn) > scratch_cap) return -1;
-    }
-    const size_t acts_bytes = acts_of(turn);
-    // tiles of a turn's rows, of the weight rows, workgroups of its launch
-    auto rows_of = [&](const Shape &sh, size_t rows) { return (rows + 32 * (size_t)sh.nw - 1) / (32 * (size_t)sh.nw); };
-    auto cols_of = [&](const Shape &sh) { return (n + 16 * (size_t)sh.ng - 1) / (16 * (size_t)sh.ng); };
-    auto grid_of = [&](const Shape &sh, size_t rows) {
-        const size_t ty = rows_of(sh, rows), tiles = ty * cols_of(sh);
-        return 8 % ty == 0 ? (tiles + 7) / 8 * 8 : tiles;
-    };
-    if (!min_m_env && rows_of(shapes[3], m) * cols_of(shapes[3]) * std::max<size_t>(1, std::min<size_t>(nb / 4, 8)) < 64) return -1;
-    auto rounds = [](double wgs, double at_once, auto us) {
-        const double whole = std::floor(wgs / at_once), rest = wgs - whole * at_once;
-        return whole * us(at_once) + (rest > 0.0 ? us(rest) : 0.0);
-    };
-    // In us, the int8 GEMM's form of estimate (dispatch_gemm_i8) fitted to 714 times of this one's shapes of seven, six and four groups in 1 to 8 parts (eight groups: 1.09 of
-    // seven's super-block, 512 to 2048 rows x 4096 to 24576): the
-    // preparation, a fixed start, the super-blocks a workgroup walks at a cost that grows with the workgroups at work, the
-    // starts of further rounds, the sum of the parts.  Over 166 shapes the picks are 0.7 % off the best measured choice on
-    // average, 5 % at the 95th percentile, 12 % at worst.
-    auto estimate = [&](const Shape &sh, size_t sp) {
-        const double wgs = (double)(grid_of(sh, m) * sp), nbl = (double)(nb / sp);
-        double us = 3.2 + 0.0048 * (double)(nb * groups);
-        if (sh.nw == 8)
-            us += 6.4 + nbl * rounds(wgs, 256.0, [](double w) { return 3.4 + 0.0035 * w; }) * (sh.ng == 8 ? 1.09 : sh.ng == 7 ? 1.0 : 0.92) +
-                  4.2 * (std::ceil(wgs / 256.0) - 1.0);
-        else
-            us += 6.6 + nbl * rounds(wgs, 512.0, [](double w) { return w <= 256.0 ? 2.24 + 0.0011 * w : 3.06 + 0.0011 * w; }) +
-                  2.5 * std::max(0.0, wgs / 512.0 - 1.5);
-        if (sp > 1) us += 0.09 * (double)sp + (double)(sp + 1) * (double)(m * n) * 4.0 / 3.4e6;
-        return us;
-    };
-    const Shape *best = nullptr;
-    size_t splits = 1;
-    double best_us = 0.0;
-    int want_nw = 0, want_ng = 0;
-    const bool forced = shape_env && sscanf(shape_env, "%d,%d", &want_nw, &want_ng) == 2;
-    for (const Shape &sh : shapes) {
-        if (forced && (sh.nw != want_nw || sh.ng != want_ng)) continue;
-        for (size_t sp = 1; sp <= 8; sp++) {
-            if (nb % sp != 0 || (sp > 1 && nb / sp < 4)) continue;
-            if (splits_env && sp != (size_t)atoi(splits_env)) continue;
-            if (sp > 1 && (m * n > 0x3FFFFFFFull || acts_bytes + (sp - 1) * turn * n * sizeof(float) > scratch_cap)) continue;
-            const double us = estimate(sh, sp);
-            if (!best || us < best_us) best = &sh, splits = sp, best_us = us;
-        }
-    }
-    if (!best) return -1;
-    if (grid_of(*best, m) > 0x7FFFFFFFull) return -1;
-    CallScratch scratch;
-    uint8_t *acts = nullptr;
-    if (scratch.get(acts_bytes + (splits - 1) * turn * n * sizeof(float), s, &acts)) return 1;
-    float *parts = (float *)(acts + acts_bytes);  // of all parts of k but the first, which is summed in place
-    auto launch = [&](auto kern, int lds, int nw, hipError_t rc) {
-        if (rc != hipSuccess) return fail("hipFuncSetAttribute: %s", hipGetErrorString(rc));
-        for (size_t m0 = 0; m0 < m; m0 += turn) {
-            const size_t rows = std::min(turn, m - m0), row_groups = (rows + 15) / 16, outs = rows * n;
-            const float *x = X + m0 * k * (swiglu_pairs ? 2 : 1);
-            float *y = Y + m0 * n;
-            const dim3 prep((unsigned)nb, (unsigned)row_groups);
-            if (swiglu_pairs) hipLaunchKernelGGL(jq::kq_gemm_h6_prep<true>, prep, dim3(128), 0, s, x, (int)rows, (int)k, acts);
-            else hipLaunchKernelGGL(jq::kq_gemm_h6_prep<false>, prep, dim3(128), 0, s, x, (int)rows, (int)k, acts);
-            hipLaunchKernelGGL(kern, dim3((unsigned)grid_of(*best, rows), (unsigned)splits), dim3(64 * nw), lds, s, W, row_bytes,
-                               (const uint8_t *)acts, y, (int)rows, (int)n, (int)(nb / splits), (int)row_groups,
-                               (int)cols_of(*best), (int)rows_of(*best, rows), (int)nb, parts);
-            if (splits > 1)
-                hipLaunchKernelGGL(jq::splitk_add, dim3((unsigned)((outs + 1023) / 1024)), dim3(256), 0, s, parts, y, outs, (int)splits - 1);
-        }
-        return 0;
-    };
-#define JQ_GEMM_H6(NW_, NG_) launch(jq::kq_gemm_h6<F, NW_, NG_>, jq::h6_lds_bytes<NG_>(), NW_, big_lds_once<&jq::kq_gemm_h6<F, NW_, NG_>>(jq::h6_lds_bytes<NG_>()))
-    const int rc = best->nw == 4 ? JQ_GEMM_H6(4, 4) : best->ng == 8 ? JQ_GEMM_H6(8, 8) : best->ng == 7 ? JQ_GEMM_H6(8, 7) : JQ_GEMM_H6(8, 6);
-#undef JQ_GEMM_H6
-    if (rc) return rc;
-    note_kernel(splits > 1 ? name_split : name, "f16+fp6");
-    HIP_TRY(hipGetLastError());
-    return 0;
-}
-
 // Q4_K with more than 16 activation rows: prepare the fixed-point activation planes in the
 // call scratch of the stream, then the MFMA GEMM, split over k when its tiles alone would leave
 // compute units idle.
@@ -1032,9 +915,9 @@ int dispatch_gemm_decoded(uint32_t type, const uint8_t *W, size_t row_bytes, con
 //
 // 17 rows and more: where its estimate is below that of what would run else, fitted to 24 shapes of 17 to 256 rows: the int8 GEMM, with at
 // most 127 rows 14.6 us and 0.62 a million weights (23 to 52 us at 4096 x 4096 to 14336 x 4096) or 0.5 a super-block of k, a third
-// more beyond; Q4_K a tenth less; rows of 4096 also dispatch_q4k_rows16's passes.  us, before / now: 32 rows x 14336 x 4096 Q4_K 27 / 19,
+// more beyond (MXFP4, gemm_h6's there: a tenth); Q4_K a tenth less; rows of 4096 also dispatch_q4k_rows16's passes.  us, before / now: 32 rows x 14336 x 4096 Q4_K 27 / 19,
 // Q6_K 43 / 26, MXFP4 42 / 17; 64 rows x 3000 x 2560 22 to 25 / 11 to 12; 96 rows x 4096 x 4096 24 to 26 / 17 to 19;
-// 64 rows x 9000 x 9984 Q6_K 71 / 71, 127 rows 79 / 109 (hence the margin).  From 128 rows Q4_K is dispatch_gemm_h6's, and prepared
+// 64 rows x 9000 x 9984 Q6_K 71 / 71, 127 rows 79 / 109 (hence the margin).  From 128 rows Q4_K is gemm_h6's, and prepared
 // activations that the second level cache of an XCD does not hold are slow (200 rows x 1100 x 12288 41 / 55).
 bool few_rows_better(uint32_t type, size_t m, size_t k, size_t n) {
     static const char *off = getenv("JQ_FEW_ROWS"), *i8_shape = getenv("JQ_Q4K_GEMM_I8_SHAPE"), *i8_min_m = getenv("JQ_Q4K_GEMM_I8_MIN_M");
@@ -1044,7 +927,7 @@ bool few_rows_better(uint32_t type, size_t m, size_t k, size_t n) {
         if ((!q4 && type != JQ_TYPE_Q6_K && type != JQ_TYPE_Q8_0 && type != JQ_TYPE_MXFP4) || i8_shape || i8_min_m || n < 512 || k < 1024 ||
             n * k < ((size_t)2 << 20) || m > (q4 ? 127 : 255) || (m > 127 && m * k > 1500000))
             return false;
-        double us = std::max(14.6 + 0.62e-6 * (double)(n * k), 9.0 + 0.5 * (double)(k / 256)) * (m > 127 ? 1.3 : 1.0) * (q4 ? 0.9 : 1.0);
+        double us = std::max(14.6 + 0.62e-6 * (double)(n * k), 9.0 + 0.5 * (double)(k / 256)) * (m > 127 ? type == JQ_TYPE_MXFP4 ? 1.1 : 1.3 : 1.0) * (q4 ? 0.9 : 1.0);
         if (q4 && k == 4096) us = std::min(us, 3.0 + (double)((m + 15) / 16) * (4.3 + 0.527 * (double)n / 1024.0));
         return few_rows_many_us(type, m, k, n) < 0.92 * us;
     }
@@ -1145,7 +1028,7 @@ int dispatch_matmul(uint32_t type, const uint8_t *W, size_t row_bytes, const flo
         return dispatch_q4k_gemm(W, row_bytes, X, Y, m, k, n, s);
     if (type == JQ_TYPE_Q4_K && q4k_mfma_applies(m, k, n)) return dispatch_q4k_mfma(W, row_bytes, X, Y, m, k, n, s);
     if (type == JQ_TYPE_Q4_K && m > Q4K_MFMA_MAX_M) {
-        int rc = dispatch_gemm_h6<jq::H6Q4K>(W, row_bytes, X, Y, m, k, n, s, "q4k_gemm_i8", "q4k_gemm_i8+splitk");
+        int rc = gemm_h6(type, W, row_bytes, X, Y, m, k, n, s, "q4k_gemm_i8", "q4k_gemm_i8+splitk");
         if (rc < 0) rc = dispatch_gemm_i8<jq::QiQ4K>(W, row_bytes, X, Y, m, k, n, s, "q4k_gemm_i8", "q4k_gemm_i8+splitk");
         if (rc >= 0) return rc;
     }
@@ -1198,7 +1081,8 @@ int dispatch_matmul(uint32_t type, const uint8_t *W, size_t row_bytes, const flo
         if (rc >= 0) return rc;
     }
     if (type == JQ_TYPE_MXFP4 && many_rows) {
-        const int rc = dispatch_gemm_i8<jq::QiMXFP4>(W, row_bytes, X, Y, m, k, n, s, "mxfp4_gemm_i8", "mxfp4_gemm_i8+splitk", false, 2);
+        int rc = gemm_h6(type, W, row_bytes, X, Y, m, k, n, s, "mxfp4_gemm_i8", "mxfp4_gemm_i8+splitk");
+        if (rc < 0) rc = dispatch_gemm_i8<jq::QiMXFP4>(W, row_bytes, X, Y, m, k, n, s, "mxfp4_gemm_i8", "mxfp4_gemm_i8+splitk", false, 2);
         if (rc >= 0) return rc;
     }
     if (type == JQ_TYPE_Q4_K && m > Q4K_MFMA_MAX_M && row_bytes % 16 == 0 && ((uintptr_t)W & 15) == 0 &&
@@ -3300,8 +3184,7 @@ int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *w
                 const jq_weight *wd = dn->second;
                 int rc = -1;
                 if (wd->type == JQ_TYPE_Q4_K)
-                    rc = dispatch_gemm_h6<jq::H6Q4K>(wd->dev, wd->row_bytes, m->g, m->proj, T, wd->k, wd->n, s, "q4k_gemm_i8",
-                                                     "q4k_gemm_i8+splitk", true);
+                    rc = gemm_h6(wd->type, wd->dev, wd->row_bytes, m->g, m->proj, T, wd->k, wd->n, s, "q4k_gemm_i8", "q4k_gemm_i8+splitk", true);
                 if (rc < 0 && wd->type == JQ_TYPE_Q4_K)
                     rc = dispatch_gemm_i8<jq::QiQ4K>(wd->dev, wd->row_bytes, m->g, m->proj, T, wd->k, wd->n, s, "q4k_gemm_i8",
                                                      "q4k_gemm_i8+splitk", true);

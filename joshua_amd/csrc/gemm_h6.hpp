@@ -1,0 +1,12 @@
+// Products of many activation rows on f16 and FP6 matrix instructions (kernels_mfma_gemm_h6.hpp).
+#pragma once
+#include "core.hpp"
+
+namespace jqh {
+
+// Device pointers, shapes validated, k and n > 0.  With `swiglu_pairs` the activations are silu(gate) * up over rows of 2 k floats in which
+// gate_j and up_j alternate.  -1: the call is outside its reach.
+int gemm_h6(uint32_t type, const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n, hipStream_t s,
+            const char *name, const char *name_split, bool swiglu_pairs = false);
+
+}  // namespace jqh

@@ -1,4 +1,4 @@
-// Q4_K matmul for many activation rows on f16 and FP6 matrix instructions.
+// Q4_K and MXFP4 matmul for many activation rows on f16 and FP6 matrix instructions.
 //
 // Per 256-element super-block of weight row n and activation row m (reference arithmetic w = d sc q - dmin m,
 // src/kquant_dot.rs:440-465), with the codes taken about their middle,
@@ -39,8 +39,13 @@
 // operands for 60 400 (counters): neither is full, and two waves a SIMD have a barrier every half super-block.  Waves of 64
 // activation rows (four a workgroup, half the LDS reads) take 131 us: one wave a SIMD has nothing to hide its vector instructions
 // behind.  E2M1 codes of p, a third less to read, would be 2.6e-5 off 64 bits.  The codes' scales cost 1.3 us of a call.
+// MXFP4 has no mins and no codes to make: behind the super-block's largest scale a weight is exact in f16, made by one conversion for
+// two, and E2M1, what the second instruction multiplies, is its code as it stands in memory, on the block's own scale.  512 x 14336 x
+// 4096: 112 -> 87 us a call, 333 x 4096 x 12288 109 -> 79, 2048 x 4096 x 12288 427 -> 277; 2.7e-5 -> 0.6e-5 off 64 bits.  Q6_K and Q8_0, whose
+// weights take 12 and 18 bits, were built here too, the weights' own remainders as E2M1 against the activations as E2M3: no faster
+// than the int8 GEMM (512 x 14336 x 4096 148 and 143 us against 128 and 130; unpacking twice Q4_K's instructions, and registers for six groups).
 #pragma once
-#include "kernels_dot4_q4k.hpp"
+#include "kernels_graph.hpp"
 
 #include <utility>
 
@@ -66,7 +71,10 @@ typedef float h6_f4 __attribute__((ext_vector_type(4)));
 //   2 halves x (64 lanes x 16 bytes, then 64 lanes x 8): the 32 remainders x' - f16(x') as E2M3 in the same order
 //   64 lanes x 16 bytes: the operand of the min term
 //   the 16 scales
+// (MXFP4: no operand of a min term)
 constexpr int H6_HI = 8192, H6_LO_HALF = 1536, H6_MIN = H6_HI + 2 * H6_LO_HALF, H6_SCALE = H6_MIN + 1024, H6_REC = H6_SCALE + 64;
+template <bool MINS>
+constexpr int h6_rec() { return MINS ? H6_REC : H6_MIN + 64; }
 
 // Whether the kernel's offsets hold rows of that many super-blocks: a record's from the start of its row group in 31 bits, a weight
 // block's from the first of 16 rows in 32.
@@ -84,12 +92,13 @@ __device__ __forceinline__ float h6_bf16_value(uint32_t b) { return __builtin_bi
 // caches hold the rest of the line (8.0 us at 512 x 14336, either way), but the pairs' 256 bytes a lane do not survive there: 2048 x
 // 12288 pairs took 86 us so and take 50 with whole rows of memory turned by the LDS, of 54 that 276 MB take in a large copy.  For
 // plain rows the detour costs 1 us.  rows_sh's padding: 16 lanes that read 16 rows at one column take 16 different groups of banks.
-template <bool PAIRS>
-__global__ __launch_bounds__(128) void kq_gemm_h6_prep(const float *__restrict__ X, int m_rows, int k, uint8_t *__restrict__ out) {
+// NIBBLES: positions 2 j and 2 j + 1 of a sub-block hold elements j and j + 16 (MXFP4's bytes), else H6_ORDER's.
+template <bool PAIRS, bool MINS, bool NIBBLES>
+static __global__ __launch_bounds__(128) void kq_gemm_h6_prep(const float *__restrict__ X, int m_rows, int k, uint8_t *__restrict__ out) {
     __shared__ float amax_sh[2][16], xs_sh[16][8];
     const int tid = threadIdx.x, lane = tid & 63, h = tid >> 6, i = lane & 15, g = lane >> 4;
     const int b = blockIdx.x, row = 16 * (int)blockIdx.y + i;
-    uint8_t *rec = out + ((size_t)blockIdx.y * gridDim.x + b) * H6_REC;
+    uint8_t *rec = out + ((size_t)blockIdx.y * gridDim.x + b) * h6_rec<MINS>();
     float v[32];
     if constexpr (PAIRS) {
         __shared__ __align__(16) float rows_sh[16][260];
@@ -139,17 +148,19 @@ __global__ __launch_bounds__(128) void kq_gemm_h6_prep(const float *__restrict__
     for (int q = 0; q < 32; q++) {
         // position 8 s + p holds element 8 s + {0, 2, 1, 3, 4, 6, 5, 7}[p]: the order in which two of a word's nibbles
         // fall into one register (H6Q4K::piece)
-        const int at = (q & ~3) | ((q & 1) << 1) | ((q >> 1) & 1);
+        const int at = NIBBLES ? (q >> 1) + 16 * (q & 1) : (q & ~3) | ((q & 1) << 1) | ((q >> 1) & 1);
         const float x = live ? v[at] * inv : 0.0f;
         hi[q] = (_Float16)x;
         const float r = x - (float)hi[q];
         lo[q] = (_Float16)fminf(fmaxf(r, -7.5f), 7.5f);
     }
-    if (live) {
+    if constexpr (MINS) {
+        if (live) {
 #pragma unroll
-        for (int q = 0; q < 32; q++) sum += v[q] * 0.03125f;
+            for (int q = 0; q < 32; q++) sum += v[q] * 0.03125f;
+        }
+        xs_sh[i][4 * h + g] = sum;
     }
-    xs_sh[i][4 * h + g] = sum;
 #pragma unroll
     for (int st = 0; st < 4; st++) {
         h6_h8 p;
@@ -160,8 +171,8 @@ __global__ __launch_bounds__(128) void kq_gemm_h6_prep(const float *__restrict__
     const h6_u6 six = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(lo, 1.0f);
     *(h6_u4 *)(rec + H6_HI + h * H6_LO_HALF + lane * 16) = h6_u4{six[0], six[1], six[2], six[3]};
     *(h6_u2 *)(rec + H6_HI + h * H6_LO_HALF + 1024 + lane * 8) = h6_u2{six[4], six[5]};
-    __syncthreads();
-    if (h == 0) {  // lane groups 0 and 2: bf16 of the eight means, 1 and 3: what is left of them
+    if constexpr (MINS) __syncthreads();
+    if (MINS && h == 0) {  // lane groups 0 and 2: bf16 of the eight means, 1 and 3: what is left of them
         uint32_t w[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -177,13 +188,14 @@ __global__ __launch_bounds__(128) void kq_gemm_h6_prep(const float *__restrict__
         }
         *(h6_u4 *)(rec + H6_MIN + lane * 16) = h6_u4{w[0], w[1], w[2], w[3]};
     }
-    if (tid < 16) ((float *)(rec + H6_SCALE))[tid] = s;
+    if (tid < 16) ((float *)(rec + h6_rec<MINS>() - 64))[tid] = s;
 }
 
 // LDS: for either half of a super-block and every 16 weight rows 4 steps x 64 lanes x 16 bytes of f16 operands, then
 // their E2M3 codes (64 lanes x 16 bytes and x 8); behind the halves, twice (by the super-block's parity), for every 16 rows
 // the min operand's two parts (16 rows x 16 bytes each) and the 16 factors d; behind those, for either half, the exponents of
 // the codes' scales, 64 lanes x 8 groups of 16 rows: one read gives a lane those of all groups.
+// (MXFP4's codes: E2M1, 64 lanes x 16 bytes, no min operand.)
 constexpr int H6_T_LO = 4096, H6_HALF = H6_T_LO + 1536, H6_META = 512 + 64, H6_EXPS = 512;
 template <int NG>
 constexpr int h6_lds_bytes() { return 2 * NG * (H6_HALF + H6_META) + 2 * H6_EXPS; }
@@ -200,12 +212,16 @@ struct H6Memory {
     __device__ __forceinline__ h6_u2 load8(uint32_t scalar, uint32_t lane) const {
         return __builtin_amdgcn_raw_buffer_load_b64(at, (int)lane, (int)scalar, 0);
     }
+    __device__ __forceinline__ uint32_t load4(uint32_t scalar, uint32_t lane) const {
+        return __builtin_amdgcn_raw_buffer_load_b32(at, (int)lane, (int)scalar, 0);
+    }
 };
 
 // A format's side.  Lane (row i = lane % 16, g = lane / 16) of the wave that unpacks 16 weight rows takes the 32 elements of
 // sub-block 4 h + g of its row for half h.
 struct H6Q4K {  // w = d sc (q - 8) + (8 d sc - dmin m), 6-bit sc and m, q in 0..15
-    static constexpr int BLOCK = 144;
+    static constexpr int BLOCK = 144, ALIGN = 16, LOW = 2;  // LOW: the codes' format, 2: E2M3, 4: E2M1
+    static constexpr bool MINS = true, NIBBLES = false;
     static constexpr float D_UNIT = 128.0f;  // the operand is p / 2^7, p = sc (q - 8)
     struct Raw {
         h6_u4 hdr, q0, q1;
@@ -213,7 +229,7 @@ struct H6Q4K {  // w = d sc (q - 8) + (8 d sc - dmin m), 6-bit sc and m, q in 0.
         float unit;     // the codes' scale, a power of two: sc / 32 with its mantissa cleared
         h6_h32 p;
     };
-    __device__ __forceinline__ static void fetch_header(const H6Memory &mem, uint32_t blk, uint32_t row_at, Raw &raw) {
+    __device__ __forceinline__ static void fetch_header(const H6Memory &mem, uint32_t blk, uint32_t row_at, int, int, Raw &raw) {
         raw.hdr = mem.load16(blk, row_at);
     }
     __device__ __forceinline__ static void fetch(const H6Memory &mem, uint32_t blk, uint32_t row_at, int g, int h, Raw &raw) {
@@ -259,16 +275,60 @@ struct H6Q4K {  // w = d sc (q - 8) + (8 d sc - dmin m), 6-bit sc and m, q in 0.
     }
 };
 
+// Blocks of 17 bytes start anywhere: what a lane needs comes in whole words that hold a byte of it, and is shifted.
+struct H6MXFP4 {  // w = 2^(e - 127) E2M1: exact as f16 against the super-block's largest scale, and the codes are E2M1 themselves
+    static constexpr int BLOCK = 136, ALIGN = 4, LOW = 4;
+    static constexpr bool MINS = false, NIBBLES = true;
+    struct Raw {
+        h6_u4 q0;
+        uint32_t q1, e0, e1, at, at_e;
+        float scale;
+        h6_u4 word;
+        h6_h32 p;
+    };
+    __device__ __forceinline__ static void fetch_header(const H6Memory &mem, uint32_t blk, uint32_t row_at, int g, int, Raw &raw) {
+        const uint32_t o = row_at + blk + 17 * (uint32_t)g;
+        raw.e0 = mem.load4(0, o & ~3u), raw.e1 = mem.load4(68, o & ~3u), raw.at_e = o & 3u;
+    }
+    __device__ __forceinline__ static void fetch(const H6Memory &mem, uint32_t blk, uint32_t row_at, int g, int h, Raw &raw) {
+        const uint32_t o = row_at + blk + 17 * (uint32_t)g + 1, a = o & ~3u;
+        raw.at = o & 3u;
+        raw.q0 = mem.load16(68 * h, a), raw.q1 = mem.load4(68 * h + 12, raw.at ? a + 4 : a);  // (the fifth word where it is needed)
+    }
+    __device__ __forceinline__ static void header(Raw &raw, int, int i, int h, uint8_t *meta, uint8_t *exponent) {
+        const uint32_t e0 = (raw.e0 >> (8 * raw.at_e)) & 0xFFu, e1 = (raw.e1 >> (8 * raw.at_e)) & 0xFFu, e = h == 0 ? e0 : e1;
+        const int most = (int)max_xor32(max_xor16(fmaxf(e0 == 0xFFu ? 0.0f : (float)e0, e1 == 0xFFu ? 0.0f : (float)e1)));
+        const bool none = e == 0xFFu || (int)e < most - 60;  // 0xFF: a block of zeros
+        const uint32_t by = none ? 0u : (uint32_t)(140 + (int)e - most);  // the largest scale takes codes to 6 x 2^13
+        raw.scale = __builtin_bit_cast(float, by << 23), *exponent = (uint8_t)by;
+        const uint32_t w[5] = {raw.q0.x, raw.q0.y, raw.q0.z, raw.q0.w, raw.q1};
+#pragma unroll
+        for (int j = 0; j < 4; j++) raw.word[j] = none ? 0u : __builtin_amdgcn_alignbyte(w[j + 1], w[j], raw.at);
+        if (h == 0) *(float *)(meta + 512 + 4 * i) = ldexpf(1.0f, most - 140);
+    }
+    template <int U>
+    __device__ __forceinline__ static void pair(Raw &raw, int, int lane, uint8_t *tile) {
+        const h6_h2 v = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(raw.word[U / 4], raw.scale, U % 4);
+        raw.p[2 * U] = v[0], raw.p[2 * U + 1] = v[1];
+        if constexpr (U % 4 == 3) {
+            constexpr int st = U / 4;
+            *(h6_h8 *)(tile + (st * 64 + lane) * 16) = h6_h8{raw.p[8 * st], raw.p[8 * st + 1], raw.p[8 * st + 2], raw.p[8 * st + 3],
+                                                             raw.p[8 * st + 4], raw.p[8 * st + 5], raw.p[8 * st + 6], raw.p[8 * st + 7]};
+        }
+    }
+    __device__ __forceinline__ static void codes(Raw &raw, int lane, uint8_t *tile) { *(h6_u4 *)(tile + H6_T_LO + lane * 16) = raw.word; }
+};
+
 __device__ __forceinline__ h6_i8 h6_operand6(h6_u6 v) {
     return h6_i8{(int)v[0], (int)v[1], (int)v[2], (int)v[3], (int)v[4], (int)v[5], 0, 0};
 }
 
 template <class F, int NW, int NG>
-__global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict__ W, size_t row_bytes,
+static __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict__ W, size_t row_bytes,
                                                       const uint8_t *__restrict__ acts, float *__restrict__ Y, int m_rows, int n,
                                                       int nb, int groups, int tx, int ty, int nb_total, float *__restrict__ parts) {
     static_assert(NG <= NW && NG <= 8, "one group of 16 weight rows a wave unpacks, a byte each of a lane's eight exponents");
-    constexpr int NT = 16 * NG, MT = 32 * NW;
+    constexpr int NT = 16 * NG, MT = 32 * NW, REC = h6_rec<F::MINS>();
     extern __shared__ __attribute__((aligned(16))) uint8_t h6_lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
     int bx, by;
@@ -285,11 +345,12 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
     // everything is read behind an address that is the same in all lanes of a wave
     const int wv = __builtin_amdgcn_readfirstlane(wave), wu = min(wv, NG - 1);  // (waves past the last group unpack it too)
     auto record_of = [&](int mg) __attribute__((always_inline)) {
-        return acts + ((size_t)min(m0 / 16 + 2 * wv + mg, groups - 1) * nb_total + b_first) * H6_REC;
+        return acts + ((size_t)min(m0 / 16 + 2 * wv + mg, groups - 1) * nb_total + b_first) * REC;
     };
     const H6Memory arec[2] = {H6Memory(record_of(0)), H6Memory(record_of(1))};
     const int first_row = min(n0 + 16 * wu, n - 1);
-    const H6Memory wsrc(W + (size_t)first_row * row_bytes + (size_t)b_first * F::BLOCK);
+    const uint8_t *const wfirst = W + (size_t)first_row * row_bytes + (size_t)b_first * F::BLOCK;
+    const H6Memory wsrc(wfirst);
     const uint32_t wlane = (uint32_t)min(r, n - 1 - first_row) * (uint32_t)row_bytes;
     uint8_t *const own = h6_lds + wu * H6_HALF, *const meta_lds = h6_lds + 2 * NG * H6_HALF;
     uint8_t *const exps = meta_lds + 2 * NG * H6_META + lane * 8;
@@ -300,22 +361,22 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
     h6_b8 minA[2];
     h6_f4 sx[2];
     auto load_hi = [&](int mg, int b, int st) __attribute__((always_inline)) {
-        A[mg][st & 3] = __builtin_bit_cast(h6_h8, arec[mg].load16(b * H6_REC + st * 1024, l16));
+        A[mg][st & 3] = __builtin_bit_cast(h6_h8, arec[mg].load16(b * REC + st * 1024, l16));
     };
     auto load_lo = [&](int mg, int b, int h) __attribute__((always_inline)) {
-        const uint32_t at = b * H6_REC + H6_HI + h * H6_LO_HALF;
+        const uint32_t at = b * REC + H6_HI + h * H6_LO_HALF;
         const h6_u4 x = arec[mg].load16(at, l16);
         const h6_u2 y = arec[mg].load8(at + 1024, l16 >> 1);
         L[mg] = h6_u6{x[0], x[1], x[2], x[3], y[0], y[1]};
     };
     auto load_min = [&](int mg, int b) __attribute__((always_inline)) {
-        minA[mg] = __builtin_bit_cast(h6_b8, arec[mg].load16(b * H6_REC + H6_MIN, l16));
+        minA[mg] = __builtin_bit_cast(h6_b8, arec[mg].load16(b * REC + H6_MIN, l16));
     };
     auto load_scale = [&](int mg, int b) __attribute__((always_inline)) {
-        sx[mg] = __builtin_bit_cast(h6_f4, arec[mg].load16(b * H6_REC + H6_SCALE, 16u * (uint32_t)g));
+        sx[mg] = __builtin_bit_cast(h6_f4, arec[mg].load16(b * REC + REC - 64, 16u * (uint32_t)g));
     };
     typename F::Raw raw;
-    F::fetch_header(wsrc, 0, wlane, raw);
+    F::fetch_header(wsrc, 0, wlane, g, 0, raw);
     F::fetch(wsrc, 0, wlane, g, 0, raw);
 #pragma unroll
     for (int mg = 0; mg < 2; mg++) {
@@ -336,22 +397,23 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
     __syncthreads();
 
     // The steps of a half: (group of weight rows, kind), kind 0..3: an f16 step of 32 k, 4: the half's remainders, 5: the
-    // min term.  The second half takes its last three kinds group by group, so that the groups' sums are complete one
-    // after the other and their scaling spreads among the matrix instructions that follow.
+    // min term.  The second half takes its last three kinds group by group, so that the
+    // groups' sums are complete one after the other and their scaling spreads among the matrix instructions that follow.
     struct Step {
         int cg, kind;
     };
+    constexpr int LEAD = F::MINS ? 3 : 2;  // kinds in front of those three
     constexpr auto step_of = [](int h, int t) constexpr {
         if (h == 0) return Step{t % NG, t / NG};
-        if (t < 3 * NG) return Step{t % NG, t < NG ? 5 : t / NG - 1};
-        return Step{(t - 3 * NG) / 3, 2 + (t - 3 * NG) % 3};
+        if (t < LEAD * NG) return Step{t % NG, LEAD == 2 ? t / NG : t < NG ? 5 : t / NG - 1};
+        return Step{(t - LEAD * NG) / 3, 2 + (t - LEAD * NG) % 3};
     };
     constexpr int AHEAD = NG == 8 ? 2 : 4;  // operand reads; with eight groups the registers are just enough for two (no difference in time)
     for (int b = 0; b < nb; b++) {
         const int b1 = min(b + 1, nb - 1);
         const uint8_t *meta = meta_lds + (b & 1) * (NG * H6_META);
         h6_each(std::make_integer_sequence<int, 2>{}, [&](auto hc) __attribute__((always_inline)) {
-            constexpr int h = decltype(hc)::value, STEPS = (h == 0 ? 5 : 6) * NG;
+            constexpr int h = decltype(hc)::value, STEPS = (h == 0 ? 5 : LEAD + 3) * NG;
             static_assert(STEPS >= 20, "a step for every pair of elements to be unpacked");
             const uint8_t *buf = h6_lds + h * (NG * H6_HALF);
             // the half that is unpacked meanwhile: the second of this super-block, then the first of the next
@@ -368,11 +430,12 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
             auto operand_tail = [&](auto tc) __attribute__((always_inline)) {
                 return *(const h6_u2 *)(buf + step_of(h, decltype(tc)::value).cg * H6_HALF + H6_T_LO + 1024 + lane * 8);
             };
+            constexpr auto has_tail = [](Step st) constexpr { return F::LOW == 2 && st.kind == 4; };
             h6_u4 B[AHEAD];
             h6_u2 B2[AHEAD];
             h6_each(std::make_integer_sequence<int, AHEAD>{}, [&](auto tc) __attribute__((always_inline)) {
                 B[decltype(tc)::value] = operand(tc);
-                if constexpr (step_of(h, decltype(tc)::value).kind == 4) B2[decltype(tc)::value] = operand_tail(tc);
+                if constexpr (has_tail(step_of(h, decltype(tc)::value))) B2[decltype(tc)::value] = operand_tail(tc);
             });
             float d[2];
             auto finish = [&](int cg, int o) __attribute__((always_inline)) {  // one of the eight results a lane holds of group cg
@@ -386,27 +449,30 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
                 const h6_u2 w2 = B2[t % AHEAD];
                 if constexpr (t + AHEAD < STEPS) {
                     B[t % AHEAD] = operand(std::integral_constant<int, t + AHEAD>{});
-                    if constexpr (step_of(h, t + AHEAD).kind == 4) B2[t % AHEAD] = operand_tail(std::integral_constant<int, t + AHEAD>{});
+                    if constexpr (has_tail(step_of(h, t + AHEAD))) B2[t % AHEAD] = operand_tail(std::integral_constant<int, t + AHEAD>{});
                 }
                 if constexpr (h == 1 && st.kind == 2) d[st.cg & 1] = *(const float *)(meta + st.cg * H6_META + 512 + 4 * r);
                 // the next half's weights become operands among the matrix instructions; then the half after that is asked for
                 if constexpr (t == 1) F::header(raw, g, r, h ^ 1, next_meta, exps + (h ^ 1) * H6_EXPS + wu);
                 if constexpr (t >= 2 && t < 18) F::template pair<t - 2>(raw, g, lane, next);
                 if constexpr (t == 18) F::codes(raw, lane, next);
-                if constexpr (t == 19) F::fetch(wsrc, src_next, wlane, g, h, raw), F::fetch_header(wsrc, src_next, wlane, raw);
+                if constexpr (t == 19) F::fetch(wsrc, src_next, wlane, g, h, raw), F::fetch_header(wsrc, src_next, wlane, g, h, raw);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int mg = 0; mg < 2; mg++) {
                     if constexpr (st.kind == 5)
                         acc[mg][st.cg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(minA[mg], __builtin_bit_cast(h6_b8, w), acc[mg][st.cg], 0, 0, 0);
-                    else if constexpr (st.kind == 4)
-                        sb[mg][st.cg] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                            h6_operand6(L[mg]), h6_operand6(h6_u6{w[0], w[1], w[2], w[3], w2[0], w2[1]}), sb[mg][st.cg], 2, 2, 0, 0x7F7F7F7F, st.cg & 3, (int)units[st.cg >> 2]);
+                    else if constexpr (st.kind == 4) {
+                        const h6_i8 low = F::LOW == 2 ? h6_operand6(h6_u6{w[0], w[1], w[2], w[3], w2[0], w2[1]})
+                                                      : h6_i8{(int)w[0], (int)w[1], (int)w[2], (int)w[3], 0, 0, 0, 0};
+                        sb[mg][st.cg] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(h6_operand6(L[mg]), low, sb[mg][st.cg], 2, F::LOW, 0, 0x7F7F7F7F,
+                                                                                          st.cg & 3, (int)units[st.cg >> 2]);
+                    }
                     else
                         sb[mg][st.cg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[mg][st.kind], __builtin_bit_cast(h6_h8, w),
                                                                                h == 0 && st.kind == 0 ? zero : sb[mg][st.cg], 0, 0, 0);
                 }
-                if constexpr (h == 1 && t >= 3 * NG && st.cg > 0) {  // behind the matrix instructions of the group before
+                if constexpr (h == 1 && t >= LEAD * NG && st.cg > 0) {  // behind the matrix instructions of the group before
                     constexpr int o = 3 * (st.kind - 2);
                     finish(st.cg - 1, o), finish(st.cg - 1, o + 1);
                     if constexpr (o < 6) finish(st.cg - 1, o + 2);
@@ -417,7 +483,8 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
                         if constexpr (st.kind == 5) load_scale(mg, b);
                         else if constexpr (st.kind == 4) load_lo(mg, h == 0 ? b : b1, h ^ 1);
                         else load_hi(mg, h == 0 ? b : b1, 4 * (h ^ 1) + st.kind);
-                        if constexpr (h == 0 && st.kind == 1) load_min(mg, b);
+                        if constexpr (F::MINS && h == 0 && st.kind == 1) load_min(mg, b);
+                        if constexpr (!F::MINS && h == 1 && st.kind == 0) load_scale(mg, b);
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -444,7 +511,7 @@ __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict_
 }
 
 // Y[i] += P[0][i], then P[1][i], .. P[parts - 1][i], four elements a thread.
-__global__ __launch_bounds__(256) void splitk_add(const float *__restrict__ P, float *__restrict__ Y, size_t count, int parts) {
+static __global__ __launch_bounds__(256) void splitk_add(const float *__restrict__ P, float *__restrict__ Y, size_t count, int parts) {
     const size_t i = 4 * ((size_t)blockIdx.x * 256 + threadIdx.x);
     if (i >= count) return;
     if ((count & 3) == 0) {

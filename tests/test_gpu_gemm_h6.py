@@ -212,3 +212,58 @@ def test_capture_on_a_stream_that_never_ran_a_product_of_that_size():
     del graph
     torch.cuda.synchronize()
     capi.stream_release(stream.cuda_stream)
+
+
+MX_CHILD = r"""
+import os, sys
+import numpy as np
+sys.path.insert(0, ROOT)
+import oracle
+from joshua_amd import capi, synth
+splits = int(os.environ["JQ_GEMM_H6_SPLITS"])
+
+
+def check(blocks, lhs, what, rms=None):
+    # the weights are exact, E2M1 in both instructions; a remainder, at most 8 s for s = 2^-14 of its super-block's largest magnitude, is
+    # at most s / 2 off as E2M3; f32 sums: 2^-20 of the terms
+    m, k = lhs.shape
+    n = blocks.size // (k // 32 * 17)
+    got = capi.Weight.upload(capi.MXFP4, blocks, n, k).matmul_t(m, lhs)
+    assert capi.last_kernel() == "mxfp4_gemm_i8" + ("+splitk" if splits > 1 else "") and capi.last_arithmetic() == "f16+fp6"
+    w, x = oracle.dequantize(capi.MXFP4, blocks).reshape(n, k).astype(np.float64), lhs.astype(np.float64)
+    want = x @ w.T
+    s = np.abs(x.reshape(m, -1, 256)).max(2) * 2.0 ** -14
+    bound = 0.5 * s @ np.abs(w).reshape(n, -1, 256).sum(2).T + 2.0 ** -20 * (np.abs(x) @ np.abs(w).T)
+    err = np.abs(got - want)
+    assert np.all(err <= bound), (what, float((err / np.maximum(bound, 1e-300)).max()))
+    if rms:
+        assert np.sqrt((err ** 2).mean() / (want ** 2).mean()) <= rms, what
+    return got
+
+
+sizes = [(17, 256, 64), (33, 512, 113), (64, 1024, 97), (129, 768, 112), (257, 512, 300), (256, 1024, 96)] if splits == 1 else [(40, 4096, 100), (300, 4096, 130)]
+for m, k, n in sizes:
+    check(synth.normal_quantized(capi.MXFP4, 5 + n, n * k, 0.02), synth.normal(6 + k, (m, k)), (m, k, n), 1.2e-5)
+rng = np.random.default_rng(4)
+n, k = 80, 2304 if splits == 1 else 4096
+raw = rng.integers(0, 256, (n * k // 32, 17), dtype=np.uint8)
+raw[:, 0] = rng.integers(105, 145, len(raw))
+raw[::13, 0], raw[::17, 0], raw[:8, 0] = 0xFF, 0, 0xFF
+lhs = synth.normal(9, (50, k))
+lhs[0] *= (10.0 ** rng.integers(-6, 7, size=k // 16)).repeat(16).astype(np.float32)
+lhs[1] = 0
+lhs[1, 1234] = 3.5
+lhs[3] *= np.float32(1e25)
+got = check(raw.reshape(-1), lhs, "every scale")
+lhs[7, 100], lhs[8, 2000] = np.inf, np.nan
+other = capi.Weight.upload(capi.MXFP4, raw.reshape(-1), n, k).matmul_t(50, lhs)
+assert np.all(np.isnan(other[7:9])) and np.array_equal(np.delete(other, [7, 8], 0), np.delete(got, [7, 8], 0))
+print("h6 ok")
+"""
+
+
+@pytest.mark.parametrize("shape,splits", [("8,8", 1), ("8,7", 1), ("8,6", 1), ("4,4", 1), ("8,8", 4), ("4,4", 2)])
+def test_mxfp4_on_f16_and_its_own_codes(shape, splits):
+    env = dict(os.environ, JQ_GEMM_H6_SHAPE=shape, JQ_GEMM_H6_SPLITS=str(splits), JQ_GEMM_H6_MIN_M="17")
+    res = subprocess.run([sys.executable, "-c", MX_CHILD.replace("ROOT", repr(ROOT), 1)], env=env, capture_output=True, text=True, timeout=110)
+    assert res.returncode == 0 and "h6 ok" in res.stdout, res.stdout + res.stderr
