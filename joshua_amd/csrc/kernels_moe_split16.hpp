@@ -6,9 +6,9 @@
 //     I1 = sum p (hi + lo)     two v_mfma_f32_16x16x32_f16 a sub-block, products exact, f32 sums
 //     I2 = sum_j m_j XS_j      one more a super-block (XS_j: the sub-block's sum / 32, again hi + lo; the mins exact)
 //     y += s (d I1 - 32 dmin I2)
-// The packed nibbles go from memory to registers and become the second operand there: (w & 0xF) | 0x6400 is 1024 + q as f16, one
+// The packed nibbles become the second operand in registers: (w & 0xF) | 0x6400 is 1024 + q as f16, one
 // v_pk_fma_f16 with sc and -1024 sc makes two products (the high nibbles: 0x5400, 64 + q): 1.1 vector instructions a
-// weight, no LDS, and the unpacking of 64 rows serves every activation row of the tile.  (The int8 GEMM's two byte
+// weight, and the unpacking of 64 rows serves every activation row of the tile.  (The int8 GEMM's two byte
 // planes of the same product cost four instructions a weight and pass through LDS, and its sums seven an output.)
 //
 // Element order.  Lane (n = lane % 16, g = lane / 16) holds weight row n and, of half a super-block (four sub-blocks, 64
@@ -24,6 +24,7 @@ namespace jq {
 constexpr int MS16_PLANES = 1024, MS16_XS = 32;  // bytes a row and super-block: hi and lo of 256 elements; of 8 sums
 constexpr int MS16_RG = 3;                        // row groups of 16 a tile holds at most
 constexpr int MS16_ROWS = 16 * MS16_RG;
+constexpr int MS16_SLOT = 1280;                   // a tile's headers and packed bytes of half a super-block, in LDS
 constexpr int MS16_MAX_NB = 32;                   // super-blocks of a row (the scales of a tile wait in LDS)
 // weight rows of a workgroup whose waves take WT tiles of 16 each (DUAL: half of them gate rows, half up rows)
 constexpr int moe_split16_cols(int WT) { return 64 * WT; }
@@ -86,13 +87,13 @@ struct MoeSplit16 {
 
 // A workgroup of four waves multiplies a tile of up to 48 pairs of one expert with 64 WT weight rows (DUAL: half gate rows, half
 // the up rows of the same columns, the gated unit in the epilogue); a wave owns WT tiles of 16 rows, RG row groups of 16 pairs.
-// Bound: the issue of matrix and vector instructions, which hardly overlap, then what the workgroups wait for at their starts and
-// between halves: at 128 experts of 768 x 2048 and 512 tokens (32 pairs an expert) the counters show 25 % of the compute units' busy
-// cycles in matrix instructions (16 cycles each) and 28 % in vector instructions (4 cycles each), in gate and up as in down.  The
-// int8 GEMM took 3 x 102 us for the three products where these take 138 + 68.
+// Bound: the issue of matrix and vector instructions, which hardly overlap: at 128 experts of 768 x 2048 and 512 tokens (32 pairs an
+// expert) gate and up take 25 % of their former 142 us in matrix and 28 % in vector instructions.  Another 40 % went into looking up cache
+// lines, two clocks for every lane that reads its own share of a row: the packed bytes now come through LDS in pieces of a
+// row, half a super-block ahead, the layer 258 -> 231 us (150 tokens 167 -> 152).  The int8 GEMM took 3 x 102 us for the three products.
 template <bool DUAL, int RG, int WT>
 __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert, int beg, int cnt, int cb, uint8_t *lds, float *s_lds,
-                                                 int *y_lds) {
+                                                 int *y_lds, uint8_t *slots) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n16 = lane & 15, g = lane >> 4;
     constexpr int BUF = RG * 8 * S16_FRAG;
     constexpr int WD = DUAL ? WT / 2 : WT;  // tiles, and distinct columns' tiles
@@ -111,12 +112,30 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
         av[r] = rec * MS16_PLANES + 16u * g;
         xsp[r] = a.acts.xs + (size_t)rec * MS16_XS + 16 * (g & 1);
     }
+    // A half's packed bytes of a tile are 64 pieces of 16, a lane's each: row lane / 4, piece lane % 4 turned by the row's quarter, so that 16
+    // rows read at one place meet all banks once.  The headers are 16 pieces.
     const uint8_t *wp[WT];
+    uint32_t wv[WT], wh[WT];
+    const int turned = (lane & 3) ^ ((lane >> 4) & 3);
 #pragma unroll
     for (int w = 0; w < WT; w++) {
-        const int row = c0 + 16 * (w % WD);
-        wp[w] = (w >= WD ? a.wb : a.wa)[expert] + (size_t)min(row + n16, a.n - 1) * a.row_bytes;
+        const int row = min(c0 + 16 * (w % WD), a.n - 1);
+        wp[w] = s16_uniform((w >= WD ? a.wb : a.wa)[expert] + (size_t)row * a.row_bytes);
+        wv[w] = (uint32_t)min(lane >> 2, a.n - 1 - row) * (uint32_t)a.row_bytes + 16u * (uint32_t)turned + 16u;
+        wh[w] = (uint32_t)min(n16, a.n - 1 - row) * (uint32_t)a.row_bytes;
     }
+    uint8_t *const own = slots + wave * WT * MS16_SLOT;
+    const uint32_t own_at = s16_lds_offset(own);
+    const uint8_t *const my_q = own + 256 + 64 * n16 + 16 * (g ^ (n16 >> 2)), *const my_hdr = own + 16 * n16;
+    auto issue_w = [&](int sb, int hs) __attribute__((always_inline)) {
+#pragma unroll
+        for (int w = 0; w < WT; w++) {
+            const uint8_t *base = wp[w] + (size_t)sb * 144;
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(own_at + w * MS16_SLOT);
+            if (hs == 0 && lane < 16) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(wh[w]), "s"(base), "s"(dst) : "memory");
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(wv[w]), "s"(base + 64 * hs), "s"(dst + 256) : "memory");
+        }
+    };
     const uint32_t lds0 = s16_lds_offset(lds);
     // wave w brings k-step w of a half: both planes of every row group
     auto issue = [&](int sb, int hs) __attribute__((always_inline)) {
@@ -129,10 +148,16 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
                 asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(av[r]), "s"(base + 64 * p), "s"(dst) : "memory");
             }
     };
-    uint4 hdr[WT], hdrn[WT], q0[WT], q1[WT];
-    auto fetch = [&](int sb, int hs, uint4 (&q)[WT]) __attribute__((always_inline)) {
+    uint4 hdr[WT], q[WT];
+    auto read_w = [&](int hs) __attribute__((always_inline)) {
 #pragma unroll
-        for (int w = 0; w < WT; w++) q[w] = *(const uint4 *)(wp[w] + (size_t)sb * 144 + 16 + 64 * hs + 16 * g);
+        for (int w = 0; w < WT; w++) {
+            if (hs == 0) hdr[w] = *(const uint4 *)(my_hdr + w * MS16_SLOT);
+            q[w] = *(const uint4 *)(my_q + w * MS16_SLOT);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // in registers: their places are free
+#pragma unroll
+        for (int w = 0; w < WT; w++) asm volatile("" : "+v"(q[w].x), "+v"(q[w].y), "+v"(q[w].z), "+v"(q[w].w));
     };
     // The products with the low plane in sums of their own, where registers are left: eight matrix instructions instead of 16 then
     // round a sum of the super-block's size.  128 experts of 2048 x 768, 6 to 16 pairs each: the layer's error against 64 bits
@@ -189,44 +214,32 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
                     }
         }
     };
-    // the compiler waits for its own loads where their registers are first read: here, behind the wait for everything, and
-    // not behind the asynchronous loads issued next, which it would then wait for too
-    auto landed = [&](uint4 (&q)[WT]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int w = 0; w < WT; w++) asm volatile("" : "+v"(q[w].x), "+v"(q[w].y), "+v"(q[w].z), "+v"(q[w].w));
-    };
     issue(0, 0);
-#pragma unroll
-    for (int w = 0; w < WT; w++) hdr[w] = *(const uint4 *)wp[w];
-    fetch(0, 0, q0);
+    issue_w(0, 0);
     const uint32_t live = g < 2 ? 0xFFFFFFFFu : 0u;
     for (int sb = 0; sb < nb; sb++) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        landed(q0), landed(hdr);
         __syncthreads();  // the half has landed, and the other buffer's readers are done
         issue(sb, 1);
-        fetch(sb, 1, q1);
         s16_h8 xs[RG];
 #pragma unroll
         for (int r = 0; r < RG; r++) xs[r] = *(const s16_h8 *)(xsp[r] + (size_t)sb * MS16_XS);
+        read_w(0);
+        issue_w(sb, 1);
         uint32_t sc4[WT];
 #pragma unroll
         for (int w = 0; w < WT; w++) sc4[w] = hdr[w].y & 0x3F3F3F3Fu;
-        multiply(q0, sc4, lds + 16 * lane);
+        multiply(q, sc4, lds + 16 * lane);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        landed(q1);
 #pragma unroll
         for (int r = 0; r < RG; r++) asm volatile("" : "+v"(xs[r]));
         __syncthreads();
-        const int next = min(sb + 1, nb - 1);
         if (sb + 1 < nb) issue(sb + 1, 0);
-        fetch(next, 0, q0);
+        read_w(1);
+        if (sb + 1 < nb) issue_w(sb + 1, 0);
 #pragma unroll
-        for (int w = 0; w < WT; w++) {
-            hdrn[w] = *(const uint4 *)(wp[w] + (size_t)next * 144);
-            sc4[w] = (hdr[w].w & 0x0F0F0F0Fu) | ((hdr[w].y >> 2) & 0x30303030u);
-        }
-        multiply(q1, sc4, lds + BUF + 16 * lane);
+        for (int w = 0; w < WT; w++) sc4[w] = (hdr[w].w & 0x0F0F0F0Fu) | ((hdr[w].y >> 2) & 0x30303030u);
+        multiply(q, sc4, lds + BUF + 16 * lane);
         // the min term, and the super-block's sums onto the results
         s16_f4 s[RG];
 #pragma unroll
@@ -251,7 +264,6 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
                 for (int i = 0; i < 4; i++) acc[w][r][i] = fmaf(s[r][i], fmaf(dm, i2[i], d * i1[w][r][i]), acc[w][r][i]);
                 i1[w][r] = zero;
             }
-            hdr[w] = hdrn[w];
         }
     }
     // every result first, then the stores one behind the other: a load or a branch between them would wait for each
@@ -288,20 +300,21 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
 
 // grid: cols x tiles (a multiple of 8; an upper bound, the rest leaves at once), ids 8 apart (one XCD) holding the column
 // blocks of one tile, which read the same activation planes.
-inline int moe_split16_lds(int nb) { return 2 * MS16_RG * 8 * S16_FRAG + 4 * MS16_ROWS * (nb + 1); }
+inline int moe_split16_lds(int nb, int WT) { return 2 * MS16_RG * 8 * S16_FRAG + 4 * MS16_ROWS * (nb + 1) + 4 * WT * MS16_SLOT; }
 
 template <bool DUAL, int WT>
-static __global__ __launch_bounds__(256, WT == 2 ? 3 : 2) void moe_split16(MoeSplit16 a) {
+static __global__ __launch_bounds__(256, 2) void moe_split16(MoeSplit16 a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // two buffers of a half, the scales, the result rows
     float *s_lds = (float *)(lds + 2 * MS16_RG * 8 * S16_FRAG);
     int *y_lds = (int *)(s_lds + MS16_ROWS * a.nb);
+    uint8_t *slots = (uint8_t *)(y_lds + MS16_ROWS);
     const int id = blockIdx.x, mt = id / (8 * a.cols) * 8 + id % 8, cb = id / 8 % a.cols;
     int grp, at;
     if (!s16_find_tile(a.offsets, a.groups, a.rows, mt, grp, at)) return;  // past the last tile: the whole workgroup
     const int beg = a.offsets[grp] + at, cnt = min(a.offsets[grp + 1] - beg, a.rows), expert = a.gexp[grp];
-    if (cnt <= 16) moe_split16_tile<DUAL, 1, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds);
-    else if (cnt <= 32) moe_split16_tile<DUAL, 2, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds);
-    else moe_split16_tile<DUAL, 3, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds);
+    if (cnt <= 16) moe_split16_tile<DUAL, 1, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds, slots);
+    else if (cnt <= 32) moe_split16_tile<DUAL, 2, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds, slots);
+    else moe_split16_tile<DUAL, 3, WT>(a, expert, beg, cnt, cb, lds, s_lds, y_lds, slots);
 }
 
 }  // namespace jq

@@ -23,10 +23,10 @@ int moe_split16(const MoeSplit16Call &c, hipStream_t s) {
     a.wa = c.wa, a.wb = c.wb, a.row_bytes = c.row_bytes;
     a.gexp = c.gexp, a.offsets = c.offsets, a.xsel = c.xsel, a.yrow = c.yrow;
     a.Y = c.Y, a.groups = c.groups, a.n = (int)c.n, a.nb = (int)nb, a.clamp = c.clamp;
-    // Few pairs an expert: workgroups of half the weight rows, three a compute unit, fill the chip more evenly (an expert of 768
-    // rows at 32 pairs each: gate and up 141 us against 151).  More: the tile's activations pass through LDS half as often
-    // (the down projection there 68 against 76; 128 pairs an expert, the layer 683 against 728).
-    const int wt = c.pairs < (c.wb ? 48 : 16) * (size_t)c.groups ? 2 : 4;
+    // Few pairs an expert: gate and up in workgroups of half the weight rows (128 experts of 768, 150 tokens: the layer 152 us against 157,
+    // 250 tokens 173 either way, 512 tokens 239 against 231).  Down in whole ones (100 tokens 143 against 147, 512 tokens 231 against 242),
+    // where the layer has that many.
+    const int wt = c.n <= 128 || (c.wb && c.pairs < 16 * (size_t)c.groups) ? 2 : 4;
     const size_t per = jq::moe_split16_cols(wt) / (c.wb ? 2 : 1);
     a.cols = (int)((c.n + per - 1) / per);
     // Calls of fewer than 16 pairs an expert, which the ring kernel's f32 products would run, take two row groups a tile at most,
@@ -35,8 +35,14 @@ int moe_split16(const MoeSplit16Call &c, hipStream_t s) {
     const size_t tiles = (c.pairs / (size_t)a.rows + (size_t)c.groups + 7) / 8 * 8;
     if (tiles * a.cols > 0x7FFFFFFFull) return -1;
     hipLaunchKernelGGL(jq::moe_split16_prep, dim3((unsigned)c.x_rows, (unsigned)((nb + 3) / 4)), dim3(256), 0, s, c.X, (int)c.k, a.acts);
-    const int lds = jq::moe_split16_lds((int)nb);
+    const int lds = jq::moe_split16_lds((int)nb, wt);
     auto *kernel = c.wb ? (wt == 2 ? jq::moe_split16<true, 2> : jq::moe_split16<true, 4>) : (wt == 2 ? jq::moe_split16<false, 2> : jq::moe_split16<false, 4>);
+    static const hipError_t big[4] = {
+#define JQ_BIG(D, WT) hipFuncSetAttribute((const void *)jq::moe_split16<D, WT>, hipFuncAttributeMaxDynamicSharedMemorySize, jq::moe_split16_lds(jq::MS16_MAX_NB, WT))
+        JQ_BIG(true, 2), JQ_BIG(true, 4), JQ_BIG(false, 2), JQ_BIG(false, 4)};
+#undef JQ_BIG
+    for (const hipError_t e : big)
+        if (e != hipSuccess) return fail("hipFuncSetAttribute: %s", hipGetErrorString(e));
     hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles * a.cols)), dim3(256), lds, s, a);
     HIP_TRY(hipGetLastError());
     note_kernel("moe_split16");
