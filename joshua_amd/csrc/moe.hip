@@ -102,7 +102,7 @@ int moe_route_dev(jq_moe *m, size_t T, const float *x, hipStream_t s, jq::MoePai
         hipLaunchKernelGGL(jq::moe_router_logits_norm, dim3(c.n_expert), dim3(256), 0, s, m->router_w, *pre, m->logits,
                            (int)c.hidden, (int)c.n_expert);
     else if (T >= tile_from && !no_tile)  // many tokens: a token's activations read once per eight experts (the same bits)
-        hipLaunchKernelGGL(jq::moe_router_logits_tile, dim3((c.n_expert + 7) / 8, (unsigned)((T + 7) / 8)), dim3(256), 0, s,
+        hipLaunchKernelGGL(jq::moe_router_logits_tile, dim3((unsigned)((T + 7) / 8), (c.n_expert + 7) / 8), dim3(256), 0, s,
                            m->router_w, x, m->logits, (int)T, (int)c.hidden, (int)c.n_expert,
                            c.hidden % 32 == 0 ? planes : jq::ActsI8{nullptr, nullptr, nullptr, nullptr});
     else
