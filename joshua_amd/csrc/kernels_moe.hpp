@@ -535,7 +535,9 @@ static __global__ __launch_bounds__(GROUP_PAIRS_THREADS) void moe_group_pairs(co
 // expert (its rank within the chunk), the last lane of an expert in the chunk records the chunk's count of
 // that expert in hist[chunk][expert]; prefix sums over the chunks and then over the experts turn the counts
 // into start positions, and a pair's place is its expert's start + the earlier chunks' count + its rank.
-// LDS: chunks * E + E + 1 ints.
+// Bound: latency of one workgroup's chain.  The pairs are put in order in LDS and leave in whole lines: stored straight to
+// their places, 64 lines an instruction, they took a sixth of it (4096 pairs of 128 experts: 12.5 -> 10.6 us).
+// LDS: max(chunks * E, pairs) + E + 1 ints.
 constexpr int GROUP_RANK_CHUNKS = 64, GROUP_RANK_PER_WAVE = GROUP_RANK_CHUNKS * 64 / GROUP_PAIRS_THREADS;
 
 static __global__ __launch_bounds__(GROUP_PAIRS_THREADS) void moe_group_pairs_ranked(const uint32_t *__restrict__ ids, int T,
@@ -543,9 +545,9 @@ static __global__ __launch_bounds__(GROUP_PAIRS_THREADS) void moe_group_pairs_ra
                                                                               int *__restrict__ offsets,
                                                                               int *__restrict__ xrow, int *__restrict__ yrow,
                                                                               int shared_group) {
-    extern __shared__ int hist[];  // [chunks][E], then start[E + 1]
+    extern __shared__ int hist[];  // [chunks][E], in the end the pairs in order; then start[E + 1]
     const int P = T * k_used, chunks = (P + 63) / 64;
-    int *start = hist + chunks * E;
+    int *start = hist + max(chunks * E, P);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     constexpr int WAVES = GROUP_PAIRS_THREADS / 64;
     const int bits = 32 - __builtin_clz((uint32_t)E);  // (the highest number, E - 1, is not all ones in them: 0xFFFFFFFF is)
@@ -616,14 +618,19 @@ static __global__ __launch_bounds__(GROUP_PAIRS_THREADS) void moe_group_pairs_ra
         if (threadIdx.x == 0) gexp[E] = E, offsets[E + 1] = P + T;
         for (int t = threadIdx.x; t < T; t += GROUP_PAIRS_THREADS) xrow[P + t] = t, yrow[P + t] = P + t;
     }
+    int at[GROUP_RANK_PER_WAVE];
 #pragma unroll
-    for (int c = 0; c < GROUP_RANK_PER_WAVE; c++) {
-        const int chunk = wave + WAVES * c, pidx = 64 * chunk + lane;
-        if (mine[c] < (uint32_t)E) {
-            const int at = start[mine[c]] + hist[chunk * E + (int)mine[c]] + rank[c];
-            xrow[at] = pidx / k_used;
-            yrow[at] = pidx;
-        }
+    for (int c = 0; c < GROUP_RANK_PER_WAVE; c++)
+        at[c] = mine[c] < (uint32_t)E ? start[mine[c]] + hist[(wave + WAVES * c) * E + (int)mine[c]] + rank[c] : -1;
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < GROUP_RANK_PER_WAVE; c++)
+        if (at[c] >= 0) hist[at[c]] = 64 * (wave + WAVES * c) + lane;
+    __syncthreads();
+    for (int i = threadIdx.x; i < start[E]; i += GROUP_PAIRS_THREADS) {
+        const int pidx = hist[i];
+        xrow[i] = pidx / k_used;
+        yrow[i] = pidx;
     }
 }
 

@@ -143,9 +143,9 @@ int moe_group_dev(jq_moe *m, size_t T, int extra, hipStream_t s) {
     const jq_moe_config &c = m->cfg;
     const int P = (int)(T * c.n_expert_used);
     const int in_lds = (size_t)P <= 12288;
-    const size_t chunks = ((size_t)P + 63) / 64, rank_ints = chunks * c.n_expert + c.n_expert + 1;
+    const size_t chunks = ((size_t)P + 63) / 64, rank_ints = std::max(chunks * c.n_expert, (size_t)P) + c.n_expert + 1;
     static const char *no_ranked = getenv("JQ_MOE_NO_RANKED_GROUPING");
-    // (its rank table: chunks x experts ints of LDS, up to 144 KB)
+    // (its rank table: chunks x experts ints of LDS, up to 144 KB; fewer experts than fit need no more than the pairs' 16 KB)
     if (!no_ranked && chunks <= (size_t)jq::GROUP_RANK_CHUNKS && rank_ints <= 36864) {
         static std::once_flag big_lds;
         static hipError_t attr_rc = hipSuccess;
