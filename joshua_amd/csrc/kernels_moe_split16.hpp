@@ -24,7 +24,9 @@ namespace jq {
 constexpr int MS16_PLANES = 1024, MS16_XS = 32;  // bytes a row and super-block: hi and lo of 256 elements; of 8 sums
 constexpr int MS16_RG = 3;                        // row groups of 16 a tile holds at most
 constexpr int MS16_ROWS = 16 * MS16_RG;
-constexpr int MS16_SLOT = 1280;                   // a tile's headers and packed bytes of half a super-block, in LDS
+constexpr int MS16_SLOTS = 2304;                  // a tile's packed bytes in LDS: headers, first half, second half of a super-block
+constexpr int MS16_BUF = MS16_RG * 4 * S16_FRAG;  // a quarter's activation planes
+constexpr int MS16_ACTS = 3 * MS16_BUF + MS16_RG * 512;  // three quarters, and a super-block's sums
 constexpr int MS16_MAX_NB = 32;                   // super-blocks of a row (the scales of a tile wait in LDS)
 // weight rows of a workgroup whose waves take WT tiles of 16 each (DUAL: half of them gate rows, half up rows)
 constexpr int moe_split16_cols(int WT) { return 64 * WT; }
@@ -87,31 +89,27 @@ struct MoeSplit16 {
 
 // A workgroup of four waves multiplies a tile of up to 48 pairs of one expert with 64 WT weight rows (DUAL: half gate rows, half
 // the up rows of the same columns, the gated unit in the epilogue); a wave owns WT tiles of 16 rows, RG row groups of 16 pairs.
-// Bound: the issue of matrix and vector instructions, which hardly overlap: at 128 experts of 768 x 2048 and 512 tokens (32 pairs an
-// expert) gate and up take 25 % of their former 142 us in matrix and 28 % in vector instructions.  Another 40 % went into looking up cache
-// lines, two clocks for every lane that reads its own share of a row: the packed bytes now come through LDS in pieces of a
-// row, half a super-block ahead, the layer 258 -> 231 us (150 tokens 167 -> 152).  The int8 GEMM took 3 x 102 us for the three products.
+// Bound: no one thing.  128 experts of 768 x 2048 and 512 tokens (32 pairs an expert), gate and up, 120 us: 31 us of matrix and 34 of vector
+// instructions, 44 us for the weights at a large copy's rate, 18 us of starts and ends of workgroups; without its copies the loop takes 30 us
+// less, without matrix instructions or unpacking 7 to 11.  The packed bytes come through LDS in pieces of a row (a lane that reads its own share
+// of one looks up a cache line for itself, two clocks): the layer 258 -> 231 us.  Two halves of them on their way, and the activations in
+// quarters, as two workgroups a compute unit leave room for: 100 tokens 139.5 -> 136.5, 150 tokens 151.5 -> 146.5, 512 tokens as before.
+// The int8 GEMM took 3 x 102 us for the three products.
 template <bool DUAL, int RG, int WT>
 __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert, int beg, int cnt, int cb, uint8_t *lds, float *s_lds,
                                                  int *y_lds, uint8_t *slots) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n16 = lane & 15, g = lane >> 4;
-    constexpr int BUF = RG * 8 * S16_FRAG;
     constexpr int WD = DUAL ? WT / 2 : WT;  // tiles, and distinct columns' tiles
     const int nb = a.nb, c0 = (4 * cb + wave) * 16 * WD;
-    if (tid < MS16_ROWS) y_lds[tid] = a.yrow[beg + min(tid, cnt - 1)];
-    // the scales of the tile's rows, [super-block][row]
-    for (int i = tid; i < 16 * RG * nb; i += 256) {
-        const int row = i % (16 * RG), sb = i / (16 * RG);
-        s_lds[i] = a.acts.s[(size_t)a.xsel[beg + min(row, cnt - 1)] * nb + sb];
-    }
     uint32_t av[RG];          // this lane's share of a fragment: row n16 of each row group, 16-byte run g
-    const uint8_t *xsp[RG];   // and of the sums' operand (lane groups 2 and 3 meet zero mins)
 #pragma unroll
     for (int r = 0; r < RG; r++) {
         const uint32_t rec = (uint32_t)a.xsel[beg + min(16 * r + n16, cnt - 1)] * (uint32_t)nb;
         av[r] = rec * MS16_PLANES + 16u * g;
-        xsp[r] = a.acts.xs + (size_t)rec * MS16_XS + 16 * (g & 1);
     }
+    // the sums: 32 RG pieces of 16 bytes, the same number for every wave
+    constexpr int XP = 8 * RG;
+    const uint32_t xv = (uint32_t)a.xsel[beg + min((XP * wave + lane) >> 1, cnt - 1)] * (uint32_t)nb * MS16_XS + 16u * (lane & 1);
     // A half's packed bytes of a tile are 64 pieces of 16, a lane's each: row lane / 4, piece lane % 4 turned by the row's quarter, so that 16
     // rows read at one place meet all banks once.  The headers are 16 pieces.
     const uint8_t *wp[WT];
@@ -124,36 +122,32 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
         wv[w] = (uint32_t)min(lane >> 2, a.n - 1 - row) * (uint32_t)a.row_bytes + 16u * (uint32_t)turned + 16u;
         wh[w] = (uint32_t)min(n16, a.n - 1 - row) * (uint32_t)a.row_bytes;
     }
-    uint8_t *const own = slots + wave * WT * MS16_SLOT;
-    const uint32_t own_at = s16_lds_offset(own);
+    uint8_t *const own = slots + wave * WT * MS16_SLOTS;
+    const uint32_t own_at = s16_lds_offset(own), lds0 = s16_lds_offset(lds);
     const uint8_t *const my_q = own + 256 + 64 * n16 + 16 * (g ^ (n16 >> 2)), *const my_hdr = own + 16 * n16;
+#define JQ_COPY(v, base, dst) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(v), "s"(base), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory")
     auto issue_w = [&](int sb, int hs) __attribute__((always_inline)) {
 #pragma unroll
         for (int w = 0; w < WT; w++) {
             const uint8_t *base = wp[w] + (size_t)sb * 144;
-            const uint32_t dst = __builtin_amdgcn_readfirstlane(own_at + w * MS16_SLOT);
-            if (hs == 0 && lane < 16) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(wh[w]), "s"(base), "s"(dst) : "memory");
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(wv[w]), "s"(base + 64 * hs), "s"(dst + 256) : "memory");
+            if (hs == 0 && lane < 16) JQ_COPY(wh[w], base, own_at + w * MS16_SLOTS);
+            JQ_COPY(wv[w], base + 64 * hs, own_at + w * MS16_SLOTS + 256 + 1024 * hs);
         }
     };
-    const uint32_t lds0 = s16_lds_offset(lds);
-    // wave w brings k-step w of a half: both planes of every row group
-    auto issue = [&](int sb, int hs) __attribute__((always_inline)) {
-        const uint8_t *base = a.acts.planes + (size_t)sb * MS16_PLANES + 512 * hs + 128 * wave;
+    // A quarter is one nibble of a half: two k-steps of two planes, a wave's each; with the last one the sums.
+    auto issue = [&](int sb, int qt, int buf) __attribute__((always_inline)) {
+        const uint8_t *base = a.acts.planes + (size_t)sb * MS16_PLANES + 256 * qt + 64 * wave;
 #pragma unroll
-        for (int r = 0; r < RG; r++)
-#pragma unroll
-            for (int p = 0; p < 2; p++) {
-                const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + hs * BUF + ((r * 4 + wave) * 2 + p) * S16_FRAG);
-                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(av[r]), "s"(base + 64 * p), "s"(dst) : "memory");
-            }
+        for (int r = 0; r < RG; r++) JQ_COPY(av[r], base, lds0 + buf * MS16_BUF + (4 * r + wave) * S16_FRAG);
+        if (qt == 3 && lane < XP) JQ_COPY(xv, a.acts.xs + (size_t)sb * MS16_XS, lds0 + 3 * MS16_BUF + 16 * XP * wave);
     };
+#undef JQ_COPY
     uint4 hdr[WT], q[WT];
     auto read_w = [&](int hs) __attribute__((always_inline)) {
 #pragma unroll
         for (int w = 0; w < WT; w++) {
-            if (hs == 0) hdr[w] = *(const uint4 *)(my_hdr + w * MS16_SLOT);
-            q[w] = *(const uint4 *)(my_q + w * MS16_SLOT);
+            if (hs == 0) hdr[w] = *(const uint4 *)(my_hdr + w * MS16_SLOTS);
+            q[w] = *(const uint4 *)(my_q + w * MS16_SLOTS + 1024 * hs);
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // in registers: their places are free
 #pragma unroll
@@ -169,18 +163,14 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
 #pragma unroll
     for (int w = 0; w < WT; w++)
 #pragma unroll
-        for (int r = 0; r < RG; r++) {
-            acc[w][r] = i1[w][r] = zero;
-            if constexpr (APART) low[w][r] = zero;
-        }
+        for (int r = 0; r < RG; r++) acc[w][r] = zero;
     // (masks and magic numbers in registers: v_and_or_b32 takes one scalar operand and no two literals)
     uint32_t m_lo = 0x000F000Fu, m_hi = 0x00F000F0u, o_lo = 0x64006400u, o_hi = 0x54005400u;
     asm("" : "+s"(m_lo), "+s"(m_hi), "+v"(o_lo), "+v"(o_hi));
     // byte selectors: scale 2 (g / 2) + nibble of the half's four into both f16 of a register, each under 0x64
     const uint32_t sel0 = 0x04000400u + 0x00010001u * (uint32_t)(2 * (g >> 1)), sel1 = sel0 + 0x00010001u;
-    auto multiply = [&](const uint4 (&q)[WT], const uint32_t (&sc4)[WT], const uint8_t *l) __attribute__((always_inline)) {
-#pragma unroll
-        for (int nib = 0; nib < 2; nib++) {
+    auto multiply = [&](int nib, bool first, const uint32_t (&sc4)[WT], const uint8_t *l) __attribute__((always_inline)) {
+        {
             s16_h8 b[2][WT];
 #pragma unroll
             for (int w = 0; w < WT; w++) {
@@ -205,41 +195,68 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
                 for (int p = 0; p < 2; p++)
 #pragma unroll
                     for (int r = 0; r < RG; r++) {
-                        const s16_h8 x = *(const s16_h8 *)(l + ((r * 4 + 2 * nib + s8) * 2 + p) * S16_FRAG);
+                        const s16_h8 x = *(const s16_h8 *)(l + ((r * 2 + s8) * 2 + p) * S16_FRAG);
 #pragma unroll
                         for (int w = 0; w < WT; w++) {
                             s16_f4 &to = APART && p ? low[APART ? w : 0][APART ? r : 0] : i1[w][r];
-                            to = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, b[s8][w], to, 0, 0, 0);
+                            to = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, b[s8][w], first && s8 == 0 && (APART || p == 0) ? zero : to, 0, 0, 0);
                         }
                     }
         }
     };
-    issue(0, 0);
+    // Two halves of the weights are on their way while one is multiplied, and two quarters of the activations.
     issue_w(0, 0);
+    issue(0, 0, 0);
+    issue_w(0, 1);
+    issue(0, 1, 1);
+    if (tid < MS16_ROWS) y_lds[tid] = a.yrow[beg + min(tid, cnt - 1)];
+    // the scales of the tile's rows, [super-block][row]
+    for (int i = tid; i < 16 * RG * nb; i += 256) {
+        const int row = i % (16 * RG), sb = i / (16 * RG);
+        s_lds[i] = a.acts.s[(size_t)a.xsel[beg + min(row, cnt - 1)] * nb + sb];
+    }
     const uint32_t live = g < 2 ? 0xFFFFFFFFu : 0u;
+    int buf = 0;
+    auto next = [](int b, int by) { return b + by >= 3 ? b + by - 3 : b + by; };
+    // a quarter has landed once no more than what was asked for behind it is on its way; the buffer of the one before is free then
+#define JQ_LANDED(behind) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(behind) : "memory")
     for (int sb = 0; sb < nb; sb++) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();  // the half has landed, and the other buffer's readers are done
-        issue(sb, 1);
-        s16_h8 xs[RG];
-#pragma unroll
-        for (int r = 0; r < RG; r++) xs[r] = *(const s16_h8 *)(xsp[r] + (size_t)sb * MS16_XS);
-        read_w(0);
-        issue_w(sb, 1);
+        const bool more = sb + 1 < nb;
         uint32_t sc4[WT];
+        JQ_LANDED(WT + RG);
+        __builtin_amdgcn_s_barrier();
+        issue(sb, 2, next(buf, 2));
+        read_w(0);
+        if (more) issue_w(sb + 1, 0);
 #pragma unroll
         for (int w = 0; w < WT; w++) sc4[w] = hdr[w].y & 0x3F3F3F3Fu;
-        multiply(q, sc4, lds + 16 * lane);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int r = 0; r < RG; r++) asm volatile("" : "+v"(xs[r]));
-        __syncthreads();
-        if (sb + 1 < nb) issue(sb + 1, 0);
+        multiply(0, true, sc4, lds + buf * MS16_BUF + 16 * lane);
+        buf = next(buf, 1);
+        if (more) JQ_LANDED(RG + 2 * WT);
+        else JQ_LANDED(RG);
+        __builtin_amdgcn_s_barrier();
+        issue(sb, 3, next(buf, 2));
+        multiply(1, false, sc4, lds + buf * MS16_BUF + 16 * lane);
+        buf = next(buf, 1);
+        if (more) JQ_LANDED(RG + 1 + 2 * WT);
+        else JQ_LANDED(RG + 1);
+        __builtin_amdgcn_s_barrier();
+        if (more) issue(sb + 1, 0, next(buf, 2));
         read_w(1);
-        if (sb + 1 < nb) issue_w(sb + 1, 0);
+        if (more) issue_w(sb + 1, 1);
 #pragma unroll
         for (int w = 0; w < WT; w++) sc4[w] = (hdr[w].w & 0x0F0F0F0Fu) | ((hdr[w].y >> 2) & 0x30303030u);
-        multiply(q, sc4, lds + BUF + 16 * lane);
+        multiply(0, false, sc4, lds + buf * MS16_BUF + 16 * lane);
+        buf = next(buf, 1);
+        if (more) JQ_LANDED(RG + WT);
+        else JQ_LANDED(0);
+        __builtin_amdgcn_s_barrier();
+        if (more) issue(sb + 1, 1, next(buf, 2));
+        multiply(1, false, sc4, lds + buf * MS16_BUF + 16 * lane);
+        buf = next(buf, 1);
+        s16_h8 xs[RG];  // (lane groups 2 and 3 meet zero mins)
+#pragma unroll
+        for (int r = 0; r < RG; r++) xs[r] = *(const s16_h8 *)(lds + 3 * MS16_BUF + (16 * r + n16) * MS16_XS + 16 * (g & 1));
         // the min term, and the super-block's sums onto the results
         s16_f4 s[RG];
 #pragma unroll
@@ -259,13 +276,13 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
 #pragma unroll
             for (int r = 0; r < RG; r++) {
                 const s16_f4 i2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xs[r], mins, zero, 0, 0, 0);
-                if constexpr (APART) i1[w][r] += low[w][r], low[w][r] = zero;
+                if constexpr (APART) i1[w][r] += low[w][r];
 #pragma unroll
                 for (int i = 0; i < 4; i++) acc[w][r][i] = fmaf(s[r][i], fmaf(dm, i2[i], d * i1[w][r][i]), acc[w][r][i]);
-                i1[w][r] = zero;
             }
         }
     }
+#undef JQ_LANDED
     // every result first, then the stores one behind the other: a load or a branch between them would wait for each
     const float limit = DUAL ? (expert >= a.clamp.n_routed ? a.clamp.shared : a.clamp.routed) : 0.0f;
     const float top = limit > 0.0f ? limit : INFINITY;
@@ -300,12 +317,12 @@ __device__ __forceinline__ void moe_split16_tile(const MoeSplit16 &a, int expert
 
 // grid: cols x tiles (a multiple of 8; an upper bound, the rest leaves at once), ids 8 apart (one XCD) holding the column
 // blocks of one tile, which read the same activation planes.
-inline int moe_split16_lds(int nb, int WT) { return 2 * MS16_RG * 8 * S16_FRAG + 4 * MS16_ROWS * (nb + 1) + 4 * WT * MS16_SLOT; }
+inline int moe_split16_lds(int nb, int WT) { return MS16_ACTS + 4 * MS16_ROWS * (nb + 1) + 4 * WT * MS16_SLOTS; }
 
 template <bool DUAL, int WT>
 static __global__ __launch_bounds__(256, 2) void moe_split16(MoeSplit16 a) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // two buffers of a half, the scales, the result rows
-    float *s_lds = (float *)(lds + 2 * MS16_RG * 8 * S16_FRAG);
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // the activations, the scales, the result rows, the weights
+    float *s_lds = (float *)(lds + MS16_ACTS);
     int *y_lds = (int *)(s_lds + MS16_ROWS * a.nb);
     uint8_t *slots = (uint8_t *)(y_lds + MS16_ROWS);
     const int id = blockIdx.x, mt = id / (8 * a.cols) * 8 + id % 8, cb = id / 8 % a.cols;

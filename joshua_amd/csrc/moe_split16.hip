@@ -23,10 +23,9 @@ int moe_split16(const MoeSplit16Call &c, hipStream_t s) {
     a.wa = c.wa, a.wb = c.wb, a.row_bytes = c.row_bytes;
     a.gexp = c.gexp, a.offsets = c.offsets, a.xsel = c.xsel, a.yrow = c.yrow;
     a.Y = c.Y, a.groups = c.groups, a.n = (int)c.n, a.nb = (int)nb, a.clamp = c.clamp;
-    // Few pairs an expert: gate and up in workgroups of half the weight rows (128 experts of 768, 150 tokens: the layer 152 us against 157,
-    // 250 tokens 173 either way, 512 tokens 239 against 231).  Down in whole ones (100 tokens 143 against 147, 512 tokens 231 against 242),
-    // where the layer has that many.
-    const int wt = c.n <= 128 || (c.wb && c.pairs < 16 * (size_t)c.groups) ? 2 : 4;
+    // Waves of two tiles only for layers whose rows do not fill workgroups of four (128 experts of 768, the layer, us: 70 tokens 144 with two
+    // and 135 with four, 150 tokens 155 / 146, 250 tokens 175 / 173, 512 tokens 235 / 220).
+    const int wt = c.n <= 128 ? 2 : 4;
     const size_t per = jq::moe_split16_cols(wt) / (c.wb ? 2 : 1);
     a.cols = (int)((c.n + per - 1) / per);
     // Calls of fewer than 16 pairs an expert, which the ring kernel's f32 products would run, take two row groups a tile at most,
