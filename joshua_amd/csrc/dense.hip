@@ -92,6 +92,42 @@ void launch_gemm(const jq::DenseGemm &a, unsigned n_tiles, hipStream_t s) {
     hipLaunchKernelGGL((jq::dense_gemm<E, BM, BN, GATED, GROUPED>), dim3((unsigned)a.m_tiles * n_tiles, (unsigned)a.splits), dim3(256), 0, s, a);
 }
 
+template <int BN, bool GATED>
+int launch_wide(const jq::DenseGemm &a, unsigned n_tiles, hipStream_t s) {
+    static const hipError_t big = hipFuncSetAttribute((const void *)jq::dense_gemm_wide<BN, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                      jq::dense_wide_lds(BN));
+    HIP_TRY(big);
+    hipLaunchKernelGGL((jq::dense_gemm_wide<BN, GATED>), dim3((unsigned)a.m_tiles * n_tiles, (unsigned)a.splits), dim3(512),
+                       jq::dense_wide_lds(BN), s, a);
+    return 0;
+}
+
+// Whether a product runs in tiles of 256 activation rows on workgroups that have a compute unit to themselves (dense_gemm_wide), in how many
+// weight rows and runs of k: where the rounds of 256 workgroups that it takes cost less than the smaller tiles, two or three to a compute
+// unit.  Per stage and round, us: 256 rows 1.9, 192 rows 1.5; 128 x 128 1.22, 64 x 128 0.8, of which a round that is not full takes 0.6
+// at least.  A split adds the writing and reading of its sums at some 6 TB/s.  Measured, smaller / wide, us: gate and up 24576 x 4096 of
+// 512 rows 146 / 99 (192), 16384 x 4096 of 2000 rows 324 / 255, 4096 x 12288 of 2000 rows 257 / 234 (two runs); 16384 x 4096 of 512 rows
+// 93 / 95 and 6144 x 4096 of 512 rows 48 / 50 stay with the smaller ones.
+struct WidePick {
+    int bn = 0, splits = 1;
+};
+WidePick wide_pick(const jq::DenseGemm &a, size_t wrows, int bm, size_t tiles, int splits) {
+    auto sums = [&](size_t s) { return s > 1 ? 4.0 + (2.0 * s + 1.0) * a.M * (double)wrows * 4e-6 / 6.0 : 0.0; };
+    auto stages = [&](size_t s) { return (double)((a.stages + s - 1) / s); };
+    const double rounds = (double)(tiles * splits) / (bm == 128 ? 512 : 768), part = rounds - std::floor(rounds);
+    double best = 0.95 * ((std::floor(rounds) + (part > 0 ? 0.6 + 0.4 * part : 0.0)) * stages(splits) * (bm == 128 ? 1.22 : 0.8) + sums(splits));
+    WidePick pick;
+    for (const int bn : {256, 192}) {
+        const size_t t = (size_t)((a.M + 255) / 256) * ((wrows + bn - 1) / bn);
+        const size_t most = a.heads ? 1 : std::max<size_t>(1, std::min<size_t>(256 / t, (size_t)a.stages / 16));
+        for (const size_t s : {(size_t)1, most}) {
+            const double us = (double)((t * s + 255) / 256) * (stages(s) * (bn == 256 ? 1.9 : 1.5) + 6.0) + sums(s);
+            if (us < best) best = us, pick = {bn, (int)s};
+        }
+    }
+    return pick;
+}
+
 // Tile of a product of `rows` activation rows (per group) and `wrows` weight rows: 128 x 128 where that makes enough
 // tiles or the row count wants it, else smaller.
 template <bool GATED, bool GROUPED>
@@ -114,10 +150,18 @@ int run_gemm(uint32_t type, jq::DenseGemm a, size_t rows_of_a, size_t k, size_t 
         const auto u = tiles(bm, bn);
         if (u.first * u.second < 128) bn = 64;
     }
+    WidePick wide;
+    if constexpr (!GROUPED) {
+        if (type == JQ_TYPE_BF16 && bn == 128) {
+            const auto u = tiles(bm, bn);
+            wide = wide_pick(a, wrows, bm, u.first * u.second, a.heads ? 1 : gemm_splits(u.first * u.second, a.stages));
+        }
+    }
+    if (wide.bn) bm = 256, bn = wide.bn;
     const auto t = tiles(bm, bn);
     if (t.first * t.second > 0x7FFFFFFFull) return fail("dense gemm: too many tiles");
     a.m_tiles = (int)t.first;
-    a.splits = GROUPED || a.heads ? 1 : gemm_splits(t.first * t.second, a.stages);
+    a.splits = wide.bn ? wide.splits : GROUPED || a.heads ? 1 : gemm_splits(t.first * t.second, a.stages);
     CallScratch scratch;
     float *C = a.C;
     if (a.splits > 1) {
@@ -133,7 +177,11 @@ int run_gemm(uint32_t type, jq::DenseGemm a, size_t rows_of_a, size_t k, size_t 
         }
     }
     if (type == JQ_TYPE_BF16) {
-        if (bm == 128) launch_gemm<jq::ElemBf16, 128, 128, GATED, GROUPED>(a, (unsigned)t.second, s);
+        if (wide.bn) {
+            if constexpr (!GROUPED) {
+                if (bn == 256 ? launch_wide<256, GATED>(a, (unsigned)t.second, s) : launch_wide<192, GATED>(a, (unsigned)t.second, s)) return 1;
+            }
+        } else if (bm == 128) launch_gemm<jq::ElemBf16, 128, 128, GATED, GROUPED>(a, (unsigned)t.second, s);
         else if (bn == 128) launch_gemm<jq::ElemBf16, 64, 128, GATED, GROUPED>(a, (unsigned)t.second, s);
         else launch_gemm<jq::ElemBf16, 64, 64, GATED, GROUPED>(a, (unsigned)t.second, s);
     } else {

@@ -423,6 +423,66 @@ __device__ __forceinline__ void dma_chunk16(const uint8_t *sbase, uint32_t voff,
 // Columns of a partial-sum row: a gated product keeps gate and up in alternating runs of 16.
 __host__ __device__ inline size_t gemm_partial_width(int N, bool gated) { return gated ? 2 * (size_t)((N + 15) / 16 * 16) : (size_t)N; }
 
+// A wave's FM x FN tiles of results: rows r0 .. of a group's rows_here, columns from the workgroup's first one, c0, on.
+template <class E, int FM, int FN, bool GATED, bool GROUPED>
+__device__ __forceinline__ void dense_gemm_store(const DenseGemm &a, const f32x4 (&acc)[FN][FM], int r0, int row_lo, int rows_here, int c0, int wn) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, l16 = lane & 15;
+    const bool partial = a.splits > 1;
+    const size_t width = partial ? gemm_partial_width(a.N, GATED) : a.ldc;
+    float *C = a.C + (partial ? (size_t)blockIdx.y * a.M * width : 0);
+#pragma unroll
+    for (int m = 0; m < FM; m++) {
+        const int lr = r0 + 16 * m + l16;
+        if (lr >= rows_here) continue;
+        int orow = row_lo + lr;
+        if constexpr (GROUPED) {
+            if (a.yrow && !partial) orow = a.yrow[orow];
+        }
+        if (!GATED && a.heads) {
+#pragma unroll
+            for (int n = 0; n < FN; n++) {
+                const int col = c0 + wn * 16 * FN + 16 * n + 4 * g;
+                if (col >= a.N) continue;  // (N is whole runs)
+                typename E::T v[4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[r] = (typename E::T)acc[n][m][r];
+                typename E::T *hp = (typename E::T *)a.heads + (size_t)(col / a.head_w) * a.head_stride + (size_t)orow * a.head_row + col % a.head_w;
+                __builtin_memcpy(__builtin_assume_aligned(hp, 4 * sizeof(typename E::T)), v, sizeof v);
+            }
+        } else if (!GATED || partial) {
+#pragma unroll
+            for (int n = 0; n < FN; n++) {
+                const int col = (GATED ? 2 * c0 : c0) + wn * 16 * FN + 16 * n + 4 * g;
+                const int lim = GATED ? (int)width : a.N;
+                float *cp = C + (size_t)orow * width + col;
+                if (col + 3 < lim && (width & 3) == 0) {
+                    *(f32x4 *)cp = acc[n][m];
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (col + r < lim) cp[r] = acc[n][m][r];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < FN / 2; q++) {
+                const int col = c0 + wn * 8 * FN + 16 * q + 4 * g;
+                typename E::T v[4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[r] = (typename E::T)a.unit(acc[2 * q][m][r], acc[2 * q + 1][m][r]);
+                typename E::T *ap = (typename E::T *)a.act + (size_t)orow * a.ld_act + col;
+                if (col + 3 < a.N) {  // (activation rows are whole runs of 64 elements: aligned)
+                    __builtin_memcpy(__builtin_assume_aligned(ap, 4 * sizeof(typename E::T)), v, sizeof v);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (col + r < a.N) ap[r] = v[r];
+                }
+            }
+        }
+    }
+}
+
 // BM activation rows x BN weight rows a workgroup of four waves (2 x 2), k in stages of 128 bytes through two LDS
 // buffers: the next stage travels global -> LDS (asynchronous 16-byte loads) while the current one is multiplied.
 // Chunk c of row r sits at position c ^ (r & 7) of its 128-byte LDS row: the 16 rows a fragment read touches then
@@ -532,60 +592,97 @@ __global__ __launch_bounds__(256) void dense_gemm(DenseGemm a) {
                 for (int m = 0; m < FM; m++) acc[n][m] = E::mma(fw[n], fa[m], acc[n][m]);
         }
     }
-    const bool partial = a.splits > 1;
-    const size_t width = partial ? gemm_partial_width(a.N, GATED) : a.ldc;
-    float *C = a.C + (partial ? (size_t)blockIdx.y * a.M * width : 0);
+    dense_gemm_store<E, FM, FN, GATED, GROUPED>(a, acc, m0 + wm * (BM / 2), row_lo, rows_here, c0, wn);
+}
+
+// The same product in bfloat16 for some hundred rows and more: 256 activation rows x BN weight rows a workgroup of eight waves (4 x 2).  The next
+// stage travels while one is multiplied, and a wave reads its operands of a half of 64 bytes while it multiplies the half before.  Bound:
+// copies to LDS, some 20 clocks of address work a KB (64-byte pieces of a row took 41), where 128 x 128 tiles need 640 clocks of it for 512 of
+// matrix instructions and 256 x 256 ones 1280 for 2048.  512 rows, gate and up 24576 x 4096: 143 -> 99 us (256 x 192; 1040 TFLOP/s); 2000
+// rows, 16384 x 4096: 314 -> 245 us (256 x 256; 1090 TFLOP/s).
+constexpr int dense_wide_lds(int bn) { return 2 * (256 + bn) * 128; }
+template <int BN, bool GATED>
+static __global__ __launch_bounds__(512, 2) void dense_gemm_wide(DenseGemm a) {
+    using E = ElemBf16;
+    constexpr int BM = 256, STAGE = (BM + BN) * 128, FM = 4, FN = BN / 32, CW = BN / 64;
+    extern __shared__ __attribute__((aligned(128))) uint8_t wide_lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 3, wn = wave >> 2, g = lane >> 4, l16 = lane & 15;
+    const int n_tiles = (int)gridDim.x / a.m_tiles;  // as in dense_gemm
+    const int total = a.m_tiles * n_tiles;
+    int id = blockIdx.x;
+    if (total >= 16) {
+        const int q = total / 8, rem = total % 8, x = id % 8, loc = id / 8;
+        id = x * q + min(x, rem) + loc;
+    }
+    const int mt = id % a.m_tiles, nt = id / a.m_tiles;
+    const int m0 = mt * BM, c0 = nt * (GATED ? BN / 2 : BN);
+    const int per_split = (a.stages + a.splits - 1) / a.splits;
+    const int st0 = (int)blockIdx.y * per_split, st1 = min(a.stages, st0 + per_split);
+    // A copy brings eight rows, wave w those from 8 w + 64 i on (GATED: runs of 16 gate rows and the 16 up rows of the same columns).
+    const int chunk = (lane & 7) ^ (lane >> 3);
+    uint32_t va[4], vw[CW];
 #pragma unroll
-    for (int m = 0; m < FM; m++) {
-        const int lr = m0 + wm * (BM / 2) + 16 * m + l16;
-        if (lr >= rows_here) continue;
-        int orow = row_lo + lr;
-        if constexpr (GROUPED) {
-            if (a.yrow && !partial) orow = a.yrow[orow];
-        }
-        if (!GATED && a.heads) {
+    for (int i = 0; i < 4; i++) va[i] = (uint32_t)min(m0 + 64 * i + 8 * wave + (lane >> 3), a.M - 1) * a.lda + 16u * chunk;
 #pragma unroll
-            for (int n = 0; n < FN; n++) {
-                const int col = c0 + wn * (BN / 2) + 16 * n + 4 * g;
-                if (col >= a.N) continue;  // (N is whole runs)
-                typename E::T v[4];
+    for (int i = 0; i < CW; i++) {
+        const int row = 64 * i + 8 * wave + (lane >> 3), col = c0 + (GATED ? row / 32 * 16 + (row & 15) : row);
+        vw[i] = (uint32_t)min(col, a.N - 1) * a.ldw + 16u * chunk;
+    }
+    const uint8_t *W = GATED && (wave & 2) ? a.W2 : a.W;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) const void *)wide_lds) + (uint32_t)wave * 1024u;
+    auto issue = [&](int st, int buf) __attribute__((always_inline)) {
+        const uint8_t *pa = a.A + (size_t)st * 128, *pw = W + (size_t)st * 128;
+        const uint32_t base = lds0 + (uint32_t)(buf * STAGE);
 #pragma unroll
-                for (int r = 0; r < 4; r++) v[r] = (typename E::T)acc[n][m][r];
-                typename E::T *hp = (typename E::T *)a.heads + (size_t)(col / a.head_w) * a.head_stride + (size_t)orow * a.head_row + col % a.head_w;
-                __builtin_memcpy(__builtin_assume_aligned(hp, 4 * sizeof(typename E::T)), v, sizeof v);
+        for (int i = 0; i < 4; i++) dma_chunk16(pa, va[i], base + 8192u * i);
+#pragma unroll
+        for (int i = 0; i < CW; i++) dma_chunk16(pw, vw[i], base + BM * 128u + 8192u * i);
+    };
+    f32x4 acc[FN][FM];
+#pragma unroll
+    for (int n = 0; n < FN; n++)
+#pragma unroll
+        for (int m = 0; m < FM; m++) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint8_t *const la = wide_lds + (wm * 16 * FM + l16) * 128, *const lw = wide_lds + (BM + wn * 16 * FN + l16) * 128;
+    struct Operands { u32x4 a[FM], w[FN]; };
+    auto read = [&](Operands &o, int buf, int kk) __attribute__((always_inline)) {
+        const int at = buf * STAGE + 16 * ((4 * kk + g) ^ (l16 & 7));
+#pragma unroll
+        for (int m = 0; m < FM; m++) o.a[m] = *(const u32x4 *)(la + at + m * 2048);
+#pragma unroll
+        for (int n = 0; n < FN; n++) o.w[n] = *(const u32x4 *)(lw + at + n * 2048);
+    };
+    auto multiply = [&](const Operands &o) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < FN; n++)
+#pragma unroll
+            for (int m = 0; m < FM; m++) acc[n][m] = E::mma(o.w[n], o.a[m], acc[n][m]);
+    };
+    // this wave's copies have landed and its reads are done, and then everyone's
+    auto landed = [&]() __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+    };
+    if (st0 < st1) {
+        Operands o[2];
+        issue(st0, 0);
+        landed();
+        if (st0 + 1 < st1) issue(st0 + 1, 1);
+        read(o[0], 0, 0);
+        for (int st = st0; st < st1; st++) {
+            const int buf = (st - st0) & 1;
+            read(o[1], buf, 1);
+            multiply(o[0]);
+            if (st + 1 < st1) {
+                landed();
+                if (st + 2 < st1) issue(st + 2, buf);
+                read(o[0], buf ^ 1, 0);
             }
-        } else if (!GATED || partial) {
-#pragma unroll
-            for (int n = 0; n < FN; n++) {
-                const int col = (GATED ? 2 * c0 : c0) + wn * (BN / 2) + 16 * n + 4 * g;
-                const int lim = GATED ? (int)width : a.N;
-                float *cp = C + (size_t)orow * width + col;
-                if (col + 3 < lim && (width & 3) == 0) {
-                    *(f32x4 *)cp = acc[n][m];
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        if (col + r < lim) cp[r] = acc[n][m][r];
-                }
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < FN / 2; q++) {
-                const int col = c0 + wn * (BN / 4) + 16 * q + 4 * g;
-                typename E::T v[4];
-#pragma unroll
-                for (int r = 0; r < 4; r++) v[r] = (typename E::T)a.unit(acc[2 * q][m][r], acc[2 * q + 1][m][r]);
-                typename E::T *ap = (typename E::T *)a.act + (size_t)orow * a.ld_act + col;
-                if (col + 3 < a.N) {  // (activation rows are whole runs of 64 elements: aligned)
-                    __builtin_memcpy(__builtin_assume_aligned(ap, 4 * sizeof(typename E::T)), v, sizeof v);
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        if (col + r < a.N) ap[r] = v[r];
-                }
-            }
+            multiply(o[1]);
         }
     }
+    dense_gemm_store<E, FM, FN, GATED, false>(a, acc, m0 + wm * 16 * FM, 0, a.M, c0, wn);
 }
 
 // The partial sums of a product split over k, in order.
