@@ -104,22 +104,22 @@ int launch_wide(const jq::DenseGemm &a, unsigned n_tiles, hipStream_t s) {
 
 // Whether a product runs in tiles of 256 activation rows on workgroups that have a compute unit to themselves (dense_gemm_wide), in how many
 // weight rows and runs of k: where the rounds of 256 workgroups that it takes cost less than the smaller tiles, two or three to a compute
-// unit.  Per stage and round, us: 256 rows 1.9, 192 rows 1.5; 128 x 128 1.22, 64 x 128 0.8, of which a round that is not full takes 0.6
-// at least.  A split adds the writing and reading of its sums at some 6 TB/s.  Measured, smaller / wide, us: gate and up 24576 x 4096 of
-// 512 rows 146 / 99 (192), 16384 x 4096 of 2000 rows 324 / 255, 4096 x 12288 of 2000 rows 257 / 234 (two runs); 16384 x 4096 of 512 rows
-// 93 / 95 and 6144 x 4096 of 512 rows 48 / 50 stay with the smaller ones.
+// unit.  Per stage and round, us, weights from HBM: 256 rows 1.9, 192 rows 1.5; 128 x 128 1.3, 64 x 128 1.13, of which a round that is not
+// full takes 0.6 at least.  A split adds the launch that reads its sums, at some 8 TB/s.  Measured, smaller / wide, us:
+// gate and up 24576 x 4096 of 512 rows 147 / 98 (192, one run), 4096 x 12288 of 512 rows 102 / 65 (256, eight runs), 6144 x 4096 of 512 rows
+// 67 / 52, 16384 x 4096 of 1000 rows 173 / 136 (256), 4096 x 12288 of 2000 rows 258 / 229, 24576 x 4096 of 140 rows 76 / 68.
 struct WidePick {
     int bn = 0, splits = 1;
 };
 WidePick wide_pick(const jq::DenseGemm &a, size_t wrows, int bm, size_t tiles, int splits) {
-    auto sums = [&](size_t s) { return s > 1 ? 4.0 + (2.0 * s + 1.0) * a.M * (double)wrows * 4e-6 / 6.0 : 0.0; };
+    auto sums = [&](size_t s) { return s > 1 ? 3.0 + (s + 1.0) * a.M * (double)wrows * 4e-6 / 8.0 : 0.0; };
     auto stages = [&](size_t s) { return (double)((a.stages + s - 1) / s); };
     const double rounds = (double)(tiles * splits) / (bm == 128 ? 512 : 768), part = rounds - std::floor(rounds);
-    double best = 0.95 * ((std::floor(rounds) + (part > 0 ? 0.6 + 0.4 * part : 0.0)) * stages(splits) * (bm == 128 ? 1.22 : 0.8) + sums(splits));
+    double best = 0.95 * ((std::floor(rounds) + (part > 0 ? 0.6 + 0.4 * part : 0.0)) * stages(splits) * (bm == 128 ? 1.3 : 1.13) + sums(splits));
     WidePick pick;
     for (const int bn : {256, 192}) {
         const size_t t = (size_t)((a.M + 255) / 256) * ((wrows + bn - 1) / bn);
-        const size_t most = a.heads ? 1 : std::max<size_t>(1, std::min<size_t>(256 / t, (size_t)a.stages / 16));
+        const size_t most = std::max<size_t>(1, std::min<size_t>(256 / t, (size_t)a.stages / 16));
         for (const size_t s : {(size_t)1, most}) {
             const double us = (double)((t * s + 255) / 256) * (stages(s) * (bn == 256 ? 1.9 : 1.5) + 6.0) + sums(s);
             if (us < best) best = us, pick = {bn, (int)s};
@@ -152,9 +152,9 @@ int run_gemm(uint32_t type, jq::DenseGemm a, size_t rows_of_a, size_t k, size_t 
     }
     WidePick wide;
     if constexpr (!GROUPED) {
-        if (type == JQ_TYPE_BF16 && bn == 128) {
+        if (type == JQ_TYPE_BF16 && bn == 128 && !a.heads) {
             const auto u = tiles(bm, bn);
-            wide = wide_pick(a, wrows, bm, u.first * u.second, a.heads ? 1 : gemm_splits(u.first * u.second, a.stages));
+            wide = wide_pick(a, wrows, bm, u.first * u.second, gemm_splits(u.first * u.second, a.stages));
         }
     }
     if (wide.bn) bm = 256, bn = wide.bn;
@@ -187,7 +187,7 @@ int run_gemm(uint32_t type, jq::DenseGemm a, size_t rows_of_a, size_t k, size_t 
     } else {
         launch_gemm<jq::ElemF32, 64, 64, GATED, GROUPED>(a, (unsigned)t.second, s);
     }
-    note_kernel(a.splits > 1 ? "dense_gemm+splitk" : "dense_gemm");
+    note_kernel(wide.bn ? (a.splits > 1 ? "dense_gemm_wide+splitk" : "dense_gemm_wide") : a.splits > 1 ? "dense_gemm+splitk" : "dense_gemm");
     if (a.splits > 1) {
         const size_t total = (size_t)a.M * a.N;
         if (GATED)

@@ -1,0 +1,40 @@
+"""Products with plain bf16 rows in tiles of 256 activation rows (one workgroup a compute unit): one run of k and several, row and column counts
+at the edges of the tiles and within them, alone and in a gated feed-forward block."""
+import numpy as np
+import pytest
+
+from joshua_amd import capi
+from joshua_amd.synth import layered as sl
+from joshua_amd.synth import normal
+from tests import layered_cases as lc
+from tests.layered_cases import build, check, feed, tokens
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (512, 4096, 4096, "dense_gemm_wide+splitk"),
+    (449, 6141, 4090, "dense_gemm_wide+splitk"),     # the last row tile of 193 rows; columns and k within a tile and a stage
+    (257, 24575, 2048, "dense_gemm_wide"),           # one row more than a tile
+    (1985, 7681, 2090, "dense_gemm_wide"),           # a column tile of one column
+    (512, 16000, 4096, "dense_gemm"),                # two full rounds of the smaller tiles
+])
+def test_products_of_many_rows(m, n, k, kernel):
+    """Against 64 bits on the operands as the matrix cores take them; f32 sums of k exact products, 2^-24 of the terms' magnitudes
+    for each of some tens of roundings of a sum's size."""
+    w, x = sl.to_bf16(normal(1, (n, k), k ** -0.5)), normal(2, (m, k))
+    got = capi.Weight.upload(capi.BF16, w, n, k).matmul_t(m, x)
+    assert capi.last_kernel() == kernel
+    rows = sorted({r for r in (0, 1, 17, 100, 127, 128, 192, 254, 255, 256, 257, 300, m - 2, m - 1) if r < m})
+    x, w = sl.from_bf16(sl.to_bf16(x[rows])).astype(np.float64), sl.from_bf16(w).astype(np.float64)
+    scale = np.abs(x) @ np.abs(w).T
+    assert np.all(np.abs(got[rows] - x @ w.T) <= 2e-6 * scale + 1e-7)
+
+
+@pytest.mark.parametrize("ff", [12283, 4096])
+def test_gated_block_of_many_rows(tmp_path, ff):
+    """A feed-forward block whose gate and up rows run in one launch, whole and in runs of k."""
+    cfg = lc.model(2048 if ff > 10000 else 4096, 40, [lc.dense(lc.mamba(16, 2, 2, 2), ff, limit=0.4)])
+    m, o, _ = build(tmp_path, cfg, 21, lc.BF16, n_ctx=512)
+    toks = tokens(cfg, 22, 500)
+    check(feed(m, toks, []), o.forward(toks), lc.BF16, "whole", o)
