@@ -405,7 +405,7 @@ __global__ __launch_bounds__(256, 2) void s16_attention(S16Attention a) {
         for (int r = 0; r < 16; r++) o[t][r] = 0.0f;
     bool spoilt = false;                    // the query sees a key that is not finite
     float m_run = -INFINITY, l_run = 0.0f;  // of the lane's query; the sum over this lane's keys only
-    float vref = LATENT ? a.fac[2 * head + 1].y : s16_pow2(-113);  // the scale the outputs are held in: the largest inv.y so far
+    float vref = LATENT ? a.fac[2 * head + 1].y : s16_pow2(-126);  // the scale the outputs are held in: the largest inv.y so far
     const float khead = LATENT ? a.fac[2 * head].y : 1.0f;
 
     // what is known of the tile, asked for with the tile

@@ -33,10 +33,11 @@ __device__ __forceinline__ void s16_split(const float (&x)[8], s16_h8 &hi, s16_h
     }
 }
 
-// The exponent s that puts magnitudes up to `amax` (as float bits, sign cleared) below 2^14; zero, tiny, infinite and NaN
-// maxima are held within +-100, so that no power of two below over- or underflows (a product or quotient of two of them may).
+// The exponent s that puts magnitudes up to `amax` (as float bits, sign cleared) at 2^13 .. 2^14, for every finite one of 2^-113 or more.
+// Below, s stays at 126, from where a magnitude of 2^-126 is still 1; zero, infinite and NaN maxima take the nearest s.  2^s and 2^-s are
+// normal numbers throughout (a product or quotient of two of them may over- or underflow).
 __device__ __forceinline__ int s16_exponent(uint32_t amax_bits) {
-    const int e = min(max((int)(amax_bits >> 23), 40), 240);
+    const int e = min(max((int)(amax_bits >> 23), 14), 254);
     return 13 - (e - 127);
 }
 __device__ __forceinline__ float s16_pow2(int s) { return __builtin_bit_cast(float, (uint32_t)(127 + s) << 23); }

@@ -134,3 +134,18 @@ def test_every_scale_and_rows_of_every_range(qtype, m):
     other = capi.Weight.upload(qtype, raw.reshape(-1), n, k).matmul_t(m, lhs)
     assert not np.isfinite(other[[0, 2]]).any()
     assert np.array_equal(np.delete(other, [0, 2], 0), np.delete(got, [0, 2], 0))
+
+
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("m", [5, 12, 40])
+def test_rows_up_to_the_ends_of_f32(qtype, m):
+    """Activations behind no power of two within 2^100 of 1: each row as exact as one of ordinary size."""
+    n, k = 1040, 2304
+    blocks = synth.normal_quantized(qtype, 5, n * k, 0.01)
+    lhs = synth.normal(6, (m, k))
+    lhs /= np.abs(lhs).max(1, keepdims=True)
+    for i, size in enumerate((1.0, 1e35, 3e36 if qtype == capi.Q4_K else 3e38, 1e-36)):
+        lhs[i] *= np.float32(size)
+    got = check(qtype, blocks, n, k, lhs, rms=None).astype(np.float64)
+    want = lhs.astype(np.float64) @ oracle.dequantize(qtype, blocks).reshape(n, k).astype(np.float64).T
+    assert np.all(np.linalg.norm(got - want, axis=1) <= 3e-7 * np.linalg.norm(want, axis=1))

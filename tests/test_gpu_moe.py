@@ -345,6 +345,21 @@ def test_q4k_experts_on_split_f16_activations_against_64_bits(alike):
     assert err < 6.4e-7, err
 
 
+def test_q4k_experts_on_split_f16_activations_near_the_end_of_f32():
+    """Gated units of up to 1e36 or so are finite, and so is the layer, whose tokens are the powers of two apart that its results are."""
+    h, inter, E, k, T = 512, 512, 64, 4, 300
+    rw, x = synth.normal(660, (E, h), sigma=0.02), synth.normal(661, (T, h))
+    w = [capi.Weight.upload(capi.Q4_K, synth.normal_quantized(capi.Q4_K, 662 + i, E * inter * h, 0.02), E * n, kk)
+         for i, (n, kk) in enumerate(((inter, h), (inter, h), (h, inter)))]
+    cfg = capi.MoeConfig(E, k, h, inter, 0, 1, 0.0, 1, 1, 0.0, 0.0)
+    out = []
+    for by in (2.0 ** 12, 2.0 ** 58):                                 # silu is max(., 0) but for gates of some 2^-8 of the rest
+        out.append(capi.Moe(cfg, rw / np.float32(by), *w).forward(x * np.float32(by)).astype(np.float64) / by ** 2)
+        assert capi.last_kernel() == "moe_split16"
+    assert np.isfinite(out[1]).all()
+    assert np.linalg.norm(out[1] - out[0]) <= 1e-5 * np.linalg.norm(out[0])
+
+
 def test_q4k_experts_on_split_f16_activations_uneven_rows_and_non_finite_ones():
     """300 of 400 tokens route alike (experts with seven tiles, with one, and with none), one token holds a NaN and one an
     infinity: their rows come out NaN and nobody else's; the same layer with a down projection that the int8 GEMM runs."""

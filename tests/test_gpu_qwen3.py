@@ -244,6 +244,24 @@ def test_attention_of_many_tokens_over_values_of_different_size(n_head, n_kv, st
         pos += n
 
 
+@pytest.mark.parametrize("by", [112, -104])
+def test_attention_of_many_tokens_over_values_at_the_ends_of_f32(by):
+    """MXFP4 values 2^by times an ordinary model's behind an output projection of 2^-by: the same logits."""
+    cfg = dict(CFG, n_ctx=256, n_layer=2, head_dim=128, n_head=8, n_kv_head=2, hidden=256)
+    logits = []
+    for b in (0, by):
+        over = {}
+        for i in range(2):
+            for name, n, k, e in (("attn_v", 256, 256, b), ("attn_output", 256, 1024, -b)):
+                raw = np.array(synth.normal_quantized(capi.MXFP4, 70 + i, n * k, 1.0)).view(np.uint8).reshape(-1, 17)
+                raw[:, 0] = raw[:, 0].astype(np.int64) + e
+                over[f"blk.{i}.{name}.weight"] = (capi.MXFP4, raw.reshape(-1))
+        m, _ = make(cfg, 52, override=over)
+        logits.append(np.stack([m.forward(list(range(100, 230)), 0), m.forward(list(range(300, 340)), 130)]))
+    ok, e = close(logits[1], logits[0])
+    assert ok, e
+
+
 def test_attention_of_many_tokens_holds_every_operand_to_more_than_f16():
     """One layer over 200 tokens against 64 bits.  The embeddings are unit vectors, so that queries, keys and values are columns
     of their weights, and the down projection is zero: the error is the attention's and that of the 16-bit activations of the
