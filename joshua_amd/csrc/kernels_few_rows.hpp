@@ -349,8 +349,8 @@ static __global__ __launch_bounds__(512, 2) void few_rows(const uint8_t *__restr
         if constexpr (F::MINS) {  // means of the lane's two sub-blocks
             float sum[2] = {0.0f, 0.0f};
 #pragma unroll
-            for (int i = 0; i < 64; i++) sum[i >> 5] += x[i];
-            const s16_f2 v = {sum[0] * (0.03125f * f), sum[1] * (0.03125f * f)};
+            for (int i = 0; i < 64; i++) sum[i >> 5] = fmaf(x[i], f, sum[i >> 5]);  // (32 of them as they are may exceed f32)
+            const s16_f2 v = {sum[0] * 0.03125f, sum[1] * 0.03125f};
             const s16_h2 h = __builtin_convertvector(v, s16_h2);
             const s16_f2 left = {v[0] - (float)h[0], v[1] - (float)h[1]};
             const s16_h2 l = __builtin_convertvector(left, s16_h2);
@@ -444,8 +444,8 @@ __device__ __forceinline__ void fr_operands(const float (&x)[64], s16_h8 (&hi)[8
     if constexpr (F::MINS) {
         float sum[2] = {0.0f, 0.0f};
 #pragma unroll
-        for (int i = 0; i < 64; i++) sum[i >> 5] += x[i];
-        const s16_f2 v = {sum[0] * (0.03125f * f), sum[1] * (0.03125f * f)};
+        for (int i = 0; i < 64; i++) sum[i >> 5] = fmaf(x[i], f, sum[i >> 5]);  // (32 of them as they are may exceed f32)
+        const s16_f2 v = {sum[0] * 0.03125f, sum[1] * 0.03125f};
         const s16_h2 h = __builtin_convertvector(v, s16_h2);
         const s16_f2 left = {v[0] - (float)h[0], v[1] - (float)h[1]};
         const s16_h2 l = __builtin_convertvector(left, s16_h2);
