@@ -31,6 +31,19 @@ __device__ __forceinline__ void fr_words(const uint8_t *p, uint32_t (&out)[N]) {
     for (int i = 0; i < N; i++) out[i] = __builtin_amdgcn_alignbyte(x[i + 1], x[i], at);
 }
 
+// Where a block of 32 has a scale of its own, those of a super-block may lie further apart than what normal f16 numbers hold exactly,
+// 2^RANGE (of products with subnormal ones a matrix instruction keeps fewer bits: 1.4e-6 off at 2^36).  Then the super-block is
+// multiplied once more for each such range that its scales span: of the blocks whose exponents e0 and e1 (-1: a block of zeros) lie under
+// `below`, put(in0, in1, most) takes the ones within RANGE of the largest, and `below` moves under those.  True where some are left.
+template <int RANGE, class F>
+__device__ __forceinline__ bool fr_level(int e0, int e1, int &below, F put) {
+    e0 = e0 < below ? e0 : -1, e1 = e1 < below ? e1 : -1;
+    const int most = (int)max_xor32(max_xor16((float)max(e0, e1))), least = max(most - RANGE, 0);
+    put(e0 >= least, e1 >= least, most);
+    below = least;
+    return (e0 >= 0 && e0 < least) || (e1 >= 0 && e1 < least);
+}
+
 // A format's side.  Lane (r = lane % 16, g = lane / 16) holds 64 elements of weight row r's super-block, eight for each of its eight
 // k-steps.  QUAD(g, q): the first element of the q-th four that the lane reads of an activation row; AT(s, p): which of those 64 stands
 // at position p of step s.
@@ -39,7 +52,7 @@ __device__ __forceinline__ void fr_words(const uint8_t *p, uint32_t (&out)[N]) {
 // sums cancel: 3.9e-7 off 64 bits instead of 1.6e-7.)
 struct FrQ4K {  // sub-blocks 2 g (low nibbles) and 2 g + 1 (high) of 32 elements
     static constexpr int BLOCK = 144, ALIGN = 16, REAL = 9, PIECES = 9, PLANES = 1;
-    static constexpr bool MINS = true;
+    static constexpr bool MINS = true, LEVELS = false;
     __device__ static int quad(int g, int q) { return 64 * g + 4 * q; }
     static constexpr int at(int s, int p) { return 8 * s + (p & 4) + ((p & 1) << 1 | (p >> 1 & 1)); }
     struct Raw {
@@ -52,7 +65,7 @@ struct FrQ4K {  // sub-blocks 2 g (low nibbles) and 2 g + 1 (high) of 32 element
     s16_h2 sc[2], off[2];
     s16_h8 mins;
     float d, dm;
-    __device__ __forceinline__ void begin(const Raw &r, int g) {
+    __device__ __forceinline__ bool begin(const Raw &r, int g, int &) {
         const uint32_t s4 = (g < 2 ? r.hdr.y & 0x3F3F3F3Fu : (r.hdr.w & 0x0F0F0F0Fu) | ((r.hdr.y >> 2) & 0x30303030u)) >> (16 * (g & 1));
         const uint32_t m4 = (g < 2 ? r.hdr.z & 0x3F3F3F3Fu : ((r.hdr.w >> 4) & 0x0F0F0F0Fu) | ((r.hdr.z >> 2) & 0x30303030u)) >> (16 * (g & 1));
         d = f16_bits(r.hdr.x);
@@ -70,6 +83,7 @@ struct FrQ4K {  // sub-blocks 2 g (low nibbles) and 2 g + 1 (high) of 32 element
         const s16_h2 h = __builtin_convertvector(s16_f2{w[0], w[1]}, s16_h2), l = __builtin_convertvector(s16_f2{w[0] - (float)h[0], w[1] - (float)h[1]}, s16_h2);
         mins = s16_h8{h[0], h[1], h[0], h[1], l[0], l[1], h[0], h[1]};
         dm = 32.0f * __builtin_bit_cast(float, be << 23), d *= 16384.0f;
+        return false;
     }
     template <int S>
     __device__ __forceinline__ void step(const Raw &r, s16_h8 (&p)[1]) const {
@@ -89,7 +103,7 @@ struct FrQ4K {  // sub-blocks 2 g (low nibbles) and 2 g + 1 (high) of 32 element
 
 struct FrQ6K {  // w = d sc (q - 32), an int8 sc for 16 elements: element 128 (g / 2) + 16 (g % 2) + 32 t + i, t = s / 2
     static constexpr int BLOCK = 210, ALIGN = 2, REAL = 14, PIECES = 15, PLANES = 2;
-    static constexpr bool MINS = false;
+    static constexpr bool MINS = false, LEVELS = false;
     __device__ static int quad(int g, int q) { return 128 * (g >> 1) + 16 * (g & 1) + 32 * (q >> 2) + 4 * (q & 3); }
     static constexpr int at(int s, int p) { return FrQ4K::at(s, p); }
     struct Raw {
@@ -105,7 +119,7 @@ struct FrQ6K {  // w = d sc (q - 32), an int8 sc for 16 elements: element 128 (g
     s16_h2 sc[4];
     float d;
     static constexpr float dm = 0.0f;
-    __device__ __forceinline__ void begin(const Raw &r, int g) {
+    __device__ __forceinline__ bool begin(const Raw &r, int g, int &) {
         const uint32_t by = 8 * (uint32_t)(g & 1);
 #pragma unroll
         for (int t = 0; t < 4; t++) {
@@ -114,6 +128,7 @@ struct FrQ6K {  // w = d sc (q - 32), an int8 sc for 16 elements: element 128 (g
             sc[t] = s16_h2{f, f};
         }
         d = f16_bits(r.dd);
+        return false;
     }
     template <int S>
     __device__ __forceinline__ void step(const Raw &r, s16_h8 (&p)[2]) const {
@@ -139,7 +154,7 @@ struct FrQ6K {  // w = d sc (q - 32), an int8 sc for 16 elements: element 128 (g
 
 struct FrQ8_0 {  // w = d q, an f16 d for 32 elements: blocks 2 g and 2 g + 1, 68 bytes.  d' = d 2^e, 2^7 <= the super-block's largest < 2^8
     static constexpr int BLOCK = 272, ALIGN = 16, REAL = 17, PIECES = 17, PLANES = 2;
-    static constexpr bool MINS = false;
+    static constexpr bool MINS = false, LEVELS = true;
     __device__ static int quad(int g, int q) { return 64 * g + 4 * q; }
     static constexpr int at(int s, int p) { return FrQ4K::at(s, p); }
     struct Raw {
@@ -150,19 +165,22 @@ struct FrQ8_0 {  // w = d q, an f16 d for 32 elements: blocks 2 g and 2 g + 1, 6
             for (int i = 0; i < 4; i++) w[i] = *(const s16_u4 *)(b + 68 * g + 16 * i);
             last = *(const uint32_t *)(b + 68 * g + 64);
         }
+        __device__ __forceinline__ void load_far(const uint8_t *b, int g) { load(b, g); }  // from memory
         __device__ __forceinline__ uint32_t word(int i) const { return i == 16 ? last : w[i >> 2][i & 3]; }
     };
     s16_h2 sc[2];
     float d;
     static constexpr float dm = 0.0f;
-    __device__ __forceinline__ void begin(const Raw &r, int) {
+    __device__ __forceinline__ bool begin(const Raw &r, int, int &below) {
         const float d0 = f16_bits(r.word(0)), d1 = f16_bits(r.word(8) >> 16);
-        const float most = max_xor32(max_xor16(fmaxf(mag_or_inf(d0), mag_or_inf(d1))));
-        const int e = 134 - (int)(__builtin_bit_cast(uint32_t, fmaxf(most, 1e-30f)) >> 23);  // (an f16 scale is 2^-24 or more, or zero)
-        const float f = s16_pow2(e);
-        const _Float16 h0 = (_Float16)(d0 * f), h1 = (_Float16)(d1 * f);
-        sc[0] = s16_h2{h0, h0}, sc[1] = s16_h2{h1, h1};
-        d = s16_pow2(-e);
+        const int e0 = s16_abs(d0) ? (int)(s16_abs(d0) >> 23) : -1, e1 = s16_abs(d1) ? (int)(s16_abs(d1) >> 23) : -1;
+        return fr_level<21>(e0, e1, below, [&](bool in0, bool in1, int most) __attribute__((always_inline)) {
+            const int e = 134 - max(most, 100);  // (an f16 scale is 2^-24 or more)
+            const float f = s16_pow2(e);
+            const _Float16 h0 = (_Float16)(in0 ? d0 * f : 0.0f), h1 = (_Float16)(in1 ? d1 * f : 0.0f);
+            sc[0] = s16_h2{h0, h0}, sc[1] = s16_h2{h1, h1};
+            d = s16_pow2(-e);
+        });
     }
     template <int S>
     __device__ __forceinline__ void step(const Raw &r, s16_h8 (&p)[2]) const {
@@ -184,7 +202,7 @@ struct FrQ8_0 {  // w = d q, an f16 d for 32 elements: blocks 2 g and 2 g + 1, 6
 
 struct FrMXFP4 {  // w = 2^(e - 127) E2M1: blocks 2 g and 2 g + 1, 34 bytes; a byte holds elements j (low nibble) and j + 16 of its block
     static constexpr int BLOCK = 136, ALIGN = 8, REAL = 9, PIECES = 9, PLANES = 1;
-    static constexpr bool MINS = false;
+    static constexpr bool MINS = false, LEVELS = true;
     __device__ static int quad(int g, int q) { return 64 * g + 4 * q; }
     static constexpr int at(int s, int p) { return 32 * (s >> 2) + 4 * (s & 3) + (p >> 1) + 16 * (p & 1); }
     struct Raw {
@@ -196,20 +214,23 @@ struct FrMXFP4 {  // w = 2^(e - 127) E2M1: blocks 2 g and 2 g + 1, 34 bytes; a b
             for (int i = 0; i < 8; i++) w[i] = first[i];
             w[8] = *(const uint16_t *)(b + 34 * g + 32);
         }
+        __device__ __forceinline__ void load_far(const uint8_t *b, int g) {  // from memory
+            const uint16_t *h = (const uint16_t *)(b + 34 * g);
+#pragma unroll
+            for (int i = 0; i < 8; i++) w[i] = h[2 * i] | (uint32_t)h[2 * i + 1] << 16;
+            w[8] = h[16];
+        }
         __device__ __forceinline__ uint32_t word(int i) const { return w[i]; }
     };
     float sc[2], d;
     static constexpr float dm = 0.0f;
-    __device__ __forceinline__ void begin(const Raw &r, int) {
+    __device__ __forceinline__ bool begin(const Raw &r, int, int &below) {
         // the scales stand against the super-block's largest, which takes codes to 6 x 2^13; 0xFF: a block of zeros
-        const uint32_t e0 = r.word(0) & 0xFFu, e1 = (r.word(4) >> 8) & 0xFFu;
-        const float m = fmaxf(e0 == 0xFFu ? 0.0f : (float)e0, e1 == 0xFFu ? 0.0f : (float)e1);
-        const int most = (int)max_xor32(max_xor16(m));
-        const auto scale = [&](uint32_t e) __attribute__((always_inline)) {
-            return e == 0xFFu || (int)e < most - 60 ? 0.0f : s16_pow2((int)e - most + 13);
-        };
-        sc[0] = scale(e0), sc[1] = scale(e1);
-        d = ldexpf(1.0f, most - 140);
+        const int e0 = (int)(r.word(0) & 0xFFu), e1 = (int)((r.word(4) >> 8) & 0xFFu);
+        return fr_level<26>(e0 == 0xFF ? -1 : e0, e1 == 0xFF ? -1 : e1, below, [&](bool in0, bool in1, int most) __attribute__((always_inline)) {
+            sc[0] = in0 ? s16_pow2(e0 - most + 13) : 0.0f, sc[1] = in1 ? s16_pow2(e1 - most + 13) : 0.0f;
+            d = ldexpf(1.0f, most - 140);
+        });
     }
     template <int S>
     __device__ __forceinline__ void step(const Raw &r, s16_h8 (&p)[1]) const {
@@ -376,25 +397,28 @@ static __global__ __launch_bounds__(512, 2) void few_rows(const uint8_t *__restr
             }
             __builtin_amdgcn_sched_barrier(0);
             F w;
-            w.begin(raw, g);
-            s16_f4 big = zero, low = zero;
-            auto step = [&](auto sc) __attribute__((always_inline)) {
-                constexpr int S = decltype(sc)::value;
-                s16_h8 p[F::PLANES];
-                w.template step<S>(raw, p);
-                big = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[S], p[0], big, 0, 0, 0);
-                if constexpr (!BOTH) low = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[S], p[0], low, 0, 0, 0);
-                if constexpr (F::PLANES == 2) low = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[S], p[1], low, 0, 0, 0);
-            };
-            step(std::integral_constant<int, 0>{}), step(std::integral_constant<int, 1>{}), step(std::integral_constant<int, 2>{});
-            step(std::integral_constant<int, 3>{}), step(std::integral_constant<int, 4>{}), step(std::integral_constant<int, 5>{});
-            step(std::integral_constant<int, 6>{}), step(std::integral_constant<int, 7>{});
-            s16_f4 i2 = zero;
-            if constexpr (F::MINS) i2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xs, w.mins, zero, 0, 0, 0);
+            int below = 256;
+            for (bool left = true; left;) {
+                left = F::LEVELS ? __any(w.begin(raw, g, below)) : w.begin(raw, g, below);
+                s16_f4 big = zero, low = zero;
+                auto step = [&](auto sc) __attribute__((always_inline)) {
+                    constexpr int S = decltype(sc)::value;
+                    s16_h8 p[F::PLANES];
+                    w.template step<S>(raw, p);
+                    big = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[S], p[0], big, 0, 0, 0);
+                    if constexpr (!BOTH) low = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[S], p[0], low, 0, 0, 0);
+                    if constexpr (F::PLANES == 2) low = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[S], p[1], low, 0, 0, 0);
+                };
+                step(std::integral_constant<int, 0>{}), step(std::integral_constant<int, 1>{}), step(std::integral_constant<int, 2>{});
+                step(std::integral_constant<int, 3>{}), step(std::integral_constant<int, 4>{}), step(std::integral_constant<int, 5>{});
+                step(std::integral_constant<int, 6>{}), step(std::integral_constant<int, 7>{});
+                s16_f4 i2 = zero;
+                if constexpr (F::MINS) i2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xs, w.mins, zero, 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float sum = w.d * (big[i] + low[i]);
-                acc[t][i] = fmaf(sx[i], F::MINS ? fmaf(w.dm, i2[i], sum) : sum, acc[t][i]);
+                for (int i = 0; i < 4; i++) {
+                    const float sum = w.d * (big[i] + low[i]);
+                    acc[t][i] = fmaf(sx[i], F::MINS ? fmaf(w.dm, i2[i], sum) : sum, acc[t][i]);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -561,8 +585,12 @@ static __global__ __launch_bounds__(512, 2) void few_rows_many(const uint8_t *__
         if (next != sb) fetch_w(next);
         __builtin_amdgcn_sched_barrier(0);
         F w[NT];
+        bool left = false;  // blocks behind scales too far below the others', multiplied further down
 #pragma unroll
-        for (int t = 0; t < NT; t++) w[t].begin(raw[t], g);
+        for (int t = 0; t < NT; t++) {
+            int below = 256;
+            left |= w[t].begin(raw[t], g, below);
+        }
         constexpr bool APART = NT * MT <= 4;  // the products with the remainders in sums of their own, where registers are left
         s16_f4 sums[NT][MT], low[APART ? NT : 1][APART ? MT : 1];
         s16_h8 xs[MT];
@@ -619,6 +647,46 @@ static __global__ __launch_bounds__(512, 2) void few_rows_many(const uint8_t *__
                     acc[t][j][i] = fmaf(unit[j][i], F::MINS ? fmaf(w[t].dm, i2[i], sum) : sum, acc[t][j][i]);
                 }
             }
+        if constexpr (F::LEVELS) {
+            if (__any(left)) {  // everything read again, so that nothing is kept for it
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    typename F::Raw far;
+                    far.load_far(first + (size_t)min(16 * t + r, n - 1 - n0) * row_bytes + (size_t)sb * F::BLOCK, g);
+                    F v;
+                    int below = 256;
+                    bool more = __any(v.begin(far, g, below));  // (the turn above)
+                    while (more) {
+                        more = __any(v.begin(far, g, below));
+                        s16_f4 again[MT];
+                        auto turn = [&](auto sc) __attribute__((always_inline)) {
+                            constexpr int S = decltype(sc)::value;
+                            s16_h8 p[F::PLANES];
+                            v.template step<S>(far, p);
+#pragma unroll
+                            for (int j = 0; j < MT; j++) {
+                                const int at_step = (int)(rec[j] + (uint32_t)sb * FR_REC + 2 * S * S16_FRAG);
+                                const s16_h8 hi = __builtin_bit_cast(s16_h8, __builtin_amdgcn_raw_buffer_load_b128(src, l16, at_step, 0));
+                                const s16_h8 lo = __builtin_bit_cast(s16_h8, __builtin_amdgcn_raw_buffer_load_b128(src, l16, at_step + S16_FRAG, 0));
+                                again[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, p[0], S == 0 ? zero : again[j], 0, 0, 0);
+                                again[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, p[0], again[j], 0, 0, 0);
+                                if constexpr (F::PLANES == 2) again[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, p[1], again[j], 0, 0, 0);
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
+                        };
+                        turn(std::integral_constant<int, 0>{}), turn(std::integral_constant<int, 1>{}), turn(std::integral_constant<int, 2>{});
+                        turn(std::integral_constant<int, 3>{}), turn(std::integral_constant<int, 4>{}), turn(std::integral_constant<int, 5>{});
+                        turn(std::integral_constant<int, 6>{}), turn(std::integral_constant<int, 7>{});
+#pragma unroll
+                        for (int j = 0; j < MT; j++)
+#pragma unroll
+                            for (int i = 0; i < 4; i++) acc[t][j][i] = fmaf(unit[j][i], v.d * again[j][i], acc[t][j][i]);
+                    }
+                }
+#pragma unroll
+                for (int s = 0; s < AHEAD; s++) load(next, s);
+            }
+        }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();

@@ -149,3 +149,24 @@ def test_rows_up_to_the_ends_of_f32(qtype, m):
     got = check(qtype, blocks, n, k, lhs, rms=None).astype(np.float64)
     want = lhs.astype(np.float64) @ oracle.dequantize(qtype, blocks).reshape(n, k).astype(np.float64).T
     assert np.all(np.linalg.norm(got - want, axis=1) <= 3e-7 * np.linalg.norm(want, axis=1))
+
+
+@pytest.mark.parametrize("qtype", [capi.Q8_0, capi.MXFP4])
+@pytest.mark.parametrize("m,k,n", [(5, 2304, 1040), (12, 2304, 1040), (16, 2048, 12289), (40, 2304, 1040), (127, 2304, 1055)])
+def test_blocks_whose_scales_lie_far_below_their_neighbours(qtype, m, k, n):
+    """Block j of every super-block behind the j-th of eight scales up to 2^190 (MXFP4) or 2^38 apart, activation row i zero but for one block
+    each: as exact as if that were alone, on either side of what one f16 operand holds (2^26 and 2^21)."""
+    if qtype == capi.MXFP4:
+        raw = np.array(synth.normal_quantized(qtype, 5, n * k, 0.02)).view(np.uint8).reshape(n, k // 256, 8, 17)
+        raw[..., 0] = [200, 173, 174, 127, 90, 40, 199, 10]
+    else:
+        raw = np.array(synth.normal_quantized(qtype, 5, n * k, 0.02)).view(np.uint8).reshape(n, k // 256, 8, 34)
+        d = np.random.default_rng(6).uniform(1, 2, (n, k // 256, 8)) * 2.0 ** np.array([14, -7, -8, -14, -18, 0, 13, -23])
+        raw[..., :2] = d.astype(np.float16)[..., None].view(np.uint8)
+    lhs = synth.normal(7, (m, k)).reshape(m, k // 256, 8, 32)
+    lhs = np.where(np.arange(8)[:, None] == np.arange(m)[:, None, None, None] % 8, lhs, np.float32(0)).reshape(m, k)
+    blocks = raw.reshape(-1)
+    got = capi.Weight.upload(qtype, blocks, n, k).matmul_t(m, lhs).astype(np.float64)
+    assert capi.last_arithmetic() == "f16 pairs"
+    want = lhs.astype(np.float64) @ oracle.dequantize(qtype, blocks).reshape(n, k).astype(np.float64).T
+    assert np.all(np.linalg.norm(got - want, axis=1) <= 3e-7 * np.linalg.norm(want, axis=1))
