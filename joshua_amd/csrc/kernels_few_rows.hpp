@@ -52,7 +52,7 @@ __device__ __forceinline__ bool fr_level(int e0, int e1, int &below, F put) {
 // sums cancel: 3.9e-7 off 64 bits instead of 1.6e-7.)
 struct FrQ4K {  // sub-blocks 2 g (low nibbles) and 2 g + 1 (high) of 32 elements
     static constexpr int BLOCK = 144, ALIGN = 16, REAL = 9, PIECES = 9, PLANES = 1;
-    static constexpr bool MINS = true, LEVELS = false;
+    static constexpr bool MINS = true, LEVELS = false, UP = false;
     __device__ static int quad(int g, int q) { return 64 * g + 4 * q; }
     static constexpr int at(int s, int p) { return 8 * s + (p & 4) + ((p & 1) << 1 | (p >> 1 & 1)); }
     struct Raw {
@@ -103,7 +103,7 @@ struct FrQ4K {  // sub-blocks 2 g (low nibbles) and 2 g + 1 (high) of 32 element
 
 struct FrQ6K {  // w = d sc (q - 32), an int8 sc for 16 elements: element 128 (g / 2) + 16 (g % 2) + 32 t + i, t = s / 2
     static constexpr int BLOCK = 210, ALIGN = 2, REAL = 14, PIECES = 15, PLANES = 2;
-    static constexpr bool MINS = false, LEVELS = false;
+    static constexpr bool MINS = false, LEVELS = false, UP = false;
     __device__ static int quad(int g, int q) { return 128 * (g >> 1) + 16 * (g & 1) + 32 * (q >> 2) + 4 * (q & 3); }
     static constexpr int at(int s, int p) { return FrQ4K::at(s, p); }
     struct Raw {
@@ -154,7 +154,7 @@ struct FrQ6K {  // w = d sc (q - 32), an int8 sc for 16 elements: element 128 (g
 
 struct FrQ8_0 {  // w = d q, an f16 d for 32 elements: blocks 2 g and 2 g + 1, 68 bytes.  d' = d 2^e, 2^7 <= the super-block's largest < 2^8
     static constexpr int BLOCK = 272, ALIGN = 16, REAL = 17, PIECES = 17, PLANES = 2;
-    static constexpr bool MINS = false, LEVELS = true;
+    static constexpr bool MINS = false, LEVELS = true, UP = false;
     __device__ static int quad(int g, int q) { return 64 * g + 4 * q; }
     static constexpr int at(int s, int p) { return FrQ4K::at(s, p); }
     struct Raw {
@@ -202,7 +202,7 @@ struct FrQ8_0 {  // w = d q, an f16 d for 32 elements: blocks 2 g and 2 g + 1, 6
 
 struct FrMXFP4 {  // w = 2^(e - 127) E2M1: blocks 2 g and 2 g + 1, 34 bytes; a byte holds elements j (low nibble) and j + 16 of its block
     static constexpr int BLOCK = 136, ALIGN = 8, REAL = 9, PIECES = 9, PLANES = 1;
-    static constexpr bool MINS = false, LEVELS = true;
+    static constexpr bool MINS = false, LEVELS = true, UP = true;
     __device__ static int quad(int g, int q) { return 64 * g + 4 * q; }
     static constexpr int at(int s, int p) { return 32 * (s >> 2) + 4 * (s & 3) + (p >> 1) + 16 * (p & 1); }
     struct Raw {
@@ -222,14 +222,14 @@ struct FrMXFP4 {  // w = 2^(e - 127) E2M1: blocks 2 g and 2 g + 1, 34 bytes; a b
         }
         __device__ __forceinline__ uint32_t word(int i) const { return w[i]; }
     };
-    float sc[2], d;
+    float sc[2], d, up;  // (d at most 1, up at least 1: the products behind the activations' unit do not overflow before their sum does)
     static constexpr float dm = 0.0f;
     __device__ __forceinline__ bool begin(const Raw &r, int, int &below) {
         // the scales stand against the super-block's largest, which takes codes to 6 x 2^13; 0xFF: a block of zeros
         const int e0 = (int)(r.word(0) & 0xFFu), e1 = (int)((r.word(4) >> 8) & 0xFFu);
         return fr_level<26>(e0 == 0xFF ? -1 : e0, e1 == 0xFF ? -1 : e1, below, [&](bool in0, bool in1, int most) __attribute__((always_inline)) {
             sc[0] = in0 ? s16_pow2(e0 - most + 13) : 0.0f, sc[1] = in1 ? s16_pow2(e1 - most + 13) : 0.0f;
-            d = ldexpf(1.0f, most - 140);
+            d = ldexpf(1.0f, min(most - 140, 0)), up = ldexpf(1.0f, max(most - 140, 0));
         });
     }
     template <int S>
@@ -417,7 +417,8 @@ static __global__ __launch_bounds__(512, 2) void few_rows(const uint8_t *__restr
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const float sum = w.d * (big[i] + low[i]);
-                    acc[t][i] = fmaf(sx[i], F::MINS ? fmaf(w.dm, i2[i], sum) : sum, acc[t][i]);
+                    if constexpr (F::UP) acc[t][i] = fmaf(sx[i] * sum, w.up, acc[t][i]);
+                    else acc[t][i] = fmaf(sx[i], F::MINS ? fmaf(w.dm, i2[i], sum) : sum, acc[t][i]);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -644,7 +645,8 @@ static __global__ __launch_bounds__(512, 2) void few_rows_many(const uint8_t *__
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const float sum = w[t].d * sums[t][j][i];
-                    acc[t][j][i] = fmaf(unit[j][i], F::MINS ? fmaf(w[t].dm, i2[i], sum) : sum, acc[t][j][i]);
+                    if constexpr (F::UP) acc[t][j][i] = fmaf(unit[j][i] * sum, w[t].up, acc[t][j][i]);
+                    else acc[t][j][i] = fmaf(unit[j][i], F::MINS ? fmaf(w[t].dm, i2[i], sum) : sum, acc[t][j][i]);
                 }
             }
         if constexpr (F::LEVELS) {
@@ -680,7 +682,10 @@ static __global__ __launch_bounds__(512, 2) void few_rows_many(const uint8_t *__
 #pragma unroll
                         for (int j = 0; j < MT; j++)
 #pragma unroll
-                            for (int i = 0; i < 4; i++) acc[t][j][i] = fmaf(unit[j][i], v.d * again[j][i], acc[t][j][i]);
+                            for (int i = 0; i < 4; i++) {
+                                if constexpr (F::UP) acc[t][j][i] = fmaf(unit[j][i] * (v.d * again[j][i]), v.up, acc[t][j][i]);
+                                else acc[t][j][i] = fmaf(unit[j][i], v.d * again[j][i], acc[t][j][i]);
+                            }
                     }
                 }
 #pragma unroll

@@ -170,3 +170,16 @@ def test_blocks_whose_scales_lie_far_below_their_neighbours(qtype, m, k, n):
     assert capi.last_arithmetic() == "f16 pairs"
     want = lhs.astype(np.float64) @ oracle.dequantize(qtype, blocks).reshape(n, k).astype(np.float64).T
     assert np.all(np.linalg.norm(got - want, axis=1) <= 3e-7 * np.linalg.norm(want, axis=1))
+
+
+@pytest.mark.parametrize("m", [5, 12, 40])
+@pytest.mark.parametrize("scale,size", [(240, 1e-30), (250, 1e-36), (5, 1e35)])
+def test_mxfp4_scales_at_the_ends_of_their_range(m, scale, size):
+    n, k = 1040, 2304
+    raw = np.array(synth.normal_quantized(capi.MXFP4, 5, n * k, 0.02)).view(np.uint8).reshape(-1, 17)
+    raw[:, 0] = scale
+    lhs = synth.normal(6, (m, k)) * np.float32(size)
+    got = capi.Weight.upload(capi.MXFP4, raw.reshape(-1), n, k).matmul_t(m, lhs).astype(np.float64)
+    assert capi.last_arithmetic() == "f16 pairs"
+    want = lhs.astype(np.float64) @ oracle.dequantize(capi.MXFP4, raw.reshape(-1)).reshape(n, k).astype(np.float64).T
+    assert np.linalg.norm(got - want) <= 3e-7 * np.linalg.norm(want)
