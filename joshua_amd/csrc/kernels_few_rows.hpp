@@ -7,7 +7,8 @@
 // tile's sums over 32 elements are two v_mfma_f32_16x16x32_f16, or three (the remainders with each other are below 2^-22): exact
 // products, f32 sums.  Up to eight rows need half of the instructions' 16 rows: there the others take the second numbers.
 //
-// Off 64 bits 0.9e-7 (MXFP4) to 1.5e-7 (relative 2-norm; the f32 row kernels 1.3e-7 to 2.4e-7, the int8 GEMM 2.7e-5, 3.7e-5 for Q8_0).
+// Off 64 bits, relative 2-norm, rows of 2048 to 12288: 0.75e-7 to 0.9e-7 (MXFP4), 1.1e-7 to 1.3e-7 (the f32 row kernels 1.2e-7 to 2.6e-7, the
+// int8 GEMM 2.7e-5, 3.7e-5 for Q8_0).
 // Bound: the issue of vector instructions (a super-block of 16 weight rows takes 190 (Q4_K), 280 (Q6_K), 210 (Q8_0) or 90 (MXFP4),
 // its activations 300 a workgroup) and, at the smallest sizes, one trip to memory.  us, 16 rows, before / now:
 //   14336 x 4096   Q6_K 42 / 22     Q8_0 43 / 20     MXFP4 41 / 14
@@ -51,7 +52,7 @@ __device__ __forceinline__ bool fr_level(int e0, int e1, int &below, F put) {
 // in two f16 numbers h + l behind a power of two, against the activations' mean there in three.  (With the codes as they are the two
 // sums cancel: 3.9e-7 off 64 bits instead of 1.6e-7.)
 struct FrQ4K {  // sub-blocks 2 g (low nibbles) and 2 g + 1 (high) of 32 elements
-    static constexpr int BLOCK = 144, ALIGN = 16, REAL = 9, PIECES = 9, PLANES = 1;
+    static constexpr int BLOCK = 144, ALIGN = 16, REAL = 9, PIECES = 9, PLANES = 1, CHAINS = 1;
     static constexpr bool MINS = true, LEVELS = false, UP = false;
     __device__ static int quad(int g, int q) { return 64 * g + 4 * q; }
     static constexpr int at(int s, int p) { return 8 * s + (p & 4) + ((p & 1) << 1 | (p >> 1 & 1)); }
@@ -102,7 +103,7 @@ struct FrQ4K {  // sub-blocks 2 g (low nibbles) and 2 g + 1 (high) of 32 element
 };
 
 struct FrQ6K {  // w = d sc (q - 32), an int8 sc for 16 elements: element 128 (g / 2) + 16 (g % 2) + 32 t + i, t = s / 2
-    static constexpr int BLOCK = 210, ALIGN = 2, REAL = 14, PIECES = 15, PLANES = 2;
+    static constexpr int BLOCK = 210, ALIGN = 2, REAL = 14, PIECES = 15, PLANES = 2, CHAINS = 1;
     static constexpr bool MINS = false, LEVELS = false, UP = false;
     __device__ static int quad(int g, int q) { return 128 * (g >> 1) + 16 * (g & 1) + 32 * (q >> 2) + 4 * (q & 3); }
     static constexpr int at(int s, int p) { return FrQ4K::at(s, p); }
@@ -154,6 +155,7 @@ struct FrQ6K {  // w = d sc (q - 32), an int8 sc for 16 elements: element 128 (g
 
 struct FrQ8_0 {  // w = d q, an f16 d for 32 elements: blocks 2 g and 2 g + 1, 68 bytes.  d' = d 2^e, 2^7 <= the super-block's largest < 2^8
     static constexpr int BLOCK = 272, ALIGN = 16, REAL = 17, PIECES = 17, PLANES = 2;
+    static constexpr int CHAINS = 2;  // of four matrix instructions each in few_rows, not one of eight: 1.28e-7 -> 1.10e-7, see fr_wave_sums
     static constexpr bool MINS = false, LEVELS = true, UP = false;
     __device__ static int quad(int g, int q) { return 64 * g + 4 * q; }
     static constexpr int at(int s, int p) { return FrQ4K::at(s, p); }
@@ -201,7 +203,7 @@ struct FrQ8_0 {  // w = d q, an f16 d for 32 elements: blocks 2 g and 2 g + 1, 6
 };
 
 struct FrMXFP4 {  // w = 2^(e - 127) E2M1: blocks 2 g and 2 g + 1, 34 bytes; a byte holds elements j (low nibble) and j + 16 of its block
-    static constexpr int BLOCK = 136, ALIGN = 8, REAL = 9, PIECES = 9, PLANES = 1;
+    static constexpr int BLOCK = 136, ALIGN = 8, REAL = 9, PIECES = 9, PLANES = 1, CHAINS = 1;
     static constexpr bool MINS = false, LEVELS = true, UP = true;
     __device__ static int quad(int g, int q) { return 64 * g + 4 * q; }
     static constexpr int at(int s, int p) { return 32 * (s >> 2) + 4 * (s & 3) + (p >> 1) + 16 * (p & 1); }
@@ -274,8 +276,23 @@ __device__ __forceinline__ void fr_split(const float (&x)[8], float f_hi, float 
 template <int N>
 __device__ __forceinline__ void fr_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
+extern __shared__ __attribute__((aligned(16))) uint8_t fr_lds[];
+
+// The i-th of the `stride` sums that each wave of a workgroup left in LDS, of up to eight waves, in pairs: three roundings of a sum's size, not
+// fifteen (Q8_0, five rows of 2048: 1.40e-7 -> 1.28e-7 off 64 bits; the f32 row kernel 1.22e-7).
+__device__ __forceinline__ s16_f4 fr_wave_sums(int i, int stride, int waves) {
+    const s16_f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    s16_f4 s[8];
+#pragma unroll
+    for (int w = 0; w < 8; w++) {
+        const s16_f4 v = *(const s16_f4 *)(fr_lds + (min(w, waves - 1) * stride + i) * 16);
+        s[w] = w < waves ? v : zero;
+    }
+    return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
+
 // A workgroup takes 16 NT weight rows; its waves take the super-blocks of a row in turn, each for itself, and add up
-// at the end in wave order.  A wave brings its super-block of the activation rows (ROWS of them, the last one again past the m-th)
+// at the end in pairs.  A wave brings its super-block of the activation rows (ROWS of them, the last one again past the m-th)
 // and of its tiles of 16 weight rows to LDS by asynchronous loads of contiguous pieces: a lane that reads its own share of a row from memory
 // looks up a cache line of its own at every load, two clocks a lane.  A place in LDS is free once its words are in registers, and
 // what the next super-block puts there is asked for at once, so up to a whole super-block of all tiles travels while one is multiplied.
@@ -283,7 +300,6 @@ __device__ __forceinline__ void fr_wait() { asm volatile("s_waitcnt vmcnt(%0)" :
 template <class F, int NT, int ROWS>
 static __global__ __launch_bounds__(512, 2) void few_rows(const uint8_t *__restrict__ W, uint32_t row_bytes, const float *__restrict__ X,
                                                           float *__restrict__ Y, int m, int n, int nb) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t fr_lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
     const int waves = blockDim.x >> 6, n0 = blockIdx.x * 16 * NT, k = 256 * nb;
     constexpr bool EVEN = F::ALIGN == 16;  // blocks start at pieces
@@ -400,12 +416,13 @@ static __global__ __launch_bounds__(512, 2) void few_rows(const uint8_t *__restr
             int below = 256;
             for (bool left = true; left;) {
                 left = F::LEVELS ? __any(w.begin(raw, g, below)) : w.begin(raw, g, below);
-                s16_f4 big = zero, low = zero;
+                s16_f4 big[2] = {zero, zero}, low = zero;
                 auto step = [&](auto sc) __attribute__((always_inline)) {
                     constexpr int S = decltype(sc)::value;
                     s16_h8 p[F::PLANES];
                     w.template step<S>(raw, p);
-                    big = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[S], p[0], big, 0, 0, 0);
+                    constexpr int c = F::CHAINS == 2 ? S & 1 : 0;
+                    big[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[S], p[0], big[c], 0, 0, 0);
                     if constexpr (!BOTH) low = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[S], p[0], low, 0, 0, 0);
                     if constexpr (F::PLANES == 2) low = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[S], p[1], low, 0, 0, 0);
                 };
@@ -416,7 +433,7 @@ static __global__ __launch_bounds__(512, 2) void few_rows(const uint8_t *__restr
                 if constexpr (F::MINS) i2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xs, w.mins, zero, 0, 0, 0);
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float sum = w.d * (big[i] + low[i]);
+                    const float sum = w.d * ((F::CHAINS == 2 ? big[0][i] + big[1][i] : big[0][i]) + low[i]);
                     if constexpr (F::UP) acc[t][i] = fmaf(sx[i] * sum, w.up, acc[t][i]);
                     else acc[t][i] = fmaf(sx[i], F::MINS ? fmaf(w.dm, i2[i], sum) : sum, acc[t][i]);
                 }
@@ -430,11 +447,7 @@ static __global__ __launch_bounds__(512, 2) void few_rows(const uint8_t *__restr
     __syncthreads();
     for (int i = tid; i < NT * 64; i += 64 * waves) {
         if (BOTH && (i & 32)) continue;  // (the second planes' sums, added below)
-        s16_f4 v = zero;
-        for (int w = 0; w < waves; w++) {
-            v += *(const s16_f4 *)(fr_lds + (w * NT * 64 + i) * 16);
-            if constexpr (BOTH) v += *(const s16_f4 *)(fr_lds + (w * NT * 64 + i + 32) * 16);
-        }
+        const s16_f4 v = fr_wave_sums(i, NT * 64, waves) + (BOTH ? fr_wave_sums(i + 32, NT * 64, waves) : zero);
         const int col = n0 + 16 * (i >> 6) + (i & 15), row = 4 * ((i >> 4) & 3);
         if (col < n) {
 #pragma unroll
@@ -516,7 +529,6 @@ constexpr int few_rows_many_lds(int waves, int nt, int mt) {
 template <class F, int NT, int MT, int AHEAD>
 static __global__ __launch_bounds__(512, 2) void few_rows_many(const uint8_t *__restrict__ W, uint32_t row_bytes, const uint8_t *__restrict__ acts,
                                                                float *__restrict__ Y, int m, int n, int nb, int groups, int blocks) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t fr_lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
     const int waves = blockDim.x >> 6, id = blockIdx.x, n0 = (id / 8 / blocks * 8 + id % 8) * 16 * NT, g0 = id / 8 % blocks * MT;
     if (n0 >= n) return;
@@ -701,8 +713,7 @@ static __global__ __launch_bounds__(512, 2) void few_rows_many(const uint8_t *__
         for (int j = 0; j < MT; j++) *(s16_f4 *)(fr_lds + ((wave * NT * MT + t * MT + j) * 64 + lane) * 16) = acc[t][j];
     __syncthreads();
     for (int i = tid; i < NT * MT * 64; i += 64 * waves) {
-        s16_f4 v = zero;
-        for (int w = 0; w < waves; w++) v += *(const s16_f4 *)(fr_lds + (w * NT * MT * 64 + i) * 16);
+        const s16_f4 v = fr_wave_sums(i, NT * MT * 64, waves);
         const int t = (i >> 6) / MT, j = (i >> 6) % MT, col = n0 + 16 * t + (i & 15), row = 16 * (g0 + j) + 4 * ((i >> 4) & 3);
         if (col < n) {
 #pragma unroll

@@ -12,6 +12,7 @@ from joshua_amd import capi, synth
 pytestmark = pytest.mark.gpu
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ON = not os.environ.get("JQ_FEW_ROWS", "1").startswith("0")
 TYPES = [capi.Q4_K, capi.Q6_K, capi.Q8_0, capi.MXFP4]
 
 
@@ -183,3 +184,18 @@ def test_mxfp4_scales_at_the_ends_of_their_range(m, scale, size):
     assert capi.last_arithmetic() == "f16 pairs"
     want = lhs.astype(np.float64) @ oracle.dequantize(capi.MXFP4, raw.reshape(-1)).reshape(n, k).astype(np.float64).T
     assert np.linalg.norm(got - want) <= 3e-7 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("qtype,bound", [(capi.Q8_0, 1.22e-7), (capi.Q6_K, 1.53e-7), (capi.MXFP4, 1.20e-7)])
+@pytest.mark.parametrize("m", [2, 5, 12])
+def test_no_further_off_than_the_f32_row_kernels(qtype, bound, m):
+    """Rows of 2048, where those have the fewest roundings; the bound is what they lie off on the same inputs."""
+    n, k = 2048, 2048
+    err = ref = 0.0
+    for seed in range(4):
+        blocks, lhs = synth.normal_quantized(qtype, 90 + seed, n * k, 0.02), synth.normal(95 + seed, (m, k))
+        got = capi.Weight.upload(qtype, blocks, n, k).matmul_t(m, lhs)
+        assert capi.last_arithmetic() == ("f16 pairs" if ON else "")
+        want = lhs.astype(np.float64) @ oracle.dequantize(qtype, blocks).reshape(n, k).astype(np.float64).T
+        err, ref = err + ((got - want) ** 2).sum(), ref + (want ** 2).sum()
+    assert np.sqrt(err / ref) <= bound, np.sqrt(err / ref)
