@@ -41,7 +41,7 @@
 // behind.  E2M1 codes of p, a third less to read, would be 2.6e-5 off 64 bits.  The codes' scales cost 1.3 us of a call.
 // MXFP4 has no mins and no codes to make: behind the super-block's largest scale a weight is exact in f16, made by one conversion for
 // two, and E2M1, what the second instruction multiplies, is its code as it stands in memory, on the block's own scale.  512 x 14336 x
-// 4096: 112 -> 87 us a call, 333 x 4096 x 12288 109 -> 79, 2048 x 4096 x 12288 427 -> 277; 2.7e-5 -> 0.6e-5 off 64 bits.  Q6_K and Q8_0, whose
+// 4096: 112 -> 87 us a call, 333 x 4096 x 12288 109 -> 79, 2048 x 4096 x 12288 427 -> 277; 2.7e-5 -> 0.57e-5 off 64 bits.  Q6_K and Q8_0, whose
 // weights take 12 and 18 bits, were built here too, the weights' own remainders as E2M1 against the activations as E2M3: no faster
 // than the int8 GEMM (512 x 14336 x 4096 148 and 143 us against 128 and 130; unpacking twice Q4_K's instructions, and registers for six groups).
 #pragma once
@@ -140,8 +140,21 @@ static __global__ __launch_bounds__(128) void kq_gemm_h6_prep(const float *__res
     // the power of two that takes the largest magnitude to 2^14 .. 2^15; exact unless the result is below f32's normal range
     const uint32_t e = min(max(__builtin_bit_cast(uint32_t, amax) >> 23, 15u), 254u);
     const bool live = amax < INFINITY;
-    const float inv = live ? __builtin_bit_cast(float, (268u - e) << 23) : 0.0f;
-    const float s = !live ? NAN : amax > 0.0f ? __builtin_bit_cast(float, (e - 14u) << 23) : 0.0f;
+    float inv = live ? __builtin_bit_cast(float, (268u - e) << 23) : 0.0f;
+    float s = !live ? NAN : amax > 0.0f ? __builtin_bit_cast(float, (e - 14u) << 23) : 0.0f;
+    if constexpr (!MINS) {
+        // What takes the largest to 2^15 itself suits f16 and E2M3 better: magnitudes that are all alike, or few binary fractions of the largest,
+        // come out whole (6e-6 off behind the power of two), normal ones 5.7e-6 off for 6.1e-6.  But not where f16 holds every element
+        // behind the power of two, as it does those of bf16 activations.
+        __shared__ bool whole_sh[2][16];
+        bool whole = true;
+#pragma unroll
+        for (int q = 0; q < 32; q++) whole &= (float)(_Float16)(v[q] * inv) == v[q] * inv;
+        const uint64_t all = __ballot(whole), row_lanes = 0x0001000100010001ull << i;
+        if (g == 0) whole_sh[h][i] = (all & row_lanes) == row_lanes;
+        __syncthreads();
+        if (live && amax >= 0x1p-100f && !(whole_sh[0][i] && whole_sh[1][i])) inv = 32768.0f / amax, s = amax * 0x1p-15f;
+    }
     float sum = 0.0f;
     h6_h32 hi, lo;
 #pragma unroll

@@ -267,3 +267,23 @@ def test_mxfp4_on_f16_and_its_own_codes(shape, splits):
     env = dict(os.environ, JQ_GEMM_H6_SHAPE=shape, JQ_GEMM_H6_SPLITS=str(splits), JQ_GEMM_H6_MIN_M="17")
     res = subprocess.run([sys.executable, "-c", MX_CHILD.replace("ROOT", repr(ROOT), 1)], env=env, capture_output=True, text=True, timeout=110)
     assert res.returncode == 0 and "h6 ok" in res.stdout, res.stdout + res.stderr
+
+
+@pytest.mark.parametrize("m,k,n", [(200, 4096, 4096), (333, 2304, 2112)])
+def test_mxfp4_activations_that_few_bits_hold(m, k, n):
+    """Magnitudes that are all alike, one element in 256, the largest's halves and quarters, bf16 values: held whole, so the products lie f32
+    roundings off; normal ones as far as f16 and an E2M3 remainder are (8 s for s = 2^-14 of the largest, s / 2 off)."""
+    blocks, rng = synth.normal_quantized(capi.MXFP4, 80, n * k, 0.02), np.random.default_rng(81)
+    w, d = capi.Weight.upload(capi.MXFP4, blocks, n, k), oracle.dequantize(capi.MXFP4, blocks).reshape(n, k).astype(np.float64)
+    normal = rng.standard_normal((m, k)).astype(np.float32)
+    one = np.zeros((m, k), np.float32)
+    one[:, 77::256] = normal[:, 77::256]
+    size = rng.uniform(0.5, 2, (m, 1)).astype(np.float32)
+    for what, x, bound in (("alike", np.sign(normal) * size, 2e-7), ("one", one, 2e-7),
+                           ("halves", np.sign(normal) * size * rng.choice([1.0, 0.5, 0.25], (m, k)).astype(np.float32), 2e-7),
+                           ("bf16", (normal.view(np.uint32) & 0xFFFF0000).view(np.float32), 2e-7), ("normal", normal, 7e-6)):
+        got = w.matmul_t(m, np.ascontiguousarray(x, dtype=np.float32))
+        assert capi.last_arithmetic() == "f16+fp6"
+        want = x.astype(np.float64) @ d.T
+        err = np.linalg.norm(got - want) / np.linalg.norm(want)
+        assert err <= bound, (what, err)
