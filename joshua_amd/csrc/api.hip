@@ -909,6 +909,11 @@ int dispatch_gemm_decoded(uint32_t type, const uint8_t *W, size_t row_bytes, con
 // MXFP4 6000 x 5120 10.2 / 18.9; Q6_K 14336 x 11264 43 / 58, but 11008 x 3840 18.6 / 18.0).
 // More rows, Q6_K, Q8_0, MXFP4: against the f32 row kernel, the one-row kernel once a row, the int8 GEMM (14336 x 4096: Q6_K 2 rows
 // 18.9 / 21.6, 16 rows 22 / 42; Q8_0 4 rows 18 / 43; MXFP4 8 rows 12 / 41; 1500 x 2304: 6.3 to 6.8 / 6.2 to 45).
+// Few weight rows: a workgroup takes 16 of them, so its time is that of a row's super-blocks however few they are (one row, 1024 x 4096 to
+// 16384: Q6_K 8 to 24, Q8_0 8 to 21, MXFP4 7 to 18), while the f32 row kernel's grows with both counts of rows.  Where they cross, over 576 to
+// 4096 x 1024 to 16384, weights from memory: Q6_K 2 rows 1024 x 4096 8.1 / 4.5, 2048 x 7168 11.9 / 10.6, 3072 x 4096 8.9 / 9.0; 3 rows 1536 x
+// 4096 8.6 / 8.1; 5 rows 1024 x 16384 24.6 / 23.9.  Q8_0 1 row 1024 x 12288 16.6 / 9.4, 2048 x 7168 10.9 / 10.5; 2 rows 1024 x 4096 7.8 /
+// 6.1, 2048 x 12288 17.2 / 13.9 (the one-row kernel twice).  MXFP4 1 row 1024 x 16384 17.8 / 14.4; 2 rows 1024 x 2048 5.2 / 4.7.
 // Q4_K: two rows are faster on the one-row kernels' up to 64M weights (11008 x 3840 13.4 / 12.2, 14336 x 11264 28 / 47).  More:
 // rows that are no multiple of 4096 long 10 to 40 / 11 to 134; the others have dispatch_q4k_rows16, whose time does not grow with the
 // rows (4096 x 4096: 7.4 to 8.8 / 9.3; 14336 x 4096: 12.7 to 17 / 14.6; 4096 x 12288: 16 to 20 / 23; 12000 x 8192: 21 to 29 / 24).
@@ -937,9 +942,14 @@ bool few_rows_better(uint32_t type, size_t m, size_t k, size_t n) {
         if (m == 1 || n < 1024 || k < 1024) return false;
         if (m == 2) return weights >= ((size_t)64 << 20) && k != 4096;
         return k % 4096 != 0 || k > 4 * 4096 || (m <= 8 ? k > 4096 || n <= 8192 : n <= 4096);
-    case JQ_TYPE_Q6_K: return weights >= (m == 1 ? (size_t)64 << 20 : (size_t)2 << 20);
-    case JQ_TYPE_Q8_0: return weights >= (m == 1 ? (size_t)8 << 20 : (size_t)2 << 20);
-    case JQ_TYPE_MXFP4: return weights >= (m == 1 ? (size_t)16 << 20 : (size_t)2 << 20);
+    case JQ_TYPE_Q6_K: return weights >= (m == 1 ? (size_t)64 << 20 : (size_t)2 << 20) && n >= (m <= 2 ? 3072 : m == 3 ? 2048 : m == 4 || (m == 5 && k % 4096 == 0) ? 1280 : 1);
+    case JQ_TYPE_Q8_0:
+        if (m == 1) return weights >= ((size_t)8 << 20) && n >= 2560;
+        if (m == 2) return weights > ((size_t)2 << 20) && n >= (k % 4096 == 0 && k <= 12288 && k > 4096 ? 2560 : 1280);
+        return m == 3 ? weights > ((size_t)2 << 20) : weights >= ((size_t)2 << 20);
+    case JQ_TYPE_MXFP4:
+        if (m == 1) return weights >= ((size_t)16 << 20) && n >= 1280;
+        return m == 2 ? weights > ((size_t)2 << 20) : weights >= ((size_t)2 << 20);
     default: return false;
     }
 }
@@ -990,6 +1000,16 @@ int dispatch_matmul(uint32_t type, const uint8_t *W, size_t row_bytes, const flo
         if (rc >= 0) return rc;
         if (few_rows_better(type, 1, k, n)) rc = few_rows_matmul(type, W, row_bytes, X, Y, 1, k, n, few_rows_name(type, 1, k, n), s);
         if (rc >= 0) return rc;
+    }
+    // Q6_K and Q8_0 with two activation rows against 16M weights or more in fewer rows than few_rows needs: the one-row kernel twice
+    // (2048 x 12288 of Q8_0 13.9 us; few_rows 17.2, the f32 row kernel 25)
+    if ((type == JQ_TYPE_Q6_K || type == JQ_TYPE_Q8_0) && m == 2 && n * k >= ((size_t)16 << 20)) {
+        static const char *no_loop = getenv("JQ_NO_ONE_ROW_LOOP");
+        int rc = no_loop ? -1 : 0;
+        for (size_t r = 0; r < m && rc == 0; r++)
+            rc = type == JQ_TYPE_Q6_K ? dispatch_q6k_dot4(W, row_bytes, X + r * k, Y + r * n, k, n, s)
+                                      : dispatch_q8_0_dot4(W, row_bytes, X + r * k, Y + r * n, k, n, s);
+        if (rc >= 0) return rc;  // (a kernel that declines does so at the first row, before anything is launched)
     }
     // Q4_K with a few activation rows.  Rows of 4096, 1024 weight rows or more: the int8 matrix-core kernel
     // on the one-row kernel's weight stream, in passes of 16 activation rows.  Other row lengths: one or two

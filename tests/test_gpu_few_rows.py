@@ -44,7 +44,7 @@ def check(qtype, blocks, n, k, lhs, rms=3e-7, w=None):
 
 # a tile of 16 weight rows a workgroup, two, four; their ragged ends; rows of 8 to 17 super-blocks over up to 8 waves
 @pytest.mark.parametrize("qtype", TYPES)
-@pytest.mark.parametrize("m,k,n", [(3, 2304, 1025), (4, 2048, 1039), (5, 4352, 1024), (8, 2560, 4097), (9, 2048, 5001), (16, 2304, 8223),
+@pytest.mark.parametrize("m,k,n", [(3, 2304, 2049), (4, 2048, 1295), (5, 4352, 1024), (8, 2560, 4097), (9, 2048, 5001), (16, 2304, 8223),
                                    (16, 2048, 12289), (7, 1280, 12337), (13, 1280, 16399)])
 def test_edges_of_tiles(qtype, m, k, n):
     blocks = synth.normal_quantized(qtype, 5 + n, n * k, 0.02)
@@ -84,7 +84,7 @@ def test_the_call_that_allocates_nothing(qtype, m, k, n, name):
     assert torch.equal(y[0], y[1])
 
 
-@pytest.mark.parametrize("qtype,k,n", [(capi.Q8_0, 5120, 1700), (capi.MXFP4, 4096, 4096), (capi.Q6_K, 7936, 8460)])
+@pytest.mark.parametrize("qtype,k,n", [(capi.Q8_0, 5120, 2561), (capi.MXFP4, 4096, 4096), (capi.Q6_K, 7936, 8460)])
 def test_one_row_that_no_other_kernel_takes(qtype, k, n):
     check(qtype, synth.normal_quantized(qtype, 7, n * k, 0.02), n, k, synth.normal(8, (1, k)))
 
@@ -190,7 +190,7 @@ def test_mxfp4_scales_at_the_ends_of_their_range(m, scale, size):
 @pytest.mark.parametrize("m", [2, 5, 12])
 def test_no_further_off_than_the_f32_row_kernels(qtype, bound, m):
     """Rows of 2048, where those have the fewest roundings; the bound is what they lie off on the same inputs."""
-    n, k = 2048, 2048
+    n, k = 3072, 2048
     err = ref = 0.0
     for seed in range(4):
         blocks, lhs = synth.normal_quantized(qtype, 90 + seed, n * k, 0.02), synth.normal(95 + seed, (m, k))
@@ -199,3 +199,16 @@ def test_no_further_off_than_the_f32_row_kernels(qtype, bound, m):
         want = lhs.astype(np.float64) @ oracle.dequantize(qtype, blocks).reshape(n, k).astype(np.float64).T
         err, ref = err + ((got - want) ** 2).sum(), ref + (want ** 2).sum()
     assert np.sqrt(err / ref) <= bound, np.sqrt(err / ref)
+
+
+@pytest.mark.parametrize("qtype,m,k,n,kernel", [
+    (capi.Q6_K, 2, 4096, 1024, "matmul_rows_staged"), (capi.Q6_K, 3, 4096, 1536, "matmul_rows_staged"), (capi.Q6_K, 5, 12288, 1024, "matmul_rows_staged"),
+    (capi.Q8_0, 1, 9984, 1024, "matmul_rows_staged"), (capi.Q8_0, 2, 4096, 1024, "matmul_rows_staged"), (capi.Q8_0, 2, 12288, 2048, "q8_0_gemv_dot4_lds"),
+    (capi.Q6_K, 2, 12288, 2048, "q6k_gemv_mfma_cols"), (capi.MXFP4, 1, 16384, 1024, "matmul_rows_staged"),
+    (capi.Q6_K, 2, 4096, 3072, None), (capi.Q6_K, 6, 4096, 1024, None), (capi.Q8_0, 2, 4096, 1280, None), (capi.MXFP4, 2, 4096, 1024, None)])
+def test_few_weight_rows_keep_the_kernels_that_are_faster_there(qtype, m, k, n, kernel):
+    blocks, lhs = synth.normal_quantized(qtype, 70, n * k, 0.02), synth.normal(71, (m, k))
+    got = capi.Weight.upload(qtype, blocks, n, k).matmul_t(m, lhs)
+    assert capi.last_kernel() == kernel if kernel else capi.last_arithmetic() == "f16 pairs"
+    want = oracle.matmul_t(qtype, (m, k, n), lhs, blocks, avx2=oracle.have_avx2())
+    assert np.all(np.abs(got - want) <= 1e-3 * np.maximum(np.abs(want), 1.0))
