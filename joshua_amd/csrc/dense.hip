@@ -107,7 +107,8 @@ int launch_wide(const jq::DenseGemm &a, unsigned n_tiles, hipStream_t s) {
 // unit.  Per stage and round, us, weights from HBM: 256 rows 1.9, 192 rows 1.5; 128 x 128 1.3, 64 x 128 1.13, of which a round that is not
 // full takes 0.6 at least.  A split adds the launch that reads its sums, at some 8 TB/s.  Measured, smaller / wide, us:
 // gate and up 24576 x 4096 of 512 rows 147 / 98 (192, one run), 4096 x 12288 of 512 rows 102 / 65 (256, eight runs), 6144 x 4096 of 512 rows
-// 67 / 52, 16384 x 4096 of 1000 rows 173 / 136 (256), 4096 x 12288 of 2000 rows 258 / 229, 24576 x 4096 of 140 rows 76 / 68.
+// 67 / 52, 16384 x 4096 of 1000 rows 173 / 136 (256), 4096 x 12288 of 2000 rows 258 / 229.  One tile of rows in two runs is not worth their
+// sums, which then meet the weights' bytes on the way: 32000 x 4096 of 140 rows 88 / 102, 24576 x 4096 of 255 rows 89 / 95, of 140 rows 76 / 73.
 struct WidePick {
     int bn = 0, splits = 1;
 };
@@ -121,6 +122,7 @@ WidePick wide_pick(const jq::DenseGemm &a, size_t wrows, int bm, size_t tiles, i
         const size_t t = (size_t)((a.M + 255) / 256) * ((wrows + bn - 1) / bn);
         const size_t most = std::max<size_t>(1, std::min<size_t>(256 / t, (size_t)a.stages / 16));
         for (const size_t s : {(size_t)1, most}) {
+            if (s == 2 && a.M <= 256) continue;
             const double us = (double)((t * s + 255) / 256) * (stages(s) * (bn == 256 ? 1.9 : 1.5) + 6.0) + sums(s);
             if (us < best) best = us, pick = {bn, (int)s};
         }

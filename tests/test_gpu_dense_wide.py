@@ -31,6 +31,13 @@ def test_products_of_many_rows(m, n, k, kernel):
     assert np.all(np.abs(got[rows] - x @ w.T) <= 2e-6 * scale + 1e-7)
 
 
+def test_one_tile_of_rows_is_not_split_in_two():
+    w = capi.Weight.upload(capi.BF16, np.zeros(24576 * 4096, np.uint16), 24576, 4096)
+    for m, kernel in ((200, "dense_gemm"), (300, "dense_gemm_wide")):
+        w.matmul_t(m, np.ones((m, 4096), np.float32))
+        assert capi.last_kernel() == kernel
+
+
 @pytest.mark.parametrize("ff", [12283, 4096])
 def test_gated_block_of_many_rows(tmp_path, ff):
     """A feed-forward block whose gate and up rows run in one launch, whole and in runs of k."""
