@@ -73,10 +73,10 @@ const char *jq_last_error(void);
  * where k is split; jq_last_arithmetic tells its forms apart. */
 const char *jq_last_kernel(void);
 
-/* What that GEMM multiplied: "int8" (two 8-bit planes a factor), "f16+fp6" (Q4_K and MXFP4 from
- * 128 activation rows on: f16 products, their remainders in FP6) or "f16 pairs" (two f16 numbers a
- * factor, 22 bits: up to some 100 activation rows, also after the kernel "few_rows" and under the
- * names "q4k_gemm_mfma" and "gemm_decoded_mfma" that fewer than 64 rows go by); "" after any other. */
+/* What a matrix-core product multiplied: in that GEMM "int8" (two 8-bit planes a factor) or
+ * "f16+fp6" (Q4_K and MXFP4 from 128 activation rows on: f16 products, their remainders in FP6),
+ * in "few_rows" (up to 16 activation rows) and "few_rows_many" (up to 127 rows of Q4_K, 255 of
+ * Q6_K, Q8_0 and MXFP4) "f16 pairs" (two f16 numbers a factor); "" after any other kernel. */
 const char *jq_last_arithmetic(void);
 
 /* Elements and bytes per block of a type id; nonzero for an unknown id

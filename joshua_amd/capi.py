@@ -212,7 +212,8 @@ def last_kernel() -> str:
 
 
 def last_arithmetic() -> str:
-    """What the matrix-core GEMM multiplied: "int8", "f16+fp6", or "f16 pairs" (up to 16 rows); "" after any other kernel."""
+    """What a matrix-core product multiplied: "int8" or "f16+fp6" (the GEMM over many rows), "f16 pairs" (few_rows and
+    few_rows_many); "" after any other kernel."""
     return lib().jq_last_arithmetic().decode()
 
 

@@ -954,23 +954,13 @@ bool few_rows_better(uint32_t type, size_t m, size_t k, size_t n) {
     }
 }
 
-// The name that callers know the product by: from 8 rows against 8M weights on (a format other than Q4_K) the many-row GEMM's, from 17
-// rows on that of the GEMM that took it else.
-const char *few_rows_name(uint32_t type, size_t m, size_t k, size_t n) {
-    if (type == JQ_TYPE_Q4_K) return m <= 16 ? "few_rows" : m < 64 ? "q4k_gemm_mfma+splitk" : "q4k_gemm_i8+splitk";
-    if ((m >= 8 && n * k >= ((size_t)8 << 20)) || m >= 64)
-        return type == JQ_TYPE_Q6_K ? "q6k_gemm_i8+splitk" : type == JQ_TYPE_Q8_0 ? "q8_0_gemm_i8+splitk" : "mxfp4_gemm_i8+splitk";
-    if (m > 16) return "gemm_decoded_mfma+splitk";
-    return "few_rows";
-}
-
 // All pointers are device pointers; shapes already validated; m, n > 0.
 int dispatch_matmul(uint32_t type, const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m,
                     size_t k, size_t n, hipStream_t s) {
     if (m > 0x7FFFFFFF || k > 0x7FFFFFFF || n > 0x7FFFFFFF) return fail("matmul: dimension exceeds 2^31-1");
     if (dense_elem_bytes(type)) return dense_matmul(type, W, row_bytes, X, Y, m, k, n, s);
     if (m >= 2 && few_rows_better(type, m, k, n)) {
-        const int rc = (m <= 16 ? few_rows_matmul : few_rows_many_matmul)(type, W, row_bytes, X, Y, m, k, n, few_rows_name(type, m, k, n), s);
+        const int rc = (m <= 16 ? few_rows_matmul : few_rows_many_matmul)(type, W, row_bytes, X, Y, m, k, n, s);
         if (rc >= 0) return rc;
     }
     if (type == JQ_TYPE_Q4_K && m == 1) {
@@ -998,7 +988,7 @@ int dispatch_matmul(uint32_t type, const uint8_t *W, size_t row_bytes, const flo
         if (rc >= 0) return rc;
         rc = dispatch_i8_gemv(type, W, row_bytes, X, Y, k, n, s);
         if (rc >= 0) return rc;
-        if (few_rows_better(type, 1, k, n)) rc = few_rows_matmul(type, W, row_bytes, X, Y, 1, k, n, few_rows_name(type, 1, k, n), s);
+        if (few_rows_better(type, 1, k, n)) rc = few_rows_matmul(type, W, row_bytes, X, Y, 1, k, n, s);
         if (rc >= 0) return rc;
     }
     // Q6_K and Q8_0 with two activation rows against 16M weights or more in fewer rows than few_rows needs: the one-row kernel twice

@@ -38,7 +38,7 @@ int launch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t 
 }
 
 template <class F>
-int dispatch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n, const char *name, hipStream_t s) {
+int dispatch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n, hipStream_t s) {
     static const char *tiles_env = getenv("JQ_FEW_ROWS_TILES");
     if (m < 1 || m > 16 || k == 0 || k % 256 != 0 || row_bytes % F::ALIGN != 0 || ((uintptr_t)W & (F::ALIGN - 1)) != 0 || ((uintptr_t)X & 15) != 0 ||
         n > 0x7FFFFF00ull || row_bytes > 0x200000)
@@ -63,7 +63,7 @@ int dispatch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_
     JQ_FEW(1, 4) JQ_FEW(1, 8) JQ_FEW(1, 16) JQ_FEW(2, 4) JQ_FEW(2, 8) JQ_FEW(2, 16) JQ_FEW(4, 4) JQ_FEW(4, 8) JQ_FEW(4, 16)
 #undef JQ_FEW
     if (rc) return rc;
-    note_kernel(name, "f16 pairs");
+    note_kernel("few_rows", "f16 pairs");
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -109,7 +109,7 @@ const ManyShape &many_shape(int planes, size_t m, size_t nb, size_t n) {
 }
 
 template <class F>
-int dispatch_many(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n, const char *name, hipStream_t s) {
+int dispatch_many(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n, hipStream_t s) {
     static const char *shape_env = getenv("JQ_FEW_ROWS_SHAPE");  // "tiles,groups": one of the shapes
     if (k == 0 || k % 256 != 0 || row_bytes % F::ALIGN != 0 || ((uintptr_t)W & (F::ALIGN - 1)) != 0 || ((uintptr_t)X & 15) != 0 ||
         n > 0x7FFFFF00ull || m > 0x7FFFFF00ull || row_bytes > 0x200000)
@@ -123,7 +123,7 @@ int dispatch_many(const uint8_t *W, size_t row_bytes, const float *X, float *Y, 
     JQ_FEW(1, 2) JQ_FEW(2, 2) JQ_FEW(4, 2) JQ_FEW(2, 3) JQ_FEW(2, 4)
 #undef JQ_FEW
     if (rc) return rc;
-    note_kernel(name, "f16 pairs");
+    note_kernel("few_rows_many", "f16 pairs");
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -136,23 +136,23 @@ double few_rows_many_us(uint32_t type, size_t m, size_t k, size_t n) {
 }
 
 int few_rows_many_matmul(uint32_t type, const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n,
-                         const char *name, hipStream_t s) {
+                         hipStream_t s) {
     switch (type) {
-    case JQ_TYPE_Q4_K: return dispatch_many<jq::FrQ4K>(W, row_bytes, X, Y, m, k, n, name, s);
-    case JQ_TYPE_Q6_K: return dispatch_many<jq::FrQ6K>(W, row_bytes, X, Y, m, k, n, name, s);
-    case JQ_TYPE_Q8_0: return dispatch_many<jq::FrQ8_0>(W, row_bytes, X, Y, m, k, n, name, s);
-    case JQ_TYPE_MXFP4: return dispatch_many<jq::FrMXFP4>(W, row_bytes, X, Y, m, k, n, name, s);
+    case JQ_TYPE_Q4_K: return dispatch_many<jq::FrQ4K>(W, row_bytes, X, Y, m, k, n, s);
+    case JQ_TYPE_Q6_K: return dispatch_many<jq::FrQ6K>(W, row_bytes, X, Y, m, k, n, s);
+    case JQ_TYPE_Q8_0: return dispatch_many<jq::FrQ8_0>(W, row_bytes, X, Y, m, k, n, s);
+    case JQ_TYPE_MXFP4: return dispatch_many<jq::FrMXFP4>(W, row_bytes, X, Y, m, k, n, s);
     default: return -1;
     }
 }
 
 int few_rows_matmul(uint32_t type, const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n,
-                    const char *name, hipStream_t s) {
+                    hipStream_t s) {
     switch (type) {
-    case JQ_TYPE_Q4_K: return dispatch<jq::FrQ4K>(W, row_bytes, X, Y, m, k, n, name, s);
-    case JQ_TYPE_Q6_K: return dispatch<jq::FrQ6K>(W, row_bytes, X, Y, m, k, n, name, s);
-    case JQ_TYPE_Q8_0: return dispatch<jq::FrQ8_0>(W, row_bytes, X, Y, m, k, n, name, s);
-    case JQ_TYPE_MXFP4: return dispatch<jq::FrMXFP4>(W, row_bytes, X, Y, m, k, n, name, s);
+    case JQ_TYPE_Q4_K: return dispatch<jq::FrQ4K>(W, row_bytes, X, Y, m, k, n, s);
+    case JQ_TYPE_Q6_K: return dispatch<jq::FrQ6K>(W, row_bytes, X, Y, m, k, n, s);
+    case JQ_TYPE_Q8_0: return dispatch<jq::FrQ8_0>(W, row_bytes, X, Y, m, k, n, s);
+    case JQ_TYPE_MXFP4: return dispatch<jq::FrMXFP4>(W, row_bytes, X, Y, m, k, n, s);
     default: return -1;
     }
 }

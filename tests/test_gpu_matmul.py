@@ -14,6 +14,12 @@ from tests.test_oracle_matmul import fixture_iq2xxs_rhs, mxfp4_pattern, ref_lhs,
 pytestmark = pytest.mark.gpu
 
 TOL = 1e-3
+FEW_ROWS = os.environ.get("JQ_FEW_ROWS", "")[:1] != "0"  # off in the child process of test_gpu_few_rows_off.py
+PAIRS = (capi.Q4_K, capi.Q6_K, capi.Q8_0, capi.MXFP4)    # the formats of few_rows and few_rows_many
+
+
+def few_rows(m):
+    return "few_rows" if m <= 16 else "few_rows_many"
 
 
 def close(got, want):
@@ -579,13 +585,14 @@ def test_non_finite_activations_show_in_the_result(qtype, m, k, n):
 @pytest.mark.parametrize("m,k,n", [(8, 12288, 1024), (16, 4096, 2100), (33, 4096, 2048 + 5), (48, 8192, 1100)])
 def test_few_rows_against_a_large_matrix_take_the_int8_gemm(qtype, m, k, n):
     """8 to 63 activation rows against 8M weights or more: the int8 GEMM split over k, most of its
-    activation-row tile empty; the partial sums are added in a fixed order (the same result on every call)."""
+    activation-row tile empty; the partial sums are added in a fixed order (the same result on every call).  Q6_K, Q8_0 and MXFP4
+    take it where few_rows does not run."""
     blocks = make_blocks(qtype, n, k, 310 + m)
     lhs = synth.normal(311 + m, (m, k))
     w = capi.Weight.upload(qtype, blocks, n, k)
     got = w.matmul_t(m, lhs)
     name = {capi.Q6_K: "q6k", capi.Q8_0: "q8_0", capi.Q2_K: "q2k", capi.IQ2_XXS: "iq2xxs", capi.MXFP4: "mxfp4"}[qtype]
-    assert capi.last_kernel() == name + "_gemm_i8+splitk"
+    assert capi.last_kernel() == (few_rows(m) if FEW_ROWS and qtype in PAIRS else name + "_gemm_i8+splitk")
     assert close(got, oracle.matmul_t(qtype, (m, k, n), lhs, blocks, avx2=True))
     assert np.array_equal(got, w.matmul_t(m, lhs))
 
@@ -602,7 +609,7 @@ def test_decoded_weights_gemm_split_over_k(qtype, m, k, n):
     w = capi.Weight.upload(qtype, blocks, n, k)
     got = w.matmul_t(m, lhs)
     assert close(got, oracle.matmul_t(qtype, (m, k, n), lhs, blocks))
-    assert capi.last_kernel().startswith("gemm_decoded_mfma")
+    assert capi.last_kernel().startswith(few_rows(m) if FEW_ROWS and qtype == capi.MXFP4 else "gemm_decoded_mfma")
     assert np.array_equal(got, w.matmul_t(m, lhs))
 
 
@@ -1079,7 +1086,7 @@ def test_q4k_mfma_gemv_switched_off_by_environment():
     assert res.returncode == 0 and "ok" in res.stdout, res.stdout + res.stderr
 
 
-KERNEL_OF_SHAPE = [  # which kernel serves the shapes the benchmarks quote: (format, m, k, n) -> jq_last_kernel()
+KERNEL_OF_SHAPE = [  # which kernel serves the shapes the benchmarks quote: (format, m, k, n) -> jq_last_kernel(), and where few_rows is off
     (capi.Q4_K, 1, 4096, 14336, "q4k_gemv_mfma_lds"),        # headline
     (capi.Q4_K, 1, 4096, 4096, "q4k_gemv_mfma_lds"),
     (capi.Q4_K, 1, 4096, 1024, "q4k_gemv_dot4_lds"),         # fewer than 2048 weight rows
@@ -1107,13 +1114,13 @@ KERNEL_OF_SHAPE = [  # which kernel serves the shapes the benchmarks quote: (for
     (capi.Q6_K, 1, 4096, 4096, "q6k_gemv_mfma_tile"),
     (capi.Q6_K, 1, 4096, 8192, "q6k_gemv_dot4_lds"),
     (capi.Q6_K, 1, 1024, 4096, "matmul_rows_staged"),
-    (capi.Q6_K, 64, 4096, 1024, "q6k_gemm_i8+splitk"),
+    (capi.Q6_K, 64, 4096, 1024, "few_rows_many", "q6k_gemm_i8+splitk"),
     (capi.Q6_K, 64, 2048, 256, "gemm_decoded_mfma+splitk"), # a small product: weights decoded in the workgroup
     (capi.Q6_K, 512, 12288, 4096, "q6k_gemm_i8+splitk"),    # a feed-forward down projection in prefill: 74 tiles of 256 x 112, three splits
-    (capi.Q6_K, 32, 4096, 14336, "q6k_gemm_i8+splitk"),     # few rows against a large matrix
+    (capi.Q6_K, 32, 4096, 14336, "few_rows_many", "q6k_gemm_i8+splitk"),     # few rows against a large matrix
     (capi.Q8_0, 512, 4096, 14336, "q8_0_gemm_i8"),
-    (capi.Q8_0, 16, 4096, 4096, "q8_0_gemm_i8+splitk"),
-    (capi.Q8_0, 32, 2048, 2048, "gemm_decoded_mfma+splitk"),# few rows against a small matrix
+    (capi.Q8_0, 16, 4096, 4096, "few_rows", "q8_0_gemm_i8+splitk"),
+    (capi.Q8_0, 32, 2048, 2048, "few_rows_many", "gemm_decoded_mfma+splitk"),# few rows against a small matrix
     (capi.Q2_K, 512, 4096, 14336, "q2k_gemm_i8"),
     (capi.Q2_K, 64, 12288, 4096, "q2k_gemm_i8+splitk"),
     (capi.Q2_K, 1, 7680, 2048, "matmul_rows_staged"),
@@ -1123,7 +1130,7 @@ KERNEL_OF_SHAPE = [  # which kernel serves the shapes the benchmarks quote: (for
 ]
 
 
-@pytest.mark.parametrize("qtype,m,k,n,kernel", KERNEL_OF_SHAPE)
+@pytest.mark.parametrize("qtype,m,k,n,kernel", [c[:4] + (c[4 if FEW_ROWS else -1],) for c in KERNEL_OF_SHAPE])
 def test_kernel_chosen_for_a_shape(qtype, m, k, n, kernel):
     """The dispatcher's crossover points are measured constants; this pins what they select, so that a
     parity test named after a kernel keeps covering that kernel."""
@@ -1542,13 +1549,14 @@ def _large_random_shapes(seed, count):
 @pytest.mark.parametrize("qtype", [t for t in capi.ALL_TYPES + capi.GENERIC_TYPES if t != capi.Q4_K])
 @pytest.mark.parametrize("m,k,n", _large_random_shapes(78, 4))
 def test_every_format_on_the_int8_gemm_at_random_large_shapes(qtype, m, k, n):
-    """Seeded random shapes against large matrices: whatever tile shape and split over k the estimate picks
+    """Seeded random shapes against large matrices (few_rows takes some of three formats' where it is on): whatever tile shape and split over k the estimate picks
     (32 x 64 tiles up to 32 rows, 128 x 64, 256 x 96 or 256 x 112 beyond), ragged in both directions, the result
     holds the reference's bound against the oracle on a sample of the weight rows."""
     blocks = synth.random_blocks(qtype, 710 + qtype, n * k) if qtype in capi.GENERIC_TYPES else make_blocks(qtype, n, k, 710 + qtype)
     lhs = synth.normal(810 + n % 89, (m, k))
     got = capi.Weight.upload(qtype, blocks, n, k).matmul_t(m, lhs)
-    assert "gemm_i8" in capi.last_kernel(), capi.last_kernel()
+    if not (FEW_ROWS and qtype in PAIRS and capi.last_kernel() == few_rows(m)):
+        assert "gemm_i8" in capi.last_kernel(), capi.last_kernel()
     rows = np.unique(np.concatenate([np.arange(130), np.arange(n - 130, n), np.arange(130, n - 130, 7)[:240]]))
     sub = blocks.reshape(n, -1)[rows].reshape(-1)
     want = oracle.matmul_t(qtype, (m, k, rows.size), lhs, sub, avx2=oracle.have_avx2() and qtype not in capi.GENERIC_TYPES)
