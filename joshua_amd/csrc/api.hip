@@ -680,6 +680,8 @@ int dispatch_q4k_rows16(const uint8_t *W, size_t row_bytes, const float *X, floa
     return 0;
 }
 
+static_assert(INT8_GEMM_REC == (size_t)jq::QI_REC, "gemm_h6 takes the rows in two turns where this GEMM's records fit a fixed scratch");
+
 // Many activation rows on the int8 matrix cores (Q4_K up to 127 of them, gemm_h6's products from there on): the activations as two int8 planes per
 // 256-element super-block in the call scratch of the stream, then kq_gemm_i8 with the workgroup shape and the
 // split over k that an estimate fitted to measurements prefers.  Returns -1 when the shape is outside its

@@ -6,8 +6,6 @@
 namespace jqh {
 namespace {
 
-constexpr size_t INT8_REC = 9280;  // bytes of the int8 GEMM's record of 16 rows and a super-block (kernels_mfma_q4k_gemm_i8.hpp)
-
 // Leave to use that much LDS, asked for once a kernel.
 template <auto KERN>
 hipError_t big_lds_once(int lds) {
@@ -43,7 +41,7 @@ int dispatch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_
     size_t turn = m;
     auto acts_of = [&](size_t rows) { return ((rows + 15) / 16 * nb * (size_t)jq::h6_rec<F::MINS>() + 255) & ~(size_t)255; };
     if (acts_of(m) > scratch_cap) {
-        if (groups * nb * INT8_REC > scratch_cap) return -1;
+        if (groups * nb * INT8_GEMM_REC > scratch_cap) return -1;
         turn = (groups + 1) / 2 * 16;
         if (acts_of(turn) > scratch_cap) return -1;
     }

@@ -4,6 +4,8 @@
 
 namespace jqh {
 
+constexpr size_t INT8_GEMM_REC = 9280;  // bytes of the int8 GEMM's record of 16 rows and a super-block, jq::QI_REC: what that GEMM's scratch is counted in
+
 // Device pointers, shapes validated, k and n > 0.  With `swiglu_pairs` the activations are silu(gate) * up over rows of 2 k floats in which
 // gate_j and up_j alternate.  -1: the call is outside its reach.
 int gemm_h6(uint32_t type, const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n, hipStream_t s,
