@@ -113,11 +113,18 @@ struct WidePick {
     int bn = 0, splits = 1;
 };
 WidePick wide_pick(const jq::DenseGemm &a, size_t wrows, int bm, size_t tiles, int splits) {
+    static const char *env = getenv("JQ_DENSE_WIDE");  // "0": never; "rows,runs": that tile, that many runs of k
+    WidePick pick;
+    if (env && env[0] == '0') return pick;
+    if (env && sscanf(env, "%d,%d", &pick.bn, &pick.splits) == 2 && (pick.bn == 192 || pick.bn == 256) && pick.splits > 0) {
+        pick.splits = std::min(pick.splits, a.stages);
+        return pick;
+    }
+    pick = {};
     auto sums = [&](size_t s) { return s > 1 ? 3.0 + (s + 1.0) * a.M * (double)wrows * 4e-6 / 8.0 : 0.0; };
     auto stages = [&](size_t s) { return (double)((a.stages + s - 1) / s); };
     const double rounds = (double)(tiles * splits) / (bm == 128 ? 512 : 768), part = rounds - std::floor(rounds);
     double best = 0.95 * ((std::floor(rounds) + (part > 0 ? 0.6 + 0.4 * part : 0.0)) * stages(splits) * (bm == 128 ? 1.3 : 1.13) + sums(splits));
-    WidePick pick;
     for (const int bn : {256, 192}) {
         const size_t t = (size_t)((a.M + 255) / 256) * ((wrows + bn - 1) / bn);
         const size_t most = std::max<size_t>(1, std::min<size_t>(256 / t, (size_t)a.stages / 16));

@@ -1,5 +1,9 @@
 """Products with plain bf16 rows in tiles of 256 activation rows (one workgroup a compute unit): one run of k and several, row and column counts
 at the edges of the tiles and within them, alone and in a gated feed-forward block."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -10,6 +14,8 @@ from tests import layered_cases as lc
 from tests.layered_cases import build, check, feed, tokens
 
 pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.mark.parametrize("m,n,k,kernel", [
@@ -45,3 +51,34 @@ def test_gated_block_of_many_rows(tmp_path, ff):
     m, o, _ = build(tmp_path, cfg, 21, lc.BF16, n_ctx=512)
     toks = tokens(cfg, 22, 500)
     check(feed(m, toks, []), o.forward(toks), lc.BF16, "whole", o)
+
+
+CHILD = r"""
+import sys
+sys.path.insert(0, ROOT)
+import pathlib
+import tempfile
+import numpy as np
+from joshua_amd import capi
+from tests import layered_cases as lc
+for ff, n_tokens in ((1283, 500), (1440, 270)):   # columns within a tile of 96 and of 128 gate rows, and where one ends; rows of the last tile
+    cfg = lc.model(2048, 40, [lc.dense(lc.mamba(16, 2, 2, 2), ff, limit=0.4)])
+    with tempfile.TemporaryDirectory() as folder:
+        m, o, _ = lc.build(pathlib.Path(folder), cfg, 31, lc.BF16, n_ctx=512)
+    toks = lc.tokens(cfg, 32, n_tokens)
+    lc.check(lc.feed(m, toks, []), o.forward(toks), lc.BF16, ff, o)
+w, x = np.full(4096 * 2048, 0x3F80, np.uint16), np.ones((300, 2048), np.float32)   # ones: every sum is 2048
+got = capi.Weight.upload(capi.BF16, w, 4096, 2048).matmul_t(300, x)
+assert capi.last_kernel() == "dense_gemm_wide" + ("+splitk" if RUNS > 1 else "") and np.all(got == 2048.0)
+print("wide ok")
+"""
+
+
+@pytest.mark.parametrize("rows", [192, 256])
+@pytest.mark.parametrize("runs", [1, 3])
+def test_gated_block_in_every_tile_and_in_runs(rows, runs):
+    """The shape is read at the first product, hence the child process; the feed-forward blocks have more than the 128 tiles of 64 x 128 from which
+    a product may take it."""
+    res = subprocess.run([sys.executable, "-c", CHILD.replace("ROOT", repr(ROOT), 1).replace("RUNS", str(runs))], capture_output=True, text=True, timeout=110,
+                         env=dict(os.environ, JQ_DENSE_WIDE=f"{rows},{runs}"))
+    assert res.returncode == 0 and "wide ok" in res.stdout, res.stdout + res.stderr
