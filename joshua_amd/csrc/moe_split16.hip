@@ -24,7 +24,8 @@ int moe_split16(const MoeSplit16Call &c, hipStream_t s) {
     a.gexp = c.gexp, a.offsets = c.offsets, a.xsel = c.xsel, a.yrow = c.yrow;
     a.Y = c.Y, a.groups = c.groups, a.n = (int)c.n, a.nb = (int)nb, a.clamp = c.clamp;
     // Waves of two tiles only for layers whose rows do not fill workgroups of four (128 experts of 768, the layer, us: 70 tokens 144 with two
-    // and 135 with four, 150 tokens 155 / 146, 250 tokens 175 / 173, 512 tokens 235 / 220).
+    // and 135 with four, 150 tokens 155 / 146, 250 tokens 175 / 173, 512 tokens 235 / 220; 256 experts of 64, whose down projection is of another
+    // type, 200 tokens 166 with two and 172 with four, of 128 870 / 878).
     const int wt = c.n <= 128 ? 2 : 4;
     const size_t per = jq::moe_split16_cols(wt) / (c.wb ? 2 : 1);
     a.cols = (int)((c.n + per - 1) / per);

@@ -315,6 +315,21 @@ def test_q4k_experts_on_split_f16_activations(h, inter, E, k, tokens, shared_int
     assert close(dev.forward(few), ora.forward(few))
 
 
+@pytest.mark.parametrize("inter", [64, 96, 128])
+def test_q4k_experts_of_few_columns_on_split_f16_activations(inter):
+    """Up to 128 gate rows an expert (a down projection of another type: Q4_K has none so short): waves of two tiles."""
+    h, E, k, T = 512, 256, 8, 140
+    rw = synth.normal(670, (E, h), sigma=0.02)
+    gate, up = (synth.normal_quantized(capi.Q4_K, 671 + i, E * inter * h, 0.02) for i in range(2))
+    down = synth.normal_quantized(capi.Q8_0, 673, E * h * inter, 0.02)
+    ora = MoeOracle(capi.Q4_K, h, inter, E, k, rw, gate, up, down, avx2=oracle.have_avx2(), qtype_down=capi.Q8_0)
+    dev = capi.Moe(capi.MoeConfig(E, k, h, inter, 0, 1, 0.0, 1, 1, 0.0, 0.0), rw, capi.Weight.upload(capi.Q4_K, gate, E * inter, h),
+                   capi.Weight.upload(capi.Q4_K, up, E * inter, h), capi.Weight.upload(capi.Q8_0, down, E * h, inter))
+    x = synth.normal(674, (T, h)) * np.float32(20.0)
+    got, want = dev.forward(x), ora.forward(x)
+    assert capi.last_kernel() == "moe_split16" and close(got, want)
+
+
 @pytest.mark.parametrize("alike", [0, 40])
 def test_q4k_experts_on_split_f16_activations_against_64_bits(alike):
     """Ten pairs an expert, the calls that the ring kernel's f32 products ran before: no further from 64 bits than those.  The
