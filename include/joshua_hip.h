@@ -118,20 +118,32 @@ const void *jq_device_ptr(const jq_weight *w);
  * ptrs_are_device == 0 the call stages lhs/dst through HBM and returns after
  * the result has landed in dst.
  * Accuracy: |dst - ref| <= 1e-3 * max(|ref|, 1) against the reference's f32 arithmetic
- * (its own bound, src/kquant_dot.rs:853).  The integer kernels hold the activations in
- * 16-bit fixed point: one scale per 32 elements of a row for Q4_K up to 63 activation rows
- * and for every one-row product, so a row whose groups span many orders of magnitude keeps
- * the bound; the matrix-core GEMM (Q4_K from 64 rows on; every other format from 17 rows
- * on, and from 8 against 8M weights or more) uses one scale per 256 elements, which
- * resolves each super-block to 2^-16 of its largest magnitude (2^-12 of the sum of the
- * terms' magnitudes on such rows; the reference's integer path quantises activations to 8
- * bits per 256, src/quant_matmul.rs:184), and from 128 rows on Q4_K's holds them as f16 with a
- * remainder of four significant bits, relative to each element down to 2^-19 of the
- * super-block's largest.  In that GEMM the formats with a scale per 32
- * elements (Q8_0, MXFP4, Q4_0, Q4_1, Q5_0, Q5_1) have the eight blocks of a 256-run put on
- * the run's largest scale at 15 or 16 bits: exact where the scales are equal or a few powers
- * of two apart, else each weight to 2^-15 of the run's largest magnitude or better.  A row
- * holding an inf or a NaN comes out all NaN. */
+ * (its own bound, src/kquant_dot.rs:853).  What the factors are held in depends on the kernel
+ * (jq_last_kernel, jq_last_arithmetic); the reference's integer path quantises activations to 8
+ * bits per 256 (src/quant_matmul.rs:184):
+ * - integer kernels of one row, and of a few rows of Q4_K: activations in 16-bit fixed point with
+ *   one scale per 32 elements of a row, so a row whose groups span many orders of magnitude keeps
+ *   the bound.
+ * - "f16 pairs", from two rows of Q6_K, Q8_0 and MXFP4 and three of Q4_K (and single rows that
+ *   no other kernel takes) to 127 of Q4_K and 255 of the others, where measurement has it faster:
+ *   an activation is the sum of two f16 numbers behind a power of two per 256 elements, 2^-22 of
+ *   itself or 2^-38 of the 256's largest off; weights are exact whatever the scales (of Q4_K the
+ *   part that does not depend on the code, per 32 elements, to 2^-22 of itself or 2^-25 of the larger of d
+ *   and dmin); the product of the two remainders, 2^-22, is left out.  Normal data lie 0.7e-7 to 1.5e-7
+ *   off 64 bits (relative 2-norm), as far as f32 kernels or less.
+ * - the GEMM over many rows on int8 (every other format from 17 rows on, from 6 against 8M weights
+ *   or more and from 4 against 32M; Q4_K from 64): one scale per 256 elements, which resolves each super-block
+ *   to 2^-16 of its largest magnitude (2^-12 of the sum of the terms' magnitudes on rows that span
+ *   many orders).  Formats with a scale per 32 elements (Q8_0, MXFP4, Q4_0, Q4_1, Q5_0, Q5_1) have
+ *   the eight blocks of a 256-run put on the run's largest scale at 15 or 16 bits: exact where the
+ *   scales are equal or a few powers of two apart, else each weight to 2^-15 of the run's largest
+ *   magnitude or better.
+ * - that GEMM on f16 and FP6 (Q4_K and MXFP4 from 128 rows on): activations as f16 with a remainder
+ *   of four significant bits, relative to each element down to 2^-19 of the super-block's largest.
+ *   MXFP4's are exact where f16 holds all 256 behind a power of two (bf16 values) or all have one
+ *   magnitude, and its weights where the scales of a 256-run are within 2^36 of the largest (zeros from
+ *   2^60 on).
+ * A row holding an inf or a NaN comes out without a finite value. */
 int jq_matmul_t(const jq_weight *w, size_t m, const float *lhs, size_t lhs_len, float *dst,
                 size_t dst_len, int ptrs_are_device, void *stream);
 
@@ -155,13 +167,15 @@ int jq_matmul_t_f16(const jq_weight *w, size_t m, const uint16_t *lhs, size_t lh
  * device's memory, held from library load until the process ends.  The call makes no
  * hipMalloc / hipFree and fails, dst untouched, when the product needs more scratch than
  * the array holds (one activation row never needs any; the matrix-core GEMM needs 9280 bytes
- * per 16 activation rows and 256 columns, whichever arithmetic it runs on, other kernels up to
- * 4 m k bytes; a product split over k adds 4 m n bytes a split).
+ * per 16 activation rows and 256 columns, whichever arithmetic it runs on, "few_rows_many" 17472,
+ * "few_rows" none, other kernels up to 4 m k bytes; a product split over k adds 4 m n bytes a split).
  * Every call on a device shares that device's array: calls whose kernels overlap on
  * one device (two streams, two threads) race; calls on one stream are safe.
  * Where jq_matmul_t would split a product over k into more partial results than the
  * array holds, this call takes fewer splits: the result then differs from jq_matmul_t's
- * in the order of its f32 additions (within the accuracy bound, not bit for bit). */
+ * in the order of its f32 additions (within the accuracy bound, not bit for bit).  Where it would
+ * take few_rows_many and the array does not hold what that prepares (127 rows of more than 61440
+ * columns), this call takes the kernel that comes next, in that one's arithmetic. */
 #define JQ_NOALLOC_SCRATCH_BYTES (32u << 20)
 int jq_matmul_t_noalloc(const jq_weight *w, size_t m, const float *lhs_dev, size_t lhs_len,
                         float *dst_dev, size_t dst_len, void *stream);
