@@ -130,7 +130,7 @@ const void *jq_device_ptr(const jq_weight *w);
  *   itself or 2^-38 of the 256's largest off; weights are exact whatever the scales (of Q4_K the
  *   part that does not depend on the code, per 32 elements, to 2^-22 of itself or 2^-25 of the larger of d
  *   and dmin); the product of the two remainders, 2^-22, is left out.  Normal data lie 0.7e-7 to 1.5e-7
- *   off 64 bits (relative 2-norm), as far as f32 kernels or less.
+ *   off 64 bits (relative 2-norm) up to 16 rows, to 2.1e-7 beyond: as far as f32 kernels or less.
  * - the GEMM over many rows on int8 (every other format from 17 rows on, from 6 against 8M weights
  *   or more and from 4 against 32M; Q4_K from 64): one scale per 256 elements, which resolves each super-block
  *   to 2^-16 of its largest magnitude (2^-12 of the sum of the terms' magnitudes on rows that span
@@ -141,8 +141,8 @@ const void *jq_device_ptr(const jq_weight *w);
  * - that GEMM on f16 and FP6 (Q4_K and MXFP4 from 128 rows on): activations as f16 with a remainder
  *   of four significant bits, relative to each element down to 2^-19 of the super-block's largest.
  *   MXFP4's are exact where f16 holds all 256 behind a power of two (bf16 values) or all have one
- *   magnitude, and its weights where the scales of a 256-run are within 2^36 of the largest (zeros from
- *   2^60 on).
+ *   magnitude, and its weights where the scales of a 256-run lie within 2^26 of the largest (2^-19 of
+ *   themselves off within 2^36, zeros from 2^60 on).
  * A row holding an inf or a NaN comes out without a finite value. */
 int jq_matmul_t(const jq_weight *w, size_t m, const float *lhs, size_t lhs_len, float *dst,
                 size_t dst_len, int ptrs_are_device, void *stream);

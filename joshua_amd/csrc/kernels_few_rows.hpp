@@ -12,9 +12,9 @@
 // Bound: the issue of vector instructions (a super-block of 16 weight rows takes 190 (Q4_K), 280 (Q6_K), 210 (Q8_0) or 90 (MXFP4),
 // its activations 300 a workgroup) and, at the smallest sizes, one trip to memory.  us, 16 rows, before / now:
 //   14336 x 4096   Q6_K 42 / 22     Q8_0 43 / 20     MXFP4 41 / 14
-//   6000 x 5120    Q4_K 34 / 15     Q6_K 28 / 16     Q8_0 27 / 15
-//   11008 x 3840   Q4_K 122 / 15    14336 x 11264   Q4_K 134 / 40   Q8_0 105 / 48   MXFP4 96 / 34
-// A byte of weights is read once: 14336 x 4096 of MXFP4 with 8 rows, 12 us, is 2.7 TB/s, of Q8_0, 18 us, 3.5.
+//   6000 x 5120    Q4_K 34 / 13     Q6_K 28 / 16     Q8_0 27 / 15
+//   11008 x 3840   Q4_K 122 / 15    14336 x 11264   Q4_K 134 / 36   Q8_0 105 / 47   MXFP4 96 / 35
+// A byte of weights is read once: 14336 x 4096 of MXFP4 with 8 rows, 12 us, is 2.7 TB/s, of Q8_0, 19 us, 3.3.
 #pragma once
 #include "split16_parts.hpp"
 

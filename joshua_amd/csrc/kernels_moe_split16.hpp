@@ -92,7 +92,7 @@ struct MoeSplit16 {
 // Bound: no one thing.  128 experts of 768 x 2048 and 512 tokens (32 pairs an expert), gate and up, 120 us: 31 us of matrix and 34 of vector
 // instructions, 44 us for the weights at a large copy's rate, 18 us of starts and ends of workgroups; without its copies the loop takes 30 us
 // less, without matrix instructions or unpacking 7 to 11.  The packed bytes come through LDS in pieces of a row (a lane that reads its own share
-// of one looks up a cache line for itself, two clocks): the layer 258 -> 231 us.  Two halves of them on their way, and the activations in
+// of one looks up a cache line for itself, two clocks): the layer 247 -> 223 us.  Two halves of them on their way, and the activations in
 // quarters, as two workgroups a compute unit leave room for: 100 tokens 139.5 -> 136.5, 150 tokens 151.5 -> 146.5, 512 tokens as before.
 // The int8 GEMM took 3 x 102 us for the three products.
 template <bool DUAL, int RG, int WT>
