@@ -682,17 +682,84 @@ int dispatch_q4k_rows16(const uint8_t *W, size_t row_bytes, const float *X, floa
 
 static_assert(INT8_GEMM_REC == (size_t)jq::QI_REC, "gemm_h6 takes the rows in two turns where this GEMM's records fit a fixed scratch");
 
+// The workgroup shapes of the int8 GEMM: two of 256 x 112 and 256 x 96 outputs (eight waves, one workgroup a compute unit), 128 x 64 (four
+// waves, two a compute unit) and, up to 32 rows, 32 x 64 (two waves that share the weight rows, two workgroups a compute unit).
+struct GemmI8Shape {
+    int nw, ng;
+    bool nsplit;  // tiles of 32 activation rows whose waves share the weight rows
+    size_t rows() const { return nsplit ? 32 : 32 * (size_t)nw; }
+    size_t cols() const { return 16 * (size_t)ng; }
+};
+constexpr GemmI8Shape GEMM_I8_SHAPES[] = {{8, 7, false}, {8, 6, false}, {4, 4, false}, {2, 4, true}};
+
+size_t gemm_i8_tiles(const GemmI8Shape &sh, size_t m, size_t n) {
+    return ((m + sh.rows() - 1) / sh.rows()) * ((n + sh.cols() - 1) / sh.cols());
+}
+
+// Workgroups of a launch of that many tiles: rounded up to eights (the rest empty) where the row tiles divide 8, so that
+// an XCD keeps to its column tiles.
+size_t gemm_i8_grid(const GemmI8Shape &sh, size_t m, size_t n) {
+    const size_t ty = (m + sh.rows() - 1) / sh.rows(), t = gemm_i8_tiles(sh, m, n);
+    return 8 % ty == 0 ? (t + 7) / 8 * 8 : t;
+}
+
+// Estimate per (shape, splits), in us, fitted to whole-call times of Q4_K products of 32 to 2048 rows
+// against 1024 to 24576 weight rows of 4096 and 12288 columns (Q6_K runs ~10 % longer with the same ordering): the preparation, a fixed part,
+// the super-blocks a workgroup walks at a cost that grows with the workgroups at work (a large workgroup:
+// 5.0 us a super-block with 74 at work, 6.6 with 256; a small one: 2.5 with 64, 3.0 with 256, 4.7 when two
+// share every compute unit), the starts of further rounds, and the sum's launch and its (splits + 1) m n floats, which the
+// last-level cache holds.  Over 1321 shapes of Q4_K, Q6_K, Q8_0 and MXFP4 (9 to 2048 rows, 512 to 32000 x 1024 to 16384) the
+// picks are 0.6 % off the best measured choice on average, 4 % at the 95th percentile, 19 % at worst.
+// Whole rounds of workgroups, then what is left at its own cost (a last round of half the workgroups or fewer is short:
+// 333 x 12288 x 4096 of Q6_K in four parts, 768 workgroups of 128 x 64, 111 us; in three, 576 of them, 137).  The empty
+// workgroups count: they go to the last XCDs, and the first ones hold as many more (215 x 3910 x 8960 of Q8_0 as seven parts of 35
+// tiles, 245 large workgroups in a grid of 280, 35 of them on an XCD's 32 compute units: 88 us; five parts of 41, 59).
+double gemm_i8_us(const GemmI8Shape &sh, size_t m, size_t nb, size_t n, size_t sp) {
+    auto rounds = [](double wgs, double at_once, auto us) {
+        const double whole = std::floor(wgs / at_once), rest = wgs - whole * at_once;
+        return whole * us(at_once) + (rest > 0.0 ? us(rest) : 0.0);
+    };
+    const double wgs = (double)(gemm_i8_grid(sh, m, n) * sp), nbl = (double)(nb / sp);
+    double us = 3.0 + 0.0035 * (double)(nb * ((m + 15) / 16));
+    if (sh.nsplit)  // 3.1 us a super-block with 64 at work, 3.4 with 256, 4.4 with 512 (two a compute unit), in whole rounds
+        us += 3.9 + nbl * (2.95 + 0.0029 * std::min(wgs, 512.0)) *
+                        (wgs <= 512.0 ? 1.0 : wgs < 2048.0 ? std::ceil(wgs / 512.0) : wgs / 512.0);
+    else if (sh.nw == 8)  // (six groups of weight rows instead of seven: six sevenths of the work a super-block)
+        us += 10.0 + nbl * rounds(wgs, 256.0, [](double w) { return 4.3 + 0.009 * w; }) * (sh.ng == 7 ? 1.0 : 0.88) +
+              6.0 * (std::ceil(wgs / 256.0) - 1.0);
+    else
+        us += 3.9 + nbl * rounds(wgs, 512.0, [](double w) { return w <= 256.0 ? 2.3 + 0.0027 * w : 3.1 + 0.0032 * w; }) +
+              3.0 * std::max(0.0, wgs / 512.0 - 1.5);
+    if (sp > 1) us += 1.0 + 0.8 * (double)sp + (double)(sp + 1) * (double)(m * n) * 4.0 / 8.0e6;
+    return us;
+}
+
+// The shape and split over k (its parts summed by splitk_sum; only where tiles alone leave compute units idle) of the least estimate among those
+// that `may(shape, splits)` admits: the estimate, a negative one if there is none.
+template <class May>
+double gemm_i8_pick(size_t m, size_t nb, size_t n, GemmI8Shape &best, size_t &splits, May may) {
+    double best_us = -1.0;
+    for (const GemmI8Shape &sh : GEMM_I8_SHAPES)
+        for (size_t sp = 1; sp <= 8; sp++) {
+            if (nb % sp != 0 || (sp > 1 && nb / sp < 4) || !may(sh, sp)) continue;
+            const double us = gemm_i8_us(sh, m, nb, n, sp);
+            if (best_us < 0.0 || us < best_us) best = sh, splits = sp, best_us = us;
+        }
+    return best_us;
+}
+
+double gemm_i8_best_us(size_t m, size_t k, size_t n) {  // scratch as large as it wants
+    GemmI8Shape best;
+    size_t splits;
+    return gemm_i8_pick(m, k / 256, n, best, splits, [&](const GemmI8Shape &sh, size_t) { return !sh.nsplit || m <= 32; });
+}
+
 // Many activation rows on the int8 matrix cores (Q4_K up to 127 of them, gemm_h6's products from there on): the activations as two int8 planes per
 // 256-element super-block in the call scratch of the stream, then kq_gemm_i8 with the workgroup shape and the
 // split over k that an estimate fitted to measurements prefers.  Returns -1 when the shape is outside its
 // reach or the product is tiny.  JQ_Q4K_GEMM_I8 = 0 switches it off; JQ_Q4K_GEMM_I8_SHAPE and _SPLITS force the
 // choice, _MIN_TILES moves the floor (small tiles times the splits that k allows; default 64), _MIN_M the
 // fewest activation rows (default: min_m_default, 64 for Q4_K, which has kernels of its own below that).
-struct GemmI8Shape {
-    int nw, ng;
-    bool nsplit;  // tiles of 32 activation rows whose waves share the weight rows
-};
-
 template <class F>
 int dispatch_gemm_i8(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n,
                      hipStream_t s, const char *name, const char *name_split, bool swiglu_pairs = false,
@@ -712,83 +779,30 @@ int dispatch_gemm_i8(const uint8_t *W, size_t row_bytes, const float *X, float *
     if ((mode && mode[0] == '0') || m < min_m || k % 256 != 0 || row_bytes % ALIGN != 0 || ((uintptr_t)W & (ALIGN - 1)) != 0 ||
         ((uintptr_t)X & 15) != 0 || m > 0x7FFFFFF0ull || n > 0x7FFFFFF0ull)
         return -1;
-    // Two workgroup shapes: 256 x 112 outputs (eight waves, one workgroup a compute unit) and 128 x 64 (four
-    // waves, two a compute unit), and a split over k (the parts summed by splitk_sum) when the tiles alone leave
-    // compute units idle: every workgroup then walks nb / splits super-blocks.
-    // Up to 32 rows also: 32 x 64 (two waves that share the weight rows, two workgroups a compute unit).
-    static const GemmI8Shape shapes[] = {{8, 7, false}, {8, 6, false}, {4, 4, false}, {2, 4, true}};
     const size_t nb = k / 256, groups = (m + 15) / 16;
-    auto tiles_of = [&](const GemmI8Shape &sh) {
-        const size_t mt = sh.nsplit ? 32 : 32 * (size_t)sh.nw, nt = 16 * (size_t)sh.ng;
-        return ((m + mt - 1) / mt) * ((n + nt - 1) / nt);
-    };
-    // Workgroups of a launch of that many tiles: rounded up to eights (the rest empty) where the row tiles divide 8, so that
-    // an XCD keeps to its column tiles.
-    auto grid_of = [&](const GemmI8Shape &sh) {
-        const size_t mt = sh.nsplit ? 32 : 32 * (size_t)sh.nw, ty = (m + mt - 1) / mt, t = tiles_of(sh);
-        return 8 % ty == 0 ? (t + 7) / 8 * 8 : t;
-    };
-    if (tiles_of(shapes[2]) * std::max<size_t>(1, std::min<size_t>(nb / 4, 8)) < min_tiles) return -1;
-    // Estimate per (shape, splits), in us, fitted to whole-call times of Q4_K products of 32 to 2048 rows
-    // against 1024 to 24576 weight rows of 4096 and 12288 columns (Q6_K runs ~10 % longer with the same ordering): the preparation, a fixed part,
-    // the super-blocks a workgroup walks at a cost that grows with the workgroups at work (a large workgroup:
-    // 5.0 us a super-block with 74 at work, 6.6 with 256; a small one: 2.5 with 64, 3.0 with 256, 4.7 when two
-    // share every compute unit), the starts of further rounds, and the sum's launch and its (splits + 1) m n floats, which the
-    // last-level cache holds.  Over 1321 shapes of Q4_K, Q6_K, Q8_0 and MXFP4 (9 to 2048 rows, 512 to 32000 x 1024 to 16384) the
-    // picks are 0.6 % off the best measured choice on average, 4 % at the 95th percentile, 19 % at worst.
+    if (gemm_i8_tiles(GEMM_I8_SHAPES[2], m, n) * std::max<size_t>(1, std::min<size_t>(nb / 4, 8)) < min_tiles) return -1;
     const size_t acts_bytes = (groups * nb * (size_t)jq::QI_REC + 255) & ~(size_t)255;
     const size_t scratch_cap = tl_fixed_scratch ? tl_fixed_scratch->bytes : (size_t)1 << 40;
-    // Whole rounds of workgroups, then what is left at its own cost (a last round of half the workgroups or fewer is short:
-    // 333 x 12288 x 4096 of Q6_K in four parts, 768 workgroups of 128 x 64, 111 us; in three, 576 of them, 137).  The empty
-    // workgroups count: they go to the last XCDs, and the first ones hold as many more (215 x 3910 x 8960 of Q8_0 as seven parts of 35
-    // tiles, 245 large workgroups in a grid of 280, 35 of them on an XCD's 32 compute units: 88 us; five parts of 41, 59).
-    auto rounds = [](double wgs, double at_once, auto us) {
-        const double whole = std::floor(wgs / at_once), rest = wgs - whole * at_once;
-        return whole * us(at_once) + (rest > 0.0 ? us(rest) : 0.0);
-    };
-    auto estimate = [&](const GemmI8Shape &sh, size_t sp) {
-        const double wgs = (double)(grid_of(sh) * sp), nbl = (double)(nb / sp);
-        double us = 3.0 + 0.0035 * (double)(nb * groups);
-        if (sh.nsplit)  // 3.1 us a super-block with 64 at work, 3.4 with 256, 4.4 with 512 (two a compute unit), in whole rounds
-            us += 3.9 + nbl * (2.95 + 0.0029 * std::min(wgs, 512.0)) *
-                            (wgs <= 512.0 ? 1.0 : wgs < 2048.0 ? std::ceil(wgs / 512.0) : wgs / 512.0);
-        else if (sh.nw == 8)  // (six groups of weight rows instead of seven: six sevenths of the work a super-block)
-            us += 10.0 + nbl * rounds(wgs, 256.0, [](double w) { return 4.3 + 0.009 * w; }) * (sh.ng == 7 ? 1.0 : 0.88) +
-                  6.0 * (std::ceil(wgs / 256.0) - 1.0);
-        else
-            us += 3.9 + nbl * rounds(wgs, 512.0, [](double w) { return w <= 256.0 ? 2.3 + 0.0027 * w : 3.1 + 0.0032 * w; }) +
-                  3.0 * std::max(0.0, wgs / 512.0 - 1.5);
-        if (sp > 1) us += 1.0 + 0.8 * (double)sp + (double)(sp + 1) * (double)(m * n) * 4.0 / 8.0e6;
-        return us;
-    };
-    const GemmI8Shape *best = nullptr;
-    size_t splits = 1;
-    double best_us = 0.0;
     static const char *splits_env = getenv("JQ_Q4K_GEMM_I8_SPLITS");
     int want_nw = 0, want_ng = 0;
     const bool forced = shape_env && sscanf(shape_env, "%d,%d", &want_nw, &want_ng) == 2;
-    for (const GemmI8Shape &sh : shapes) {
-        if (forced && (sh.nw != want_nw || sh.ng != want_ng)) continue;
-        if (sh.nsplit && !forced && m > 32) continue;
-        for (size_t sp = 1; sp <= 8; sp++) {
-            if (nb % sp != 0 || (sp > 1 && nb / sp < 4)) continue;
-            if (splits_env && sp != (size_t)atoi(splits_env)) continue;
-            if (sp > 1 && (m * n > 0x3FFFFFFFull || acts_bytes + sp * m * n * sizeof(float) > scratch_cap)) continue;
-            const double us = estimate(sh, sp);
-            if (!best || us < best_us) best = &sh, splits = sp, best_us = us;
-        }
-    }
-    if (!best) return -1;
+    GemmI8Shape best{};
+    size_t splits = 1;
+    const double us = gemm_i8_pick(m, nb, n, best, splits, [&](const GemmI8Shape &sh, size_t sp) {
+        if (forced ? sh.nw != want_nw || sh.ng != want_ng : sh.nsplit && m > 32) return false;
+        if (splits_env && sp != (size_t)atoi(splits_env)) return false;
+        return sp == 1 || (m * n <= 0x3FFFFFFFull && acts_bytes + sp * m * n * sizeof(float) <= scratch_cap);
+    });
+    if (us < 0.0) return -1;
     CallScratch scratch;
     uint8_t *acts = nullptr;
     if (scratch.get(acts_bytes + (splits > 1 ? splits * m * n * sizeof(float) : 0), s, &acts)) return 1;
     float *parts = (float *)(acts + acts_bytes);
-    const size_t mt = best->nsplit ? 32 : 32 * (size_t)best->nw, nt = 16 * (size_t)best->ng;
-    const size_t tx = (n + nt - 1) / nt, ty = (m + mt - 1) / mt, grid = grid_of(*best);
+    const size_t tx = (n + best.cols() - 1) / best.cols(), ty = (m + best.rows() - 1) / best.rows(), grid = gemm_i8_grid(best, m, n);
     if (grid > 0x7FFFFFFFull) return -1;
     hipError_t attr_rc = hipSuccess;
 #define JQ_GEMM_I8(NW_, NG_, NSPLIT_)                                                                                 \
-    if (best->nw == NW_ && best->ng == NG_) {                                                                         \
+    if (best.nw == NW_ && best.ng == NG_) {                                                                         \
         auto kern = jq::kq_gemm_i8<F, NW_, NG_, false, NSPLIT_>;                                                      \
         constexpr int lds = jq::qi_lds_bytes<F, NG_>();                                                                  \
         static std::once_flag big_lds;                                                                                \
@@ -920,23 +934,31 @@ int dispatch_gemm_decoded(uint32_t type, const uint8_t *W, size_t row_bytes, con
 // rows that are no multiple of 4096 long 10 to 40 / 11 to 134; the others have dispatch_q4k_rows16, whose time does not grow with the
 // rows (4096 x 4096: 7.4 to 8.8 / 9.3; 14336 x 4096: 12.7 to 17 / 14.6; 4096 x 12288: 16 to 20 / 23; 12000 x 8192: 21 to 29 / 24).
 //
-// 17 rows and more: where its estimate is below that of what would run else, fitted to 24 shapes of 17 to 256 rows: the int8 GEMM, with at
-// most 127 rows 14.6 us and 0.62 a million weights (23 to 52 us at 4096 x 4096 to 14336 x 4096) or 0.5 a super-block of k, a third
-// more beyond (MXFP4, gemm_h6's there: a tenth); Q4_K a tenth less; rows of 4096 also dispatch_q4k_rows16's passes.  us, before / now: 32 rows x 14336 x 4096 Q4_K 27 / 19,
-// Q6_K 43 / 26, MXFP4 42 / 17; 64 rows x 3000 x 2560 22 to 25 / 11 to 12; 96 rows x 4096 x 4096 24 to 26 / 17 to 19;
-// 64 rows x 9000 x 9984 Q6_K 71 / 71, 127 rows 79 / 109 (hence the margin).  From 128 rows Q4_K is gemm_h6's, and prepared
+// 17 rows and more: where its estimate is below that of what would run else.  From 64 rows on that is a many-row GEMM's own, times what
+// calls of the format with weights from memory came to of it.  Fewer rows: the int8 GEMM's 14.6 us and 0.62 a million weights (23 to 52 us at
+// 4096 x 4096 to 14336 x 4096) or 0.5 a super-block of k, and the kernels of products under 8M weights, which take about as long; Q4_K a
+// tenth less; rows of 4096 also dispatch_q4k_rows16's passes.  us, before / now: 32 rows x 14336 x 4096 Q4_K 27 / 19, Q6_K 43 / 26, MXFP4
+// 42 / 17; 64 rows x 3000 x 2560 22 to 25 / 11 to 12; 96 rows x 4096 x 4096 24 to 26 / 17 to 19.  Of 96 rows and more against many weight
+// rows the rounds of workgroups weigh most, each with a start of its own (few_rows_many / GEMM: 128 rows x 14336 x 2304 Q6_K 50 / 39, MXFP4 40 /
+// 30; 127 x 24576 x 1024 Q4_K 37 / 26).  Over 2727 shapes of 17 to 255 rows, 576 to 24576 x 1024 to 12288, the choice is right but
+// for some 25, by 5 to 17 %.  From 128 rows Q4_K is gemm_h6's, and prepared
 // activations that the second level cache of an XCD does not hold are slow (200 rows x 1100 x 12288 41 / 55).
 bool few_rows_better(uint32_t type, size_t m, size_t k, size_t n) {
     static const char *off = getenv("JQ_FEW_ROWS"), *i8_shape = getenv("JQ_Q4K_GEMM_I8_SHAPE"), *i8_min_m = getenv("JQ_Q4K_GEMM_I8_MIN_M");
     if (off && off[0] == '0') return false;
     if (m > 16) {
         const bool q4 = type == JQ_TYPE_Q4_K;
-        if ((!q4 && type != JQ_TYPE_Q6_K && type != JQ_TYPE_Q8_0 && type != JQ_TYPE_MXFP4) || i8_shape || i8_min_m || n < 512 || k < 1024 ||
+        if ((!q4 && type != JQ_TYPE_Q6_K && type != JQ_TYPE_Q8_0 && type != JQ_TYPE_MXFP4) || i8_shape || i8_min_m || n < 512 || k < 1024 || k % 256 != 0 ||
             n * k < ((size_t)2 << 20) || m > (q4 ? 127 : 255) || (m > 127 && m * k > 1500000))
             return false;
-        double us = std::max(14.6 + 0.62e-6 * (double)(n * k), 9.0 + 0.5 * (double)(k / 256)) * (m > 127 ? type == JQ_TYPE_MXFP4 ? 1.1 : 1.3 : 1.0) * (q4 ? 0.9 : 1.0);
-        if (q4 && k == 4096) us = std::min(us, 3.0 + (double)((m + 15) / 16) * (4.3 + 0.527 * (double)n / 1024.0));
-        return few_rows_many_us(type, m, k, n) < 0.92 * us;
+        const double rows16_us = q4 && k == 4096 ? 3.0 + (double)((m + 15) / 16) * (4.3 + 0.527 * (double)n / 1024.0) : HUGE_VAL, mine = few_rows_many_us(type, m, k, n);
+        if (m >= 64) {
+            if (type == JQ_TYPE_MXFP4 && m > 127) return mine < 0.95 * gemm_h6_us(m, k, n);
+            const double to = q4 ? 0.97 : type == JQ_TYPE_MXFP4 ? 1.08 : m > 127 ? 1.09 : 1.2;
+            return mine < std::min(to * gemm_i8_best_us(m, k, n), rows16_us);
+        }
+        const double us = std::max(14.6 + 0.62e-6 * (double)(n * k), 9.0 + 0.5 * (double)(k / 256)) * (q4 ? 0.9 : 1.0);
+        return mine < 1.1 * std::min(us, rows16_us);
     }
     const size_t weights = n * k;
     switch (type) {

@@ -13,6 +13,53 @@ hipError_t big_lds_once(int lds) {
     return rc;
 }
 
+struct Shape {
+    int nw, ng;
+    // tiles of the activation rows, of the weight rows, workgroups of a launch
+    size_t rows(size_t m) const { return (m + 32 * (size_t)nw - 1) / (32 * (size_t)nw); }
+    size_t cols(size_t n) const { return (n + 16 * (size_t)ng - 1) / (16 * (size_t)ng); }
+    size_t grid(size_t m, size_t n) const {
+        const size_t ty = rows(m), tiles = ty * cols(n);
+        return 8 % ty == 0 ? (tiles + 7) / 8 * 8 : tiles;
+    }
+};
+constexpr Shape SHAPES[] = {{8, 8}, {8, 7}, {8, 6}, {4, 4}};
+
+// In us, the int8 GEMM's form of estimate (gemm_i8_us) fitted to 714 times of this one's shapes of seven, six and four groups in 1 to 8
+// parts (eight groups: 1.09 of seven's super-block, 512 to 2048 rows x 4096 to 24576): the
+// preparation, a fixed start, the super-blocks a workgroup walks at a cost that grows with the workgroups at work, the
+// starts of further rounds, the sum of the parts.  Over 166 shapes the picks are 0.7 % off the best measured choice on
+// average, 5 % at the 95th percentile, 12 % at worst.
+double estimate(const Shape &sh, size_t m, size_t nb, size_t n, size_t sp) {
+    auto rounds = [](double wgs, double at_once, auto us) {
+        const double whole = std::floor(wgs / at_once), rest = wgs - whole * at_once;
+        return whole * us(at_once) + (rest > 0.0 ? us(rest) : 0.0);
+    };
+    const double wgs = (double)(sh.grid(m, n) * sp), nbl = (double)(nb / sp);
+    double us = 3.2 + 0.0048 * (double)(nb * ((m + 15) / 16));
+    if (sh.nw == 8)
+        us += 6.4 + nbl * rounds(wgs, 256.0, [](double w) { return 3.4 + 0.0035 * w; }) * (sh.ng == 8 ? 1.09 : sh.ng == 7 ? 1.0 : 0.92) +
+              4.2 * (std::ceil(wgs / 256.0) - 1.0);
+    else
+        us += 6.6 + nbl * rounds(wgs, 512.0, [](double w) { return w <= 256.0 ? 2.24 + 0.0011 * w : 3.06 + 0.0011 * w; }) +
+              2.5 * std::max(0.0, wgs / 512.0 - 1.5);
+    if (sp > 1) us += 0.09 * (double)sp + (double)(sp + 1) * (double)(m * n) * 4.0 / 3.4e6;
+    return us;
+}
+
+// The shape and split over k of the least estimate among those that `may(shape, splits)` admits: the estimate, a negative one if there is none.
+template <class May>
+double pick(size_t m, size_t nb, size_t n, Shape &best, size_t &splits, May may) {
+    double best_us = -1.0;
+    for (const Shape &sh : SHAPES)
+        for (size_t sp = 1; sp <= 8; sp++) {
+            if (nb % sp != 0 || (sp > 1 && nb / sp < 4) || !may(sh, sp)) continue;
+            const double us = estimate(sh, m, nb, n, sp);
+            if (best_us < 0.0 || us < best_us) best = sh, splits = sp, best_us = us;
+        }
+    return best_us;
+}
+
 // Q4_K and MXFP4 with 128 activation rows or more on f16 and FP6 operands (kq_gemm_h6), us against the int8 GEMM's, whole calls back to back (Q4_K):
 // 512 x 14336 x 4096 95 / 116, 2048 x 24576 x 4096 604 / 738, 512 x 4096 x 4096 48 / 50.  166 shapes of 128 to 2048 rows against
 // 1000 to 24576 weight rows of 1024 to 16384: 0.77 to 1.08 of its time, 0.91 on average; the 18 that are more than 2 % slower, by
@@ -30,10 +77,6 @@ int dispatch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_
     if ((mode && mode[0] == '0') || i8_mode || i8_shape || m < min_m || k % 256 != 0 || k == 0 || row_bytes % F::ALIGN != 0 ||
         !jq::h6_offsets_hold(k / 256, row_bytes) || ((uintptr_t)W & (F::ALIGN - 1)) != 0 || ((uintptr_t)X & 15) != 0 || m > 0x7FFFFFF0ull || n > 0x7FFFFFF0ull)
         return -1;
-    struct Shape {
-        int nw, ng;
-    };
-    static constexpr Shape shapes[] = {{8, 8}, {8, 7}, {8, 6}, {4, 4}};
     const size_t nb = k / 256, groups = (m + 15) / 16;
     const size_t scratch_cap = tl_fixed_scratch ? tl_fixed_scratch->bytes : (size_t)1 << 40;
     // A fixed scratch that holds the int8 GEMM's records of all rows, three quarters of these in size, takes the rows in two turns;
@@ -46,52 +89,17 @@ int dispatch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_
         if (acts_of(turn) > scratch_cap) return -1;
     }
     const size_t acts_bytes = acts_of(turn);
-    // tiles of a turn's rows, of the weight rows, workgroups of its launch
-    auto rows_of = [&](const Shape &sh, size_t rows) { return (rows + 32 * (size_t)sh.nw - 1) / (32 * (size_t)sh.nw); };
-    auto cols_of = [&](const Shape &sh) { return (n + 16 * (size_t)sh.ng - 1) / (16 * (size_t)sh.ng); };
-    auto grid_of = [&](const Shape &sh, size_t rows) {
-        const size_t ty = rows_of(sh, rows), tiles = ty * cols_of(sh);
-        return 8 % ty == 0 ? (tiles + 7) / 8 * 8 : tiles;
-    };
-    if (!min_m_env && rows_of(shapes[3], m) * cols_of(shapes[3]) * std::max<size_t>(1, std::min<size_t>(nb / 4, 8)) < 64) return -1;
-    auto rounds = [](double wgs, double at_once, auto us) {
-        const double whole = std::floor(wgs / at_once), rest = wgs - whole * at_once;
-        return whole * us(at_once) + (rest > 0.0 ? us(rest) : 0.0);
-    };
-    // In us, the int8 GEMM's form of estimate (dispatch_gemm_i8) fitted to 714 times of this one's shapes of seven, six and four groups in 1 to 8 parts (eight groups: 1.09 of
-    // seven's super-block, 512 to 2048 rows x 4096 to 24576): the
-    // preparation, a fixed start, the super-blocks a workgroup walks at a cost that grows with the workgroups at work, the
-    // starts of further rounds, the sum of the parts.  Over 166 shapes the picks are 0.7 % off the best measured choice on
-    // average, 5 % at the 95th percentile, 12 % at worst.
-    auto estimate = [&](const Shape &sh, size_t sp) {
-        const double wgs = (double)(grid_of(sh, m) * sp), nbl = (double)(nb / sp);
-        double us = 3.2 + 0.0048 * (double)(nb * groups);
-        if (sh.nw == 8)
-            us += 6.4 + nbl * rounds(wgs, 256.0, [](double w) { return 3.4 + 0.0035 * w; }) * (sh.ng == 8 ? 1.09 : sh.ng == 7 ? 1.0 : 0.92) +
-                  4.2 * (std::ceil(wgs / 256.0) - 1.0);
-        else
-            us += 6.6 + nbl * rounds(wgs, 512.0, [](double w) { return w <= 256.0 ? 2.24 + 0.0011 * w : 3.06 + 0.0011 * w; }) +
-                  2.5 * std::max(0.0, wgs / 512.0 - 1.5);
-        if (sp > 1) us += 0.09 * (double)sp + (double)(sp + 1) * (double)(m * n) * 4.0 / 3.4e6;
-        return us;
-    };
-    const Shape *best = nullptr;
-    size_t splits = 1;
-    double best_us = 0.0;
+    if (!min_m_env && SHAPES[3].rows(m) * SHAPES[3].cols(n) * std::max<size_t>(1, std::min<size_t>(nb / 4, 8)) < 64) return -1;
     int want_nw = 0, want_ng = 0;
     const bool forced = shape_env && sscanf(shape_env, "%d,%d", &want_nw, &want_ng) == 2;
-    for (const Shape &sh : shapes) {
-        if (forced && (sh.nw != want_nw || sh.ng != want_ng)) continue;
-        for (size_t sp = 1; sp <= 8; sp++) {
-            if (nb % sp != 0 || (sp > 1 && nb / sp < 4)) continue;
-            if (splits_env && sp != (size_t)atoi(splits_env)) continue;
-            if (sp > 1 && (m * n > 0x3FFFFFFFull || acts_bytes + (sp - 1) * turn * n * sizeof(float) > scratch_cap)) continue;
-            const double us = estimate(sh, sp);
-            if (!best || us < best_us) best = &sh, splits = sp, best_us = us;
-        }
-    }
-    if (!best) return -1;
-    if (grid_of(*best, m) > 0x7FFFFFFFull) return -1;
+    Shape best{};
+    size_t splits = 1;
+    const double us = pick(m, nb, n, best, splits, [&](const Shape &sh, size_t sp) {
+        if (forced && (sh.nw != want_nw || sh.ng != want_ng)) return false;
+        if (splits_env && sp != (size_t)atoi(splits_env)) return false;
+        return sp == 1 || (m * n <= 0x3FFFFFFFull && acts_bytes + (sp - 1) * turn * n * sizeof(float) <= scratch_cap);
+    });
+    if (us < 0.0 || best.grid(m, n) > 0x7FFFFFFFull) return -1;
     CallScratch scratch;
     uint8_t *acts = nullptr;
     if (scratch.get(acts_bytes + (splits - 1) * turn * n * sizeof(float), s, &acts)) return 1;
@@ -105,16 +113,16 @@ int dispatch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_
             const dim3 prep((unsigned)nb, (unsigned)row_groups);
             if (swiglu_pairs) hipLaunchKernelGGL((jq::kq_gemm_h6_prep<true, F::MINS, F::NIBBLES>), prep, dim3(128), 0, s, x, (int)rows, (int)k, acts);
             else hipLaunchKernelGGL((jq::kq_gemm_h6_prep<false, F::MINS, F::NIBBLES>), prep, dim3(128), 0, s, x, (int)rows, (int)k, acts);
-            hipLaunchKernelGGL(kern, dim3((unsigned)grid_of(*best, rows), (unsigned)splits), dim3(64 * nw), lds, s, W, row_bytes,
+            hipLaunchKernelGGL(kern, dim3((unsigned)best.grid(rows, n), (unsigned)splits), dim3(64 * nw), lds, s, W, row_bytes,
                                (const uint8_t *)acts, y, (int)rows, (int)n, (int)(nb / splits), (int)row_groups,
-                               (int)cols_of(*best), (int)rows_of(*best, rows), (int)nb, parts);
+                               (int)best.cols(n), (int)best.rows(rows), (int)nb, parts);
             if (splits > 1)
                 hipLaunchKernelGGL(jq::splitk_add, dim3((unsigned)((outs + 1023) / 1024)), dim3(256), 0, s, parts, y, outs, (int)splits - 1);
         }
         return 0;
     };
 #define JQ_GEMM_H6(NW_, NG_) launch(jq::kq_gemm_h6<F, NW_, NG_>, jq::h6_lds_bytes<NG_>(), NW_, big_lds_once<&jq::kq_gemm_h6<F, NW_, NG_>>(jq::h6_lds_bytes<NG_>()))
-    const int rc = best->nw == 4 ? JQ_GEMM_H6(4, 4) : best->ng == 8 ? JQ_GEMM_H6(8, 8) : best->ng == 7 ? JQ_GEMM_H6(8, 7) : JQ_GEMM_H6(8, 6);
+    const int rc = best.nw == 4 ? JQ_GEMM_H6(4, 4) : best.ng == 8 ? JQ_GEMM_H6(8, 8) : best.ng == 7 ? JQ_GEMM_H6(8, 7) : JQ_GEMM_H6(8, 6);
 #undef JQ_GEMM_H6
     if (rc) return rc;
     note_kernel(splits > 1 ? name_split : name, "f16+fp6");
@@ -123,6 +131,12 @@ int dispatch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_
 }
 
 }  // namespace
+
+double gemm_h6_us(size_t m, size_t k, size_t n) {
+    Shape best;
+    size_t splits;
+    return pick(m, k / 256, n, best, splits, [](const Shape &, size_t) { return true; });
+}
 
 int gemm_h6(uint32_t type, const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n, hipStream_t s,
             const char *name, const char *name_split, bool swiglu_pairs) {

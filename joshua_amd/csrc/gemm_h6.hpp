@@ -10,5 +10,6 @@ constexpr size_t INT8_GEMM_REC = 9280;  // bytes of the int8 GEMM's record of 16
 // gate_j and up_j alternate.  -1: the call is outside its reach.
 int gemm_h6(uint32_t type, const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n, hipStream_t s,
             const char *name, const char *name_split, bool swiglu_pairs = false);
+double gemm_h6_us(size_t m, size_t k, size_t n);  // its time by estimate, scratch as large as it wants
 
 }  // namespace jqh

@@ -211,3 +211,17 @@ def test_few_weight_rows_keep_the_kernels_that_are_faster_there(qtype, m, k, n, 
     assert capi.last_kernel() == kernel if kernel else capi.last_arithmetic() == "f16 pairs"
     want = oracle.matmul_t(qtype, (m, k, n), lhs, blocks, avx2=oracle.have_avx2())
     assert np.all(np.abs(got - want) <= 1e-3 * np.maximum(np.abs(want), 1.0))
+
+
+@pytest.mark.parametrize("qtype,m,k,n,kernel", [
+    (capi.Q4_K, 127, 1024, 14336, "q4k_gemm_i8"), (capi.Q6_K, 128, 2304, 14336, "q6k_gemm_i8"), (capi.Q8_0, 127, 1024, 14336, "q8_0_gemm_i8"),
+    (capi.MXFP4, 128, 2304, 14336, "mxfp4_gemm_i8"), (capi.MXFP4, 160, 1024, 24576, "mxfp4_gemm_i8"), (capi.Q6_K, 200, 7168, 576, "q6k_gemm_i8+splitk"),
+    (capi.Q4_K, 64, 1024, 9000, "few_rows_many"), (capi.Q6_K, 144, 9984, 700, "few_rows_many"), (capi.Q8_0, 80, 2048, 11008, "few_rows_many"),
+    (capi.MXFP4, 130, 9984, 1500, "few_rows_many")])
+def test_some_hundred_rows_go_where_they_are_faster(qtype, m, k, n, kernel):
+    """Shapes on either side of the line between few_rows_many and the GEMMs behind it, each at least a sixth slower on the other."""
+    blocks, lhs = synth.normal_quantized(qtype, 72, n * k, 0.02), synth.normal(73, (m, k))
+    got = capi.Weight.upload(qtype, blocks, n, k).matmul_t(m, lhs)
+    assert capi.last_kernel() == kernel or not ON
+    want = lhs.astype(np.float64) @ oracle.dequantize(qtype, blocks).reshape(n, k).astype(np.float64).T
+    assert np.all(np.abs(got - want) <= 1e-3 * np.maximum(np.abs(want), 1.0))
