@@ -932,7 +932,7 @@ int dispatch_gemm_decoded(uint32_t type, const uint8_t *W, size_t row_bytes, con
 // 6.1, 2048 x 12288 17.2 / 13.9 (the one-row kernel twice).  MXFP4 1 row 1024 x 16384 17.8 / 14.4; 2 rows 1024 x 2048 5.2 / 4.7.
 // Q4_K: two rows are faster on the one-row kernels' up to 64M weights (11008 x 3840 13.4 / 12.2, 14336 x 11264 28 / 47).  More:
 // rows that are no multiple of 4096 long 10 to 40 / 11 to 134; the others have dispatch_q4k_rows16, whose time does not grow with the
-// rows (4096 x 4096: 7.4 to 8.8 / 9.3; 14336 x 4096: 12.7 to 17 / 14.6; 4096 x 12288: 16 to 20 / 23; 12000 x 8192: 21 to 29 / 24).
+// rows (4096 x 4096: 7.4 to 8.8 / 9.3; 14336 x 4096: 12.7 to 17 / 14.6; 4096 x 12288: 16 to 20 / 23; 12000 x 8192: 21 to 29 / 24; 24576 x 12288 of 3 to 8 rows: 62 to 64 / 59 to 56).
 //
 // 17 rows and more: where its estimate is below that of what would run else.  From 64 rows on that is a many-row GEMM's own, times what
 // calls of the format with weights from memory came to of it.  Fewer rows: the int8 GEMM's 14.6 us and 0.62 a million weights (23 to 52 us at
@@ -965,7 +965,7 @@ bool few_rows_better(uint32_t type, size_t m, size_t k, size_t n) {
     case JQ_TYPE_Q4_K:
         if (m == 1 || n < 1024 || k < 1024) return false;
         if (m == 2) return weights >= ((size_t)64 << 20) && k != 4096;
-        return k % 4096 != 0 || k > 4 * 4096 || (m <= 8 ? k > 4096 || n <= 8192 : n <= 4096);
+        return k % 4096 != 0 || k > 4 * 4096 || (m <= 8 ? (k > 4096 && n <= 16384) || n <= 8192 : n <= 4096);
     case JQ_TYPE_Q6_K: return weights >= (m == 1 ? (size_t)64 << 20 : (size_t)2 << 20) && n >= (m <= 2 ? 3072 : m == 3 ? 2048 : m == 4 || (m == 5 && k % 4096 == 0) ? 1280 : 1);
     case JQ_TYPE_Q8_0:
         if (m == 1) return weights >= ((size_t)8 << 20) && n >= 2560;
