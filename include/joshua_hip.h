@@ -142,7 +142,9 @@ const void *jq_device_ptr(const jq_weight *w);
  *   of four significant bits, relative to each element down to 2^-19 of the super-block's largest.
  *   MXFP4's are exact where f16 holds all 256 behind a power of two (bf16 values) or all have one
  *   magnitude, and its weights where the scales of a 256-run lie within 2^26 of the largest (2^-19 of
- *   themselves off within 2^36, zeros from 2^60 on).
+ *   themselves off within 2^36, zeros from 2^60 on).  Where a scale times the
+ *   activations' largest is below 2^-99, the factor in front of their sums is a subnormal f32
+ *   (weights of 2^-107, activations of 1e-3: 6e-3 off).
  * A row holding an inf or a NaN comes out without a finite value. */
 int jq_matmul_t(const jq_weight *w, size_t m, const float *lhs, size_t lhs_len, float *dst,
                 size_t dst_len, int ptrs_are_device, void *stream);
