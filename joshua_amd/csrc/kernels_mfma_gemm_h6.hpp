@@ -336,8 +336,9 @@ __device__ __forceinline__ h6_i8 h6_operand6(h6_u6 v) {
     return h6_i8{(int)v[0], (int)v[1], (int)v[2], (int)v[3], (int)v[4], (int)v[5], 0, 0};
 }
 
+// (Four waves: two workgroups a compute unit.  Not told so, the compiler keeps the sums in accumulation registers and copies them out.)
 template <class F, int NW, int NG>
-static __global__ __launch_bounds__(64 * NW) void kq_gemm_h6(const uint8_t *__restrict__ W, size_t row_bytes,
+static __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void kq_gemm_h6(const uint8_t *__restrict__ W, size_t row_bytes,
                                                       const uint8_t *__restrict__ acts, float *__restrict__ Y, int m_rows, int n,
                                                       int nb, int groups, int tx, int ty, int nb_total, float *__restrict__ parts) {
     static_assert(NG <= NW && NG <= 8, "one group of 16 weight rows a wave unpacks, a byte each of a lane's eight exponents");
