@@ -2593,9 +2593,20 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
     }
     if (comp == m->comp && dispatch_matmul(m->kv_a->type, m->kv_a->dev, m->kv_a->row_bytes, x, m->comp, S, c.n_embd, lkv + rope, s))
         return 1;
+    static const char *no_absorb_rope = getenv("JQ_MLA_NO_ABSORB_ROPE"), *mla_env = getenv("JQ_MLA_ATTENTION"), *split_env = getenv("JQ_MLA_SPLIT");
+    // One token over a context of up to 900 or so and those blocks: from the query to the output projection in one launch, whose workgroups,
+    // one a compute unit, each read the whole context.  A layer's step, us, three launches / one: 128 heads behind 61 tokens 44.8 /
+    // 37.4, 320 53.5 / 42.7, 640 55.4 / 50.3, 1000 59.0 / 58.6, 1300 62 / 66; 64 heads behind 61 34.9 / 27.8, 1000 48.4 / 45.5, 1300 51 /
+    // 53; 16 heads behind 61 28.6 / 21.9, 1000 50.5 / 42.0, 1560 55 / 57.
+    constexpr size_t MLA_STEP_CONTEXT = 896;
+    if (kv_q4k && pos < MLA_STEP_CONTEXT && rope == jq::MLA_M_ROPE && nh * (vh / 64) <= 256 && !no_absorb_rope && !mla_env && !split_env) {
+        hipLaunchKernelGGL(jq::mla_step_q4k, dim3((unsigned)nh, (unsigned)(vh / 64)), dim3(1024), 0, s, (const float *)m->qv, (const uint8_t *)m->kv_b->dev,
+                           m->ctx, (int)vh, comp, (const float *)m->kv_a_norm, (const float2 *)m->cs, m->lat, m->kpe, (int)pos, c.rms_eps, m->scale);
+        HIP_TRY(hipGetLastError());
+        return dispatch_matmul(m->o->type, m->o->dev, m->o->row_bytes, m->ctx, out, S, nh * vh, c.n_embd, s);
+    }
     const bool vec4 = lkv % 4 == 0;
     const unsigned st = S == 1 ? 1 : 4;
-    static const char *no_absorb_rope = getenv("JQ_MLA_NO_ABSORB_ROPE");
     if (S == 1 && !no_absorb_rope) {
         // one token: the rotation / latent kernel's work rides in a wave of the absorption's workgroups
         if (kv_q4k)
@@ -2638,12 +2649,10 @@ int mla_forward_dev(jq_mla *m, size_t S, size_t pos, const float *x, float *out,
     }
     const size_t total = pos + S;
     size_t n_split;
-    static const char *mla_env = getenv("JQ_MLA_ATTENTION");  // "valu": never the matrix-core kernel
-    const bool mfma = lkv == jq::MLA_M_LKV && rope == jq::MLA_M_ROPE && nh % 32 == 0 && nope % 4 == 0 && !(mla_env && !strcmp(mla_env, "valu"));
+    const bool mfma = lkv == jq::MLA_M_LKV && rope == jq::MLA_M_ROPE && nh % 32 == 0 && nope % 4 == 0 && !(mla_env && !strcmp(mla_env, "valu"));  // "valu": never the matrix-core kernel
     // One token over a short context: waves of two heads and 16 tokens (a layer's step of 128 heads, us, matrix cores / this: behind
     // 4 tokens 51.3 / 44.6, 100 tokens 52.3 / 46.5, 230 tokens 53.4 / 49.9, 460 tokens 54.7 / 55.0, 950 tokens 59.5 / 68.1).
     constexpr size_t MLA_SHORT_CONTEXT = 320;
-    static const char *split_env = getenv("JQ_MLA_SPLIT");
     if (S == 1 && total <= MLA_SHORT_CONTEXT && !mla_env && !split_env && lkv == jq::MLA_M_LKV && rope == jq::MLA_M_ROPE && nh % 8 == 0 && nope % 4 == 0) {
         n_split = (total + jq::MLA_SHORT_TOKENS - 1) / jq::MLA_SHORT_TOKENS;
         hipLaunchKernelGGL(jq::mla_attention_short, dim3((unsigned)(nh / 8), (unsigned)n_split), dim3(256), 0, s, (const float *)m->qabs,

@@ -15,7 +15,7 @@
 //                     context split over workgroups (partial maximum, sum and vector per split)
 //   mla_merge         merge the splits into o_lat[h]
 //   mla_vproj         ctx[h] = W_v[h] o_lat[h]
-// (one token over a Q4_K up-projection: mla_absorb_rope_q4k, the attention, mla_merge_vproj_q4k)
+// (one token over a Q4_K up-projection: mla_step_q4k, behind a long context mla_absorb_rope_q4k, the attention, mla_merge_vproj_q4k)
 // around the quantized projections (q, kv_a, o), which run on the matmul kernels.
 #pragma once
 #include "kernels_graph.hpp"
@@ -612,6 +612,184 @@ __global__ __launch_bounds__(512) void mla_merge_vproj_q4k(const float *__restri
         if (lane == i) mine = y;
     }
     if (lane < ROWS && row0 + lane < vh) ctx[(size_t)h * vh + row0 + lane] = mine;
+}
+
+// Everything of a step between the query and the output projection in one launch, for one token over a short context and Q4_K blocks
+// of 128 key and vh value rows of 512 columns a head.  grid (n_head, vh / 64), 16 waves: a workgroup absorbs its head's query (a
+// quarter-wave a row and super-block, a lane two words of it), rotates the query's rope part, norms the new token's latent and rotates
+// its key (everybody makes them for himself, the first workgroup appends them to the cache), scores the cached tokens, a wave eight at a
+// time with their rows in registers, merges the waves' sums and multiplies with 64 value rows.  f32 throughout.
+// Bound: a chain of some 900 vector instructions a wave, four waves a SIMD, and three trips to memory.  128 heads of 128 + 64 elements
+// behind 100 tokens: 9.5 to 11.5 us where absorbing, scoring and merging with the value rows, a launch each, take 6.2, 5.1 and 5.0 and
+// their boundaries: a layer's step 44.6 -> 37.0 us.  All value rows in one workgroup a head, half the compute units idle: 37.5.
+__device__ __forceinline__ float mla_sum_half(float v) {  // over the 32 lanes of a half-wave
+    v = sum_xor16(v);
+    return sum_row16(v);
+}
+struct MlaQ4kPair {  // two words next to each other: 8 columns of either sub-block
+    float lo[8], hi[8], dl, dh, ml, mh;
+};
+__device__ __forceinline__ MlaQ4kPair mla_q4k_pair(const uint4 &hdr, const uint2 &q, int c) {
+    MlaQ4kPair w;
+    const MlaQ4kWord a = mla_q4k_word(hdr, q.x, c);
+    w.dl = a.dl, w.dh = a.dh, w.ml = a.ml, w.mh = a.mh;
+    const uint32_t lo = q.y & 0x0F0F0F0Fu, hi = (q.y >> 4) & 0x0F0F0F0Fu;
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+        w.lo[b] = a.lo[b], w.hi[b] = a.hi[b];
+        w.lo[4 + b] = (float)((lo >> (8 * b)) & 0xFFu), w.hi[4 + b] = (float)((hi >> (8 * b)) & 0xFFu);
+    }
+    return w;
+}
+__global__ __launch_bounds__(1024) void mla_step_q4k(const float *__restrict__ q, const uint8_t *__restrict__ Wkv, float *__restrict__ ctx, int vh,
+                                                      const float *__restrict__ comp, const float *__restrict__ w,
+                                                      const float2 *__restrict__ cs, float *__restrict__ lat, float *__restrict__ kpe,
+                                                      int pos, float eps, float scale) {
+    constexpr int LKV = MLA_M_LKV, ROPE = MLA_M_ROPE, NOPE = 128, WAVES = 16, RUN = 4, N = 8;  // rows, tokens a wave at a time
+    __shared__ __attribute__((aligned(16))) float red[WAVES][LKV], mid[LKV];
+    __shared__ float max_sh[WAVES], sum_sh[WAVES];
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l = lane & 15, sb = (lane >> 4) & 1, half = lane >> 5, c = l >> 2, col = 256 * sb + 64 * c + 8 * (l & 3);
+    const float *qh = q + (size_t)h * (NOPE + ROPE);
+    const uint8_t *rows = Wkv + (size_t)h * (NOPE + vh) * (2 * 144) + 144 * sb;
+    uint4 hdr[RUN];
+    uint2 qs[RUN];
+    auto fetch = [&](int first, int n) __attribute__((always_inline)) {  // rows first + 2 (wave + 16 i) + half, i < n
+#pragma unroll
+        for (int i = 0; i < RUN; i++) {
+            if (i >= n) break;
+            const uint8_t *src = rows + (size_t)(first + 2 * (wave + WAVES * i) + half) * (2 * 144);
+            hdr[i] = *(const uint4 *)src, qs[i] = *(const uint2 *)(src + 16 + 8 * l);
+        }
+    };
+    fetch(0, RUN);
+    float x[RUN];
+#pragma unroll
+    for (int i = 0; i < RUN; i++) x[i] = qh[2 * (wave + WAVES * i) + half];
+    const float2 turn = cs[(size_t)pos * (ROPE / 2) + (lane >> 1)];
+    const float2 pair = *(const float2 *)(qh + NOPE + (lane & ~1));
+    float4 k[N][2];
+    float kp[N];
+    auto tokens = [&](int t0) __attribute__((always_inline)) {  // t0 + wave + 16 i, those there are
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const size_t at = (size_t)min(t0 + wave + WAVES * i, pos - 1);
+            const float4 *src = (const float4 *)(lat + at * LKV + 8 * lane);
+            k[i][0] = src[0], k[i][1] = src[1];
+            kp[i] = kpe[at * ROPE + lane];
+        }
+    };
+    float4 o[2] = {float4{0.0f, 0.0f, 0.0f, 0.0f}, float4{0.0f, 0.0f, 0.0f, 0.0f}};
+    float key = 0.0f;
+    {
+        float lo[8], hi[8], ml = 0.0f, mh = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) lo[e] = hi[e] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < RUN; i++) {
+            const MlaQ4kPair v = mla_q4k_pair(hdr[i], qs[i], c);
+            const float a = x[i] * v.dl, b = x[i] * v.dh;
+#pragma unroll
+            for (int e = 0; e < 8; e++) lo[e] = fmaf(a, v.lo[e], lo[e]), hi[e] = fmaf(b, v.hi[e], hi[e]);
+            ml = fmaf(x[i], v.ml, ml), mh = fmaf(x[i], v.mh, mh);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) lo[e] = sum_xor32(lo[e] - ml), hi[e] = sum_xor32(hi[e] - mh);
+        if (half == 0) {
+            float *to = &red[wave][col];
+            *(float4 *)to = float4{lo[0], lo[1], lo[2], lo[3]}, *(float4 *)(to + 4) = float4{lo[4], lo[5], lo[6], lo[7]};
+            *(float4 *)(to + 32) = float4{hi[0], hi[1], hi[2], hi[3]}, *(float4 *)(to + 36) = float4{hi[4], hi[5], hi[6], hi[7]};
+        }
+    }
+    if (wave < pos) tokens(0);
+    if (wave == pos % WAVES) {  // the new token (of the waves, one of those with the fewest cached tokens)
+        float ss = 0.0f;  // (in the order of mla_rope_latent)
+#pragma unroll
+        for (int i = 0; i < LKV; i += 64) ss = fmaf(comp[i + lane], comp[i + lane], ss);
+        const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)LKV + eps);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const float4 v = *(const float4 *)(comp + 8 * lane + 4 * i), g = *(const float4 *)(w + 8 * lane + 4 * i);
+            o[i] = float4{v.x * inv * g.x, v.y * inv * g.y, v.z * inv * g.z, v.w * inv * g.w};
+        }
+        const float2 key2 = *(const float2 *)(comp + LKV + (lane & ~1));
+        key = lane & 1 ? key2.x * turn.y + key2.y * turn.x : key2.x * turn.x - key2.y * turn.y;
+        if (h == 0 && blockIdx.y == 0) {
+            float4 *to = (float4 *)(lat + (size_t)pos * LKV + 8 * lane);
+            to[0] = o[0], to[1] = o[1];
+            kpe[(size_t)pos * ROPE + lane] = key;
+        }
+    }
+    __syncthreads();
+    if (tid < LKV) {
+        float v = 0.0f;
+#pragma unroll
+        for (int i = 0; i < WAVES; i++) v += red[i][tid];
+        mid[tid] = v;
+    }
+    __syncthreads();
+    const float4 qa = *(const float4 *)&mid[8 * lane], qb = *(const float4 *)&mid[8 * lane + 4];
+    const float qp = lane & 1 ? pair.x * turn.y + pair.y * turn.x : pair.x * turn.x - pair.y * turn.y;
+    auto score = [&](const float4 &a, const float4 &b, float key) __attribute__((always_inline)) {
+        float v = qp * key;
+        v = fmaf(qa.x, a.x, fmaf(qa.y, a.y, fmaf(qa.z, a.z, fmaf(qa.w, a.w, v))));
+        v = fmaf(qb.x, b.x, fmaf(qb.y, b.y, fmaf(qb.z, b.z, fmaf(qb.w, b.w, v))));
+        return wave_sum(v) * scale;
+    };
+    float m = -INFINITY, sum = 0.0f;
+    if (wave == pos % WAVES) m = score(o[0], o[1], key), sum = 1.0f;
+    for (int t0 = 0; t0 + wave < pos; t0 += WAVES * N) {
+        if (t0 > 0) tokens(t0);
+        float s[N], top = m;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            s[i] = score(k[i][0], k[i][1], kp[i]);
+            if (t0 + wave + WAVES * i < pos) top = fmaxf(top, s[i]);
+        }
+        const float keep = m == -INFINITY ? 0.0f : __expf(m - top);
+        m = top, sum *= keep;
+#pragma unroll
+        for (int j = 0; j < 2; j++) o[j].x *= keep, o[j].y *= keep, o[j].z *= keep, o[j].w *= keep;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const float p = t0 + wave + WAVES * i < pos ? __expf(s[i] - m) : 0.0f;
+            sum += p;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                o[j].x = fmaf(p, k[i][j].x, o[j].x), o[j].y = fmaf(p, k[i][j].y, o[j].y);
+                o[j].z = fmaf(p, k[i][j].z, o[j].z), o[j].w = fmaf(p, k[i][j].w, o[j].w);
+            }
+        }
+    }
+    const int first = NOPE + 64 * (int)blockIdx.y;
+    fetch(first, 2);
+    *(float4 *)&red[wave][8 * lane] = o[0], *(float4 *)&red[wave][8 * lane + 4] = o[1];
+    if (lane == 0) max_sh[wave] = m, sum_sh[wave] = sum;
+    __syncthreads();
+    if (tid < LKV) {
+        const float mi = max_sh[lane & 15], M = wave_max(mi);
+        const float fi = mi == -INFINITY ? 0.0f : __expf(mi - M);  // a wave without tokens
+        const float L = wave_sum(lane < WAVES ? sum_sh[lane & 15] * fi : 0.0f);
+        float v = 0.0f;
+#pragma unroll
+        for (int i = 0; i < WAVES; i++) v = fmaf(red[i][tid], __shfl(fi, i, 64), v);
+        mid[tid] = v * (1.0f / L);
+    }
+    __syncthreads();
+    float xl[8], xh[8], sl = 0.0f, sh = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) xl[e] = mid[col + e], xh[e] = mid[col + 32 + e], sl += xl[e], sh += xh[e];
+    float mine = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const MlaQ4kPair v = mla_q4k_pair(hdr[i], qs[i], c);
+        float a = v.lo[0] * xl[0], b = v.hi[0] * xh[0];
+#pragma unroll
+        for (int e = 1; e < 8; e++) a = fmaf(v.lo[e], xl[e], a), b = fmaf(v.hi[e], xh[e], b);
+        const float y = mla_sum_half(fmaf(v.dl, a, fmaf(v.dh, b, -fmaf(v.ml, sl, v.mh * sh))));
+        if (l == i) mine = y;
+    }
+    if (l < 2 && sb == 0) ctx[(size_t)h * vh + (first - NOPE) + 2 * (wave + WAVES * l) + half] = mine;
 }
 
 }  // namespace jq

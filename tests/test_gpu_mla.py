@@ -348,6 +348,29 @@ def test_one_token_over_q4k_blocks_of_the_up_projection(n_head, vh, prompt):
         assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max(), p
 
 
+@pytest.mark.parametrize("n_head,vh,prompt", [(4, 64, 0), (2, 128, 14), (4, 192, 126), (128, 128, 253), (4, 64, 893)])
+def test_a_step_in_one_launch_over_q4k_blocks(n_head, vh, prompt):
+    """Steps of one launch between the query and the output projection: an empty cache, around a wave's turn (16 tokens), a run of
+    all waves' (128), two of them, and the line to the launches of long contexts (896); few heads, as many workgroups as compute units.
+    The cache that the steps leave is read by a call of two tokens, which has other kernels.  1e-5 of the largest as above."""
+    c = cfg(n_embd=256, n_head=n_head, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=vh, context_length=prompt + 8)
+    ref, dev = build(c, qtype=capi.Q4_K, seed=470 + n_head)
+    raw = {n: (r, k) for n, r, k in (("q", n_head * 192, 256), ("kv_a_mqa", 576, 256), ("o", 256, n_head * vh))}
+    w = {n: capi.Weight.upload(capi.Q4_K, ref.t[n][1], r, k) for n, (r, k) in raw.items()}
+    mc = capi.MlaConfig(n_embd=256, n_head=n_head, q_lora_rank=0, kv_lora_rank=512, qk_nope_head_dim=128, qk_rope_head_dim=64,
+                        v_head_dim=vh, n_ctx=prompt + 8, rms_eps=1e-6, rope_theta=1e4)
+    values = oracle.dequantize(capi.Q4_K, ref.t["kv_b"][1]).reshape(n_head * (128 + vh), 512).astype(np.float32)
+    dense = capi.Mla(mc, w["q"], w["kv_a_mqa"], ref.t["kv_a_norm"], values, w["o"])
+    x = normal(19, (prompt + 8, 256)) * np.float32(2.0)
+    if prompt:
+        dev.forward(x[:prompt], 0), dense.forward(x[:prompt], 0)
+    for p in range(prompt, prompt + 6):
+        a, b = dev.forward(x[p:p + 1], p), dense.forward(x[p:p + 1], p)
+        assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max(), p
+    a, b = dev.forward(x[prompt + 6:], prompt + 6), dense.forward(x[prompt + 6:], prompt + 6)
+    assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
+
+
 def test_dense_kv_b_and_other_formats():
     c = cfg(kv_lora_rank=256, n_embd=256, v_head_dim=64)
     for qtype in (capi.Q4_K, capi.Q6_K):
