@@ -168,7 +168,10 @@ __global__ __launch_bounds__(256) void dense_gemv_gated(const uint8_t *__restric
 // The one-row products with the residual update and norm of `nm` in front: y = W h, or with GATED
 // y = gated(Wg h, Wu h).  A workgroup makes the normed row h for itself (workgroup 0 stores it; few, large
 // workgroups, since each reads the norm's vectors whole); then every wave takes pairs of weight rows (gated: the gate and the
-// up row of a column) on its own, the first chunks of its first pair on their way since before the norm.
+// up row of a column) on its own, the first chunks of its first pair on their way while the norm is made: asked for
+// behind the norm's own vectors, which otherwise waited for 32 MB of weights.
+// Bound: memory.  bf16 rows of 4096, us, weights first / vectors first: 6144 rows 14.4 / 13.0, 16384 30.0 / 26.8 (5.0 TB/s), gate and up of
+// 12288 each 42.6 / 39.5 (5.1), 32000 52.6 / 46.8 (5.6).  A row's eight chunks in registers, each refilled once it is multiplied: 17.9, 27.2, 39.0, 47.3.
 template <class E, int WAVES, int NV, bool GATED>
 __global__ __launch_bounds__(64 * WAVES) void norm_gemv(const uint8_t *__restrict__ W, const uint8_t *__restrict__ Wu, size_t pitch,
                                                                   float *__restrict__ Y, int k, int n, GatedUnit act, ResidualNorm nm) {
@@ -199,10 +202,9 @@ __global__ __launch_bounds__(64 * WAVES) void norm_gemv(const uint8_t *__restric
         }
     };
     int grp = (int)blockIdx.x + (int)gridDim.x * wave;
-    ask(min(grp, groups - 1));
     {
         float h[NV];
-        residual_norm_row<NV, 64 * WAVES>(nm, h, blockIdx.x == 0);
+        residual_norm_row<NV, 64 * WAVES>(nm, h, blockIdx.x == 0, [&]() __attribute__((always_inline)) { ask(min(grp, groups - 1)); });
         store_row<NV, 64 * WAVES>(hrow, k, h);
     }
     __syncthreads();

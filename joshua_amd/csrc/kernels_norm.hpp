@@ -35,10 +35,10 @@ __device__ __forceinline__ float sum_block(float v, float *red) {
 template <int BT>
 __device__ __forceinline__ int norm_col(int i) { return 4 * (int)threadIdx.x + 4 * BT * (i / 4) + i % 4; }
 
-// The thread's share of a row; columns past the width are zero.  Every load is issued whatever the width (past it, from
-// the row's end), so that the loads of a row's vectors travel together.
+// The thread's share of a row as it is read: every load is issued whatever the width (past it, from the row's end), so that the
+// loads of a row's vectors travel together.
 template <int NV, int BT>
-__device__ __forceinline__ void load_row(const float *__restrict__ p, int width, float (&v)[NV]) {
+__device__ __forceinline__ void ask_row(const float *__restrict__ p, int width, float (&v)[NV]) {
     if ((width & 3) == 0) {
 #pragma unroll
         for (int i = 0; i < NV; i += 4) {
@@ -49,6 +49,10 @@ __device__ __forceinline__ void load_row(const float *__restrict__ p, int width,
 #pragma unroll
         for (int i = 0; i < NV; i++) v[i] = p[min(norm_col<BT>(i), width - 1)];
     }
+}
+// Zeros past the width.
+template <int NV, int BT>
+__device__ __forceinline__ void end_row(int width, float (&v)[NV]) {
 #pragma unroll
     for (int i = 0; i < NV; i++) v[i] = norm_col<BT>(i) < width ? v[i] : 0.0f;
 }
@@ -88,33 +92,45 @@ __device__ __forceinline__ void row_stats(const float (&v)[NV], int width, float
 
 // The update of one row by a workgroup; x ends as this thread's share of the normed row.  With `store` the stream goes to
 // x_out and the normed row to h_out.  The norms' vectors are asked for together with the row: a single row's time is its
-// round trips to memory.
-template <int NV, int BT>
-__device__ __forceinline__ void residual_norm_row(const ResidualNorm &a, float (&x)[NV], bool store) {
+// round trips to memory.  `behind` asks for what the caller wants in flight meanwhile, behind the row: a compute unit's requests are
+// served in order.
+template <int NV, int BT, class Behind>
+__device__ __forceinline__ void residual_norm_row(const ResidualNorm &a, float (&x)[NV], bool store, Behind behind) {
     __shared__ float red[4 * (BT / 64)];  // a part for each of the sums
     const int w = a.width;
     float g[NV], b[NV], mean, inv;
-    load_row<NV, BT>(a.x, w, x);
+    ask_row<NV, BT>(a.x, w, x);
     if (a.y) {
         float y[NV], pg[NV], pb[NV];
-        load_row<NV, BT>(a.y, w, y);
-        if (a.post_w) load_row<NV, BT>(a.post_w, w, pg);
-        if (a.post_w && a.post_b) load_row<NV, BT>(a.post_b, w, pb);
-        load_row<NV, BT>(a.pre_w, w, g);
-        if (a.pre_b) load_row<NV, BT>(a.pre_b, w, b);
+        ask_row<NV, BT>(a.y, w, y);
+        if (a.post_w) ask_row<NV, BT>(a.post_w, w, pg);
+        if (a.post_w && a.post_b) ask_row<NV, BT>(a.post_b, w, pb);
+        ask_row<NV, BT>(a.pre_w, w, g);
+        if (a.pre_b) ask_row<NV, BT>(a.pre_b, w, b);
+        __builtin_amdgcn_sched_barrier(0);
+        behind();
+        __builtin_amdgcn_sched_barrier(0);
+        end_row<NV, BT>(w, y);
         if (a.post_w) {
             row_stats<NV, BT>(y, w, a.eps, a.rms, red, &mean, &inv);
 #pragma unroll
             for (int i = 0; i < NV; i++) y[i] = norm_col<BT>(i) < w ? fmaf((y[i] - mean) * inv, pg[i], a.post_b ? pb[i] : 0.0f) : 0.0f;
         }
+        end_row<NV, BT>(w, x);
 #pragma unroll
         for (int i = 0; i < NV; i++) x[i] = fmaf(a.mult, y[i], x[i]);
     } else {
-        load_row<NV, BT>(a.pre_w, w, g);
-        if (a.pre_b) load_row<NV, BT>(a.pre_b, w, b);
+        ask_row<NV, BT>(a.pre_w, w, g);
+        if (a.pre_b) ask_row<NV, BT>(a.pre_b, w, b);
+        __builtin_amdgcn_sched_barrier(0);
+        behind();
+        __builtin_amdgcn_sched_barrier(0);
+        end_row<NV, BT>(w, x);
     }
     if (store && a.x_out) store_row<NV, BT>(a.x_out, w, x);
     row_stats<NV, BT>(x, w, a.eps, a.rms, red + 2 * (BT / 64), &mean, &inv);
+    end_row<NV, BT>(w, g);
+    if (a.pre_b) end_row<NV, BT>(w, b);
 #pragma unroll
     for (int i = 0; i < NV; i++) x[i] = fmaf((x[i] - mean) * inv, g[i], a.pre_b ? b[i] : 0.0f);
     if (store && a.h_out) store_row<NV, BT>(a.h_out, w, x);
