@@ -3066,16 +3066,40 @@ bool model_norm_mm(const jq_weight *w, const float *x, const float *res, const f
 // 4000 tokens 9 tokens 1973 / 1237.  Where heads are grouped as no f32 kernel takes them (`tiled` false) the line is 32 tokens.
 bool split16_attention_pays(uint32_t T, uint32_t pos, bool tiled) { return T >= (tiled ? 64u : 32u) || pos + T >= 128; }
 
-int model_forward_dev(Qwen3Model *m, uint32_t T, uint32_t pos, const uint32_t *want, uint32_t n_want, hipStream_t s) {
+// A short step's rows of the embedding, position and angles in one launch; -1 where the embedding is in no block format.
+int model_step_begin(Qwen3Model *m, const jq_weight *emb, const uint32_t *tokens, uint32_t T, uint32_t pos, hipStream_t s) {
+    jq::StepTokens ids{};
+    std::copy(tokens, tokens + T, ids.id);
+    const size_t k = emb->k;
+    switch (emb->type) {
+#define JQ_CASE(ID, Q)                                                                                                                 \
+    case ID:                                                                                                                           \
+        hipLaunchKernelGGL(jq::step_begin<jq::Q>, dim3((unsigned)((T * (k / jq::Q::BLOCK_ELEMS) * jq::Q::UNITS + 255) / 256 + 1)), dim3(256), 0, s, \
+                           emb->dev, emb->row_bytes, ids, m->x, (int)T, (int)k, m->pos, (int)pos, (int)m->cfg.head_dim, m->cfg.rope_theta, m->rope_cs); \
+        break;
+        JQ_FOR_EACH_FORMAT(JQ_CASE)
+#undef JQ_CASE
+    default: return -1;
+    }
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+int model_forward_dev(Qwen3Model *m, const uint32_t *tokens, uint32_t T, uint32_t pos, const uint32_t *want, uint32_t n_want, hipStream_t s) {
     const jq_qwen3_config &c = m->cfg;
     const int d = (int)c.head_dim, nh = (int)c.n_head, nkv = (int)c.n_kv_head, h = (int)c.hidden;
     auto emb = m->q.find("token_embd.weight");
     if (emb == m->q.end()) return fail("qwen3: missing tensor `token_embd.weight`");
-    if (dispatch_decode(emb->second, m->ids, m->x, T, s)) return 1;
     // few query rows over a long cache: split the keys over the chip
     const bool split = T <= 8 && (d == 64 || d == 128 || d == 256);
-    // the step's position for the kernels, and with split attention the rotary angles of its tokens
-    hipLaunchKernelGGL(jq::rope_table, dim3(1), dim3(256), 0, s, m->pos, (int)pos, split ? (int)T : 0, d, c.rope_theta, m->rope_cs);
+    // the tokens' rows, the step's position for the kernels, and with split attention the rotary angles of its tokens
+    const int begun = split ? model_step_begin(m, emb->second, tokens, T, pos, s) : -1;
+    if (begun > 0) return 1;
+    if (begun < 0) {
+        HIP_TRY(hipMemcpyAsync(m->ids, tokens, T * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+        if (dispatch_decode(emb->second, m->ids, m->x, T, s)) return 1;
+        hipLaunchKernelGGL(jq::rope_table, dim3(1), dim3(256), 0, s, m->pos, (int)pos, split ? (int)T : 0, d, c.rope_theta, m->rope_cs);
+    }
     const float sqrt_d = sqrtf((float)d);
     const int n_chunks = (int)((pos + T + jq::ATT_CHUNK - 1) / jq::ATT_CHUNK);
     const float *pending = nullptr;  // residual not yet added into x
@@ -3295,8 +3319,7 @@ Qwen3Model::~Qwen3Model() {
 int Qwen3Model::step(const uint32_t *tokens, uint32_t n, const uint32_t *want, uint32_t n_want, hipStream_t s) {
     if (model_reserve(this, std::max(n, n_want))) return 1;
     if (model_prepare_fused(this)) return 1;  // first step only: q|k(|v) and gate|up as single matrices
-    HIP_TRY(hipMemcpyAsync(ids, tokens, n * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-    return model_forward_dev(this, n, n_past, want, n_want, s);
+    return model_forward_dev(this, tokens, n, n_past, want, n_want, s);
 }
 
 extern "C" {

@@ -11,14 +11,32 @@ namespace jq {
 
 // cs[t][i] = mag (cos, sin)((pos0 + t) freq[i]), the angle formed and reduced in f64 so that far positions keep an
 // f32's accuracy.
-static __global__ __launch_bounds__(256) void rope_angles(const double *__restrict__ freq, int half, int pos0, int T, float mag,
-                                                          float2 *__restrict__ cs) {
-    const int total = T * half;
-    for (int e = (int)blockIdx.x * 256 + (int)threadIdx.x; e < total; e += (int)gridDim.x * 256) {
-        double s, c;
-        sincos((double)(pos0 + e / half) * freq[e % half], &s, &c);
-        cs[e] = float2{mag * (float)c, mag * (float)s};
+struct RopeAngles {
+    const double *freq;
+    int half, pos0, T;
+    float mag;
+    float2 *cs;
+    __device__ __forceinline__ void make(int workgroup, int workgroups) const {
+        for (int e = workgroup * 256 + (int)threadIdx.x; e < T * half; e += workgroups * 256) {
+            double s, c;
+            sincos((double)(pos0 + e / half) * freq[e % half], &s, &c);
+            cs[e] = float2{mag * (float)c, mag * (float)s};
+        }
     }
+};
+static __global__ __launch_bounds__(256) void rope_angles(RopeAngles a) { a.make((int)blockIdx.x, (int)gridDim.x); }
+
+// The beginning of a step of up to STEP_TOKENS tokens in one launch: their rows of the embedding, and the angles of one rotary table (cs null:
+// none) in a workgroup a token behind them.  grid (T, ceil(k / 1024) + 1).  The tokens are an argument, so that nothing is copied to the device first.
+template <class E>
+__global__ __launch_bounds__(256) void dense_step_begin(const uint8_t *__restrict__ W, size_t pitch, StepTokens tokens, float *__restrict__ out, int k,
+                                                        float scale, RopeAngles a) {
+    if (blockIdx.y + 1 == gridDim.y) {
+        if (a.cs) a.make((int)blockIdx.x, (int)gridDim.x);
+        return;
+    }
+    const typename E::T *row = (const typename E::T *)(W + tokens.id[blockIdx.x] * pitch);
+    for (int c = (int)blockIdx.y * 256 + (int)threadIdx.x; c < k; c += ((int)gridDim.y - 1) * 256) out[(size_t)blockIdx.x * k + c] = (float)row[c] * scale;
 }
 
 // What the kernels of one attention layer share.

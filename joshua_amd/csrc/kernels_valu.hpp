@@ -239,6 +239,20 @@ struct ToFloat<Q2_K> {
     }
 };
 
+// Unit u of a row (UNITS to a block) as floats at their places in out_row.
+template <class Q>
+__device__ __forceinline__ void decode_unit(const uint8_t *__restrict__ row, int u, float *__restrict__ out_row) {
+    constexpr int UE = Q::SEGS * Q::SEGLEN;
+    const int b = u / Q::UNITS, ub = u % Q::UNITS;
+    float w[UE];
+    ToFloat<Q>::decode(row + (size_t)b * Q::BLOCK_BYTES, ub, w);
+    float *o = out_row + (size_t)b * Q::BLOCK_ELEMS + Q::elem_base(ub);
+#pragma unroll
+    for (int s = 0; s < Q::SEGS; s++)
+#pragma unroll
+        for (int e = 0; e < Q::SEGLEN; e++) o[s * Q::SEG_STRIDE + e] = w[s * Q::SEGLEN + e];
+}
+
 // out[r*k + ...] = decode(row ids[r]) (ids == nullptr: row r itself).
 template <class Q>
 __global__ __launch_bounds__(256) void decode_rows(const uint8_t *__restrict__ W, size_t row_bytes,
@@ -246,21 +260,17 @@ __global__ __launch_bounds__(256) void decode_rows(const uint8_t *__restrict__ W
                                                     size_t n_out_rows, int k) {
     const int units_per_row = (k / Q::BLOCK_ELEMS) * Q::UNITS;
     const size_t total = n_out_rows * (size_t)units_per_row;
-    constexpr int UE = Q::SEGS * Q::SEGLEN;
     for (size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x; g < total; g += (size_t)gridDim.x * blockDim.x) {
-        const size_t r = g / units_per_row;
-        const int u = (int)(g % units_per_row);
-        const size_t src_row = ids ? ids[r] : r;
-        const int b = u / Q::UNITS, ub = u % Q::UNITS;
-        float w[UE];
-        ToFloat<Q>::decode(W + src_row * row_bytes + (size_t)b * Q::BLOCK_BYTES, ub, w);
-        float *o = out + r * (size_t)k + (size_t)b * Q::BLOCK_ELEMS + Q::elem_base(ub);
-#pragma unroll
-        for (int s = 0; s < Q::SEGS; s++)
-#pragma unroll
-            for (int e = 0; e < Q::SEGLEN; e++) o[s * Q::SEG_STRIDE + e] = w[s * Q::SEGLEN + e];
+        const size_t r = g / units_per_row, src_row = ids ? ids[r] : r;
+        decode_unit<Q>(W + src_row * row_bytes, (int)(g % units_per_row), out + r * (size_t)k);
     }
 }
+
+// The tokens of a short step, as a kernel's argument.
+constexpr int STEP_TOKENS = 8;
+struct StepTokens {
+    uint32_t id[STEP_TOKENS];
+};
 
 // Raw tensor bytes that are no weight format of the matmuls, to f32 (reference: src/quant_matmul.rs:36-103
 // decode_raw_to_f32): KIND 1 = F16 elements, 9 = Q8_1 blocks (f16 d, f16 s, 32 int8: d * q, the published ggml

@@ -156,7 +156,7 @@ struct LayeredModel : jq_model {
     int step(const uint32_t *tokens, uint32_t n, const uint32_t *want, uint32_t n_want, hipStream_t s) override;
     void forget() override { broken = false; }
     int reserve(size_t T, size_t W, size_t keys);
-    int run_layers(int T, const uint32_t *want, int n_want, hipStream_t s);
+    int run_layers(const uint32_t *tokens, int T, const uint32_t *want, int n_want, hipStream_t s);
     size_t esz() const { return dense_elem_bytes(type); }
 
     template <class T>
@@ -274,10 +274,10 @@ int LayeredModel::step(const uint32_t *tokens, uint32_t n, const uint32_t *want,
     bool latent = false;
     for (const Layer &l : layers) latent |= l.c.mixer == LayerConfig::LATENT;
     if (reserve(n, std::max<uint32_t>(n_want, 1), latent && n > (uint32_t)GEMV_MAX_ROWS ? n_past + n : 0)) return 1;
-    HIP_TRY(hipMemcpyAsync(ids, tokens, n * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+    if (n > (uint32_t)jq::STEP_TOKENS) HIP_TRY(hipMemcpyAsync(ids, tokens, n * sizeof(uint32_t), hipMemcpyHostToDevice, s));
     if (n_want && n > 1) HIP_TRY(hipMemcpyAsync(want_ids, want, n_want * sizeof(uint32_t), hipMemcpyHostToDevice, s));
     broken = true;
-    if (run_layers((int)n, want, (int)n_want, s)) return 1;
+    if (run_layers(tokens, (int)n, want, (int)n_want, s)) return 1;
     HIP_TRY(hipGetLastError());
     broken = false;
     return 0;
@@ -528,15 +528,25 @@ int run_mamba(LayeredModel *m, const Layer &l, LayerRun &r, int T, bool small, h
     return 0;
 }
 
-int LayeredModel::run_layers(int T, const uint32_t *want, int n_want, hipStream_t s) {
+int LayeredModel::run_layers(const uint32_t *tokens, int T, const uint32_t *want, int n_want, hipStream_t s) {
     const int w = (int)cfg.width;
     const size_t sw = dense_stride(w);
     const bool small = T <= GEMV_MAX_ROWS;             // f32 activations through the GEMV
     const bool one = T == 1 && w <= FUSED_NORM_MAX_WIDTH;  // and the residual update and norm inside the product's launch
     const int pos0 = (int)n_past;
-    if (dense_decode(embed, ids, x, T, cfg.embedding_scale, s)) return 1;
-    for (const RotaryTable &r : rots)
-        hipLaunchKernelGGL(jq::rope_angles, dim3(grid_for((size_t)T * (r.c.dims / 2))), dim3(256), 0, s, r.freq, r.c.dims / 2, pos0, T, r.mag, r.cs);
+    auto angles = [&](const RotaryTable &r) { return jq::RopeAngles{r.freq, r.c.dims / 2, pos0, T, r.mag, r.cs}; };
+    size_t tables = 0;  // made so far
+    if (T <= jq::STEP_TOKENS) {
+        jq::StepTokens by_value{};
+        std::copy(tokens, tokens + T, by_value.id);
+        const jq::RopeAngles first = rots.empty() ? jq::RopeAngles{} : angles(rots[tables++]);
+        JQ_ELEM_OF(embed->type, hipLaunchKernelGGL((jq::dense_step_begin<E>), dim3((unsigned)T, (unsigned)(w + 1023) / 1024 + 1), dim3(256), 0, s, embed->dev,
+                                                   embed->row_bytes, by_value, x, w, cfg.embedding_scale, first));
+    } else if (dense_decode(embed, ids, x, T, cfg.embedding_scale, s)) {
+        return 1;
+    }
+    for (; tables < rots.size(); tables++)
+        hipLaunchKernelGGL(jq::rope_angles, dim3(grid_for((size_t)T * (rots[tables].c.dims / 2))), dim3(256), 0, s, angles(rots[tables]));
     if (pos0 == 0) {  // a new sequence: its states start at zero
         for (LayerRun &r : runs)
             if (zero_floats(r.S, r.S_floats, s) || zero_floats(r.tail[r.tail_at], r.tail_floats, s)) return 1;

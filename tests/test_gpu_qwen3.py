@@ -146,6 +146,20 @@ def test_paired_gate_up_rows_serve_prefill_and_replacement():
     assert ok, e
 
 
+@pytest.mark.parametrize("qtype", [capi.Q8_0, capi.Q6_K, capi.Q4_1, capi.MXFP4])
+def test_short_steps_over_embeddings_of_any_format(qtype):
+    """Steps of up to eight tokens gather their rows in the launch that makes the angles, nine in launches of their own; first and last
+    rows of the table, a token twice."""
+    count = CFG["vocab"] * CFG["hidden"]
+    blocks = synth.random_blocks(qtype, 61, count) if qtype in capi.GENERIC_TYPES else synth.normal_quantized(qtype, 61, count, 1.0)
+    m, o = make(CFG, 62, override={"token_embd.weight": (qtype, blocks)})
+    pos = 0
+    for tokens in ([0], [767, 5], [3, 3, 700, 41, 256, 9, 88], [767, 0, 41, 41, 256, 9, 88, 511], [2, 640, 77, 5, 9, 1, 766, 4, 4], [123]):
+        ok, e = close(m.forward(tokens, pos), o.forward(tokens, pos))
+        assert ok, f"{len(tokens)} tokens at {pos}: {e}"
+        pos += len(tokens)
+
+
 def test_prefill_in_two_chunks_matches_one():
     m, o = make(CFG, 22)
     toks = list(range(10, 30))
