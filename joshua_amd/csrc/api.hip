@@ -191,17 +191,25 @@ int dispatch_q4k_dot4(const uint8_t *W, size_t row_bytes, const float *X, float 
     if (mode == "auto" && !swiglu && !(tile_env && tile_env[0] == '0') && (nb == 8 || nb == 6) && k == 256 * nb && row_bytes == nb * 144 &&
         n >= 64 && n <= 0x7FFFFFF0ull) {
         const jq::QdNorm nm = norm ? *norm : jq::QdNorm{};
-        static_assert(jq::gemv_mfma_tile_lds<jq::QvQ4K, 8>() <= 64 * 1024, "within the default dynamic LDS limit");
+        static_assert(jq::gemv_mfma_tile_lds<jq::QvQ4K, 8, true>() <= 64 * 1024 && jq::gemv_mfma_tile_lds<jq::QvQ4KFine, 6, true, 2>() <= 64 * 1024, "within the default dynamic LDS limit");
         note_kernel("q4k_gemv_mfma_tile");
-        auto launch = [&](auto kern, int waves, int lds) {
-            hipLaunchKernelGGL(kern, dim3((unsigned)((n + 15) / 16)), dim3(64 * waves), lds, s, W, X, Y, (int)n, nm.res, nm.w, nm.eps, nm.x_out,
+        const size_t all = (n + 15) / 16;
+        auto launch = [&](auto kern, int waves, int lds, size_t tiles) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)((all + tiles - 1) / tiles)), dim3(64 * waves), lds, s, W, X, Y, (int)n, nm.res, nm.w, nm.eps, nm.x_out,
                                nm.hn_out);
         };
-        constexpr int lds8 = jq::gemv_mfma_tile_lds<jq::QvQ4K, 8>(), lds6 = jq::gemv_mfma_tile_lds<jq::QvQ4KFine, 6>();
-        if (nb == 8 && norm) launch(jq::gemv_mfma_tile<jq::QvQ4K, 8, true>, 8, lds8);
-        else if (nb == 8) launch(jq::gemv_mfma_tile<jq::QvQ4K, 8, false>, 8, lds8);
-        else if (norm) launch(jq::gemv_mfma_tile<jq::QvQ4KFine, 6, true>, 6, lds6);
-        else launch(jq::gemv_mfma_tile<jq::QvQ4KFine, 6, false>, 6, lds6);
+#define JQ_TILE(F, NB, NORM, NT) launch(jq::gemv_mfma_tile<jq::F, NB, NORM, NT>, NB, jq::gemv_mfma_tile_lds<jq::F, NB, NORM, NT>(), NT)
+        // Two tiles a workgroup of six waves where single ones would not run side by side any more (four to six workgroups a compute unit):
+        // 24576 rows behind the norm 9.0 -> 7.5 us, without it 7.5 -> 7.4, 49152 12.2 -> 11.0, but 18432 6.4 -> 6.8.  Eight waves
+        // have the requests of one tile out as fast (24576 rows 8.3 / 8.2, 49152 13.0 / 13.5).
+        const bool two = nb == 6 && all > 1152;
+        if (nb == 8 && norm) JQ_TILE(QvQ4K, 8, true, 1);
+        else if (nb == 8) JQ_TILE(QvQ4K, 8, false, 1);
+        else if (norm && two) JQ_TILE(QvQ4KFine, 6, true, 2);
+        else if (norm) JQ_TILE(QvQ4KFine, 6, true, 1);
+        else if (two) JQ_TILE(QvQ4KFine, 6, false, 2);
+        else JQ_TILE(QvQ4KFine, 6, false, 1);
+#undef JQ_TILE
         HIP_TRY(hipGetLastError());
         return 0;
     }
@@ -402,7 +410,7 @@ template <class F>
 int launch_gemv_tile8(const char *name, const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t n, hipStream_t s) {
     if (row_bytes != (size_t)8 * F::BLOCK) return -1;
     auto kern = jq::gemv_mfma_tile<F, 8, false>;
-    constexpr int lds = jq::gemv_mfma_tile_lds<F, 8>();
+    constexpr int lds = jq::gemv_mfma_tile_lds<F, 8, false>();
     static const hipError_t attr_rc = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     HIP_TRY(attr_rc);
     note_kernel(name);
@@ -419,7 +427,7 @@ template <class F>
 int launch_gemv_tile16(const char *name, const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t n, hipStream_t s) {
     if (row_bytes != (size_t)16 * F::BLOCK) return -1;
     auto kern = jq::gemv_mfma_tile<F, 16, false>;
-    constexpr int lds = jq::gemv_mfma_tile_lds<F, 16>();
+    constexpr int lds = jq::gemv_mfma_tile_lds<F, 16, false>();
     static_assert(lds <= 160 * 1024, "one workgroup's LDS");
     static const hipError_t attr_rc = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     HIP_TRY(attr_rc);

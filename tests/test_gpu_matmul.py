@@ -1171,6 +1171,17 @@ def test_q4k_mfma_gemv_over_rows_of_1536(n):
     assert np.all(np.isnan(w.matmul_t(1, lhs)))
 
 
+@pytest.mark.parametrize("n", [16 * 1152, 16 * 1152 + 1, 16 * 1153 + 1, 16 * 1160 - 5])
+def test_q4k_mfma_gemv_over_rows_of_1536_two_tiles_a_workgroup(n):
+    """The last count with one tile a workgroup; odd and even counts of tiles, the last workgroup with one or two of them."""
+    k = 1536
+    blocks = make_blocks(capi.Q4_K, n, k, 540 + n % 89)
+    lhs = synth.normal(541, (1, k))
+    got = capi.Weight.upload(capi.Q4_K, blocks, n, k).matmul_t(1, lhs)
+    assert capi.last_kernel() == "q4k_gemv_mfma_tile"
+    assert close(got, oracle.matmul_t(capi.Q4_K, (1, k, n), lhs, blocks, avx2=oracle.have_avx2()))
+
+
 @pytest.mark.parametrize("qtype,kernel", [(capi.Q6_K, "q6k_gemv_mfma_tile"), (capi.Q8_0, "q8_0_gemv_mfma_tile"),
                                           (capi.Q5_K, "q5k_gemv_mfma_tile")])
 @pytest.mark.parametrize("n", [64, 512 + 7, 16 * 700 + 3])

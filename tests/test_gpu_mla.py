@@ -479,6 +479,17 @@ def test_one_token_whose_query_norm_rides_in_the_product():
             pos += n
 
 
+@pytest.mark.parametrize("n_head", [96, 100])
+def test_a_query_norm_in_front_of_one_and_two_tiles_a_workgroup(n_head):
+    """1152 and 1200 tiles of 16 rows of 1536 columns."""
+    c = cfg(n_embd=256, n_head=n_head, q_lora_rank=1536, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=64)
+    ref, dev = build(c, qtype=capi.Q4_K, seed=970)
+    x, pos = normal(31, (5, 256)), 0
+    for n in (3, 1, 1):
+        assert close(dev.forward(x[pos:pos + n], pos), ref.forward(x[pos:pos + n], pos)), pos
+        pos += n
+
+
 def test_query_and_latent_down_projections_as_one_product():
     """256 tokens over 4096 columns take q_a and kv_a as one product, 96 take two: both between single tokens, which take one."""
     c = cfg(n_embd=4096, n_head=2, q_lora_rank=256, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=128, context_length=640)
