@@ -3250,12 +3250,16 @@ int model_forward_dev(Qwen3Model *m, const uint32_t *tokens, uint32_t T, uint32_
             gp = m->cat, up = m->cat + c.ffn;
         } else if (fgm != m->fused.end()) {
             const jq_weight *w = fgm->second;
-            if (dispatch_matmul(w->type, w->dev, w->row_bytes, m->hn, m->g, T, w->k, w->n, s)) return 1;
+            // the GEMM that takes Q4_K from 128 rows on applies SwiGLU itself, unless it has k in parts
+            const int rc = gemm_h6_swiglu(w->type, w->dev, w->row_bytes, m->hn, m->mid, T, w->k, w->n, s);
+            if (rc > 0) return 1;
+            activated = rc == 0;
+            if (!activated && dispatch_matmul(w->type, w->dev, w->row_bytes, m->hn, m->g, T, w->k, w->n, s)) return 1;
             // many rows into a Q4_K or Q6_K down projection: the int8 GEMM's activation preparation applies
             // SwiGLU to the pairs as it reads them
             auto dn = m->q.find(p + ".ffn_down.weight");
             static const char *no_fused_swiglu = getenv("JQ_NO_SWIGLU_IN_PREP");
-            if (dn != m->q.end() && !no_fused_swiglu && dn->second->k == c.ffn) {
+            if (!activated && dn != m->q.end() && !no_fused_swiglu && dn->second->k == c.ffn) {
                 const jq_weight *wd = dn->second;
                 int rc = -1;
                 if (wd->type == JQ_TYPE_Q4_K)
@@ -3269,7 +3273,7 @@ int model_forward_dev(Qwen3Model *m, const uint32_t *tokens, uint32_t T, uint32_
                 if (rc > 0) return 1;
                 down_done = rc == 0;
             }
-            if (!down_done)
+            if (!activated && !down_done)
                 hipLaunchKernelGGL(jq::swiglu_pairs, dim3(grid_for((size_t)T * c.ffn)), dim3(256), 0, s, m->g, m->mid, (size_t)T * c.ffn);
             activated = true;
         } else if (model_mm(m, p + ".ffn_gate.weight", m->hn, m->g, T, s) ||

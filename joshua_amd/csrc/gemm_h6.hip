@@ -68,7 +68,8 @@ double pick(size_t m, size_t nb, size_t n, Shape &best, size_t &splits, May may)
 // callers of jq_last_kernel know the many-row product by; jq_last_arithmetic says which of the two ran.
 // Returns -1 when the shape is outside its reach and where the environment names a shape or a switch of that GEMM.  JQ_GEMM_H6 = 0
 // switches this one off, JQ_GEMM_H6_SHAPE and _SPLITS force the choice, _MIN_M moves the fewest rows.
-template <class F>
+// SWIGLU (the kernel's): declined where k is in parts, whose sums are no products yet.
+template <class F, bool SWIGLU = false>
 int dispatch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n, hipStream_t s, const char *name, const char *name_split, bool swiglu_pairs = false) {
     static const char *mode = getenv("JQ_GEMM_H6"), *i8_mode = getenv("JQ_Q4K_GEMM_I8"), *i8_shape = getenv("JQ_Q4K_GEMM_I8_SHAPE");
     static const char *shape_env = getenv("JQ_GEMM_H6_SHAPE"), *splits_env = getenv("JQ_GEMM_H6_SPLITS");
@@ -99,7 +100,7 @@ int dispatch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_
         if (splits_env && sp != (size_t)atoi(splits_env)) return false;
         return sp == 1 || (m * n <= 0x3FFFFFFFull && acts_bytes + (sp - 1) * turn * n * sizeof(float) <= scratch_cap);
     });
-    if (us < 0.0 || best.grid(m, n) > 0x7FFFFFFFull) return -1;
+    if (us < 0.0 || best.grid(m, n) > 0x7FFFFFFFull || (SWIGLU && (splits > 1 || n % 2 != 0))) return -1;
     CallScratch scratch;
     uint8_t *acts = nullptr;
     if (scratch.get(acts_bytes + (splits - 1) * turn * n * sizeof(float), s, &acts)) return 1;
@@ -109,7 +110,7 @@ int dispatch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_
         for (size_t m0 = 0; m0 < m; m0 += turn) {
             const size_t rows = std::min(turn, m - m0), row_groups = (rows + 15) / 16, outs = rows * n;
             const float *x = X + m0 * k * (swiglu_pairs ? 2 : 1);
-            float *y = Y + m0 * n;
+            float *y = Y + m0 * (SWIGLU ? n / 2 : n);
             const dim3 prep((unsigned)nb, (unsigned)row_groups);
             if (swiglu_pairs) hipLaunchKernelGGL((jq::kq_gemm_h6_prep<true, F::MINS, F::NIBBLES>), prep, dim3(128), 0, s, x, (int)rows, (int)k, acts);
             else hipLaunchKernelGGL((jq::kq_gemm_h6_prep<false, F::MINS, F::NIBBLES>), prep, dim3(128), 0, s, x, (int)rows, (int)k, acts);
@@ -121,7 +122,7 @@ int dispatch(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_
         }
         return 0;
     };
-#define JQ_GEMM_H6(NW_, NG_) launch(jq::kq_gemm_h6<F, NW_, NG_>, jq::h6_lds_bytes<NG_>(), NW_, big_lds_once<&jq::kq_gemm_h6<F, NW_, NG_>>(jq::h6_lds_bytes<NG_>()))
+#define JQ_GEMM_H6(NW_, NG_) launch(jq::kq_gemm_h6<F, NW_, NG_, SWIGLU>, jq::h6_lds_bytes<NG_>(), NW_, big_lds_once<&jq::kq_gemm_h6<F, NW_, NG_, SWIGLU>>(jq::h6_lds_bytes<NG_>()))
     const int rc = best.nw == 4 ? JQ_GEMM_H6(4, 4) : best.ng == 8 ? JQ_GEMM_H6(8, 8) : best.ng == 7 ? JQ_GEMM_H6(8, 7) : JQ_GEMM_H6(8, 6);
 #undef JQ_GEMM_H6
     if (rc) return rc;
@@ -145,6 +146,10 @@ int gemm_h6(uint32_t type, const uint8_t *W, size_t row_bytes, const float *X, f
     case JQ_TYPE_MXFP4: return dispatch<jq::H6MXFP4>(W, row_bytes, X, Y, m, k, n, s, name, name_split, swiglu_pairs);
     default: return -1;
     }
+}
+
+int gemm_h6_swiglu(uint32_t type, const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t m, size_t k, size_t n, hipStream_t s) {
+    return type == JQ_TYPE_Q4_K ? dispatch<jq::H6Q4K, true>(W, row_bytes, X, Y, m, k, n, s, "q4k_gemm_i8", nullptr) : -1;
 }
 
 }  // namespace jqh

@@ -336,8 +336,11 @@ __device__ __forceinline__ h6_i8 h6_operand6(h6_u6 v) {
     return h6_i8{(int)v[0], (int)v[1], (int)v[2], (int)v[3], (int)v[4], (int)v[5], 0, 0};
 }
 
+// SWIGLU: the weight rows are gate_j and up_j in turn, and Y gets n / 2 values silu(gate_j) up_j a row: two lanes beside each other hold
+// a pair's two products of four rows, and each finishes two of them.  (The 201 MB of 2048 x 24576 products were stored and read again by
+// the next product's preparation; times at gemm_h6_swiglu's declaration.)
 // (Four waves: two workgroups a compute unit.  Not told so, the compiler keeps the sums in accumulation registers and copies them out.)
-template <class F, int NW, int NG>
+template <class F, int NW, int NG, bool SWIGLU = false>
 static __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void kq_gemm_h6(const uint8_t *__restrict__ W, size_t row_bytes,
                                                       const uint8_t *__restrict__ acts, float *__restrict__ Y, int m_rows, int n,
                                                       int nb, int groups, int tx, int ty, int nb_total, float *__restrict__ parts) {
@@ -509,6 +512,23 @@ static __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void kq_gemm_h6(co
             }
             __syncthreads();
         });
+    }
+    if constexpr (SWIGLU) {
+        const bool odd = r & 1;
+#pragma unroll
+        for (int mg = 0; mg < 2; mg++)
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {
+                const int row = m0 + 16 * (2 * wave + mg) + 4 * g + i + (odd ? 1 : 0);
+#pragma unroll
+                for (int cg = 0; cg < NG; cg++) {
+                    const float other = dpp_f<0xB1>(odd ? acc[mg][cg][i] : acc[mg][cg][i + 1]);  // quad_perm: of the lane beside this one
+                    const float gate = odd ? other : acc[mg][cg][i], up = odd ? acc[mg][cg][i + 1] : other;
+                    const int col = n0 + 16 * cg + r;
+                    if (row < m_rows && col < n) Y[(size_t)row * (n / 2) + col / 2] = silu(gate) * up;
+                }
+            }
+        return;
     }
 #pragma unroll
     for (int mg = 0; mg < 2; mg++)

@@ -588,3 +588,16 @@ def test_single_token_steps_with_1536_wide_rows(mix):
         ok, e = close(m.forward(toks[pos:pos + n], pos), o.forward(toks[pos:pos + n], pos))
         assert ok, f"pos {pos}: {e}"
         pos += n
+
+
+@pytest.mark.parametrize("ffn,tokens", [(2048, 128), (2304, 131), (2304, 257), (3840, 160)])
+def test_gate_and_up_of_many_tokens_with_the_activation_in_the_product(ffn, tokens):
+    """hidden = 1024 leaves the paired product one part of k, so that SwiGLU is its epilogue: whole tiles, ragged ones of either side,
+    a row of the result in odd and even lanes; a down projection of Q4_K and of Q6_K."""
+    cfg = dict(CFG, n_layer=4, hidden=1024, n_head=8, n_kv_head=2, head_dim=128, ffn=ffn, vocab=512, n_ctx=300)
+    m, o = make(cfg, 41, "q4_k_m")
+    toks = np.random.default_rng(23).integers(0, 512, tokens + 1).tolist()
+    ok, e = close(m.forward(toks[:tokens], 0), o.forward(toks[:tokens], 0))
+    assert ok, e
+    ok, e = close(m.forward(toks[tokens:], tokens), o.forward(toks[tokens:], tokens))
+    assert ok, e
