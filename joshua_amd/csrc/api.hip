@@ -469,12 +469,15 @@ int dispatch_gemv_tile8(uint32_t type, const uint8_t *W, size_t row_bytes, const
 
 // Q6_K, one activation row, rows of 4096, 8192 or 12288: the v_dot4 LDS-ring kernel.
 // Returns -1 when the shape is outside its reach.
-int dispatch_q6k_dot4(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t k, size_t n, hipStream_t s) {
+// `norm`: residual add + RMSNorm in front of the product (rows of 4096; nothing else of it is stored).
+int dispatch_q6k_dot4(const uint8_t *W, size_t row_bytes, const float *X, float *Y, size_t k, size_t n, hipStream_t s,
+                      const jq::QdNorm *norm = nullptr) {
     static const char *mode = getenv("JQ_Q6K_DOT4");
     const size_t ng = k / 4096;
     if ((mode && mode[0] == '0') || k % 4096 != 0 || ng < 1 || ng > 3 || row_bytes != ng * jq::Q6D_SLICE ||
         ((uintptr_t)W & 15) != 0 || ((uintptr_t)X & 15) != 0)
         return -1;
+    if (norm && (ng != 1 || (((uintptr_t)norm->res | (uintptr_t)norm->w) & 15) != 0 || norm->x_out || norm->hn_out)) return -1;
     // The int8 matrix-core GEMV over the Q6_K policy, for rows of 8192 and 12288 columns and up to 8192 weight
     // rows (4096 x 12288, a feed-forward down projection: 11.4 us against 12.0 on v_dot4).  A tile of 16 rows is
     // 54 KB, so its ring has two slots and one tile in flight while a tile is multiplied: with more tiles a
@@ -483,7 +486,7 @@ int dispatch_q6k_dot4(const uint8_t *W, size_t row_bytes, const float *X, float 
     // every shape it can.
     static const char *mfma_env = getenv("JQ_Q6K_GEMV_MFMA");
     const bool mfma_all = mfma_env && !strcmp(mfma_env, "all"), mfma_off = mfma_env && mfma_env[0] == '0';
-    if (!mfma_off && n >= 256 && n <= 0x7FFFFFF0ull && (mfma_all || (ng >= 2 && n <= 8192))) {
+    if (!mfma_off && n >= 256 && n <= 0x7FFFFFF0ull && !norm && (mfma_all || (ng >= 2 && n <= 8192))) {
         const size_t tiles16 = (n + 15) / 16, rounds_up = (tiles16 + 255) / 256, G = (tiles16 + rounds_up - 1) / rounds_up;
         const jq::QvColsWork wk{(int)n, (int)G, (int)(tiles16 / G), (int)(tiles16 % G), (int)(16 * ng)};
         note_kernel(ng == 1 ? "q6k_gemv_mfma_lds" : "q6k_gemv_mfma_cols");
@@ -502,9 +505,12 @@ int dispatch_q6k_dot4(const uint8_t *W, size_t row_bytes, const float *X, float 
     static const char *genv = getenv("JQ_Q6K_DOT4_GRID");
     const unsigned grid = (unsigned)std::min<size_t>(tiles, genv ? (size_t)std::max(atoi(genv), 1) : (tiles + rounds - 1) / rounds);
     note_kernel("q6k_gemv_dot4_lds");
-    if (ng == 1) hipLaunchKernelGGL(jq::q6k_gemv_dot4_lds<1>, dim3(grid), dim3(1024), 0, s, W, X, Y, (int)n, (int)grid);
-    else if (ng == 2) hipLaunchKernelGGL(jq::q6k_gemv_dot4_lds<2>, dim3(grid), dim3(1024), 0, s, W, X, Y, (int)n, (int)grid);
-    else hipLaunchKernelGGL(jq::q6k_gemv_dot4_lds<3>, dim3(grid), dim3(1024), 0, s, W, X, Y, (int)n, (int)grid);
+#define JQ_Q6D(...) hipLaunchKernelGGL((jq::q6k_gemv_dot4_lds<__VA_ARGS__>), dim3(grid), dim3(1024), 0, s, W, X, Y, (int)n, (int)grid, norm ? norm->res : nullptr, norm ? norm->w : nullptr, norm ? norm->eps : 0.0f)
+    if (norm) JQ_Q6D(1, true);
+    else if (ng == 1) JQ_Q6D(1);
+    else if (ng == 2) JQ_Q6D(2);
+    else JQ_Q6D(3);
+#undef JQ_Q6D
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -3293,7 +3299,18 @@ int model_forward_dev(Qwen3Model *m, const uint32_t *tokens, uint32_t T, uint32_
     if (!n_want) return 0;
     const float *w_on;
     if (model_vec(m, "output_norm.weight", &w_on)) return 1;
-    // logits only for the wanted positions (the last one of a plugin step; reference: src/quantized_qwen3_moe.rs:816-818)
+    // tie_word_embeddings conversions ship no output head (src/quantized_qwen3_moe.rs:739-743)
+    const char *head = m->q.count("output.weight") ? "output.weight" : "token_embd.weight";
+    // logits only for the wanted positions (the last one of a plugin step; reference: src/quantized_qwen3_moe.rs:816-818).  One position:
+    // the norm rides in a head of Q6_K rows of 4096
+    auto hw = m->q.find(head);
+    static const char *no_norm = getenv("JQ_NO_FUSED_NORM");
+    if (n_want == 1 && hw != m->q.end() && hw->second->type == JQ_TYPE_Q6_K && !no_norm) {
+        const size_t at = (size_t)want[0] * h;
+        const jq::QdNorm nm{pending ? pending + at : nullptr, w_on, c.rms_eps, nullptr, nullptr};
+        const int rc = dispatch_q6k_dot4(hw->second->dev, hw->second->row_bytes, xc + at, m->logits, hw->second->k, hw->second->n, s, &nm);
+        if (rc >= 0) return rc;
+    }
     for (uint32_t i = 0; i < n_want; i++) {
         const size_t at = (size_t)want[i] * h;
         // (a position wanted twice: its residual is added once)
@@ -3302,8 +3319,6 @@ int model_forward_dev(Qwen3Model *m, const uint32_t *tokens, uint32_t T, uint32_
         hipLaunchKernelGGL(jq::rmsnorm_rows, dim3(1), dim3(1024), 0, s, xc + at, pending && !again ? pending + at : nullptr, w_on,
                            c.rms_eps, m->hn + (size_t)i * h, h, h);
     }
-    // tie_word_embeddings conversions ship no output head (src/quantized_qwen3_moe.rs:739-743)
-    const char *head = m->q.count("output.weight") ? "output.weight" : "token_embd.weight";
     if (model_mm(m, head, m->hn, m->logits, n_want, s)) return 1;
     HIP_TRY(hipGetLastError());
     return 0;

@@ -601,3 +601,21 @@ def test_gate_and_up_of_many_tokens_with_the_activation_in_the_product(ffn, toke
     assert ok, e
     ok, e = close(m.forward(toks[tokens:], tokens), o.forward(toks[tokens:], tokens))
     assert ok, e
+
+
+@pytest.mark.parametrize("vocab", [4088, 4104])
+def test_the_last_norm_in_front_of_and_inside_the_head(vocab):
+    """Rows of 4096 of Q6_K: 511 tiles of eight rows take the norm as a launch, 513 take it into the product; the last position of several,
+    single tokens, and a norm that is not finite."""
+    cfg = dict(CFG, n_layer=1, hidden=4096, n_head=4, n_kv_head=2, head_dim=128, ffn=512, vocab=vocab, n_ctx=32)
+    m, o = make(cfg, 43, "q4_k_m")
+    assert {n: qt for n, qt, _ in qwen3_tensors(cfg, 43, "q4_k_m")}["output.weight"] == capi.Q6_K
+    toks, pos = np.random.default_rng(29).integers(0, vocab, 16).tolist(), 0
+    for n in (5, 1, 1):
+        ok, e = close(m.forward(toks[pos:pos + n], pos), o.forward(toks[pos:pos + n], pos))
+        assert ok, f"pos {pos}: {e}"
+        pos += n
+    w = np.ones(4096, np.float32)
+    w[77] = np.nan
+    m.set_tensor("output_norm.weight", 0, w)
+    assert np.isnan(m.forward(toks[pos:pos + 1], pos)).all()
