@@ -138,8 +138,7 @@ __device__ __forceinline__ void residual_norm_row(const ResidualNorm &a, float (
 
 // The update of many rows, a workgroup a row: x in place, h in f32 (h_out) and / or in the products' element type (he, rows
 // `stride` apart, zeros behind the width).  `at`: the rows to take, into the first rows of h (x_out is then left alone), or
-// null for rows 0, 1, ..  A thread has columns BT apart, and the norms' vectors are read as they are needed: what counts here
-// is how many rows are under way at once, that is registers.
+// null for rows 0, 1, ..  A thread has columns BT apart.
 template <class E, int NV, int BT>
 __global__ __launch_bounds__(BT) void residual_norm_rows(ResidualNorm a, typename E::T *__restrict__ he, size_t stride,
                                                          const uint32_t *__restrict__ at) {
@@ -149,13 +148,18 @@ __global__ __launch_bounds__(BT) void residual_norm_rows(ResidualNorm a, typenam
     const int w = a.width, c0 = threadIdx.x;
     const size_t row = at ? at[blockIdx.x] : blockIdx.x;
     const float *xr = a.x + row * (a.ldx ? a.ldx : (size_t)w);
-    float x[NV];
+    // Loads past the width repeat the last column, so that none needs a branch, and all of a row's vector are asked for before the first
+    // is waited for, and in front of any store: one by one they were 12 of 17.5 us, of one row of 4096 columns or of 512.
+    auto ask = [&](const float *src, float (&v)[NV]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NV; i++) v[i] = src[min(c0 + BT * i, w - 1)];
+    };
     auto stats = [&](const float (&v)[NV], float *r, float *mean, float *inv) __attribute__((always_inline)) {
         float mu = 0.0f, ss = 0.0f;
         if (!a.rms) {
             float s = 0.0f;
 #pragma unroll
-            for (int i = 0; i < NV; i++) s += v[i];
+            for (int i = 0; i < NV; i++) s += c0 + BT * i < w ? v[i] : 0.0f;
             mu = sum_block<BT>(s, r) / (float)w;
         }
 #pragma unroll
@@ -165,33 +169,45 @@ __global__ __launch_bounds__(BT) void residual_norm_rows(ResidualNorm a, typenam
         }
         *mean = mu, *inv = 1.0f / sqrtf(sum_block<BT>(ss, r + NW) / (float)w + a.eps);
     };
-#pragma unroll
-    for (int i = 0; i < NV; i++) x[i] = c0 + BT * i < w ? xr[c0 + BT * i] : 0.0f;
-    float mean, inv;
+    float x[NV], g[NV], mean, inv;
+    ask(xr, x);
     if (a.y) {
-        const float *yr = a.y + row * w;
         float y[NV];
-#pragma unroll
-        for (int i = 0; i < NV; i++) y[i] = c0 + BT * i < w ? yr[c0 + BT * i] : 0.0f;
+        ask(a.y + row * w, y);
         if (a.post_w) {
+            ask(a.post_w, g);
             stats(y, red, &mean, &inv);
 #pragma unroll
-            for (int i = 0; i < NV; i++) {
-                const int c = c0 + BT * i;
-                if (c < w) y[i] = fmaf((y[i] - mean) * inv, a.post_w[c], a.post_b ? a.post_b[c] : 0.0f);
+            for (int i = 0; i < NV; i++) y[i] = (y[i] - mean) * inv;
+            if (a.post_b) {
+                float b[NV];
+                ask(a.post_b, b);
+#pragma unroll
+                for (int i = 0; i < NV; i++) y[i] = fmaf(y[i], g[i], b[i]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < NV; i++) y[i] = fmaf(y[i], g[i], 0.0f);
             }
         }
 #pragma unroll
         for (int i = 0; i < NV; i++) x[i] = fmaf(a.mult, y[i], x[i]);
     }
+    ask(a.pre_w, g);
     stats(x, red + 2 * NW, &mean, &inv);
+    float b[NV];
+    if (a.pre_b) {
+        ask(a.pre_b, b);
+    } else {
+#pragma unroll
+        for (int i = 0; i < NV; i++) b[i] = 0.0f;
+    }
     float *xo = at ? nullptr : a.x_out, *ho = a.h_out ? a.h_out + (size_t)blockIdx.x * w : nullptr;
     T *eo = he ? he + (size_t)blockIdx.x * stride : nullptr;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         const int c = c0 + BT * i;
         if (c < w) {
-            const float v = fmaf((x[i] - mean) * inv, a.pre_w[c], a.pre_b ? a.pre_b[c] : 0.0f);
+            const float v = fmaf((x[i] - mean) * inv, g[i], b[i]);
             if (xo) xo[row * w + c] = x[i];
             if (ho) ho[c] = v;
             if (eo) eo[c] = (T)v;
