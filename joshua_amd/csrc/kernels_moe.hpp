@@ -343,10 +343,11 @@ static __global__ __launch_bounds__(256) void moe_gate_topk(const float *__restr
     }
 }
 
-// The same gating by ONE wave per token, for layers without expert groups and with at most 256 experts: lane l
-// holds experts l, l + 64, ..., the softmax and each of the k_used arg-max rounds are register-to-register
+// The same gating by ONE wave per token, for layers with at most 256 experts, in groups of 2 to 64, a power of two, or in none: lane l
+// holds experts l, l + 64, ..., the softmax, the groups' best and each of the k_used arg-max rounds are register-to-register
 // reductions (no LDS, no barrier), where moe_gate_topk's 256 threads meet at eight barriers and rank every
-// expert against every other through LDS: 3 us a launch instead of 7.  Equal scores go to the lower expert
+// expert against every other through LDS: 3 us a launch instead of 7 (groups: 7.9 for
+// 12.6, and in the kernel behind it one token of 256 experts of 7168 x 2048 92 -> 85).  Equal scores go to the lower expert
 // index, as there.
 // The gating of token t by one wave.  Lane r < k_used ends with slot r's expert in *slot_e; `write`: the slots go
 // to ids / wts and the pair groups as well (a kernel that runs the gating in every workgroup writes them once).
@@ -388,6 +389,44 @@ __device__ __forceinline__ void moe_gate_topk_wave_body(int t, int T, int lane, 
         for (int i = 0; i < NE; i++)
             sel[i] = lane + 64 * i < p.E ? prob[i] + (bias && !p.logit_bias() ? bias[lane + 64 * i] : 0.0f) : -INFINITY;
     }
+    // What a taken expert's score becomes, and in front of groups that of lanes without one: nothing compares with it.  (Behind groups a
+    // score that is not a number comes last, -inf, and is not to be taken twice.)
+    float taken = -INFINITY;
+    if (p.n_group > 1) {
+        const int per = p.E / p.n_group, shift = 31 - __builtin_clz((uint32_t)per);  // 2 to 64, a power of two (moe_wave_gate): a group lies in one slot
+        taken = NAN;
+        float gs[NE], second[NE];  // the two best of the lane's group
+#pragma unroll
+        for (int i = 0; i < NE; i++) gs[i] = sel[i] = sel[i] == sel[i] ? sel[i] : -INFINITY, second[i] = -INFINITY;
+        for (int off = 1; off < per; off <<= 1) {  // (the slots side by side: an exchange is 100 clocks on its way)
+            float c1[NE], c2[NE];
+#pragma unroll
+            for (int i = 0; i < NE; i++) c1[i] = __shfl_xor(gs[i], off, 64), c2[i] = __shfl_xor(second[i], off, 64);
+#pragma unroll
+            for (int i = 0; i < NE; i++) second[i] = fmaxf(fminf(gs[i], c1[i]), fmaxf(second[i], c2[i])), gs[i] = fmaxf(gs[i], c1[i]);
+        }
+        if (p.is_sigmoid()) {
+#pragma unroll
+            for (int i = 0; i < NE; i++) gs[i] += second[i];
+        }
+        int rank[NE];
+#pragma unroll
+        for (int i = 0; i < NE; i++) rank[i] = 0;
+#pragma unroll
+        for (int i = 0; i < NE; i++)
+            for (int from = 0; from < 64 && 64 * i + from < p.E; from += per) {
+                const float other = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, gs[i]), from));
+                const int o = (64 * i + from) >> shift;
+#pragma unroll
+                for (int j = 0; j < NE; j++) rank[j] += other > gs[j] || (other == gs[j] && o < ((lane + 64 * j) >> shift));
+            }
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            // selection + (mask*1e30 - 1e30): unchanged inside the kept groups
+            if (rank[i] >= p.topk_group) sel[i] = sel[i] + (0.0f * 1e30f - 1e30f);
+            if (lane + 64 * i >= p.E) sel[i] = taken;
+        }
+    }
     int my_e = 0;
     float my_p = 0.0f;  // lane r keeps slot r
     for (int r = 0; r < p.k_used; r++) {
@@ -410,7 +449,7 @@ __device__ __forceinline__ void moe_gate_topk_wave_body(int t, int T, int lane, 
         for (int i = 0; i < NE; i++) {
             if (i == slot) {
                 pw = prob[i];
-                if (lane == owner) sel[i] = -INFINITY;
+                if (lane == owner) sel[i] = taken;
             }
         }
         pw = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, pw), owner));

@@ -67,7 +67,8 @@ jq::MoeGateParams moe_gate_params(const jq_moe_config &c) {
 
 bool moe_wave_gate(const jq_moe_config &c) {
     static const char *no_wave = getenv("JQ_MOE_NO_WAVE_GATE");
-    return !no_wave && c.n_group <= 1 && c.n_expert <= 256 && c.n_expert_used <= 64;
+    const uint32_t per = c.n_expert / std::max<uint32_t>(c.n_group, 1);  // (groups: a lane's neighbours hold the rest of its expert's)
+    return !no_wave && (c.n_group <= 1 || (per >= 2 && per <= 64 && (per & (per - 1)) == 0)) && c.n_expert <= 256 && c.n_expert_used <= 64;
 }
 
 // `planes`: also leave x as fixed-point planes there (the one-expert-a-workgroup router kernel does; *planes_made
@@ -122,7 +123,7 @@ int moe_route_dev(jq_moe *m, size_t T, const float *x, hipStream_t s, jq::MoePai
 
 int moe_gate_dev(jq_moe *m, size_t T, const float *logits, const jq::MoeGateParams &gp, jq::MoePairGroups pg, hipStream_t s) {
     const jq_moe_config &c = m->cfg;
-    // no expert groups and at most 256 experts: one wave a token, reductions in registers
+    // at most 256 experts, in groups that a wave holds side by side or in none: one wave a token, reductions in registers
     if (moe_wave_gate(c)) {
         const int ne = (int)(c.n_expert + 63) / 64;
 #define JQ_GATE(NE) hipLaunchKernelGGL(jq::moe_gate_topk_wave<NE>, dim3((unsigned)T), dim3(64), 0, s, logits, m->router_bias, gp, m->ids, m->wts, pg)

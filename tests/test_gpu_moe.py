@@ -51,6 +51,29 @@ def test_route_matches_oracle(kw):
     assert np.allclose(w, ow, rtol=2e-5, atol=1e-7)
 
 
+@pytest.mark.parametrize("gating", ["sigmoid", "softmax"])
+@pytest.mark.parametrize("E,groups,kept,used", [(256, 8, 4, 8), (256, 4, 1, 6), (96, 3, 2, 5), (40, 5, 2, 16), (24, 12, 7, 9), (60, 4, 2, 6)])
+def test_route_of_experts_in_groups(gating, E, groups, kept, used):
+    """Groups that lie in one slot of a wave's lanes (64, 32, 8 and 2 experts, the last slot part-filled), and 15, which do not; equal
+    scores, and scores that are not numbers, go to the lower expert, each taken once."""
+    bias = np.linspace(0.05, -0.05, E).astype(np.float32) if gating == "sigmoid" else None
+    ora, dev = build(capi.Q8_0, 512, 32, E, used, 45 + E, gating=gating, n_group=groups, topk_group=kept, router_bias=bias)
+    x = synth.normal(46, (11, 512))
+    ids, w = dev.route(x)
+    oid, ow = ora.route(x)
+    assert np.array_equal(ids, oid)
+    assert np.allclose(w, ow, rtol=2e-5, atol=1e-7)
+    per = E // groups
+    x[:] = 0.0
+    x[1, 7], x[2, 500] = np.nan, np.inf
+    ids, w = dev.route(x)
+    if used <= kept * per:  # all scores equal, or falling with the expert's number
+        assert np.array_equal(ids[0], np.arange(used)) and np.isfinite(w[0]).all()
+    for row in ids:
+        assert len(set(row.tolist())) == used and row.max() < E
+    assert np.array_equal(ids[1], np.arange(used)) and np.isnan(w[1]).all()
+
+
 @pytest.mark.parametrize("h,E,tokens", [(544, 30, 45), (2080, 9, 33), (1024, 64, 128)])
 def test_router_logits_of_many_tokens_are_those_of_few(h, E, tokens):
     """From 32 tokens on the logits come from a kernel that works on 8 experts x 8 tokens a workgroup (an expert
