@@ -37,6 +37,31 @@ def test_products_of_many_rows(m, n, k, kernel):
     assert np.all(np.abs(got[rows] - x @ w.T) <= 2e-6 * scale + 1e-7)
 
 
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (64, 24571, 2048, "dense_gemm+splitk"),    # 192 tiles of 128 weight rows, the last of them ragged: four runs
+    (9, 32640, 1090, "dense_gemm+splitk"),     # 255 tiles: three runs of 18 stages, the last one part-filled
+    (33, 32769, 1024, "dense_gemm"),           # 257
+    (65, 24571, 1024, "dense_gemm"),           # a second tile of rows
+    (20, 24571, 900, "dense_gemm"),            # 15 stages
+])
+def test_products_of_one_tile_of_rows(m, n, k, kernel):
+    """As above, of up to 64 rows, which wait for the weights."""
+    w, x = sl.to_bf16(normal(3, (n, k), k ** -0.5)), normal(4, (m, k))
+    got = capi.Weight.upload(capi.BF16, w, n, k).matmul_t(m, x)
+    assert capi.last_kernel() == kernel
+    x, w = sl.from_bf16(sl.to_bf16(x)).astype(np.float64), sl.from_bf16(w).astype(np.float64)
+    scale = np.abs(x) @ np.abs(w).T
+    assert np.all(np.abs(got - x @ w.T) <= 2e-6 * scale + 1e-7)
+
+
+@pytest.mark.parametrize("rows", [9, 64])
+def test_gated_block_of_one_tile_of_rows(tmp_path, rows):
+    cfg = lc.model(2048, 40, [lc.dense(lc.mamba(16, 2, 2, 2), 12283, limit=0.4)])
+    m, o, _ = build(tmp_path, cfg, 23, lc.BF16, n_ctx=512)
+    toks = tokens(cfg, 24, rows)
+    check(feed(m, toks, []), o.forward(toks), lc.BF16, "whole", o)
+
+
 def test_one_tile_of_rows_is_not_split_in_two():
     w = capi.Weight.upload(capi.BF16, np.zeros(24576 * 4096, np.uint16), 24576, 4096)
     for m, kernel in ((200, "dense_gemm"), (300, "dense_gemm_wide")):
