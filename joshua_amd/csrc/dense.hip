@@ -82,11 +82,17 @@ namespace {
 // How many runs a product's k is split into: one workgroup a tile fills the 256 compute units only from 256 tiles
 // on.  Runs of at least 4 stages (512 bytes of a row); depends on the shape only, so a shape keeps its order of
 // additions.
-// Up to 64 rows, one tile of them, wait for the weights: three workgroups a compute unit ask for them sooner than one (with the sums' launch,
-// us, one run / 768 workgroups, 16 and 64 rows: 24576 x 4096 61 / 45 and 63 / 52, 32000 x 4096 68 / 57 and 69 / 67), where that
-// takes three runs or more (two: 49152 x 4096 95 / 106).
-int gemm_splits(size_t tiles, int stages, bool one_row_tile) {
-    if (one_row_tile && tiles >= 192 && tiles <= 256 && stages >= 16) return (int)(768 / tiles);
+// `rows`, not 0: so many activation rows, one tile of them (64 at most), which wait for the weights: with more workgroups a compute unit they are
+// asked for sooner.  Two runs; three where two would begin a multiple of 4096 bytes apart, in the same memory channels; four where those
+// are three workgroups for every compute unit, from rows of 2560 on.  One where k is so short that the sums cost more.  With the sums' launch, us, weights from memory,
+// one / two / three / four runs: 32768 x 4096 of 16 rows 75 / 76 / 63 / 69, x 5120 90 / 72 / 72 / 77, x 6144 (three runs of 4096 bytes)
+// 117 / 86 / 107 / 102, x 8192 148 / 140 / 124 / 153; 24576 x 2048 38 / 28 / 30 / 30, x 4096 68 / 60 / 50 / 47, x 5120 82 / 60 / 61 / 57; of 64 rows
+// 32000 x 1024 24.0 / 27.2, x 1536 33.9 / 34.7, x 2048 42 / 40, x 4096 74 / 72 / 71; of 32 rows 32000 x 1024 23.2 / 22.9.
+int gemm_splits(size_t tiles, int stages, int rows) {
+    if (rows && tiles >= 192 && tiles <= 256 && stages >= 16 && 2 * stages >= rows) {
+        if (768 / tiles == 4 && stages >= 40) return 4;
+        return (stages + 1) / 2 % 32 == 0 ? 3 : 2;
+    }
     if (tiles >= 192) return tiles < 384 && stages >= 96 ? 2 : 1;  // long rows: a second workgroup a compute unit pays for the addition
     return (int)std::max<size_t>(1, std::min<size_t>({512 / tiles, (size_t)stages / 4, 16}));
 }
@@ -167,14 +173,14 @@ int run_gemm(uint32_t type, jq::DenseGemm a, size_t rows_of_a, size_t k, size_t 
     if constexpr (!GROUPED) {
         if (type == JQ_TYPE_BF16 && bn == 128 && !a.heads) {
             const auto u = tiles(bm, bn);
-            wide = wide_pick(a, wrows, bm, u.first * u.second, gemm_splits(u.first * u.second, a.stages, bm == 64 && u.first == 1));
+            wide = wide_pick(a, wrows, bm, u.first * u.second, gemm_splits(u.first * u.second, a.stages, bm == 64 && u.first == 1 ? a.M : 0));
         }
     }
     if (wide.bn) bm = 256, bn = wide.bn;
     const auto t = tiles(bm, bn);
     if (t.first * t.second > 0x7FFFFFFFull) return fail("dense gemm: too many tiles");
     a.m_tiles = (int)t.first;
-    a.splits = wide.bn ? wide.splits : GROUPED || a.heads ? 1 : gemm_splits(t.first * t.second, a.stages, type == JQ_TYPE_BF16 && bn == 128 && bm == 64 && t.first == 1);
+    a.splits = wide.bn ? wide.splits : GROUPED || a.heads ? 1 : gemm_splits(t.first * t.second, a.stages, type == JQ_TYPE_BF16 && bn == 128 && bm == 64 && t.first == 1 ? a.M : 0);
     CallScratch scratch;
     float *C = a.C;
     if (a.splits > 1) {

@@ -38,8 +38,11 @@ def test_products_of_many_rows(m, n, k, kernel):
 
 
 @pytest.mark.parametrize("m,n,k,kernel", [
-    (64, 24571, 2048, "dense_gemm+splitk"),    # 192 tiles of 128 weight rows, the last of them ragged: four runs
-    (9, 32640, 1090, "dense_gemm+splitk"),     # 255 tiles: three runs of 18 stages, the last one part-filled
+    (64, 24571, 2048, "dense_gemm+splitk"),    # 192 tiles of 128 weight rows, the last of them ragged: two runs
+    (61, 24571, 2530, "dense_gemm+splitk"),    # four runs of 10 stages, the last one part-filled
+    (9, 32640, 1090, "dense_gemm+splitk"),     # 255 tiles: two runs of 9 stages
+    (17, 32640, 4000, "dense_gemm+splitk"),    # 63 stages, of which two runs would begin 4096 bytes apart: three
+    (64, 32640, 1984, "dense_gemm"),           # 31 stages: the sums of 64 rows would cost more
     (33, 32769, 1024, "dense_gemm"),           # 257
     (65, 24571, 1024, "dense_gemm"),           # a second tile of rows
     (20, 24571, 900, "dense_gemm"),            # 15 stages
