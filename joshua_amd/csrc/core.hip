@@ -147,7 +147,7 @@ CallScratch::~CallScratch() {
     if (transient_) (void)hipFreeAsync(transient_, stream_);
 }
 
-int CallScratch::get(size_t bytes, hipStream_t s, uint8_t **out) {
+int CallScratch::get(size_t bytes, hipStream_t s, uint8_t **out, bool capturable) {
     stream_ = s;
     if (const FixedScratch *f = kind_ == 0 ? tl_fixed_scratch : nullptr) {
         if (bytes > f->bytes)
@@ -174,7 +174,7 @@ int CallScratch::get(size_t bytes, hipStream_t s, uint8_t **out) {
     }
     lock_ = std::unique_lock<std::mutex>(b->mu);
     if (b->bytes < bytes) {
-        if (bytes > SCRATCH_CAPTURABLE) {
+        if (capturable || bytes > SCRATCH_CAPTURABLE) {
             hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
             if (hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
             if (capture != hipStreamCaptureStatusNone) {

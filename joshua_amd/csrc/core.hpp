@@ -79,7 +79,8 @@ struct FixedScratchScope {
 // stream-ordered allocations, freed behind the call's launches.  First use and growth allocate: neither
 // is possible while the stream is being captured, so a caller warms a stream up with its largest call
 // before capturing it.  Requests above SCRATCH_CAPTURABLE need no such call: where the buffer does not hold one yet
-// and the stream is being captured, it is a stream-ordered allocation of the graph, like those above SCRATCH_KEEP.
+// and the stream is being captured, it is a stream-ordered allocation of the graph, like those above SCRATCH_KEEP; so are
+// smaller ones of a caller whose smaller calls can need more than its larger ones (`capturable`).
 //
 // jq_matmul_t_noalloc serves the same requests from a fixed array in device memory instead (below): it
 // installs the array for the calling thread with FixedScratchScope, and get() then hands out that
@@ -99,7 +100,7 @@ public:
     CallScratch &operator=(const CallScratch &) = delete;
     ~CallScratch();
     // 0 on success; on failure the message is set
-    int get(size_t bytes, hipStream_t s, uint8_t **out);
+    int get(size_t bytes, hipStream_t s, uint8_t **out, bool capturable = false);
 };
 
 // Frees a device allocation when it goes out of scope.

@@ -180,7 +180,8 @@ int run_gemm(uint32_t type, jq::DenseGemm a, size_t rows_of_a, size_t k, size_t 
     const auto t = tiles(bm, bn);
     if (t.first * t.second > 0x7FFFFFFFull) return fail("dense gemm: too many tiles");
     a.m_tiles = (int)t.first;
-    a.splits = wide.bn ? wide.splits : GROUPED || a.heads ? 1 : gemm_splits(t.first * t.second, a.stages, type == JQ_TYPE_BF16 && bn == 128 && bm == 64 && t.first == 1 ? a.M : 0);
+    const int few = type == JQ_TYPE_BF16 && bn == 128 && bm == 64 && t.first == 1 ? a.M : 0;
+    a.splits = wide.bn ? wide.splits : GROUPED || a.heads ? 1 : gemm_splits(t.first * t.second, a.stages, few);
     CallScratch scratch;
     float *C = a.C;
     if (a.splits > 1) {
@@ -191,7 +192,8 @@ int run_gemm(uint32_t type, jq::DenseGemm a, size_t rows_of_a, size_t k, size_t 
         }
         uint8_t *p = nullptr;
         if (a.splits > 1) {
-            if (scratch.get((size_t)a.splits * a.M * width * sizeof(float), s, &p)) return 1;
+            // (a second tile of rows against as many weight rows has one run, so a call of more rows leaves no buffer for these)
+            if (scratch.get((size_t)a.splits * a.M * width * sizeof(float), s, &p, few && t.second >= 192)) return 1;
             a.C = (float *)p;
         }
     }

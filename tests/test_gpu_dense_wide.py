@@ -110,3 +110,36 @@ def test_gated_block_in_every_tile_and_in_runs(rows, runs):
     res = subprocess.run([sys.executable, "-c", CHILD.replace("ROOT", repr(ROOT), 1).replace("RUNS", str(runs))], capture_output=True, text=True, timeout=110,
                          env=dict(os.environ, JQ_DENSE_WIDE=f"{rows},{runs}"))
     assert res.returncode == 0 and "wide ok" in res.stdout, res.stdout + res.stderr
+
+
+def test_capture_of_one_tile_of_rows_behind_a_larger_call():
+    """100 rows need no sums, 64 have two runs' worth: a stream that ran the larger call can be captured over the smaller one."""
+    import torch
+    n, k = 24571, 2048
+    w = capi.Weight.upload(capi.BF16, sl.to_bf16(normal(5, (n, k), k ** -0.5)), n, k)
+    x = torch.from_numpy(normal(6, (100, k))).cuda()
+    want, y = torch.empty(64, n, device="cuda"), torch.empty(100, n, device="cuda")
+
+    def product(m, out, stream):
+        w.matmul_t_dev(m, x.data_ptr(), m * k, out.data_ptr(), m * n, stream)
+
+    product(64, want, torch.cuda.current_stream().cuda_stream)
+    assert capi.last_kernel() == "dense_gemm+splitk"
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    product(100, y, stream.cuda_stream)
+    assert capi.last_kernel() == "dense_gemm"
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        product(64, y, stream.cuda_stream)
+    for _ in range(3):
+        y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y[:64], want)
+        product(64, torch.empty_like(want), torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+    del graph
+    torch.cuda.synchronize()
+    capi.stream_release(stream.cuda_stream)
