@@ -85,12 +85,29 @@ lhs[7, 100], lhs[8, 2000], lhs[9, 5] = np.inf, np.nan, -np.inf
 other = capi.Weight.upload(capi.Q4_K, raw.reshape(-1), n, k).matmul_t(50, lhs)
 assert np.all(np.isnan(other[7:10])), "a row that is not finite"
 assert np.array_equal(np.delete(other, [7, 8, 9], 0), np.delete(got, [7, 8, 9], 0)), "its neighbours"
-if splits == 1:  # SwiGLU in the preparation: the down projection of a decoder's prompt
-    from tests.test_gpu_qwen3 import CFG, make, close
-    m, o = make(dict(CFG, n_ctx=64), 77, "q4_k")
-    tokens = rng.integers(0, 768, 45).tolist()
-    ok, e = close(m.forward(tokens, 0), o.forward(tokens, 0))
-    assert ok, e
+# gate and up rows in turn: SwiGLU where the product is stored, in one part of k
+from tests.h6_swiglu import swiglu_product
+for m, k, n in [(17, 256, 64), (33, 512, 114), (64, 1024, 98), (129, 768, 112), (257, 512, 300), (256, 1024, 96), (40, 4096, 130)]:
+    blocks, lhs = synth.normal_quantized(capi.Q4_K, 15 + n, n * k, 0.02), synth.normal(16 + k, (m, k))
+    rc, got = swiglu_product(blocks, n, lhs)
+    if splits > 1:
+        assert rc == -1 and np.isnan(got).all()
+        continue
+    assert rc == 0 and np.isnan(got[m]).all() and np.isfinite(got[:m]).all(), (m, k, n)
+    y = lhs.astype(np.float64) @ oracle.dequantize(capi.Q4_K, blocks).reshape(n, k).astype(np.float64).T
+    gate, up = y[:, 0::2], y[:, 1::2]
+    act = gate / (1 + np.exp(-gate))
+    # the products are 2e-5 of their root mean square off (above) and silu's slope is at most 1.1; silu and the last product: some 2^-20
+    rms = lambda v: np.sqrt((v ** 2).mean())
+    assert rms(got[:m] - act * up) <= 2e-5 * rms(up) * (1.1 * rms(gate) + rms(act)) + 1e-6 * rms(act * up), (m, k, n)
+    assert np.abs(got[:m] - act * up).max() <= 12 * 2e-5 * (1.1 * rms(gate) * np.abs(up).max() + np.abs(act).max() * rms(up)), (m, k, n)
+assert swiglu_product(synth.normal_quantized(capi.Q4_K, 8, 113 * 512, 0.02), 113, synth.normal(9, (33, 512)))[0] == -1  # a gate without its up
+# a decoder's prompt over such rows (4096 wide): in one part of k as above, in several the down projection's preparation applies SwiGLU
+from tests.test_gpu_qwen3 import CFG, make, close
+m, o = make(dict(CFG, n_layer=2, hidden=4096, n_head=4, n_kv_head=2, head_dim=128, ffn=4096, n_ctx=64), 77, "q4_k")
+tokens = rng.integers(0, 768, 45).tolist()
+ok, e = close(m.forward(tokens, 0), o.forward(tokens, 0))
+assert ok, e
 print("h6 ok")
 """
 

@@ -7,7 +7,8 @@ import pytest
 import oracle
 from oracle import qwen3 as oq
 from joshua_amd import capi, synth
-from joshua_amd.synth.model import qwen3_tensors
+from joshua_amd.synth.model import qwen3_tensor_plan, qwen3_tensors
+from tests.h6_swiglu import swiglu_product
 
 pytestmark = pytest.mark.gpu
 
@@ -591,10 +592,26 @@ def test_single_token_steps_with_1536_wide_rows(mix):
 
 
 @pytest.mark.parametrize("ffn,tokens", [(2048, 128), (2304, 131), (2304, 257), (3840, 160)])
-def test_gate_and_up_of_many_tokens_with_the_activation_in_the_product(ffn, tokens):
-    """hidden = 1024 leaves the paired product one part of k, so that SwiGLU is its epilogue: whole tiles, ragged ones of either side,
-    a row of the result in odd and even lanes; a down projection of Q4_K and of Q6_K."""
+def test_gate_and_up_of_many_tokens(ffn, tokens):
+    """hidden = 1024: gate and up as products of their own, SwiGLU between two launches; a down projection of Q4_K and of Q6_K."""
     cfg = dict(CFG, n_layer=4, hidden=1024, n_head=8, n_kv_head=2, head_dim=128, ffn=ffn, vocab=512, n_ctx=300)
+    m, o = make(cfg, 41, "q4_k_m")
+    toks = np.random.default_rng(23).integers(0, 512, tokens + 1).tolist()
+    ok, e = close(m.forward(toks[:tokens], 0), o.forward(toks[:tokens], 0))
+    assert ok, e
+    ok, e = close(m.forward(toks[tokens:], tokens), o.forward(toks[tokens:], tokens))
+    assert ok, e
+
+
+@pytest.mark.parametrize("ffn,tokens,inside", [(4864, 257, True), (6144, 257, True), (8192, 257, True), (4096, 600, True), (2048, 131, False)])
+def test_gate_and_up_of_many_tokens_with_the_activation_in_the_product(ffn, tokens, inside):
+    """hidden = 4096 pairs gate and up rows.  SwiGLU where their product is stored, in workgroups of four waves and of eight with six, eight and
+    seven groups of weight rows, rows ragged (and columns, of six and seven groups); in four parts of k, in the down projection's preparation.
+    Down projections of Q4_K and of Q6_K."""
+    cfg = dict(CFG, n_layer=4, hidden=4096, n_head=4, n_kv_head=2, head_dim=128, ffn=ffn, vocab=512, n_ctx=640)
+    assert {qt for n, qt, _, _ in qwen3_tensor_plan(cfg, "q4_k_m") if n.endswith("ffn_down.weight")} == {capi.Q4_K, capi.Q6_K}
+    rc, out = swiglu_product(np.zeros(2 * ffn * 16 * 144, np.uint8), 2 * ffn, np.ones((tokens, 4096), np.float32))
+    assert (rc == 0 and not out[:-1].any()) if inside else rc == -1
     m, o = make(cfg, 41, "q4_k_m")
     toks = np.random.default_rng(23).integers(0, 512, tokens + 1).tolist()
     ok, e = close(m.forward(toks[:tokens], 0), o.forward(toks[:tokens], 0))
