@@ -331,8 +331,8 @@ def test_memory_of_an_object_over_a_long_context():
 @pytest.mark.parametrize("n_head,vh,prompt", [(4, 64, 1), (4, 128, 300), (32, 128, 40), (32, 64, 700)])
 def test_one_token_over_q4k_blocks_of_the_up_projection(n_head, vh, prompt):
     """Single-token steps that read kv_b as Q4_K blocks (512 latents, 128 unrotated elements a head), against the same layer
-    over its f32 values: one context split and many, either attention kernel, value rows of one and two workgroups a head.  The
-    same weights up to the order of f32 sums of 128 and 512 terms and of their offsets: 1e-5 of the largest."""
+    over its f32 values: short contexts, which take one launch between the query and the output projection, value rows of one and two
+    workgroups a head.  The same weights up to the order of f32 sums of 128 and 512 terms and of their offsets: 1e-5 of the largest."""
     c = cfg(n_embd=256, n_head=n_head, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=vh, context_length=prompt + 8)
     ref, dev = build(c, qtype=capi.Q4_K, seed=450 + n_head)
     raw = {n: (r, k) for n, r, k in (("q", n_head * 192, 256), ("kv_a_mqa", 576, 256), ("o", 256, n_head * vh))}
@@ -344,6 +344,26 @@ def test_one_token_over_q4k_blocks_of_the_up_projection(n_head, vh, prompt):
     x = normal(17, (prompt + 3, 256)) * np.float32(2.0)
     dev.forward(x[:prompt], 0), dense.forward(x[:prompt], 0)
     for p in range(prompt, prompt + 3):
+        a, b = dev.forward(x[p:p + 1], p), dense.forward(x[p:p + 1], p)
+        assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max(), p
+
+
+@pytest.mark.parametrize("n_head,vh,prompt", [(4, 128, 894), (32, 64, 894), (32, 128, 1500), (128, 128, 893), (264, 64, 5), (136, 128, 318), (160, 128, 318)])
+def test_steps_in_three_launches_over_q4k_blocks(n_head, vh, prompt):
+    """As above, absorption, attention and merging with the value rows a launch each: from 896 cached tokens on (the first steps of some cases
+    are still one launch), by either attention kernel, and with more heads times 64 value rows than compute units, where the attention of up
+    to 320 tokens has a kernel of its own."""
+    c = cfg(n_embd=256, n_head=n_head, kv_lora_rank=512, qk_nope=128, qk_rope=64, v_head_dim=vh, context_length=prompt + 8)
+    ref, dev = build(c, qtype=capi.Q4_K, seed=460 + n_head)
+    raw = {n: (r, k) for n, r, k in (("q", n_head * 192, 256), ("kv_a_mqa", 576, 256), ("o", 256, n_head * vh))}
+    w = {n: capi.Weight.upload(capi.Q4_K, ref.t[n][1], r, k) for n, (r, k) in raw.items()}
+    mc = capi.MlaConfig(n_embd=256, n_head=n_head, q_lora_rank=0, kv_lora_rank=512, qk_nope_head_dim=128, qk_rope_head_dim=64,
+                        v_head_dim=vh, n_ctx=prompt + 8, rms_eps=1e-6, rope_theta=1e4)
+    values = oracle.dequantize(capi.Q4_K, ref.t["kv_b"][1]).reshape(n_head * (128 + vh), 512).astype(np.float32)
+    dense = capi.Mla(mc, w["q"], w["kv_a_mqa"], ref.t["kv_a_norm"], values, w["o"])
+    x = normal(18, (prompt + 6, 256)) * np.float32(2.0)
+    dev.forward(x[:prompt], 0), dense.forward(x[:prompt], 0)
+    for p in range(prompt, prompt + 6):
         a, b = dev.forward(x[p:p + 1], p), dense.forward(x[p:p + 1], p)
         assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max(), p
 
