@@ -2185,7 +2185,9 @@ int moe_forward_dev(jq_moe *m, size_t T, const float *x, float *y, hipStream_t s
             planes = m->qi8;
         // the matrix-core gate and up kernel can run the gating itself
         static const char *no_late_gate = getenv("JQ_MOE_NO_GATING_IN_GATE_UP");
-        const bool late = !no_late_gate && m->gate->type == m->up->type && moe_gate_up_mfma_takes(m, x);
+        // (rows of more than 8 super-blocks: as many workgroups as run side by side)
+        const size_t gate_up_wgs = c.hidden > 8 * 256 ? 512 : ((size_t)c.inter + 7) / 8 * ((size_t)P + (size_t)extra * T);
+        const bool late = !no_late_gate && m->gate->type == m->up->type && moe_gate_up_mfma_takes(m, x) && moe_gate_rides(c, gate_up_wgs);
         // one token of a decoder layer: the norm in front of the experts runs inside the router launch
         static const char *no_pre = getenv("JQ_MOE_NO_NORM_IN_ROUTER");
         if (pre) {

@@ -373,7 +373,8 @@ int moe_forward_dense(jq_moe *m, size_t T, const float *x, const void *xe, float
     gp.ld = ex.logits ? (int)ex.ld : 0;
     auto gate = [&] { return moe_gate_dev(m, T, ex.logits ? ex.logits : m->logits, gp, no_groups, s); };
     if (decode) {
-        const bool wave = moe_wave_gate(c);
+        const dim3 grid((unsigned)((std::max(inter, sn) + 3) / 4), (unsigned)(P + (sn ? (int)T : 0)));
+        const bool wave = moe_gate_rides(c, (size_t)grid.x * grid.y);
         jq::MoeGateIn gi{ex.logits ? ex.logits : m->logits, m->router_bias, gp, m->ids, m->wts, no_groups, (int)T};
         if (ex.logits) {
             if (!wave && gate()) return 1;
@@ -388,7 +389,6 @@ int moe_forward_dense(jq_moe *m, size_t T, const float *x, const void *xe, float
             if (moe_route_dev(m, T, x, s, no_groups, jq::ActsI8{nullptr, nullptr, nullptr, nullptr}, nullptr, wave ? &later : nullptr)) return 1;
         }
         const jq::SharedRows sh{sn ? m->sgate->dev : nullptr, sn ? m->sup->dev : nullptr, sn, m->sG, sl, ld_sl, P, shared_unit.limit};
-        const dim3 grid((unsigned)((std::max(inter, sn) + 3) / 4), (unsigned)(P + (sn ? (int)T : 0)));
 #define JQ_GU(NE)                                                                                                             \
     JQ_ELEM(type, hipLaunchKernelGGL((jq::moe_dense_gate_up<E, NE>), grid, dim3(256), 0, s, m->pgate, m->pup, m->gate->row_bytes, x, \
                                      (size_t)h, m->G, (size_t)inter, h, inter, ku, m->ids, unit, gi, sh))

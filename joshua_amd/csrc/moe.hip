@@ -71,10 +71,15 @@ bool moe_wave_gate(const jq_moe_config &c) {
     return !no_wave && (c.n_group <= 1 || (per >= 2 && per <= 64 && (per & (per - 1)) == 0)) && c.n_expert <= 256 && c.n_expert_used <= 64;
 }
 
+// Experts in groups: some 5 us of a wave, against a launch of 4 to 8, so only where every workgroup is there from the start.  A layer call, 256 experts in 8
+// groups, inside / a launch of its own, us: Q4_K 2048 x 512, 512 workgroups a token, 1 token 17.0 / 18.2, 2 19.7 / 20.6, 3 30.0 / 26.6, 8 63 / 45,
+// 16 108 / 70; 2048 x 768 1 token 18.3 / 19.4, 2 29.4 / 25.0; 64 experts of 2048 x 1536, 1152 workgroups, 1 token 27.7 / 23.3.  Without groups it is 2 us and hidden.
+bool moe_gate_rides(const jq_moe_config &c, size_t workgroups) { return moe_wave_gate(c) && (c.n_group <= 1 || workgroups <= 1024); }
+
 // `planes`: also leave x as fixed-point planes there (the one-expert-a-workgroup router kernel does; *planes_made
 // says whether it ran)
 // `gate_later`: when the gating can run by one wave a token, it is left to the caller's next kernel (the logits are
-// in m->logits) and *gate_later holds its operands; else it is cleared.
+// in m->logits) and *gate_later holds its operands; else it is cleared.  Null: it is not left to anyone.
 // `pre`: the decoder layer's residual add and RMSNorm run inside the router launch (one token; x is then pre->hn_out,
 // which that launch writes).
 int moe_route_dev(jq_moe *m, size_t T, const float *x, hipStream_t s, jq::MoePairGroups pg,

@@ -77,6 +77,8 @@ int moe_group_dev(jq_moe *m, size_t T, int extra, hipStream_t s);
 jq::MoeGateParams moe_gate_params(const jq_moe_config &c);
 // Whether the gating runs by one wave a token.
 bool moe_wave_gate(const jq_moe_config &c);
+// Whether it then rides in a kernel behind it of so many workgroups, every one of which runs it for its token.
+bool moe_gate_rides(const jq_moe_config &c, size_t workgroups);
 void moe_swap_scratch(jq_moe *a, jq_moe *b);
 
 }  // namespace jqh

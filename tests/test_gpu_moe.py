@@ -6,6 +6,7 @@ import pytest
 import oracle
 from oracle.moe import MoeOracle
 from joshua_amd import capi, synth
+from joshua_amd.synth import layered as sl
 
 pytestmark = pytest.mark.gpu
 
@@ -72,6 +73,34 @@ def test_route_of_experts_in_groups(gating, E, groups, kept, used):
     for row in ids:
         assert len(set(row.tolist())) == used and row.max() < E
     assert np.array_equal(ids[1], np.arange(used)) and np.isnan(w[1]).all()
+
+
+@pytest.mark.parametrize("qtype,tokens", [(capi.Q4_K, 1), (capi.Q4_K, 2), (capi.Q4_K, 3), (capi.Q4_K, 9), (capi.BF16, 1), (capi.BF16, 4), (capi.BF16, 5), (capi.BF16, 8)])
+def test_decode_sized_calls_over_experts_in_groups(qtype, tokens):
+    """Gating inside the expert kernel up to 1024 workgroups of it (two tokens of Q4_K, four of plain rows), a launch of its own from there."""
+    E, used, bias = (64, 8, 0.02) if qtype == capi.Q4_K else (16, 4, 0.02)
+    kw = dict(gating="sigmoid", n_group=4, topk_group=2, weights_scale=2.5, router_bias=np.linspace(bias, -bias, E).astype(np.float32))
+    x = synth.normal(47, (tokens, 512))
+    if qtype == capi.Q4_K:
+        ora, dev = build(qtype, 512, 512, E, used, 48, **kw)
+        assert close(dev.forward(x), ora.forward(x))
+        return
+    inter, rw = 256, synth.normal(50, (E, 512), 0.05)
+    w = [sl.to_bf16(synth.normal(51 + i, (E * n, k), k ** -0.5)) for i, (n, k) in enumerate([(inter, 512), (inter, 512), (512, inter)])]
+    cfg = capi.MoeConfig(E, used, 512, inter, 1, 1, 2.5, 4, 2)
+    dev = capi.Moe(cfg, rw, *(capi.Weight.upload(qtype, v, *v.shape) for v in w), router_bias=kw["router_bias"])
+    gate, up, down = (sl.from_bf16(v).astype(np.float64).reshape(E, -1, v.shape[1]) for v in w)
+    ids, wts = dev.route(x)
+    logits = x.astype(np.float64) @ rw.astype(np.float64).T
+    best = np.sort((1 / (1 + np.exp(-logits)) + kw["router_bias"]).reshape(tokens, 4, 4), 2)[:, :, 2:].sum(2).argsort(1)[:, 2:]
+    assert all(set(row // 4) <= set(kept) for row, kept in zip(ids, best))
+    want = np.zeros((tokens, 512))
+    for t, v in enumerate(x.astype(np.float64)):
+        for e, wt in zip(ids[t], wts[t]):
+            g = gate[e] @ v
+            want[t] += wt * (down[e] @ (g / (1 + np.exp(-g)) * (up[e] @ v)))
+    # f32 sums of 512 and 256 terms: some 2^-24 of the terms' magnitudes a rounding
+    assert np.abs(dev.forward(x) - want).max() <= 1e-5 * np.abs(want).max()
 
 
 @pytest.mark.parametrize("h,E,tokens", [(544, 30, 45), (2080, 9, 33), (1024, 64, 128)])
