@@ -3082,8 +3082,10 @@ bool model_norm_mm(const jq_weight *w, const float *x, const float *res, const f
 // 4000 tokens 9 tokens 1973 / 1237.  Where heads are grouped as no f32 kernel takes them (`tiled` false) the line is 32 tokens.
 bool split16_attention_pays(uint32_t T, uint32_t pos, bool tiled) { return T >= (tiled ? 64u : 32u) || pos + T >= 128; }
 
-// A short step's rows of the embedding, position and angles in one launch; -1 where the embedding is in no block format.
+// A short step's rows of the embedding, position and angles in one launch; -1 where the embedding is in no block format or the tokens are more
+// than the launch has room for.
 int model_step_begin(Qwen3Model *m, const jq_weight *emb, const uint32_t *tokens, uint32_t T, uint32_t pos, hipStream_t s) {
+    if (T > (uint32_t)jq::STEP_TOKENS) return -1;
     jq::StepTokens ids{};
     std::copy(tokens, tokens + T, ids.id);
     const size_t k = emb->k;
