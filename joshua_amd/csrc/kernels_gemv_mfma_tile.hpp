@@ -26,7 +26,7 @@ template <class F, bool NORM>
 constexpr int gemv_mfma_tile_stage() { return (F::STAGE_BYTES + 15) / 16 * 16 + (NORM ? 3 : 1) * 1024; }  // prepare()'s words, then x, norm weight, res
 
 // A row's stride: an odd number of 16 bytes, so that 16 rows read at one place meet all banks once.
-constexpr int gemv_mfma_tile_row_lds(int bytes) { return (bytes / 16 + 1) / 2 * 32 + 16; }
+constexpr int gemv_mfma_tile_row_lds(int bytes) { return (bytes / 16 | 1) * 16; }
 
 // The sums take the place of prepare()'s words and the raw rows.
 template <class F, int NB, bool NORM, int NT = 1>
