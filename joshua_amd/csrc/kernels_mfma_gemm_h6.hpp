@@ -339,7 +339,8 @@ __device__ __forceinline__ h6_i8 h6_operand6(h6_u6 v) {
 // SWIGLU: the weight rows are gate_j and up_j in turn, and Y gets n / 2 values silu(gate_j) up_j a row: two lanes beside each other hold
 // a pair's two products of four rows, and each finishes two of them.  (The 201 MB of 2048 x 24576 products were stored and read again by
 // the next product's preparation; times at gemm_h6_swiglu's declaration.)
-// (Four waves: two workgroups a compute unit.  Not told so, the compiler keeps the sums in accumulation registers and copies them out.)
+// (Four waves: two workgroups a compute unit.  Not told so, the compiler keeps the sums in accumulation registers and copies them out:
+// 128 to 512 rows x 4096 to 14336 x 4096 to 12288 on this shape, Q4_K 0.96 to 1.00 of the time, MXFP4 0.98 to 1.04, on the picked one 0.96 to 1.01.)
 template <class F, int NW, int NG, bool SWIGLU = false>
 static __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void kq_gemm_h6(const uint8_t *__restrict__ W, size_t row_bytes,
                                                       const uint8_t *__restrict__ acts, float *__restrict__ Y, int m_rows, int n,

@@ -927,7 +927,7 @@ struct QiGrouped {
 // multiply (for the tiles of few rows, whose two waves a workgroup leave the unpacking's lookups nothing to hide behind).
 // Four waves: two workgroups a compute unit, which leaves a wave 256 registers.  Not told so, the compiler keeps the integer sums in
 // accumulation registers and copies every one out in front of its conversion, 96 of 800 vector instructions a super-block (Q6_K 333 x
-// 4096 x 12288 107.4 -> 105.5 us a call: the clock gives back most of it, the chip being at its power limit).
+// 4096 x 12288 107.4 -> 105.5 us a call; 128, 200 and 333 rows x 4096 x 4096 of eleven formats 0.93 to 1.00 of the time).
 template <class F, int NW, int NG, bool GROUPED = false, bool NSPLIT = false, bool SINGLE = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void kq_gemm_i8(const uint8_t *__restrict__ W, size_t row_bytes,
                                                       const uint8_t *__restrict__ acts, float *__restrict__ Y,

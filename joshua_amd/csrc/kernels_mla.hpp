@@ -621,7 +621,7 @@ __global__ __launch_bounds__(512) void mla_merge_vproj_q4k(const float *__restri
 // time with their rows in registers, merges the waves' sums and multiplies with 64 value rows.  f32 throughout.
 // Bound: a chain of some 900 vector instructions a wave, four waves a SIMD, and three trips to memory.  128 heads of 128 + 64 elements
 // behind 100 tokens: 9.5 to 11.5 us where absorbing, scoring and merging with the value rows, a launch each, take 6.2, 5.1 and 5.0 and
-// their boundaries: a layer's step 44.6 -> 37.0 us.  All value rows in one workgroup a head, half the compute units idle: 37.5.
+// their boundaries (whole steps: at the dispatch).  All value rows in one workgroup a head, half the compute units idle: 0.5 us a step slower.
 __device__ __forceinline__ float mla_sum_half(float v) {  // over the 32 lanes of a half-wave
     v = sum_xor16(v);
     return sum_row16(v);

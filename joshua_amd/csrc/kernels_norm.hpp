@@ -150,6 +150,8 @@ __global__ __launch_bounds__(BT) void residual_norm_rows(ResidualNorm a, typenam
     const float *xr = a.x + row * (a.ldx ? a.ldx : (size_t)w);
     // Loads past the width repeat the last column, so that none needs a branch, and all of a row's vector are asked for before the first
     // is waited for, and in front of any store: one by one they were 12 of 17.5 us, of one row of 4096 columns or of 512.
+    // (128 registers for 70 to 84, so four waves a SIMD for six or seven: rows of 1024 to 16384, 1 to 4096 of them, with and without a norm on y and
+    // biases, take 0.62 to 0.98 of the time all the same; 4096 rows of 16384 206 -> 178 us.)
     auto ask = [&](const float *src, float (&v)[NV]) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < NV; i++) v[i] = src[min(c0 + BT * i, w - 1)];
